@@ -274,6 +274,37 @@ int mxmoe_unpermute_combine_planned(const void* down_out, const void* d_plan_dow
 int mxmoe_combine_planned(const void* down_out, const void* d_plan_down, int num_problems, const float* topk_weights, const int32_t* row_of_slot, int num_tokens,
                           int topk, int K, void* out, void* stream);
 
+/* ---- the planned forward in its short form ----
+ *
+ * One call enqueues the whole forward of one layer for one (tokens, top-k): permutation, planning and the quantisation of every
+ * token once per activation format in one launch; the gate_up GroupGEMM with rows gathered by token and silu(gate) * up as its
+ * output; quantisation of those rows (left out when every second block reads fp16); the down GroupGEMM; the combine.  Results are
+ * bit for bit those of the separate entry points above.
+ *
+ * mxmoe_layer_desc names everything that does not change from call to call; every buffer belongs to the caller, is device memory
+ * (h_* excepted) and is sized for the worst routing (R = num_tokens * topk rows):
+ *   d_* / h_*      block descriptors of the experts (+ the shared one last), on the device and on the host;
+ *   token_store    per activation tag (0 fp16, 1 int8, 2 int4, 3 int4 group-128, 5 fp8) that a first block uses: [num_tokens] packed
+ *   token_scales   rows and their scales; tag 0 only with rotate = 2 (else the tokens are read where they are), others may be NULL;
+ *   act            fp16 [R][inter], then [num_tokens][inter_shared];
+ *   down_inp, down_scales, down_out   as for mxmoe_plan_block;
+ *   plan_*         mxmoe_plan_bytes() each;
+ *   dst_exp, token_of_row, row_of_slot   int32 [R]; iota   int32 [num_tokens] = 0, 1, 2, ...; recv   int64 [num_experts];
+ *   workspace      mxmoe_permute_workspace_bytes(R, num_experts), 16-byte aligned.
+ * grid_*: mxmoe_plan_grid_bound of each block.  rotate, had_*: of the intermediate rows, as for mxmoe_silu_mul_quant (bits 0 - 1 only).
+ *
+ * mxmoe_layer_supported   1 when the short form takes the layer: hidden 512, 1024, 2048 or 4096; at most 1024 experts; inter a
+ *                         multiple of 32; no bf6 operands; token stores and fp16 weights below 2 GiB; and R <= 65536, or
+ *                         ceil(R / 256) * num_experts <= 16384.  Else 0: use the separate entry points.
+ * mxmoe_layer_create      checks the description and copies it; the handle is read only afterwards (mxmoe_layer_run may be called from several
+ *                         threads as far as the buffers it names allow) and is given back with mxmoe_layer_destroy.
+ * mxmoe_layer_run         enqueues on `stream`; hidden fp16 [num_tokens][hidden], topk_ids int32 [num_tokens][topk] (ids out of range are
+ *                         dropped), topk_weights fp32, out fp16 [num_tokens][hidden].  Neither allocates nor synchronises. */
+int mxmoe_layer_supported(const mxmoe_layer_desc* desc);
+int mxmoe_layer_create(const mxmoe_layer_desc* desc, void** handle);
+void mxmoe_layer_destroy(void* handle);
+int mxmoe_layer_run(const void* handle, const void* hidden, const int32_t* topk_ids, const float* topk_weights, void* out, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -17,6 +17,15 @@ class PlanCall(C.Structure):
                 ("out_store", C.c_void_p), ("d_plan", C.c_void_p)]
 
 
+class LayerDesc(C.Structure):
+    """mxmoe_layer_desc."""
+    _fields_ = [*((n, C.c_int32) for n in ("num_tokens", "topk", "num_experts", "has_shared", "hidden", "inter", "inter_shared", "rotate", "had_k", "had_f")),
+                ("had_signs", C.c_void_p), *((n, C.c_int32) for n in ("kernel_gate_up", "kernel_down", "grid_gate_up", "grid_down")),
+                *((n, C.c_void_p) for n in ("d_gate_up", "h_gate_up", "d_down", "h_down")), ("token_store", C.c_void_p * 6), ("token_scales", C.c_void_p * 6),
+                *((n, C.c_void_p) for n in ("act", "down_inp", "down_scales", "down_out", "plan_gate_up", "plan_down", "dst_exp", "token_of_row", "row_of_slot", "iota",
+                                            "recv", "workspace"))]
+
+
 class BlockDesc(C.Structure):
     """mxmoe_block_desc: one linear block of one expert for the device-side planner (40 bytes)."""
     _fields_ = [("a_bits", C.c_int32), ("w_bits", C.c_int32), ("gsize", C.c_int32), ("sym", C.c_uint8), ("_pad", C.c_uint8 * 3),
@@ -70,6 +79,10 @@ SIGNATURES = {
     "mxmoe_unpermute_combine_planned": (_I, [_P, _P, _I, _P, _P, _I, _I, _I, _P, _P, _P]),
     "mxmoe_group_gemm_plan_tables": (_I, [_I, C.POINTER(Dim3), C.POINTER(QParams), _I, C.POINTER(C.c_int32), _I]),
     "mxmoe_group_gemm_plan_tile_map": (_I, [_I, C.POINTER(Dim3), C.POINTER(QParams), _I, _I, C.POINTER(C.c_int32)]),
+    "mxmoe_layer_supported": (_I, [_P]),
+    "mxmoe_layer_create": (_I, [_P, C.POINTER(_P)]),
+    "mxmoe_layer_destroy": (None, [_P]),
+    "mxmoe_layer_run": (_I, [_P, _P, _P, _P, _P, _P]),
     "mxmoe_combine_workspace_bytes": (C.c_size_t, [_I, _I]),
     "mxmoe_unpermute_combine": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P]),
 }

@@ -23,6 +23,7 @@
 #include "include/mxmoe_launch.hpp"
 #include "include/mxmoe_plan.hpp"
 #include "include/mxmoe_perm.hpp"
+#include "include/mxmoe_rows.hpp"
 
 namespace mxmoe {
 
@@ -53,9 +54,9 @@ __global__ void __launch_bounds__(64) perm_scan_kernel(int32_t* __restrict__ his
   for (int b0 = 0; b0 < blocks; b0 += 64) {
     const int b = b0 + lane;
     const int v = b < blocks ? hist[b * E + e] : 0;
-    const int inc = wave_inclusive_scan(v, lane);
+    const int inc = wave_inclusive_scan(v);
     if (b < blocks) hist[b * E + e] = carry + inc - v;
-    carry += __shfl(inc, 63);
+    carry += wave_last(inc);
   }
   if (lane == 0) recv[e] = carry;
 }
@@ -116,8 +117,7 @@ __global__ void __launch_bounds__(256) route_topk_kernel(const RouteArgs a) {
     p[e] = x;
     mx = fmaxf(mx, x);
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+  mx = wave_max(mx);
   float sum = 0.0f;
   for (int e = lane; e < a.E; e += 64) {
     const float v = expf(p[e] - mx);
@@ -178,12 +178,13 @@ struct RowArgs {
   uint8_t* inp_store;
   _Float16* scale_store;
   const int32_t* dst_exp;
-  const int64_t* perm;
+  const int64_t* perm;   // source row of each routed row, or null: the row itself
   const int64_t* table;  // [4][Et]: tag, start_row, inp_off, scale_off (offsets in fp16 elements)
   const float* signs;    // B as +-1.0f, [kb][kb], or null
   int R, T, E, Et;
   int rows;
   int rotate;  // 0 never, 1 rows of quantised experts, 2 every row
+  int direct;  // leave fp16 rows (tag 0) alone: their consumer reads the source
   RotPlan plan, plan_shared;
   // Planned mode (the tables were written by the device-side planner, the host never saw the counts): R is then the CAPACITY of the
   // routed part (tokens x top-k), rows routed .. R-1 do not exist when expert ids were dropped, and the shared expert's source rows
@@ -194,65 +195,13 @@ struct RowArgs {
 
 // rows [routed, R) of a planned launch do not exist
 __device__ __forceinline__ bool row_exists(const RowArgs& a, int row) { return !a.routed_ptr || row >= a.R || row < (int)*a.routed_ptr; }
+// source row of a routed row (not the activation step, whose source rows are the rows themselves)
+__device__ __forceinline__ long source_row(const RowArgs& a, int row) { return a.perm ? (long)const_load(a.perm + row) : (long)row; }
+// fp16 rows that their consumer reads at their source
+__device__ __forceinline__ bool row_stays(const RowArgs& a, int tag) { return a.direct && tag == 0; }
 __device__ __forceinline__ const _Float16* shared_src(const RowArgs& a) {
   return a.shared_src_addr ? reinterpret_cast<const _Float16*>(*a.shared_src_addr) : a.src_shared;
 }
-// Load of a value that no kernel of this launch writes (routing arrays, expert table), through the constant address space: with a
-// wave-uniform address it is a scalar load into scalar registers, off the vector register budget.
-template <class T>
-__device__ __forceinline__ T const_load(const T* p) {
-  return *(const __attribute__((address_space(4))) T*)(p);
-}
-
-// silu(g) = g / (1 + exp(-g)) as a fixed sequence of correctly rounded fp32 operations and exact integer ones, identical to the CPU
-// restatement (every multiply-add is fused: one rounding): exp(-g) = 2^t with t = clamp(-g log2(e), +-100) split into k = rint(t) and
-// f = t - k (exact), 2^f by a degree-4 Horner polynomial (relative error 3.7e-6), 2^k added to the exponent field (the result stays a
-// normal number); the reciprocal of d = 1 + exp(-g) from an integer-subtraction seed (within 5.06 %) and two Newton steps (7e-6).
-// silu(g) * u rounded to fp16 lies within 0.52 fp16 ulp of the exact value for every fp16 g.
-__device__ __forceinline__ float silu_fixed(float g) {
-  float t = g * -1.4426950408889634f;
-  t = fminf(fmaxf(t, -100.0f), 100.0f);
-  const float k = rintf(t);
-  const float f = t - k;
-  float p = 0.00967604f;
-  p = __builtin_fmaf(p, f, 0.05592204f);
-  p = __builtin_fmaf(p, f, 0.24022107f);
-  p = __builtin_fmaf(p, f, 0.693121f);
-  p = __builtin_fmaf(p, f, 1.0000001f);
-  const float e = __int_as_float(__float_as_int(p) + (int)((unsigned)(int)k << 23));
-  const float d = 1.0f + e;
-  float r = __int_as_float(0x7EF31000 - __float_as_int(d));
-  r = __builtin_fmaf(r, __builtin_fmaf(-d, r, 1.0f), r);
-  r = __builtin_fmaf(r, __builtin_fmaf(-d, r, 1.0f), r);
-  return g * r;
-}
-
-__device__ __forceinline__ float round_h(float v) { return (float)(_Float16)v; }
-
-// Integer code of a value already clamped to the code range, as the low bits of a word: the addition of 1.5 * 2^23 rounds to an
-// integer by itself (to nearest, ties to even: rintf) and leaves its two's complement in the low mantissa bits.  push_code<BITS>
-// shifts a word of codes right by BITS and puts the new code on top: after 32 / BITS pushes the first code sits in the lowest bits.
-__device__ __forceinline__ unsigned code_word(float clamped) { return __float_as_uint(clamped + 12582912.0f); }
-template <int BITS>
-__device__ __forceinline__ unsigned push_code(unsigned w, unsigned code) {
-  return __builtin_amdgcn_alignbit(code, w, BITS);
-}
-
-// v / s in fp32 for fp16-valued v and s, given r = 1.0f / s: the rounded product v * r corrected once with its exact remainder.
-// With r the correctly rounded reciprocal this is the correctly rounded quotient, i.e. bit for bit what the division instruction
-// sequence returns, for every pair of fp16 values (checked with exact integer arithmetic over all 2^20 mantissa pairs in
-// tests/test_oracle_quant.py); a row's elements share one scale, so the division proper is done once per row.
-// An infinite scale (a row that already holds an infinity) keeps the plain result: finite / inf = 0.
-struct ScaleDiv {
-  float r, s;
-  __device__ __forceinline__ explicit ScaleDiv(float scale) : r(1.0f / scale), s(__builtin_isinf(scale) ? 0.0f : scale) {}
-  __device__ __forceinline__ float operator()(float v) const {
-    const float q0 = v * r;
-    const float e = __builtin_fmaf(-s, q0, v);
-    return __builtin_fmaf(e, r, q0);
-  }
-};
-
 // Power-of-two factors of the dense stage of the non-power-of-two rotations for a row whose largest magnitude is mx (an fp16
 // value held in fp32): with mx < 2^E, to_grid = 2^(17-E) turns the row into integers of magnitude <= 2^17 and from_grid = 2^(E-17)
 // turns sums of them back.  Taken from the exponent field of mx; an all-zero row gets 1 and 1.
@@ -264,27 +213,6 @@ struct DenseGrid {
     from_grid = e_field == 0 ? 1.0f : __int_as_float(max(e_field - 16, 1) << 23);
   }
 };
-
-// Value of lane (l ^ M).  Distances 1 .. 8 stay inside a row of 16 lanes and are data-parallel-primitive moves in the vector ALU
-// (quad permutations; l ^ 4 = mirror of 8 lanes, then of 4; l ^ 8 = a rotation of the row by 8); 16 and 32 go through the LDS
-// crossbar, whose throughput is what bounds this kernel once the arithmetic is trimmed.
-template <int M>
-__device__ __forceinline__ float lane_xor(float v) {
-  int x = __float_as_int(v);
-  if constexpr (M == 1) {
-    x = __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xF, 0xF, true);   // quad_perm [1,0,3,2]
-  } else if constexpr (M == 2) {
-    x = __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xF, 0xF, true);   // quad_perm [2,3,0,1]
-  } else if constexpr (M == 4) {
-    x = __builtin_amdgcn_update_dpp(0, x, 0x141, 0xF, 0xF, true);  // row_half_mirror: l ^ 7
-    x = __builtin_amdgcn_update_dpp(0, x, 0x1B, 0xF, 0xF, true);   // quad_perm [3,2,1,0]: l ^ 3
-  } else if constexpr (M == 8) {
-    x = __builtin_amdgcn_update_dpp(0, x, 0x128, 0xF, 0xF, true);  // row_ror:8: lane (l + 8) mod 16 = l ^ 8
-  } else {
-    return __shfl_xor(v, M);
-  }
-  return __int_as_float(x);
-}
 
 // ---- tag 4: per-token int4 codes written as bf6 fragments, the operand layout of the w4a4 tiles on the 6-bit float matrix path
 // (mxmoe_bf6_tiles.hpp).  Scale and codes are those of tag 2; only the storage differs: an expert's region holds ceil(rows / 32) row
@@ -303,22 +231,6 @@ __device__ __forceinline__ v8h bf6_chunk_codes(const float (&v)[8], const Div& d
 #pragma unroll
   for (int j = 0; j < 8; ++j) o[j] = (_Float16)rintf(fminf(fmaxf(round_h(div(v[j])), -7.0f), 7.0f));
   return o;
-}
-
-// ---- tag 5: per-token fp8 (OCP e4m3) codes for the kernels whose w8a8 tiles run the fp8 matrix instruction.  scale = max|x| / 448
-// (the largest e4m3 number) in fp16 like the integer scales; code = e4m3(clamp(fp16(x / scale), +-448)), round to nearest even; rows
-// are stored like int8 rows, one byte per value.
-template <class Div>
-__device__ __forceinline__ uint2 fp8_chunk_codes(const float (&v)[8], const Div& div) {
-  float r[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) r[j] = fminf(fmaxf(round_h(div(v[j])), -448.0f), 448.0f);
-  int lo = 0, hi = 0;
-  lo = __builtin_amdgcn_cvt_pk_fp8_f32(r[0], r[1], lo, false);
-  lo = __builtin_amdgcn_cvt_pk_fp8_f32(r[2], r[3], lo, true);
-  hi = __builtin_amdgcn_cvt_pk_fp8_f32(r[4], r[5], hi, false);
-  hi = __builtin_amdgcn_cvt_pk_fp8_f32(r[6], r[7], hi, true);
-  return make_uint2((unsigned)lo, (unsigned)hi);
 }
 
 // Codes of one row in LDS (fp16; value k at byte (k / row_elems) * pitch + (k % row_elems) * 2) -> the row's place in its expert's
@@ -392,6 +304,7 @@ __global__ void __launch_bounds__(NT) row_quant_kernel(const RowArgs a) {
     m.exists = row_exists(a, row);
     m.e = m.shared_row ? a.E : (m.exists ? a.dst_exp[row] : 0);
     m.tag = (int)a.table[m.e];
+    m.exists = m.exists && !row_stays(a, m.tag);
     m.start_row = a.table[a.Et + m.e];
     m.inp_off = a.table[2 * a.Et + m.e];
     m.scale_off = a.table[3 * a.Et + m.e];
@@ -399,7 +312,7 @@ __global__ void __launch_bounds__(NT) row_quant_kernel(const RowArgs a) {
     if (SILU) {
       m.srow = m.shared_row ? src_shared + (long)(row - a.R) * 2 * n : a.src + (long)row * 2 * n;
     } else {
-      m.srow = (m.shared_row ? src_shared : a.src) + (m.shared_row ? (long)(row - a.R) : (m.exists ? (long)a.perm[row] : 0l)) * n;
+      m.srow = (m.shared_row ? src_shared : a.src) + (m.shared_row ? (long)(row - a.R) : (m.exists ? source_row(a, row) : 0l)) * n;
     }
     return m;
   };
@@ -488,12 +401,11 @@ __global__ void __launch_bounds__(NT) row_quant_kernel(const RowArgs a) {
         const int hc = h >> 3;
         if (hc < 64) {
           // the partner chunk c ^ hc sits in the same wave, hc lanes away (NT is a multiple of 64): exchange in registers
-          const float sgn = (tid & hc) ? -1.0f : 1.0f;
           auto stage = [&](auto mc) {
 #pragma unroll
             for (int i = 0; i < MAXC; ++i)
 #pragma unroll
-              for (int j = 0; j < 8; ++j) v[i][j] = __builtin_fmaf(sgn, v[i][j], lane_xor<decltype(mc)::value>(v[i][j]));
+              for (int j = 0; j < 8; j += 2) lane_butterfly<decltype(mc)::value>(v[i][j], v[i][j + 1], tid);
           };
           switch (hc) {
             case 1: stage(std::integral_constant<int, 1>{}); break;
@@ -553,8 +465,7 @@ __global__ void __launch_bounds__(NT) row_quant_kernel(const RowArgs a) {
             for (int j = 0; j < 8; ++j) mx = fmaxf(mx, fabsf(v[i][j]));
           }
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+        mx = wave_max(mx);
         if ((tid & 63) == 0) red[tid >> 6] = mx;
         __syncthreads();
         mx = red[0];
@@ -656,8 +567,7 @@ __global__ void __launch_bounds__(NT) row_quant_kernel(const RowArgs a) {
 #pragma unroll
           for (int j = 0; j < 8; ++j) gmax = fmaxf(gmax, fabsf(v[i][j]));
         }
-#pragma unroll
-        for (int o = 8; o > 0; o >>= 1) gmax = fmaxf(gmax, __shfl_xor(gmax, o));
+        gmax = row16_max(gmax);
         float scale = round_h(gmax / 7.0f);
         if (scale == 0.0f) scale = 1.0f;
         const ScaleDiv div(scale);
@@ -683,8 +593,7 @@ __global__ void __launch_bounds__(NT) row_quant_kernel(const RowArgs a) {
         for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[i][j]));
       }
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
+    amax = wave_max(amax);
     __syncthreads();
     if ((tid & 63) == 0) red[tid >> 6] = amax;
     __syncthreads();
@@ -741,56 +650,6 @@ __global__ void __launch_bounds__(NT) row_quant_kernel(const RowArgs a) {
   }
 }
 
-// H_n x * scale for a row of n = 512 * NI values held by one wave (lane l: the NI chunks l + 64 i of 8 values), every level rounded
-// to fp32 in ascending order of stride and the scaled result rounded to fp16: strides 1, 2, 4 inside a chunk, 8 .. 256 across
-// lanes, 512 and up across the chunks of a lane.
-template <int NI>
-__device__ __forceinline__ void wave_rotate(float (&v)[NI][8], int lane, float scale) {
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int h = 1; h < 8; h <<= 1)
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (!(j & h)) {
-          const float p = v[i][j], q = v[i][j + h];
-          v[i][j] = p + q;
-          v[i][j + h] = p - q;
-        }
-  auto lane_stage = [&](auto mc) {
-    constexpr int m = decltype(mc)::value;
-    // upper half of a pair: other - own, lower half: own + other; one fused multiply-add with own's sign, which rounds once
-    // exactly like the sum / difference (the product with +-1 is exact)
-    const float sgn = (lane & m) ? -1.0f : 1.0f;
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[i][j] = __builtin_fmaf(sgn, v[i][j], lane_xor<m>(v[i][j]));
-  };
-  lane_stage(std::integral_constant<int, 1>{});
-  lane_stage(std::integral_constant<int, 2>{});
-  lane_stage(std::integral_constant<int, 4>{});
-  lane_stage(std::integral_constant<int, 8>{});
-  lane_stage(std::integral_constant<int, 16>{});
-  lane_stage(std::integral_constant<int, 32>{});
-#pragma unroll
-  for (int hi = 1; hi < NI; hi <<= 1)
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-      if (!(i & hi)) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float p = v[i][j], q = v[i + hi][j];
-          v[i][j] = p + q;
-          v[i + hi][j] = p - q;
-        }
-      }
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[i][j] = round_h(keep_f32(v[i][j] * scale));
-}
-
 // One row per WAVE, for rows whose rotation is a pure Sylvester transform (n = 512 * NI, NI a power of two): lane l holds the NI
 // 8-element chunks l + 64*i.  The butterfly strides map to three levels, taken in the same ascending order as everywhere else:
 // 1, 2, 4 inside a chunk (registers), 8 .. 256 across the lanes (cross-lane exchange, no LDS staging, no barrier),
@@ -808,6 +667,7 @@ __global__ void __launch_bounds__(256) row_quant_wave_kernel(const RowArgs a) {
     const bool shared_row = row >= a.R;
     const int e = shared_row ? a.E : a.dst_exp[row];
     const int tag = (int)a.table[e];
+    if (row_stays(a, tag)) continue;
     const long lrow = shared_row ? row - a.R : row - a.table[a.Et + e];
     const long inp_off = a.table[2 * a.Et + e];
     const long scale_off = a.table[3 * a.Et + e];
@@ -816,7 +676,7 @@ __global__ void __launch_bounds__(256) row_quant_wave_kernel(const RowArgs a) {
     if (SILU) {
       srow = shared_row ? src_shared + (long)(row - a.R) * 2 * n : a.src + (long)row * 2 * n;
     } else {
-      srow = (shared_row ? src_shared : a.src) + (shared_row ? (long)(row - a.R) : (long)a.perm[row]) * n;
+      srow = (shared_row ? src_shared : a.src) + (shared_row ? (long)(row - a.R) : source_row(a, row)) * n;
     }
     float v[NI][8];
 #pragma unroll
@@ -857,8 +717,7 @@ __global__ void __launch_bounds__(256) row_quant_wave_kernel(const RowArgs a) {
         float gmax = 0.0f;
 #pragma unroll
         for (int j = 0; j < 8; ++j) gmax = fmaxf(gmax, fabsf(v[i][j]));
-#pragma unroll
-        for (int o = 8; o > 0; o >>= 1) gmax = fmaxf(gmax, __shfl_xor(gmax, o));
+        gmax = row16_max(gmax);
         float scale = round_h(gmax / 7.0f);
         if (scale == 0.0f) scale = 1.0f;
         const ScaleDiv div(scale);
@@ -878,8 +737,7 @@ __global__ void __launch_bounds__(256) row_quant_wave_kernel(const RowArgs a) {
     for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[i][j]));
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
+    amax = wave_max(amax);
     const float upper = tag == 1 ? 127.0f : (EXT && tag == 5 ? 448.0f : 7.0f);
     float scale = round_h(amax / upper);   // fp16 division: fp32 quotient of two fp16 values, rounded to fp16
     if (scale == 0.0f) scale = 1.0f;       // quantize.cuh:258
@@ -1011,8 +869,7 @@ __global__ void __launch_bounds__(256) token_quant_wave_kernel(const TokenArgs a
         float gmax = 0.0f;
 #pragma unroll
         for (int j = 0; j < 8; ++j) gmax = fmaxf(gmax, fabsf(v[i][j]));
-#pragma unroll
-        for (int o = 8; o > 0; o >>= 1) gmax = fmaxf(gmax, __shfl_xor(gmax, o));
+        gmax = row16_max(gmax);
         float scale = round_h(gmax / 7.0f);
         if (scale == 0.0f) scale = 1.0f;
         const ScaleDiv div(scale);
@@ -1044,8 +901,7 @@ __global__ void __launch_bounds__(256) token_quant_wave_kernel(const TokenArgs a
     for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[i][j]));
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
+    amax = wave_max(amax);
     if (present & 0x2u) {  // tag 1: int8 per token
       float scale = round_h(amax / 127.0f);  // fp16 division: fp32 quotient of two fp16 values, rounded to fp16
       if (scale == 0.0f) scale = 1.0f;       // quantize.cuh:258
@@ -1151,13 +1007,14 @@ __global__ void __launch_bounds__(256) row_quant_dense_kernel(const RowArgs a) {
     m.exists = row < routed || shared_row;
     const int e = shared_row ? a.E : (m.exists ? const_load(a.dst_exp + row) : 0);
     m.tag = (int)const_load(a.table + e);
+    m.exists = m.exists && !row_stays(a, m.tag);
     m.lrow = shared_row ? row - a.R : row - const_load(a.table + a.Et + e);
     m.inp_off = const_load(a.table + 2 * a.Et + e);
     m.scale_off = const_load(a.table + 3 * a.Et + e);
     if (SILU) {
       m.srow = shared_row ? src_shared + (long)(row - a.R) * 2 * n : a.src + (long)row * 2 * n;
     } else {
-      m.srow = (shared_row ? src_shared : a.src) + (shared_row ? (long)(row - a.R) : (m.exists ? (long)const_load(a.perm + row) : 0l)) * n;
+      m.srow = (shared_row ? src_shared : a.src) + (shared_row ? (long)(row - a.R) : (m.exists ? source_row(a, row) : 0l)) * n;
     }
     return m;
   };
@@ -1230,8 +1087,7 @@ __global__ void __launch_bounds__(256) row_quant_dense_kernel(const RowArgs a) {
           mx = fmaxf(mx, fabsf(v[i][j]));
         }
       }
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+      mx = wave_max(mx);
       const DenseGrid grid(mx);
       const float to16 = grid.to_grid * 0.0625f;  // exact (a power of two well inside the range); rint(v * to_grid) / 16 below
       // transposed write: chunk c = blk * kb + b' -> columns blk * 8 + j, position b'
@@ -1361,8 +1217,7 @@ __global__ void __launch_bounds__(256) row_quant_dense_kernel(const RowArgs a) {
         float gmax = 0.0f;
 #pragma unroll
         for (int j = 0; j < 8; ++j) gmax = fmaxf(gmax, fabsf(v[i][j]));
-#pragma unroll
-        for (int o = 8; o > 0; o >>= 1) gmax = fmaxf(gmax, __shfl_xor(gmax, o));
+        gmax = row16_max(gmax);
         float scale = round_h(gmax / 7.0f);
         if (scale == 0.0f) scale = 1.0f;
         const ScaleDiv div(scale);
@@ -1384,8 +1239,7 @@ __global__ void __launch_bounds__(256) row_quant_dense_kernel(const RowArgs a) {
     for (int i = 0; i < MAXC; ++i)
 #pragma unroll
       for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[i][j]));  // chunks past the row hold zeros
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
+    amax = wave_max(amax);
     const float upper = tag == 1 ? 127.0f : (EXT && tag == 5 ? 448.0f : 7.0f);
     float scale = round_h(amax / upper);   // fp16 division: fp32 quotient of two fp16 values, rounded to fp16
     if (scale == 0.0f) scale = 1.0f;       // quantize.cuh:258
@@ -1480,6 +1334,7 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
     const bool shared_row = row >= a.R;
     const int e = shared_row ? a.E : a.dst_exp[row];
     const int tag = (int)a.table[e];
+    if (row_stays(a, tag)) continue;
     const long lrow = shared_row ? row - a.R : row - a.table[a.Et + e];
     const long inp_off = a.table[2 * a.Et + e];
     const long scale_off = a.table[3 * a.Et + e];
@@ -1488,7 +1343,7 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
     if (SILU) {
       srow = shared_row ? src_shared + (long)(row - a.R) * 2 * n : a.src + (long)row * 2 * n;
     } else {
-      srow = (shared_row ? src_shared : a.src) + (shared_row ? (long)(row - a.R) : (long)a.perm[row]) * n;
+      srow = (shared_row ? src_shared : a.src) + (shared_row ? (long)(row - a.R) : source_row(a, row)) * n;
     }
     // A k row past kb (the last of a wave's four when kb is not a multiple of 8: waves 4 .. 7 of a 28-row view) costs nothing: the
     // whole wave skips its loads, its SiLU and its butterflies, and the slot holds zeros.
@@ -1532,10 +1387,8 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
               v[i][j + h] = p - q;
             }
         auto lane_stage = [&](auto mc) {
-          constexpr int m = decltype(mc)::value;
-          const float sgn = (lane & m) ? -1.0f : 1.0f;
 #pragma unroll
-          for (int j = 0; j < 8; ++j) v[i][j] = __builtin_fmaf(sgn, v[i][j], lane_xor<m>(v[i][j]));
+          for (int j = 0; j < 8; j += 2) lane_butterfly<decltype(mc)::value>(v[i][j], v[i][j + 1], lane);
         };
         lane_stage(std::integral_constant<int, 1>{});
         lane_stage(std::integral_constant<int, 2>{});
@@ -1549,8 +1402,7 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
           mx = fmaxf(mx, fabsf(v[i][j]));
         }
       }
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+      mx = wave_max(mx);
       if (lane == 0) red[wave] = mx;
       __syncthreads();  // (also: the previous row's readers of xt / yrow are done)
       mx = red[0];
@@ -1625,8 +1477,7 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
         float gmax = 0.0f;
 #pragma unroll
         for (int j = 0; j < 8; ++j) gmax = fmaxf(gmax, fabsf(v[i][j]));
-#pragma unroll
-        for (int o = 8; o > 0; o >>= 1) gmax = fmaxf(gmax, __shfl_xor(gmax, o));
+        gmax = row16_max(gmax);
         float scale = round_h(gmax / 7.0f);
         if (scale == 0.0f) scale = 1.0f;
         const ScaleDiv div(scale);
@@ -1646,8 +1497,7 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
     for (int i = 0; i < MAXC; ++i)
 #pragma unroll
       for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[i][j]));
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
+    amax = wave_max(amax);
     if (lane == 0) red[8 + wave] = amax;
     __syncthreads();
     amax = red[8];
@@ -1705,6 +1555,8 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
   }
 }
 
+constexpr int kSplitSharedRows = 512;
+
 static int make_plan(int n, int had_k, int had_f, bool rotate, RotPlan* p) {
   p->n = n;
   p->scale = 1.0f / sqrtf((float)n);
@@ -1723,6 +1575,18 @@ static int make_plan(int n, int had_k, int had_f, bool rotate, RotPlan* p) {
 
 template <bool SILU, bool EXT>
 static int launch_rows_as(const RowArgs& a, int lds_bytes, hipStream_t s) {
+  // Shared rows of another length keep the routed rows out of the kernels made for one length: from some hundred rows on, two launches
+  // with the best kernel for each cost less than one with the kernel that takes any mixture.
+  if (a.plan_shared.n != a.plan.n && a.R >= kSplitSharedRows && a.rows > a.R) {
+    RowArgs routed = a, shared = a;
+    routed.rows = a.R;
+    routed.plan_shared = a.plan;
+    shared.R = 0;
+    shared.rows = a.rows - a.R;
+    shared.plan = a.plan_shared;
+    const int rc = launch_rows_as<SILU, EXT>(routed, lds_bytes, s);
+    return rc ? rc : launch_rows_as<SILU, EXT>(shared, lds_bytes, s);
+  }
   const int nmax = a.plan.n > a.plan_shared.n ? a.plan.n : a.plan_shared.n;
   int dev = 0, cus = 256;
   (void)hipGetDevice(&dev);
@@ -2235,6 +2099,34 @@ int mxmoe_silu_mul_quant_planned(const void* gate_up, const void* d_plan_gate_up
   const int lds = (nmax + a.plan.kb * a.plan.kb + 16) * (int)sizeof(float);
   return launch_rows<true>(a, lds, (hipStream_t)stream, variants);
 }
+
+}  // extern "C"
+namespace mxmoe {
+int quant_rows_behind(const RowsBehind& b, hipStream_t stream) {
+  const int et = b.num_experts + (b.has_shared ? 1 : 0);
+  const PlanLayout lay(et);
+  RowArgs a{};
+  a.src = reinterpret_cast<const _Float16*>(b.rows);
+  a.shared_src_addr = b.has_shared ? reinterpret_cast<const int64_t*>(b.plan_gate_up + lay.misc) + 1 : nullptr;
+  a.inp_store = b.inp_store;
+  a.scale_store = b.scale_store;
+  a.dst_exp = b.dst_exp;
+  a.table = reinterpret_cast<const int64_t*>(b.plan_down + lay.table);
+  a.routed_ptr = reinterpret_cast<const int64_t*>(b.plan_down + lay.misc);
+  a.R = b.rows_capacity;
+  a.T = b.num_tokens;
+  a.E = b.num_experts;
+  a.Et = et;
+  a.rows = b.rows_capacity + (b.has_shared ? b.num_tokens : 0);
+  a.rotate = b.rotate;
+  a.direct = b.rotate != 2;
+  if (const int rc = fill_common(a, b.n, b.has_shared ? b.n_shared : b.n, b.rotate ? b.had_k : 1, b.rotate ? b.had_f : 1, b.had_signs)) return rc;
+  const int nmax = b.n > a.plan_shared.n ? b.n : a.plan_shared.n;
+  const int lds = (nmax + a.plan.kb * a.plan.kb + 16) * (int)sizeof(float);
+  return launch_rows<false>(a, lds, stream, b.variants);
+}
+}  // namespace mxmoe
+extern "C" {
 
 size_t mxmoe_combine_workspace_bytes(int num_tokens, int topk) { return (size_t)num_tokens * topk * sizeof(int32_t); }
 

@@ -75,7 +75,9 @@ struct Bf6Tile {
   static constexpr int kWavesWanted = 2;  // waves per SIMD a kernel of such tiles is compiled for
   static constexpr int kABits = 6, kWBits = 6;       // bits per activation / weight element as stored
 
+  template <bool GU>
   __device__ static __forceinline__ void run(const TileArgs& t, uint8_t* __restrict__ smem) {
+    static_assert(!GU, "bf6 fragments hold an expert's rows in blocks of 32: no gather, so no gate_up form");
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int M = t.M, N = t.N;

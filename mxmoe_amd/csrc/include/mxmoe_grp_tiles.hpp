@@ -32,17 +32,22 @@ struct WxAxGTile {
   static constexpr int kPieces = BM / 16;                       // 1 KB pieces (16 rows) of one activation slice
   static constexpr int kQ = (kPieces + kWaves - 1) / kWaves;    // pieces a wave copies per slice
 
+  template <bool GU>
   __device__ static __forceinline__ void run(const TileArgs& t, uint8_t* __restrict__ smem) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int M = t.M, N = t.N;
+    const int M = t.M, N = GU ? t.N / 2 : t.N;  // N: output channels (gate_up form: block 0 of a wave = gate, block 1 = up channels)
     const int G = t.K / 128;  // K slices = quantisation groups
     const long row_bytes = t.K / 2;
-    const int m0 = t.row0 + t.tile_m * BM, n0 = t.tile_n * BN;
+    const int m0 = t.row0 + t.tile_m * BM, n0 = t.tile_n * (GU ? BN / 2 : BN);
     const int lrow = lane & 31, nq = (lane >> 5) * 4;
 
     // ---- activations: global -> registers -> LDS ----
+    auto row_of = [&](int m) {  // the stored row behind row m (clamped to the last valid one)
+      if constexpr (GU) return gload<int>(t.rows + min(m, M - 1));
+      else return min(m, M - 1);
+    };
     const uint8_t* a_src[kQ];
     int a_lds[kQ];
     bool a_mine[kQ];
@@ -51,7 +56,7 @@ struct WxAxGTile {
       const int piece = wave + kWaves * q;
       a_mine[q] = piece < kPieces;
       const int row = (a_mine[q] ? piece : 0) * 16 + (lane >> 2);
-      a_src[q] = t.A + (long)min(m0 + row, M - 1) * row_bytes + (lane & 3) * 16;
+      a_src[q] = t.A + (long)row_of(m0 + row) * row_bytes + (lane & 3) * 16;
       a_lds[q] = row * kRowBytes + (((lane & 3) ^ lds_swizzle(row)) << 4);
     }
     auto a_gload = [&](int kt, v4i (&r)[kQ]) {
@@ -73,24 +78,25 @@ struct WxAxGTile {
     const int nblk = (N + 31) / 32;
     const uint8_t* bptr[FN];
 #pragma unroll
-    for (int j = 0; j < FN; ++j) bptr[j] = t.B + (long)min(n0 / 32 + wave * FN + j, nblk - 1) * G * 2048 + lane * 16;
+    for (int j = 0; j < FN; ++j)
+      bptr[j] = t.B + (long)(GU ? min(n0 / 32 + wave, nblk - 1) + j * nblk : min(n0 / 32 + wave * FN + j, nblk - 1)) * G * 2048 + lane * 16;
     auto b_gload = [&](int j, int s, int kt) { return gload<v4i>(bptr[j] + ((long)min(kt, G - 1) * 2 + s) * 1024); };
 
     // ---- scales of one group: token scales of the lane's rows, channel scales of its 4-channel runs ----
     const _Float16* sa_ptr[FM];
 #pragma unroll
-    for (int i = 0; i < FM; ++i) sa_ptr[i] = t.sa + (long)min(m0 + i * 32 + lrow, M - 1) * G;
+    for (int i = 0; i < FM; ++i) sa_ptr[i] = t.sa + (long)row_of(m0 + i * 32 + lrow) * G;
     // channel scales: the lane's first run of 4 channels; the others sit 8 channels (16 bytes) apart and are clamped one by one
-    const int nbase = n0 + wave * 64 + nq;
+    const int nbase = n0 + wave * (GU ? 32 : 64) + nq;
     auto s_gload = [&](int kt, _Float16 (&sa_h)[FM], v4h (&sb_h)[FN][4]) {
       const int g = min(kt, G - 1);
 #pragma unroll
       for (int i = 0; i < FM; ++i) sa_h[i] = gload<_Float16>(sa_ptr[i] + g);
-      const _Float16* sbg = t.sb + (long)g * N;
+      const _Float16* sbg = t.sb + (long)g * t.N;
 #pragma unroll
       for (int j = 0; j < FN; ++j)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) sb_h[j][q] = gload<v4h>(sbg + min(nbase + j * 32 + q * 8, N - 4));
+        for (int q = 0; q < 4; ++q) sb_h[j][q] = gload<v4h>(sbg + (GU ? j * N + min(nbase + q * 8, N - 4) : min(nbase + j * 32 + q * 8, N - 4)));
     };
 
     v16f facc[FM][FN];
@@ -185,16 +191,19 @@ struct WxAxGTile {
     for (int i = 0; i < FM; ++i) {
       const int m = m0 + i * 32 + lrow;
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
+      for (int j = 0; j < (GU ? 1 : FN); ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int n = n0 + wave * 64 + j * 32 + q * 8 + nq;
+          const int n = n0 + wave * (GU ? 32 : 64) + j * 32 + q * 8 + nq;
           if (m < M && n < N) {
             v4h o;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = (_Float16)facc[i][j][q * 4 + e];
+            for (int e = 0; e < 4; ++e) {
+              if constexpr (GU) o[e] = silu_mul_half((_Float16)facc[i][0][q * 4 + e], (_Float16)facc[i][1][q * 4 + e]);
+              else o[e] = (_Float16)facc[i][j][q * 4 + e];
+            }
             gstore(t.C + (long)m * N + n, o);
-            if (t.acc_dump) {  // parity tests only: the fp32 sums as bit patterns
+            if (!GU && t.acc_dump) {  // parity tests only: the fp32 sums as bit patterns
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
                 const float f = facc[i][j][q * 4 + e];  // a copy: a bit cast applied to a vector element reads element 0

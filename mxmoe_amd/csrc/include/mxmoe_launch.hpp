@@ -61,6 +61,7 @@ struct FusedArgs {
     int first, row0, rows, problem_branch;
   };
   Entry entry[kMaxEntries];
+  const int32_t* const* rows;  // gate_up form (see TileArgs): per problem, the activation row behind each of its rows
 };
 static_assert(sizeof(FusedArgs) <= 4096, "kernel arguments are limited to 4 KB");
 
@@ -69,14 +70,14 @@ static_assert(sizeof(FusedArgs) <= 4096, "kernel arguments are limited to 4 KB")
 #define MXMOE_GROUP_BYTES (2 << 20)
 #endif
 
-template <int I, class... Tiles>
+template <int I, bool GU, class... Tiles>
 struct Dispatch;
-template <int I>
-struct Dispatch<I> {
+template <int I, bool GU>
+struct Dispatch<I, GU> {
   __device__ static __forceinline__ void go(int, TileArgs&, int, uint8_t*) {}
 };
-template <int I, class T, class... Rest>
-struct Dispatch<I, T, Rest...> {
+template <int I, bool GU, class T, class... Rest>
+struct Dispatch<I, GU, T, Rest...> {
   __device__ static __forceinline__ void go(int branch, TileArgs& t, int local, uint8_t* smem) {
     if (branch == I) {
       // local index -> (row tile, column tile) as tile_scheduler.cuh:40-49, but row tile fastest: neighbouring workgroups then share
@@ -103,9 +104,9 @@ struct Dispatch<I, T, Rest...> {
       const int rows_g = min(rg, grid_m - g * rg);
       t.tile_n = r / rows_g;
       t.tile_m = g * rg + (r - t.tile_n * rows_g);
-      T::run(t, smem);
+      T::template run<GU>(t, smem);
     } else {
-      Dispatch<I + 1, Rest...>::go(branch, t, local, smem);
+      Dispatch<I + 1, GU, Rest...>::go(branch, t, local, smem);
     }
   }
 };
@@ -156,7 +157,7 @@ __host__ __device__ __forceinline__ int tile_of_workgroup(ArgsPtr args, int wg) 
   return pt < ntiles ? tile0 + pt : -1;
 }
 
-template <class ArgsPtr, class... Tiles>
+template <bool GU, class ArgsPtr, class... Tiles>
 __device__ __forceinline__ void fused_body(ArgsPtr args, uint8_t* smem) {
   const int tile = tile_of_workgroup(args, (int)blockIdx.x);
   if (tile < 0) return;
@@ -189,22 +190,25 @@ __device__ __forceinline__ void fused_body(ArgsPtr args, uint8_t* smem) {
   t.N = uni((int)cload(&sizes[gp].y));
   t.K = uni((int)cload(&sizes[gp].z));
   t.tile_m = t.tile_n = 0;
-  Dispatch<0, Tiles...>::go(en_pb >> 16, t, local, smem);
+  t.rows = nullptr;
+  if constexpr (GU) t.rows = cload(args->rows + gp);
+  Dispatch<0, GU, Tiles...>::go(en_pb >> 16, t, local, smem);
 }
 
 template <class... Tiles>
 __global__ void __launch_bounds__(kThreads, kWavesPerSimd<Tiles...>) fused_group_gemm_kernel(const FusedArgs args) {
   extern __shared__ __align__(16) uint8_t smem[];
-  fused_body<const FusedArgs*, Tiles...>(&args, smem);
+  fused_body<false, const FusedArgs*, Tiles...>(&args, smem);
 }
 
 // The same kernel with its tables in device memory, where a planning kernel wrote them from the tokens-per-expert counts: the
 // host then needs no copy of the counts, so a layer forward neither synchronises nor depends on its routing when it is enqueued
 // (or captured into a graph).  The grid is sized for the worst case; workgroups past the planned tiles leave at once.
-template <class... Tiles>
+// GU: the tiles' gate_up form (TileArgs::rows).
+template <bool GU, class... Tiles>
 __global__ void __launch_bounds__(kThreads, kWavesPerSimd<Tiles...>) fused_group_gemm_planned_kernel(const FusedArgs* __restrict__ args) {
   extern __shared__ __align__(16) uint8_t smem[];
-  fused_body<const MXMOE_CONST FusedArgs*, Tiles...>((const MXMOE_CONST FusedArgs*)args, smem);
+  fused_body<GU, const MXMOE_CONST FusedArgs*, Tiles...>((const MXMOE_CONST FusedArgs*)args, smem);
 }
 
 // ------------------------------------------------------------------ host side ------------------------------------------------------------------
@@ -317,6 +321,7 @@ struct FusedKernel {
   Policy policy;
   mxmoe_func_t func;  // the kernel as a function of the reference's FuncType (registry.cuh:28-39)
   LaunchPlannedFn launch_planned;  // the same kernel reading its tables from device memory (device-side planning)
+  LaunchPlannedFn launch_gate_up;  // ... with its tiles in their gate_up form; null for kernels that are not a layer's
   int plan_index;                  // index into plan_infos()
   // Largest row count per problem this kernel is meant for, 0 = any.  A kernel with a limit is preferred by the automatic choice when
   // every problem of the list stays within it (the few-token kernels: same results, more workgroups per CU).
@@ -510,19 +515,19 @@ hipError_t launch_fused(const FusedArgs& a, int grid, int lds, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <class... Tiles>
+template <bool GU, class... Tiles>
 hipError_t launch_fused_planned(const FusedArgs* d_args, int grid, int lds, hipStream_t s) {
   static bool lds_opted_in[64] = {};
   if (lds > 64 * 1024) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return hipGetLastError();
     if (dev >= 0 && dev < 64 && !lds_opted_in[dev]) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&fused_group_gemm_planned_kernel<Tiles...>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&fused_group_gemm_planned_kernel<GU, Tiles...>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
       if (e != hipSuccess) return e;
       lds_opted_in[dev] = true;
     }
   }
-  hipLaunchKernelGGL((fused_group_gemm_planned_kernel<Tiles...>), dim3(grid), dim3(kThreads), lds, s, d_args);
+  hipLaunchKernelGGL((fused_group_gemm_planned_kernel<GU, Tiles...>), dim3(grid), dim3(kThreads), lds, s, d_args);
   return hipGetLastError();
 }
 
@@ -569,7 +574,7 @@ struct FuncThunk {
 };
 
 template <class... Tiles>
-int register_fused(const char* fn_name, Policy policy = Policy::Fused, int max_rows_hint = 0) {
+int register_fused(const char* fn_name, Policy policy = Policy::Fused, int max_rows_hint = 0, LaunchPlannedFn launch_gate_up = nullptr) {
   static_assert(sizeof...(Tiles) <= kMaxBranches, "the planners' branch table holds kMaxBranches tile shapes per kernel");
   FusedKernel k;
   k.policy = policy;
@@ -587,7 +592,8 @@ int register_fused(const char* fn_name, Policy policy = Policy::Fused, int max_r
   }
   k.name = n + fn_name;
   k.launch = &launch_fused<Tiles...>;
-  k.launch_planned = &launch_fused_planned<Tiles...>;
+  k.launch_planned = &launch_fused_planned<false, Tiles...>;
+  k.launch_gate_up = launch_gate_up;
   k.plan_index = (int)plan_infos().size();
   plan_infos().push_back(make_plan_info(k.branches));
   const int id = (int)registry().size();
@@ -598,6 +604,12 @@ int register_fused(const char* fn_name, Policy policy = Policy::Fused, int max_r
   }
   registry().push_back(k);
   return id;
+}
+
+// A kernel that a layer's first block may run on: its tiles in both forms.
+template <class... Tiles>
+int register_layer_kernel(const char* fn_name, Policy policy, int max_rows_hint = 0) {
+  return register_fused<Tiles...>(fn_name, policy, max_rows_hint, &launch_fused_planned<true, Tiles...>);
 }
 
 // Operand variant (BranchInfo::variant) of the kernel's tiles for format `f`, 0 when it has none or the plain ones.

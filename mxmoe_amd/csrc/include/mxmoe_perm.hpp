@@ -18,14 +18,39 @@ __device__ __forceinline__ uint64_t match_same(int e, int nbits) {
   return m;
 }
 
-// inclusive scan of one value per lane across the wave
-__device__ __forceinline__ int wave_inclusive_scan(int v, int lane) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int t = __shfl_up(v, o);
-    if (lane >= o) v += t;
-  }
+// Inclusive scan of one value per lane across the wave, by data-parallel-primitive moves (row shifts of 1, 2, 4, 8, then the last lane of
+// a row of 16 broadcast into the next rows): the six dependent steps stay in the vector ALU, where a lane shuffle through the LDS
+// crossbar costs an LDS round trip each.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_or_zero(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false); }
+__device__ __forceinline__ int wave_inclusive_scan(int v) {
+  v += dpp_or_zero<0x111, 0xF>(v);
+  v += dpp_or_zero<0x112, 0xF>(v);
+  v += dpp_or_zero<0x114, 0xF>(v);
+  v += dpp_or_zero<0x118, 0xF>(v);
+  v += dpp_or_zero<0x142, 0xA>(v);
+  v += dpp_or_zero<0x143, 0xC>(v);
   return v;
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ long dpp_or_zero(long v) {
+  const unsigned lo = (unsigned)dpp_or_zero<CTRL, ROWS>((int)v), hi = (unsigned)dpp_or_zero<CTRL, ROWS>((int)((unsigned long)v >> 32));
+  return (long)(((unsigned long)hi << 32) | lo);
+}
+__device__ __forceinline__ long wave_inclusive_scan(long v) {
+  v += dpp_or_zero<0x111, 0xF>(v);
+  v += dpp_or_zero<0x112, 0xF>(v);
+  v += dpp_or_zero<0x114, 0xF>(v);
+  v += dpp_or_zero<0x118, 0xF>(v);
+  v += dpp_or_zero<0x142, 0xA>(v);
+  v += dpp_or_zero<0x143, 0xC>(v);
+  return v;
+}
+// value of the wave's last lane, as a scalar
+__device__ __forceinline__ int wave_last(int v) { return __builtin_amdgcn_readlane(v, 63); }
+__device__ __forceinline__ long wave_last(long v) {
+  const unsigned lo = (unsigned)wave_last((int)v), hi = (unsigned)wave_last((int)((unsigned long)v >> 32));
+  return (long)(((unsigned long)hi << 32) | lo);
 }
 
 // Stable permutation by expert of at most kPermChunk (token, slot) entries by the first wave of a workgroup: count, scan the experts,
@@ -49,12 +74,12 @@ __device__ __forceinline__ void perm_small_body(const int32_t* __restrict__ ids,
     for (int e0 = 0; e0 < E; e0 += 64) {
       const int e = e0 + lane;
       const int v = e < E ? run[e] : 0;
-      const int inc = wave_inclusive_scan(v, lane);
+      const int inc = wave_inclusive_scan(v);
       if (e < E) {
         recv[e] = v;
         run[e] = carry + inc - v;
       }
-      carry += __shfl(inc, 63);
+      carry += wave_last(inc);
     }
   }
   __syncthreads();
@@ -128,9 +153,9 @@ __device__ __forceinline__ void perm_scatter_body(const int32_t* __restrict__ id
           before = hist[block * E + e];
         }
       }
-      const int inc = wave_inclusive_scan(v, lane);
+      const int inc = wave_inclusive_scan(v);
       if (e < E) run[e] = carry + inc - v + before;
-      carry += __shfl(inc, 63);
+      carry += wave_last(inc);
     }
   }
   __syncthreads();

@@ -1,0 +1,327 @@
+// The planner: from tokens-per-expert counts to the tables of one fused launch, by one workgroup in device memory.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "../../../include/mxmoe_amd.h"
+#include "mxmoe_launch.hpp"
+#include "mxmoe_perm.hpp"
+#include "mxmoe_plan.hpp"
+
+namespace mxmoe {
+
+// A block descriptor (not the QParams arrays of the launcher, whose padding bytes belong to the caller) may name an operand variant
+// in q._pad[0]: 1 = the int4 codes of per-token activations as bf6 fragments (for the kernels whose w4a4 tiles run on the 6-bit float
+// matrix path), 2 = per-token fp8 e4m3 codes instead of int8 ones (for the kernels whose w8a8 tiles run the fp8 instruction).
+__host__ __device__ inline bool wants_bf6(const mxmoe_qparams& q) { return q._pad[0] == 1 && q.a_bits == 4 && q.w_bits == 4 && q.gsize == -1; }
+__host__ __device__ inline bool wants_fp8(const mxmoe_qparams& q) { return q._pad[0] == 2 && q.a_bits == 8 && q.w_bits == 8 && q.gsize == -1; }
+
+__host__ __device__ inline int act_tag_of(const mxmoe_qparams& q) {  // ref_bind.cu:461-473
+  if (q.a_bits >= 16) return 0;
+  if (wants_fp8(q)) return 5;
+  if (q.a_bits == 8 && q.gsize == -1) return 1;
+  if (wants_bf6(q)) return 4;
+  if (q.a_bits == 4 && q.gsize == -1) return 2;
+  if (q.a_bits == 4 && q.gsize == 128) return 3;
+  return -1;
+}
+
+__host__ __device__ inline int fmt_of(const mxmoe_qparams& q) { return (int)classify(q); }
+
+constexpr int kNumTags = 6;
+
+// How a block's operands are laid out.
+//   kPlain    activations as rows sorted by expert, the output as the GEMM's [rows, N] (the operators' layout);
+//   kGateUp   the gate_up form of the tiles (TileArgs): activations are one store per tag that holds every token once, each problem
+//             reads them through its part of `token_of_row` (the shared expert through `iota`), the output is [rows, N / 2];
+//   kBehind   the block behind a gate_up form: as kPlain, but fp16 activations are read where that form left them (`act`).
+struct LayerForm {
+  enum Kind { kPlain = 0, kGateUp = 1, kBehind = 2 };
+  int kind;
+  const uint8_t* store[kNumTags];
+  const uint8_t* scales[kNumTags];
+  const int32_t* token_of_row;
+  const int32_t* iota;
+  const uint8_t* act;
+};
+
+struct PlanParams {
+  const int64_t* recv;
+  const mxmoe_block_desc* desc;
+  const uint8_t* inp;
+  const uint8_t* scale;
+  uint8_t* out;
+  uint8_t* plan;
+  int E, Et, shared_rows;
+  LayerForm form;
+  PlanInfo info;
+};
+
+constexpr int kPlanThreads = 128;
+constexpr int kMaxPlannedProblems = 4096;  // experts of a planned block (run as launches of kMaxProblems experts each)
+static_assert(kMaxProblems <= kPlanThreads, "one thread per problem");
+static_assert(kMaxBranches <= 64, "one lane per branch");
+
+struct PlanPair {
+  PlanParams p[2];
+  int chunks;  // launches per block
+};
+
+// One workgroup of two waves per launch, thread e = expert e0 + e of the launch's chunk of experts [e0, e0 + kMaxProblems) (the shared
+// expert, if any, is expert E with `shared_rows` rows).  Everything the host launcher computes (launch_range), with the same
+// functions and in the same order, so the two produce identical tables; prefix sums over experts are wave scans (a later chunk
+// first sums what the experts before it occupy), and an entry finds its place from per-branch counts instead of a sequential walk.
+// A chain of dependent steps that the whole forward waits for: its scans run on lane moves in the vector ALU and the sums over the
+// branches take one lane per branch (with LDS shuffles and a serial walk over the branches the chain took 1.4 times as long).
+// `recv`: the tokens-per-expert counts (device memory, or LDS when the planning workgroup counted them itself).
+template <class Count>
+__device__ __forceinline__ void plan_block_body(const PlanParams& p, const int chunk, const int chunks, const Count* recv) {
+  const int e0 = chunk * kMaxProblems;                       // first expert of this launch
+  const int ecnt = min(kMaxProblems, p.Et - e0);             // experts of this launch
+  constexpr int kSums = 5;                           // rows, packed input, scales, output elements, fp16 input elements
+  __shared__ long s_tot[kSums][2];                   // per wave
+  __shared__ long s_base[kSums + 1][2];              // the same five, and the routed rows, summed over the experts before this launch
+  __shared__ int s_cnt[kMaxBranches][2], s_til[kMaxBranches][2];  // per run-order rank and wave: entries, tiles
+  __shared__ int s_cnt_long[kMaxBranches][2], s_til_long[kMaxBranches][2];  // ... of which belong to long-K problems
+  // the kernel's branch table, from the kernel arguments into LDS: the planning functions walk it entry by entry, and each step of
+  // such a walk through the argument segment costs a trip to the scalar cache
+  __shared__ PlanInfo info;
+  static_assert(sizeof(PlanInfo) % 4 == 0, "copied word by word");
+  for (int i = threadIdx.x; i < (int)(sizeof(PlanInfo) / 4); i += kPlanThreads) reinterpret_cast<int*>(&info)[i] = reinterpret_cast<const int*>(&p.info)[i];
+  const int e = threadIdx.x, lane = e & 63, wave = e >> 6;
+  const int ge = e0 + e;                             // this thread's expert
+  __shared__ unsigned s_used[2];                     // per wave: branches in use
+  if (e < kMaxBranches) {
+    s_cnt[e][0] = s_cnt[e][1] = s_til[e][0] = s_til[e][1] = 0;
+    s_cnt_long[e][0] = s_cnt_long[e][1] = s_til_long[e][0] = s_til_long[e][1] = 0;
+  }
+  if (e < 2) s_used[e] = 0;
+  const bool mine = e < ecnt;
+  const PlanLayout lay(p.Et);
+  FusedArgs* fa = reinterpret_cast<FusedArgs*>(p.plan + chunk * kFusedArgsStride);
+  int64_t* table = reinterpret_cast<int64_t*>(p.plan + lay.table);
+  const void** ptrs = reinterpret_cast<const void**>(p.plan + lay.ptrs);
+  int64_t* misc = reinterpret_cast<int64_t*>(p.plan + lay.misc);
+  mxmoe_dim3* sizes = reinterpret_cast<mxmoe_dim3*>(p.plan + lay.sizes);
+  const int32_t** row_maps = reinterpret_cast<const int32_t**>(p.plan + lay.rows);
+  const int kind = p.form.kind;
+
+  // what one expert occupies: rows, packed activation elements, scales, output elements, fp16 input elements (in fp16 elements but the rows)
+  auto footprint = [&](int x, long (&f)[kSums], int* tag_out, mxmoe_block_desc* d_out) {
+    const mxmoe_block_desc d = p.desc[x];
+    const long rows = x < p.E ? (long)recv[x] : (long)p.shared_rows;
+    const int tag = act_tag_of(d.q), K = (int)d.K;
+    const long qld = tag == 0 ? K : (tag == 1 || tag == 5 ? K / 2 : K / 4);  // fp16 elements per packed activation row (ref_bind.cu:491)
+    const long sld = tag == 0 ? 0 : (tag == 3 ? K / 128 : 1);                // scales per row (ref_bind.cu:492)
+    f[0] = rows;
+    // packed activations: rows of qld elements, or (tag 4) whole blocks of 32 rows of K / 64 fragments
+    f[1] = tag == 4 ? ((rows + 31) >> 5) * (long)(K >> 6) * (kBf6Frag / 2) : qld * rows;
+    f[2] = sld * rows;
+    f[3] = (long)(kind == LayerForm::kGateUp ? d.N / 2 : d.N) * rows;
+    f[4] = (long)K * rows;
+    if (tag_out) *tag_out = tag;
+    if (d_out) *d_out = d;
+  };
+  // experts before this launch (none for the first: most blocks are one launch)
+  if (e0 > 0) {
+    long base[kSums + 1] = {0, 0, 0, 0, 0, 0};
+    for (int x = e; x < e0; x += kPlanThreads) {
+      long f[kSums];
+      footprint(x, f, nullptr, nullptr);
+#pragma unroll
+      for (int i = 0; i < kSums; ++i) base[i] += f[i];
+      if (x < p.E) base[kSums] += f[0];
+    }
+#pragma unroll
+    for (int i = 0; i <= kSums; ++i) {
+      const long all = wave_last(wave_inclusive_scan(base[i]));
+      if (lane == 0) s_base[i][wave] = all;
+    }
+  } else if (lane == 0) {
+#pragma unroll
+    for (int i = 0; i <= kSums; ++i) s_base[i][wave] = 0;
+  }
+
+  long rows = 0, sld = 0;
+  long foot[kSums] = {0, 0, 0, 0, 0};
+  int tag = 0, fmt = 0, N = 0, K = 0;
+  mxmoe_block_desc d{};
+  if (mine) {
+    footprint(ge, foot, &tag, &d);
+    rows = foot[0];
+    fmt = fmt_of(d.q);
+    N = (int)d.N;
+    K = (int)d.K;
+    sld = tag == 0 ? 0 : (tag == 3 ? K / 128 : 1);
+  }
+  // exclusive sums over the experts of this launch before this one
+  long before_me[kSums];
+#pragma unroll
+  for (int i = 0; i < kSums; ++i) {
+    const long inc = wave_inclusive_scan(foot[i]);
+    before_me[i] = inc - foot[i];
+    const long tot = wave_last(inc);
+    if (lane == 0) s_tot[i][wave] = tot;
+  }
+  // smallest K of the launch: problems above it run first inside their branch (see launch_range)
+  __shared__ int s_kmin[2];
+  __shared__ long s_routed[2];
+  {
+    const long routed_tot = wave_last(wave_inclusive_scan(mine && ge < p.E ? rows : 0l));
+    int km = mine ? K : 0x7fffffff;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) km = min(km, __shfl_xor(km, o));
+    if (lane == 0) {
+      s_kmin[wave] = km;
+      s_routed[wave] = routed_tot;
+    }
+  }
+  __syncthreads();
+  const bool long_k = mine && K > min(s_kmin[0], s_kmin[1]);
+  // segments of this problem and, per branch in run order, this wave's entries and tiles
+  Segment sg[2];
+  const int ns = mine ? plan_segments(info, fmt, (int)rows, N, sg) : 0;
+  int seg_tiles[2], seg_rank[2], seg_pos[2], seg_first[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    seg_tiles[j] = j < ns ? segment_tiles(info, sg[j], N) : 0;
+    seg_rank[j] = -1;
+    seg_pos[j] = seg_first[j] = 0;
+  }
+  // branches that this wave's problems use at all (most branches of a kernel are not used by a given launch: their counters stay zero)
+  {
+    unsigned mask = 0;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      if (j < ns && seg_tiles[j] > 0) mask |= 1u << sg[j].branch;
+    if (mask) atomicOr(&s_used[wave], mask);
+  }
+  __builtin_amdgcn_wave_barrier();
+  const unsigned used = (unsigned)__builtin_amdgcn_readfirstlane((int)*(volatile unsigned*)&s_used[wave]);
+  for (int r = 0; r < info.nb; ++r) {
+    const int b = info.order[r];
+    if (!(used >> b & 1)) continue;
+    int mine_tiles = 0, which = -1;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      if (j < ns && sg[j].branch == b && seg_tiles[j] > 0) {
+        mine_tiles = seg_tiles[j];
+        which = j;
+      }
+    // entries of this branch in this wave, long-K problems first: position = matching lanes that run earlier, first tile = their tiles
+    const uint64_t has = __ballot(which >= 0), has_long = __ballot(which >= 0 && long_k);
+    const int tc = __popcll(has), tc_long = __popcll(has_long);
+    const int inc_long = wave_inclusive_scan(long_k ? mine_tiles : 0), inc_rest = wave_inclusive_scan(long_k ? 0 : mine_tiles);
+    const int tt_long = wave_last(inc_long), tt = tt_long + wave_last(inc_rest);
+    const uint64_t before = (1ull << lane) - 1;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      if (which == j) {
+        seg_rank[j] = r;
+        // position / first tile inside this wave's entries of its own class; the other wave's and the other class's are added below
+        seg_pos[j] = long_k ? __popcll(has_long & before) : __popcll(has & ~has_long & before);
+        seg_first[j] = long_k ? inc_long - mine_tiles : inc_rest - mine_tiles;
+      }
+    if (lane == 0) {
+      s_cnt[r][wave] = tc;
+      s_til[r][wave] = tt;
+      s_cnt_long[r][wave] = tc_long;
+      s_til_long[r][wave] = tt_long;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kSums; ++i) before_me[i] += s_base[i][0] + s_base[i][1] + (wave == 1 ? s_tot[i][0] : 0l);
+  const long first_row = before_me[0], inp_off = before_me[1], sc_off = before_me[2], out_off = before_me[3];
+  if (mine) {
+    table[ge] = tag;
+    table[p.Et + ge] = first_row;
+    table[2 * p.Et + ge] = inp_off;
+    table[3 * p.Et + ge] = sc_off;
+    const void* a_ptr = p.inp + 2 * inp_off;
+    const void* sa_ptr = sld > 0 ? p.scale + 2 * sc_off : nullptr;
+    if (kind == LayerForm::kGateUp) {
+      a_ptr = p.form.store[tag];
+      sa_ptr = sld > 0 ? p.form.scales[tag] : nullptr;
+      row_maps[ge] = ge < p.E ? p.form.token_of_row + first_row : p.form.iota;
+    } else if (kind == LayerForm::kBehind && tag == 0) {
+      a_ptr = p.form.act + 2 * before_me[4];
+    }
+    ptrs[ge] = a_ptr;
+    ptrs[p.Et + ge] = d.B;
+    ptrs[2 * p.Et + ge] = sa_ptr;
+    ptrs[3 * p.Et + ge] = d.scale_b;
+    ptrs[4 * p.Et + ge] = p.out + 2 * out_off;
+    sizes[ge] = mxmoe_dim3{(uint32_t)rows, (uint32_t)N, (uint32_t)K};
+    if (ge == p.E) misc[1] = (int64_t)(p.out + 2 * out_off);
+  }
+  // Branches in run order, one per lane (both waves hold the same): entries and tiles before each.
+  const int b_til = lane < info.nb ? s_til[lane][0] + s_til[lane][1] : 0, b_cnt = lane < info.nb ? s_cnt[lane][0] + s_cnt[lane][1] : 0;
+  const int til_inc = wave_inclusive_scan(b_til), cnt_inc = wave_inclusive_scan(b_cnt);
+  const int total = wave_last(til_inc), ne = wave_last(cnt_inc);
+  const int tile0 = til_inc - b_til, ent0 = cnt_inc - b_cnt;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int r = max(seg_rank[j], 0);
+    int pos = seg_pos[j] + __shfl(ent0, r), first = seg_first[j] + __shfl(tile0, r);
+    if (seg_rank[j] >= 0) {
+      // inside the branch: [long-K entries of wave 0][of wave 1][other entries of wave 0][of wave 1]
+      if (long_k) {
+        if (wave == 1) {
+          pos += s_cnt_long[r][0];
+          first += s_til_long[r][0];
+        }
+      } else {
+        pos += s_cnt_long[r][0] + s_cnt_long[r][1];
+        first += s_til_long[r][0] + s_til_long[r][1];
+        if (wave == 1) {
+          pos += s_cnt[r][0] - s_cnt_long[r][0];
+          first += s_til[r][0] - s_til_long[r][0];
+        }
+      }
+      fa->entry[pos] = FusedArgs::Entry{first, sg[j].row0, sg[j].rows, e | (sg[j].branch << 16)};  // problem index relative to the launch's first
+    }
+  }
+  if (wave == 0) {
+    // Phases: every branch with tiles is one, in run order; shapes beyond the phase table share the last phase.
+    const uint64_t live = __ballot(b_til > 0);
+    const int ord = __popcll(live & ((1ull << lane) - 1)), np = min(__popcll(live), kMaxPhases);
+    const bool starts = b_til > 0 && ord < kMaxPhases;
+    // workgroups of the phases that are one branch (all that may have a successor)
+    const int padded = b_til > 0 && ord < kMaxPhases - 1 ? (b_til + kNumXcd - 1) / kNumXcd * kNumXcd : 0;
+    const int wg0 = wave_inclusive_scan(padded) - padded;
+    const int flat = wave_last(wave_inclusive_scan(starts && flat_phase(info.b[info.order[min(lane, kMaxBranches - 1)]]) ? 1 << ord : 0));
+    if (starts) {
+      fa->phase_tile0[ord] = tile0;
+      fa->phase_wg0[ord] = wg0;
+      if (ord == np - 1) {  // the last phase: up to the last tile
+        fa->phase_tile0[np] = total;
+        fa->phase_wg0[np] = wg0 + (total - tile0 + kNumXcd - 1) / kNumXcd * kNumXcd;
+      }
+    }
+    if (lane == 0) {
+      // rows routed = sum over the routed experts of every launch: the last launch knows them all
+      if (chunk == chunks - 1) misc[0] = s_base[kSums][0] + s_base[kSums][1] + s_routed[0] + s_routed[1];
+      if (chunk == 0 && p.Et == p.E) misc[1] = 0;
+      if (np == 0) fa->phase_tile0[0] = fa->phase_wg0[0] = fa->phase_tile0[1] = fa->phase_wg0[1] = 0;  // a plan without tiles still holds one (empty) phase range
+      fa->num_phases = np;
+      fa->phase_flat = flat;
+      fa->num_entries = ne;
+      fa->total_tiles = total;
+      fa->problem_offset = e0;
+      fa->As = reinterpret_cast<const uint8_t* const*>(ptrs);
+      fa->Bs = reinterpret_cast<const uint8_t* const*>(ptrs + p.Et);
+      fa->sa = reinterpret_cast<const _Float16* const*>(ptrs + 2 * p.Et);
+      fa->sb = reinterpret_cast<const _Float16* const*>(ptrs + 3 * p.Et);
+      fa->Cs = reinterpret_cast<_Float16* const*>(const_cast<void**>(ptrs + 4 * p.Et));
+      fa->acc = nullptr;
+      fa->sizes = sizes;
+      fa->rows = row_maps;
+    }
+  }
+}
+
+// Kernel for the formats of `h_desc`, checked once on the host: every problem's format has a branch and its shape fits it (negative:
+// none, see last_error()).
+int resolve_kernel(int kernel_id, const mxmoe_block_desc* h_desc, int et);
+
+}  // namespace mxmoe

@@ -22,6 +22,7 @@
 
 #include <type_traits>
 
+#include "mxmoe_silu.hpp"
 #include "mxmoe_types.h"
 
 namespace mxmoe {
@@ -51,15 +52,21 @@ struct TileArgs {
   int M, N, K;           // M = end row of the segment this tile belongs to (rows at or past M are not computed)
   int row0;              // first row of the segment: tile_m counts BM-row tiles from here
   int tile_m, tile_n;
+  const int32_t* rows;   // gate_up form only: the row of A (and of sa) behind each row of the problem
 };
 
-// Keeps a freshly computed fp32 value opaque to the optimiser.  Without it the compiler folds "fp32 multiply, then convert to
-// fp16" into one v_fma_mixlo_f16, which rounds the exact product once; the reference arithmetic (and its CPU restatement) rounds
-// to fp32 first and to fp16 second, and the two differ on ties.
-__device__ __forceinline__ float keep_f32(float v) {
-  asm("" : "+v"(v));  // not volatile: it may be scheduled freely, it just cannot be looked through
-  return v;
-}
+// Every tile comes in two forms, run<false> and run<true>.  run<false> is the plain GEMM.  run<true>, the gate_up form, is what the
+// planned layer forward launches for its first block, and differs at both ends of the tile:
+//   * activations are not a contiguous [M, K] block but rows of a store that holds every token once: row m is row t.rows[m] of A (and
+//     of the token scales).  The index only enters the per-lane offsets of the tile's loads, which are the same for every K slice, so
+//     the gather costs one index load per tile, and top-k destinations of a token share one stored (and cached) row;
+//   * the weights are [gate; up] of 2I channels and the output is silu(gate) * up, [M, I] fp16: half of the tile's channels are gate
+//     channels and the other half the up channels of the same outputs, arranged so that both land in the same lane.  gate and up are
+//     rounded to fp16 first, as if they had been stored: the result is bit for bit what the activation step computes from the
+//     stored gate_up rows, without their write and read (8 bytes per output value).
+// A gathered load of a row past M must read zeros: it is given an offset past the end of its buffer resource.
+constexpr unsigned kGatherBytes = 0x7FFFFFFFu;  // size of such a resource: the stores of a gate_up form are below 2 GiB
+constexpr int kGatherPast = (int)0x80000000u;   // an offset past it whatever is added for the K slice
 
 // Loads / stores through pointers known to be global memory.  Pointers fetched from the per-problem pointer arrays are
 // generic to the compiler, which would emit flat_* instructions; those also count on the LDS counter, so every wait for an
@@ -106,9 +113,26 @@ __device__ __forceinline__ v4i gload16_untracked(const uint8_t* p) {
   asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(v) : "v"(p) : "memory");
   return v;
 }
-template <int N>
-__device__ __forceinline__ void vm_wait_for(v4i& v) {
+__device__ __forceinline__ int gload4_untracked(const int32_t* p) {
+  int v;
+  asm volatile("global_load_dword %0, %1, off" : "=v"(v) : "v"(p) : "memory");
+  return v;
+}
+__device__ __forceinline__ int gload2_untracked(const _Float16* p) {  // 16 bits, zero-extended
+  int v;
+  asm volatile("global_load_ushort %0, %1, off" : "=v"(v) : "v"(p) : "memory");
+  return v;
+}
+template <int N, class T>
+__device__ __forceinline__ void vm_wait_for(T& v) {
   asm volatile("s_waitcnt vmcnt(%1) ; landed %0" : "+v"(v) : "n"(N) : "memory");  // the comment names the register for the build's ISA check
+}
+// the same for several values at once (none of them may be touched before all have landed)
+template <int N, int S>
+__device__ __forceinline__ void vm_wait_for_all(int (&v)[S]) {
+  static_assert(S == 2 || S == 3, "as many as the tiles need");
+  if constexpr (S == 2) asm volatile("s_waitcnt vmcnt(%2) ; landed %0 %1" : "+v"(v[0]), "+v"(v[1]) : "n"(N) : "memory");
+  else asm volatile("s_waitcnt vmcnt(%3) ; landed %0 %1 %2" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]) : "n"(N) : "memory");
 }
 template <int N>
 __device__ __forceinline__ void vm_wait() {
@@ -201,23 +225,26 @@ struct MfmaTile {
   static constexpr int A_IT = (A_CHUNKS + kThreads - 1) / kThreads, B_IT = (B_CHUNKS + kThreads - 1) / kThreads;
   using Acc = typename OpTraits<OP>::Acc;
 
+  template <bool GU>
   __device__ static __forceinline__ void run(const TileArgs& t, uint8_t* __restrict__ smem) {
+    static_assert(!GU || OP == Op::F16, "the gate_up form is built for fp16 (integer problems take WxAxTile)");
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
     const int wm = wave / WGN, wn = wave % WGN;
-    const int M = t.M, N = t.N;
+    const int M = t.M, N = GU ? t.N / 2 : t.N;  // N: output channels
     const long row_bytes = (long)t.K * kBits / 8;
     const int KT = (int)(row_bytes / kRowBytes);
-    const int m0 = t.row0 + t.tile_m * BM, n0 = t.tile_n * BN;
+    constexpr int TNO = GU ? TN / 2 : TN;  // output channels of a wave
+    const int m0 = t.row0 + t.tile_m * BM, n0 = t.tile_n * (GU ? BN / 2 : BN);
 
     // ---- global -> LDS staging plan.  A K slice of the tile is (BM + BN) rows of 64 bytes = (BM + BN) / 16 wave-wide loads of
     // 1 KB, dealt round-robin to the 4 waves.  Each load writes 16 consecutive LDS rows; lane l fills 16-byte slot (row l/4, slot
     // l%4) and therefore fetches the chunk the swizzle maps there.  The buffer resources cover exactly the valid rows of the
     // tile, so rows past M (or N) arrive as zeros.
     const int a_rows = min(BM, M - m0), b_rows = min(BN, N - n0);
-    const v4i rs_a = make_rsrc(t.A + (long)m0 * row_bytes, (unsigned)(a_rows * row_bytes));
-    const v4i rs_b = make_rsrc(t.B + (long)n0 * row_bytes, (unsigned)(b_rows * row_bytes));
+    const v4i rs_a = GU ? make_rsrc(t.A, kGatherBytes) : make_rsrc(t.A + (long)m0 * row_bytes, (unsigned)(a_rows * row_bytes));
+    const v4i rs_b = GU ? make_rsrc(t.B, kGatherBytes) : make_rsrc(t.B + (long)n0 * row_bytes, (unsigned)(b_rows * row_bytes));
     constexpr int kDmaTotal = (BM + BN) / 16, kDmaA = BM / 16;
     constexpr int kDma = (kDmaTotal + kWaves - 1) / kWaves;  // loads per wave per slice
     const int uwave = __builtin_amdgcn_readfirstlane(wave);
@@ -227,7 +254,20 @@ struct MfmaTile {
     for (int i = 0; i < kDma; ++i) {
       const int ii = uwave + kWaves * i;
       const int r = (ii < kDmaA ? ii : ii - kDmaA) * 16 + (lane >> 2);
-      dma_voff[i] = r * (int)row_bytes + (((lane & 3) ^ lds_swizzle(r)) << 4);
+      const int chunk = ((lane & 3) ^ lds_swizzle(r)) << 4;
+      if constexpr (GU) {
+        // activation row r: the stored row of its token; weight row r of wave w = r / TN: gate channels first, then their up channels
+        if (ii < kDmaA) {
+          const int m = min(m0 + r, M - 1);
+          const int src = gload<int>(t.rows + m);
+          dma_voff[i] = r < a_rows ? src * (int)row_bytes + chunk : kGatherPast;
+        } else {
+          const int c = n0 + (r / TN) * TNO + r % TNO;
+          dma_voff[i] = c < N ? (c + (r % TN >= TNO ? N : 0)) * (int)row_bytes + chunk : kGatherPast;
+        }
+      } else {
+        dma_voff[i] = r * (int)row_bytes + chunk;
+      }
     }
     // load i of this wave (i < kDma) of the slice at byte offset koff, into stage `stage`; `live` = false turns it into a load of
     // zero bytes (nothing is fetched, nothing lands in LDS, the load still counts for s_waitcnt like any other)
@@ -411,7 +451,7 @@ struct MfmaTile {
           s_b[j][q] = gload<v4h>(t.sb + n);
         }
     }
-    if (t.acc_dump) {  // parity tests only
+    if (!GU && t.acc_dump) {  // parity tests only
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -427,12 +467,12 @@ struct MfmaTile {
           }
     }
     __syncthreads();  // every wave is done reading the pipeline stages: LDS can be reused
-    constexpr int kPitch = TN * 2 + 8;  // bytes per token row of the patch; the odd multiple of 8 spreads rows over banks
+    constexpr int kPitch = TNO * 2 + 8;  // bytes per token row of the patch; the odd multiple of 8 spreads rows over banks
     // the patch holds FI of the wave's FM 32-row blocks at a time (all of them when the pipeline's LDS is large enough)
     constexpr int FI = kWaves * TM * kPitch <= kLdsBytes ? FM : (kWaves * (TM / 2) * kPitch <= kLdsBytes ? FM / 2 : 1);
     static_assert(kWaves * FI * 32 * kPitch <= kLdsBytes && FM % FI == 0, "epilogue patch must fit the pipeline's LDS");
     uint8_t* patch = smem + wave * (FI * 32 * kPitch);
-    constexpr int kLanesPerRow = TN / 8;           // 16-byte pieces per token row
+    constexpr int kLanesPerRow = TNO / 8;          // 16-byte pieces per token row
     constexpr int kRowsPerPass = 64 / kLanesPerRow;
     const int pr = lane / kLanesPerRow, pc = lane % kLanesPerRow;
 #pragma unroll
@@ -442,12 +482,15 @@ struct MfmaTile {
         const int i = i0 + ii;
         const int ml = ii * 32 + lrow;
 #pragma unroll
-        for (int j = 0; j < FN; ++j) {
+        for (int j = 0; j < TNO / 32; ++j) {
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             const int nl = j * 32 + q * 8 + nq;
             v4h o;
-            if constexpr (OP == Op::F16) {
+            if constexpr (GU) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) o[e] = silu_mul_half((_Float16)acc[i][j][q * 4 + e], (_Float16)acc[i][j + FN / 2][q * 4 + e]);
+            } else if constexpr (OP == Op::F16) {
 #pragma unroll
               for (int e = 0; e < 4; ++e) o[e] = (_Float16)acc[i][j][q * 4 + e];
             } else if constexpr (OP == Op::BF16) {
@@ -473,7 +516,7 @@ struct MfmaTile {
       for (int r0 = 0; r0 < FI * 32; r0 += kRowsPerPass) {
         const int ml = r0 + pr;
         const int m = m0 + wm * TM + i0 * 32 + ml;
-        const int n = n0 + wn * TN + pc * 8;
+        const int n = n0 + wn * TNO + pc * 8;
         const v4i v = *reinterpret_cast<const v4i*>(patch + ml * kPitch + pc * 16);
         if (m < M && n < N) gstore_stream<v4i>(t.C + (long)m * N + n, v);
       }
@@ -515,7 +558,8 @@ struct WxAxTile {
   static constexpr int kPitch = TN * 2 + 8;                      // bytes per token row of the epilogue patch
   static constexpr int FI = FM >= 2 ? 2 : 1;                     // 32-row blocks of the patch written per round
   static constexpr int kPatchBytes = kWaves * FI * 32 * kPitch;
-  static constexpr int kLdsBytes = kStages * kStageBytes > kPatchBytes ? kStages * kStageBytes : kPatchBytes;
+  static constexpr int kScaleLds = kStages * kStageBytes > kPatchBytes ? kStages * kStageBytes : kPatchBytes;  // gate_up form: BM token scales (fp32)
+  static constexpr int kLdsBytes = kScaleLds + BM * 4;
   static constexpr int kAccRegs = FM * FN * 16;
   static constexpr int kWavesWanted = 2;  // waves per SIMD a kernel of such tiles is compiled for
   static constexpr int kABits = OpTraits<OP>::kBitsPerElem, kWBits = kABits;  // bits per activation / weight element
@@ -575,24 +619,37 @@ struct WxAxTile {
     }
   }
 
+  template <bool GU>
   __device__ static __forceinline__ void run(const TileArgs& t, uint8_t* __restrict__ smem) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int M = t.M, N = t.N;
+    const int M = t.M, N = GU ? t.N / 2 : t.N;  // N: output channels
     const long row_bytes = (long)t.K * kBits / 8;
     const int KT = (int)(row_bytes / kRowBytes);
-    const int m0 = t.row0 + t.tile_m * BM, n0 = t.tile_n * BN;
+    constexpr int TNO = GU ? TN / 2 : TN;       // output channels of a wave (gate_up form: block 0 = gate, block 1 = up channels)
+    const int m0 = t.row0 + t.tile_m * BM, n0 = t.tile_n * (GU ? BN / 2 : BN);
 
     // activations: global -> LDS
     const int a_rows = min(BM, M - m0);
-    const v4i rs_a = make_rsrc(t.A + (long)m0 * row_bytes, (unsigned)(a_rows * row_bytes));
+    const v4i rs_a = GU ? make_rsrc(t.A, kGatherBytes) : make_rsrc(t.A + (long)m0 * row_bytes, (unsigned)(a_rows * row_bytes));
     const int lds_base = (int)(uintptr_t)smem;
     int dma_voff[kDma];
+    // gate_up form: stored row of each row this lane loads (and, lanes 0 .. BM - 1 of the workgroup, of the row whose scale it fetches);
+    // issued before anything else and awaited only behind the first weight loads, which do not depend on it
+    int src_row[kDma + 1];
+    if constexpr (GU) {
 #pragma unroll
-    for (int i = 0; i < kDma; ++i) {
-      const int r = ((wave + kWaves * i) % kDmaTotal) * 16 + (lane >> 2);
-      dma_voff[i] = r * (int)row_bytes + (((lane & 3) ^ lds_swizzle(r)) << 4);
+      for (int i = 0; i <= kDma; ++i) {
+        const int m = min(m0 + (i < kDma ? ((wave + kWaves * i) % kDmaTotal) * 16 + (lane >> 2) : tid), M - 1);
+        src_row[i] = gload4_untracked(t.rows + m);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < kDma; ++i) {
+        const int r = ((wave + kWaves * i) % kDmaTotal) * 16 + (lane >> 2);
+        dma_voff[i] = r * (int)row_bytes + (((lane & 3) ^ lds_swizzle(r)) << 4);
+      }
     }
     auto dma_a = [&](int i, int kt, int stage) {
       const int ii = (wave + kWaves * i) % kDmaTotal;
@@ -614,7 +671,8 @@ struct WxAxTile {
     const uint8_t* bptr[FN];
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
-      const int nb = min(n0 / 32 + wave * FN + j, nblk - 1);  // blocks past N re-read the last one; their results are never stored
+      // blocks past N re-read the last one; their results are never stored
+      const int nb = GU ? min(n0 / 32 + wave, nblk - 1) + j * nblk : min(n0 / 32 + wave * FN + j, nblk - 1);
       bptr[j] = t.B + (long)nb * KT * 2048 + lane * 16;
     }
     auto load_b = [&](int j, int step, int kt) { return gload16_untracked(bptr[j] + ((long)min(kt, KT - 1) * 2 + step) * 1024); };
@@ -639,20 +697,38 @@ struct WxAxTile {
 
     // ---- prologue: slices 0 .. kDepth-2 complete, then the load pattern of one (virtual) iteration for slice kDepth-1, so that
     // the counts below hold from kt = 0
+    if constexpr (!GU) {
 #pragma unroll
-    for (int i = 0; i < kDma; ++i) dma_a(i, 0, 0);
+      for (int i = 0; i < kDma; ++i) dma_a(i, 0, 0);
+    }
 #pragma unroll
     for (int d = 0; d < kDepth - 1; ++d)
 #pragma unroll
       for (int j = 0; j < FN; ++j)
 #pragma unroll
         for (int s = 0; s < 2; ++s) pbq[d][j][s] = load_b(j, s, d);
+    int scale_bits = 0;
+    if constexpr (GU) {
+      vm_wait_for_all<(kDepth - 1) * FN * 2>(src_row);  // (only the weight loads above are younger)
+#pragma unroll
+      for (int i = 0; i < kDma; ++i) {
+        const int r = ((wave + kWaves * i) % kDmaTotal) * 16 + (lane >> 2);
+        dma_voff[i] = r < a_rows ? src_row[i] * (int)row_bytes + (((lane & 3) ^ lds_swizzle(r)) << 4) : kGatherPast;
+      }
+#pragma unroll
+      for (int i = 0; i < kDma; ++i) dma_a(i, 0, 0);
+      scale_bits = gload2_untracked(t.sa + src_row[kDma]);
+    }
 #pragma unroll
     for (int d = 0; d < kDepth - 1; ++d)
 #pragma unroll
       for (int j = 0; j < FN; ++j)
 #pragma unroll
         for (int s = 0; s < 2; ++s) vm_wait_for<0>(pbq[d][j][s]);
+    if constexpr (GU) {
+      vm_wait_for<0>(scale_bits);
+      if (tid < BM) reinterpret_cast<float*>(smem + kScaleLds)[tid] = (float)__builtin_bit_cast(_Float16, (unsigned short)scale_bits);
+    }
     __syncthreads();
     static_for<U>([&](auto uc) {
       constexpr int u = decltype(uc)::value;
@@ -758,18 +834,22 @@ struct WxAxTile {
     v4h s_b[FN][4];
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
-      const int m = min(m0 + i * 32 + lrow, M - 1);
-      s_a[i] = (float)gload<_Float16>(t.sa + m);
+      if constexpr (GU) {
+        s_a[i] = reinterpret_cast<const float*>(smem + kScaleLds)[i * 32 + lrow];
+      } else {
+        const int m = min(m0 + i * 32 + lrow, M - 1);
+        s_a[i] = (float)gload<_Float16>(t.sa + m);
+      }
       if constexpr (OP == Op::I4) s_a[i] *= 0.00390625f;  // the int4 accumulator holds 256 * sum (exact power of two)
     }
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int n = min(n0 + wave * TN + j * 32 + q * 8 + nq, N - 4);
+        const int n = GU ? j * N + min(n0 + wave * TNO + q * 8 + nq, N - 4) : min(n0 + wave * TN + j * 32 + q * 8 + nq, N - 4);
         s_b[j][q] = gload<v4h>(t.sb + n);
       }
-    if (t.acc_dump) {  // parity tests only
+    if (!GU && t.acc_dump) {  // parity tests only
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -785,8 +865,9 @@ struct WxAxTile {
           }
     }
     __syncthreads();  // every wave is done reading the activation stages: LDS can be reused
-    uint8_t* patch = smem + wave * (FI * 32 * kPitch);
-    constexpr int kLanesPerRow = TN / 8, kRowsPerPass = 64 / kLanesPerRow;
+    constexpr int kPitchO = TNO * 2 + 8;
+    uint8_t* patch = smem + wave * (FI * 32 * kPitchO);
+    constexpr int kLanesPerRow = TNO / 8, kRowsPerPass = 64 / kLanesPerRow;
     const int pr = lane / kLanesPerRow, pc = lane % kLanesPerRow;
 #pragma unroll
     for (int i0 = 0; i0 < FM; i0 += FI) {
@@ -794,26 +875,30 @@ struct WxAxTile {
       for (int ii = 0; ii < FI; ++ii) {
         const int i = i0 + ii;
         const int ml = ii * 32 + lrow;
+        // float(acc) * (sa * sb) rounded once to half; the scale product stays in fp32 (see MfmaTile)
+        auto scaled = [&](int j, int q, int e) {
+          const float sc = s_a[i] * (float)s_b[j][q][e];
+          return (_Float16)keep_f32((float)acc[i][j][q * 4 + e] * sc);
+        };
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
+        for (int j = 0; j < (GU ? 1 : FN); ++j)
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             v4h o;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-              // float(acc) * (sa * sb) rounded once to half; the scale product stays in fp32 (see MfmaTile)
-              const float sc = s_a[i] * (float)s_b[j][q][e];
-              o[e] = (_Float16)keep_f32((float)acc[i][j][q * 4 + e] * sc);
+              if constexpr (GU) o[e] = silu_mul_half(scaled(0, q, e), scaled(1, q, e));
+              else o[e] = scaled(j, q, e);
             }
-            *reinterpret_cast<v4h*>(patch + ml * kPitch + (j * 32 + q * 8 + nq) * 2) = o;
+            *reinterpret_cast<v4h*>(patch + ml * kPitchO + (j * 32 + q * 8 + nq) * 2) = o;
           }
       }
 #pragma unroll
       for (int r0 = 0; r0 < FI * 32; r0 += kRowsPerPass) {
         const int ml = r0 + pr;
         const int m = m0 + i0 * 32 + ml;
-        const int n = n0 + wave * TN + pc * 8;
-        const v4i v = *reinterpret_cast<const v4i*>(patch + ml * kPitch + pc * 16);
+        const int n = n0 + wave * TNO + pc * 8;
+        const v4i v = *reinterpret_cast<const v4i*>(patch + ml * kPitchO + pc * 16);
         if (m < M && n < N) gstore_stream<v4i>(t.C + (long)m * N + n, v);
       }
     }

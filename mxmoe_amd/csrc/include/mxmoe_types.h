@@ -51,6 +51,22 @@ typedef struct {
   void* d_plan;                     // plan buffer of mxmoe_plan_bytes() bytes
 } mxmoe_plan_call;
 
+// A layer for the short form of the planned forward (mxmoe_layer_create); what each buffer holds is described there.
+typedef struct {
+  int32_t num_tokens, topk, num_experts, has_shared;
+  int32_t hidden, inter, inter_shared, rotate;
+  int32_t had_k, had_f;
+  const float* had_signs;
+  int32_t kernel_gate_up, kernel_down, grid_gate_up, grid_down;
+  const mxmoe_block_desc *d_gate_up, *h_gate_up, *d_down, *h_down;
+  void* token_store[6];
+  void* token_scales[6];
+  void *act, *down_inp, *down_scales, *down_out, *plan_gate_up, *plan_down;
+  int32_t *dst_exp, *token_of_row, *row_of_slot, *iota;
+  int64_t* recv;
+  void* workspace;
+} mxmoe_layer_desc;
+
 #ifdef __cplusplus
 }
 #endif

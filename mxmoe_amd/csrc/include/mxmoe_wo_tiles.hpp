@@ -137,8 +137,10 @@ struct SkinnyWoTile {
   // kRing KB per wave are always in flight.  Per 128-wide group g and channel n the pass adds
   //   s * (sum_k x[k] * (q[k] + bias[k])  -  sum_k x[k] * bias[k])  +  z * sum_k x[k]
   // where the first sum comes from 4 MFMAs on the biased weights and the other two from MFMAs of x against constant operands.
-  template <int NKB>
-  __device__ static __forceinline__ void pass(const TileArgs& t, int kb0, int m0, int n0, int nbv, int lane, uint8_t* __restrict__ spatch, v4f (&acc)[NB][MB]) {
+  // Gate_up form: channel blocks 0 .. NB/2 - 1 are gate channels from n0 on, blocks NB/2 .. NB - 1 the up channels of the same outputs;
+  // nbv counts the existing ones of either half.  `src`: the activation row of this lane in each token block.
+  template <bool GU, int NKB>
+  __device__ static __forceinline__ void pass(const TileArgs& t, int kb0, int m0, int n0, int nbv, int lane, const int (&src)[MB], uint8_t* __restrict__ spatch, v4f (&acc)[NB][MB]) {
     const int K = t.K, KB = K / 128;
     const int lm = lane & 15, lg = lane >> 4;
     const v8h ones = {(_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f};
@@ -149,7 +151,12 @@ struct SkinnyWoTile {
     // the stream, the activations and the (scale, zero) pairs then arrive together, one memory latency after the pass began
     // (waiting for the scales before requesting the weights costs a second one, which is a third of a short tile's life).
     const uint8_t* wb = t.B + ((long)(n0 / 16) * KB + kb0) * kBlockBytes + lane * kLaneBytes;
-    auto w_of = [&](int q) { const int nb = q / NKB < nbv ? q / NKB : 0; return load_w(wb + ((long)nb * KB + q % NKB) * kBlockBytes); };
+    // channel block nb of the tile, relative to its first one (blocks that do not exist re-read an existing one)
+    auto block_of = [&](int nb) {
+      if constexpr (GU) return (nb % (NB / 2) < nbv ? nb % (NB / 2) : 0) + (nb >= NB / 2 ? t.N / 32 : 0);
+      else return nb < nbv ? nb : 0;
+    };
+    auto w_of = [&](int q) { return load_w(wb + ((long)block_of(q / NKB) * KB + q % NKB) * kBlockBytes); };
     WReg wr[kRing];
 #pragma unroll
     for (int q = 0; q < kRing && q < Q; ++q) wr[q] = w_of(q);
@@ -159,7 +166,7 @@ struct SkinnyWoTile {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
       const int m = m0 + mb * 16 + lm;
-      const _Float16* xr = reinterpret_cast<const _Float16*>(t.A) + (long)(m < t.M ? m : 0) * K + kb0 * 128 + lg * 32;
+      const _Float16* xr = reinterpret_cast<const _Float16*>(t.A) + (long)src[mb] * K + kb0 * 128 + lg * 32;
 #pragma unroll
       for (int s = 0; s < NKB; ++s)
 #pragma unroll
@@ -176,7 +183,7 @@ struct SkinnyWoTile {
     for (int i = 0; i < kPieces; ++i) {
       const int c = min(lane + 64 * i, Q * 4 - 1);
       const int nb = c / (NKB * 4), rest = c % (NKB * 4);
-      sv[i] = gload<v4i>(sb + ((long)(nb < nbv ? nb : 0) * KB) * 64 + rest * 16);
+      sv[i] = gload<v4i>(sb + ((long)block_of(nb) * KB) * 64 + rest * 16);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -218,15 +225,24 @@ struct SkinnyWoTile {
     });
   }
 
+  template <bool GU>
   __device__ static __forceinline__ void run(const TileArgs& t, uint8_t* __restrict__ smem) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int M = t.M, N = t.N, K = t.K;
-    const int m0 = t.row0 + t.tile_m * BM, n0 = t.tile_n * BN;
+    const int M = t.M, N = GU ? t.N / 2 : t.N, K = t.K;  // N: output channels
+    constexpr int NBO = GU ? NB / 2 : NB;                // output channel blocks of the tile
+    const int m0 = t.row0 + t.tile_m * BM, n0 = t.tile_n * 16 * NBO;
     const int KB = K / 128;  // k blocks (= quantisation groups) per row
     const int lm = lane & 15, lg = lane >> 4;
-    const int nbv = min(NB, (N - n0) / 16);  // channel blocks of this tile that exist
+    const int nbv = min(NBO, (N - n0) / 16);  // output channel blocks of this tile that exist
+    int src[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      const int m = min(m0 + mb * 16 + lm, M - 1);
+      if constexpr (GU) src[mb] = gload<int>(t.rows + m);
+      else src[mb] = m;
+    }
 
     // the K range is dealt to the 4 waves in contiguous quarters; each wave sums its quarter for every channel of the tile
     const int KW = (KB + kWaves - 1) / kWaves;
@@ -240,15 +256,15 @@ struct SkinnyWoTile {
     for (int kb = kb_lo; kb < kb_hi; kb += KP) {
       const int nk = min(KP, kb_hi - kb);
       if constexpr (KP >= 4) {
-        if (nk == 4) { pass<4>(t, kb, m0, n0, nbv, lane, spatch, acc); continue; }
+        if (nk == 4) { pass<GU, 4>(t, kb, m0, n0, nbv, lane, src, spatch, acc); continue; }
       }
       if constexpr (KP >= 3) {
-        if (nk == 3) { pass<3>(t, kb, m0, n0, nbv, lane, spatch, acc); continue; }
+        if (nk == 3) { pass<GU, 3>(t, kb, m0, n0, nbv, lane, src, spatch, acc); continue; }
       }
       if constexpr (KP >= 2) {
-        if (nk == 2) { pass<2>(t, kb, m0, n0, nbv, lane, spatch, acc); continue; }
+        if (nk == 2) { pass<GU, 2>(t, kb, m0, n0, nbv, lane, src, spatch, acc); continue; }
       }
-      pass<1>(t, kb, m0, n0, nbv, lane, spatch, acc);
+      pass<GU, 1>(t, kb, m0, n0, nbv, lane, src, spatch, acc);
     }
 
     // reduction over the 4 waves in a fixed order (wave 0 + 1 + 2 + 3), 16-channel blocks dealt round-robin to the waves
@@ -258,26 +274,37 @@ struct SkinnyWoTile {
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) red[((wave * NB + nb) * MB + mb) * 64 + lane] = acc[nb][mb];
     __syncthreads();
+    auto total = [&](int nb, int mb) {
+      v4f sum = red[(nb * MB + mb) * 64 + lane];
 #pragma unroll
-    for (int r = 0; r < NB / kWaves; ++r) {
+      for (int w = 1; w < kWaves; ++w) {
+        const v4f p = red[((w * NB + nb) * MB + mb) * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[e] += p[e];
+      }
+      return sum;
+    };
+#pragma unroll
+    for (int r = 0; r < (NBO + kWaves - 1) / kWaves; ++r) {
       const int nb = wave + kWaves * r;
+      if (NBO % kWaves != 0 && nb >= NBO) break;
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
         const int m = m0 + mb * 16 + lm;
-        v4f sum = red[(nb * MB + mb) * 64 + lane];
+        const v4f sum = total(nb, mb);
+        v4h o;
+        if constexpr (GU) {
+          const v4f up = total(nb + NB / 2, mb);
 #pragma unroll
-        for (int w = 1; w < kWaves; ++w) {
-          const v4f p = red[((w * NB + nb) * MB + mb) * 64 + lane];
+          for (int e = 0; e < 4; ++e) o[e] = silu_mul_half((_Float16)sum[e], (_Float16)up[e]);
+        } else {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) sum[e] += p[e];
+          for (int e = 0; e < 4; ++e) o[e] = (_Float16)sum[e];
         }
         if (m < M && nb < nbv) {
           const int n = n0 + nb * 16 + lg * 4;
-          v4h o;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = (_Float16)sum[e];
           gstore<v4h>(t.C + (long)m * N + n, o);
-          if (t.acc_dump) {
+          if (!GU && t.acc_dump) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               const float f = sum[e];  // a copy: a bit cast applied to a vector element reads element 0
@@ -318,30 +345,39 @@ struct WoMfmaTile {
   static constexpr int kLaneBytes = Sk::kLaneBytes, kBlockBytes = Sk::kBlockBytes;
   static constexpr int kDma = kStageBytes / 1024 / kWaves;  // direct-to-LDS loads per wave per stage
 
+  template <bool GU>
   __device__ static __forceinline__ void run(const TileArgs& t, uint8_t* __restrict__ smem) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = WM == 2 ? wave >> 1 : 0, wn = WM == 2 ? wave & 1 : wave;
-    const int M = t.M, N = t.N, K = t.K;
-    const int m0 = t.row0 + t.tile_m * BM, n0 = t.tile_n * BN;
+    const int M = t.M, N = GU ? t.N / 2 : t.N, K = t.K;  // N: output channels
+    constexpr int NBO = GU ? 2 : 4;                      // output channel blocks of a wave (gate_up form: blocks 0, 1 gate, 2, 3 up)
+    const int m0 = t.row0 + t.tile_m * BM, n0 = t.tile_n * (GU ? BN / 2 : BN);
     const int KB = K / 128;
     const int lm = lane & 15, lg = lane >> 4;
     // channel blocks of this wave that exist; a wave whose 64 channels all lie past N runs on the tile's first blocks instead
     // (every wave must take part in the barriers) and stores nothing
-    const int nbv = max(0, min(4, (N - n0) / 16 - wn * 4));
-    const int nb0 = n0 / 16 + (nbv > 0 ? wn * 4 : 0);
+    const int nbv = max(0, min(NBO, (N - n0) / 16 - wn * NBO));
+    const int nb0 = n0 / 16 + (nbv > 0 ? wn * NBO : 0);
+    auto block_of = [&](int nb) { return GU ? (nb % NBO < nbv ? nb % NBO : 0) + nb / NBO * (N / 16) : (nb < nbv ? nb : 0); };
 
     // activations: buffer resource over the valid rows of the tile (rows past M read as zeros)
     const int a_rows = min(BM, M - m0);
-    const v4i rs_x = make_rsrc(t.A + (long)m0 * K * 2, (unsigned)((long)a_rows * K * 2));
+    const v4i rs_x = GU ? make_rsrc(t.A, kGatherBytes) : make_rsrc(t.A + (long)m0 * K * 2, (unsigned)((long)a_rows * K * 2));
     const int lds_base = (int)(uintptr_t)smem;
     int dma_voff[kDma], dma_lds[kDma];
 #pragma unroll
     for (int i = 0; i < kDma; ++i) {
       const int ii = wave * kDma + i;             // 1 KB piece = 4 rows
       const int row = 4 * ii + (lane >> 4);
-      dma_voff[i] = row * K * 2 + (((lane & 15) ^ (row & 15)) << 4);
+      const int chunk = ((lane & 15) ^ (row & 15)) << 4;
+      if constexpr (GU) {
+        const int src = gload<int>(t.rows + min(m0 + row, M - 1));
+        dma_voff[i] = row < a_rows ? src * (K * 2) + chunk : kGatherPast;
+      } else {
+        dma_voff[i] = row * K * 2 + chunk;
+      }
       dma_lds[i] = ii * 1024;
     }
     auto dma_x = [&](int kb, int stage) {
@@ -360,8 +396,8 @@ struct WoMfmaTile {
     // (never used) so that every iteration issues the same number of loads, which the wait for the activation stage relies on.
     const uint8_t* wb = t.B + ((long)nb0 * KB) * kBlockBytes + lane * kLaneBytes;
     const uint8_t* sb = reinterpret_cast<const uint8_t*>(t.sb) + ((long)nb0 * KB) * 64 + lm * 4;
-    auto w_of = [&](int nb, int kb) { return Sk::load_w(wb + ((long)(nb < nbv ? nb : 0) * KB + min(kb, KB - 1)) * kBlockBytes); };
-    auto s_of = [&](int nb, int kb) { return gload<int>(sb + ((long)(nb < nbv ? nb : 0) * KB + min(kb, KB - 1)) * 64); };
+    auto w_of = [&](int nb, int kb) { return Sk::load_w(wb + ((long)block_of(nb) * KB + min(kb, KB - 1)) * kBlockBytes); };
+    auto s_of = [&](int nb, int kb) { return gload<int>(sb + ((long)block_of(nb) * KB + min(kb, KB - 1)) * 64); };
     typename Sk::WReg wr[8];
     int sr[8];
 
@@ -448,22 +484,30 @@ struct WoMfmaTile {
 
     // epilogue, 64 tokens at a time: [token][channel] fp16 patch per wave (64 x 64, row pitch 136 B), then 16-byte
     // row-contiguous stores
-    constexpr int kPitch = 64 * 2 + 8;
+    constexpr int kWidth = NBO * 16;                // output channels of a wave
+    constexpr int kPitch = kWidth * 2 + 8;
+    constexpr int kLanes = kWidth / 8, kRows = 64 / kLanes;  // lanes (16 bytes each) per row, rows per pass
     uint8_t* patch = smem + wave * (64 * kPitch);
-    const int pr = lane >> 3, pc = lane & 7;  // 8 lanes x 16 B per 64-channel row, 8 rows per pass
+    const int pr = lane / kLanes, pc = lane % kLanes;
 #pragma unroll
     for (int h = 0; h < TM / 64; ++h) {
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb)
+      for (int nb = 0; nb < NBO; ++nb)
 #pragma unroll
         for (int mb = 0; mb < 4; ++mb) {
           const v4f a = acc[nb][h * 4 + mb];
           v4h o;
+          if constexpr (GU) {
+            const v4f up = acc[nb + NBO][h * 4 + mb];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = (_Float16)a[e];
+            for (int e = 0; e < 4; ++e) o[e] = silu_mul_half((_Float16)a[e], (_Float16)up[e]);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = (_Float16)a[e];
+          }
           *reinterpret_cast<v4h*>(patch + (mb * 16 + lm) * kPitch + (nb * 16 + lg * 4) * 2) = o;
-          if (t.acc_dump) {
-            const int m = m0 + wm * TM + h * 64 + mb * 16 + lm, n = n0 + wn * 64 + nb * 16 + lg * 4;
+          if (!GU && t.acc_dump) {
+            const int m = m0 + wm * TM + h * 64 + mb * 16 + lm, n = n0 + wn * kWidth + nb * 16 + lg * 4;
             if (m < M && n < N) {
 #pragma unroll
               for (int e = 0; e < 4; ++e) gstore<int>(t.acc_dump + (long)m * N + n + e, __float_as_int(a[e]));
@@ -471,9 +515,9 @@ struct WoMfmaTile {
           }
         }
 #pragma unroll
-      for (int r0 = 0; r0 < 64; r0 += 8) {
+      for (int r0 = 0; r0 < 64; r0 += kRows) {
         const int ml = r0 + pr;
-        const int m = m0 + wm * TM + h * 64 + ml, n = n0 + wn * 64 + pc * 8;
+        const int m = m0 + wm * TM + h * 64 + ml, n = n0 + wn * kWidth + pc * 8;
         const v4i v = *reinterpret_cast<const v4i*>(patch + ml * kPitch + pc * 16);
         if (m < M && n < N) gstore_stream<v4i>(t.C + (long)m * N + n, v);
       }

@@ -12,315 +12,9 @@
 #include "include/mxmoe_launch.hpp"
 #include "include/mxmoe_plan.hpp"
 #include "include/mxmoe_perm.hpp"
+#include "include/mxmoe_plan_body.hpp"
 
 namespace mxmoe {
-
-// A block descriptor (not the QParams arrays of the launcher, whose padding bytes belong to the caller) may name an operand variant
-// in q._pad[0]: 1 = the int4 codes of per-token activations as bf6 fragments (for the kernels whose w4a4 tiles run on the 6-bit float
-// matrix path), 2 = per-token fp8 e4m3 codes instead of int8 ones (for the kernels whose w8a8 tiles run the fp8 instruction).
-__host__ __device__ inline bool wants_bf6(const mxmoe_qparams& q) { return q._pad[0] == 1 && q.a_bits == 4 && q.w_bits == 4 && q.gsize == -1; }
-__host__ __device__ inline bool wants_fp8(const mxmoe_qparams& q) { return q._pad[0] == 2 && q.a_bits == 8 && q.w_bits == 8 && q.gsize == -1; }
-
-__host__ __device__ inline int act_tag_of(const mxmoe_qparams& q) {  // ref_bind.cu:461-473
-  if (q.a_bits >= 16) return 0;
-  if (wants_fp8(q)) return 5;
-  if (q.a_bits == 8 && q.gsize == -1) return 1;
-  if (wants_bf6(q)) return 4;
-  if (q.a_bits == 4 && q.gsize == -1) return 2;
-  if (q.a_bits == 4 && q.gsize == 128) return 3;
-  return -1;
-}
-
-__host__ __device__ inline int fmt_of(const mxmoe_qparams& q) { return (int)classify(q); }
-
-struct PlanParams {
-  const int64_t* recv;
-  const mxmoe_block_desc* desc;
-  const uint8_t* inp;
-  const uint8_t* scale;
-  uint8_t* out;
-  uint8_t* plan;
-  int E, Et, shared_rows;
-  PlanInfo info;
-};
-
-constexpr int kPlanThreads = 128;
-constexpr int kMaxPlannedProblems = 4096;  // experts of a planned block (run as launches of kMaxProblems experts each)
-static_assert(kMaxProblems <= kPlanThreads, "one thread per problem");
-
-__device__ __forceinline__ long wave_excl_scan(long v, int lane, long* total) {
-  long inc = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const long t = __shfl_up(inc, o);
-    if (lane >= o) inc += t;
-  }
-  *total = __shfl(inc, 63);
-  return inc - v;
-}
-
-// One workgroup of two waves per launch, thread e = expert e0 + e of the launch's chunk of experts [e0, e0 + kMaxProblems) (the shared
-// expert, if any, is expert E with `shared_rows` rows).  Everything the host launcher computes (launch_range), with the same
-// functions and in the same order, so the two produce identical tables; prefix sums over experts are wave scans (a later chunk
-// first sums what the experts before it occupy), and an entry finds its place from per-branch counts instead of a sequential walk.
-struct PlanPair {
-  PlanParams p[2];
-  int chunks;  // launches per block
-};
-
-// `recv`: the tokens-per-expert counts (device memory, or LDS when the planning workgroup counted them itself).
-__device__ __forceinline__ void plan_block_body(const PlanParams& p, const int chunk, const int chunks, const int64_t* recv) {
-  const int e0 = chunk * kMaxProblems;                       // first expert of this launch
-  const int ecnt = min(kMaxProblems, p.Et - e0);             // experts of this launch
-  __shared__ long s_tot[4][2];                       // per wave: rows, packed input, scales, output elements
-  __shared__ long s_base[5][2];                      // the same four, and the routed rows, summed over the experts before this launch
-  __shared__ int s_cnt[kMaxBranches][2], s_til[kMaxBranches][2];  // per run-order rank and wave: entries, tiles
-  __shared__ int s_cnt_long[kMaxBranches][2], s_til_long[kMaxBranches][2];  // ... of which belong to long-K problems
-  // the kernel's branch table, from the kernel arguments into LDS: the planning functions walk it entry by entry, and each step of
-  // such a walk through the argument segment costs a trip to the scalar cache
-  __shared__ PlanInfo info;
-  static_assert(sizeof(PlanInfo) % 4 == 0, "copied word by word");
-  for (int i = threadIdx.x; i < (int)(sizeof(PlanInfo) / 4); i += kPlanThreads) reinterpret_cast<int*>(&info)[i] = reinterpret_cast<const int*>(&p.info)[i];
-  const int e = threadIdx.x, lane = e & 63, wave = e >> 6;
-  const int ge = e0 + e;                             // this thread's expert
-  __shared__ unsigned s_used[2];                     // per wave: branches in use
-  if (e < kMaxBranches) {
-    s_cnt[e][0] = s_cnt[e][1] = s_til[e][0] = s_til[e][1] = 0;
-    s_cnt_long[e][0] = s_cnt_long[e][1] = s_til_long[e][0] = s_til_long[e][1] = 0;
-  }
-  if (e < 2) s_used[e] = 0;
-  const bool mine = e < ecnt;
-  const PlanLayout lay(p.Et);
-  FusedArgs* fa = reinterpret_cast<FusedArgs*>(p.plan + chunk * kFusedArgsStride);
-  int64_t* table = reinterpret_cast<int64_t*>(p.plan + lay.table);
-  const void** ptrs = reinterpret_cast<const void**>(p.plan + lay.ptrs);
-  int64_t* misc = reinterpret_cast<int64_t*>(p.plan + lay.misc);
-  mxmoe_dim3* sizes = reinterpret_cast<mxmoe_dim3*>(p.plan + lay.sizes);
-
-  // what one expert occupies: rows, packed activation elements, scales, output elements (all in fp16 elements but the rows)
-  auto footprint = [&](int x, long (&f)[4], int* tag_out, mxmoe_block_desc* d_out) {
-    const mxmoe_block_desc d = p.desc[x];
-    const long rows = x < p.E ? (long)recv[x] : (long)p.shared_rows;
-    const int tag = act_tag_of(d.q), K = (int)d.K;
-    const long qld = tag == 0 ? K : (tag == 1 || tag == 5 ? K / 2 : K / 4);  // fp16 elements per packed activation row (ref_bind.cu:491)
-    const long sld = tag == 0 ? 0 : (tag == 3 ? K / 128 : 1);                // scales per row (ref_bind.cu:492)
-    f[0] = rows;
-    // packed activations: rows of qld elements, or (tag 4) whole blocks of 32 rows of K / 64 fragments
-    f[1] = tag == 4 ? ((rows + 31) >> 5) * (long)(K >> 6) * (kBf6Frag / 2) : qld * rows;
-    f[2] = sld * rows;
-    f[3] = (long)d.N * rows;
-    if (tag_out) *tag_out = tag;
-    if (d_out) *d_out = d;
-  };
-  // experts before this launch (none for the first: most blocks are one launch)
-  if (e0 > 0) {
-    long base[5] = {0, 0, 0, 0, 0};
-    for (int x = e; x < e0; x += kPlanThreads) {
-      long f[4];
-      footprint(x, f, nullptr, nullptr);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) base[i] += f[i];
-      if (x < p.E) base[4] += f[0];
-    }
-#pragma unroll
-    for (int i = 0; i < 5; ++i) {
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) base[i] += __shfl_xor(base[i], o);
-      if (lane == 0) s_base[i][wave] = base[i];
-    }
-  } else if (lane == 0) {
-#pragma unroll
-    for (int i = 0; i < 5; ++i) s_base[i][wave] = 0;
-  }
-
-  long rows = 0, sld = 0;
-  long foot[4] = {0, 0, 0, 0};
-  int tag = 0, fmt = 0, N = 0, K = 0;
-  mxmoe_block_desc d{};
-  if (mine) {
-    footprint(ge, foot, &tag, &d);
-    rows = foot[0];
-    fmt = fmt_of(d.q);
-    N = (int)d.N;
-    K = (int)d.K;
-    sld = tag == 0 ? 0 : (tag == 3 ? K / 128 : 1);
-  }
-  // exclusive sums over the experts of this launch before this one
-  long tot[4], routed_tot;
-  long first_row = wave_excl_scan(foot[0], lane, &tot[0]);
-  long inp_off = wave_excl_scan(foot[1], lane, &tot[1]);
-  long sc_off = wave_excl_scan(foot[2], lane, &tot[2]);
-  long out_off = wave_excl_scan(foot[3], lane, &tot[3]);
-  wave_excl_scan(mine && ge < p.E ? rows : 0, lane, &routed_tot);
-  if (lane == 0) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) s_tot[i][wave] = tot[i];
-  }
-  // smallest K of the launch: problems above it run first inside their branch (see launch_range)
-  __shared__ int s_kmin[2];
-  __shared__ long s_routed[2];
-  {
-    int km = mine ? K : 0x7fffffff;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) km = min(km, __shfl_xor(km, o));
-    if (lane == 0) {
-      s_kmin[wave] = km;
-      s_routed[wave] = routed_tot;
-    }
-  }
-  __syncthreads();
-  const bool long_k = mine && K > min(s_kmin[0], s_kmin[1]);
-  // segments of this problem and, per branch in run order, this wave's entries and tiles
-  Segment sg[2];
-  const int ns = mine ? plan_segments(info, fmt, (int)rows, N, sg) : 0;
-  int seg_tiles[2], seg_rank[2], seg_pos[2], seg_first[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    seg_tiles[j] = j < ns ? segment_tiles(info, sg[j], N) : 0;
-    seg_rank[j] = -1;
-    seg_pos[j] = seg_first[j] = 0;
-  }
-  // branches that this wave's problems use at all (most branches of a kernel are not used by a given launch: their counters stay zero)
-  {
-    unsigned mask = 0;
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      if (j < ns && seg_tiles[j] > 0) mask |= 1u << sg[j].branch;
-    if (mask) atomicOr(&s_used[wave], mask);
-  }
-  __builtin_amdgcn_wave_barrier();
-  const unsigned used = (unsigned)__builtin_amdgcn_readfirstlane((int)*(volatile unsigned*)&s_used[wave]);
-  for (int r = 0; r < info.nb; ++r) {
-    const int b = info.order[r];
-    if (!(used >> b & 1)) continue;
-    int mine_tiles = 0, which = -1;
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      if (j < ns && sg[j].branch == b && seg_tiles[j] > 0) {
-        mine_tiles = seg_tiles[j];
-        which = j;
-      }
-    // entries of this branch in this wave, long-K problems first: position = matching lanes that run earlier, first tile = their tiles
-    const uint64_t has = __ballot(which >= 0);
-    int tc = 0, tt = 0, tc_long = 0, tt_long = 0;
-    if (has != 0) {  // (wave-uniform: most branches of a kernel are not used by a given launch)
-      const uint64_t has_long = __ballot(which >= 0 && long_k);
-      tc = __popcll(has);
-      tc_long = __popcll(has_long);
-      int inc_long = long_k ? mine_tiles : 0, inc_rest = long_k ? 0 : mine_tiles;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int t0 = __shfl_up(inc_long, o), t1 = __shfl_up(inc_rest, o);
-        if (lane >= o) {
-          inc_long += t0;
-          inc_rest += t1;
-        }
-      }
-      tt_long = __shfl(inc_long, 63);
-      tt = tt_long + __shfl(inc_rest, 63);
-      const uint64_t before = (1ull << lane) - 1;
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        if (which == j) {
-          seg_rank[j] = r;
-          // position / first tile inside this wave's entries of its own class; the other wave's and the other class's are added below
-          seg_pos[j] = long_k ? __popcll(has_long & before) : __popcll(has & ~has_long & before);
-          seg_first[j] = long_k ? inc_long - mine_tiles : inc_rest - mine_tiles;
-        }
-    }
-    if (lane == 0) {
-      s_cnt[r][wave] = tc;
-      s_til[r][wave] = tt;
-      s_cnt_long[r][wave] = tc_long;
-      s_til_long[r][wave] = tt_long;
-    }
-  }
-  __syncthreads();
-  if (wave == 1) {
-    first_row += s_tot[0][0];
-    inp_off += s_tot[1][0];
-    sc_off += s_tot[2][0];
-    out_off += s_tot[3][0];
-  }
-  first_row += s_base[0][0] + s_base[0][1];
-  inp_off += s_base[1][0] + s_base[1][1];
-  sc_off += s_base[2][0] + s_base[2][1];
-  out_off += s_base[3][0] + s_base[3][1];
-  if (mine) {
-    table[ge] = tag;
-    table[p.Et + ge] = first_row;
-    table[2 * p.Et + ge] = inp_off;
-    table[3 * p.Et + ge] = sc_off;
-    ptrs[ge] = p.inp + 2 * inp_off;
-    ptrs[p.Et + ge] = d.B;
-    ptrs[2 * p.Et + ge] = sld > 0 ? p.scale + 2 * sc_off : nullptr;
-    ptrs[3 * p.Et + ge] = d.scale_b;
-    ptrs[4 * p.Et + ge] = p.out + 2 * out_off;
-    sizes[ge] = mxmoe_dim3{(uint32_t)rows, (uint32_t)N, (uint32_t)K};
-    if (ge == p.E) misc[1] = (int64_t)(p.out + 2 * out_off);
-  }
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    if (seg_rank[j] >= 0) {
-      int pos = seg_pos[j], first = seg_first[j];
-      for (int r = 0; r < seg_rank[j]; ++r) {
-        pos += s_cnt[r][0] + s_cnt[r][1];
-        first += s_til[r][0] + s_til[r][1];
-      }
-      // inside the branch: [long-K entries of wave 0][of wave 1][other entries of wave 0][of wave 1]
-      const int r = seg_rank[j];
-      if (long_k) {
-        if (wave == 1) {
-          pos += s_cnt_long[r][0];
-          first += s_til_long[r][0];
-        }
-      } else {
-        pos += s_cnt_long[r][0] + s_cnt_long[r][1];
-        first += s_til_long[r][0] + s_til_long[r][1];
-        if (wave == 1) {
-          pos += s_cnt[r][0] - s_cnt_long[r][0];
-          first += s_til[r][0] - s_til_long[r][0];
-        }
-      }
-      fa->entry[pos] = FusedArgs::Entry{first, sg[j].row0, sg[j].rows, e | (sg[j].branch << 16)};  // problem index relative to the launch's first
-    }
-  }
-  if (e == 0) {
-    // rows routed = sum over the routed experts of every launch: the last launch knows them all
-    if (chunk == chunks - 1) misc[0] = s_base[4][0] + s_base[4][1] + s_routed[0] + s_routed[1];
-    if (chunk == 0 && p.Et == p.E) misc[1] = 0;
-    int total = 0, wg = 0, np = 0, ne = 0, flat = 0;
-    int last_tile0 = 0, last_wg0 = 0;  // of the phase being filled (kept here: reading them back from the table would wait for the store)
-    for (int r = 0; r < info.nb; ++r) {
-      const int tile0 = total;
-      total += s_til[r][0] + s_til[r][1];
-      ne += s_cnt[r][0] + s_cnt[r][1];
-      if (total == tile0) continue;
-      if (np < kMaxPhases) {  // shapes beyond the phase table share the last phase
-        fa->phase_tile0[np] = last_tile0 = tile0;
-        fa->phase_wg0[np] = last_wg0 = wg;
-        if (flat_phase(info.b[info.order[r]])) flat |= 1 << np;
-        ++np;
-      }
-      wg = last_wg0 + (total - last_tile0 + kNumXcd - 1) / kNumXcd * kNumXcd;
-    }
-    fa->phase_tile0[np] = total;
-    fa->phase_wg0[np] = wg;
-    if (np == 0) fa->phase_tile0[1] = fa->phase_wg0[1] = 0;  // a plan without tiles still holds one (empty) phase range
-    fa->num_phases = np;
-    fa->phase_flat = flat;
-    fa->num_entries = ne;
-    fa->total_tiles = total;
-    fa->problem_offset = e0;
-    fa->As = reinterpret_cast<const uint8_t* const*>(ptrs);
-    fa->Bs = reinterpret_cast<const uint8_t* const*>(ptrs + p.Et);
-    fa->sa = reinterpret_cast<const _Float16* const*>(ptrs + 2 * p.Et);
-    fa->sb = reinterpret_cast<const _Float16* const*>(ptrs + 3 * p.Et);
-    fa->Cs = reinterpret_cast<_Float16* const*>(const_cast<void**>(ptrs + 4 * p.Et));
-    fa->acc = nullptr;
-    fa->sizes = sizes;
-  }
-}
 
 __global__ void __launch_bounds__(kPlanThreads) plan_block_kernel(const PlanPair pair) {
   // one workgroup per launch of each block of the layer (gate_up, down): all only read the counts
@@ -391,7 +85,7 @@ __global__ void __launch_bounds__(kPlanThreads) perm_scatter_plan_kernel(const P
 }
 
 // Kernel for the formats of `h_desc`, checked once on the host: every problem's format has a branch and its shape fits it.
-static int resolve_kernel(int kernel_id, const mxmoe_block_desc* h_desc, int et) {
+int resolve_kernel(int kernel_id, const mxmoe_block_desc* h_desc, int et) {
   auto& reg = registry();
   auto covers = [&](const FusedKernel& k) {
     for (int i = 0; i < et; ++i) {
@@ -553,6 +247,7 @@ static int fill_plan_params(PlanParams& p, int kernel_id, const int64_t* d_recv,
   p.E = num_experts;
   p.Et = et;
   p.shared_rows = shared_rows;
+  p.form = LayerForm{};
   p.info = plan_of(registry()[kid]);
   return 0;
 }

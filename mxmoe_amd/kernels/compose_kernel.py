@@ -150,8 +150,11 @@ def build_kernel_source(tile_cfg, kname: str, kernel_type: KernelType = KernelTy
     pairs = [(q, t) for q, item in tile_cfg.items() for t in _flat([item])]
     tiles = ", ".join(t.cpp_type() for _, t in pairs)
     comment = "; ".join(f"{q} if {BRANCH_CONDITION_MAP[q]} -> {t.to_str()}" for q, t in pairs)
+    # the library's own fused kernels also carry their tiles' gate_up form, which the layer forward launches (bf6 and bf16 tiles have none)
+    layer = deferred and kernel_type == KernelType.Fused and not any(t.is_bf6() or q == "bf16" for q, t in pairs)
     defn = (KERNEL_DEFERRED_TEMPLATE if deferred else KERNEL_DEFINITION_TEMPLATE).substitute(KernelName=kname, Tiles=tiles, Comment=comment, Policy=POLICY[str(kernel_type)],
-                                                                                                  Hint=f", {max_rows_hint}" if max_rows_hint else "")
+                                                                                                  Hint=f", {max_rows_hint}" if max_rows_hint else "",
+                                                                                                  Register="register_layer_kernel" if layer else "register_fused")
     decl = f"//   {kname}: " + ", ".join(f"[{q}: ({t.BM},{t.BN},{t.BK}) ({t.WM},{t.WN},{t.WK}) {t.STAGE}]" for q, t in pairs)
     return decl, defn
 

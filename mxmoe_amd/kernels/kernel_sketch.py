@@ -29,7 +29,7 @@ KERNEL_DEFERRED_TEMPLATE = Template("""// generated by mxmoe_amd.kernels.compose
 #include "mxmoe_launch.hpp"
 
 namespace mxmoe {
-int register_${KernelName}() { return register_fused<${Tiles}>("${KernelName}", ${Policy}${Hint}); }
+int register_${KernelName}() { return ${Register}<${Tiles}>("${KernelName}", ${Policy}${Hint}); }
 }  // namespace mxmoe
 """)
 

@@ -131,6 +131,28 @@ class MxMoELayer:
         return self._static
 
     # ---- the forward that never waits for its routing ---------------------------------------------------------
+    def _block_descs(self, qps, ns, ks, ws, bf6: bool):
+        """Host-side block descriptors of one linear block, one per expert (the shared one last)."""
+        h = (_lib.BlockDesc * len(ws))()
+        for e, w in enumerate(ws):
+            a, wb, g, sym = qps[e]
+            variant = 1 if bf6 and (int(a), int(wb), int(g)) == (4, 4, -1) else (2 if self.fp8 and (int(a), int(wb), int(g)) == (8, 8, -1) else 0)
+            layout = (C.c_uint8 * 3)(variant, 0, 0)  # operand variant: 1 activations as bf6 fragments, 2 fp8 e4m3 codes
+            h[e] = _lib.BlockDesc(int(a), int(wb), int(g), 1 if sym else 0, layout, int(ns[e]), int(ks[e]), w.data.data_ptr(), 0 if w.scale is None else w.scale.data_ptr())
+        return h
+
+    def _planned_kernel(self, h, t: int, topk: int) -> int:
+        """The kernel that a block's planned launch runs on for t tokens."""
+        lib, et = _lib.load(), len(h)
+        kid = lib.mxmoe_plan_select_kernel(-1, h, et)
+        if kid < 0:
+            raise RuntimeError(lib.mxmoe_last_error().decode())
+        if t <= 64 and t * topk <= 12 * self.cfg.num_experts:  # few tokens, and on average well under one 16-row tile per expert: a kernel made of 16-row few-token tiles alone, if one covers the formats
+            few = lib.mxmoe_find_kernel(b"groupgemm_hz_fused_wo_skinny")
+            if few >= 0 and lib.mxmoe_plan_select_kernel(few, h, et) == few:
+                kid = few
+        return kid
+
     def _planned_setup(self, t: int, topk: int):
         """Everything of the planned forward that depends only on the layer and on (tokens, top-k): block descriptors on both sides,
         kernels, worst-case grids, plan buffers, and the stores sized for the worst case.  Built once and reused."""
@@ -150,21 +172,9 @@ class MxMoELayer:
             return torch.empty(max(int(n), 16), dtype=torch.uint8, device=dev)
 
         def block(qps, ns, ks, ws, bf6):
-            h = (_lib.BlockDesc * et)()
-            for e in range(et):
-                a, w, g, sym = qps[e]
-                variant = 1 if bf6 and (int(a), int(w), int(g)) == (4, 4, -1) else (2 if self.fp8 and (int(a), int(w), int(g)) == (8, 8, -1) else 0)
-                layout = (C.c_uint8 * 3)(variant, 0, 0)  # operand variant: 1 activations as bf6 fragments, 2 fp8 e4m3 codes
-                h[e] = _lib.BlockDesc(int(a), int(w), int(g), 1 if sym else 0, layout, int(ns[e]), int(ks[e]), ws[e].data.data_ptr(),
-                                      0 if ws[e].scale is None else ws[e].scale.data_ptr())
+            h = self._block_descs(qps, ns, ks, ws, bf6)
             d = torch.frombuffer(bytearray(bytes(h)), dtype=torch.uint8).to(dev)
-            kid = lib.mxmoe_plan_select_kernel(-1, h, et)
-            if kid < 0:
-                raise RuntimeError(lib.mxmoe_last_error().decode())
-            if t <= 64 and t * topk <= 12 * e_cnt:  # few tokens, and on average well under one 16-row tile per expert: a kernel made of 16-row few-token tiles alone, if one covers the formats
-                few = lib.mxmoe_find_kernel(b"groupgemm_hz_fused_wo_skinny")
-                if few >= 0 and lib.mxmoe_plan_select_kernel(few, h, et) == few:
-                    kid = few
+            kid = self._planned_kernel(h, t, topk)
             grid = lib.mxmoe_plan_grid_bound(kid, h, e_cnt, r_cap, shared_rows)
             if grid < 0:
                 raise RuntimeError(lib.mxmoe_last_error().decode())
@@ -211,6 +221,73 @@ class MxMoELayer:
         cache[key] = ps
         return ps
 
+    def _short_setup(self, t: int, topk: int):
+        """The short form of the planned forward for (tokens, top-k): a handle of `mxmoe_layer_create` with the buffers it names, or None
+        when the library does not take the layer in that form (row length, bf6 operands).  Built once and reused."""
+        cache = self.__dict__.setdefault("_short", {})
+        key = (t, topk)
+        if key in cache:
+            return cache[key]
+        cfg, dev, lib = self.cfg, self.device, _lib.load()
+        e_cnt, has_shared, et = cfg.num_experts, cfg.num_shared > 0, self.n_exp_total
+        if self.bf6_gate_up or self.bf6_down:
+            cache[key] = None
+            return None
+        r_cap, shared_rows, i_sh = t * topk, t if has_shared else 0, cfg.inter * max(cfg.num_shared, 1)
+        sh = [i_sh] if has_shared else []
+        gate_up = self._block_descs(self.qp_gate_up, [2 * cfg.inter] * e_cnt + [2 * n for n in sh], [cfg.hidden] * et, self.w13, False)
+        down = self._block_descs(self.qp_down, [cfg.hidden] * et, [cfg.inter] * e_cnt + sh, self.w2, False)
+        d = _lib.LayerDesc(num_tokens=t, topk=topk, num_experts=e_cnt, has_shared=int(has_shared), hidden=cfg.hidden, inter=cfg.inter, inter_shared=i_sh, rotate=cfg.rotate,
+                           had_k=1, had_f=1, h_gate_up=C.cast(gate_up, C.c_void_p), h_down=C.cast(down, C.c_void_p))
+        d.kernel_gate_up, d.kernel_down = self._planned_kernel(gate_up, t, topk), self._planned_kernel(down, t, topk)
+        if not lib.mxmoe_layer_supported(C.byref(d)):
+            cache[key] = None
+            return None
+        grids = [lib.mxmoe_plan_grid_bound(k, h, e_cnt, r_cap, shared_rows) for k, h in ((d.kernel_gate_up, gate_up), (d.kernel_down, down))]
+        if min(grids) < 0:
+            raise RuntimeError(lib.mxmoe_last_error().decode())
+        d.grid_gate_up, d.grid_down = grids
+        if cfg.rotate:
+            d.had_k, d.had_f, signs = device_signs(cfg.inter, dev)
+            d.had_signs = None if signs is None else signs.data_ptr()
+            if has_shared and device_signs(i_sh, dev)[0] != d.had_k:
+                raise RuntimeError("routed and shared intermediate sizes need the same Hadamard order")
+        keep = []
+
+        def buf(n, dtype=torch.uint8):
+            b = torch.empty(max(int(n), 16), dtype=dtype, device=dev)
+            keep.append(b)
+            return b.data_ptr()
+
+        for tag in {ops.act_tag(int(q[0]), int(q[2]), False, self.fp8 and int(q[1]) == 8) for q in self.qp_gate_up}:
+            if tag == 0 and cfg.rotate != 2:
+                continue  # (the launch reads the tokens where they are)
+            d.token_store[tag] = buf(2 * ops.packed_elems(tag, t, cfg.hidden))
+            d.token_scales[tag] = buf(2 * t * (cfg.hidden // 128 if tag == 3 else 1))
+        # the rows the second block reads: packed, every routed row as wide as the widest routed expert's
+        tags = [ops.act_tag(int(q[0]), int(q[2]), False, self.fp8 and int(q[1]) == 8) for q in self.qp_down]
+        packed = [0 if tg == 0 and cfg.rotate != 2 else ops.packed_elems(tg, 1, k) for tg, k in zip(tags, [cfg.inter] * e_cnt + sh)]
+        scales = [0 if tg == 0 else (k // 128 if tg == 3 else 1) for tg, k in zip(tags, [cfg.inter] * e_cnt + sh)]
+        # (the planner's offsets count fp16 rows too, whether or not anybody writes them: room for the widest of all)
+        wide = [ops.packed_elems(tg, 1, k) for tg, k in zip(tags, [cfg.inter] * e_cnt + sh)] if any(packed) else [0] * et
+        d.down_inp = buf(2 * (max(wide[:e_cnt]) * r_cap + sum(wide[e_cnt:]) * shared_rows))
+        d.down_scales = buf(2 * (max(scales[:e_cnt]) * r_cap + sum(scales[e_cnt:]) * shared_rows))
+        d.act = buf(2 * (cfg.inter * r_cap + sum(sh) * shared_rows))
+        d.down_out = buf(2 * cfg.hidden * (r_cap + shared_rows))
+        d.plan_gate_up, d.plan_down = buf(lib.mxmoe_plan_bytes(et)), buf(lib.mxmoe_plan_bytes(et))
+        d.dst_exp, d.token_of_row, d.row_of_slot = (buf(r_cap, torch.int32) for _ in range(3))
+        d.recv = buf(e_cnt, torch.int64)
+        d.workspace = buf(lib.mxmoe_permute_workspace_bytes(r_cap, e_cnt))
+        keep.append(torch.arange(max(t, 16), dtype=torch.int32, device=dev))
+        d.iota = keep[-1].data_ptr()
+        for name, h in (("d_gate_up", gate_up), ("d_down", down)):
+            keep.append(torch.frombuffer(bytearray(bytes(h)), dtype=torch.uint8).to(dev))
+            setattr(d, name, keep[-1].data_ptr())
+        handle = C.c_void_p()
+        _lib.check(lib, lib.mxmoe_layer_create(C.byref(d), C.byref(handle)))
+        cache[key] = _ShortForward(lib, handle, keep)
+        return cache[key]
+
     def __call__(self, hidden: torch.Tensor, topk_ids: torch.Tensor, topk_weights: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
         """The whole MoE MLP, `(hidden [T, K] fp16, topk_ids [T, k] int32, topk_weights [T, k] fp32) -> [T, K] fp16`: what a serving
         framework's fused-MoE operator computes after routing (permute, quantise, gate_up, SiLU * up, down, un-permute + combine).
@@ -218,22 +295,27 @@ class MxMoELayer:
         Same kernels and results as `forward` + `combine`, but nothing here waits for the routing: the tables of both launches are
         derived from the tokens-per-expert counts by a planning kernel on the device (`mxmoe_plan_layer`: both blocks in one launch), the stores and plan
         buffers are allocated once per (tokens, top-k) for the worst case, and every launch argument is independent of the data.
-        The call only enqueues six kernels (seven when more than 256 (token, slot) pairs are permuted, nine beyond what `mxmoe_permute_plan_layer_ws` takes; no synchronisation, no allocation after the first call when `out` is given), so it can
+        The call only enqueues four or five kernels (`mxmoe_layer_run`; six to nine, in separate calls, for the layers that form does
+        not take: rows that are not a power of two, bf6 operands); no synchronisation, no allocation after the first call when `out` is given, so it can
         be captured into a HIP graph.  Intermediate buffers belong to the layer and are reused by the next call of the same shape."""
         cfg, dev = self.cfg, self.device
-        lib = _lib.load()
         hidden = hidden.to(dev).contiguous()
-        ids = topk_ids.to(dev).to(torch.int32).contiguous()
-        w = topk_weights.to(dev).to(torch.float32).contiguous()
+        ids = topk_ids.to(dev, torch.int32).contiguous()
+        w = topk_weights.to(dev, torch.float32).contiguous()
         t, k_hid = hidden.shape
         topk = ids.shape[1]
         assert hidden.dtype == torch.float16 and k_hid == cfg.hidden and w.shape == ids.shape
-        e_cnt, has_shared = cfg.num_experts, int(cfg.num_shared > 0)
-        ps = self._planned_setup(t, topk)
-        b1, b2 = ps["b1"], ps["b2"]
         stream = torch.cuda.current_stream().cuda_stream
         final = out if out is not None else torch.empty((t, cfg.hidden), dtype=torch.float16, device=dev)
         assert final.shape == (t, cfg.hidden) and final.dtype == torch.float16 and final.is_contiguous()
+        short = self._short_setup(t, topk)
+        if short is not None:
+            short.run(hidden.data_ptr(), ids.data_ptr(), w.data_ptr(), final.data_ptr(), stream)
+            return final
+        lib = _lib.load()
+        e_cnt, has_shared = cfg.num_experts, int(cfg.num_shared > 0)
+        ps = self._planned_setup(t, topk)
+        b1, b2 = ps["b1"], ps["b2"]
         ck = lambda rc: _lib.check(lib, rc)  # noqa: E731
         if ps["r_cap"] <= 256:  # decode-sized batch: permutation and planning in one launch
             ck(lib.mxmoe_permute_plan_layer(ids.data_ptr(), t, topk, e_cnt, ps["dst"].data_ptr(), ps["perm"].data_ptr(), ps["slot"].data_ptr(), ps["recv"].data_ptr(),
@@ -271,12 +353,12 @@ class MxMoELayer:
         t = hidden.shape[0]
         topk = self.cfg.topk if topk is None else topk
         assert router_logits.shape == (t, self.cfg.num_experts)
-        ps = self._planned_setup(t, topk)
-        if "route_ids" not in ps:
-            ps["route_ids"] = torch.empty((t, topk), dtype=torch.int32, device=self.device)
-            ps["route_w"] = torch.empty((t, topk), dtype=torch.float32, device=self.device)
-        ops.route_topk(router_logits.to(self.device), topk, renormalise, out_ids=ps["route_ids"], out_weights=ps["route_w"])
-        return self(hidden, ps["route_ids"], ps["route_w"], out=out)
+        route = self.__dict__.setdefault("_route", {})
+        if (t, topk) not in route:
+            route[t, topk] = (torch.empty((t, topk), dtype=torch.int32, device=self.device), torch.empty((t, topk), dtype=torch.float32, device=self.device))
+        ids, w = route[t, topk]
+        ops.route_topk(router_logits.to(self.device), topk, renormalise, out_ids=ids, out_weights=w)
+        return self(hidden, ids, w, out=out)
 
     def capture(self, tokens: int, topk: int | None = None, logits_dtype: torch.dtype | None = None, renormalise: bool = False) -> "CapturedForward":
         """The planned forward for a fixed (tokens, top-k) shape, captured into a HIP graph: write the inputs into the returned
@@ -384,6 +466,22 @@ class MxMoELayer:
                 c += 2 * m * n
             out[name] = {"weights": w, "activations": a, "outputs": c, "total": w + a + c}
         return out
+
+
+class _ShortForward:
+    """A handle of `mxmoe_layer_create`, the buffers it names, and its release."""
+
+    def __init__(self, lib, handle, keep):
+        self._lib, self._handle, self._keep = lib, handle, keep
+        self._run = lib.mxmoe_layer_run
+
+    def run(self, hidden, ids, weights, out, stream):
+        rc = self._run(self._handle, hidden, ids, weights, out, stream)
+        if rc:
+            _lib.check(self._lib, rc)
+
+    def __del__(self):
+        self._lib.mxmoe_layer_destroy(self._handle)
 
 
 class CapturedForward:

@@ -1,0 +1,88 @@
+"""The short form of the planned forward (mxmoe_layer_run: one head launch, rows gathered by token, silu(gate) * up as gate_up's output)
+against the forward with host tables and stored gate_up rows: identical outputs."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+W8A16 = (16, 8, 128, False)
+
+
+def _layer(tokens, topk, formats, hidden=512, inter=1408, num_shared=1, rotate=1, fp8=False):
+    from mxmoe_amd import synth
+    from mxmoe_amd.layer import MxMoELayer
+
+    n = len(formats) - (1 if num_shared else 0)
+    cfg = synth.MoEConfig("t", "test", n, topk, hidden, inter, tokens, num_shared=num_shared, rotate=rotate)
+    return cfg, MxMoELayer(cfg, formats=formats, fp8=fp8)
+
+
+def _check(cfg, layer, drop=True):
+    from mxmoe_amd import synth
+
+    assert layer._short_setup(cfg.tokens, cfg.topk) is not None
+    hidden = synth.make_hidden(cfg)
+    ids, w = synth.make_routing(cfg)
+    if drop:
+        ids[0, 0] = cfg.num_experts + 2
+        ids[cfg.tokens // 2, cfg.topk - 1] = -1
+    got = layer(hidden, ids, w)
+    want = layer.call_with_host_tables(hidden, ids, w)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    again = layer(hidden, ids, w)                                       # (buffers of the previous call)
+    assert torch.equal(again, want)
+
+
+# tokens: one row, the edges of the 16 / 32 / 64 / 128-row tiles over a few experts, and past one chunk of 256 permuted entries
+@pytest.mark.parametrize("tokens", [1, 2, 31, 33, 129, 700])
+@pytest.mark.parametrize("mix", ["wxax", "wo", "fp16", "all", "fp8"])
+def test_short_forward_equals_the_forward_with_host_tables(tokens, mix):
+    from mxmoe_amd import synth as S
+
+    fm = {"wxax": [(S.W4A4, S.W8A8), (S.W8A8, S.W4A4), (S.W4A4, S.W4A4), (S.W8A8, S.W8A8)],
+          "wo": [(S.W4A16, S.W3A16), (S.W3A16, S.W2A16), (S.W2A16, S.W4A16), (S.W4A16, S.W4A16)],
+          "fp16": [(S.FP16, S.FP16)] * 4,
+          "all": [(S.W4A4G128, S.W4A16), (S.FP16, S.W8A8), (W8A16, S.W4A4G128), (S.W4A4, S.FP16), (S.W8A8, W8A16), (S.W2A16, S.W4A4), (S.W4A16, S.W2A16)],
+          "fp8": [(S.W8A8, S.W8A8), (S.W4A4, S.W8A8), (S.W8A8, S.W4A4), (S.W8A8, S.W8A8)]}[mix]
+    cfg, layer = _layer(tokens, 2, fm, fp8=mix == "fp8")
+    _check(cfg, layer, drop=tokens > 1)
+
+
+@pytest.mark.parametrize("hidden,inter,num_shared,rotate", [(1024, 224, 0, 2), (2048, 64, 2, 0), (4096, 96, 1, 0), (512, 32, 0, 0)])
+def test_short_forward_row_lengths_and_rotations(hidden, inter, num_shared, rotate):
+    """Every row length of the head's token kernel; intermediate sizes that end inside a tile's gate half."""
+    from mxmoe_amd import synth as S
+
+    if inter % 128 == 0 or rotate:
+        fm = [(S.W4A4, S.FP16), (S.W8A8, S.FP16), (S.FP16, S.FP16), (S.W4A4G128, S.FP16), (S.W4A16, S.FP16)]
+    else:
+        fm = [(S.W4A16, S.FP16), (S.W8A8, S.FP16), (S.FP16, S.FP16), (S.W4A4, S.FP16), (S.W3A16, S.FP16)]
+    cfg, layer = _layer(70, 3, fm, hidden=hidden, inter=inter, num_shared=num_shared, rotate=rotate)
+    _check(cfg, layer)
+
+
+def test_short_forward_of_more_experts_than_one_launch_holds():
+    from mxmoe_amd import synth as S
+
+    cfg, layer = _layer(300, 3, [((S.W4A4, S.W8A8), (S.W8A8, S.FP16), (S.FP16, S.W4A4))[i % 3] for i in range(131)], inter=512)
+    _check(cfg, layer)
+
+
+def test_short_forward_counts_ids_in_a_launch_of_its_own():
+    """More than 65536 (token, slot) entries: the per-chunk counting launch in front of the head."""
+    from mxmoe_amd import synth as S
+
+    cfg, layer = _layer(33001, 2, [(S.W4A4, S.FP16), (S.W8A8, S.W4A16), (S.FP16, S.FP16), (S.W4A16, S.FP16)], inter=128, num_shared=0, rotate=0)
+    _check(cfg, layer)
+
+
+def test_layers_the_short_form_does_not_take():
+    from mxmoe_amd import synth as S
+
+    for hidden in (256, 1536):                                          # rows below 512 values, or no power of two
+        cfg, layer = _layer(20, 2, [(S.FP16, S.FP16)] * 3, hidden=hidden, num_shared=0, rotate=0)
+        assert layer._short_setup(cfg.tokens, cfg.topk) is None
+        hidden_t = S.make_hidden(cfg)
+        ids, w = S.make_routing(cfg)
+        assert torch.equal(layer(hidden_t, ids, w), layer.call_with_host_tables(hidden_t, ids, w))
