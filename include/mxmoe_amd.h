@@ -274,6 +274,16 @@ int mxmoe_unpermute_combine_planned(const void* down_out, const void* d_plan_dow
 int mxmoe_combine_planned(const void* down_out, const void* d_plan_down, int num_problems, const float* topk_weights, const int32_t* row_of_slot, int num_tokens,
                           int topk, int K, void* out, void* stream);
 
+/* mxmoe_unpermute_combine when the permutation delivered the inverse map (mxmoe_build_permutation_inv) and the tokens-per-expert counts
+ * are in DEVICE memory: one launch, no workspace, and the caller need not know how many rows were routed.  down_out holds the routed
+ * rows in sorted order followed, with has_shared, by the shared expert's num_tokens rows. */
+int mxmoe_combine_sorted(const void* down_out, const int64_t* recv_tokens_per_exp, int num_experts, int has_shared, const float* topk_weights,
+                         const int32_t* row_of_slot, int num_tokens, int topk, int K, void* out, void* stream);
+
+/* Copies `bytes` bytes from host memory to device memory on `stream`, in kernel arguments (about 3.5 KB per launch; meant for tables of
+ * a few KB): the host array may be changed or freed as soon as the call returns, and the call waits for nothing. */
+int mxmoe_upload(void* dst, const void* host_src, size_t bytes, void* stream);
+
 /* ---- the planned forward in its short form ----
  *
  * One call enqueues the whole forward of one layer for one (tokens, top-k): permutation, planning and the quantisation of every

@@ -4,6 +4,8 @@ from __future__ import annotations
 import ctypes as C
 from pathlib import Path
 
+import torch
+
 LIB_PATH = Path(__file__).resolve().parent / "libmxmoe_amd.so"
 
 
@@ -79,6 +81,8 @@ SIGNATURES = {
     "mxmoe_unpermute_combine_planned": (_I, [_P, _P, _I, _P, _P, _I, _I, _I, _P, _P, _P]),
     "mxmoe_group_gemm_plan_tables": (_I, [_I, C.POINTER(Dim3), C.POINTER(QParams), _I, C.POINTER(C.c_int32), _I]),
     "mxmoe_group_gemm_plan_tile_map": (_I, [_I, C.POINTER(Dim3), C.POINTER(QParams), _I, _I, C.POINTER(C.c_int32)]),
+    "mxmoe_upload": (_I, [_P, _P, C.c_size_t, _P]),
+    "mxmoe_combine_sorted": (_I, [_P, _P, _I, _I, _P, _P, _I, _I, _I, _P, _P]),
     "mxmoe_layer_supported": (_I, [_P]),
     "mxmoe_layer_create": (_I, [_P, C.POINTER(_P)]),
     "mxmoe_layer_destroy": (None, [_P]),
@@ -124,6 +128,11 @@ def load(path: str | Path | None = None) -> C.CDLL:
         fn.argtypes = args
     _cached[key] = _cached[str(p)] = lib
     return lib
+
+
+def current_stream() -> int:
+    """Handle of torch's current stream on the current device (torch.cuda.current_stream().cuda_stream without the Stream object)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def check(lib: C.CDLL, rc: int) -> None:

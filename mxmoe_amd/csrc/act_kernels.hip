@@ -1723,35 +1723,91 @@ __global__ void combine_invert_kernel(const int64_t* __restrict__ src_slot, int 
     if (sl >= 0 && sl < slots) row_of_slot[sl] = r;
   }
 }
+struct CombineArgs {
+  const _Float16* down;
+  // the shared expert's rows: at `shared`, or (planned launches) where *shared_addr says (0: none), or behind the routed rows of `down`,
+  // whose number is the sum of recv[0 .. E-1]; all null: no shared expert
+  const _Float16* shared;
+  const int64_t* shared_addr;
+  const int64_t* recv;
+  int E;
+  const float* weights;        // [T][topk]
+  const int32_t* row_of_slot;  // [T][topk], negative: dropped
+  int topk, K;
+  _Float16* out;
+};
 // One workgroup per token: out[t] = half( sum_k w[t,k] * float(down[row(t,k)])  (k ascending, fp32: product rounded, then the
 // sum rounded)  + float(shared[t]) ).  Pure streaming: every down row is read once, 16 bytes per lane.
-__global__ void __launch_bounds__(256) combine_kernel(const _Float16* __restrict__ down, const _Float16* __restrict__ shared, const float* __restrict__ weights,
-                                                      const int32_t* __restrict__ row_of_slot, int topk, int K, _Float16* __restrict__ out,
-                                                      const int64_t* __restrict__ shared_addr) {
-  const int t = blockIdx.x;
-  if (shared_addr) shared = reinterpret_cast<const _Float16*>(*shared_addr);  // planned mode: where the planner put the shared expert's rows (0: none)
+__global__ void __launch_bounds__(256) combine_kernel(const CombineArgs a) {
+  const int t = blockIdx.x, lane = threadIdx.x & 63;
+  const int topk = a.topk, K = a.K;
+  const _Float16* shared = a.shared;
+  if (a.shared_addr) shared = reinterpret_cast<const _Float16*>(const_load(a.shared_addr));
+  if (a.recv) {
+    long rows = 0;
+    for (int e = lane; e < a.E; e += 64) rows += (long)a.recv[e];
+    shared = a.down + wave_last(wave_inclusive_scan(rows)) * K;
+  }
+  // up to kSlots slots of the token at a time: their rows and weights in scalar registers, then all their loads in flight together
+  // (one row after the other costs a trip to memory each, which is what a small batch's combine consists of)
+  constexpr int kSlots = 8;
   for (int c = threadIdx.x * 8; c < K; c += 256 * 8) {
+    v8h sh{};
+    if (shared) sh = gload<v8h>(shared + (size_t)t * K + c);
     float acc[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
-    for (int k = 0; k < topk; ++k) {
-      const int r = row_of_slot[t * topk + k];
-      if (r < 0) continue;
-      const float w = weights[t * topk + k];
-      const v8h v = *reinterpret_cast<const v8h*>(down + (size_t)r * K + c);
+    for (int k0 = 0; k0 < topk; k0 += kSlots) {
+      int r[kSlots];
+      v8h v[kSlots];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] = acc[e] + w * (float)v[e];
+      for (int i = 0; i < kSlots; ++i) r[i] = k0 + i < topk ? const_load(a.row_of_slot + t * topk + k0 + i) : -1;
+#pragma unroll
+      for (int i = 0; i < kSlots; ++i)
+        if (r[i] >= 0) v[i] = gload<v8h>(a.down + (size_t)r[i] * K + c);
+#pragma unroll
+      for (int i = 0; i < kSlots; ++i)
+        if (r[i] >= 0) {
+          const float w = const_load(a.weights + t * topk + k0 + i);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[e] = acc[e] + w * (float)v[i][e];
+        }
     }
     v8h o;
     if (shared) {
-      const v8h v = *reinterpret_cast<const v8h*>(shared + (size_t)t * K + c);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] = acc[e] + (float)v[e];
+      for (int e = 0; e < 8; ++e) acc[e] = acc[e] + (float)sh[e];
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = (_Float16)keep_f32(acc[e]);
-    *reinterpret_cast<v8h*>(out + (size_t)t * K + c) = o;
+    *reinterpret_cast<v8h*>(a.out + (size_t)t * K + c) = o;
   }
+}
+
+static int launch_combine(CombineArgs a, const float* weights, const int32_t* row_of_slot, int num_tokens, int topk, int K, void* out, void* stream) {
+  a.weights = weights;
+  a.row_of_slot = row_of_slot;
+  a.topk = topk;
+  a.K = K;
+  a.out = reinterpret_cast<_Float16*>(out);
+  hipLaunchKernelGGL(combine_kernel, dim3(num_tokens), dim3(256), 0, (hipStream_t)stream, a);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    last_error() = std::string("kernel launch failed: ") + hipGetErrorString(e);
+    return 4;
+  }
+  return 0;
+}
+
+// Bytes that travel in the kernel arguments.
+struct UploadArgs {
+  static constexpr int kWords = 896;
+  uint32_t* dst;
+  int words;
+  uint32_t w[kWords];
+};
+__global__ void __launch_bounds__(256) upload_kernel(const UploadArgs a) {
+  for (int i = threadIdx.x; i < a.words; i += 256) a.dst[i] = a.w[i];
 }
 
 extern "C" {
@@ -2128,6 +2184,34 @@ int quant_rows_behind(const RowsBehind& b, hipStream_t stream) {
 }  // namespace mxmoe
 extern "C" {
 
+int mxmoe_upload(void* dst, const void* host_src, size_t bytes, void* stream) {
+  if (bytes == 0) return 0;
+  if (!dst || !host_src) {
+    last_error() = "null pointer";
+    return 5;
+  }
+  if (bytes % 4 || (reinterpret_cast<uintptr_t>(dst) & 3)) {
+    last_error() = "uploads are whole 4-byte words";
+    return 3;
+  }
+  const uint8_t* src = reinterpret_cast<const uint8_t*>(host_src);
+  for (size_t at = 0; at < bytes;) {
+    UploadArgs a;
+    const size_t n = std::min(bytes - at, sizeof a.w);
+    a.dst = reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(dst) + at);
+    a.words = (int)(n / 4);
+    std::memcpy(a.w, src + at, n);
+    hipLaunchKernelGGL(upload_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+      last_error() = std::string("kernel launch failed: ") + hipGetErrorString(e);
+      return 4;
+    }
+    at += n;
+  }
+  return 0;
+}
+
 size_t mxmoe_combine_workspace_bytes(int num_tokens, int topk) { return (size_t)num_tokens * topk * sizeof(int32_t); }
 
 int mxmoe_unpermute_combine(const void* down_out, const void* shared_out, const float* topk_weights, const int64_t* src_slot, int rows, int num_tokens, int topk,
@@ -2145,14 +2229,10 @@ int mxmoe_unpermute_combine(const void* down_out, const void* shared_out, const 
   int32_t* row_of_slot = reinterpret_cast<int32_t*>(workspace);
   hipLaunchKernelGGL(combine_fill_kernel, dim3((slots + 255) / 256), dim3(256), 0, s, row_of_slot, slots);
   if (rows > 0) hipLaunchKernelGGL(combine_invert_kernel, dim3((rows + 255) / 256), dim3(256), 0, s, src_slot, rows, slots, row_of_slot, (const int64_t*)nullptr);
-  hipLaunchKernelGGL(combine_kernel, dim3(num_tokens), dim3(256), 0, s, reinterpret_cast<const _Float16*>(down_out), reinterpret_cast<const _Float16*>(shared_out),
-                     topk_weights, row_of_slot, topk, K, reinterpret_cast<_Float16*>(out), (const int64_t*)nullptr);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) {
-    last_error() = std::string("kernel launch failed: ") + hipGetErrorString(e);
-    return 4;
-  }
-  return 0;
+  CombineArgs a{};
+  a.down = reinterpret_cast<const _Float16*>(down_out);
+  a.shared = reinterpret_cast<const _Float16*>(shared_out);
+  return launch_combine(a, topk_weights, row_of_slot, num_tokens, topk, K, out, stream);
 }
 
 int mxmoe_combine_planned(const void* down_out, const void* d_plan_down, int num_problems, const float* topk_weights, const int32_t* row_of_slot, int num_tokens,
@@ -2166,14 +2246,27 @@ int mxmoe_combine_planned(const void* down_out, const void* d_plan_down, int num
     return 5;
   }
   const int64_t* misc = reinterpret_cast<const int64_t*>(reinterpret_cast<const uint8_t*>(d_plan_down) + mxmoe::PlanLayout(num_problems).misc);
-  hipLaunchKernelGGL(combine_kernel, dim3(num_tokens), dim3(256), 0, (hipStream_t)stream, reinterpret_cast<const _Float16*>(down_out), (const _Float16*)nullptr, topk_weights,
-                     row_of_slot, topk, K, reinterpret_cast<_Float16*>(out), misc + 1);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) {
-    last_error() = std::string("kernel launch failed: ") + hipGetErrorString(e);
-    return 4;
+  CombineArgs a{};
+  a.down = reinterpret_cast<const _Float16*>(down_out);
+  a.shared_addr = misc + 1;
+  return launch_combine(a, topk_weights, row_of_slot, num_tokens, topk, K, out, stream);
+}
+
+int mxmoe_combine_sorted(const void* down_out, const int64_t* recv_tokens_per_exp, int num_experts, int has_shared, const float* topk_weights,
+                         const int32_t* row_of_slot, int num_tokens, int topk, int K, void* out, void* stream) {
+  if (num_tokens <= 0 || topk <= 0 || K <= 0 || K % 8 || num_experts <= 0) {
+    last_error() = "bad combine size (K must be a multiple of 8)";
+    return 3;
   }
-  return 0;
+  if (!down_out || !recv_tokens_per_exp || !topk_weights || !row_of_slot || !out) {
+    last_error() = "null pointer";
+    return 5;
+  }
+  CombineArgs a{};
+  a.down = reinterpret_cast<const _Float16*>(down_out);
+  a.recv = has_shared ? recv_tokens_per_exp : nullptr;
+  a.E = num_experts;
+  return launch_combine(a, topk_weights, row_of_slot, num_tokens, topk, K, out, stream);
 }
 
 int mxmoe_unpermute_combine_planned(const void* down_out, const void* d_plan_down, int num_problems, const float* topk_weights, const int64_t* src_slot, int num_tokens,
@@ -2192,14 +2285,10 @@ int mxmoe_unpermute_combine_planned(const void* down_out, const void* d_plan_dow
   int32_t* row_of_slot = reinterpret_cast<int32_t*>(workspace);
   hipLaunchKernelGGL(combine_fill_kernel, dim3((slots + 255) / 256), dim3(256), 0, s, row_of_slot, slots);
   hipLaunchKernelGGL(combine_invert_kernel, dim3((slots + 255) / 256), dim3(256), 0, s, src_slot, slots, slots, row_of_slot, misc);
-  hipLaunchKernelGGL(combine_kernel, dim3(num_tokens), dim3(256), 0, s, reinterpret_cast<const _Float16*>(down_out), (const _Float16*)nullptr, topk_weights, row_of_slot,
-                     topk, K, reinterpret_cast<_Float16*>(out), misc + 1);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) {
-    last_error() = std::string("kernel launch failed: ") + hipGetErrorString(e);
-    return 4;
-  }
-  return 0;
+  CombineArgs a{};
+  a.down = reinterpret_cast<const _Float16*>(down_out);
+  a.shared_addr = misc + 1;
+  return launch_combine(a, topk_weights, row_of_slot, num_tokens, topk, K, out, stream);
 }
 
 }  // extern "C"

@@ -7,11 +7,27 @@ every launch (the reference re-allocates and re-copies them on every call, ref_b
 from __future__ import annotations
 
 import ctypes as C
+from functools import lru_cache
 
+import numpy as np
 import torch
 
 from . import _lib
 from .weights import PackedWeight  # noqa: F401  (re-export for callers)
+
+
+@lru_cache(maxsize=64)
+def _qparams_array(qparams: tuple) -> np.ndarray:
+    return np.array([(int(a), int(w), int(g), 1 if s else 0) for (a, w, g, s) in qparams], np.int32)
+
+
+def _upload(host: np.ndarray, device) -> torch.Tensor:
+    """`host` (contiguous) as a device tensor of bytes.  The bytes travel in kernel arguments (mxmoe_upload): unlike a copy from pageable
+    memory, which first waits for everything enqueued on the stream, the host goes on at once."""
+    d = torch.empty(max(host.nbytes, 8), dtype=torch.uint8, device=device)
+    lib = _lib.load()
+    _lib.check(lib, lib.mxmoe_upload(d.data_ptr(), host.ctypes.data, host.nbytes, _lib.current_stream()))
+    return d
 
 
 class GroupGemmLaunch:
@@ -26,30 +42,35 @@ class GroupGemmLaunch:
         self._keep = (As, Bs, scale_a, scale_b, Cs, acc)  # keep the tensors alive
         dev = Cs[0].device if p else torch.device("cuda")
 
-        def ptrs(ts):
-            return [0 if t is None or t.numel() == 0 else t.data_ptr() for t in ts]
-
-        cols = [ptrs(As), ptrs(Bs), ptrs(scale_a or [None] * p), ptrs(scale_b or [None] * p), ptrs(Cs), ptrs(acc or [None] * p)]
-        table = torch.tensor(cols, dtype=torch.int64).reshape(6, p)
-        self.h_sizes = (_lib.Dim3 * max(p, 1))(*[_lib.Dim3(int(m), int(n), int(k)) for (m, n, k) in sizes])
-        self.h_q = (_lib.QParams * max(p, 1))(*[_lib.QParams(int(a), int(w), int(g), 1 if s else 0) for (a, w, g, s) in qparams])
-        sz = torch.tensor([[int(m), int(n), int(k)] for (m, n, k) in sizes], dtype=torch.int32).reshape(p, 3)
-        self.d_table = table.to(dev)
-        self.d_sizes = sz.to(dev)
+        # host tables as arrays: the six pointer rows and the sizes go to the device as one block, sizes and QParams also stay for the launcher
+        block = np.zeros(6 * p * 8 + p * 12 + 12, np.uint8)
+        table = block[:6 * p * 8].view(np.int64).reshape(6, p)
+        for row, ts in zip(table, (As, Bs, scale_a, scale_b, Cs, acc)):
+            if ts:
+                row[:] = [0 if t is None else t.data_ptr() for t in ts]  # (0 for a tensor without elements)
+        h_sizes = block[6 * p * 8:6 * p * 8 + p * 12].view(np.uint32).reshape(p, 3)
+        h_sizes[:] = sizes if isinstance(sizes, np.ndarray) else np.array(sizes, np.int64).reshape(p, 3)
+        h_q = np.zeros((max(p, 1), 4), np.int32)                        # (a_bits, w_bits, gsize, sym byte): the QParams layout
+        if p:
+            h_q[:p] = _qparams_array(tuple(map(tuple, qparams)))
+        self.h_sizes = (_lib.Dim3 * max(p, 1)).from_buffer(block, 6 * p * 8)
+        self.h_q = (_lib.QParams * max(p, 1)).from_buffer(h_q)
+        self.d_block = _upload(block, dev)
+        self._base = self.d_block.data_ptr()
         self.has_acc = acc is not None
-        self.sizes = [tuple(int(v) for v in s) for s in sizes]
-        self.ops = sum(2 * m * n * k for (m, n, k) in self.sizes)
+        self.sizes = [tuple(s) for s in h_sizes.tolist()]
+        self.ops = int(2 * h_sizes.astype(np.int64).prod(axis=1).sum())
 
     def _ptr(self, row: int) -> int:
-        return self.d_table.data_ptr() + row * self.count * 8
+        return self._base + row * self.count * 8
 
     def run(self, stream=None) -> None:
         if self.count == 0:
             return
-        s = stream if stream is not None else torch.cuda.current_stream().cuda_stream
+        s = stream if stream is not None else _lib.current_stream()
         rc = self.lib.mxmoe_group_gemm(
             self.kernel_id, self._ptr(0), self._ptr(1), self._ptr(2), self._ptr(3), self._ptr(4), self._ptr(4),
-            None, None, None, None, self.d_sizes.data_ptr(), self.h_sizes, None, self.h_q, self.count,
+            None, None, None, None, self._ptr(6), self.h_sizes, None, self.h_q, self.count,
             self._ptr(5) if self.has_acc else None, s,
         )
         _lib.check(self.lib, rc)

@@ -305,7 +305,7 @@ class MxMoELayer:
         t, k_hid = hidden.shape
         topk = ids.shape[1]
         assert hidden.dtype == torch.float16 and k_hid == cfg.hidden and w.shape == ids.shape
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = _lib.current_stream()
         final = out if out is not None else torch.empty((t, cfg.hidden), dtype=torch.float16, device=dev)
         assert final.shape == (t, cfg.hidden) and final.dtype == torch.float16 and final.is_contiguous()
         short = self._short_setup(t, topk)
@@ -403,7 +403,7 @@ class MxMoELayer:
         d_tab = torch.from_numpy(staging).to(dev)
         base = d_tab.data_ptr()
         count = p1.shape[1]
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = _lib.current_stream()
         final = torch.empty((t, cfg.hidden), dtype=torch.float16, device=dev)
         if count == 0:
             return final.zero_()

@@ -10,15 +10,17 @@ Differences a caller can see, all deliberate:
 """
 from __future__ import annotations
 
+from functools import lru_cache
+
+import numpy as np
 import torch
 
 from . import _lib
-from .group_gemm import GroupGemmLaunch
+from .group_gemm import GroupGemmLaunch, _upload
 from .hadamard import device_signs
 
 
-def _stream():
-    return torch.cuda.current_stream().cuda_stream
+_stream = _lib.current_stream
 
 
 def act_tag(a_bits: int, gsize: int, bf6: bool = False, fp8: bool = False) -> int:
@@ -145,18 +147,13 @@ def build_permutation(topk_ids: torch.Tensor, num_experts: int, with_inverse: bo
     return dst, perm, slot, recv
 
 
-def _offsets(recv_cpu, num_tokens: int, num_experts: int, has_shared: bool, qparams_per_exp, ld: int, ld_shared: int, bf6: bool = False, fp8: bool = False):
-    """Host offset builder of ref_bind.cu:475-505 / 635-671 (units: fp16 elements)."""
-    et = num_experts + (1 if has_shared else 0)
-    if len(qparams_per_exp) < et:
-        raise RuntimeError(f"qparams_per_exp has {len(qparams_per_exp)} entries, need {et}")
-    rows, inp_sizes, scale_sizes, lds = [], [], [], []
-    cols = [[], [], [], []]                                  # tag, first row, input offset, scale offset per expert
-    recv_list = recv_cpu.tolist() if hasattr(recv_cpu, "tolist") else list(recv_cpu)
-    acc = io = so = 0
-    for e in range(et):
-        a_bits, _w, g, _s = qparams_per_exp[e]
-        tag = act_tag(int(a_bits), int(g), bf6 and int(_w) == 4, fp8 and int(_w) == 8)
+@lru_cache(maxsize=64)
+def _layout(qparams: tuple, ld: int, ld_shared: int, num_experts: int, bf6: bool, fp8: bool):
+    """Per expert (shared one last) int64 arrays (tag, row length, fp16 elements per packed row, scales per row) for one set of
+    formats: what the offset builders of ref_bind.cu:461-505 / 635-671 derive before they look at the counts."""
+    tags, widths = [], []
+    for e, (a_bits, w_bits, g, _s) in enumerate(qparams):
+        tag = act_tag(int(a_bits), int(g), bf6 and int(w_bits) == 4, fp8 and int(w_bits) == 8)
         if tag not in (0, 1, 2, 3, 4, 5):
             raise RuntimeError("quant type not supported")
         width = ld_shared if e == num_experts else ld
@@ -164,32 +161,84 @@ def _offsets(recv_cpu, num_tokens: int, num_experts: int, has_shared: bool, qpar
             raise RuntimeError(f"group-128 activations need a row length that is a multiple of 128, got {width}")
         if tag == 4 and (width % 128 or width < 256):
             raise RuntimeError(f"bf6 fragments need a row length that is a multiple of 128 and at least 256, got {width}")
-        qld = width * 3 // 8 if tag == 4 else (width if tag == 0 else (width // 2 if tag in (1, 5) else width // 4))
-        sld = 0 if tag == 0 else (width // 128 if tag == 3 else 1)    # scales per row (ref_bind.cu:492)
-        n = num_tokens if e == num_experts else int(recv_list[e])
-        for c, v in zip(cols, (tag, acc, io, so)):
-            c.append(v)
-        rows.append(n)
-        inp_sizes.append(packed_elems(tag, n, width))
-        scale_sizes.append(sld * n)
-        lds.append(qld)
-        acc += n
-        io += inp_sizes[-1]
-        so += sld * n
-    return torch.tensor(cols, dtype=torch.int64), rows, inp_sizes, scale_sizes, lds, io, so
+        tags.append(tag)
+        widths.append(width)
+    tag, width = np.array(tags, np.int64), np.array(widths, np.int64)
+    qld = np.where(tag == 4, width * 3 // 8, np.where(tag == 0, width, np.where((tag == 1) | (tag == 5), width // 2, width // 4)))
+    sld = np.where(tag == 0, 0, np.where(tag == 3, width // 128, 1))    # scales per row (ref_bind.cu:492)
+    return tag, width, qld, sld
+
+
+def _qp_key(qparams, count: int) -> tuple:
+    key = tuple(qparams[:count])
+    try:
+        hash(key)
+        return key
+    except TypeError:  # (entries that are lists)
+        return tuple(tuple(q) for q in key)
+
+
+def _offset_arrays(rows: np.ndarray, num_experts: int, qparams_per_exp, ld: int, ld_shared: int, bf6: bool, fp8: bool):
+    """(table int64 [4, Et], elements and scales per expert, elements per packed row) of the experts' `rows`."""
+    et = rows.size
+    if len(qparams_per_exp) < et:
+        raise RuntimeError(f"qparams_per_exp has {len(qparams_per_exp)} entries, need {et}")
+    tag, width, qld, sld = _layout(_qp_key(qparams_per_exp, et), ld, ld_shared, num_experts, bool(bf6), bool(fp8))
+    inp = qld * rows
+    if bf6:  # tag 4: whole blocks of 32 rows
+        inp = np.where(tag == 4, -(-rows // 32) * (width // 64) * BF6_FRAGMENT_HALVES, inp)
+    scales = sld * rows
+    table = np.zeros((4, et), np.int64)                      # tag, first row, input offset, scale offset per expert
+    table[0] = tag
+    for dst, x in ((table[1], rows), (table[2], inp), (table[3], scales)):
+        np.cumsum(x[:-1], out=dst[1:])
+    return table, inp, scales, qld
+
+
+def _rows_of(recv_cpu, num_tokens: int, num_experts: int, has_shared: bool) -> np.ndarray:
+    recv = recv_cpu.numpy() if isinstance(recv_cpu, torch.Tensor) else np.asarray(recv_cpu)
+    return np.append(recv[:num_experts], num_tokens).astype(np.int64) if has_shared else recv[:num_experts].astype(np.int64)
+
+
+def _offsets(recv_cpu, num_tokens: int, num_experts: int, has_shared: bool, qparams_per_exp, ld: int, ld_shared: int, bf6: bool = False, fp8: bool = False):
+    """Host offset builder of ref_bind.cu:475-505 / 635-671 (units: fp16 elements)."""
+    rows = _rows_of(recv_cpu, num_tokens, num_experts, has_shared)
+    table, inp, scales, qld = _offset_arrays(rows, num_experts, qparams_per_exp, ld, ld_shared, bf6, fp8)
+    return torch.from_numpy(table), rows.tolist(), inp.tolist(), scales.tolist(), qld.tolist(), int(inp.sum()), int(scales.sum())
+
+
+def _row_views(store, offsets, sizes, lds):
+    """One [-1, ld] view per (offset, elements, ld), back to back from the start of `store`.  Experts of one row length (the usual case)
+    are cut by a single call."""
+    if not lds:
+        return []
+    ld, total = lds[0], offsets[-1] + sizes[-1]
+    if lds.count(ld) == len(lds):
+        return list((store if store.numel() == total else store[:total]).view(-1, ld).split_with_sizes([s // ld for s in sizes]))
+    return [store.as_strided((s // w, w), (w, 1), o) for o, s, w in zip(offsets, sizes, lds)]
 
 
 def _views(store, scale_store, table, rows, inp_sizes, scale_sizes, lds):
-    inp_list, scale_list = [], []
-    inp_off, scale_off = table[2].tolist(), table[3].tolist()
-    for e, n in enumerate(rows):
-        if n == 0:
-            continue
-        off = inp_off[e]
-        inp_list.append(store[off:off + inp_sizes[e]].view(-1, lds[e]))   # [n, row] (tag 4: [32 * blocks, 3/8 of the row]: fragments, not rows)
-        soff = scale_off[e]
-        scale_list.append(scale_store[soff:soff + scale_sizes[e]])
-    return inp_list, scale_list
+    """Per non-empty expert its packed rows [n, row] (tag 4: [32 * blocks, 3/8 of the row]: fragments, not rows) and its scales."""
+    live = [e for e, n in enumerate(rows) if n]
+    if not live:
+        return [], []
+    inp_off = table[2].tolist()
+    inp_list = _row_views(store, [inp_off[e] for e in live], [inp_sizes[e] for e in live], [lds[e] for e in live])
+    sizes = [scale_sizes[e] for e in live]
+    total = sum(sizes)
+    return inp_list, list((scale_store if scale_store.numel() == total else scale_store[:total]).split_with_sizes(sizes))
+
+
+def _out_views(store, rows, ld: int, ld_shared: int, num_experts: int):
+    """Per non-empty expert its [rows, ld] output buffer, back to back from the start of `store` (the shared expert's rows are `ld_shared` wide)."""
+    routed = [n for n in rows[:num_experts] if n]
+    total = sum(routed) * ld
+    out = list(store[:total].view(-1, ld).split_with_sizes(routed)) if routed else []
+    if len(rows) > num_experts and rows[num_experts]:
+        n = rows[num_experts]
+        out.append(store[total:total + n * ld_shared].view(n, ld_shared))
+    return out
 
 
 def quant_inp_act(hidden, topk_ids, num_experts: int, N: int, num_shared_experts: int, qparams_per_exp, verbose: bool = False, rotate: int = 0, bf6: bool = False, fp8: bool = False):
@@ -211,7 +260,7 @@ def quant_inp_act(hidden, topk_ids, num_experts: int, N: int, num_shared_experts
     inp_store = torch.empty(io, dtype=torch.float16, device=dev)
     scale_store = torch.empty(so, dtype=torch.float16, device=dev)
     out_store = torch.empty((num_shared_experts + topk) * t * N * 2, dtype=torch.float16, device=dev)
-    d_table = table.to(dev)
+    d_table = _upload(table.numpy(), dev)
     hk, hf, signs = device_signs(k, dev) if rotate else (1, 1, None)
     routed = int(recv_cpu.sum())                            # rows whose expert id was in range; the sorted arrays hold exactly these
     if per_token:
@@ -223,13 +272,7 @@ def quant_inp_act(hidden, topk_ids, num_experts: int, N: int, num_shared_experts
                                             k, routed, t, num_experts, int(has_shared), rotate | (ROWS_VARIANTS if bf6 or fp8 else 0), hk, hf,
                                             None if signs is None else signs.data_ptr(), _stream()))
     inp_list, scale_list = _views(inp_store, scale_store, table, rows, inp_sizes, scale_sizes, lds)
-    out_list, off = [], 0
-    for e, n in enumerate(rows):
-        if n == 0:
-            continue
-        ld = N * 2 * num_shared_experts if e == num_experts else N * 2
-        out_list.append(out_store[off:off + n * ld].view(n, ld))
-        off += n * ld
+    out_list = _out_views(out_store, rows, N * 2, N * 2 * num_shared_experts, num_experts)
     if verbose:
         for e, n in enumerate(rows):
             print(f"exp: {e} tokens: {n} qinp_size: {inp_sizes[e]} qinp_scale_size: {scale_sizes[e]}")
@@ -250,7 +293,7 @@ def silu_mul_then_quant(inp, num_problems: int, num_experts: int, K: int, N: int
     inp_store = torch.empty(io, dtype=torch.float16, device=dev)
     scale_store = torch.empty(so, dtype=torch.float16, device=dev)
     out_store = torch.empty((1 + topk) * num_tokens * K, dtype=torch.float16, device=dev)
-    d_table = table.to(dev)
+    d_table = _upload(table.numpy(), dev)
     flat = inp.reshape(-1)
     n_sh = N * num_shared_experts
     hk, hf, signs = device_signs(N, dev) if rotate else (1, 1, None)
@@ -260,12 +303,7 @@ def silu_mul_then_quant(inp, num_problems: int, num_experts: int, K: int, N: int
     _lib.check(lib, lib.mxmoe_silu_mul_quant(flat.data_ptr(), shared_ptr, inp_store.data_ptr(), scale_store.data_ptr(), values_sorted.data_ptr(), d_table.data_ptr(),
                                              N, n_sh, r, num_tokens, num_experts, int(has_shared), rotate | (ROWS_VARIANTS if bf6 or fp8 else 0), hk, hf, None if signs is None else signs.data_ptr(), _stream()))
     inp_list, scale_list = _views(inp_store, scale_store, table, rows, inp_sizes, scale_sizes, lds)
-    out_list, off = [], 0
-    for e, n in enumerate(rows):
-        if n == 0:
-            continue
-        out_list.append(out_store[off:off + n * K].view(n, K))
-        off += n * K
+    out_list = _out_views(out_store, rows, K, K, num_experts)
     return inp_list, scale_list, out_list, inp_store, scale_store, out_store
 
 
@@ -280,27 +318,19 @@ def gg_unpermute_out(out_store: torch.Tensor, topk_ids: torch.Tensor, topk_weigh
     t, k = ids.shape
     w = topk_weights.to(torch.float32).contiguous()
     assert w.shape == (t, k) and w.is_cuda and out_store.is_cuda and out_store.dtype == torch.float16
-    _dst, _perm, slot, recv = build_permutation(ids, num_experts)  # stable, so the same order the rows were produced in
-    rows = int(recv.sum().item())
+    # stable, so the same order the rows were produced in; the inverse map says where each (token, slot) went
+    _dst, _perm, _slot, recv, inv = build_permutation(ids, num_experts, with_inverse=True)
     flat = out_store.reshape(-1)
-    need = (rows + (t if num_shared_experts else 0)) * K
-    if flat.numel() < need:
-        raise RuntimeError(f"out_store holds {flat.numel()} elements, the layer produced {need}")
+    most = (t * k + (t if num_shared_experts else 0)) * K
+    if flat.numel() < most:  # (ids out of range are dropped: only a store below the bound needs the exact count, and with it a synchronisation)
+        need = (int(recv.sum().item()) + (t if num_shared_experts else 0)) * K
+        if flat.numel() < need:
+            raise RuntimeError(f"out_store holds {flat.numel()} elements, the layer produced {need}")
     out = output if output is not None else torch.empty((t, K), dtype=torch.float16, device=flat.device)
     assert out.shape == (t, K) and out.dtype == torch.float16 and out.is_contiguous()
-    ws = torch.empty(lib.mxmoe_combine_workspace_bytes(t, k), dtype=torch.uint8, device=flat.device)
-    shared_ptr = flat.data_ptr() + rows * K * 2 if num_shared_experts else None
-    _lib.check(lib, lib.mxmoe_unpermute_combine(flat.data_ptr(), shared_ptr, w.data_ptr(), slot.data_ptr(), rows, t, k, K, out.data_ptr(), ws.data_ptr(), _stream()))
+    _lib.check(lib, lib.mxmoe_combine_sorted(flat.data_ptr(), recv.data_ptr(), num_experts, int(num_shared_experts > 0), w.data_ptr(), inv.data_ptr(), t, k, K, out.data_ptr(),
+                                             _stream()))
     return out
-
-
-def _problem_lists(num_experts: int, experts, recv_cpu, num_tokens: int):
-    has_shared = len(experts) > num_experts
-    recv_list = recv_cpu.tolist()
-    for e in range(num_experts + (1 if has_shared else 0)):
-        n = num_tokens if e == num_experts else int(recv_list[e])
-        if n:
-            yield e, n
 
 
 def gg_mxmoe_share_fused(inp, experts, scale_zp_a, scale_zp_b, output, N: int, K: int, shared_N: int, shared_K: int, qparams_per_exp,
@@ -323,18 +353,20 @@ def prepare_gg(inp, experts, scale_zp_a, scale_zp_b, output, N, K, shared_N, sha
     recv_cpu = recv_tokens_per_exp.cpu()
     e_cnt = recv_cpu.shape[0]
     num_tokens = output[-1].shape[0] if len(output) else 0             # rows of the last problem (the shared expert's, when there is one)
-    As, Bs, sa, sb, Cs, sizes, qps = [], [], [], [], [], [], []
-    for p, (e, n) in enumerate(_problem_lists(e_cnt, experts, recv_cpu, num_tokens)):
-        As.append(inp[p])
-        Bs.append(experts[e])
-        sa.append(scale_zp_a[p] if scale_zp_a is not None and p < len(scale_zp_a) else None)
-        sb.append(scale_zp_b[e] if scale_zp_b is not None else None)
-        Cs.append(output[p])
-        sizes.append((n, shared_N, shared_K) if e == e_cnt else (n, N, K))
-        qps.append(tuple(qparams_per_exp[e]))
-    if len(As) != len(inp):
-        raise RuntimeError(f"{len(inp)} inputs for {len(As)} non-empty problems")
-    g = GroupGemmLaunch(As, Bs, sa, sb, Cs, sizes, qps, kernel_id=kernel_id, acc=acc_dump)
+    rows = _rows_of(recv_cpu, num_tokens, e_cnt, len(experts) > e_cnt)
+    live = np.flatnonzero(rows)
+    idx = live.tolist()
+    if len(idx) != len(inp):
+        raise RuntimeError(f"{len(inp)} inputs for {len(idx)} non-empty problems")
+    sa = [scale_zp_a[p] if p < len(scale_zp_a) else None for p in range(len(idx))] if scale_zp_a is not None else None
+    sizes = np.empty((len(idx), 3), np.uint32)
+    sizes[:, 0], sizes[:, 1], sizes[:, 2] = rows[live], N, K
+    if idx and idx[-1] == e_cnt:
+        sizes[-1, 1:] = shared_N, shared_K
+    qps = [qparams_per_exp[e] for e in idx]
+    qps = qps if type(qps[0] if qps else ()) is tuple else [tuple(q) for q in qps]
+    g = GroupGemmLaunch(inp, [experts[e] for e in idx], sa, None if scale_zp_b is None else [scale_zp_b[e] for e in idx], output[:len(idx)], sizes, qps,
+                        kernel_id=kernel_id, acc=acc_dump)
     g.qparams = qps
     return g
 

@@ -86,3 +86,46 @@ def test_layers_the_short_form_does_not_take():
         hidden_t = S.make_hidden(cfg)
         ids, w = S.make_routing(cfg)
         assert torch.equal(layer(hidden_t, ids, w), layer.call_with_host_tables(hidden_t, ids, w))
+
+
+@pytest.mark.parametrize("num_bytes", [4, 3584, 3588, 10000])
+def test_upload_in_kernel_arguments(num_bytes):
+    """Host tables of less than one, exactly one and several launches' arguments; the bytes behind them stay as they were."""
+    import numpy as np
+
+    from mxmoe_amd import _lib
+
+    lib = _lib.load()
+    host = np.random.default_rng(num_bytes).integers(0, 256, num_bytes, dtype=np.uint8)
+    dst = torch.full((num_bytes + 8,), 7, dtype=torch.uint8, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    _lib.check(lib, lib.mxmoe_upload(dst.data_ptr(), host.ctypes.data, num_bytes, stream))
+    want = host.copy()
+    host[:] = 0                                                         # the caller's array is free again at once
+    assert np.array_equal(dst[:num_bytes].cpu().numpy(), want) and bool((dst[num_bytes:] == 7).all())
+    assert lib.mxmoe_upload(dst.data_ptr(), host.ctypes.data, 3, stream) == 3 and lib.mxmoe_upload(None, host.ctypes.data, 4, stream) == 5
+
+
+@pytest.mark.parametrize("topk,num_shared", [(1, 0), (8, 1), (9, 1), (17, 0)])
+def test_combine_of_more_slots_than_it_loads_at_a_time(topk, num_shared):
+    """gg_unpermute_out (combine_kernel takes eight slots at a time) against the oracle, ids out of range included."""
+    import numpy as np
+
+    from mxmoe_amd import ops
+    from oracle import mxmoe_oracle as O
+
+    rng = np.random.default_rng(topk)
+    t, e, k = 13, 20, 136
+    ids = np.stack([rng.permutation(e)[:topk] for _ in range(t)]).astype(np.int32)
+    ids[4, 0] = e + 1
+    w = rng.random((t, topk), dtype=np.float32)
+    slots = np.argsort(ids.reshape(-1), kind="stable")
+    slots = slots[ids.reshape(-1)[slots] < e]                           # sorted rows in (expert, token, slot) order
+    rows = len(slots)
+    down = rng.standard_normal((rows + (t if num_shared else 0), k)).astype(np.float16)
+    want = O.unpermute_combine(down[:rows], slots, w, down[rows:] if num_shared else None)
+    store = torch.from_numpy(down).cuda()
+    got = ops.gg_unpermute_out(store, torch.from_numpy(ids).cuda(), torch.from_numpy(w).cuda(), e, k, num_shared)
+    assert np.array_equal(got.cpu().numpy().view(np.uint16), want.view(np.uint16))
+    with pytest.raises(RuntimeError, match="out_store holds"):
+        ops.gg_unpermute_out(store[:-1], torch.from_numpy(ids).cuda(), torch.from_numpy(w).cuda(), e, k, num_shared)
