@@ -303,7 +303,7 @@ int mxmoe_upload(void* dst, const void* host_src, size_t bytes, void* stream);
  *   workspace      mxmoe_permute_workspace_bytes(R, num_experts), 16-byte aligned.
  * grid_*: mxmoe_plan_grid_bound of each block.  rotate, had_*: of the intermediate rows, as for mxmoe_silu_mul_quant (bits 0 - 1 only).
  *
- * mxmoe_layer_supported   1 when the short form takes the layer: hidden 512, 1024, 2048 or 4096; at most 1024 experts; inter a
+ * mxmoe_layer_supported   1 when the short form takes the layer: hidden 512, 1024, 2048 or 4096; at most 512 experts; inter a
  *                         multiple of 32; no bf6 operands; token stores and fp16 weights below 2 GiB; and R <= 65536, or
  *                         ceil(R / 256) * num_experts <= 16384.  Else 0: use the separate entry points.
  * mxmoe_layer_create      checks the description and copies it; the handle is read only afterwards (mxmoe_layer_run may be called from several

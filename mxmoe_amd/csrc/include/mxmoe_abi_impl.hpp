@@ -88,7 +88,10 @@ int mxmoe_group_gemm_plan(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_
     Segment sg[2];
     const int ns = f == Fmt::UNSUPPORTED ? -1 : plan_segments(plan_of(k), (int)f, (int)h_sizes[i].x, (int)h_sizes[i].y, sg);
     if (ns < 0) { last_error() = "quant type not supported"; return 1; }
-    if (branch_out) branch_out[i] = ns ? sg[0].branch : pick_branch(plan_of(k), (int)f, 1, (int)h_sizes[i].y);
+    if (branch_out) {  // (an empty problem: the branch one row would take)
+      if (ns == 0) plan_segments(plan_of(k), (int)f, 1, (int)h_sizes[i].y, sg);
+      branch_out[i] = sg[0].branch;
+    }
     for (int j = 0; j < ns; ++j) {
       const BranchInfo& bi = k.branches[sg[j].branch];
       if (!shape_ok(bi, h_sizes[i])) {  // what the launch itself would refuse

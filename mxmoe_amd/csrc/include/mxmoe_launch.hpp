@@ -381,114 +381,116 @@ inline double branch_cost(const BranchInfo& b) {
 // What the planners (the host launcher and the device-side planning kernel) need to know of a kernel's branches, as plain data.
 constexpr int kMaxBranches = 32;
 struct PlanBranch {
-  int fmt, BM, BN, k_multiple;
-  int bm_log2, bn_log2;  // of a tile dimension that is a power of two (the usual case: the planners shift instead of dividing), else -1
+  int index;             // position among the kernel's branches
+  int fmt, BM, BN;
+  int bm_log2, bn_log2;  // tile dimensions are powers of two (register_fused): the planners shift instead of dividing
   double cost;           // tile_cost
   double cost_per_row;   // tile_cost / BM
 };
 // A phase of such tiles keeps the plain workgroup order (no XCD remap): the few-token weight-only tiles stream their own weights
 // and share nothing but a few rows of activations with their neighbours.
 __host__ __device__ inline bool flat_phase(const PlanBranch& b) { return b.BM <= 16 || (is_weight_only((Fmt)b.fmt) && b.BM < 128); }
-// Tiles of size `dim` (2^`lg` when lg >= 0) that cover `x`.
-__host__ __device__ inline int tiles_over(int x, int dim, int lg) { return lg >= 0 ? (x + dim - 1) >> lg : (x + dim - 1) / dim; }
+// Tiles of size 2^lg that cover `x`.
+__host__ __device__ inline int tiles_over(int x, int lg) { return (x + (1 << lg) - 1) >> lg; }
 constexpr int kNumFmts = (int)Fmt::UNSUPPORTED;
 struct PlanInfo {
-  int nb;                    // branches
-  int order[kMaxBranches];   // branch indices, most expensive tile first (branch_cost); ties keep the registration order
-  // the branches of one format as a list in registration order (-1 ends it): the planners look at no other branch
-  int first_of_fmt[kNumFmts];
-  int next_of_fmt[kMaxBranches];
+  int nb;                       // branches
+  uint8_t order[kMaxBranches];  // positions in b, most expensive tile first (branch_cost); ties keep the registration order
+  uint8_t fmt_start[kNumFmts + 4];
+  // by format, in registration order inside a format: those of format f are b[fmt_start[f]] .. b[fmt_start[f + 1] - 1], and the planners
+  // look at no other branch
   PlanBranch b[kMaxBranches];
 };
-
-// Cheapest branch of format `f` for a block of `rows` x `N` run with one tile shape: cost = row tiles * column tiles * tile_cost.
-__host__ __device__ inline int pick_branch(const PlanInfo& k, int f, int rows, int N) {
-  int best = -1;
-  double best_cost = 0;
-  if (f < 0 || f >= kNumFmts) return -1;
-  for (int i = k.first_of_fmt[f]; i >= 0; i = k.next_of_fmt[i]) {
-    const PlanBranch& b = k.b[i];
-    const double c = (double)tiles_over(rows, b.BM, b.bm_log2) * tiles_over(N, b.BN, b.bn_log2) * b.cost;
-    if (best < 0 || c < best_cost - 1e-9 || (c < best_cost + 1e-9 && b.BM > k.b[best].BM)) {
-      best = i;
-      best_cost = c;
-    }
-  }
-  return best;
-}
+static_assert(sizeof(PlanInfo) % 8 == 0, "copied word by word");
 
 struct Segment {
-  int row0, rows, branch;
+  int row0, rows, branch, tiles;
 };
 
 // Split the M rows of an M x N problem into at most two segments: whole tiles of the shape that is cheapest per output element,
-// then the remainder with the shape that covers it most cheaply.  Returns the number of segments (0 for M == 0), or -1 when
-// the kernel has no tile for `f`.
+// then the remainder with the shape that covers it most cheaply (cost of a block run with one shape = row tiles * column tiles *
+// tile_cost).  Returns the number of segments (0 for M == 0), or -1 when the kernel has no tile for `f`.
+// Two rolled loops on purpose: the device planner runs this once per launch, when none of its code is in the instruction cache, and
+// what it costs there is the fetching of its instructions.
 __host__ __device__ inline int plan_segments(const PlanInfo& k, int f, int M, int N, Segment out[2]) {
-  int big = -1;
-  double big_unit = 0;
   if (f < 0 || f >= kNumFmts) return -1;
-  for (int i = k.first_of_fmt[f]; i >= 0; i = k.next_of_fmt[i]) {
+  const int lo = k.fmt_start[f], hi = k.fmt_start[f + 1];
+  if (lo == hi) return -1;
+  if (M <= 0) return 0;
+  struct Pick {
+    int branch = -1, bm = 0, tiles = 0;
+    double cost = 0;
+  };
+  auto offer = [](Pick& best, const PlanBranch& b, int tiles, double c, double eps) {
+    if (best.branch < 0 || c < best.cost - eps || (c < best.cost + eps && b.BM > best.bm)) {
+      best.branch = b.index;
+      best.bm = b.BM;
+      best.tiles = tiles;
+      best.cost = c;
+    }
+  };
+  Pick unit, whole;  // cheapest per row of the problem; cheapest for all of it
+  int full = 0;
+  double full_cost = 0;
+#pragma unroll 1
+  for (int i = lo; i < hi; ++i) {
     const PlanBranch& b = k.b[i];
-    const double unit = b.cost_per_row * tiles_over(N, b.BN, b.bn_log2);  // cost per row of the problem
-    if (big < 0 || unit < big_unit - 1e-12 || (unit < big_unit + 1e-12 && b.BM > k.b[big].BM)) {
-      big = i;
-      big_unit = unit;
+    const int tm = tiles_over(M, b.bm_log2), tn = tiles_over(N, b.bn_log2), rows = M >> b.bm_log2 << b.bm_log2;
+    offer(whole, b, tm * tn, (double)tm * tn * b.cost, 1e-9);
+    const int had = unit.branch;
+    offer(unit, b, (M >> b.bm_log2) * tn, b.cost_per_row * tn, 1e-12);
+    if (unit.branch != had) {
+      full = rows;
+      full_cost = (double)(M >> b.bm_log2) * tn * b.cost;
     }
   }
-  if (big < 0) return -1;
-  if (M <= 0) return 0;
-  auto cost_of = [&](int branch, int rows) {
-    const PlanBranch& b = k.b[branch];
-    return (double)tiles_over(rows, b.BM, b.bm_log2) * tiles_over(N, b.BN, b.bn_log2) * b.cost;
-  };
-  const int bm = k.b[big].BM, bm_lg = k.b[big].bm_log2;
-  const int full = bm_lg >= 0 ? (M >> bm_lg) << bm_lg : (M / bm) * bm, rem = M - full;
-  const int whole = pick_branch(k, f, M, N);
-  if (rem == 0 || full == 0) {
-    out[0] = Segment{0, M, whole};
+  const int rem = M - full;
+  out[0] = Segment{0, M, whole.branch, whole.tiles};
+  if (rem == 0 || full == 0) return 1;
+  Pick rest;
+  int all_unit = 0;  // tiles of the whole problem in the shape that is cheapest per row
+#pragma unroll 1
+  for (int i = lo; i < hi; ++i) {
+    const PlanBranch& b = k.b[i];
+    const int tm = tiles_over(rem, b.bm_log2), tn = tiles_over(N, b.bn_log2);
+    offer(rest, b, tm * tn, (double)tm * tn * b.cost, 1e-9);
+    if (b.index == unit.branch) all_unit = tiles_over(M, b.bm_log2) * tn;
+  }
+  if (rest.branch == unit.branch) {
+    out[0] = Segment{0, M, unit.branch, all_unit};
     return 1;
   }
-  const int rb = pick_branch(k, f, rem, N);
-  if (cost_of(whole, M) <= cost_of(big, full) + cost_of(rb, rem) + 1e-9 || rb == big) {
-    out[0] = Segment{0, M, rb == big ? big : whole};
-    return 1;
-  }
-  out[0] = Segment{0, full, big};
-  out[1] = Segment{full, rem, rb};
+  if (whole.cost <= full_cost + rest.cost + 1e-9) return 1;
+  out[0] = Segment{0, full, unit.branch, unit.tiles};
+  out[1] = Segment{full, rem, rest.branch, rest.tiles};
   return 2;
-}
-
-__host__ __device__ inline int segment_tiles(const PlanInfo& k, const Segment& sg, int N) {
-  const PlanBranch& b = k.b[sg.branch];
-  return tiles_over(sg.rows, b.BM, b.bm_log2) * tiles_over(N, b.BN, b.bn_log2);
 }
 
 inline PlanInfo make_plan_info(const std::vector<BranchInfo>& branches) {
   PlanInfo k;
   std::memset(&k, 0, sizeof k);
   k.nb = std::min((int)branches.size(), kMaxBranches);
-  for (int i = 0; i < k.nb; ++i) {
-    auto log2_of = [](int v) {
-      int lg = -1;
-      if (v > 0 && (v & (v - 1)) == 0)
-        for (lg = 0; (1 << lg) < v; ++lg) {}
-      return lg;
-    };
-    const double cost = tile_cost(branches[i]);
-    k.b[i] = PlanBranch{(int)branches[i].fmt, branches[i].BM, branches[i].BN, branches[i].k_multiple, log2_of(branches[i].BM), log2_of(branches[i].BN), cost,
-                        cost / branches[i].BM};
-    k.order[i] = i;
+  auto log2_of = [](int v) {
+    int lg = 0;
+    while ((1 << lg) < v) ++lg;
+    return lg;
+  };
+  int at = 0;
+  for (int f = 0; f < kNumFmts; ++f) {
+    k.fmt_start[f] = (uint8_t)at;
+    for (int i = 0; i < k.nb; ++i)
+      if ((int)branches[i].fmt == f) {
+        const double cost = tile_cost(branches[i]);
+        k.b[at++] = PlanBranch{i, f, branches[i].BM, branches[i].BN, log2_of(branches[i].BM), log2_of(branches[i].BN), cost, cost / branches[i].BM};
+      }
   }
-  std::stable_sort(k.order, k.order + k.nb, [&](int x, int y) { return branch_cost(branches[x]) > branch_cost(branches[y]); });
-  for (int f = 0; f < kNumFmts; ++f) k.first_of_fmt[f] = -1;
-  for (int i = k.nb - 1; i >= 0; --i) {
-    const int f = k.b[i].fmt;
-    k.next_of_fmt[i] = -1;
-    if (f < 0 || f >= kNumFmts) continue;
-    k.next_of_fmt[i] = k.first_of_fmt[f];
-    k.first_of_fmt[f] = i;
-  }
+  k.fmt_start[kNumFmts] = (uint8_t)at;
+  std::vector<int> order(k.nb);
+  for (int i = 0; i < k.nb; ++i) order[i] = i;
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return branch_cost(branches[x]) > branch_cost(branches[y]); });
+  for (int r = 0; r < k.nb; ++r)
+    for (int i = 0; i < k.nb; ++i)
+      if (k.b[i].index == order[r]) k.order[r] = (uint8_t)i;
   return k;
 }
 
@@ -576,6 +578,7 @@ struct FuncThunk {
 template <class... Tiles>
 int register_fused(const char* fn_name, Policy policy = Policy::Fused, int max_rows_hint = 0, LaunchPlannedFn launch_gate_up = nullptr) {
   static_assert(sizeof...(Tiles) <= kMaxBranches, "the planners' branch table holds kMaxBranches tile shapes per kernel");
+  static_assert((((Tiles::BM & (Tiles::BM - 1)) == 0 && (Tiles::BN & (Tiles::BN - 1)) == 0) && ...), "the planners shift: tile dimensions are powers of two");
   FusedKernel k;
   k.policy = policy;
   k.max_rows_hint = max_rows_hint;
@@ -699,7 +702,7 @@ inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, c
         last_error() = buf;
         return 3;
       }
-      entries[nent++] = Entry{sg[j].row0, sg[j].rows, i, sg[j].branch, segment_tiles(pi, sg[j], (int)sz.y)};
+      entries[nent++] = Entry{sg[j].row0, sg[j].rows, i, sg[j].branch, sg[j].tiles};
     }
   }
   // Most expensive tile shape first.  Inside a shape, the problems whose K is above the launch's smallest K go first (their tiles
@@ -710,7 +713,8 @@ inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, c
   for (int i = 0; i < n; ++i) kmin = std::min(kmin, h_sizes[base + i].z);
   int total = 0, ne = 0, wg = 0, np = 0;
   for (int oi = 0; oi < pi.nb; ++oi) {
-    const int b = pi.order[oi];
+    const PlanBranch& pb = pi.b[pi.order[oi]];
+    const int b = pb.index;
     const int tile0 = total;
     for (int pass = 0; pass < 2; ++pass)
       for (int ei = 0; ei < nent; ++ei) {
@@ -725,7 +729,7 @@ inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, c
     if (np < kMaxPhases) {
       a.phase_tile0[np] = tile0;
       a.phase_wg0[np] = wg;
-      if (flat_phase(pi.b[b])) a.phase_flat |= 1 << np;
+      if (flat_phase(pb)) a.phase_flat |= 1 << np;
       ++np;
     }
     const int p0 = a.phase_tile0[np - 1];

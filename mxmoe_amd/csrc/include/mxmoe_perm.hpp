@@ -46,6 +46,15 @@ __device__ __forceinline__ long wave_inclusive_scan(long v) {
   v += dpp_or_zero<0x143, 0xC>(v);
   return v;
 }
+__device__ __forceinline__ int wave_inclusive_max(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x111, 0xF, 0xF, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x112, 0xF, 0xF, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x114, 0xF, 0xF, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x118, 0xF, 0xF, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xA, 0xF, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xC, 0xF, false));
+  return v;
+}
 // value of the wave's last lane, as a scalar
 __device__ __forceinline__ int wave_last(int v) { return __builtin_amdgcn_readlane(v, 63); }
 __device__ __forceinline__ long wave_last(long v) {

@@ -70,31 +70,49 @@ struct PlanPair {
 // expert, if any, is expert E with `shared_rows` rows).  Everything the host launcher computes (launch_range), with the same
 // functions and in the same order, so the two produce identical tables; prefix sums over experts are wave scans (a later chunk
 // first sums what the experts before it occupy), and an entry finds its place from per-branch counts instead of a sequential walk.
-// A chain of dependent steps that the whole forward waits for: its scans run on lane moves in the vector ALU and the sums over the
-// branches take one lane per branch (with LDS shuffles and a serial walk over the branches the chain took 1.4 times as long).
-// `recv`: the tokens-per-expert counts (device memory, or LDS when the planning workgroup counted them itself).
+// A chain of dependent steps that the whole forward waits for, so every step is kept short: what does not depend on the counts (the
+// experts' descriptors, the kernel's branch table) is fetched first, by plan_block_prepare, while the counts are still being made;
+// scans run on lane moves in the vector ALU; sums over the branches take one lane per branch.  Its code is
+// cold in every launch and costs its fetching, so it is small: loops are rolled, and no division is left (a version with the branch walk
+// unrolled into registers and 2.3 times the code was slower at 8192 tokens: 5.5 us for the walk alone).  Measured inside the workgroup from
+// the counts to the end, Qwen1.5-MoE: 12.8 -> 7.3 us at 8192 tokens, 8.7 -> 5.2 us at 64.
+struct PlanShared {
+  static constexpr int kSums = 5;                    // rows, packed input, scales, output elements, fp16 input elements
+  long tot[kSums][2];                                // per wave
+  long base[kSums][2];                               // the same five, summed over the experts before this launch
+  int cnt[kMaxBranches][2], til[kMaxBranches][2];    // per run-order rank and wave: entries, tiles
+  int cnt_long[kMaxBranches][2], til_long[kMaxBranches][2];  // ... of which belong to long-K problems
+  int kmin[2];
+  // the kernel's branch table, from the kernel arguments: the planning functions walk it entry by entry, and each step of such a
+  // walk through the argument segment costs a trip to the scalar cache
+  PlanInfo info;
+};
+
+// Threads 0 .. kPlanThreads - 1 of the planning workgroup, before the counts are there: this thread's expert's descriptor (returned), the
+// branch table and cleared counters in LDS.  A barrier must lie between this and plan_block_body.
+__device__ __forceinline__ mxmoe_block_desc plan_block_prepare(const PlanParams& p, const int chunk, PlanShared& sh) {
+  const int e = threadIdx.x, ge = chunk * kMaxProblems + e;
+  mxmoe_block_desc d{};
+  if (e < min(kMaxProblems, p.Et - chunk * kMaxProblems)) d = p.desc[ge];
+  static_assert(sizeof(PlanInfo) % 4 == 0, "copied word by word");
+  for (int i = e; i < (int)(sizeof(PlanInfo) / 4); i += kPlanThreads) reinterpret_cast<int*>(&sh.info)[i] = reinterpret_cast<const int*>(&p.info)[i];
+  if (e < kMaxBranches) {
+    sh.cnt[e][0] = sh.cnt[e][1] = sh.til[e][0] = sh.til[e][1] = 0;
+    sh.cnt_long[e][0] = sh.cnt_long[e][1] = sh.til_long[e][0] = sh.til_long[e][1] = 0;
+  }
+  return d;
+}
+
+// `recv`: the tokens-per-expert counts (device memory, or LDS when the planning workgroup counted them itself); `d`: what
+// plan_block_prepare returned.
 template <class Count>
-__device__ __forceinline__ void plan_block_body(const PlanParams& p, const int chunk, const int chunks, const Count* recv) {
+__device__ __forceinline__ void plan_block_body(const PlanParams& p, const int chunk, const int chunks, const Count* recv, const mxmoe_block_desc& d, PlanShared& sh) {
   const int e0 = chunk * kMaxProblems;                       // first expert of this launch
   const int ecnt = min(kMaxProblems, p.Et - e0);             // experts of this launch
-  constexpr int kSums = 5;                           // rows, packed input, scales, output elements, fp16 input elements
-  __shared__ long s_tot[kSums][2];                   // per wave
-  __shared__ long s_base[kSums + 1][2];              // the same five, and the routed rows, summed over the experts before this launch
-  __shared__ int s_cnt[kMaxBranches][2], s_til[kMaxBranches][2];  // per run-order rank and wave: entries, tiles
-  __shared__ int s_cnt_long[kMaxBranches][2], s_til_long[kMaxBranches][2];  // ... of which belong to long-K problems
-  // the kernel's branch table, from the kernel arguments into LDS: the planning functions walk it entry by entry, and each step of
-  // such a walk through the argument segment costs a trip to the scalar cache
-  __shared__ PlanInfo info;
-  static_assert(sizeof(PlanInfo) % 4 == 0, "copied word by word");
-  for (int i = threadIdx.x; i < (int)(sizeof(PlanInfo) / 4); i += kPlanThreads) reinterpret_cast<int*>(&info)[i] = reinterpret_cast<const int*>(&p.info)[i];
+  constexpr int kSums = PlanShared::kSums;
+  const PlanInfo& info = sh.info;
   const int e = threadIdx.x, lane = e & 63, wave = e >> 6;
   const int ge = e0 + e;                             // this thread's expert
-  __shared__ unsigned s_used[2];                     // per wave: branches in use
-  if (e < kMaxBranches) {
-    s_cnt[e][0] = s_cnt[e][1] = s_til[e][0] = s_til[e][1] = 0;
-    s_cnt_long[e][0] = s_cnt_long[e][1] = s_til_long[e][0] = s_til_long[e][1] = 0;
-  }
-  if (e < 2) s_used[e] = 0;
   const bool mine = e < ecnt;
   const PlanLayout lay(p.Et);
   FusedArgs* fa = reinterpret_cast<FusedArgs*>(p.plan + chunk * kFusedArgsStride);
@@ -106,110 +124,81 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
   const int kind = p.form.kind;
 
   // what one expert occupies: rows, packed activation elements, scales, output elements, fp16 input elements (in fp16 elements but the rows)
-  auto footprint = [&](int x, long (&f)[kSums], int* tag_out, mxmoe_block_desc* d_out) {
-    const mxmoe_block_desc d = p.desc[x];
+  auto footprint = [&](int x, const mxmoe_block_desc& dx, long (&f)[kSums]) {
     const long rows = x < p.E ? (long)recv[x] : (long)p.shared_rows;
-    const int tag = act_tag_of(d.q), K = (int)d.K;
+    const int tag = act_tag_of(dx.q), K = (int)dx.K;
     const long qld = tag == 0 ? K : (tag == 1 || tag == 5 ? K / 2 : K / 4);  // fp16 elements per packed activation row (ref_bind.cu:491)
     const long sld = tag == 0 ? 0 : (tag == 3 ? K / 128 : 1);                // scales per row (ref_bind.cu:492)
     f[0] = rows;
     // packed activations: rows of qld elements, or (tag 4) whole blocks of 32 rows of K / 64 fragments
     f[1] = tag == 4 ? ((rows + 31) >> 5) * (long)(K >> 6) * (kBf6Frag / 2) : qld * rows;
     f[2] = sld * rows;
-    f[3] = (long)(kind == LayerForm::kGateUp ? d.N / 2 : d.N) * rows;
+    f[3] = (long)(kind == LayerForm::kGateUp ? dx.N / 2 : dx.N) * rows;
     f[4] = (long)K * rows;
-    if (tag_out) *tag_out = tag;
-    if (d_out) *d_out = d;
   };
   // experts before this launch (none for the first: most blocks are one launch)
   if (e0 > 0) {
-    long base[kSums + 1] = {0, 0, 0, 0, 0, 0};
+    long base[kSums] = {0, 0, 0, 0, 0};
     for (int x = e; x < e0; x += kPlanThreads) {
       long f[kSums];
-      footprint(x, f, nullptr, nullptr);
+      footprint(x, p.desc[x], f);
 #pragma unroll
       for (int i = 0; i < kSums; ++i) base[i] += f[i];
-      if (x < p.E) base[kSums] += f[0];
     }
 #pragma unroll
-    for (int i = 0; i <= kSums; ++i) {
+    for (int i = 0; i < kSums; ++i) {
       const long all = wave_last(wave_inclusive_scan(base[i]));
-      if (lane == 0) s_base[i][wave] = all;
+      if (lane == 0) sh.base[i][wave] = all;
     }
-  } else if (lane == 0) {
-#pragma unroll
-    for (int i = 0; i <= kSums; ++i) s_base[i][wave] = 0;
+  } else if (lane < kSums) {
+    sh.base[lane][wave] = 0;
   }
 
-  long rows = 0, sld = 0;
   long foot[kSums] = {0, 0, 0, 0, 0};
-  int tag = 0, fmt = 0, N = 0, K = 0;
-  mxmoe_block_desc d{};
-  if (mine) {
-    footprint(ge, foot, &tag, &d);
-    rows = foot[0];
-    fmt = fmt_of(d.q);
-    N = (int)d.N;
-    K = (int)d.K;
-    sld = tag == 0 ? 0 : (tag == 3 ? K / 128 : 1);
-  }
-  // exclusive sums over the experts of this launch before this one
-  long before_me[kSums];
-#pragma unroll
-  for (int i = 0; i < kSums; ++i) {
+  if (mine) footprint(ge, d, foot);
+  const long rows = foot[0];
+  const int N = (int)d.N, K = (int)d.K, fmt = fmt_of(d.q), tag = act_tag_of(d.q);
+  const bool scaled = tag != 0;
+  // exclusive sums over the experts of this launch before this one (those that the block's form has a use for)
+  long before_me[kSums] = {0, 0, 0, 0, 0};
+  auto sum_before = [&](int i) {
     const long inc = wave_inclusive_scan(foot[i]);
     before_me[i] = inc - foot[i];
-    const long tot = wave_last(inc);
-    if (lane == 0) s_tot[i][wave] = tot;
+    const long all = wave_last(inc);
+    if (lane == 0) sh.tot[i][wave] = all;
+  };
+  sum_before(0);
+  sum_before(3);
+  if (kind != LayerForm::kGateUp) {
+    sum_before(1);
+    sum_before(2);
   }
+  if (kind == LayerForm::kBehind) sum_before(4);
   // smallest K of the launch: problems above it run first inside their branch (see launch_range)
-  __shared__ int s_kmin[2];
-  __shared__ long s_routed[2];
-  {
-    const long routed_tot = wave_last(wave_inclusive_scan(mine && ge < p.E ? rows : 0l));
-    int km = mine ? K : 0x7fffffff;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) km = min(km, __shfl_xor(km, o));
-    if (lane == 0) {
-      s_kmin[wave] = km;
-      s_routed[wave] = routed_tot;
-    }
-  }
-  __syncthreads();
-  const bool long_k = mine && K > min(s_kmin[0], s_kmin[1]);
-  // segments of this problem and, per branch in run order, this wave's entries and tiles
+  const int km = -wave_last(wave_inclusive_max(mine ? -K : -0x7fffffff));
+  if (lane == 0) sh.kmin[wave] = km;
+  // segments of this problem (no need of the other wave)
   Segment sg[2];
   const int ns = mine ? plan_segments(info, fmt, (int)rows, N, sg) : 0;
-  int seg_tiles[2], seg_rank[2], seg_pos[2], seg_first[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    seg_tiles[j] = j < ns ? segment_tiles(info, sg[j], N) : 0;
-    seg_rank[j] = -1;
-    seg_pos[j] = seg_first[j] = 0;
-  }
-  // branches that this wave's problems use at all (most branches of a kernel are not used by a given launch: their counters stay zero)
-  {
-    unsigned mask = 0;
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      if (j < ns && seg_tiles[j] > 0) mask |= 1u << sg[j].branch;
-    if (mask) atomicOr(&s_used[wave], mask);
-  }
-  __builtin_amdgcn_wave_barrier();
-  const unsigned used = (unsigned)__builtin_amdgcn_readfirstlane((int)*(volatile unsigned*)&s_used[wave]);
+  __syncthreads();
+  const bool long_k = mine && K > min(sh.kmin[0], sh.kmin[1]);
+  // per branch in run order, this wave's entries and tiles
+  int seg_rank[2] = {-1, -1}, seg_pos[2] = {0, 0}, seg_first[2] = {0, 0};
+  const PlanBranch& my_branch = info.b[info.order[min(lane, kMaxBranches - 1)]];  // lane r: the branch of rank r
+  const int my_order = my_branch.index;
   for (int r = 0; r < info.nb; ++r) {
-    const int b = info.order[r];
-    if (!(used >> b & 1)) continue;
+    const int b = __builtin_amdgcn_readlane(my_order, r);
     int mine_tiles = 0, which = -1;
 #pragma unroll
     for (int j = 0; j < 2; ++j)
-      if (j < ns && sg[j].branch == b && seg_tiles[j] > 0) {
-        mine_tiles = seg_tiles[j];
+      if (j < ns && sg[j].branch == b && sg[j].tiles > 0) {
+        mine_tiles = sg[j].tiles;
         which = j;
       }
     // entries of this branch in this wave, long-K problems first: position = matching lanes that run earlier, first tile = their tiles
-    const uint64_t has = __ballot(which >= 0), has_long = __ballot(which >= 0 && long_k);
-    const int tc = __popcll(has), tc_long = __popcll(has_long);
+    const uint64_t has = __ballot(which >= 0);
+    if (has == 0) continue;  // (most branches of a kernel are not used by a given launch: their counters stay zero)
+    const uint64_t has_long = __ballot(which >= 0 && long_k);
     const int inc_long = wave_inclusive_scan(long_k ? mine_tiles : 0), inc_rest = wave_inclusive_scan(long_k ? 0 : mine_tiles);
     const int tt_long = wave_last(inc_long), tt = tt_long + wave_last(inc_rest);
     const uint64_t before = (1ull << lane) - 1;
@@ -222,26 +211,28 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
         seg_first[j] = long_k ? inc_long - mine_tiles : inc_rest - mine_tiles;
       }
     if (lane == 0) {
-      s_cnt[r][wave] = tc;
-      s_til[r][wave] = tt;
-      s_cnt_long[r][wave] = tc_long;
-      s_til_long[r][wave] = tt_long;
+      sh.cnt[r][wave] = __popcll(has);
+      sh.til[r][wave] = tt;
+      sh.cnt_long[r][wave] = __popcll(has_long);
+      sh.til_long[r][wave] = tt_long;
     }
   }
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < kSums; ++i) before_me[i] += s_base[i][0] + s_base[i][1] + (wave == 1 ? s_tot[i][0] : 0l);
+  for (int i = 0; i < kSums; ++i) before_me[i] += sh.base[i][0] + sh.base[i][1] + (wave == 1 ? sh.tot[i][0] : 0l);  // (a sum without a use stays garbage)
   const long first_row = before_me[0], inp_off = before_me[1], sc_off = before_me[2], out_off = before_me[3];
   if (mine) {
     table[ge] = tag;
     table[p.Et + ge] = first_row;
-    table[2 * p.Et + ge] = inp_off;
-    table[3 * p.Et + ge] = sc_off;
+    if (kind != LayerForm::kGateUp) {
+      table[2 * p.Et + ge] = inp_off;
+      table[3 * p.Et + ge] = sc_off;
+    }
     const void* a_ptr = p.inp + 2 * inp_off;
-    const void* sa_ptr = sld > 0 ? p.scale + 2 * sc_off : nullptr;
+    const void* sa_ptr = scaled ? p.scale + 2 * sc_off : nullptr;
     if (kind == LayerForm::kGateUp) {
       a_ptr = p.form.store[tag];
-      sa_ptr = sld > 0 ? p.form.scales[tag] : nullptr;
+      sa_ptr = scaled ? p.form.scales[tag] : nullptr;
       row_maps[ge] = ge < p.E ? p.form.token_of_row + first_row : p.form.iota;
     } else if (kind == LayerForm::kBehind && tag == 0) {
       a_ptr = p.form.act + 2 * before_me[4];
@@ -255,7 +246,7 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
     if (ge == p.E) misc[1] = (int64_t)(p.out + 2 * out_off);
   }
   // Branches in run order, one per lane (both waves hold the same): entries and tiles before each.
-  const int b_til = lane < info.nb ? s_til[lane][0] + s_til[lane][1] : 0, b_cnt = lane < info.nb ? s_cnt[lane][0] + s_cnt[lane][1] : 0;
+  const int b_til = lane < info.nb ? sh.til[lane][0] + sh.til[lane][1] : 0, b_cnt = lane < info.nb ? sh.cnt[lane][0] + sh.cnt[lane][1] : 0;
   const int til_inc = wave_inclusive_scan(b_til), cnt_inc = wave_inclusive_scan(b_cnt);
   const int total = wave_last(til_inc), ne = wave_last(cnt_inc);
   const int tile0 = til_inc - b_til, ent0 = cnt_inc - b_cnt;
@@ -267,15 +258,15 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
       // inside the branch: [long-K entries of wave 0][of wave 1][other entries of wave 0][of wave 1]
       if (long_k) {
         if (wave == 1) {
-          pos += s_cnt_long[r][0];
-          first += s_til_long[r][0];
+          pos += sh.cnt_long[r][0];
+          first += sh.til_long[r][0];
         }
       } else {
-        pos += s_cnt_long[r][0] + s_cnt_long[r][1];
-        first += s_til_long[r][0] + s_til_long[r][1];
+        pos += sh.cnt_long[r][0] + sh.cnt_long[r][1];
+        first += sh.til_long[r][0] + sh.til_long[r][1];
         if (wave == 1) {
-          pos += s_cnt[r][0] - s_cnt_long[r][0];
-          first += s_til[r][0] - s_til_long[r][0];
+          pos += sh.cnt[r][0] - sh.cnt_long[r][0];
+          first += sh.til[r][0] - sh.til_long[r][0];
         }
       }
       fa->entry[pos] = FusedArgs::Entry{first, sg[j].row0, sg[j].rows, e | (sg[j].branch << 16)};  // problem index relative to the launch's first
@@ -289,7 +280,7 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
     // workgroups of the phases that are one branch (all that may have a successor)
     const int padded = b_til > 0 && ord < kMaxPhases - 1 ? (b_til + kNumXcd - 1) / kNumXcd * kNumXcd : 0;
     const int wg0 = wave_inclusive_scan(padded) - padded;
-    const int flat = wave_last(wave_inclusive_scan(starts && flat_phase(info.b[info.order[min(lane, kMaxBranches - 1)]]) ? 1 << ord : 0));
+    const int flat = wave_last(wave_inclusive_scan(starts && flat_phase(my_branch) ? 1 << ord : 0));
     if (starts) {
       fa->phase_tile0[ord] = tile0;
       fa->phase_wg0[ord] = wg0;
@@ -299,8 +290,8 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
       }
     }
     if (lane == 0) {
-      // rows routed = sum over the routed experts of every launch: the last launch knows them all
-      if (chunk == chunks - 1) misc[0] = s_base[kSums][0] + s_base[kSums][1] + s_routed[0] + s_routed[1];
+      // rows routed: those of every launch without the shared expert's; the last launch knows them all
+      if (chunk == chunks - 1) misc[0] = sh.base[0][0] + sh.base[0][1] + sh.tot[0][0] + sh.tot[0][1] - (p.Et > p.E ? p.shared_rows : 0);
       if (chunk == 0 && p.Et == p.E) misc[1] = 0;
       if (np == 0) fa->phase_tile0[0] = fa->phase_wg0[0] = fa->phase_tile0[1] = fa->phase_wg0[1] = 0;  // a plan without tiles still holds one (empty) phase range
       fa->num_phases = np;

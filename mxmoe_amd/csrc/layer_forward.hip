@@ -27,9 +27,14 @@
 
 namespace mxmoe {
 
-constexpr int kHeadThreads = 256;
-// Experts of the short form: its permutation workgroups keep six counters per expert in LDS (24 KiB at this many).
-constexpr int kHeadMaxExperts = 1024;
+// Threads of the head's workgroups: kHeadSmall up to kHeadSmallMax entries (tokens x top-k), kHeadLarge beyond.  A small batch's head is a
+// chain of latencies, and its tokens are better off on many CUs; workgroups that count a larger batch's ids are bound by their own
+// instructions (32768 ids: 7.7 us with 256 threads, 3.3 with 1024), but tokens in workgroups of 1024 threads fill the chip worse
+// (head of 8192 tokens: 24.3 / 25.3 / 28.9 us with 256 / 512 / 1024 threads, of 2049 tokens with top-6: 17.4 / 16.3 / 19.4).
+constexpr int kHeadSmall = 256, kHeadLarge = 512;
+constexpr int kHeadSmallMax = 4096;
+// Experts of the short form: its permutation workgroups keep up to 26 counters per expert in LDS (52 KiB at this many).
+constexpr int kHeadMaxExperts = 512;
 // Entries (tokens x top-k) up to which every workgroup that needs counts takes them from the ids themselves, all of them: 128 KiB of ids
 // out of L2 and as many LDS counter updates take some 6 us, which the token workgroups of the same launch hide; beyond, the cost
 // per workgroup would grow with the batch, and a counting launch (perm_hist_kernel) goes first.
@@ -38,7 +43,8 @@ constexpr int kHeadCountMax = 65536;
 struct HeadArgs {
   const int32_t* ids;
   int total, E, topk, nbits;
-  int perm_wgs;          // workgroups of kPermChunk entries each
+  int perm_wgs;          // workgroups of one entry per thread
+  int chunks;            // chunks of kPermChunk entries
   const int32_t* hist;   // per-chunk counts, expert-major (perm_hist_stride), or null: count the ids
   int64_t* recv;         // [E] tokens per expert
   int32_t* dst_exp;      // [total] expert of each sorted row
@@ -55,60 +61,86 @@ struct HeadArgs {
 };
 
 // Counts of every expert over all ids (all) and over those before entry `base` (before; not counted when null), by a whole workgroup.
-__device__ __forceinline__ void count_ids(const int32_t* __restrict__ ids, int total, int E, int base, int32_t* before, int32_t* all) {
-  for (int e = threadIdx.x; e < E; e += kHeadThreads) {
-    all[e] = 0;
-    if (before) before[e] = 0;
-  }
+// `copies`: LDS for kCountCopies (all) or twice as many counters per expert: lane l adds to copy l % kCountCopies, since lanes that hit one
+// counter take turns (60 experts: four or five of 64 lanes on average, twenty under a skewed routing).
+constexpr int kCountCopies = 8;
+template <int TH>
+__device__ __forceinline__ void count_ids(const int32_t* __restrict__ ids, int total, int E, int base, int32_t* before, int32_t* all, int32_t* copies) {
+  const int sets = before ? 2 : 1;
+  // the first ids are on their way while the counters are cleared (a barrier waits for every load in front of it, so this one round trip
+  // also covers whatever the caller has just requested)
+  constexpr int kFirst = TH == kHeadSmall ? 8 : 4;
+  int first[kFirst];
+#pragma unroll
+  for (int k = 0; k < kFirst; ++k) first[k] = (int)threadIdx.x + k * TH < total ? gload<int>(ids + threadIdx.x + k * TH) : -1;
+  for (int i = threadIdx.x; i < sets * kCountCopies * E; i += TH) copies[i] = 0;
   __syncthreads();
+  int32_t* const mine = copies + (threadIdx.x % kCountCopies) * E;
+  // (an entry counts in one set only: those before `base` are added to both results at the end)
   auto add = [&](int idx, int e) {
-    if (e >= 0 && e < E) {
-      atomicAdd(&all[e], 1);
-      if (before && idx < base) atomicAdd(&before[e], 1);
-    }
+    if (e >= 0 && e < E) atomicAdd(mine + (before && idx < base ? kCountCopies * E : 0) + e, 1);
   };
-  if ((reinterpret_cast<uintptr_t>(ids) & 15) == 0) {  // 16 bytes per lane and load, eight loads in flight: a handful of round trips for a full batch
-    const int n4 = total >> 2;
+#pragma unroll 1
+  for (int k = 0; k < kFirst && k * TH < total; ++k) {  // (rolled: cold code costs its fetch)
+    add(threadIdx.x + k * TH, first[0]);
+#pragma unroll
+    for (int j = 0; j + 1 < kFirst; ++j) first[j] = first[j + 1];
+  }
+  int done = kFirst * TH;
+  if constexpr (TH == kHeadLarge) {  // 16 bytes per lane and load, eight loads in flight: two round trips for 32768 ids
+    const int n4 = (reinterpret_cast<uintptr_t>(ids) & 15) == 0 ? total >> 2 : 0;
     constexpr int kAhead = 8;
-    for (int i0 = threadIdx.x; i0 < n4; i0 += kAhead * kHeadThreads) {
+    for (int i0 = done / 4 + (int)threadIdx.x; i0 < n4; i0 += kAhead * TH) {
       v4i v[kAhead];
 #pragma unroll
-      for (int k = 0; k < kAhead; ++k) v[k] = reinterpret_cast<const v4i*>(ids)[min(i0 + k * kHeadThreads, n4 - 1)];
+      for (int k = 0; k < kAhead; ++k) v[k] = gload<v4i>(reinterpret_cast<const v4i*>(ids) + min(i0 + k * TH, n4 - 1));
 #pragma unroll
       for (int k = 0; k < kAhead; ++k) {
-        const int i = i0 + k * kHeadThreads;
+        const int i = i0 + k * TH;
         if (i < n4) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) add(4 * i + j, v[k][j]);
         }
       }
     }
-    for (int i = (n4 << 2) + threadIdx.x; i < total; i += kHeadThreads) add(i, ids[i]);
-  } else {
-    for (int i = threadIdx.x; i < total; i += kHeadThreads) add(i, ids[i]);
+    done = max(n4 << 2, done);
+  }
+  for (int i = done + (int)threadIdx.x; i < total; i += TH) add(i, ids[i]);
+  __syncthreads();
+  for (int e = threadIdx.x; e < E; e += TH) {
+    int n = 0, nb = 0;
+#pragma unroll
+    for (int c = 0; c < kCountCopies; ++c) {
+      n += copies[c * E + e];
+      if (before) nb += copies[(kCountCopies + c) * E + e];
+    }
+    all[e] = n + nb;
+    if (before) before[e] = nb;
   }
   __syncthreads();
 }
 
-// One chunk of the stable permutation by expert: each wave places 64 consecutive entries.
+// TH consecutive entries of the stable permutation by expert: each wave places 64.
+template <int TH>
 __device__ __forceinline__ void head_scatter(const HeadArgs& a, int block, int32_t* lds) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int32_t *all = lds, *run = lds + a.E, *in_wave = lds + 2 * a.E;  // [E] totals, [E] first row of this chunk's entries, [4][E] entries per wave
-  const int idx = block * kPermChunk + wave * 64 + lane;
+  constexpr int kWavesHere = TH / 64;
+  int32_t *all = lds, *run = lds + a.E, *in_wave = lds + 2 * a.E;  // [E] totals, [E] first row of this workgroup's entries, [waves][E] entries per wave
+  const int idx = block * TH + threadIdx.x;
   const bool ok = idx < a.total;
   int e = ok ? a.ids[idx] : -1;
   if (e < 0 || e >= a.E) e = a.E;  // parked on a dummy id, never written
-  for (int i = threadIdx.x; i < 4 * a.E; i += kHeadThreads) in_wave[i] = 0;
+  for (int i = threadIdx.x; i < kWavesHere * a.E; i += TH) in_wave[i] = 0;
   if (a.hist) {
-    for (int x = threadIdx.x; x < a.E; x += kHeadThreads) {
+    for (int x = threadIdx.x; x < a.E; x += TH) {
       int v, before;
-      perm_hist_row_sums(a.hist + (long)x * perm_hist_stride(a.perm_wgs), a.perm_wgs, block, &v, &before);
+      perm_hist_row_sums(a.hist + (long)x * perm_hist_stride(a.chunks), a.chunks, block * (TH / kPermChunk), &v, &before);
       all[x] = v;
       run[x] = before;
     }
     __syncthreads();
   } else {
-    count_ids(a.ids, a.total, a.E, block * kPermChunk, run, all);
+    count_ids<TH>(a.ids, a.total, a.E, block * TH, run, all, lds + (2 + kWavesHere) * a.E);
   }
   const uint64_t same = match_same(e, a.nbits);
   const int before = __popcll(same & ((1ull << lane) - 1));
@@ -222,36 +254,43 @@ __device__ __forceinline__ void head_token(const HeadArgs& a, int t, int lane) {
   }
 }
 
-// Workgroups: planning first (the longest chain of dependent steps), then the permutation's chunks, then tokens, four per workgroup.
-template <int NI>
-__global__ void __launch_bounds__(kHeadThreads) layer_head_kernel(const HeadArgs a, const PlanPair pair) {
+// Workgroups: planning first (the longest chain of dependent steps), then the permutation's entries, then tokens, one per wave.
+template <int NI, int TH>
+__global__ void __launch_bounds__(TH) layer_head_kernel(const HeadArgs a, const PlanPair pair) {
   extern __shared__ __align__(16) int32_t head_lds[];
   const int plan_wgs = 2 * pair.chunks;
   int wg = blockIdx.x;
   if (wg < plan_wgs) {
+    __builtin_amdgcn_s_setprio(3);  // one chain of dependent steps against the token waves' full issue slots on the same SIMDs
+    __shared__ PlanShared sh;
+    const PlanParams& p = pair.p[wg / pair.chunks];
+    const int chunk = wg % pair.chunks;
+    mxmoe_block_desc d{};
+    if (threadIdx.x < kPlanThreads) d = plan_block_prepare(p, chunk, sh);
     if (a.hist) {
-      for (int e = threadIdx.x; e < a.E; e += kHeadThreads) {
+      for (int e = threadIdx.x; e < a.E; e += TH) {
         int v, before;
-        perm_hist_row_sums(a.hist + (long)e * perm_hist_stride(a.perm_wgs), a.perm_wgs, 0, &v, &before);
+        perm_hist_row_sums(a.hist + (long)e * perm_hist_stride(a.chunks), a.chunks, 0, &v, &before);
         head_lds[e] = v;
       }
       __syncthreads();
     } else {
-      count_ids(a.ids, a.total, a.E, 0, nullptr, head_lds);
+      count_ids<TH>(a.ids, a.total, a.E, 0, nullptr, head_lds, head_lds + a.E);
     }
-    if (threadIdx.x < kPlanThreads) plan_block_body(pair.p[wg / pair.chunks], wg % pair.chunks, pair.chunks, head_lds);
+    if (threadIdx.x < kPlanThreads) plan_block_body(p, chunk, pair.chunks, head_lds, d, sh);
     return;
   }
   wg -= plan_wgs;
   if (wg < a.perm_wgs) {
-    head_scatter(a, wg, head_lds);
+    __builtin_amdgcn_s_setprio(2);
+    head_scatter<TH>(a, wg, head_lds);
     return;
   }
   wg -= a.perm_wgs;
   const int token_wgs = (int)gridDim.x - plan_wgs - a.perm_wgs;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (int t = wg * 4 + wave; t < a.T; t += token_wgs * 4) head_token<NI>(a, t, lane);
+  for (int t = wg * (TH / 64) + wave; t < a.T; t += token_wgs * (TH / 64)) head_token<NI>(a, t, lane);
 }
 
 // What a layer keeps for one (tokens, top-k): its description and both launches' planning parameters.
@@ -259,7 +298,7 @@ struct LayerForward {
   mxmoe_layer_desc d;
   HeadArgs head;
   PlanPair pair;
-  int et, token_wgs;
+  int et, threads, token_wgs;
   bool fp16_first;   // a first block reads the tokens as they are
   bool rows_step;    // a second block takes quantised (or rotated) rows
   RowsBehind rows;
@@ -336,7 +375,9 @@ int mxmoe_layer_create(const mxmoe_layer_desc* d, void** handle) {
   h.topk = d->topk;
   h.nbits = 1;
   while ((1 << h.nbits) <= d->num_experts) ++h.nbits;  // ids 0..E (E = parked lanes)
-  h.perm_wgs = (h.total + kPermChunk - 1) / kPermChunk;
+  f->threads = h.total <= kHeadSmallMax ? kHeadSmall : kHeadLarge;
+  h.perm_wgs = (h.total + f->threads - 1) / f->threads;
+  h.chunks = (h.total + kPermChunk - 1) / kPermChunk;
   h.hist = h.total > kHeadCountMax ? reinterpret_cast<const int32_t*>(d->workspace) : nullptr;
   h.recv = d->recv;
   h.dst_exp = d->dst_exp;
@@ -353,7 +394,8 @@ int mxmoe_layer_create(const mxmoe_layer_desc* d, void** handle) {
   int dev = 0, cus = 256;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  f->token_wgs = tags ? std::min((d->num_tokens + 3) / 4, cus * 8) : 0;
+  const int per_wg = f->threads / 64;
+  f->token_wgs = tags ? std::min((d->num_tokens + per_wg - 1) / per_wg, cus * 32 / per_wg) : 0;
 
   auto fill = [&](PlanParams& p, int kernel_id, const mxmoe_block_desc* desc, const mxmoe_block_desc* h_desc, void* out, void* plan) {
     p = PlanParams{};
@@ -424,13 +466,18 @@ int mxmoe_layer_run(const void* handle, const void* hidden, const int32_t* topk_
   h.hidden = reinterpret_cast<const _Float16*>(hidden);
   if (f.fp16_first) pair.p[0].form.store[0] = reinterpret_cast<const uint8_t*>(hidden);
   if (h.hist) launch_perm_hist(topk_ids, h.total, h.E, const_cast<int32_t*>(h.hist), true, s);
-  const dim3 grid(2 * pair.chunks + h.perm_wgs + f.token_wgs), block(kHeadThreads);
-  const size_t lds = (size_t)6 * h.E * sizeof(int32_t);
+  const dim3 grid(2 * pair.chunks + h.perm_wgs + f.token_wgs), block(f.threads);
+  const size_t lds = (size_t)(2 + f.threads / 64 + 2 * kCountCopies) * h.E * sizeof(int32_t);
+  auto head = [&](auto ni) {
+    constexpr int NI = decltype(ni)::value;
+    if (f.threads == kHeadSmall) hipLaunchKernelGGL((layer_head_kernel<NI, kHeadSmall>), grid, block, lds, s, h, pair);
+    else hipLaunchKernelGGL((layer_head_kernel<NI, kHeadLarge>), grid, block, lds, s, h, pair);
+  };
   switch (d.hidden / 512) {
-    case 1: hipLaunchKernelGGL((layer_head_kernel<1>), grid, block, lds, s, h, pair); break;
-    case 2: hipLaunchKernelGGL((layer_head_kernel<2>), grid, block, lds, s, h, pair); break;
-    case 4: hipLaunchKernelGGL((layer_head_kernel<4>), grid, block, lds, s, h, pair); break;
-    default: hipLaunchKernelGGL((layer_head_kernel<8>), grid, block, lds, s, h, pair); break;
+    case 1: head(std::integral_constant<int, 1>{}); break;
+    case 2: head(std::integral_constant<int, 2>{}); break;
+    case 4: head(std::integral_constant<int, 4>{}); break;
+    default: head(std::integral_constant<int, 8>{}); break;
   }
   if (const int rc = check_launch()) return rc;
   auto gemm = [&](LaunchPlannedFn fn, const FusedKernel& k, const void* plan, int launch_grid) {

@@ -18,7 +18,11 @@ namespace mxmoe {
 
 __global__ void __launch_bounds__(kPlanThreads) plan_block_kernel(const PlanPair pair) {
   // one workgroup per launch of each block of the layer (gate_up, down): all only read the counts
-  plan_block_body(pair.p[blockIdx.x / pair.chunks], blockIdx.x % pair.chunks, pair.chunks, pair.p[0].recv);
+  __shared__ PlanShared sh;
+  const PlanParams& p = pair.p[blockIdx.x / pair.chunks];
+  const mxmoe_block_desc d = plan_block_prepare(p, blockIdx.x % pair.chunks, sh);
+  __syncthreads();
+  plan_block_body(p, blockIdx.x % pair.chunks, pair.chunks, pair.p[0].recv, d, sh);
 }
 
 // Permutation and planning of a decode-sized batch (at most kPermChunk (token, slot) entries) in ONE launch: workgroup 0 builds the
@@ -39,6 +43,9 @@ __global__ void __launch_bounds__(kPlanThreads) perm_plan_small_kernel(const Per
     perm_small_body(a.ids, a.total, a.E, a.topk, a.nbits, a.recv, a.dst, a.perm, a.slot, a.row_of_slot, reinterpret_cast<int32_t*>(pp_lds), threadIdx.x < 64);
     return;
   }
+  __shared__ PlanShared sh;
+  const int b = blockIdx.x - 1, chunk = b % pair.chunks;
+  const mxmoe_block_desc d = plan_block_prepare(pair.p[b / pair.chunks], chunk, sh);
   int64_t* counts = reinterpret_cast<int64_t*>(pp_lds);
   unsigned long long* cnt = reinterpret_cast<unsigned long long*>(pp_lds);
   for (int e = threadIdx.x; e < a.E; e += kPlanThreads) counts[e] = 0;
@@ -48,8 +55,7 @@ __global__ void __launch_bounds__(kPlanThreads) perm_plan_small_kernel(const Per
     if (e >= 0 && e < a.E) atomicAdd(&cnt[e], 1ull);
   }
   __syncthreads();
-  const int b = blockIdx.x - 1;
-  plan_block_body(pair.p[b / pair.chunks], b % pair.chunks, pair.chunks, counts);
+  plan_block_body(pair.p[b / pair.chunks], chunk, pair.chunks, counts, d, sh);
 }
 
 // The same for larger batches, after perm_hist_kernel has counted the experts per chunk of kPermChunk entries: the first `blocks`
@@ -73,6 +79,9 @@ __global__ void __launch_bounds__(kPlanThreads) perm_scatter_plan_kernel(const P
                       reinterpret_cast<int32_t*>(pp_lds), threadIdx.x < 64);
     return;
   }
+  __shared__ PlanShared sh;
+  const int b = blockIdx.x - a.blocks, chunk = b % pair.chunks;
+  const mxmoe_block_desc d = plan_block_prepare(pair.p[b / pair.chunks], chunk, sh);
   int64_t* counts = reinterpret_cast<int64_t*>(pp_lds);
   for (int e = threadIdx.x; e < a.E; e += kPlanThreads) {
     int v, before;
@@ -80,8 +89,7 @@ __global__ void __launch_bounds__(kPlanThreads) perm_scatter_plan_kernel(const P
     counts[e] = v;
   }
   __syncthreads();
-  const int b = blockIdx.x - a.blocks;
-  plan_block_body(pair.p[b / pair.chunks], b % pair.chunks, pair.chunks, counts);
+  plan_block_body(pair.p[b / pair.chunks], chunk, pair.chunks, counts, d, sh);
 }
 
 // Kernel for the formats of `h_desc`, checked once on the host: every problem's format has a branch and its shape fits it.
@@ -175,7 +183,7 @@ int mxmoe_plan_grid_bound(int kernel_id, const mxmoe_block_desc* h_desc, int num
     Segment sg[2];
     const int ns = plan_segments(pi, f, m, n, sg);
     int t = 0;
-    for (int j = 0; j < ns; ++j) t += segment_tiles(pi, sg[j], n);
+    for (int j = 0; j < ns; ++j) t += sg[j].tiles;
     return t;
   };
   // And tiles(M) <= extra + per_row * M, with per_row the columns per row of the shape that very long problems run on and extra the
@@ -198,7 +206,8 @@ int mxmoe_plan_grid_bound(int kernel_id, const mxmoe_block_desc* h_desc, int num
     if (!hit) {
       Segment sg[2];
       plan_segments(pi, f, 1 << 20, n, sg);
-      const int bm = pi.b[sg[0].branch].BM, cols = (n + pi.b[sg[0].branch].BN - 1) / pi.b[sg[0].branch].BN;
+      const BranchInfo& bi = registry()[kid].branches[sg[0].branch];
+      const int bm = bi.BM, cols = (n + bi.BN - 1) / bi.BN;
       Seen sn{f, n, tiles_of(f, 1, n), 0, 0.0, (double)cols / bm};
       const int limit = std::min(std::max(routed_rows_max, 2), 64 * bm);
       for (int m = 1; m <= limit; ++m) {
