@@ -216,7 +216,9 @@ struct MfmaTile {
   static constexpr int kBits = OpTraits<OP>::kBitsPerElem;
   static constexpr int BK = kRowBytes * 8 / kBits;  // K elements per pipeline stage: 64 (int8), 128 (int4), 32 (fp16)
   static constexpr int kStageBytes = (BM + BN) * kRowBytes;
-  static constexpr int kStages = 3;
+  // as many LDS stages as let two workgroups share a CU's 160 KB
+  static constexpr int kStages = 80 * 1024 / kStageBytes < 4 ? 80 * 1024 / kStageBytes : 4;
+  static_assert(kStages >= 3, "the read-ahead of the main loop needs three stages");
   static constexpr int kLdsBytes = kStages * kStageBytes;
   static constexpr int kAccRegs = FM * FN * 16;
   static constexpr int kWavesWanted = 2;  // waves per SIMD a kernel of such tiles is compiled for
@@ -303,10 +305,14 @@ struct MfmaTile {
     // unit of a k-step and widened, a few registers per unit, into a second operand buffer during its last units.  So LDS
     // latency (which grows well beyond its idle value while direct-to-LDS loads are landing) and the unpack VALU work hide
     // under the matrix pipe, and the VALU work is spread evenly between the MFMAs.
-    // Three LDS stages let the read-ahead run into the next K slice:
-    //   iteration kt:  the loads of slice kt+2 into stage (kt+2)%3 are issued one or two per unit (a burst of them delays the
-    //   LDS reads of every wave on the CU); units 0..UB-1 touch stage kt%3 only; at unit UB the wave waits for its loads of
-    //   slice kt+1 and passes the barrier; the remaining units also read stage (kt+1)%3.
+    // The LDS stages (S of them) let the read-ahead run into the next K slice:
+    //   iteration kt:  units 0..UB-1 touch stage kt%S only; at unit UB the wave waits for its loads of slice kt+1 and passes the
+    //   barrier; the remaining units also read stage (kt+1)%S.  Stage kt%S is free from that barrier on: the loads of slice kt+S are
+    //   issued right behind it, one or two per unit (a burst of them delays the LDS reads of every wave on the CU) through unit UB-1 of
+    //   the next iteration, so that S-1 whole slices are in flight or landed at any time and a load has S-1 iterations to arrive.
+    // (With few rows per expert the weight stream bounds the launch, and what it reaches follows the bytes in flight: 692 MB of fp16
+    // gate_up weights at 64 tokens take 131 us, 5.3 TB/s, against 163 with three stages whose loads began a whole barrier later; 512
+    // tokens 150 against 176.  With hundreds of rows it is the rate of 64-byte requests to L2 that bounds it, and this is neutral.)
     // The loop body is branch-free: past the end of K the loads are zero-length (they fetch nothing) and the read-ahead touches
     // a stage whose contents are never used.
     constexpr int U = 2 * FN;  // units per K slice
@@ -317,10 +323,9 @@ struct MfmaTile {
     constexpr int NW = FN >= 4 ? 2 : 1;              // units over which the next k-step's A operands are widened
     constexpr int kAPiece = FM * 4 / NW;             // dwords of packed A widened per such unit
     constexpr int kOps = OP == Op::I4 ? 2 : 1;       // operand registers per fragment (low / high nibbles)
-    // load i of a slice is issued at the top of unit i * U / kDma; at the barrier unit the loads of the current iteration issued
-    // so far are the only ones that may still be in flight
-    constexpr int kIssuedAtBarrier = ((UB + 1) * kDma + U - 1) / U;
-    constexpr bool kLastBeforeBarrier = (kDma - 1) * U / kDma <= UB;
+    // load i of a slice is issued in unit UB + i * U / kDma, counted from the iteration whose barrier freed its stage; the loads of
+    // slices kt+2 .. kt+S-1 are the ones that may still be in flight at the barrier of iteration kt
+    constexpr int S = kStages, kYounger = (S - 2) * kDma, kYoungerLess = (S - 2) * (kDma - 1);
     auto lds_a = [&](const uint8_t* st, int step, int i) { return *reinterpret_cast<const v4i*>(st + ((fa + i * 32 * kRowBytes) ^ (step << 5))); };
     auto lds_b = [&](const uint8_t* st, int step, int j) { return *reinterpret_cast<const v4i*>(st + ((fb + j * 32 * kRowBytes) ^ (step << 5))); };
     // nibble n of a byte -> int8 holding 16 * signed(n): even elements via (x << 4), odd via x, both masked to the high nibbles
@@ -351,35 +356,37 @@ struct MfmaTile {
     v4i pb[RB];            // packed B fragments of units u+1 .. u+LA
     v4i bop[2][kOps];      // B operands of units u, u+1
 
-    // prologue: slices 0 and 1 in flight, wait for slice 0 (loads retire in order), prime the fragment pipeline
+    // prologue: slices 0 .. S-2 in flight, wait for slice 0 (loads retire in order), the part of slice S-1 that an iteration before the
+    // first would have issued, prime the fragment pipeline
 #pragma unroll
-    for (int i = 0; i < kDma; ++i) dma_one(i, 0, 0, true);
+    for (int k = 0; k < S - 1; ++k)
 #pragma unroll
-    for (int i = 0; i < kDma; ++i) dma_one(i, kRowBytes, 1, KT > 1);
-    if (has_last) vm_wait<kDma>(); else vm_wait<kDma - 1>();
+      for (int i = 0; i < kDma; ++i) dma_one(i, k * kRowBytes, k, KT > k);
+    if (has_last) vm_wait<kYounger>(); else vm_wait<kYoungerLess>();
     __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kDma; ++i)
+      if (UB + i * U / kDma < U) dma_one(i, (S - 1) * kRowBytes, S - 1, KT > S - 1);
 #pragma unroll
     for (int i = 0; i < FM; ++i) widen(lds_a(smem, 0, i), aop[0][i]);
 #pragma unroll
     for (int u = 1; u < LA; ++u) pb[u] = lds_b(smem, u / FN, u % FN);
     widen(lds_b(smem, 0, 0), bop[0]);
 
-    int sidx = 0;
+    int sidx = 0, pidx = S - 1;  // stages of slices kt, kt-1
 #pragma unroll 1
     for (int kt = 0; kt < KT; ++kt) {
       const uint8_t* sc = smem + sidx * kStageBytes;
-      const int nidx = sidx == 2 ? 0 : sidx + 1;
+      const int nidx = sidx == S - 1 ? 0 : sidx + 1;
       const uint8_t* sn = smem + nidx * kStageBytes;
-      // slice kt+2 goes into the stage that was last read before the previous iteration's barrier
-      const int nstage = nidx == 2 ? 0 : nidx + 1;
-      const int nkoff = __builtin_amdgcn_readfirstlane((kt + 2) * kRowBytes);
-      const bool nlive = kt + 2 < KT;
+      const int nkoff = __builtin_amdgcn_readfirstlane((kt + S) * kRowBytes);
       static_for<U>([&](auto uc) {
         constexpr int u = decltype(uc)::value;
         constexpr int step = u / FN, j = u % FN;
         static_for<kDma>([&](auto ic) {
           constexpr int i = decltype(ic)::value;
-          if constexpr (i * U / kDma == u) dma_one(i, nkoff, nstage, nlive);
+          constexpr int at = UB + i * U / kDma;
+          if constexpr (at >= U && at - U == u) dma_one(i, nkoff - kRowBytes, pidx, kt + S - 1 < KT);
         });
         // reads of this slice's stage: packed B fragment of unit u+LA, A fragments of k-step 1
         if (u + LA < U) pb[(u + LA) % RB] = lds_b(sc, (u + LA) / FN, (u + LA) % FN);
@@ -390,11 +397,15 @@ struct MfmaTile {
           }
         }
         if (u == UB) {
-          // this wave's part of slice kt+1 is in LDS (only its loads of slice kt+2 may be in flight); after the barrier
-          // everybody's part is, and everybody is done reading the stage that the next iteration's loads overwrite
-          if (!kLastBeforeBarrier || has_last) vm_wait<kIssuedAtBarrier>(); else vm_wait<kIssuedAtBarrier - 1>();
+          // this wave's part of slice kt+1 is in LDS (only its loads of later slices may be in flight); after the barrier
+          // everybody's part is, and everybody is done reading stage kt%S, which the loads below overwrite
+          if (has_last) vm_wait<kYounger>(); else vm_wait<kYoungerLess>();
           __syncthreads();
         }
+        static_for<kDma>([&](auto ic) {
+          constexpr int i = decltype(ic)::value;
+          if constexpr (UB + i * U / kDma == u) dma_one(i, nkoff, sidx, kt + S < KT);
+        });
         // reads of the next slice's stage
         if (u + LA >= U) pb[(u + LA) % RB] = lds_b(sn, (u + LA - U) / FN, (u + LA - U) % FN);
         if (u == FN) {
@@ -421,6 +432,7 @@ struct MfmaTile {
         sched_mfma_valu<(OP == Op::I4 ? 12 + (j >= FN - NW ? 3 * kAPiece : 0) : 0), kOps * FM, 0>();
         __builtin_amdgcn_sched_barrier(0);  // keep the units in program order: the pipeline above is the schedule
       });
+      pidx = sidx;
       sidx = nidx;
     }
     vm_wait<0>();  // nothing may still land in LDS once the epilogue reuses it
