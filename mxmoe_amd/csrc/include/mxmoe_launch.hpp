@@ -407,12 +407,28 @@ struct Segment {
   int row0, rows, branch, tiles;
 };
 
+// Tiles of a long-K problem from which on the launch is as busy with them as with the rest (a quarter of the 512 workgroups that run at a time).
+constexpr int kLongTiles = 128;
+// Whether a problem of a launch whose smallest K is `kmin` counts as long: above that, and a tile of it takes long at all (a 128 x 256
+// weight-only tile 2.4 us per 128 of K: 40 us, a whole launch of few-row experts).
+constexpr int kLongK = 2048;
+__host__ __device__ inline bool runs_long(int K, int kmin) { return K > kmin && K >= kLongK; }
+
 // Split the M rows of an M x N problem into at most two segments: whole tiles of the shape that is cheapest per output element,
 // then the remainder with the shape that covers it most cheaply (cost of a block run with one shape = row tiles * column tiles *
 // tile_cost).  Returns the number of segments (0 for M == 0), or -1 when the kernel has no tile for `f`.
 // Two rolled loops on purpose: the device planner runs this once per launch, when none of its code is in the instruction cache, and
 // what it costs there is the fetching of its instructions.
-__host__ __device__ inline int plan_segments(const PlanInfo& k, int f, int M, int N, Segment out[2]) {
+//
+// `long_k`: runs_long of the problem (a shared expert behind several intermediates' width).  Its tiles run that
+// many times longer than the others', and a launch is not over before they are: as long as the problem has too few tiles to share the
+// chip with the rest, what counts is the time of one.  Where the choice by total cost takes the largest shape, such a problem takes the one
+// of the smallest max(tile_cost, tiles * tile_cost / kLongTiles) instead.  Weight-only formats: the 32-token tile up to some 600 rows.  The
+// 16-, 8- and 4-bit operand formats do that up to one large row tile only: their shorter tiles need half as long, not a third, for a
+// quarter of the rows (201 .. 800 rows measured slower).  Down launch with 60 experts and a shared expert of four times their width, us,
+// large shape -> this rule: w4a16 / w3a16 103 -> 36 (100 tokens), 103 -> 40 (201), 106 -> 58 (400); w4a4 45 -> 31, w4a4 / w8a8 49 -> 40, fp16
+// 151 -> 128 (100); 64 experts and twice the width: w4a16 / w3a16 61 -> 37 (128), 60 -> 41 (201), 80 -> 67 (600), w8a16 / w2a16 60 -> 44 (128).
+__host__ __device__ inline int plan_segments(const PlanInfo& k, int f, int M, int N, bool long_k, Segment out[2]) {
   if (f < 0 || f >= kNumFmts) return -1;
   const int lo = k.fmt_start[f], hi = k.fmt_start[f + 1];
   if (lo == hi) return -1;
@@ -429,20 +445,27 @@ __host__ __device__ inline int plan_segments(const PlanInfo& k, int f, int M, in
       best.cost = c;
     }
   };
-  Pick unit, whole;  // cheapest per row of the problem; cheapest for all of it
+  Pick unit, whole, quick;  // cheapest per row of the problem; cheapest for all of it; soonest done on a part of the chip
   int full = 0;
   double full_cost = 0;
 #pragma unroll 1
   for (int i = lo; i < hi; ++i) {
     const PlanBranch& b = k.b[i];
     const int tm = tiles_over(M, b.bm_log2), tn = tiles_over(N, b.bn_log2), rows = M >> b.bm_log2 << b.bm_log2;
-    offer(whole, b, tm * tn, (double)tm * tn * b.cost, 1e-9);
+    const double all = (double)tm * tn * b.cost, share = all * (1.0 / kLongTiles);
+    offer(whole, b, tm * tn, all, 1e-9);
+    offer(quick, b, tm * tn, share > b.cost ? share : b.cost, 1e-9);
     const int had = unit.branch;
     offer(unit, b, (M >> b.bm_log2) * tn, b.cost_per_row * tn, 1e-12);
     if (unit.branch != had) {
       full = rows;
       full_cost = (double)(M >> b.bm_log2) * tn * b.cost;
     }
+  }
+  const bool large = full > 0 || whole.branch == unit.branch;
+  if (long_k && large && quick.branch != unit.branch && whole.tiles < kLongTiles && (M <= 128 || is_weight_only((Fmt)f))) {
+    out[0] = Segment{0, M, quick.branch, quick.tiles};
+    return 1;
   }
   const int rem = M - full;
   out[0] = Segment{0, M, whole.branch, whole.tiles};
@@ -635,7 +658,7 @@ inline bool kernel_covers(const FusedKernel& k, const mxmoe_qparams* q, int coun
   for (int i = 0; i < count; ++i) {
     const Fmt f = classify(q[i]);
     Segment sg[2];
-    if (f == Fmt::UNSUPPORTED || plan_segments(plan_of(k), (int)f, 1, 256, sg) < 0) return false;
+    if (f == Fmt::UNSUPPORTED || plan_segments(plan_of(k), (int)f, 1, 256, false, sg) < 0) return false;
   }
   return true;
 }
@@ -685,11 +708,13 @@ inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, c
   };
   Entry entries[kMaxEntries];
   int nent = 0;
+  uint32_t kmin = ~0u;
+  for (int i = 0; i < n; ++i) kmin = std::min(kmin, h_sizes[base + i].z);
   for (int i = 0; i < n; ++i) {
     const mxmoe_dim3& sz = h_sizes[base + i];
     const Fmt f = classify(h_q[base + i]);
     Segment sg[2];
-    const int ns = f == Fmt::UNSUPPORTED ? -1 : plan_segments(pi, (int)f, (int)sz.x, (int)sz.y, sg);
+    const int ns = f == Fmt::UNSUPPORTED ? -1 : plan_segments(pi, (int)f, (int)sz.x, (int)sz.y, runs_long((int)sz.z, (int)kmin), sg);
     if (ns < 0) {
       last_error() = "quant type not supported";
       return 1;
@@ -709,8 +734,6 @@ inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, c
   // run longest: a shared expert with a wider intermediate, say; workgroups are dispatched in index order, and the longest
   // jobs first is what keeps the tail of the launch short), then the others; problems keep their order otherwise (neighbouring tiles
   // share operands).
-  uint32_t kmin = ~0u;
-  for (int i = 0; i < n; ++i) kmin = std::min(kmin, h_sizes[base + i].z);
   int total = 0, ne = 0, wg = 0, np = 0;
   for (int oi = 0; oi < pi.nb; ++oi) {
     const PlanBranch& pb = pi.b[pi.order[oi]];

@@ -177,11 +177,11 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
   // smallest K of the launch: problems above it run first inside their branch (see launch_range)
   const int km = -wave_last(wave_inclusive_max(mine ? -K : -0x7fffffff));
   if (lane == 0) sh.kmin[wave] = km;
-  // segments of this problem (no need of the other wave)
-  Segment sg[2];
-  const int ns = mine ? plan_segments(info, fmt, (int)rows, N, sg) : 0;
   __syncthreads();
-  const bool long_k = mine && K > min(sh.kmin[0], sh.kmin[1]);
+  const int kmin = min(sh.kmin[0], sh.kmin[1]);
+  const bool long_k = mine && K > kmin;
+  Segment sg[2];
+  const int ns = mine ? plan_segments(info, fmt, (int)rows, N, runs_long(K, kmin), sg) : 0;
   // per branch in run order, this wave's entries and tiles
   int seg_rank[2] = {-1, -1}, seg_pos[2] = {0, 0}, seg_first[2] = {0, 0};
   const PlanBranch& my_branch = info.b[info.order[min(lane, kMaxBranches - 1)]];  // lane r: the branch of rank r

@@ -99,7 +99,7 @@ int resolve_kernel(int kernel_id, const mxmoe_block_desc* h_desc, int et) {
     for (int i = 0; i < et; ++i) {
       Segment sg[2];
       const int f = fmt_of(h_desc[i].q);
-      if (f == (int)Fmt::UNSUPPORTED || plan_segments(plan_of(k), f, 1, 256, sg) < 0) return false;
+      if (f == (int)Fmt::UNSUPPORTED || plan_segments(plan_of(k), f, 1, 256, false, sg) < 0) return false;
       // a kernel's w4a4 tiles take packed int4 rows or bf6 fragments, never both: the descriptor says which the block will get
       if (f == (int)Fmt::W4A4 && kernel_takes_bf6(k) != wants_bf6(h_desc[i].q)) return false;
       if (f == (int)Fmt::W8A8 && (kernel_variant(k, Fmt::W8A8) == kVariantFp8) != wants_fp8(h_desc[i].q)) return false;
@@ -179,39 +179,49 @@ int mxmoe_plan_grid_bound(int kernel_id, const mxmoe_block_desc* h_desc, int num
   // For every routed expert tiles(M) <= first + slope * (M - 1) for all M >= 1, with first = tiles(1) and slope the steepest rise
   // found by walking M over 64 rows of the format's largest tile (the planner's decisions repeat with that tile's period).  With at
   // most n = min(experts, rows) experts non-empty, the launch has at most (sum of the n largest `first`) + max slope * (rows - n) tiles.
-  auto tiles_of = [&](int f, int m, int n) {
-    Segment sg[2];
-    const int ns = plan_segments(pi, f, m, n, sg);
-    int t = 0;
-    for (int j = 0; j < ns; ++j) t += sg[j].tiles;
-    return t;
+  // A block that is long against the smallest K may be so in its launch (or not, when the block is run as several launches): the
+  // larger count holds.
+  auto tiles_of = [&](int f, int m, int n, bool maybe_long) {
+    int most = 0;
+    for (int lk = 0; lk <= (maybe_long ? 1 : 0); ++lk) {
+      Segment sg[2];
+      const int ns = plan_segments(pi, f, m, n, lk != 0, sg);
+      int t = 0;
+      for (int j = 0; j < ns; ++j) t += sg[j].tiles;
+      most = std::max(most, t);
+    }
+    return most;
   };
+  uint32_t kmin = ~0u;
+  for (int e = 0; e < et; ++e) kmin = std::min(kmin, (uint32_t)h_desc[e].K);
   // And tiles(M) <= extra + per_row * M, with per_row the columns per row of the shape that very long problems run on and extra the
   // largest excess over it: the smaller of the two sums holds.
   long shared_tiles = 0;
   double slope = 0, per_row = 0;
   long extras = 0;
   std::vector<int> firsts;
-  struct Seen { int f, n, first, extra; double slope, per_row; };
+  struct Seen { int f, n, maybe_long, first, extra; double slope, per_row; };
   std::vector<Seen> seen;
   for (int e = 0; e < et; ++e) {
     const int f = fmt_of(h_desc[e].q), n = (int)h_desc[e].N;
+    const bool maybe_long = runs_long((int)h_desc[e].K, (int)kmin);
     if (e >= num_experts) {  // the shared expert's row count is known
-      shared_tiles += tiles_of(f, shared_rows, n);
+      shared_tiles += tiles_of(f, shared_rows, n, maybe_long);
       continue;
     }
     const Seen* hit = nullptr;
     for (const Seen& sn : seen)
-      if (sn.f == f && sn.n == n) hit = &sn;
+      if (sn.f == f && sn.n == n && sn.maybe_long == maybe_long) hit = &sn;
     if (!hit) {
       Segment sg[2];
-      plan_segments(pi, f, 1 << 20, n, sg);
+      plan_segments(pi, f, 1 << 20, n, false, sg);
       const BranchInfo& bi = registry()[kid].branches[sg[0].branch];
       const int bm = bi.BM, cols = (n + bi.BN - 1) / bi.BN;
-      Seen sn{f, n, tiles_of(f, 1, n), 0, 0.0, (double)cols / bm};
-      const int limit = std::min(std::max(routed_rows_max, 2), 64 * bm);
+      Seen sn{f, n, maybe_long, tiles_of(f, 1, n, maybe_long), 0, 0.0, (double)cols / bm};
+      // (a long block of one column may be short of kLongTiles tiles for that many row tiles)
+      const int limit = std::min(std::max(routed_rows_max, 2), std::max(64, maybe_long ? kLongTiles + 1 : 0) * bm);
       for (int m = 1; m <= limit; ++m) {
-        const int t = tiles_of(f, m, n);
+        const int t = tiles_of(f, m, n, maybe_long);
         if (m > 1) sn.slope = std::max(sn.slope, (double)(t - sn.first) / (m - 1));
         sn.extra = std::max(sn.extra, t - (m / bm) * cols);
       }
