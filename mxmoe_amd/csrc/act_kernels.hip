@@ -265,8 +265,7 @@ __device__ __forceinline__ int xcd_row_group(int wg) { return (wg & ~63) | ((wg 
 
 // NT threads per workgroup (256, or 192 when that wastes fewer lanes: a 1408-element row is 176 chunks of 8).
 template <int MAXC, bool SILU, int NT, bool EXT>
-__global__ void __launch_bounds__(NT) row_quant_kernel(const RowArgs a) {
-  extern __shared__ __align__(16) float lds[];
+__device__ __forceinline__ void row_quant_body(const RowArgs& a, const int wg, const int wgs, float* const lds) {
   const int tid = threadIdx.x;
   const int nmax = max(a.plan.n, a.plan_shared.n);
   float* x = lds;                  // [nmax]
@@ -329,12 +328,12 @@ __global__ void __launch_bounds__(NT) row_quant_kernel(const RowArgs a) {
   };
   RowMeta next_meta;
   v8h next_g[MAXC], next_u[MAXC];
-  if ((int)blockIdx.x < a.rows) {
-    next_meta = load_meta(blockIdx.x);
+  if (wg < a.rows) {
+    next_meta = load_meta(wg);
     load_data(next_meta, next_g, next_u);
   }
 
-  for (int row = blockIdx.x; row < a.rows; row += gridDim.x) {
+  for (int row = wg; row < a.rows; row += wgs) {
     const RowMeta cur = next_meta;
     v8h cur_g[MAXC], cur_u[MAXC];
 #pragma unroll
@@ -342,8 +341,8 @@ __global__ void __launch_bounds__(NT) row_quant_kernel(const RowArgs a) {
       cur_g[i] = next_g[i];
       if (SILU) cur_u[i] = next_u[i];
     }
-    if (row + (int)gridDim.x < a.rows) {
-      next_meta = load_meta(row + gridDim.x);
+    if (row + wgs < a.rows) {
+      next_meta = load_meta(row + wgs);
       load_data(next_meta, next_g, next_u);
     }
     if (!cur.exists) continue;  // (the whole workgroup: a row belongs to one workgroup)
@@ -648,6 +647,11 @@ __global__ void __launch_bounds__(NT) row_quant_kernel(const RowArgs a) {
       }
     }
   }
+}
+template <int MAXC, bool SILU, int NT, bool EXT>
+__global__ void __launch_bounds__(NT) row_quant_kernel(const RowArgs a) {
+  extern __shared__ __align__(16) float lds[];
+  row_quant_body<MAXC, SILU, NT, EXT>(a, blockIdx.x, gridDim.x, lds);
 }
 
 // One row per WAVE, for rows whose rotation is a pure Sylvester transform (n = 512 * NI, NI a power of two): lane l holds the NI
@@ -964,8 +968,7 @@ constexpr int kDensePitch = 144;             // bytes per column of the transpos
 __host__ __device__ constexpr int dense_wave_lds(int n) { return 32 * kDensePitch + (n + 8) * 2; }
 __host__ __device__ constexpr int dense_lds(int n, int kb) { return ((kb + 15) >> 4) * ((kb + 31) >> 5) * 1024 + 4 * dense_wave_lds(n); }
 template <int MAXC, bool SILU, bool EXT>
-__global__ void __launch_bounds__(256) row_quant_dense_kernel(const RowArgs a) {
-  extern __shared__ __align__(16) uint8_t dlds[];
+__device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int wg, const int wgs, uint8_t* const dlds) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lm = lane & 15, lg = lane >> 4;
@@ -1026,12 +1029,12 @@ __global__ void __launch_bounds__(256) row_quant_dense_kernel(const RowArgs a) {
       if (SILU) u[i] = *reinterpret_cast<const v8h*>(m.srow + n + c * 8);
     }
   };
-  const int stride_rows = gridDim.x * 4;
+  const int stride_rows = wgs * 4;
   // One row ahead: the bookkeeping of the next row (a chain of dependent loads) is fetched at the top of a row, its data as soon as
   // this row's data has been turned into values, so the same registers hold both and the loads fly under the rotation and the stores.
   RowMeta next_meta;
   v8h row_g[MAXC], row_u[MAXC];
-  const int row0 = xcd_row_group(blockIdx.x) * 4 + wave;
+  const int row0 = xcd_row_group(wg) * 4 + wave;
   if (row0 < a.rows) {
     next_meta = load_meta(row0);
     load_data(next_meta, row_g, row_u);
@@ -1290,6 +1293,22 @@ __global__ void __launch_bounds__(256) row_quant_dense_kernel(const RowArgs a) {
       }
     }
   }
+}
+template <int MAXC, bool SILU, bool EXT>
+__global__ void __launch_bounds__(256) row_quant_dense_kernel(const RowArgs a) {
+  extern __shared__ __align__(16) uint8_t dlds[];
+  row_quant_dense_body<MAXC, SILU, EXT>(a, blockIdx.x, gridDim.x, dlds);
+}
+
+// Routed rows by row_quant_dense_kernel's code and the shared expert's rows, of another length, by row_quant_kernel's, next to each other in
+// one launch: neither needs anything of the other, and a launch of a few hundred shared rows is one long chain per row (15 us) on a chip
+// that is mostly idle.  The first `shared_wgs` workgroups (a multiple of 64: xcd_row_group) take the shared rows, which run longest.
+template <int MAXC, bool EXT>
+__global__ void __launch_bounds__(256) row_quant_pair_kernel(const RowArgs routed, const RowArgs shared, const int shared_wgs) {
+  extern __shared__ __align__(16) uint8_t plds[];
+  const int wg = blockIdx.x;
+  if (wg < shared_wgs) row_quant_body<3, false, 256, EXT>(shared, wg, shared_wgs, reinterpret_cast<float*>(plds));
+  else row_quant_dense_body<MAXC, false, EXT>(routed, wg - shared_wgs, (int)gridDim.x - shared_wgs, plds);
 }
 
 // One row per WORKGROUP of 8 waves for rotations B_kb kron H_512 (kb <= 32, no Sylvester factor in the table: a 14336-value row is
@@ -1556,6 +1575,7 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
 }
 
 constexpr int kSplitSharedRows = 512;
+constexpr int kPairSharedRows = 2304;  // (row_quant_pair_kernel)
 
 static int make_plan(int n, int had_k, int had_f, bool rotate, RotPlan* p) {
   p->n = n;
@@ -1573,6 +1593,37 @@ static int make_plan(int n, int had_k, int had_f, bool rotate, RotPlan* p) {
   return 0;
 }
 
+// Rows that row_quant_dense_kernel and row_quant_wide_kernel take: one length, a table-driven factor times H_8 / times H_512.
+static bool dense_rows(const RowArgs& a) {
+  return a.plan.kb > 1 && a.plan.m == 8 && a.plan.f <= 4 && a.plan.kb <= 64 && a.plan.n <= 2048 && a.plan_shared.n == a.plan.n && a.plan_shared.kb == a.plan.kb && a.rotate != 0;
+}
+static bool wide_rows(const RowArgs& a) {
+  return a.plan.kb > 1 && a.plan.kb <= 32 && a.plan.m == 512 && a.plan.f == 1 && a.plan_shared.n == a.plan.n && a.plan_shared.kb == a.plan.kb && a.rotate != 0;
+}
+
+template <bool EXT>
+static int launch_pair(const RowArgs& routed, const RowArgs& shared, int lds_bytes, hipStream_t s) {
+  int dev = 0, cus = 256;
+  (void)hipGetDevice(&dev);
+  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  const int lds = std::max(lds_bytes, dense_lds(routed.plan.n, routed.plan.kb));  // (dense_rows: below 64 KiB)
+  const int shared_wgs = std::min(shared.rows, cus * 2) + 63 & ~63;
+  const int routed_wgs = std::min((routed.rows + 3) / 4, cus * 3) + 63 & ~63;
+  const dim3 grid(shared_wgs + routed_wgs);
+  switch ((routed.plan.n / 8 + 63) / 64) {
+    case 1: hipLaunchKernelGGL((row_quant_pair_kernel<1, EXT>), grid, dim3(256), lds, s, routed, shared, shared_wgs); break;
+    case 2: hipLaunchKernelGGL((row_quant_pair_kernel<2, EXT>), grid, dim3(256), lds, s, routed, shared, shared_wgs); break;
+    case 3: hipLaunchKernelGGL((row_quant_pair_kernel<3, EXT>), grid, dim3(256), lds, s, routed, shared, shared_wgs); break;
+    default: hipLaunchKernelGGL((row_quant_pair_kernel<4, EXT>), grid, dim3(256), lds, s, routed, shared, shared_wgs); break;
+  }
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    last_error() = std::string("kernel launch failed: ") + hipGetErrorString(e);
+    return 4;
+  }
+  return 0;
+}
+
 template <bool SILU, bool EXT>
 static int launch_rows_as(const RowArgs& a, int lds_bytes, hipStream_t s) {
   // Shared rows of another length keep the routed rows out of the kernels made for one length: from some hundred rows on, two launches
@@ -1584,6 +1635,10 @@ static int launch_rows_as(const RowArgs& a, int lds_bytes, hipStream_t s) {
     shared.R = 0;
     shared.rows = a.rows - a.R;
     shared.plan = a.plan_shared;
+    if constexpr (!SILU) {
+      if (shared.rows <= kPairSharedRows && dense_rows(routed) && !dense_rows(shared) && !wide_rows(shared) && shared.plan.kb > 1 && shared.plan.n <= 8 * 256 * 3 && lds_bytes <= 64 * 1024)
+        return launch_pair<EXT>(routed, shared, lds_bytes, s);
+    }
     const int rc = launch_rows_as<SILU, EXT>(routed, lds_bytes, s);
     return rc ? rc : launch_rows_as<SILU, EXT>(shared, lds_bytes, s);
   }
@@ -1616,7 +1671,7 @@ static int launch_rows_as(const RowArgs& a, int lds_bytes, hipStream_t s) {
     return 0;
   }
   // table-driven factor times H_8, one size of row: one row per wave, dense stage on the matrix cores
-  if (a.plan.kb > 1 && a.plan.m == 8 && a.plan.f <= 4 && a.plan.kb <= 64 && n <= 2048 && a.plan_shared.n == n && a.plan_shared.kb == a.plan.kb && a.rotate != 0) {
+  if (dense_rows(a)) {
     const int dlds = dense_lds(n, a.plan.kb);
     // as many workgroups as stay resident together (registers and LDS decide how many share a CU), each looping over its rows
     auto launch = [&](auto kernel, int which) {
@@ -1646,7 +1701,7 @@ static int launch_rows_as(const RowArgs& a, int lds_bytes, hipStream_t s) {
   }
   // table-driven order times H_512, one size of row: one row per 512-thread workgroup, Sylvester part inside the waves, dense stage on
   // the matrix cores
-  if (a.plan.kb > 1 && a.plan.kb <= 32 && a.plan.m == 512 && a.plan.f == 1 && a.plan_shared.n == n && a.plan_shared.kb == a.plan.kb && a.rotate != 0) {
+  if (wide_rows(a)) {
     static bool opted_in[64] = {};
     if (dev >= 0 && dev < 64 && !opted_in[dev]) {
       if (hipFuncSetAttribute(reinterpret_cast<const void*>(&row_quant_wide_kernel<SILU, EXT>), hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds) != hipSuccess) {

@@ -34,8 +34,8 @@ def test_shape_of_a_long_problem(q, want):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tokens", [33, 100, 128, 129, 201, 420])
-@pytest.mark.parametrize("mix", ["wo", "wo8", "wxax", "fp16"])
+@pytest.mark.parametrize("tokens", [33, 100, 128, 129, 201, 256, 420])
+@pytest.mark.parametrize("mix", ["wo", "wo8", "wxax", "fp16", "fp8"])
 def test_layer_with_a_wide_shared_expert(tokens, mix):
     """Device-planned and host-planned forwards pick the same tiles, so they agree bit for bit; the outputs stay within 1e-2 (2-norm) of the
     same layer through one row tile at a time, i.e. of its tokens in batches too small for any large tile."""
@@ -43,9 +43,10 @@ def test_layer_with_a_wide_shared_expert(tokens, mix):
     from mxmoe_amd.layer import MxMoELayer
 
     f = {"wo": [(S.W4A16, S.W3A16), (S.W3A16, S.W4A16), (S.W2A16, S.W2A16)], "wo8": [((16, 8, 128, False),) * 2] * 3,
-         "wxax": [(S.W4A4, S.W8A8), (S.W8A8, S.W4A4), (S.W4A4, S.W4A4)], "fp16": [(S.FP16, S.FP16)] * 3}[mix]
+         "wxax": [(S.W4A4, S.W8A8), (S.W8A8, S.W4A4), (S.W4A4, S.W4A4)], "fp16": [(S.FP16, S.FP16)] * 3,
+         "fp8": [(S.W8A8, S.W8A8), (S.W4A4, S.W8A8), (S.W4A4, S.W4A4)]}[mix]
     cfg = S.MoEConfig("t", "test", 4, 2, 512, 1408, tokens, num_shared=4, rotate=1)
-    layer = MxMoELayer(cfg, formats=[f[i % 3] for i in range(5)])
+    layer = MxMoELayer(cfg, formats=[f[i % 3] for i in range(5)], fp8=mix == "fp8")
     hidden = S.make_hidden(cfg)
     ids, w = S.make_routing(cfg)
     got = layer(hidden, ids, w)
