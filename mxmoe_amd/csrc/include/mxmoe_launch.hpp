@@ -407,86 +407,119 @@ struct Segment {
   int row0, rows, branch, tiles;
 };
 
-// Tiles of a long-K problem from which on the launch is as busy with them as with the rest (a quarter of the 512 workgroups that run at a time).
+// Tiles of a launch's long-K problems, all of them together, from which on it is as busy with them as with the rest (a quarter of the 512
+// workgroups that run at a time).
 constexpr int kLongTiles = 128;
 // Whether a problem of a launch whose smallest K is `kmin` counts as long: above that, and a tile of it takes long at all (a 128 x 256
 // weight-only tile 2.4 us per 128 of K: 40 us, a whole launch of few-row experts).
 constexpr int kLongK = 2048;
 __host__ __device__ inline bool runs_long(int K, int kmin) { return K > kmin && K >= kLongK; }
 
-// Split the M rows of an M x N problem into at most two segments: whole tiles of the shape that is cheapest per output element,
-// then the remainder with the shape that covers it most cheaply (cost of a block run with one shape = row tiles * column tiles *
-// tile_cost).  Returns the number of segments (0 for M == 0), or -1 when the kernel has no tile for `f`.
-// Two rolled loops on purpose: the device planner runs this once per launch, when none of its code is in the instruction cache, and
-// what it costs there is the fetching of its instructions.
-//
-// `long_k`: runs_long of the problem (a shared expert behind several intermediates' width).  Its tiles run that
-// many times longer than the others', and a launch is not over before they are: as long as the problem has too few tiles to share the
-// chip with the rest, what counts is the time of one.  Where the choice by total cost takes the largest shape, such a problem takes the one
-// of the smallest max(tile_cost, tiles * tile_cost / kLongTiles) instead.  Weight-only formats: the 32-token tile up to some 600 rows.  The
-// 16-, 8- and 4-bit operand formats do that up to one large row tile only: their shorter tiles need half as long, not a third, for a
-// quarter of the rows (201 .. 800 rows measured slower).  Down launch with 60 experts and a shared expert of four times their width, us,
-// large shape -> this rule: w4a16 / w3a16 103 -> 36 (100 tokens), 103 -> 40 (201), 106 -> 58 (400); w4a4 45 -> 31, w4a4 / w8a8 49 -> 40, fp16
-// 151 -> 128 (100); 64 experts and twice the width: w4a16 / w3a16 61 -> 37 (128), 60 -> 41 (201), 80 -> 67 (600), w8a16 / w2a16 60 -> 44 (128).
-__host__ __device__ inline int plan_segments(const PlanInfo& k, int f, int M, int N, bool long_k, Segment out[2]) {
+// The choice of tile shapes for an M x N problem, as far as it does not depend on the rest of the launch.
+struct PlanPick {
+  int branch = -1, bm = 0, tiles = 0;
+  double cost = 0;
+  __host__ __device__ void offer(const PlanBranch& b, int t, double c, double eps) {
+    if (branch < 0 || c < cost - eps || (c < cost + eps && b.BM > bm)) {
+      branch = b.index;
+      bm = b.BM;
+      tiles = t;
+      cost = c;
+    }
+  }
+};
+struct PlanChoice {
+  PlanPick unit, whole;  // cheapest per row of the problem; cheapest for all of it (cost of a block run with one shape = row tiles * column tiles * tile_cost)
+  int full = 0;          // rows that fill whole tiles of `unit`
+  double full_cost = 0;
+  // Tiles in the largest shape, what a problem of long K adds to its launch's `long_tiles` (up to kLongTiles: more makes no difference), or 0
+  // when it takes a shorter shape anyway or there is no other.
+  int large_tiles = 0;
+};
+
+// Returns 1, or 0 for M == 0, or -1 when the kernel has no tile for `f`.  Rolled loops here and below on purpose: the device planner runs
+// this once per launch, when none of its code is in the instruction cache, and what it costs there is the fetching of its instructions.
+__host__ __device__ inline int plan_choose(const PlanInfo& k, int f, int M, int N, PlanChoice& c) {
   if (f < 0 || f >= kNumFmts) return -1;
   const int lo = k.fmt_start[f], hi = k.fmt_start[f + 1];
   if (lo == hi) return -1;
   if (M <= 0) return 0;
-  struct Pick {
-    int branch = -1, bm = 0, tiles = 0;
-    double cost = 0;
-  };
-  auto offer = [](Pick& best, const PlanBranch& b, int tiles, double c, double eps) {
-    if (best.branch < 0 || c < best.cost - eps || (c < best.cost + eps && b.BM > best.bm)) {
-      best.branch = b.index;
-      best.bm = b.BM;
-      best.tiles = tiles;
-      best.cost = c;
-    }
-  };
-  Pick unit, whole, quick;  // cheapest per row of the problem; cheapest for all of it; soonest done on a part of the chip
-  int full = 0;
-  double full_cost = 0;
 #pragma unroll 1
   for (int i = lo; i < hi; ++i) {
     const PlanBranch& b = k.b[i];
     const int tm = tiles_over(M, b.bm_log2), tn = tiles_over(N, b.bn_log2), rows = M >> b.bm_log2 << b.bm_log2;
-    const double all = (double)tm * tn * b.cost, share = all * (1.0 / kLongTiles);
-    offer(whole, b, tm * tn, all, 1e-9);
-    offer(quick, b, tm * tn, share > b.cost ? share : b.cost, 1e-9);
-    const int had = unit.branch;
-    offer(unit, b, (M >> b.bm_log2) * tn, b.cost_per_row * tn, 1e-12);
-    if (unit.branch != had) {
-      full = rows;
-      full_cost = (double)(M >> b.bm_log2) * tn * b.cost;
+    c.whole.offer(b, tm * tn, (double)tm * tn * b.cost, 1e-9);
+    const int had = c.unit.branch;
+    c.unit.offer(b, (M >> b.bm_log2) * tn, b.cost_per_row * tn, 1e-12);
+    if (c.unit.branch != had) {
+      c.full = rows;
+      c.full_cost = (double)(M >> b.bm_log2) * tn * b.cost;
     }
   }
-  const bool large = full > 0 || whole.branch == unit.branch;
-  if (long_k && large && quick.branch != unit.branch && whole.tiles < kLongTiles && (M <= 128 || is_weight_only((Fmt)f))) {
-    out[0] = Segment{0, M, quick.branch, quick.tiles};
-    return 1;
+  if (hi - lo > 1 && (c.full > 0 || c.whole.branch == c.unit.branch)) c.large_tiles = c.whole.tiles < kLongTiles ? c.whole.tiles : kLongTiles;
+  return 1;
+}
+
+// Split the M rows of an M x N problem (M > 0, `c` from plan_choose) into at most two segments: whole tiles of the shape that is cheapest
+// per output element, then the remainder with the shape that covers it most cheaply.  Returns the number of segments.
+//
+// `long_tiles`: 0, or for a problem of long K (runs_long: a shared expert behind several intermediates' width, say) the sum of large_tiles
+// over all such problems of its launch.  Their tiles run that many times longer than the others', and a launch is not over before they
+// are: as long as there are too few of them to share the chip with the rest, what counts is the time of one.  Where the choice by
+// total cost takes the largest shape, such a problem takes the one of the smallest max(tile_cost, t / kLongTiles) instead, t being the
+// cost of its own tiles and two thirds of what the launch's other long problems add to them (taken in proportion to their large tiles).  It is
+// the launch's sum that is asked, since short tiles are 2 to 2.5 times the work.  c problems of K = 4096, N = 2048 beside one of K = 2048, us, large
+// shape / shapes by each problem alone / this rule: w4a16 64 rows 52 / 37 / 33 (c = 6), 55 / 58 / 56 (15), 103 / 202 / 107 (60); 200 rows 69 / 48 / 48
+// (4), 73 / 102 / 74 (12); 600 rows 550 / 998 / 557 (60); w4a4 128 rows 31 / 28 / 23 (8), 70 / 95 / 70 (60); fp16 128 rows 57 / 75 / 52 (8), 246 / 441 / 246 (60).
+// Weight-only formats: the 32-token tile up to some 600 rows.  The
+// 16-, 8- and 4-bit operand formats do that up to one large row tile only: their shorter tiles need half as long, not a third, for a
+// quarter of the rows (201 .. 800 rows measured slower).  Down launch with 60 experts and a shared expert of four times their width, us,
+// large shape -> this rule: w4a16 / w3a16 103 -> 36 (100 tokens), 103 -> 40 (201), 106 -> 58 (400); w4a4 45 -> 31, w4a4 / w8a8 49 -> 40, fp16
+// 151 -> 128 (100); 64 experts and twice the width: w4a16 / w3a16 61 -> 37 (128), 60 -> 41 (201), 80 -> 67 (600), w8a16 / w2a16 60 -> 44 (128).
+__host__ __device__ inline int plan_split(const PlanInfo& k, int f, int M, int N, const PlanChoice& c, int long_tiles, Segment out[2]) {
+  const int lo = k.fmt_start[f], hi = k.fmt_start[f + 1];
+  if (long_tiles > 0 && long_tiles < kLongTiles && c.large_tiles > 0 && (M <= 128 || is_weight_only((Fmt)f))) {
+    PlanPick quick;  // soonest done on a part of the chip (both terms times 3 * kLongTiles * own tiles)
+    const double own = (double)(3 * kLongTiles) * c.whole.tiles, shared = c.whole.tiles + 2.0 * long_tiles;
+#pragma unroll 1
+    for (int i = lo; i < hi; ++i) {
+      const PlanBranch& b = k.b[i];
+      const int tiles = tiles_over(M, b.bm_log2) * tiles_over(N, b.bn_log2);
+      const double one = own * b.cost, all = (double)tiles * b.cost * shared;
+      quick.offer(b, tiles, all > one ? all : one, 1e-9);
+    }
+    if (quick.branch != c.unit.branch) {
+      out[0] = Segment{0, M, quick.branch, quick.tiles};
+      return 1;
+    }
   }
-  const int rem = M - full;
-  out[0] = Segment{0, M, whole.branch, whole.tiles};
-  if (rem == 0 || full == 0) return 1;
-  Pick rest;
+  const int rem = M - c.full;
+  out[0] = Segment{0, M, c.whole.branch, c.whole.tiles};
+  if (rem == 0 || c.full == 0) return 1;
+  PlanPick rest;
   int all_unit = 0;  // tiles of the whole problem in the shape that is cheapest per row
 #pragma unroll 1
   for (int i = lo; i < hi; ++i) {
     const PlanBranch& b = k.b[i];
     const int tm = tiles_over(rem, b.bm_log2), tn = tiles_over(N, b.bn_log2);
-    offer(rest, b, tm * tn, (double)tm * tn * b.cost, 1e-9);
-    if (b.index == unit.branch) all_unit = tiles_over(M, b.bm_log2) * tn;
+    rest.offer(b, tm * tn, (double)tm * tn * b.cost, 1e-9);
+    if (b.index == c.unit.branch) all_unit = tiles_over(M, b.bm_log2) * tn;
   }
-  if (rest.branch == unit.branch) {
-    out[0] = Segment{0, M, unit.branch, all_unit};
+  if (rest.branch == c.unit.branch) {
+    out[0] = Segment{0, M, c.unit.branch, all_unit};
     return 1;
   }
-  if (whole.cost <= full_cost + rest.cost + 1e-9) return 1;
-  out[0] = Segment{0, full, unit.branch, unit.tiles};
-  out[1] = Segment{full, rem, rest.branch, rest.tiles};
+  if (c.whole.cost <= c.full_cost + rest.cost + 1e-9) return 1;
+  out[0] = Segment{0, c.full, c.unit.branch, c.unit.tiles};
+  out[1] = Segment{c.full, rem, rest.branch, rest.tiles};
   return 2;
+}
+
+// Both steps: the number of segments (0 for M == 0), or -1 when the kernel has no tile for `f`.
+inline int plan_segments(const PlanInfo& k, int f, int M, int N, int long_tiles, Segment out[2]) {
+  PlanChoice c;
+  const int rc = plan_choose(k, f, M, N, c);
+  return rc <= 0 ? rc : plan_split(k, f, M, N, c, long_tiles, out);
 }
 
 inline PlanInfo make_plan_info(const std::vector<BranchInfo>& branches) {
@@ -658,7 +691,7 @@ inline bool kernel_covers(const FusedKernel& k, const mxmoe_qparams* q, int coun
   for (int i = 0; i < count; ++i) {
     const Fmt f = classify(q[i]);
     Segment sg[2];
-    if (f == Fmt::UNSUPPORTED || plan_segments(plan_of(k), (int)f, 1, 256, false, sg) < 0) return false;
+    if (f == Fmt::UNSUPPORTED || plan_segments(plan_of(k), (int)f, 1, 256, 0, sg) < 0) return false;
   }
   return true;
 }
@@ -697,6 +730,24 @@ inline bool shape_ok(const BranchInfo& bi, const mxmoe_dim3& sz) {
   return sz.z != 0 && sz.z % bi.k_multiple == 0 && (int)sz.z >= bi.k_min && sz.y % 8 == 0 && !(wo && sz.y % 16 != 0);
 }
 
+// What the planning of one launch's problems has in common: its smallest K, and the large tiles of its long problems.
+struct LaunchScope {
+  int kmin = 0x7fffffff, long_tiles = 0;
+  // the `long_tiles` argument of a problem's plan
+  int long_tiles_of(const mxmoe_dim3& sz) const { return runs_long((int)sz.z, kmin) ? long_tiles : 0; }
+};
+inline LaunchScope launch_scope(const PlanInfo& pi, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int n) {
+  LaunchScope s;
+  for (int i = 0; i < n; ++i) s.kmin = std::min(s.kmin, (int)h_sizes[i].z);
+  for (int i = 0; i < n; ++i) {
+    const Fmt f = classify(h_q[i]);
+    PlanChoice c;
+    if (f != Fmt::UNSUPPORTED && runs_long((int)h_sizes[i].z, s.kmin) && plan_choose(pi, (int)f, (int)h_sizes[i].x, (int)h_sizes[i].y, c) > 0)
+      s.long_tiles = std::min(s.long_tiles + c.large_tiles, kLongTiles);
+  }
+  return s;
+}
+
 // Tile tables of one launch over problems [base, base + n) (n <= kMaxProblems): entries, phases, totals of `a`; *grid receives the
 // workgroups to launch.  Host-only arithmetic.
 inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int base, int n, FusedArgs& a, int* grid) {
@@ -708,13 +759,12 @@ inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, c
   };
   Entry entries[kMaxEntries];
   int nent = 0;
-  uint32_t kmin = ~0u;
-  for (int i = 0; i < n; ++i) kmin = std::min(kmin, h_sizes[base + i].z);
+  const LaunchScope scope = launch_scope(pi, h_sizes + base, h_q + base, n);
   for (int i = 0; i < n; ++i) {
     const mxmoe_dim3& sz = h_sizes[base + i];
     const Fmt f = classify(h_q[base + i]);
     Segment sg[2];
-    const int ns = f == Fmt::UNSUPPORTED ? -1 : plan_segments(pi, (int)f, (int)sz.x, (int)sz.y, runs_long((int)sz.z, (int)kmin), sg);
+    const int ns = f == Fmt::UNSUPPORTED ? -1 : plan_segments(pi, (int)f, (int)sz.x, (int)sz.y, scope.long_tiles_of(sz), sg);
     if (ns < 0) {
       last_error() = "quant type not supported";
       return 1;
@@ -742,7 +792,7 @@ inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, c
     for (int pass = 0; pass < 2; ++pass)
       for (int ei = 0; ei < nent; ++ei) {
         const Entry& en = entries[ei];
-        if (en.branch != b || en.tiles == 0 || (h_sizes[base + en.problem].z > kmin) != (pass == 0)) continue;
+        if (en.branch != b || en.tiles == 0 || ((int)h_sizes[base + en.problem].z > scope.kmin) != (pass == 0)) continue;
         a.entry[ne] = FusedArgs::Entry{total, en.row0, en.rows, en.problem | (en.branch << 16)};
         total += en.tiles;
         ++ne;
@@ -788,6 +838,19 @@ inline int launch_range(const FusedKernel& k, const void* const* As, const void*
     return 4;
   }
   return 0;
+}
+
+// Problems of the launch that starts at `base`: up to kMaxProblems, under the other policies than Fused of one format (kernel_sketch.py:192-246
+// compares the QParams of neighbours the same way).
+inline int launch_length(const FusedKernel& k, const mxmoe_qparams* h_q, int base, int count) {
+  const mxmoe_qparams& a = h_q[base];
+  int n = 1;
+  while (base + n < count && n < kMaxProblems) {
+    const mxmoe_qparams& b = h_q[base + n];
+    if (k.policy != Policy::Fused && !(a.a_bits == b.a_bits && a.w_bits == b.w_bits && a.gsize == b.gsize && a.sym == b.sym)) break;
+    ++n;
+  }
+  return n;
 }
 
 // Side streams of the multi-stream policy, created on first use per device (default priority, non-blocking) and kept for the
@@ -845,8 +908,6 @@ inline int group_gemm(int kernel_id, const void* const* As, const void* const* B
       if (const int rc = run(base, std::min(kMaxProblems, count - base), stream)) return rc;
     return 0;
   }
-  // runs of consecutive problems of equal format (kernel_sketch.py:192-246 compares the QParams of neighbours the same way)
-  auto same = [&](int x, int y) { return h_q[x].a_bits == h_q[y].a_bits && h_q[x].w_bits == h_q[y].w_bits && h_q[x].gsize == h_q[y].gsize && h_q[x].sym == h_q[y].sym; };
   SideStreams* side = nullptr;
   if (k.policy == Policy::MultiStream) {
     side = side_streams();
@@ -858,8 +919,7 @@ inline int group_gemm(int kernel_id, const void* const* As, const void* const* B
   int nrun = 0, rc = 0;
   unsigned used = 0;
   for (int base = 0; base < count && rc == 0;) {
-    int n = 1;
-    while (base + n < count && n < kMaxProblems && same(base, base + n)) ++n;
+    const int n = launch_length(k, h_q, base, count);
     hipStream_t s = stream;
     if (side) {
       const int si = nrun % kSideStreams;

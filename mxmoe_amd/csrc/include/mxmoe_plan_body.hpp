@@ -83,6 +83,7 @@ struct PlanShared {
   int cnt[kMaxBranches][2], til[kMaxBranches][2];    // per run-order rank and wave: entries, tiles
   int cnt_long[kMaxBranches][2], til_long[kMaxBranches][2];  // ... of which belong to long-K problems
   int kmin[2];
+  int long_tiles[2], long_tiles_kmin[2];             // large tiles of the wave's problems with K >= kLongK; of those with K = kmin
   // the kernel's branch table, from the kernel arguments: the planning functions walk it entry by entry, and each step of such a
   // walk through the argument segment costs a trip to the scalar cache
   PlanInfo info;
@@ -177,11 +178,26 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
   // smallest K of the launch: problems above it run first inside their branch (see launch_range)
   const int km = -wave_last(wave_inclusive_max(mine ? -K : -0x7fffffff));
   if (lane == 0) sh.kmin[wave] = km;
+  // what this problem's tile shapes are, as far as the rest of the launch has no say in it, and the large tiles of the long problems
+  // (launch_scope): whether one of K >= kLongK is above the launch's smallest is known behind the barrier
+  PlanChoice choice;
+  const int have = mine ? plan_choose(info, fmt, (int)rows, N, choice) : 0;
+  const int large = have > 0 && K >= kLongK ? choice.large_tiles : 0;
+  if (__ballot(large > 0) != 0) {
+    const int all = wave_last(wave_inclusive_scan(large)), at_km = wave_last(wave_inclusive_scan(K == km ? large : 0));
+    if (lane == 0) {
+      sh.long_tiles[wave] = all;
+      sh.long_tiles_kmin[wave] = at_km;
+    }
+  } else if (lane == 0) {
+    sh.long_tiles[wave] = sh.long_tiles_kmin[wave] = 0;
+  }
   __syncthreads();
   const int kmin = min(sh.kmin[0], sh.kmin[1]);
   const bool long_k = mine && K > kmin;
+  const int long_tiles = sh.long_tiles[0] - (sh.kmin[0] == kmin ? sh.long_tiles_kmin[0] : 0) + sh.long_tiles[1] - (sh.kmin[1] == kmin ? sh.long_tiles_kmin[1] : 0);
   Segment sg[2];
-  const int ns = mine ? plan_segments(info, fmt, (int)rows, N, runs_long(K, kmin), sg) : 0;
+  const int ns = have > 0 ? plan_split(info, fmt, (int)rows, N, choice, runs_long(K, kmin) ? min(long_tiles, kLongTiles) : 0, sg) : 0;
   // per branch in run order, this wave's entries and tiles
   int seg_rank[2] = {-1, -1}, seg_pos[2] = {0, 0}, seg_first[2] = {0, 0};
   const PlanBranch& my_branch = info.b[info.order[min(lane, kMaxBranches - 1)]];  // lane r: the branch of rank r

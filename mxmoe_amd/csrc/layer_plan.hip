@@ -99,7 +99,7 @@ int resolve_kernel(int kernel_id, const mxmoe_block_desc* h_desc, int et) {
     for (int i = 0; i < et; ++i) {
       Segment sg[2];
       const int f = fmt_of(h_desc[i].q);
-      if (f == (int)Fmt::UNSUPPORTED || plan_segments(plan_of(k), f, 1, 256, false, sg) < 0) return false;
+      if (f == (int)Fmt::UNSUPPORTED || plan_segments(plan_of(k), f, 1, 256, 0, sg) < 0) return false;
       // a kernel's w4a4 tiles take packed int4 rows or bf6 fragments, never both: the descriptor says which the block will get
       if (f == (int)Fmt::W4A4 && kernel_takes_bf6(k) != wants_bf6(h_desc[i].q)) return false;
       if (f == (int)Fmt::W8A8 && (kernel_variant(k, Fmt::W8A8) == kVariantFp8) != wants_fp8(h_desc[i].q)) return false;
@@ -179,13 +179,16 @@ int mxmoe_plan_grid_bound(int kernel_id, const mxmoe_block_desc* h_desc, int num
   // For every routed expert tiles(M) <= first + slope * (M - 1) for all M >= 1, with first = tiles(1) and slope the steepest rise
   // found by walking M over 64 rows of the format's largest tile (the planner's decisions repeat with that tile's period).  With at
   // most n = min(experts, rows) experts non-empty, the launch has at most (sum of the n largest `first`) + max slope * (rows - n) tiles.
-  // A block that is long against the smallest K may be so in its launch (or not, when the block is run as several launches): the
-  // larger count holds.
+  // A block that is long against the smallest K may be so in its launch (or not, when the block is run as several launches), beside
+  // any number of others: the larger count holds, and with more of the others it takes shapes of less total cost and more each,
+  // hence fewer tiles, so it is enough to look at the block with none.
   auto tiles_of = [&](int f, int m, int n, bool maybe_long) {
     int most = 0;
+    PlanChoice c;
+    if (plan_choose(pi, f, m, n, c) <= 0) return 0;
     for (int lk = 0; lk <= (maybe_long ? 1 : 0); ++lk) {
       Segment sg[2];
-      const int ns = plan_segments(pi, f, m, n, lk != 0, sg);
+      const int ns = plan_split(pi, f, m, n, c, lk ? c.large_tiles : 0, sg);
       int t = 0;
       for (int j = 0; j < ns; ++j) t += sg[j].tiles;
       most = std::max(most, t);
@@ -214,7 +217,7 @@ int mxmoe_plan_grid_bound(int kernel_id, const mxmoe_block_desc* h_desc, int num
       if (sn.f == f && sn.n == n && sn.maybe_long == maybe_long) hit = &sn;
     if (!hit) {
       Segment sg[2];
-      plan_segments(pi, f, 1 << 20, n, false, sg);
+      plan_segments(pi, f, 1 << 20, n, 0, sg);
       const BranchInfo& bi = registry()[kid].branches[sg[0].branch];
       const int bm = bi.BM, cols = (n + bi.BN - 1) / bi.BN;
       Seen sn{f, n, maybe_long, tiles_of(f, 1, n, maybe_long), 0, 0.0, (double)cols / bm};

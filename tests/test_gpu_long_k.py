@@ -56,3 +56,114 @@ def test_layer_with_a_wide_shared_expert(tokens, mix):
     part = torch.cat([layer.call_with_host_tables(hidden[i:i + 16].contiguous(), ids[i:i + 16].contiguous(), w[i:i + 16].contiguous()) for i in range(0, tokens, 16)])
     a, b = got.double().cpu().numpy(), part.double().cpu().numpy()
     assert np.linalg.norm(a - b) <= 1e-2 * np.linalg.norm(b)
+
+
+def _tables(lib, kid, probs):
+    from mxmoe_amd import _lib
+
+    n = len(probs)
+    sizes = (_lib.Dim3 * n)(*[_lib.Dim3(*p[0]) for p in probs])
+    qs = (_lib.QParams * n)(*[_lib.QParams(q[0], q[1], q[2], int(q[3])) for _, q in probs])
+    if kid < 0:
+        kid = lib.mxmoe_group_gemm_plan(-1, sizes, qs, n, None, None) - 1000
+        assert kid >= 0, lib.mxmoe_last_error()
+    out = (C.c_int32 * 1200)()
+    assert lib.mxmoe_group_gemm_plan_tables(kid, sizes, qs, n, out, 1200) == 0, lib.mxmoe_last_error()
+    return kid, np.array(out[:], np.int32)
+
+
+def _tiles_of(lib, probs):
+    from mxmoe_amd import _lib
+
+    n = len(probs)
+    sizes = (_lib.Dim3 * n)(*[_lib.Dim3(*p[0]) for p in probs])
+    qs = (_lib.QParams * n)(*[_lib.QParams(q[0], q[1], q[2], int(q[3])) for _, q in probs])
+    tiles = C.c_int32()
+    assert lib.mxmoe_group_gemm_plan(-1, sizes, qs, n, None, C.byref(tiles)) >= 1000, lib.mxmoe_last_error()
+    return tiles.value
+
+
+@pytest.mark.parametrize("q,m", [((16, 4, 128, False), 64), ((16, 4, 128, False), 600), ((16, 8, 128, False), 200), ((4, 4, -1, True), 128), ((16, 16, -1, True), 128)])
+def test_many_long_problems_keep_their_shapes(q, m):
+    """Sixty problems of K = 4096 fill the chip: one of K = 2048 beside them is no reason for more and shorter tiles.  Nor is it for a few
+    whose shorter tiles would together be the longer run; two small ones still take them."""
+    from mxmoe_amd import _lib
+
+    lib = _lib.load()
+    short = ((m, 2048, 2048), q)
+    long = ((m, 2048, 4096), q)
+    assert _tiles_of(lib, [long] * 60 + [short]) == _tiles_of(lib, [long] * 60) + _tiles_of(lib, [short])
+    assert _tiles_of(lib, [long] * 200 + [short]) == _tiles_of(lib, [long] * 200) + _tiles_of(lib, [short])   # (two launches)
+    few = ((100, 512, 4096), q)
+    two = _tiles_of(lib, [few] * 2 + [((5, 512, 2048), q)])
+    one = _tiles_of(lib, [few] + [((5, 512, 2048), q)])
+    assert two - one == one - _tiles_of(lib, [((5, 512, 2048), q)]) > _tiles_of(lib, [few])
+
+
+LONG_LISTS = [  # (formats, N, K of each expert, rows of each expert, shared rows)
+    ([(16, 4, 128, False), (16, 3, 128, False)], 2048, [4096] * 9 + [2048], [64] * 9 + [7], 0),
+    ([(16, 4, 128, False)], 2048, [2048, 4096, 2048, 4096], [40, 100, 3, 0], 100),                  # two long ones, one without rows
+    ([(16, 4, 128, False), (4, 4, -1, True)], 512, [4096] * 3 + [2048] * 100 + [4096] * 2, [90] * 105, 128),   # in both waves of the planner
+    ([(4, 4, -1, True), (16, 16, -1, True)], 1024, [4096, 4096, 2048, 2048, 5632], [100, 128, 50, 1, 30], 60),
+    ([(16, 8, 128, False)], 2048, [2048] * 5, [100] * 5, 300),                                      # long by the shared one alone
+    ([(16, 4, 128, False)], 2048, [2048] * 120 + [4096] * 5, [20] * 125, 64),                      # two launches, one without a short problem
+]
+
+
+def _long_list(case):
+    fmts, n, ks, rows, shared = case
+    ks = ks + ([2 * max(ks)] if shared else [])
+    return [fmts[i % len(fmts)] for i in range(len(ks))], n, ks, rows, shared
+
+
+@pytest.mark.parametrize("case", range(len(LONG_LISTS)))
+def test_grid_bound_covers_lists_of_long_problems(case):
+    """The worst-case grid against the host's plan for random routings, where any number of problems may be the long ones of their launch."""
+    import random
+
+    from mxmoe_amd import _lib
+
+    lib = _lib.load()
+    qs, n, ks, rows, shared = _long_list(LONG_LISTS[case])
+    e, et, total = len(rows), len(ks), sum(rows)
+    desc = (_lib.BlockDesc * et)(*[_lib.BlockDesc(q[0], q[1], q[2], int(q[3]), (C.c_uint8 * 3)(), n, k, 0, 0) for q, k in zip(qs, ks)])
+    kid = lib.mxmoe_plan_select_kernel(-1, desc, et)
+    bound = lib.mxmoe_plan_grid_bound(kid, desc, e, total, shared)
+    assert kid >= 0 and bound > 0, lib.mxmoe_last_error()
+    rnd = random.Random(case)
+    for trial in range(60):
+        cuts = sorted(rnd.randint(0, total) for _ in range(e - 1))
+        counts = rows if trial == 0 else [b - a for a, b in zip([0] + cuts, cuts + [total])]
+        probs = [((m, n, k), q) for m, k, q in zip(counts + [shared] * (shared > 0), ks, qs)]
+        for at in range(0, et, 120):
+            _, host = _tables(lib, kid, probs[at:at + 120])
+            assert host[3] <= bound, (trial, host[:4], bound)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", range(len(LONG_LISTS)))
+def test_device_planner_agrees_on_lists_of_long_problems(case):
+    """Entries, phases and totals of the planning kernel against the host's (nothing is launched on them: the operands' addresses are not read)."""
+    from mxmoe_amd import _lib
+
+    lib = _lib.load()
+    qs, n, ks, rows, shared = _long_list(LONG_LISTS[case])
+    e, et = len(rows), len(ks)
+    desc = (_lib.BlockDesc * et)(*[_lib.BlockDesc(q[0], q[1], q[2], int(q[3]), (C.c_uint8 * 3)(), n, k, 0, 0) for q, k in zip(qs, ks)])
+    kid = lib.mxmoe_plan_select_kernel(-1, desc, et)
+    assert kid >= 0, lib.mxmoe_last_error()
+    d_desc = torch.frombuffer(bytearray(bytes(desc)), dtype=torch.uint8).cuda()
+    recv = torch.tensor(rows, dtype=torch.int64, device="cuda")
+    plan = torch.zeros(lib.mxmoe_plan_bytes(et), dtype=torch.uint8, device="cuda")
+    some = torch.zeros(16, dtype=torch.uint8, device="cuda")
+    _lib.check(lib, lib.mxmoe_plan_block(kid, recv.data_ptr(), e, shared, d_desc.data_ptr(), desc, some.data_ptr(), some.data_ptr(), some.data_ptr(), plan.data_ptr(),
+                                         torch.cuda.current_stream().cuda_stream))
+    got = plan.cpu().numpy()
+    probs = [((m, n, k), q) for m, k, q in zip(rows + [shared] * (shared > 0), ks, qs)]
+    for chunk, at in enumerate(range(0, et, 120)):
+        _, host = _tables(lib, kid, probs[at:at + 120])
+        ne, tiles, nph, _grid = host[:4]
+        hdr = got[chunk * 4096:(chunk + 1) * 4096].view(np.int32)[14:]      # behind seven pointers
+        assert list(hdr[:4]) == [at, ne, tiles, nph]
+        assert np.array_equal(hdr[4:5 + nph], host[4:5 + nph]) and np.array_equal(hdr[13:14 + nph], host[13:14 + nph])
+        assert np.array_equal(hdr[23:23 + 4 * ne], host[22:22 + 4 * ne])
