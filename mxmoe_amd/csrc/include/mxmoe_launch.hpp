@@ -730,7 +730,8 @@ inline bool shape_ok(const BranchInfo& bi, const mxmoe_dim3& sz) {
   return sz.z != 0 && sz.z % bi.k_multiple == 0 && (int)sz.z >= bi.k_min && sz.y % 8 == 0 && !(wo && sz.y % 16 != 0);
 }
 
-// What the planning of one launch's problems has in common: its smallest K, and the large tiles of its long problems.
+// What the planning of one launch's problems has in common: its smallest K, and the large tiles of its long problems.  Problems without rows
+// have no part in it: a list plans the same with and without them (the device planner sees every expert, the operators leave out empty ones).
 struct LaunchScope {
   int kmin = 0x7fffffff, long_tiles = 0;
   // the `long_tiles` argument of a problem's plan
@@ -738,7 +739,8 @@ struct LaunchScope {
 };
 inline LaunchScope launch_scope(const PlanInfo& pi, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int n) {
   LaunchScope s;
-  for (int i = 0; i < n; ++i) s.kmin = std::min(s.kmin, (int)h_sizes[i].z);
+  for (int i = 0; i < n; ++i)
+    if (h_sizes[i].x != 0) s.kmin = std::min(s.kmin, (int)h_sizes[i].z);
   for (int i = 0; i < n; ++i) {
     const Fmt f = classify(h_q[i]);
     PlanChoice c;

@@ -175,8 +175,8 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
     sum_before(2);
   }
   if (kind == LayerForm::kBehind) sum_before(4);
-  // smallest K of the launch: problems above it run first inside their branch (see launch_range)
-  const int km = -wave_last(wave_inclusive_max(mine ? -K : -0x7fffffff));
+  // smallest K of the launch's problems with rows: those above it run first inside their branch (see build_fused_tables)
+  const int km = -wave_last(wave_inclusive_max(mine && rows > 0 ? -K : -0x7fffffff));
   if (lane == 0) sh.kmin[wave] = km;
   // what this problem's tile shapes are, as far as the rest of the launch has no say in it, and the large tiles of the long problems
   // (launch_scope): whether one of K >= kLongK is above the launch's smallest is known behind the barrier

@@ -100,6 +100,32 @@ def test_many_long_problems_keep_their_shapes(q, m):
     assert two - one == one - _tiles_of(lib, [((5, 512, 2048), q)]) > _tiles_of(lib, [few])
 
 
+def test_problems_without_rows_have_no_say_in_the_shapes_of_others():
+    """The device planner sees every expert, the operators leave out those without tokens: a problem without rows changes nothing."""
+    from mxmoe_amd import _lib
+
+    lib = _lib.load()
+    q = (16, 4, 128, False)
+    live = [((201, 2048, 5632), q), ((40, 2048, 5632), q)]
+    kid, alone = _tables(lib, -1, live)
+    _, beside = _tables(lib, kid, live + [((0, 2048, 1408), q)])
+    assert np.array_equal(alone, beside)
+
+
+def test_plan_of_a_sequential_kernel_is_that_of_its_launches():
+    """One launch per run of equal formats: the problem of smaller K is in another launch and makes nothing long."""
+    from mxmoe_amd import _lib
+
+    lib = _lib.load()
+    seq = lib.mxmoe_find_kernel(b"groupgemm_seq_launch_all")
+    probs = [((201, 2048, 5632), (16, 4, 128, False)), ((201, 2048, 1408), (16, 16, -1, True))]
+    sizes = (_lib.Dim3 * 2)(*[_lib.Dim3(*p[0]) for p in probs])
+    qs = (_lib.QParams * 2)(*[_lib.QParams(q[0], q[1], q[2], int(q[3])) for _, q in probs])
+    tiles = C.c_int32()
+    assert lib.mxmoe_group_gemm_plan(seq, sizes, qs, 2, None, C.byref(tiles)) == 1000 + seq
+    assert tiles.value == sum(int(_tables(lib, seq, [p])[1][1]) for p in probs)
+
+
 LONG_LISTS = [  # (formats, N, K of each expert, rows of each expert, shared rows)
     ([(16, 4, 128, False), (16, 3, 128, False)], 2048, [4096] * 9 + [2048], [64] * 9 + [7], 0),
     ([(16, 4, 128, False)], 2048, [2048, 4096, 2048, 4096], [40, 100, 3, 0], 100),                  # two long ones, one without rows
@@ -167,3 +193,21 @@ def test_device_planner_agrees_on_lists_of_long_problems(case):
         assert list(hdr[:4]) == [at, ne, tiles, nph]
         assert np.array_equal(hdr[4:5 + nph], host[4:5 + nph]) and np.array_equal(hdr[13:14 + nph], host[13:14 + nph])
         assert np.array_equal(hdr[23:23 + 4 * ne], host[22:22 + 4 * ne])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("routed", [False, True])
+def test_layer_whose_tokens_all_go_to_its_shared_expert(routed):
+    """No expert id in range (or of one slot only): the shared expert is alone in its launches, in the device's plan and in the host's."""
+    from mxmoe_amd import synth as S
+    from mxmoe_amd.layer import MxMoELayer
+
+    cfg = S.MoEConfig("t", "test", 4, 2, 512, 1408, 201, num_shared=4, rotate=1)
+    layer = MxMoELayer(cfg, formats=[(S.W4A16, S.W3A16)] * 5)
+    hidden = S.make_hidden(cfg)
+    ids, w = S.make_routing(cfg)
+    ids = torch.full_like(ids, -1)
+    if routed:
+        ids[17, 1] = 2
+    got = layer(hidden, ids, w)
+    assert torch.equal(got, layer.call_with_host_tables(hidden, ids, w)) and bool((got != 0).any())
