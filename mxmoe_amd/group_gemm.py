@@ -47,9 +47,11 @@ class GroupGemmLaunch:
         table = block[:6 * p * 8].view(np.int64).reshape(6, p)
         for row, ts in zip(table, (As, Bs, scale_a, scale_b, Cs, acc)):
             if ts:
+                if len(ts) != p:  # (numpy would spread a list of one over all problems)
+                    raise ValueError(f"a list of {len(ts)} tensors for {p} problems")
                 row[:] = [0 if t is None else t.data_ptr() for t in ts]  # (0 for a tensor without elements)
         h_sizes = block[6 * p * 8:6 * p * 8 + p * 12].view(np.uint32).reshape(p, 3)
-        h_sizes[:] = sizes if isinstance(sizes, np.ndarray) else np.array(sizes, np.int64).reshape(p, 3)
+        h_sizes[:] = (sizes if isinstance(sizes, np.ndarray) else np.array(sizes, np.int32)).reshape(p, 3)
         h_q = np.zeros((max(p, 1), 4), np.int32)                        # (a_bits, w_bits, gsize, sym byte): the QParams layout
         if p:
             h_q[:p] = _qparams_array(tuple(map(tuple, qparams)))

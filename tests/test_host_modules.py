@@ -4,7 +4,9 @@ import json
 import re
 from pathlib import Path
 
+import numpy as np
 import pytest
+import torch
 
 from mxmoe_amd import synth
 from mxmoe_amd.kernels import gen_workload, qconfig, tile_config
@@ -393,3 +395,25 @@ def test_run_mxmoe_gg_up_to_the_library(tmp_path, monkeypatch):
     assert lib.mxmoe_num_kernels() == 1
     name = lib.mxmoe_kernel_name(0).decode()
     assert name.endswith("groupgemm_hz_fused_0") and "w4a16_g128_asym" in name and "w3a16_g128_asym" in name
+
+
+@pytest.mark.parametrize("which", ["scale_a", "scale_b", "acc"])
+@pytest.mark.parametrize("length", [1, 2, 4])
+def test_group_gemm_refuses_lists_that_are_not_one_per_problem(lib, which, length):
+    """A list of one must not stand for all problems: every accumulator dump would land in one buffer."""
+    from mxmoe_amd.group_gemm import GroupGemmLaunch
+
+    t = [torch.zeros(8, dtype=torch.float16)] * 3
+    args = dict(scale_a=t, scale_b=t, acc=None)
+    args[which] = t[:1] * length
+    with pytest.raises(ValueError):
+        GroupGemmLaunch(t, t, args["scale_a"], args["scale_b"], t, [(1, 8, 32)] * 3, [(16, 16, -1, True)] * 3, acc=args["acc"])
+
+
+def test_group_gemm_refuses_sizes_that_are_not_three_per_problem(lib):
+    from mxmoe_amd.group_gemm import GroupGemmLaunch
+
+    t = [torch.zeros(8, dtype=torch.float16)] * 3
+    for sizes in (np.ones((3, 1), np.uint32), [(1, 8)] * 3, [(1, 8, 2 ** 33)] * 3):
+        with pytest.raises((ValueError, OverflowError)):
+            GroupGemmLaunch(t, t, None, None, t, sizes, [(16, 16, -1, True)] * 3)
