@@ -105,16 +105,18 @@ __device__ __forceinline__ mxmoe_block_desc plan_block_prepare(const PlanParams&
 }
 
 // `recv`: the tokens-per-expert counts (device memory, or LDS when the planning workgroup counted them itself); `d`: what
-// plan_block_prepare returned.
+// plan_block_prepare returned.  Every thread of the workgroup must call this (it holds workgroup barriers); threads with `active` false
+// (those past kPlanThreads of a wider workgroup) only pass the barriers.
 template <class Count>
-__device__ __forceinline__ void plan_block_body(const PlanParams& p, const int chunk, const int chunks, const Count* recv, const mxmoe_block_desc& d, PlanShared& sh) {
+__device__ __forceinline__ void plan_block_body(const PlanParams& p, const int chunk, const int chunks, const Count* recv, const mxmoe_block_desc& d, PlanShared& sh,
+                                                const bool active) {
   const int e0 = chunk * kMaxProblems;                       // first expert of this launch
   const int ecnt = min(kMaxProblems, p.Et - e0);             // experts of this launch
   constexpr int kSums = PlanShared::kSums;
   const PlanInfo& info = sh.info;
   const int e = threadIdx.x, lane = e & 63, wave = e >> 6;
   const int ge = e0 + e;                             // this thread's expert
-  const bool mine = e < ecnt;
+  const bool mine = active && e < ecnt;
   const PlanLayout lay(p.Et);
   FusedArgs* fa = reinterpret_cast<FusedArgs*>(p.plan + chunk * kFusedArgsStride);
   int64_t* table = reinterpret_cast<int64_t*>(p.plan + lay.table);
@@ -137,60 +139,61 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
     f[3] = (long)(kind == LayerForm::kGateUp ? dx.N / 2 : dx.N) * rows;
     f[4] = (long)K * rows;
   };
-  // experts before this launch (none for the first: most blocks are one launch)
-  if (e0 > 0) {
-    long base[kSums] = {0, 0, 0, 0, 0};
-    for (int x = e; x < e0; x += kPlanThreads) {
-      long f[kSums];
-      footprint(x, p.desc[x], f);
-#pragma unroll
-      for (int i = 0; i < kSums; ++i) base[i] += f[i];
-    }
-#pragma unroll
-    for (int i = 0; i < kSums; ++i) {
-      const long all = wave_last(wave_inclusive_scan(base[i]));
-      if (lane == 0) sh.base[i][wave] = all;
-    }
-  } else if (lane < kSums) {
-    sh.base[lane][wave] = 0;
-  }
-
-  long foot[kSums] = {0, 0, 0, 0, 0};
-  if (mine) footprint(ge, d, foot);
-  const long rows = foot[0];
   const int N = (int)d.N, K = (int)d.K, fmt = fmt_of(d.q), tag = act_tag_of(d.q);
   const bool scaled = tag != 0;
-  // exclusive sums over the experts of this launch before this one (those that the block's form has a use for)
-  long before_me[kSums] = {0, 0, 0, 0, 0};
-  auto sum_before = [&](int i) {
-    const long inc = wave_inclusive_scan(foot[i]);
-    before_me[i] = inc - foot[i];
-    const long all = wave_last(inc);
-    if (lane == 0) sh.tot[i][wave] = all;
-  };
-  sum_before(0);
-  sum_before(3);
-  if (kind != LayerForm::kGateUp) {
-    sum_before(1);
-    sum_before(2);
-  }
-  if (kind == LayerForm::kBehind) sum_before(4);
-  // smallest K of the launch's problems with rows: those above it run first inside their branch (see build_fused_tables)
-  const int km = -wave_last(wave_inclusive_max(mine && rows > 0 ? -K : -0x7fffffff));
-  if (lane == 0) sh.kmin[wave] = km;
-  // what this problem's tile shapes are, as far as the rest of the launch has no say in it, and the large tiles of the long problems
-  // (launch_scope): whether one of K >= kLongK is above the launch's smallest is known behind the barrier
+  long foot[kSums] = {0, 0, 0, 0, 0}, before_me[kSums] = {0, 0, 0, 0, 0}, rows = 0;
   PlanChoice choice;
-  const int have = mine ? plan_choose(info, fmt, (int)rows, N, choice) : 0;
-  const int large = have > 0 && K >= kLongK ? choice.large_tiles : 0;
-  if (__ballot(large > 0) != 0) {
-    const int all = wave_last(wave_inclusive_scan(large)), at_km = wave_last(wave_inclusive_scan(K == km ? large : 0));
-    if (lane == 0) {
-      sh.long_tiles[wave] = all;
-      sh.long_tiles_kmin[wave] = at_km;
+  int have = 0;
+  if (active) {
+    // experts before this launch (none for the first: most blocks are one launch)
+    if (e0 > 0) {
+      long base[kSums] = {0, 0, 0, 0, 0};
+      for (int x = e; x < e0; x += kPlanThreads) {
+        long f[kSums];
+        footprint(x, p.desc[x], f);
+#pragma unroll
+        for (int i = 0; i < kSums; ++i) base[i] += f[i];
+      }
+#pragma unroll
+      for (int i = 0; i < kSums; ++i) {
+        const long all = wave_last(wave_inclusive_scan(base[i]));
+        if (lane == 0) sh.base[i][wave] = all;
+      }
+    } else if (lane < kSums) {
+      sh.base[lane][wave] = 0;
     }
-  } else if (lane == 0) {
-    sh.long_tiles[wave] = sh.long_tiles_kmin[wave] = 0;
+    if (mine) footprint(ge, d, foot);
+    rows = foot[0];
+    // exclusive sums over the experts of this launch before this one (those that the block's form has a use for)
+    auto sum_before = [&](int i) {
+      const long inc = wave_inclusive_scan(foot[i]);
+      before_me[i] = inc - foot[i];
+      const long all = wave_last(inc);
+      if (lane == 0) sh.tot[i][wave] = all;
+    };
+    sum_before(0);
+    sum_before(3);
+    if (kind != LayerForm::kGateUp) {
+      sum_before(1);
+      sum_before(2);
+    }
+    if (kind == LayerForm::kBehind) sum_before(4);
+    // smallest K of the launch's problems with rows: those above it run first inside their branch (see build_fused_tables)
+    const int km = -wave_last(wave_inclusive_max(mine && rows > 0 ? -K : -0x7fffffff));
+    if (lane == 0) sh.kmin[wave] = km;
+    // what this problem's tile shapes are, as far as the rest of the launch has no say in it, and the large tiles of the long problems
+    // (launch_scope): whether one of K >= kLongK is above the launch's smallest is known behind the barrier
+    have = mine ? plan_choose(info, fmt, (int)rows, N, choice) : 0;
+    const int large = have > 0 && K >= kLongK ? choice.large_tiles : 0;
+    if (__ballot(large > 0) != 0) {
+      const int all = wave_last(wave_inclusive_scan(large)), at_km = wave_last(wave_inclusive_scan(K == km ? large : 0));
+      if (lane == 0) {
+        sh.long_tiles[wave] = all;
+        sh.long_tiles_kmin[wave] = at_km;
+      }
+    } else if (lane == 0) {
+      sh.long_tiles[wave] = sh.long_tiles_kmin[wave] = 0;
+    }
   }
   __syncthreads();
   const int kmin = min(sh.kmin[0], sh.kmin[1]);
@@ -198,11 +201,11 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
   const int long_tiles = sh.long_tiles[0] - (sh.kmin[0] == kmin ? sh.long_tiles_kmin[0] : 0) + sh.long_tiles[1] - (sh.kmin[1] == kmin ? sh.long_tiles_kmin[1] : 0);
   Segment sg[2];
   const int ns = have > 0 ? plan_split(info, fmt, (int)rows, N, choice, runs_long(K, kmin) ? min(long_tiles, kLongTiles) : 0, sg) : 0;
-  // per branch in run order, this wave's entries and tiles
-  int seg_rank[2] = {-1, -1}, seg_pos[2] = {0, 0}, seg_first[2] = {0, 0};
   const PlanBranch& my_branch = info.b[info.order[min(lane, kMaxBranches - 1)]];  // lane r: the branch of rank r
   const int my_order = my_branch.index;
-  for (int r = 0; r < info.nb; ++r) {
+  int seg_rank[2] = {-1, -1}, seg_pos[2] = {0, 0}, seg_first[2] = {0, 0};
+  // per branch in run order, this wave's entries and tiles
+  for (int r = 0; active && r < info.nb; ++r) {
     const int b = __builtin_amdgcn_readlane(my_order, r);
     int mine_tiles = 0, which = -1;
 #pragma unroll
@@ -234,6 +237,7 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
     }
   }
   __syncthreads();
+  if (!active) return;
 #pragma unroll
   for (int i = 0; i < kSums; ++i) before_me[i] += sh.base[i][0] + sh.base[i][1] + (wave == 1 ? sh.tot[i][0] : 0l);  // (a sum without a use stays garbage)
   const long first_row = before_me[0], inp_off = before_me[1], sc_off = before_me[2], out_off = before_me[3];

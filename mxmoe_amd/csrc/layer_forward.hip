@@ -266,7 +266,8 @@ __global__ void __launch_bounds__(TH) layer_head_kernel(const HeadArgs a, const 
     const PlanParams& p = pair.p[wg / pair.chunks];
     const int chunk = wg % pair.chunks;
     mxmoe_block_desc d{};
-    if (threadIdx.x < kPlanThreads) d = plan_block_prepare(p, chunk, sh);
+    const bool plans = __builtin_amdgcn_readfirstlane(threadIdx.x) < kPlanThreads;
+    if (plans) d = plan_block_prepare(p, chunk, sh);
     if (a.hist) {
       for (int e = threadIdx.x; e < a.E; e += TH) {
         int v, before;
@@ -277,7 +278,7 @@ __global__ void __launch_bounds__(TH) layer_head_kernel(const HeadArgs a, const 
     } else {
       count_ids<TH>(a.ids, a.total, a.E, 0, nullptr, head_lds, head_lds + a.E);
     }
-    if (threadIdx.x < kPlanThreads) plan_block_body(p, chunk, pair.chunks, head_lds, d, sh);
+    plan_block_body(p, chunk, pair.chunks, head_lds, d, sh, plans);
     return;
   }
   wg -= plan_wgs;

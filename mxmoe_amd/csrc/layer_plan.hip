@@ -22,7 +22,7 @@ __global__ void __launch_bounds__(kPlanThreads) plan_block_kernel(const PlanPair
   const PlanParams& p = pair.p[blockIdx.x / pair.chunks];
   const mxmoe_block_desc d = plan_block_prepare(p, blockIdx.x % pair.chunks, sh);
   __syncthreads();
-  plan_block_body(p, blockIdx.x % pair.chunks, pair.chunks, pair.p[0].recv, d, sh);
+  plan_block_body(p, blockIdx.x % pair.chunks, pair.chunks, pair.p[0].recv, d, sh, true);
 }
 
 // Permutation and planning of a decode-sized batch (at most kPermChunk (token, slot) entries) in ONE launch: workgroup 0 builds the
@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(kPlanThreads) perm_plan_small_kernel(const Per
     if (e >= 0 && e < a.E) atomicAdd(&cnt[e], 1ull);
   }
   __syncthreads();
-  plan_block_body(pair.p[b / pair.chunks], chunk, pair.chunks, counts, d, sh);
+  plan_block_body(pair.p[b / pair.chunks], chunk, pair.chunks, counts, d, sh, true);
 }
 
 // The same for larger batches, after perm_hist_kernel has counted the experts per chunk of kPermChunk entries: the first `blocks`
@@ -89,7 +89,7 @@ __global__ void __launch_bounds__(kPlanThreads) perm_scatter_plan_kernel(const P
     counts[e] = v;
   }
   __syncthreads();
-  plan_block_body(pair.p[b / pair.chunks], chunk, pair.chunks, counts, d, sh);
+  plan_block_body(pair.p[b / pair.chunks], chunk, pair.chunks, counts, d, sh, true);
 }
 
 // Kernel for the formats of `h_desc`, checked once on the host: every problem's format has a branch and its shape fits it.

@@ -69,6 +69,15 @@ def test_short_forward_of_more_experts_than_one_launch_holds():
     _check(cfg, layer)
 
 
+@pytest.mark.parametrize("tokens", [50, 1100])
+def test_short_forward_of_the_most_experts_it_takes(tokens):
+    """512 experts, the most LDS the head asks for, in workgroups of 256 and of 512 threads; five launches per block to plan."""
+    from mxmoe_amd import synth as S
+
+    cfg, layer = _layer(tokens, 4, [((S.W4A4, S.W8A8), (S.W8A8, S.FP16), (S.FP16, S.W4A4))[i % 3] for i in range(513)], inter=128, rotate=0)
+    _check(cfg, layer)
+
+
 def test_short_forward_counts_ids_in_a_launch_of_its_own():
     """More than 65536 (token, slot) entries: the per-chunk counting launch in front of the head."""
     from mxmoe_amd import synth as S

@@ -417,3 +417,67 @@ def test_group_gemm_refuses_sizes_that_are_not_three_per_problem(lib):
     for sizes in (np.ones((3, 1), np.uint32), [(1, 8)] * 3, [(1, 8, 2 ** 33)] * 3):
         with pytest.raises((ValueError, OverflowError)):
             GroupGemmLaunch(t, t, None, None, t, sizes, [(16, 16, -1, True)] * 3)
+
+
+def _enclosing_conditions(body: str, at: int):
+    """Text in front of every statement or block that position `at` of a function's body lies in, from the inside out."""
+    out, end, i, skipping = [], at, at - 1, False
+    while i >= 0:
+        c = body[i]
+        if c == "{":                                                       # opens a block around `at`
+            if not skipping:
+                out.append(body[i + 1:end])
+            end, skipping = i, False
+        elif c in ";}":                                                    # an earlier statement, or the end of an earlier block
+            if not skipping:
+                out.append(body[i + 1:end])
+                skipping = True
+            if c == "}":
+                depth = 1
+                while depth:
+                    i -= 1
+                    depth += {"}": 1, "{": -1}.get(body[i], 0)
+        i -= 1
+    return out if skipping else out + [body[:end]]
+
+
+def _barriers_under_thread_conditions(sources):
+    """(function, call) of every workgroup barrier, or call of a function that holds one, that stands under a condition on the thread's
+    index.  All threads of a workgroup have to reach the same barrier: that waves which have ended leave its count is the hardware's
+    behaviour, and no promise of the language."""
+    params = r"\((?:[^(){}]|\([^()]*\))*\)"
+    start = re.compile(r"__(?:device|global)__[^;{}]*?\b(\w+)\s*" + params + r"\s*\{")
+    bodies = []
+    for s in sources:
+        s = re.sub(r"//[^\n]*", "", s)
+        for m in start.finditer(s):
+            depth, j = 1, m.end()
+            while depth:
+                depth += {"{": 1, "}": -1}.get(s[j], 0)
+                j += 1
+            bodies.append((m.group(1), s[m.end():j - 1]))
+    call = lambda name: re.compile(rf"\b{name}\b\s*(?:<[^;()]*>)?\(")  # noqa: E731
+    holders = {"__syncthreads"}
+    while more := {n for n, b in bodies if n not in holders and any(call(x).search(b) for x in holders)}:
+        holders |= more
+    found = []
+    for n, b in bodies:
+        for x in sorted(holders):
+            for m in call(x).finditer(b):
+                for text in _enclosing_conditions(b, m.start()):
+                    if any(re.search(r"threadIdx|\b(lane|wave|active|plans|mine)\b", text[k.end():]) for k in re.finditer(r"\b(?:if|while|for)\s*\(", text)):
+                        found.append((n, x))
+    return holders, found
+
+
+def test_no_workgroup_barrier_stands_under_a_condition_on_the_thread():
+    planted = """
+__device__ void inner(int a) { if (a) { x = 1; } __syncthreads(); }
+__global__ void k1() { if (blockIdx.x == 0) { inner(0); return; } for (int i = threadIdx.x; i < 4; ++i) { y[i] = 0; } __syncthreads(); }
+__global__ void k2() { int z = 0; if (threadIdx.x < 128) inner(z); }
+__global__ void k3() { if (lane == 0) { z = 1; if (z) { __syncthreads(); } } }"""
+    assert _barriers_under_thread_conditions([planted])[1] == [("k2", "inner"), ("k3", "__syncthreads")]
+    csrc = Path(__file__).resolve().parent.parent / "mxmoe_amd" / "csrc"
+    holders, found = _barriers_under_thread_conditions([f.read_text() for f in sorted([*csrc.glob("*.hip"), *(csrc / "include").glob("*.hpp")])])
+    assert {"plan_block_body", "count_ids", "layer_head_kernel", "fused_body"} <= holders
+    assert not found
