@@ -309,7 +309,8 @@ int mxmoe_upload(void* dst, const void* host_src, size_t bytes, void* stream);
  * mxmoe_layer_create      checks the description and copies it; the handle is read only afterwards (mxmoe_layer_run may be called from several
  *                         threads as far as the buffers it names allow) and is given back with mxmoe_layer_destroy.
  * mxmoe_layer_run         enqueues on `stream`; hidden fp16 [num_tokens][hidden], topk_ids int32 [num_tokens][topk] (ids out of range are
- *                         dropped), topk_weights fp32, out fp16 [num_tokens][hidden].  Neither allocates nor synchronises. */
+ *                         dropped), topk_weights fp32, out fp16 [num_tokens][hidden].  Neither allocates nor synchronises.  hidden is
+ *                         16-byte aligned where a first block takes 16-bit activations and rotate is not 2 (error 3 otherwise). */
 int mxmoe_layer_supported(const mxmoe_layer_desc* desc);
 int mxmoe_layer_create(const mxmoe_layer_desc* desc, void** handle);
 void mxmoe_layer_destroy(void* handle);

@@ -300,7 +300,7 @@ struct LayerForward {
   HeadArgs head;
   PlanPair pair;
   int et, threads, token_wgs;
-  bool fp16_first;   // a first block reads the tokens as they are
+  bool fp16_first;   // a first block reads the tokens as they are (its tiles load them straight into LDS)
   bool rows_step;    // a second block takes quantised (or rotated) rows
   RowsBehind rows;
 };
@@ -460,6 +460,10 @@ int mxmoe_layer_run(const void* handle, const void* hidden, const int32_t* topk_
   }
   const LayerForward& f = *reinterpret_cast<const LayerForward*>(handle);
   const mxmoe_layer_desc& d = f.d;
+  if (f.fp16_first && (reinterpret_cast<uintptr_t>(hidden) & 15)) {
+    last_error() = "hidden must be 16-byte aligned: first blocks of 16-bit activations read the tokens where they are, in 16-byte pieces";
+    return 3;
+  }
   hipStream_t s = (hipStream_t)stream;
   HeadArgs h = f.head;
   PlanPair pair = f.pair;

@@ -300,6 +300,8 @@ class MxMoELayer:
         be captured into a HIP graph.  Intermediate buffers belong to the layer and are reused by the next call of the same shape."""
         cfg, dev = self.cfg, self.device
         hidden = hidden.to(dev).contiguous()
+        if hidden.data_ptr() & 15:  # a view that starts in the middle of its storage: tiles may load the tokens straight into LDS, in 16-byte pieces
+            hidden = hidden.clone()
         ids = topk_ids.to(dev, torch.int32).contiguous()
         w = topk_weights.to(dev, torch.float32).contiguous()
         t, k_hid = hidden.shape

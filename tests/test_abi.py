@@ -283,3 +283,34 @@ def test_planned_grid_bound_covers_every_routing(lib):
     assert lib.mxmoe_plan_select_kernel(-1, desc, 4097) < 0               # checked before any entry is read
     assert lib.mxmoe_plan_bytes(130) >= 2 * 4096 + 130 * (32 + 40 + 12)   # a block of more than 120 experts: one table header per launch
     assert lib.mxmoe_plan_bytes(60) >= 4096 + 60 * (32 + 40 + 12)
+
+
+@pytest.mark.parametrize("a_bits,rotate,refused", [(16, 1, True), (16, 2, False), (4, 1, False)])
+def test_layer_run_wants_aligned_tokens_where_tiles_read_them_in_place(lib, a_bits, rotate, refused):
+    """First blocks of 16-bit activations load `hidden` straight into LDS in 16-byte pieces.  Host-only: a handle over addresses that are
+    never read, and calls that are refused before any launch (the accepted forms are not called)."""
+    from mxmoe_amd import _lib
+
+    def block(a, n, k):
+        return (_lib.BlockDesc * 2)(*[_lib.BlockDesc(a, 16 if a == 16 else 4, -1, 1, (C.c_uint8 * 3)(), n, k, 0, 0)] * 2)
+
+    gate_up, down = block(a_bits, 2 * 1024, 512), block(16, 512, 1024)
+    page = (C.c_uint8 * 4096)()
+    some = (C.addressof(page) + 255) & ~255
+    d = _lib.LayerDesc(num_tokens=4, topk=2, num_experts=2, hidden=512, inter=1024, inter_shared=1024, rotate=rotate, had_k=1, had_f=1,
+                       h_gate_up=C.cast(gate_up, C.c_void_p), h_down=C.cast(down, C.c_void_p), grid_gate_up=64, grid_down=64)
+    d.kernel_gate_up, d.kernel_down = lib.mxmoe_plan_select_kernel(-1, gate_up, 2), lib.mxmoe_plan_select_kernel(-1, down, 2)
+    for name in ("d_gate_up", "d_down", "act", "down_inp", "down_scales", "down_out", "plan_gate_up", "plan_down", "dst_exp", "token_of_row", "row_of_slot", "iota", "recv", "workspace"):
+        setattr(d, name, some)
+    for tag in range(6):
+        d.token_store[tag] = d.token_scales[tag] = some
+    assert lib.mxmoe_layer_supported(C.byref(d)) == 1
+    handle = C.c_void_p()
+    assert lib.mxmoe_layer_create(C.byref(d), C.byref(handle)) == 0, lib.mxmoe_last_error()
+    try:
+        if refused:
+            for off in (2, 4, 8, 14):
+                assert lib.mxmoe_layer_run(handle, some + off, some, some, some, None) == 3 and b"16-byte" in lib.mxmoe_last_error()
+        assert lib.mxmoe_layer_run(handle, None, some, some, some, None) == 5
+    finally:
+        lib.mxmoe_layer_destroy(handle)

@@ -86,6 +86,24 @@ def test_short_forward_counts_ids_in_a_launch_of_its_own():
     _check(cfg, layer)
 
 
+@pytest.mark.parametrize("mix", ["fp16", "wo", "wxax"])
+@pytest.mark.parametrize("offset", [1, 2, 4, 7])
+def test_tokens_from_the_middle_of_a_buffer(mix, offset):
+    """A contiguous view whose address is not a multiple of 16 bytes, with enough rows for the tiles that load tokens straight into LDS."""
+    from mxmoe_amd import synth as S
+
+    fm = {"fp16": (S.FP16, S.FP16), "wo": (S.W4A16, S.W3A16), "wxax": (S.W4A4, S.W8A8)}[mix]
+    cfg, layer = _layer(300, 2, [fm] * 4)
+    hidden = S.make_hidden(cfg).cuda()
+    ids, w = S.make_routing(cfg)
+    store = torch.zeros(hidden.numel() + 16, dtype=torch.float16, device="cuda")
+    view = store[offset:offset + hidden.numel()].view(hidden.shape)
+    view.copy_(hidden)
+    assert view.is_contiguous() and view.data_ptr() % 16 == 2 * offset
+    assert torch.equal(layer(view, ids, w), layer(hidden, ids, w))
+    assert torch.equal(view, hidden)
+
+
 def test_layers_the_short_form_does_not_take():
     from mxmoe_amd import synth as S
 
