@@ -481,3 +481,23 @@ __global__ void k3() { if (lane == 0) { z = 1; if (z) { __syncthreads(); } } }""
     holders, found = _barriers_under_thread_conditions([f.read_text() for f in sorted([*csrc.glob("*.hip"), *(csrc / "include").glob("*.hpp")])])
     assert {"plan_block_body", "count_ids", "layer_head_kernel", "fused_body"} <= holders
     assert not found
+
+
+def test_current_stream_without_torchs_private_names(monkeypatch):
+    from mxmoe_amd import _lib
+
+    class Stream:
+        cuda_stream = 77
+
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: Stream)
+    monkeypatch.setattr(_lib, "_current_stream", None, raising=False)
+    assert _lib.current_stream() == 77
+
+
+def test_library_loads_without_torch():
+    import subprocess
+    import sys
+
+    code = "import sys; from mxmoe_amd import _lib; _lib.load().mxmoe_num_kernels(); sys.exit('torch' in sys.modules)"
+    assert subprocess.run([sys.executable, "-c", code], cwd=Path(__file__).resolve().parent.parent).returncode == 0
