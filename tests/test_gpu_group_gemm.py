@@ -461,6 +461,55 @@ def test_random_shapes_every_format_in_mixed_launches(seed):
             assert np.isfinite(out).all() and _rel(out, p["ref"]) <= 1e-2, (i, p["size"], p["q"], _rel(out, p["ref"]))
 
 
+@pytest.mark.parametrize("q,rows", [((16, 4, 128, False), (33, 128, 201)), ((16, 3, 128, False), (100, 201)), ((16, 2, 128, True), (64, 201)), ((16, 8, 128, False), (100, 129)),
+                                     ((4, 4, -1, True), (100, 128)), ((8, 8, -1, True), (100, 128)), ((16, 16, -1, True), (100, 128))])
+def test_short_tiles_of_a_long_problem_against_the_exact_product(q, rows):
+    """A problem of more than the launch's smallest K takes tiles of fewer rows than it would alone.  Integer formats: the oracle's bits.
+    The others against the product in 64 bits of the fp16 rows and the exactly dequantised weights: the output's rounding is at
+    most 2^-11 of each value, and the sums (fp32 products and sums of 16-bit values; the weight-only tiles for many rows also round
+    every weight, by 2^-11 and without correlation) add less than that, so 2^-10 in the 2-norm."""
+    import ctypes as C
+
+    from mxmoe_amd import _lib
+    from mxmoe_amd.weights import quantize_and_pack
+
+    rng = np.random.default_rng(29)
+    n, k = 528, 4096
+    short = ("w", 2, n, 2048)
+    for m in rows:
+        probs, exact = [], []
+        for _, mm, nn, kk in (("long", m, n, k), short):
+            if q[0] < 16:
+                probs.append(_wxax_problem(rng, mm, nn, kk, q[0]))
+                continue
+            x = rng.standard_normal((mm, kk)).astype(F16)
+            w = (rng.standard_normal((nn, kk)) * 0.02).astype(F16)
+            if q[1] >= 16:
+                probs.append(dict(A=torch.from_numpy(x).to(DEV), B=torch.from_numpy(w).to(DEV), size=(mm, nn, kk), q=q))
+                exact.append(x.astype(np.float64) @ w.astype(np.float64).T)
+                continue
+            pw = quantize_and_pack(torch.from_numpy(w), q)
+            c, s, z = O.quant_minmax(w, q[1], q[2], q[3])
+            wd = (c.reshape(-1, q[2]).astype(np.float64) * s.astype(np.float64) + (0 if q[3] else z.astype(np.float64))).reshape(nn, kk)
+            probs.append(dict(A=torch.from_numpy(x).to(DEV), B=pw.data.to(DEV), sb=pw.scale.to(DEV), size=(mm, nn, kk), q=q))
+            exact.append(x.astype(np.float64) @ wd.T)
+        g, outs, accs = _launch(probs, dump=q[0] < 16)
+        alone, _, _ = _launch(probs[:1], dump=q[0] < 16)
+        heights = []
+        for launch in (g, alone):
+            info = (C.c_int32 * 8)()
+            kid, branches, _ = launch.plan()
+            assert _lib.load().mxmoe_kernel_branch(kid, branches[0], info) == 0
+            heights.append(info[1])
+        assert heights[0] < heights[1] == 128
+        for i, (p, out) in enumerate(zip(probs, outs)):
+            if q[0] < 16:
+                assert np.array_equal(accs[i], p["acc"]) and np.array_equal(out.view(np.uint16), p["out"].view(np.uint16)), (i, p["size"])
+            else:
+                err = np.linalg.norm(out.astype(np.float64) - exact[i]) / np.linalg.norm(exact[i])
+                assert err <= 2.0 ** -10, (i, p["size"], err)
+
+
 def test_unsupported_format_raises_reference_message():
     rng = np.random.default_rng(4)
     p = _wxax_problem(rng, 4, 256, 128, 8)

@@ -69,6 +69,24 @@ def test_short_forward_of_more_experts_than_one_launch_holds():
     _check(cfg, layer)
 
 
+@pytest.mark.parametrize("inter,had,down,num_shared,rotate", [(320, None, "W8A8", 2, 1), (480, None, "FP16", 4, 2), (1024, (64, 2), "W4A4", 2, 1), (1408, None, "W4A4", 4, 1),
+                                                              (2048, (64, 4), "W8A8", 2, 1)])
+def test_routed_and_shared_rows_of_two_lengths_in_one_launch(monkeypatch, inter, had, down, num_shared, rotate):
+    """row_quant_pair_kernel at 1, 2, 3 and 4 chunks of 8 values per lane of a routed row.  Rows of 1024 and 2048 values are powers of two and
+    would take no table of their own: they get one of kb x kb signs (the rotation's sums are exact for any signs) on both sides."""
+    from mxmoe_amd import layer as L
+    from mxmoe_amd import synth as S
+
+    if had:
+        kb, f = had
+        signs = (1.0 - 2.0 * torch.randint(0, 2, (kb, kb), generator=torch.Generator().manual_seed(inter))).cuda()
+        plain = L.device_signs
+        monkeypatch.setattr(L, "device_signs", lambda n, dev: (kb * f, f, signs) if n % inter == 0 else plain(n, dev))
+    fmt = getattr(S, down)
+    cfg, layer = _layer(260, 2, [(S.W8A8, fmt), (S.W4A4, fmt), (S.FP16, fmt), (S.W8A8, fmt)], inter=inter, num_shared=num_shared, rotate=rotate)
+    _check(cfg, layer)
+
+
 @pytest.mark.parametrize("tokens", [50, 1100])
 def test_short_forward_of_the_most_experts_it_takes(tokens):
     """512 experts, the most LDS the head asks for, in workgroups of 256 and of 512 threads; five launches per block to plan."""
