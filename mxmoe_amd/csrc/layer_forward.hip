@@ -37,7 +37,8 @@ constexpr int kHeadSmallMax = 4096;
 constexpr int kHeadMaxExperts = 512;
 // Entries (tokens x top-k) up to which every workgroup that needs counts takes them from the ids themselves, all of them: 128 KiB of ids
 // out of L2 and as many LDS counter updates take some 6 us, which the token workgroups of the same launch hide; beyond, the cost
-// per workgroup would grow with the batch, and a counting launch (perm_hist_kernel) goes first.
+// per workgroup would grow with the batch, and a counting launch (perm_hist_kernel) goes first.  Its counts are summed by every workgroup
+// that needs them, so that form in turn ends at kPermFusedScanMax counts (mxmoe_layer_supported): with 64 experts or more, here.
 constexpr int kHeadCountMax = 65536;
 
 struct HeadArgs {

@@ -223,7 +223,7 @@ class MxMoELayer:
 
     def _short_setup(self, t: int, topk: int):
         """The short form of the planned forward for (tokens, top-k): a handle of `mxmoe_layer_create` with the buffers it names, or None
-        when the library does not take the layer in that form (row length, bf6 operands).  Built once and reused."""
+        when the library does not take the layer or the batch in that form (mxmoe_layer_supported).  Built once and reused."""
         cache = self.__dict__.setdefault("_short", {})
         key = (t, topk)
         if key in cache:
@@ -295,9 +295,11 @@ class MxMoELayer:
         Same kernels and results as `forward` + `combine`, but nothing here waits for the routing: the tables of both launches are
         derived from the tokens-per-expert counts by a planning kernel on the device (`mxmoe_plan_layer`: both blocks in one launch), the stores and plan
         buffers are allocated once per (tokens, top-k) for the worst case, and every launch argument is independent of the data.
-        The call only enqueues four or five kernels (`mxmoe_layer_run`; six to nine, in separate calls, for the layers that form does
-        not take: rows that are not a power of two, bf6 operands); no synchronisation, no allocation after the first call when `out` is given, so it can
-        be captured into a HIP graph.  Intermediate buffers belong to the layer and are reused by the next call of the same shape."""
+        The call only enqueues four or five kernels (`mxmoe_layer_run`; six to nine, in separate calls, for what that form does not take:
+        hidden sizes other than 512, 1024, 2048 and 4096, intermediate sizes that are no multiple of 32, more than 512 experts, bf6
+        operands, and batches of more than 65536 (token, slot) pairs whose chunks of 256 times the experts exceed 16384, i.e. every
+        larger batch from 64 experts on); no synchronisation, no allocation after the first call when `out` is given (but a copy of a
+        `hidden` that is not 16-byte aligned), so it can be captured into a HIP graph.  Intermediate buffers belong to the layer and are reused by the next call of the same shape."""
         cfg, dev = self.cfg, self.device
         hidden = hidden.to(dev).contiguous()
         if hidden.data_ptr() & 15:  # a view that starts in the middle of its storage: tiles may load the tokens straight into LDS, in 16-byte pieces
@@ -366,7 +368,7 @@ class MxMoELayer:
         """The planned forward for a fixed (tokens, top-k) shape, captured into a HIP graph: write the inputs into the returned
         object's `hidden`, `topk_ids`, `topk_weights` tensors, call `replay()`, read `out`.  Nothing in the forward depends on the
         routing at enqueue time, so one capture serves every routing; a replay has no per-kernel launch gaps (decode-sized batches
-        gain most: 0.105 against 0.12 ms for DeepSeek-V2-Lite at 32 tokens).  With `logits_dtype` the graph starts at the router's
+        gain most).  With `logits_dtype` the graph starts at the router's
         logits instead (`forward_from_logits`): the input is then `router_logits` [tokens, experts] of that dtype."""
         return CapturedForward(self, tokens, self.cfg.topk if topk is None else topk, logits_dtype, renormalise)
 
