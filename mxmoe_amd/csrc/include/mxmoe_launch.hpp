@@ -469,10 +469,10 @@ __host__ __device__ inline int plan_choose(const PlanInfo& k, int f, int M, int 
 // total cost takes the largest shape, such a problem takes the one of the smallest max(tile_cost, t / kLongTiles) instead, t being the
 // cost of its own tiles and two thirds of what the launch's other long problems add to them (taken in proportion to their large tiles).  It is
 // the launch's sum that is asked, since short tiles are 2 to 2.5 times the work.  c problems of K = 4096, N = 2048 beside one of K = 2048, us, large
-// shape / shapes by each problem alone / this rule: w4a16 64 rows 52 / 37 / 33 (c = 6), 55 / 58 / 44 (15), 103 / 202 / 107 (60); 200 rows 69 / 48 / 48
-// (4), 73 / 102 / 74 (12); 600 rows 550 / 998 / 557 (60); w4a4 128 rows 31 / 28 / 23 (8), 70 / 95 / 70 (60); fp16 128 rows 57 / 75 / 52 (8), 246 / 441 / 246 (60).
-// Weight-only formats take the 32-token tile up to some 600 rows that way.  The 16-, 8- and 4-bit operand formats do it up to one large row tile only: their shorter tiles need half as long, not a third, for a
-// quarter of the rows (201 .. 800 rows measured slower).  Down launch with 60 experts and a shared expert of four times their width, us,
+// shape / shapes by each problem alone / this rule: w4a16 64 rows 52 / 37 / 33 (c = 6), 55 / 58 / 44 (15), 107 / 202 / 107 (60); 200 rows 69 / 48 / 48
+// (4), 73 / 102 / 74 (12); 600 rows 557 / 998 / 557 (60); w4a4 128 rows 31 / 28 / 23 (8), 70 / 95 / 70 (60); fp16 128 rows 57 / 75 / 52 (8), 246 / 441 / 246 (60).
+// Weight-only formats take the 32-token tile up to some 600 rows that way.  The 16-, 8- and 4-bit operand formats do it up to one large row
+// tile only: their shorter tiles need half as long, not a third, for a quarter of the rows (201 .. 800 rows measured slower).  Down launch with 60 experts and a shared expert of four times their width, us,
 // large shape -> this rule: w4a16 / w3a16 103 -> 36 (100 tokens), 103 -> 40 (201), 106 -> 58 (400); w4a4 45 -> 31, w4a4 / w8a8 49 -> 40, fp16
 // 151 -> 128 (100); 64 experts and twice the width: w4a16 / w3a16 61 -> 37 (128), 60 -> 41 (201), 80 -> 67 (600), w8a16 / w2a16 60 -> 44 (128).
 __host__ __device__ inline int plan_split(const PlanInfo& k, int f, int M, int N, const PlanChoice& c, int long_tiles, Segment out[2]) {
