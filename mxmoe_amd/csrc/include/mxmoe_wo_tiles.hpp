@@ -32,11 +32,16 @@
 
 namespace mxmoe {
 
-// KP: k blocks (128 wide) per pass of a wave, whose activations live in registers; RING: packed weight blocks in flight per wave;
 // WAVES: waves per SIMD a kernel made of such tiles alone is compiled for (fewer registers per wave, more workgroups per CU);
 // MB: blocks of 16 tokens per tile.  Every unpacked weight operand is multiplied into all MB token blocks, so an expert with 17 .. 32
 // tokens still streams its weights once (two 16-token tiles stream them twice, the second time out of L2 at best, and take nearly
-// twice as long); the activations of a pass and the partial sums take MB times the registers, which is why KP shrinks as MB grows.
+// twice as long).
+// 4, 3 and 2 bits: a wave walks its K range as one stream (stream()), with as many packed blocks in flight as the tile has channel blocks.
+// 8 bits, whose packed blocks take twice the registers: in passes (pass()) of KP k blocks (128 wide), whose activations live in registers, with
+// RING packed blocks in flight; the activations of a pass take MB times the registers, which is why KP shrinks as MB grows.
+// The stream replaced passes for every width but 8 (there it spills at 32 tokens and gains nothing at 16).  A pass starts with an empty ring and waits
+// out a memory latency, two or more times per tile.  64 problems of N = 2816, K = 2048, us, pass -> stream: 24 tokens w4 57 -> 45, w3 57 -> 44, w2
+// 53 -> 41; 16 tokens and fewer the same there, but 23 -> 20 at N = 2048, K = 1408 (w4, 3 tokens: waves of 3, 3, 3 and 2 k blocks).
 template <int WBITS_, int BN_, int KP_ = 4, int RING_ = (WBITS_ == 8 ? 6 : 12), int WAVES_ = 2, int MB_ = 1>
 struct SkinnyWoTile {
   static constexpr int WBITS = WBITS_, MB = MB_, BM = 16 * MB_, BN = BN_;
@@ -45,7 +50,9 @@ struct SkinnyWoTile {
   static constexpr int NB = BN / 16;                 // 16-channel blocks per tile
   static constexpr int KP = KP_;                     // k blocks (128 wide) per pass of a wave: their activations live in registers
   static constexpr int kRedBytes = kWaves * NB * MB * 64 * 16;  // per-wave partial sums for the final reduction
-  static constexpr int kScaleBytes = NB * KP * 64;         // per-wave patch of (scale, zero) pairs of one pass
+  static constexpr bool kStream = WBITS != 8;                 // stream() instead of pass()
+  static constexpr int kChunk = kStream ? 4 : KP;              // k blocks whose (scale, zero) pairs a wave holds at a time
+  static constexpr int kScaleBytes = NB * kChunk * 64;        // its patch for them
   static constexpr int kLdsBytes = kRedBytes + kWaves * kScaleBytes;
   static constexpr int kAccRegs = NB * MB * 4;
   static constexpr int kWavesWanted = WAVES_;
@@ -81,15 +88,19 @@ struct SkinnyWoTile {
 
   // 8 packed values of one dword -> 8 fp16 numbers in k order, each still carrying the bias of its magic constant:
   // 0x6400 | q is the fp16 number 1024 + q (elements 0, 1, 4, 5), 0x5400 | (q << 4) is 64 + q (elements 2, 3, 6, 7).
-  // The biases are taken out of the 128-wide partial sum instead of out of every weight (see pass()).
+  // The biases are taken out of the 128-wide partial sum instead of out of every weight (see stream()).
+  // One v_and_or_b32 per pair (decode of one token, 64 experts of w4a16 / w3a16: 34.0 -> 31.4 us a layer): the instruction takes one scalar operand and no literal, so a mask goes into a scalar register and a magic constant
+  // into a vector register, both hidden from the compiler, which would otherwise see two literals and split it into an and and an or.
   template <int MASK_LO, int MASK_HI>
   __device__ static __forceinline__ v8h cvt8(int d) {
+    int lo = MASK_LO, hi = MASK_HI, m_lo = 0x64006400, m_hi = 0x54005400;
+    asm("" : "+s"(lo), "+s"(hi), "+v"(m_lo), "+v"(m_hi));
     const int d8 = (int)((unsigned)d >> 8);
     v4i o;
-    o[0] = (d & MASK_LO) | 0x64006400;
-    o[1] = (d & MASK_HI) | 0x54005400;
-    o[2] = (d8 & MASK_LO) | 0x64006400;
-    o[3] = (d8 & MASK_HI) | 0x54005400;
+    o[0] = (d & lo) | m_lo;
+    o[1] = (d & hi) | m_hi;
+    o[2] = (d8 & lo) | m_lo;
+    o[3] = (d8 & hi) | m_hi;
     return __builtin_bit_cast(v8h, o);
   }
 
@@ -134,11 +145,7 @@ struct SkinnyWoTile {
   // One pass of a wave: NKB (<= KP) consecutive k blocks starting at kb0, against all NB channel blocks of the tile.
   // The wave's activations of these k blocks are loaded once into registers and its (scale, zero) pairs into a private LDS
   // patch; the packed weight blocks then stream through a ring of kRing register buffers with no barrier in the loop, so
-  // kRing KB per wave are always in flight.  Per 128-wide group g and channel n the pass adds
-  //   s * (sum_k x[k] * (q[k] + bias[k])  -  sum_k x[k] * bias[k])  +  z * sum_k x[k]
-  // where the first sum comes from 4 MFMAs on the biased weights and the other two from MFMAs of x against constant operands.
-  // Gate_up form: channel blocks 0 .. NB/2 - 1 are gate channels from n0 on, blocks NB/2 .. NB - 1 the up channels of the same outputs;
-  // nbv counts the existing ones of either half.  `src`: the activation row of this lane in each token block.
+  // kRing KB per wave are always in flight.  The sums: see stream().
   template <bool GU, int NKB>
   __device__ static __forceinline__ void pass(const TileArgs& t, int kb0, int m0, int n0, int nbv, int lane, const int (&src)[MB], uint8_t* __restrict__ spatch, v4f (&acc)[NB][MB]) {
     const int K = t.K, KB = K / 128;
@@ -225,6 +232,129 @@ struct SkinnyWoTile {
     });
   }
 
+  // The K range [kb_lo, kb_hi) of a wave as one stream, k block by k block against all NB channel blocks of the tile.  The packed blocks of the next k
+  // block are requested channel block by channel block as those of this one have been unpacked, and its activations at the start, so NB blocks per
+  // wave are always in flight whatever the length of the range; no barrier.  Per 128-wide group g and channel n a k block adds
+  //   s * (sum_k x[k] * (q[k] + bias[k])  -  sum_k x[k] * bias[k])  +  z * sum_k x[k]
+  // where the first sum comes from 4 MFMAs on the biased weights and the other two from MFMAs of x against constant operands.  (scale, zero) pairs lie in a private LDS patch, kChunk k blocks at a time: in a register ring beside the weights (16 bytes per lane
+  // and block) they made the 32-token tile spill, and it lost all it gains (24 tokens: w4 57 us).
+  // Gate_up form: channel blocks 0 .. NB/2 - 1 are gate channels from n0 on, blocks NB/2 .. NB - 1 the up channels of the same outputs;
+  // nbv counts the existing ones of either half.  `src`: the activation row of this lane in each token block.
+  template <bool GU>
+  __device__ static __forceinline__ void stream(const TileArgs& t, int kb_lo, int kb_hi, int n0, int nbv, int lane, const int (&src)[MB], uint8_t* __restrict__ spatch, v4f (&acc)[NB][MB]) {
+    if (kb_lo >= kb_hi) return;
+    const int K = t.K, KB = K / 128;
+    const int lg = lane >> 4;
+    const v8h ones = {(_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f};
+    const v8h bias = bias8();
+    auto block_of = [&](int nb) {
+      if constexpr (GU) return (nb % (NB / 2) < nbv ? nb % (NB / 2) : 0) + (nb >= NB / 2 ? t.N / 32 : 0);
+      else return nb < nbv ? nb : 0;
+    };
+    const uint8_t* wb = t.B + ((long)(n0 / 16) * KB) * kBlockBytes;
+    const uint8_t* sb = reinterpret_cast<const uint8_t*>(t.sb) + ((long)(n0 / 16) * KB) * 64;
+    const int wl = lane * kLaneBytes;
+    auto w_of = [&](int nb, int kb) { return load_w(wb + ((long)block_of(nb) * KB + kb) * kBlockBytes + wl); };
+    // (scale, zero) pairs of kChunk k blocks: 64 bytes per block -> LDS [nb][k block][64 B], requested a chunk ahead
+    constexpr int kPieces = NB * kChunk * 4 / 64;  // 16-byte pieces per lane
+    v4i sv[kPieces];
+    auto request_scales = [&](int kb) {
+#pragma unroll
+      for (int i = 0; i < kPieces; ++i) {
+        const int c = lane + 64 * i, nb = c / (kChunk * 4), rest = c % (kChunk * 4);
+        sv[i] = gload<v4i>(sb + ((long)block_of(nb) * KB + min(kb + rest / 4, KB - 1)) * 64 + rest % 4 * 16);
+      }
+    };
+    const _Float16* xr[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) xr[mb] = reinterpret_cast<const _Float16*>(t.A) + (long)src[mb] * K + lg * 32;
+    auto x_of = [&](int mb, int j, int kb) { return __builtin_bit_cast(v8h, gload<v4i>(xr[mb] + kb * 128 + j * 8)); };
+
+    WReg wr[NB];
+    v8h xf[MB][4];  // (rows past M repeat the last one: their columns are never stored)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) xf[mb][j] = x_of(mb, j, kb_lo);
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) wr[nb] = w_of(nb, kb_lo);
+    request_scales(kb_lo);
+    __builtin_amdgcn_sched_barrier(0);
+    auto step = [&](auto morec, int kb, const uint8_t* sp) {
+      constexpr bool kMore = decltype(morec)::value;
+      v8h xn[MB][4];
+      if constexpr (kMore) {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) xn[mb][j] = x_of(mb, j, kb + 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      v4f sx[MB], sxb[MB];
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        sx[mb] = sxb[mb] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          sx[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, xf[mb][j], sx[mb], 0, 0, 0);
+          sxb[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bias, xf[mb][j], sxb[mb], 0, 0, 0);
+        }
+      }
+      // pipelined by channel block: between the matrix instructions of block nb, the sums of block nb - 1 are scaled and block nb + 1 is unpacked, operand
+      // by operand into the registers that block nb has just used
+      v8h wf[4], s8[2];
+      v4f part[2][MB];
+      unpack(wr[0], wf);
+      static_for<NB>([&](auto nbc) {
+        constexpr int nb = decltype(nbc)::value, cur = nb & 1, prev = cur ^ 1;
+        s8[cur] = __builtin_bit_cast(v8h, *reinterpret_cast<const v4i*>(sp + nb * (kChunk * 64)));  // (scale, zero) of channels 4*lg .. 4*lg+3
+        if constexpr (kMore) wr[nb] = w_of(nb, kb + 1);  // (unpacked already)
+        __builtin_amdgcn_sched_barrier(0);  // the refill is issued here
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) part[cur][mb] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) part[cur][mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[j], xf[mb][j], part[cur][mb], 0, 0, 0);
+          if constexpr (nb + 1 < NB) {
+            v8h w[4];
+            unpack(wr[nb + 1], w);
+            wf[j] = w[j];
+          }
+          if constexpr (nb > 0) {
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+              acc[nb - 1][mb][j] = __builtin_fmaf(part[prev][mb][j] - sxb[mb][j], (float)s8[prev][2 * j], __builtin_fmaf(sx[mb][j], (float)s8[prev][2 * j + 1], acc[nb - 1][mb][j]));
+          }
+          sched_mfma_valu<(nb + 1 < NB ? 5 : 0) + (nb > 0 ? 3 * MB : 0), MB, 0>();
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      });
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc[NB - 1][mb][e] = __builtin_fmaf(part[(NB - 1) & 1][mb][e] - sxb[mb][e], (float)s8[(NB - 1) & 1][2 * e], __builtin_fmaf(sx[mb][e], (float)s8[(NB - 1) & 1][2 * e + 1], acc[NB - 1][mb][e]));
+      if constexpr (kMore) {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) xf[mb][j] = xn[mb][j];
+      }
+    };
+#pragma unroll 1
+    for (int kb0 = kb_lo; kb0 < kb_hi; kb0 += kChunk) {
+#pragma unroll
+      for (int i = 0; i < kPieces; ++i) *reinterpret_cast<v4i*>(spatch + (lane + 64 * i) * 16) = sv[i];
+      if (kb0 + kChunk < kb_hi) request_scales(kb0 + kChunk);
+      const uint8_t* sp = spatch + lg * 16;
+      const int end = min(kb0 + kChunk, kb_hi - 1);
+#pragma unroll 1
+      for (int kb = kb0; kb < end; ++kb, sp += 64) step(std::true_type{}, kb, sp);
+      if (kb0 + kChunk >= kb_hi) step(std::false_type{}, kb_hi - 1, sp);
+    }
+  }
+
   template <bool GU>
   __device__ static __forceinline__ void run(const TileArgs& t, uint8_t* __restrict__ smem) {
     const int tid = threadIdx.x;
@@ -253,18 +383,22 @@ struct SkinnyWoTile {
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = v4f{0.f, 0.f, 0.f, 0.f};
-    for (int kb = kb_lo; kb < kb_hi; kb += KP) {
-      const int nk = min(KP, kb_hi - kb);
-      if constexpr (KP >= 4) {
-        if (nk == 4) { pass<GU, 4>(t, kb, m0, n0, nbv, lane, src, spatch, acc); continue; }
+    if constexpr (kStream) {
+      stream<GU>(t, kb_lo, kb_hi, n0, nbv, lane, src, spatch, acc);
+    } else {
+      for (int kb = kb_lo; kb < kb_hi; kb += KP) {
+        const int nk = min(KP, kb_hi - kb);
+        if constexpr (KP >= 4) {
+          if (nk == 4) { pass<GU, 4>(t, kb, m0, n0, nbv, lane, src, spatch, acc); continue; }
+        }
+        if constexpr (KP >= 3) {
+          if (nk == 3) { pass<GU, 3>(t, kb, m0, n0, nbv, lane, src, spatch, acc); continue; }
+        }
+        if constexpr (KP >= 2) {
+          if (nk == 2) { pass<GU, 2>(t, kb, m0, n0, nbv, lane, src, spatch, acc); continue; }
+        }
+        pass<GU, 1>(t, kb, m0, n0, nbv, lane, src, spatch, acc);
       }
-      if constexpr (KP >= 3) {
-        if (nk == 3) { pass<GU, 3>(t, kb, m0, n0, nbv, lane, src, spatch, acc); continue; }
-      }
-      if constexpr (KP >= 2) {
-        if (nk == 2) { pass<GU, 2>(t, kb, m0, n0, nbv, lane, src, spatch, acc); continue; }
-      }
-      pass<GU, 1>(t, kb, m0, n0, nbv, lane, src, spatch, acc);
     }
 
     // reduction over the 4 waves in a fixed order (wave 0 + 1 + 2 + 3), 16-channel blocks dealt round-robin to the waves

@@ -3,7 +3,7 @@
 `TileConfig` / `QConfig` / `NO_QUANT` keep the fields (and therefore the dataclass `repr`, which is the key of the
 kernel-profile table) of mxmoe/kernels/tile_config.py:122-286.  What changes is the meaning the hardware gives them:
 WM x WN x WK counts 64-lane wavefronts (always 4 per workgroup here), MMA names an MFMA instruction, STAGE is the number of
-LDS ring slots of the DMA pipeline (3 for the MFMA tiles; for the few-token weight-only tiles 2 names the 12-deep register ring with 4 k blocks per pass and 4 the few-register shape), and the candidate lists are those compiled for gfx950.
+LDS ring slots of the DMA pipeline (3 for the MFMA tiles; for the few-token weight-only tiles 2 names the shape for mixed kernels and 4 the one compiled for three waves per SIMD), and the candidate lists are those compiled for gfx950.
 """
 from __future__ import annotations
 
@@ -199,8 +199,8 @@ class TileConfig:
 
     def smem_bytes_tile(self):
         """LDS bytes of the tile as compiled (csrc/include/mxmoe_tiles.hpp, mxmoe_wo_tiles.hpp)."""
-        if self.is_skinny():  # per-wave partial sums of the final reduction + (scale, zero) patches of one pass (4 k blocks, or 2)
-            kp = 2 if self.STAGE == 4 or self.BM == 32 else 4
+        if self.is_skinny():  # per-wave partial sums of the final reduction + (scale, zero) patches of 4 k blocks (2 in the 32-token 8-bit tile's passes)
+            kp = 2 if self.QCFGB.QBITS == 8 and self.BM == 32 else 4
             return 4 * (self.BN // 16) * (64 * 16 * (self.BM // 16) + kp * 64)
         if self.is_weight_only():
             return 2 * self.BM * 256  # two stages of BM activation rows x one 128-wide k block
@@ -217,7 +217,7 @@ class TileConfig:
         if self.is_skinny():
             if self.BM == 32:  # two blocks of 16 tokens against every unpacked weight: 2 k blocks per pass, 8 (8-bit: 4) packed blocks in flight
                 return f"SkinnyWoTile<{self.QCFGB.QBITS}, {self.BN}, 2, {4 if self.QCFGB.QBITS == 8 else 8}, 2, 2>"
-            # STAGE 4: the few-register shape (2 k blocks per pass, 4 packed blocks in flight per wave, compiled for 3 waves per SIMD)
+            # STAGE 4: compiled for 3 waves per SIMD (the two numbers in front count for 8-bit weights only)
             return f"SkinnyWoTile<{self.QCFGB.QBITS}, {self.BN}, 2, 4, 3>" if self.STAGE == 4 else f"SkinnyWoTile<{self.QCFGB.QBITS}, {self.BN}>"
         if self.is_weight_only():
             return f"WoMfmaTile<{self.QCFGB.QBITS}, {self.BM}, {self.BN}>"
@@ -289,7 +289,7 @@ def get_possible_tile_list(arch: str, qcfg: str) -> list:
     if mma == "MFMA_F32_16x16x32_F16":
         skinny = [_with_q(TileConfig(BM=16, BN=bn, BK=128, WM=1, WN=4, WK=1, STAGE=2, MMA=mma), qcfg) for bn in (128, 64)]
         skinny.append(_with_q(TileConfig(BM=32, BN=128, BK=128, WM=1, WN=4, WK=1, STAGE=2, MMA=mma), qcfg))  # experts with 17 .. 32 (.. 64) tokens
-        if QCFG_MAP[qcfg].QCFGB.QBITS != 8:  # the few-register shape, for kernels made of few-token tiles alone (three workgroups per CU)
+        if QCFG_MAP[qcfg].QCFGB.QBITS != 8:  # compiled for 3 waves per SIMD, for kernels made of few-token tiles alone (three workgroups per CU)
             skinny.append(_with_q(TileConfig(BM=16, BN=128, BK=128, WM=1, WN=4, WK=1, STAGE=4, MMA=mma), qcfg))
         # (8-bit weights: the ring of packed blocks is twice as large, which leaves room for the 2 x 2 shape's accumulators only)
         shapes = ((128, 2, 2),) if QCFG_MAP[qcfg].QCFGB.QBITS == 8 else ((128, 2, 2), (256, 1, 4))

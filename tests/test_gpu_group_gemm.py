@@ -354,6 +354,31 @@ def test_weight_only_tiles_of_32_tokens():
                     assert np.array_equal(a.view(np.uint16), b.view(np.uint16)), p["size"]
 
 
+@pytest.mark.parametrize("k", [128, 384, 512, 640, 2048, 2560, 4096, 4608])
+@pytest.mark.parametrize("bits", [4, 3, 2, 8])
+def test_weight_only_streams_of_every_length(k, bits):
+    """The few-token tiles deal K to four waves, and each walks its part as one stream whose (scale, zero) pairs come four 128-wide blocks at a
+    time: parts of no block, fewer than four, exactly four, one more, and more than eight; 1, 16, 17 and 32 rows.  Against the product with
+    the dequantised weights in float64: one rounding of an output to fp16 is at most 2^-11 of it, so 2^-11 of the norm; the fp32 sums, of
+    terms that still carry the codes' bias of 1024 (128 of them: partial sums near 2^14, steps of 2^-10 against a result near 2^8), get as much again."""
+    from mxmoe_amd.weights import quantize_and_pack
+
+    rng = np.random.default_rng(k + bits)
+    probs = []
+    for m, n in [(1, 144), (16, 128), (17, 256), (32, 160)]:
+        x = rng.standard_normal((m, k)).astype(F16)
+        w = (rng.standard_normal((n, k)) * 0.02).astype(F16)
+        pw = quantize_and_pack(torch.from_numpy(w), (16, bits, 128, False))
+        q, s, z = O.quant_minmax(w, bits, 128, False)
+        deq = q.reshape(n, k // 128, 128).astype(np.float64) * s.reshape(n, -1, 1).astype(np.float64) + z.reshape(n, -1, 1).astype(np.float64)
+        probs.append(dict(A=torch.from_numpy(x).to(DEV), B=pw.data.to(DEV), sb=pw.scale.to(DEV), ref=x.astype(np.float64) @ deq.reshape(n, k).T,
+                          size=(m, n, k), q=(16, bits, 128, False)))
+    _, outs, _ = _launch(probs, dump=False)
+    for p, out in zip(probs, outs):
+        err = np.linalg.norm(out.astype(np.float64) - p["ref"]) / np.linalg.norm(p["ref"])
+        assert err <= 2.0 ** -10, (p["size"], err)
+
+
 def test_weight_only_many_tokens():
     """Experts with many tokens run the 128 x 256 dequantise-to-fp16 MFMA tile (and the remainder rows the skinny one); channel
     counts that leave one or two of its four waves without channels are among the cases."""
