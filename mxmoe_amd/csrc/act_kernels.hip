@@ -263,6 +263,123 @@ __device__ __forceinline__ void bf6_emit_row(const uint8_t* codes, int row_elems
 // that is a multiple of 64.
 __device__ __forceinline__ int xcd_row_group(int wg) { return (wg & ~63) | ((wg & 7) << 3) | ((wg >> 3) & 7); }
 
+// What every kernel of one row per workgroup does with a finished row, chunk tid + NT i of it in v[i]: fp16 copy or symmetric quantisation.  `red`: one slot per
+// wave; `codes`: LDS for the row as fp16 (tag 4).  Passes barriers only where `tag` is
+// neither 0 nor 3.
+template <int MAXC, int NT, bool EXT>
+__device__ __forceinline__ void store_row(const float (&v)[MAXC][8], int n, int tag, long lrow, long inp_off, long scale_off, uint8_t* inp_store, _Float16* scale_store,
+                                          float* red, uint8_t* codes) {
+  const int tid = threadIdx.x, nchunks = n >> 3;
+  if (tag == 0) {
+    _Float16* out = reinterpret_cast<_Float16*>(inp_store) + inp_off + lrow * n;
+#pragma unroll
+    for (int i = 0; i < MAXC; ++i) {
+      const int c = tid + i * NT;
+      if (c < nchunks) {
+        v8h o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[j] = (_Float16)v[i][j];
+        *reinterpret_cast<v8h*>(out + c * 8) = o;
+      }
+    }
+    return;
+  }
+  if (tag == 3) {
+    // int4 with one scale per 128 values: a group is 16 consecutive chunks, i.e. the 16 lanes of an aligned lane group (the chunk
+    // index and the lane index agree modulo 16), so its absmax is a 4-step exchange inside those lanes.  Row: n / 2 bytes of codes,
+    // n / 128 scales.
+    uint8_t* out = inp_store + 2 * (inp_off + lrow * (n / 4));
+    _Float16* sout = scale_store + scale_off + lrow * (n >> 7);
+#pragma unroll
+    for (int i = 0; i < MAXC; ++i) {
+      const int c = tid + i * NT;
+      const bool live = c < nchunks;  // whole lane groups are live or not: n is a multiple of 128
+      float gmax = 0.0f;
+      if (live) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) gmax = fmaxf(gmax, fabsf(v[i][j]));
+      }
+      gmax = row16_max(gmax);
+      float scale = round_h(gmax / 7.0f);
+      if (scale == 0.0f) scale = 1.0f;
+      const ScaleDiv div(scale);
+      if (live) {
+        if ((c & 15) == 0) sout[c >> 4] = (_Float16)scale;
+        unsigned w = 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float r = round_h(div(v[i][j]));
+          w = push_code<4>(w, code_word(fminf(fmaxf(r, -7.0f), 7.0f)));
+        }
+        *reinterpret_cast<unsigned*>(out + c * 4) = w;
+      }
+    }
+    return;
+  }
+  float amax = 0.0f;
+#pragma unroll
+  for (int i = 0; i < MAXC; ++i) {
+    const int c = tid + i * NT;
+    if (c < nchunks) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[i][j]));
+    }
+  }
+  amax = wave_max(amax);
+  __syncthreads();
+  if ((tid & 63) == 0) red[tid >> 6] = amax;
+  __syncthreads();
+  amax = red[0];
+#pragma unroll
+  for (int w = 1; w < NT / 64; ++w) amax = fmaxf(amax, red[w]);
+  const float upper = tag == 1 ? 127.0f : (EXT && tag == 5 ? 448.0f : 7.0f);
+  float scale = round_h(amax / upper);   // fp16 division: fp32 quotient of two fp16 values, rounded to fp16
+  if (scale == 0.0f) scale = 1.0f;       // quantize.cuh:258
+  const ScaleDiv div(scale);
+  if (tid == 0) scale_store[scale_off + lrow] = (_Float16)scale;
+  if (EXT && tag == 4) {  // the row's codes as fp16 in LDS (in place of the row itself, which every thread is done reading), then fragments
+#pragma unroll
+    for (int i = 0; i < MAXC; ++i) {
+      const int c = tid + i * NT;
+      if (c < nchunks) *reinterpret_cast<v8h*>(codes + c * 16) = bf6_chunk_codes(v[i], div);
+    }
+    __syncthreads();
+    bf6_emit_row(codes, n, 0, n, inp_store + 2 * inp_off, lrow, tid, NT);
+    return;  // (the next row begins with a barrier before it touches LDS)
+  }
+  uint8_t* out = inp_store + 2 * (inp_off + lrow * (tag == 1 || (EXT && tag == 5) ? n / 2 : n / 4));
+#pragma unroll
+  for (int i = 0; i < MAXC; ++i) {
+    const int c = tid + i * NT;
+    if (c < nchunks) {
+      if (EXT && tag == 5) {
+        *reinterpret_cast<uint2*>(out + c * 8) = fp8_chunk_codes(v[i], div);
+        continue;
+      }
+      unsigned q[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float r = round_h(div(v[i][j]));
+        q[j] = code_word(fminf(fmaxf(r, -upper), upper));
+      }
+      if (tag == 1) {
+        uint2 w{0, 0};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          w.x = push_code<8>(w.x, q[j]);
+          w.y = push_code<8>(w.y, q[j + 4]);
+        }
+        *reinterpret_cast<uint2*>(out + c * 8) = w;
+      } else {
+        unsigned w = 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) w = push_code<4>(w, q[j]);
+        *reinterpret_cast<unsigned*>(out + c * 4) = w;
+      }
+    }
+  }
+}
+
 // NT threads per workgroup (256, or 192 when that wastes fewer lanes: a 1408-element row is 176 chunks of 8).
 template <int MAXC, bool SILU, int NT, bool EXT>
 __device__ __forceinline__ void row_quant_body(const RowArgs& a, const int wg, const int wgs, float* const lds) {
@@ -536,118 +653,10 @@ __device__ __forceinline__ void row_quant_body(const RowArgs& a, const int wg, c
       }
     }
 
-    // ---- store: fp16 copy or per-token symmetric quantisation ----
-    if (tag == 0) {
-      _Float16* out = reinterpret_cast<_Float16*>(a.inp_store) + inp_off + lrow * n;
-#pragma unroll
-      for (int i = 0; i < MAXC; ++i) {
-        const int c = tid + i * NT;
-        if (c < nchunks) {
-          v8h o;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) o[j] = (_Float16)v[i][j];
-          *reinterpret_cast<v8h*>(out + c * 8) = o;
-        }
-      }
-      continue;
-    }
-    if (tag == 3) {
-      // int4 with one scale per 128 values: a group is 16 consecutive chunks, i.e. the 16 lanes of an aligned lane group (the chunk
-      // index and the lane index agree modulo 16), so its absmax is a 4-step exchange inside those lanes.  Row: n / 2 bytes of codes,
-      // n / 128 scales.
-      uint8_t* out = a.inp_store + 2 * (inp_off + lrow * (n / 4));
-      _Float16* sout = a.scale_store + scale_off + lrow * (n >> 7);
-#pragma unroll
-      for (int i = 0; i < MAXC; ++i) {
-        const int c = tid + i * NT;
-        const bool live = c < nchunks;  // whole lane groups are live or not: n is a multiple of 128
-        float gmax = 0.0f;
-        if (live) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) gmax = fmaxf(gmax, fabsf(v[i][j]));
-        }
-        gmax = row16_max(gmax);
-        float scale = round_h(gmax / 7.0f);
-        if (scale == 0.0f) scale = 1.0f;
-        const ScaleDiv div(scale);
-        if (live) {
-          if ((c & 15) == 0) sout[c >> 4] = (_Float16)scale;
-          unsigned w = 0;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const float r = round_h(div(v[i][j]));
-            w = push_code<4>(w, code_word(fminf(fmaxf(r, -7.0f), 7.0f)));
-          }
-          *reinterpret_cast<unsigned*>(out + c * 4) = w;
-        }
-      }
-      continue;
-    }
-    float amax = 0.0f;
-#pragma unroll
-    for (int i = 0; i < MAXC; ++i) {
-      const int c = tid + i * NT;
-      if (c < nchunks) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[i][j]));
-      }
-    }
-    amax = wave_max(amax);
-    __syncthreads();
-    if ((tid & 63) == 0) red[tid >> 6] = amax;
-    __syncthreads();
-    amax = red[0];
-#pragma unroll
-    for (int w = 1; w < NT / 64; ++w) amax = fmaxf(amax, red[w]);
-    const float upper = tag == 1 ? 127.0f : (EXT && tag == 5 ? 448.0f : 7.0f);
-    float scale = round_h(amax / upper);   // fp16 division: fp32 quotient of two fp16 values, rounded to fp16
-    if (scale == 0.0f) scale = 1.0f;       // quantize.cuh:258
-    const ScaleDiv div(scale);
-    if (tid == 0) a.scale_store[scale_off + lrow] = (_Float16)scale;
-    if (EXT && tag == 4) {  // the row's codes as fp16 in LDS (in place of the row itself, which every thread is done reading), then fragments
-      uint8_t* codes = reinterpret_cast<uint8_t*>(x);
-#pragma unroll
-      for (int i = 0; i < MAXC; ++i) {
-        const int c = tid + i * NT;
-        if (c < nchunks) *reinterpret_cast<v8h*>(codes + c * 16) = bf6_chunk_codes(v[i], div);
-      }
-      __syncthreads();
-      bf6_emit_row(codes, n, 0, n, a.inp_store + 2 * inp_off, lrow, tid, NT);
-      continue;  // (the next row begins with a barrier before it touches LDS)
-    }
-    uint8_t* out = a.inp_store + 2 * (inp_off + lrow * (tag == 1 || (EXT && tag == 5) ? n / 2 : n / 4));
-#pragma unroll
-    for (int i = 0; i < MAXC; ++i) {
-      const int c = tid + i * NT;
-      if (c < nchunks) {
-        if (EXT && tag == 5) {
-          *reinterpret_cast<uint2*>(out + c * 8) = fp8_chunk_codes(v[i], div);
-          continue;
-        }
-        unsigned q[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float r = round_h(div(v[i][j]));
-          q[j] = code_word(fminf(fmaxf(r, -upper), upper));
-        }
-        if (tag == 1) {
-          uint2 w{0, 0};
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            w.x = push_code<8>(w.x, q[j]);
-            w.y = push_code<8>(w.y, q[j + 4]);
-          }
-          *reinterpret_cast<uint2*>(out + c * 8) = w;
-        } else {
-          unsigned w = 0;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) w = push_code<4>(w, q[j]);
-          *reinterpret_cast<unsigned*>(out + c * 4) = w;
-        }
-      }
-    }
+    store_row<MAXC, NT, EXT>(v, n, tag, lrow, inp_off, scale_off, a.inp_store, a.scale_store, red, reinterpret_cast<uint8_t*>(x));
   }
 }
+
 template <int MAXC, bool SILU, int NT, bool EXT>
 __global__ void __launch_bounds__(NT) row_quant_kernel(const RowArgs a) {
   extern __shared__ __align__(16) float lds[];
@@ -1300,15 +1309,307 @@ __global__ void __launch_bounds__(256) row_quant_dense_kernel(const RowArgs a) {
   row_quant_dense_body<MAXC, SILU, EXT>(a, blockIdx.x, gridDim.x, dlds);
 }
 
-// Routed rows by row_quant_dense_kernel's code and the shared expert's rows, of another length, by row_quant_kernel's, next to each other in
-// one launch: neither needs anything of the other, and a launch of a few hundred shared rows is one long chain per row (15 us) on a chip
-// that is mostly idle.  The first `shared_wgs` workgroups (a multiple of 64: xcd_row_group) take the shared rows, which run longest.
-template <int MAXC, bool EXT>
+// One row per WORKGROUP of four waves with the dense stage on the matrix cores, for rotations S_f kron B_kb kron H_m: a shared expert's rows (m = 16 .. 128: 2816 =
+// 4 x 44 x 16, 5632 = 4 x 44 x 32), and those of m = 8 (1408 = 4 x 44 x 8) that row_quant_dense_kernel takes one row per wave, where there are too few of
+// them to fill the chip.  The Sylvester part runs in registers (a k row is at most 16 lanes long).  The snapped row goes to LDS as it is, [block of kb k
+// rows][k][column]; a wave gathers the second operand of 16 columns from there, two bytes per read, multiplies B (first operand, in LDS in operand
+// order) into them, and the results return through LDS in row order.  Arithmetic of the other row kernels, bit for bit.
+struct BlockRows {  // LDS of a workgroup, in bytes
+  int kb, m, f, ksteps, mblocks;
+  int pitch;   // k row of m values.  m > 8: 8 k rows are 64 bytes modulo 256, so the lane groups of a gather touch different banks
+  int blk;     // block of kb k rows of the snapped row, padded to whole k steps
+  int snapped, rotated, codes;
+  __host__ __device__ explicit BlockRows(const RotPlan& p) {
+    kb = p.kb, m = p.m, f = p.f;
+    ksteps = (kb + 31) >> 5, mblocks = (kb + 15) >> 4;
+    pitch = m > 8 ? 2 * m + 8 : 16;
+    blk = ksteps * 32 * pitch + (m > 8 ? 0 : 32);
+    snapped = (m > 8 || f > 2 ? f : 2) * blk;  // (H_8: 16 columns are two blocks)
+    rotated = f * kb * pitch + 16;             // (a slot for discarded values at the end)
+    codes = mblocks * ksteps * 1024;
+  }
+  __host__ __device__ int lds() const { return codes + ((snapped + 15) & ~15) + ((rotated + 15) & ~15) + 2 * 12 * 4; }
+};
+template <int NT, int MAXC, bool SILU, bool EXT>
+__device__ __forceinline__ void row_quant_block_body(const RowArgs& a, const int wg, const int wgs, uint8_t* const lds) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lm = lane & 15, lg = lane >> 4;
+  constexpr int kW = NT / 64;
+  const RotPlan pl = a.plan;
+  const BlockRows g(pl);
+  const int n = pl.n, nchunks = n >> 3, kb = pl.kb, ksteps = g.ksteps, mblocks = g.mblocks;
+  const int mc = pl.m >> 3, mc_log2 = 31 - __clz(mc);  // chunks per k row
+  const int f_rows = pl.f * kb;                        // k rows
+  uint8_t* const xt = lds + g.codes;
+  uint8_t* const yrow = xt + ((g.snapped + 15) & ~15);
+  float* const red = reinterpret_cast<float*>(yrow + ((g.rotated + 15) & ~15));  // [kW] row maxima, [kW] for store_row
+  // place of chunk c (k row c / mc) in the snapped and in the rotated row
+  auto at_x = [&](int c) {
+    const int k = c >> mc_log2, blk = (k >= kb) + (k >= 2 * kb) + (k >= 3 * kb);
+    return blk * g.blk + (k - blk * kb) * g.pitch + (c & (mc - 1)) * 16;
+  };
+  auto at_y = [&](int c) { return (c >> mc_log2) * g.pitch + (c & (mc - 1)) * 16; };
+
+  // B as the first operand of v_mfma_f32_16x16x32_f16: lane holds row 16 mb + (lane & 15), k = 32 ks + 8 (lane >> 4) + 0..7.  Requested before anything else:
+  // it does not wait for the row's bookkeeping.
+  float sv[8];
+  auto load_signs = [&](int blkid) {
+    const int mb = blkid / ksteps, ks = blkid - mb * ksteps;
+    const float* const p = a.signs + min(16 * mb + lm, kb - 1) * kb;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sv[i] = gload<float>(p + min(32 * ks + 8 * lg + i, kb - 1));
+  };
+  auto put_signs = [&](int blkid) {
+    const int mb = blkid / ksteps, ks = blkid - mb * ksteps;
+    v8h bs;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) bs[i] = (16 * mb + lm < kb && 32 * ks + 8 * lg + i < kb) ? (_Float16)sv[i] : (_Float16)0.0f;
+    *reinterpret_cast<v8h*>(lds + blkid * 1024 + lane * 16) = bs;
+  };
+  load_signs(min(wave, mblocks * ksteps - 1));
+  // columns and k positions that no row ever writes must read as zero
+  for (int i = tid; i < g.snapped / 8; i += NT) reinterpret_cast<uint2*>(xt)[i] = make_uint2(0, 0);
+
+  struct RowMeta {
+    int tag;
+    long lrow, inp_off, scale_off;
+    const _Float16* srow;
+    bool exists;
+  };
+  const _Float16* const src_shared = shared_src(a);
+  const int routed = a.routed_ptr ? (int)const_load(a.routed_ptr) : a.R;  // rows [routed, R) of a planned launch do not exist
+  auto load_meta = [&](int row) {
+    RowMeta m;
+    const bool shared_row = row >= a.R;
+    m.exists = row < routed || shared_row;
+    const int e = shared_row ? a.E : (m.exists ? const_load(a.dst_exp + row) : 0);
+    // (the source of a row that is read in place does not wait for the row's expert: rows [routed, R) lie inside the store)
+    const long r = shared_row ? (long)(row - a.R) : (a.perm ? (m.exists ? (long)const_load(a.perm + row) : 0l) : (long)row);
+    m.srow = (shared_row ? src_shared : a.src) + r * n * (SILU ? 2 : 1);
+    m.tag = (int)const_load(a.table + e);
+    m.exists = m.exists && !row_stays(a, m.tag);
+    m.lrow = shared_row ? row - a.R : row - const_load(a.table + a.Et + e);
+    m.inp_off = const_load(a.table + 2 * a.Et + e);
+    m.scale_off = const_load(a.table + 3 * a.Et + e);
+    return m;
+  };
+  auto load_data = [&](const RowMeta& m, v8h (&gt)[MAXC], v8h (&up)[MAXC]) {
+#pragma unroll
+    for (int i = 0; i < MAXC; ++i) {
+      const int c = min(tid + NT * i, nchunks - 1);  // threads past the row re-read its last chunk (never used)
+      gt[i] = gload<v8h>(m.srow + c * 8);
+      if (SILU) up[i] = gload<v8h>(m.srow + n + c * 8);
+    }
+  };
+  RowMeta next_meta;
+  v8h row_g[MAXC], row_u[MAXC];
+  if (wg < a.rows) {
+    next_meta = load_meta(wg);
+    load_data(next_meta, row_g, row_u);
+  }
+  for (int blkid = wave; blkid < mblocks * ksteps; blkid += kW) {
+    if (blkid != wave) load_signs(blkid);
+    put_signs(blkid);
+  }
+
+  for (int row = wg; row < a.rows; row += wgs) {
+    const RowMeta cur = next_meta;
+    const bool has_next = row + wgs < a.rows;
+    if (has_next) next_meta = load_meta(row + wgs);
+    float v[MAXC][8];
+#pragma unroll
+    for (int i = 0; i < MAXC; ++i) {
+      const bool live = tid + NT * i < nchunks;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float x = (float)row_g[i][j];
+        const float y = SILU ? round_h(keep_f32(silu_fixed(x) * (float)row_u[i][j])) : x;
+        v[i][j] = live ? y : 0.0f;  // (chunks past the row count as zeros in its maxima and are never stored)
+      }
+    }
+    if (has_next) load_data(next_meta, row_g, row_u);
+    if (!cur.exists) continue;  // (the whole workgroup)
+    const int tag = cur.tag;
+    const bool rot = a.rotate == 2 || (a.rotate == 1 && tag != 0);
+    __syncthreads();  // previous row fully consumed (and B and the zeros staged)
+    if (rot) {
+      float mx = 0.0f;
+#pragma unroll
+      for (int i = 0; i < MAXC; ++i) {
+#pragma unroll
+        for (int h = 1; h < 8; h <<= 1)
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            if (!(j & h)) {
+              const float p = v[i][j], q = v[i][j + h];
+              v[i][j] = p + q;
+              v[i][j + h] = p - q;
+            }
+        // strides 8 .. m / 2: the partner chunk is 1 .. 8 lanes away
+        auto stage = [&](auto dc) {
+#pragma unroll
+          for (int j = 0; j < 8; j += 2) lane_butterfly<decltype(dc)::value>(v[i][j], v[i][j + 1], lane);
+        };
+        if (mc > 1) stage(std::integral_constant<int, 1>{});
+        if (mc > 2) stage(std::integral_constant<int, 2>{});
+        if (mc > 4) stage(std::integral_constant<int, 4>{});
+        if (mc > 8) stage(std::integral_constant<int, 8>{});
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          v[i][j] = round_h(keep_f32(v[i][j] * pl.scale));
+          mx = fmaxf(mx, fabsf(v[i][j]));
+        }
+      }
+      mx = wave_max(mx);
+      if (lane == 0) red[wave] = mx;
+      __syncthreads();
+      mx = red[0];
+#pragma unroll
+      for (int w = 1; w < kW; ++w) mx = fmaxf(mx, red[w]);
+      const DenseGrid grid(mx);
+#pragma unroll
+      for (int i = 0; i < MAXC; ++i) {
+        const int c = tid + NT * i;
+        if (c < nchunks) {
+          v8h q;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) q[j] = (_Float16)(rintf(v[i][j] * grid.to_grid) * 0.0625f);
+          *reinterpret_cast<v8h*>(xt + at_x(c)) = q;
+        }
+      }
+      __syncthreads();
+      const float back = grid.from_grid * 16.0f;
+      auto b_of = [&](int mb, int ks) { return *reinterpret_cast<const v8h*>(lds + (mb * ksteps + ks) * 1024 + lane * 16); };
+      const int discard = f_rows * g.pitch;
+      auto dense_stage = [&](auto f_const) {
+        constexpr int F = decltype(f_const)::value;
+        if (pl.m > 8) {
+          // 16 columns x 16 rows of B at a time, the f blocks in f sets of accumulators: lane holds column col and rows b = 16 mb + 4 lg + r of each, so the S_f
+          // butterflies stay in its registers
+#pragma unroll 1
+          for (int unit = wave; unit < (pl.m >> 4) * mblocks; unit += kW) {
+            const int ct = unit / mblocks, mb = unit - ct * mblocks;
+            const int col2 = (ct * 16 + lm) * 2;
+            v4f acc[F];
+#pragma unroll
+            for (int q = 0; q < F; ++q) acc[q] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (int ks = 0; ks < ksteps; ++ks) {
+              const v8h bs = b_of(mb, ks);
+              const uint8_t* const x0 = xt + (32 * ks + 8 * lg) * g.pitch + col2;
+#pragma unroll
+              for (int q = 0; q < F; ++q) {
+                v8h xf;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) xf[i] = *reinterpret_cast<const _Float16*>(x0 + q * g.blk + i * g.pitch);
+                acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bs, xf, acc[q], 0, 0, 0);
+              }
+            }
+#pragma unroll
+            for (int h = 1; h < F; h <<= 1)
+#pragma unroll
+              for (int q = 0; q < F; ++q)
+                if (!(q & h)) {
+                  const v4f lo = acc[q], hi = acc[q + h];
+#pragma unroll
+                  for (int r = 0; r < 4; ++r) {
+                    const float x = lo[r], y = hi[r];
+                    acc[q][r] = x + y;
+                    acc[q + h][r] = x - y;
+                  }
+                }
+#pragma unroll
+            for (int q = 0; q < F; ++q)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                const int b = 16 * mb + 4 * lg + r;
+                *reinterpret_cast<_Float16*>(yrow + (b < kb ? (q * kb + b) * g.pitch + col2 : discard)) = (_Float16)(acc[q][r] * back);
+              }
+          }
+        } else if (wave < mblocks) {
+          // 16 rows of B, all 8 f columns: lane holds column 16 nb + lm, i.e. value lm & 7 of block blk0 + 2 nb, and rows b = 16 wave + 4 lg + r; the S_f
+          // butterflies across blocks (bit 0 = lane bit 3, bit 1 = nb; ascending), then the one rounding to fp16
+          constexpr int NCOLS = F > 2 ? 2 : 1;
+          const float sgn8 = (lane & 8) ? -1.0f : 1.0f;
+          const int blk0 = lm >> 3, jj = lm & 7;
+          v4f acc[NCOLS];
+#pragma unroll
+          for (int nb = 0; nb < NCOLS; ++nb) acc[nb] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+          for (int ks = 0; ks < ksteps; ++ks) {
+            const v8h bs = b_of(wave, ks);
+            const uint8_t* const x0 = xt + blk0 * g.blk + (32 * ks + 8 * lg) * 16 + jj * 2;
+#pragma unroll
+            for (int nb = 0; nb < NCOLS; ++nb) {
+              v8h xf;
+#pragma unroll
+              for (int i = 0; i < 8; ++i) xf[i] = *reinterpret_cast<const _Float16*>(x0 + 2 * nb * g.blk + i * 16);
+              acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bs, xf, acc[nb], 0, 0, 0);
+            }
+          }
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int b = 16 * wave + 4 * lg + r;
+            const bool ok = b < kb && blk0 < F;
+            float t0 = acc[0][r], t1 = 0.0f;
+            if constexpr (F > 1) t0 = __builtin_fmaf(sgn8, t0, lane_xor<8>(t0));
+            if constexpr (F > 2) {
+              t1 = acc[NCOLS - 1][r];
+              t1 = __builtin_fmaf(sgn8, t1, lane_xor<8>(t1));
+              const float p = t0, q = t1;
+              t0 = p + q;
+              t1 = p - q;
+            }
+            *reinterpret_cast<_Float16*>(yrow + (ok ? (blk0 * kb + b) * 16 + jj * 2 : discard)) = (_Float16)(t0 * back);
+            if constexpr (F > 2) *reinterpret_cast<_Float16*>(yrow + (ok ? ((blk0 + 2) * kb + b) * 16 + jj * 2 : discard)) = (_Float16)(t1 * back);
+          }
+        }
+      };
+      switch (pl.f) {
+        case 1: dense_stage(std::integral_constant<int, 1>{}); break;
+        case 2: dense_stage(std::integral_constant<int, 2>{}); break;
+        default: dense_stage(std::integral_constant<int, 4>{}); break;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < MAXC; ++i) {
+        const int c = tid + NT * i;
+        if (c < nchunks) {
+          const v8h y = *reinterpret_cast<const v8h*>(yrow + at_y(c));
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[i][j] = (float)y[j];
+        }
+      }
+    }
+    store_row<MAXC, NT, EXT>(v, n, tag, cur.lrow, cur.inp_off, cur.scale_off, a.inp_store, a.scale_store, red + kW, yrow);
+  }
+}
+template <int MAXC, bool SILU, bool EXT>
+__global__ void __launch_bounds__(256) row_quant_block_kernel(const RowArgs a) {
+  extern __shared__ __align__(16) uint8_t blds[];
+  row_quant_block_body<256, MAXC, SILU, EXT>(a, blockIdx.x, gridDim.x, blds);
+}
+
+// Routed rows and the shared expert's rows, of another length, next to each other in one launch: neither needs anything of the other, and either alone
+// leaves most of the chip idle when it is short.  The first `shared_wgs` workgroups (a multiple of 64: xcd_row_group) take the shared rows, which run longest,
+// by row_quant_block_kernel's code, the others the routed rows by row_quant_dense_kernel's.
+template <int MAXC, bool SILU, bool EXT>
 __global__ void __launch_bounds__(256) row_quant_pair_kernel(const RowArgs routed, const RowArgs shared, const int shared_wgs) {
   extern __shared__ __align__(16) uint8_t plds[];
   const int wg = blockIdx.x;
-  if (wg < shared_wgs) row_quant_body<3, false, 256, EXT>(shared, wg, shared_wgs, reinterpret_cast<float*>(plds));
-  else row_quant_dense_body<MAXC, false, EXT>(routed, wg - shared_wgs, (int)gridDim.x - shared_wgs, plds);
+  if (wg < shared_wgs) row_quant_block_body<256, 3, SILU, EXT>(shared, wg, shared_wgs, plds);
+  else row_quant_dense_body<MAXC, SILU, EXT>(routed, wg - shared_wgs, (int)gridDim.x - shared_wgs, plds);
+}
+// The same for few rows, one of either kind per workgroup: the chain of one row's steps is all there is.  64 shared rows of 5632 values and 256 routed ones
+// of 1408: 15.6 us in row_quant_kernel, 11.3 / 9.4 / 11.5 here with 256 / 384 / 768 threads.
+constexpr int kFewThreads = 384;
+template <int NT, int MAXC, bool SILU, bool EXT>
+__global__ void __launch_bounds__(NT) row_quant_few_kernel(const RowArgs routed, const RowArgs shared, const int shared_wgs) {
+  extern __shared__ __align__(16) uint8_t plds[];
+  const int wg = blockIdx.x;
+  if (wg < shared_wgs) row_quant_block_body<NT, MAXC, SILU, EXT>(shared, wg, shared_wgs, plds);
+  else row_quant_block_body<NT, 1, SILU, EXT>(routed, wg - shared_wgs, (int)gridDim.x - shared_wgs, plds);
 }
 
 // One row per WORKGROUP of 8 waves for rotations B_kb kron H_512 (kb <= 32, no Sylvester factor in the table: a 14336-value row is
@@ -1601,46 +1902,66 @@ static bool wide_rows(const RowArgs& a) {
   return a.plan.kb > 1 && a.plan.kb <= 32 && a.plan.m == 512 && a.plan.f == 1 && a.plan_shared.n == a.plan.n && a.plan_shared.kb == a.plan.kb && a.rotate != 0;
 }
 
-template <bool EXT>
-static int launch_pair(const RowArgs& routed, const RowArgs& shared, int lds_bytes, hipStream_t s) {
-  int dev = 0, cus = 256;
-  (void)hipGetDevice(&dev);
-  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  const int lds = std::max(lds_bytes, dense_lds(routed.plan.n, routed.plan.kb));  // (dense_rows: below 64 KiB)
-  const int shared_wgs = std::min(shared.rows, cus * 2) + 63 & ~63;
-  const int routed_wgs = std::min((routed.rows + 3) / 4, cus * 3) + 63 & ~63;
-  const dim3 grid(shared_wgs + routed_wgs);
-  switch ((routed.plan.n / 8 + 63) / 64) {
-    case 1: hipLaunchKernelGGL((row_quant_pair_kernel<1, EXT>), grid, dim3(256), lds, s, routed, shared, shared_wgs); break;
-    case 2: hipLaunchKernelGGL((row_quant_pair_kernel<2, EXT>), grid, dim3(256), lds, s, routed, shared, shared_wgs); break;
-    case 3: hipLaunchKernelGGL((row_quant_pair_kernel<3, EXT>), grid, dim3(256), lds, s, routed, shared, shared_wgs); break;
-    default: hipLaunchKernelGGL((row_quant_pair_kernel<4, EXT>), grid, dim3(256), lds, s, routed, shared, shared_wgs); break;
-  }
+// Rows that row_quant_block_kernel takes: one length of at most 6144 values (three chunks per thread).
+static bool block_rows(const RowArgs& a) {
+  return a.plan.kb > 1 && a.plan.kb <= 64 && a.plan.n <= 8 * 256 * 3 && a.plan.f <= 4 && a.plan.m <= 128 &&
+         a.plan_shared.n == a.plan.n && a.plan_shared.kb == a.plan.kb && a.rotate != 0;
+}
+
+static int rows_launched() {
   const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) {
-    last_error() = std::string("kernel launch failed: ") + hipGetErrorString(e);
-    return 4;
-  }
-  return 0;
+  if (e == hipSuccess) return 0;
+  last_error() = std::string("kernel launch failed: ") + hipGetErrorString(e);
+  return 4;
 }
 
 template <bool SILU, bool EXT>
+static int launch_pair(const RowArgs& routed, const RowArgs& shared, bool dense, hipStream_t s) {
+  int dev = 0, cus = 256;
+  (void)hipGetDevice(&dev);
+  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  // (dense_rows and block_rows: at most 64 KiB of LDS)
+  // (workgroups per CU: 2049 shared rows of 2816 values and 12 294 routed ones of 1408, us, shared + routed per CU: 1 + 2 46, 1 + 3 50, 2 + 3 52, 2 + 4 48, 3 + 2 55;
+  // with the shared rows by row_quant_kernel's code 56)
+  const int lds = std::max(BlockRows(shared.plan).lds(), dense ? dense_lds(routed.plan.n, routed.plan.kb) : BlockRows(routed.plan).lds());
+  const int shared_wgs = std::min(shared.rows, cus) + 63 & ~63;
+  if (!dense) {
+    hipLaunchKernelGGL((row_quant_few_kernel<kFewThreads, 2, SILU, EXT>), dim3(shared.rows + routed.rows), dim3(kFewThreads), lds, s, routed, shared, shared.rows);
+    return rows_launched();
+  }
+  const int routed_wgs = std::min((routed.rows + 3) / 4, cus * 2) + 63 & ~63;
+  const dim3 grid(shared_wgs + routed_wgs);
+  switch ((routed.plan.n / 8 + 63) / 64) {
+    case 1: hipLaunchKernelGGL((row_quant_pair_kernel<1, SILU, EXT>), grid, dim3(256), lds, s, routed, shared, shared_wgs); break;
+    case 2: hipLaunchKernelGGL((row_quant_pair_kernel<2, SILU, EXT>), grid, dim3(256), lds, s, routed, shared, shared_wgs); break;
+    case 3: hipLaunchKernelGGL((row_quant_pair_kernel<3, SILU, EXT>), grid, dim3(256), lds, s, routed, shared, shared_wgs); break;
+    default: hipLaunchKernelGGL((row_quant_pair_kernel<4, SILU, EXT>), grid, dim3(256), lds, s, routed, shared, shared_wgs); break;
+  }
+  return rows_launched();
+}
+
+// Routed rows up to which one row per workgroup beats one row per wave (rows of 1408 values: 32 rows 7.8 -> 6.2 us).
+constexpr int kBlockRowsMax = 512;
+
+template <bool SILU, bool EXT>
 static int launch_rows_as(const RowArgs& a, int lds_bytes, hipStream_t s) {
-  // Shared rows of another length keep the routed rows out of the kernels made for one length: from some hundred rows on, two launches
-  // with the best kernel for each cost less than one with the kernel that takes any mixture.
-  if (a.plan_shared.n != a.plan.n && a.R >= kSplitSharedRows && a.rows > a.R) {
+  // Shared rows of another length keep the routed rows out of the kernels made for one length: both lengths' kernels side by side in one launch, or one launch
+  // after the other.
+  if (a.plan_shared.n != a.plan.n && a.rows > a.R) {
     RowArgs routed = a, shared = a;
     routed.rows = a.R;
     routed.plan_shared = a.plan;
     shared.R = 0;
     shared.rows = a.rows - a.R;
     shared.plan = a.plan_shared;
-    if constexpr (!SILU) {
-      if (shared.rows <= kPairSharedRows && dense_rows(routed) && !dense_rows(shared) && !wide_rows(shared) && shared.plan.kb > 1 && shared.plan.n <= 8 * 256 * 3 && lds_bytes <= 64 * 1024)
-        return launch_pair<EXT>(routed, shared, lds_bytes, s);
+    if (a.R > 0 && shared.rows <= kPairSharedRows && dense_rows(routed) && block_rows(shared)) {
+      const bool few = a.R <= kBlockRowsMax;
+      if (!few || block_rows(routed)) return launch_pair<SILU, EXT>(routed, shared, !few, s);
     }
-    const int rc = launch_rows_as<SILU, EXT>(routed, lds_bytes, s);
-    return rc ? rc : launch_rows_as<SILU, EXT>(shared, lds_bytes, s);
+    if (a.R >= kSplitSharedRows || (a.R == 0 && block_rows(shared))) {
+      const int rc = a.R ? launch_rows_as<SILU, EXT>(routed, lds_bytes, s) : 0;
+      return rc ? rc : launch_rows_as<SILU, EXT>(shared, lds_bytes, s);
+    }
   }
   const int nmax = a.plan.n > a.plan_shared.n ? a.plan.n : a.plan_shared.n;
   int dev = 0, cus = 256;
@@ -1669,6 +1990,15 @@ static int launch_rows_as(const RowArgs& a, int lds_bytes, hipStream_t s) {
       return 4;
     }
     return 0;
+  }
+  if (block_rows(a) && (!dense_rows(a) || a.rows <= kBlockRowsMax) && !wide_rows(a)) {
+    const int blds = BlockRows(a.plan).lds();
+    switch ((n / 8 + 255) / 256) {
+      case 1: hipLaunchKernelGGL((row_quant_block_kernel<1, SILU, EXT>), dim3(grid), dim3(256), blds, s, a); break;
+      case 2: hipLaunchKernelGGL((row_quant_block_kernel<2, SILU, EXT>), dim3(grid), dim3(256), blds, s, a); break;
+      default: hipLaunchKernelGGL((row_quant_block_kernel<3, SILU, EXT>), dim3(grid), dim3(256), blds, s, a); break;
+    }
+    return rows_launched();
   }
   // table-driven factor times H_8, one size of row: one row per wave, dense stage on the matrix cores
   if (dense_rows(a)) {

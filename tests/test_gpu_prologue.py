@@ -216,6 +216,70 @@ def test_silu_mul_then_quant_bit_exact(n, n_sh, rotate):
         p += 1
 
 
+def _check_rows(got, scales, y, q, what):
+    """Rows `y` of one expert (rotated where they have to be) against what a quantiser wrote for format `q`, bit for bit."""
+    tag = O.act_tag(q[0], q[2])
+    if tag == 0:
+        assert np.array_equal(got.cpu().numpy().view(np.uint16), y.view(np.uint16)), what
+        return
+    codes, s, _ = O.quant_minmax(y, q[0], 128 if tag == 3 else -1, True)
+    assert np.array_equal(scales.cpu().numpy().view(np.uint16), s.reshape(-1).view(np.uint16)), (what, "scales")
+    assert np.array_equal(_unpack(got, tag, y.shape[1]), codes.astype(np.int8)), (what, "codes")
+
+
+# routed and shared rows of two lengths: up to 512 routed rows one row of either kind per workgroup, beyond the shared ones beside one routed row per wave
+# (300 shared rows: more than their workgroups); orders 4 x 44, 2 x 20 and 28, one and two k steps of 32, k rows of 16, 32, 64 and 128 values
+@pytest.mark.parametrize("n,n_sh,t,rotate", [(1408, 2, 40, 1), (1408, 4, 256, 2), (1408, 4, 300, 1), (1408, 2, 300, 2), (224, 2, 33, 1), (224, 8, 300, 1), (224, 16, 20, 2), (320, 4, 33, 1)])
+def test_rows_of_two_lengths_bit_exact(n, n_sh, t, rotate):
+    from mxmoe_amd import ops
+
+    rng = np.random.default_rng(n + n_sh + t)
+    e, topk = 4, 2
+    ids = _ids(rng, t, e, topk)
+    o_dst, _, _, o_recv = O.permute_by_expert(ids, e)
+    gu = (rng.standard_normal((t * topk, 2 * n)) * 2).astype(F16)
+    gu_sh = (rng.standard_normal((t, 2 * n * n_sh)) * 2).astype(F16)
+    gu_sh[1] = 0
+    for last in ((4, 4, -1, True), (8, 8, -1, True)):
+        qp = [(4, 4, -1, True), (8, 8, -1, True), (16, 4, 128, False), (8, 8, -1, True) if n % 128 else (4, 4, 128, True), last]
+        inp, sc = ops.silu_mul_then_quant(torch.from_numpy(np.concatenate([gu.reshape(-1), gu_sh.reshape(-1)])).to(DEV), int((o_recv != 0).sum()), e, 2048, n, n_sh, t, topk,
+                                          torch.from_numpy(o_dst).to(DEV), torch.from_numpy(o_recv), qp, rotate=rotate)[:2]
+        torch.cuda.synchronize()
+        p = st = 0
+        for ex in range(e + 1):
+            m = t if ex == e else int(o_recv[ex])
+            if m == 0:
+                continue
+            y = O.silu_mul(gu_sh if ex == e else gu[st:st + m])
+            st += m if ex < e else 0
+            _check_rows(inp[p], sc[p], O.online_hadamard(y) if rotate == 2 or O.act_tag(qp[ex][0], qp[ex][2]) else y, qp[ex], (ex, last))
+            p += 1
+
+
+# one length, one row per workgroup: more rows than workgroups (2048), two and three chunks per thread, two orders
+@pytest.mark.parametrize("k,t", [(448, 1100), (2816, 20), (5632, 9), (3584, 9), (448, 3)])
+def test_rows_by_workgroups_bit_exact(k, t):
+    from mxmoe_amd import ops
+
+    rng = np.random.default_rng(k + t)
+    e = 3
+    x = rng.standard_normal((t, k)).astype(F16)
+    ids = _ids(rng, t, e, 1)
+    qp = [(4, 4, -1, True), (8, 8, -1, True), (16, 16, -1, True), (4, 4, -1, True)]
+    inp, sc = ops.quant_inp_act(torch.from_numpy(x).to(DEV), torch.from_numpy(ids).to(DEV), e, 256, 1, qp, rotate=1)[:2]
+    torch.cuda.synchronize()
+    _, o_perm, _, o_recv = O.permute_by_expert(ids, e)
+    p = st = 0
+    for ex in range(e + 1):
+        m = t if ex == e else int(o_recv[ex])
+        if m == 0:
+            continue
+        rows = x if ex == e else x[o_perm[st:st + m]]
+        st += m if ex < e else 0
+        _check_rows(inp[p], sc[p], O.online_hadamard(rows) if qp[ex][0] < 16 else rows, qp[ex], ex)
+        p += 1
+
+
 def _bf6_rows(view, m, k):
     """Codes of the m rows of an expert whose activations were written as bf6 fragments (tag 4)."""
     from mxmoe_amd import pack
