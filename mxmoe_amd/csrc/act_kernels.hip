@@ -2186,7 +2186,7 @@ static int launch_combine(CombineArgs a, const float* weights, const int32_t* ro
 
 // Bytes that travel in the kernel arguments.
 struct UploadArgs {
-  static constexpr int kWords = 896;
+  static constexpr int kWords = 1008;  // (4 KiB of kernel arguments: the tables of a launch over 67 problems, at 60 bytes each, go in one)
   uint32_t* dst;
   int words;
   uint32_t w[kWords];

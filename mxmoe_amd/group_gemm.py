@@ -7,6 +7,8 @@ every launch (the reference re-allocates and re-copies them on every call, ref_b
 from __future__ import annotations
 
 import ctypes as C
+import struct
+from array import array
 from functools import lru_cache
 
 import numpy as np
@@ -16,9 +18,15 @@ from . import _lib
 from .weights import PackedWeight  # noqa: F401  (re-export for callers)
 
 
-@lru_cache(maxsize=64)
-def _qparams_array(qparams: tuple) -> np.ndarray:
-    return np.array([(int(a), int(w), int(g), 1 if s else 0) for (a, w, g, s) in qparams], np.int32)
+@lru_cache(maxsize=256)
+def _qparams_bytes(q: tuple) -> bytes:
+    a, w, g, s = q
+    return struct.pack("=4i", int(a), int(w), int(g), 1 if s else 0)  # (a_bits, w_bits, gsize, sym byte): the QParams layout
+
+
+@lru_cache(maxsize=256)
+def _array_types(p: int):
+    return _lib.Dim3 * p, _lib.QParams * p
 
 
 def _upload(host: np.ndarray, device) -> torch.Tensor:
@@ -43,25 +51,36 @@ class GroupGemmLaunch:
         dev = Cs[0].device if p else torch.device("cuda")
 
         # host tables as arrays: the six pointer rows and the sizes go to the device as one block, sizes and QParams also stay for the launcher
-        block = np.zeros(6 * p * 8 + p * 12 + 12, np.uint8)
-        table = block[:6 * p * 8].view(np.int64).reshape(6, p)
-        for row, ts in zip(table, (As, Bs, scale_a, scale_b, Cs, acc)):
-            if ts:
-                if len(ts) != p:  # (numpy would spread a list of one over all problems)
-                    raise ValueError(f"a list of {len(ts)} tensors for {p} problems")
-                row[:] = [0 if t is None else t.data_ptr() for t in ts]  # (0 for a tensor without elements)
+        # (one conversion of all pointers, not one per row, and QParams as bytes)
+        block = np.empty(6 * p * 8 + p * 12 + 12, np.uint8)
+        ptrs = []
+        for ts in (As, Bs, scale_a, scale_b, Cs, acc):
+            if not ts:
+                ptrs += [0] * p
+                continue
+            if len(ts) != p:
+                raise ValueError(f"a list of {len(ts)} tensors for {p} problems")
+            ptrs += [0 if t is None else t.data_ptr() for t in ts]  # (0 for a tensor without elements)
+        if p:
+            block[:6 * p * 8] = np.frombuffer(array("q", ptrs), np.uint8)
+        block[6 * p * 8 + p * 12:] = 0
         h_sizes = block[6 * p * 8:6 * p * 8 + p * 12].view(np.uint32).reshape(p, 3)
         h_sizes[:] = (sizes if isinstance(sizes, np.ndarray) else np.array(sizes, np.int32)).reshape(p, 3)
-        h_q = np.zeros((max(p, 1), 4), np.int32)                        # (a_bits, w_bits, gsize, sym byte): the QParams layout
-        if p:
-            h_q[:p] = _qparams_array(tuple(map(tuple, qparams)))
-        self.h_sizes = (_lib.Dim3 * max(p, 1)).from_buffer(block, 6 * p * 8)
-        self.h_q = (_lib.QParams * max(p, 1)).from_buffer(h_q)
+        sizes_t, qparams_t = _array_types(max(p, 1))
+        self.h_sizes = sizes_t.from_buffer(block, 6 * p * 8)
+        self.h_q = qparams_t.from_buffer_copy(b"".join([_qparams_bytes(q if type(q) is tuple else tuple(q)) for q in qparams]) or bytes(16))
         self.d_block = _upload(block, dev)
         self._base = self.d_block.data_ptr()
         self.has_acc = acc is not None
-        self.sizes = [tuple(s) for s in h_sizes.tolist()]
-        self.ops = int(2 * h_sizes.astype(np.int64).prod(axis=1).sum())
+        self._host_sizes = h_sizes
+
+    @property
+    def sizes(self) -> list:
+        return [tuple(s) for s in self._host_sizes.tolist()]
+
+    @property
+    def ops(self) -> int:
+        return int(2 * self._host_sizes.astype(np.int64).prod(axis=1).sum())
 
     def _ptr(self, row: int) -> int:
         return self._base + row * self.count * 8

@@ -208,14 +208,15 @@ def _offsets(recv_cpu, num_tokens: int, num_experts: int, has_shared: bool, qpar
 
 
 def _row_views(store, offsets, sizes, lds):
-    """One [-1, ld] view per (offset, elements, ld), back to back from the start of `store`.  Experts of one row length (the usual case)
-    are cut by a single call."""
+    """One [-1, ld] view per (offset, elements, ld), back to back from the start of `store`, cut by a single call as rows of the shortest length;
+    the others, where it divides theirs (int4 next to int8 rows), are those rows taken together."""
     if not lds:
         return []
-    ld, total = lds[0], offsets[-1] + sizes[-1]
-    if lds.count(ld) == len(lds):
-        return list((store if store.numel() == total else store[:total]).view(-1, ld).split_with_sizes([s // ld for s in sizes]))
-    return [store.as_strided((s // w, w), (w, 1), o) for o, s, w in zip(offsets, sizes, lds)]
+    ld, total = min(lds), offsets[-1] + sizes[-1]
+    if any(w % ld for w in set(lds)):
+        return [store.as_strided((s // w, w), (w, 1), o) for o, s, w in zip(offsets, sizes, lds)]
+    cut = (store if store.numel() == total else store[:total]).view(-1, ld).split_with_sizes([s // ld for s in sizes])
+    return [v if w == ld else v.view(-1, w) for v, w in zip(cut, lds)]
 
 
 def _views(store, scale_store, table, rows, inp_sizes, scale_sizes, lds):
@@ -223,7 +224,7 @@ def _views(store, scale_store, table, rows, inp_sizes, scale_sizes, lds):
     live = [e for e, n in enumerate(rows) if n]
     if not live:
         return [], []
-    inp_off = table[2].tolist()
+    inp_off = (table if isinstance(table, np.ndarray) else table.numpy())[2].tolist()
     inp_list = _row_views(store, [inp_off[e] for e in live], [inp_sizes[e] for e in live], [lds[e] for e in live])
     sizes = [scale_sizes[e] for e in live]
     total = sum(sizes)
@@ -255,14 +256,16 @@ def quant_inp_act(hidden, topk_ids, num_experts: int, N: int, num_shared_experts
     per_token = per_token_prologue(k, topk) and not (bf6 or fp8)
     dst, perm, _slot, recv, *inv = build_permutation(topk_ids, num_experts, with_inverse=per_token)
     recv_cpu = recv.cpu()                                   # one small D2H copy, as ref_bind.cu:451
-    table, rows, inp_sizes, scale_sizes, lds, io, so = _offsets(recv_cpu, t, num_experts, has_shared, qparams_per_exp, k, k, bf6, fp8)
+    counts = _rows_of(recv_cpu, t, num_experts, has_shared)
+    table, inp_sizes, scale_sizes, lds = _offset_arrays(counts, num_experts, qparams_per_exp, k, k, bf6, fp8)
+    io, so = int(inp_sizes.sum()), int(scale_sizes.sum())
     dev = hidden.device
     inp_store = torch.empty(io, dtype=torch.float16, device=dev)
     scale_store = torch.empty(so, dtype=torch.float16, device=dev)
     out_store = torch.empty((num_shared_experts + topk) * t * N * 2, dtype=torch.float16, device=dev)
-    d_table = _upload(table.numpy(), dev)
+    d_table = _upload(table, dev)
     hk, hf, signs = device_signs(k, dev) if rotate else (1, 1, None)
-    routed = int(recv_cpu.sum())                            # rows whose expert id was in range; the sorted arrays hold exactly these
+    routed = int(counts[:num_experts].sum())                # rows whose expert id was in range; the sorted arrays hold exactly these
     if per_token:
         ids32 = topk_ids.to(torch.int32).contiguous()
         _lib.check(lib, lib.mxmoe_quant_act_tokens(hidden.data_ptr(), inp_store.data_ptr(), scale_store.data_ptr(), ids32.data_ptr(), inv[0].data_ptr(), d_table.data_ptr(),
@@ -271,7 +274,8 @@ def quant_inp_act(hidden, topk_ids, num_experts: int, N: int, num_shared_experts
         _lib.check(lib, lib.mxmoe_quant_act(hidden.data_ptr(), inp_store.data_ptr(), scale_store.data_ptr(), dst.data_ptr(), perm.data_ptr(), d_table.data_ptr(),
                                             k, routed, t, num_experts, int(has_shared), rotate | (ROWS_VARIANTS if bf6 or fp8 else 0), hk, hf,
                                             None if signs is None else signs.data_ptr(), _stream()))
-    inp_list, scale_list = _views(inp_store, scale_store, table, rows, inp_sizes, scale_sizes, lds)
+    rows, inp_sizes, scale_sizes = counts.tolist(), inp_sizes.tolist(), scale_sizes.tolist()
+    inp_list, scale_list = _views(inp_store, scale_store, table, rows, inp_sizes, scale_sizes, lds.tolist())
     out_list = _out_views(out_store, rows, N * 2, N * 2 * num_shared_experts, num_experts)
     if verbose:
         for e, n in enumerate(rows):
@@ -287,13 +291,14 @@ def silu_mul_then_quant(inp, num_problems: int, num_experts: int, K: int, N: int
     lib = _lib.load()
     has_shared = num_shared_experts > 0
     dev = inp.device
-    recv_cpu = recv_tokens_per_exp.cpu()
-    r = int(recv_cpu.sum())                                 # routed rows in the store (ids out of range were dropped by the permutation)
-    table, rows, inp_sizes, scale_sizes, lds, io, so = _offsets(recv_cpu, num_tokens, num_experts, has_shared, qparams_per_exp, N, N * max(num_shared_experts, 1), bf6, fp8)
+    counts = _rows_of(recv_tokens_per_exp.cpu(), num_tokens, num_experts, has_shared)
+    r = int(counts[:num_experts].sum())                     # routed rows in the store (ids out of range were dropped by the permutation)
+    table, inp_sizes, scale_sizes, lds = _offset_arrays(counts, num_experts, qparams_per_exp, N, N * max(num_shared_experts, 1), bf6, fp8)
+    io, so = int(inp_sizes.sum()), int(scale_sizes.sum())
     inp_store = torch.empty(io, dtype=torch.float16, device=dev)
     scale_store = torch.empty(so, dtype=torch.float16, device=dev)
     out_store = torch.empty((1 + topk) * num_tokens * K, dtype=torch.float16, device=dev)
-    d_table = _upload(table.numpy(), dev)
+    d_table = _upload(table, dev)
     flat = inp.reshape(-1)
     n_sh = N * num_shared_experts
     hk, hf, signs = device_signs(N, dev) if rotate else (1, 1, None)
@@ -302,7 +307,8 @@ def silu_mul_then_quant(inp, num_problems: int, num_experts: int, K: int, N: int
     shared_ptr = flat.data_ptr() + r * N * 2 * 2
     _lib.check(lib, lib.mxmoe_silu_mul_quant(flat.data_ptr(), shared_ptr, inp_store.data_ptr(), scale_store.data_ptr(), values_sorted.data_ptr(), d_table.data_ptr(),
                                              N, n_sh, r, num_tokens, num_experts, int(has_shared), rotate | (ROWS_VARIANTS if bf6 or fp8 else 0), hk, hf, None if signs is None else signs.data_ptr(), _stream()))
-    inp_list, scale_list = _views(inp_store, scale_store, table, rows, inp_sizes, scale_sizes, lds)
+    rows = counts.tolist()
+    inp_list, scale_list = _views(inp_store, scale_store, table, rows, inp_sizes.tolist(), scale_sizes.tolist(), lds.tolist())
     out_list = _out_views(out_store, rows, K, K, num_experts)
     return inp_list, scale_list, out_list, inp_store, scale_store, out_store
 
