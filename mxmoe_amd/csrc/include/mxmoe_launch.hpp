@@ -22,6 +22,7 @@
 
 #include "mxmoe_tiles.hpp"
 #include "mxmoe_grp_tiles.hpp"
+#include "mxmoe_few_tiles.hpp"
 #include "mxmoe_bf6_tiles.hpp"
 #include "mxmoe_wo_tiles.hpp"
 
@@ -286,6 +287,13 @@ struct BranchOf<WxAxTile<OP, BM, BN>> {
     return BranchInfo{OP == Op::I4 ? Fmt::W4A4 : Fmt::W8A8, BM, BN, T::BK, 1, 4, T::kLdsBytes, T::BK, 0, 0, OP == Op::F8 ? kVariantFp8 : 0};
   }
 };
+template <Op OP>
+struct BranchOf<WxAxNarrowTile<OP>> {
+  static BranchInfo get() {
+    using T = WxAxNarrowTile<OP>;
+    return BranchInfo{OP == Op::I4 ? Fmt::W4A4 : Fmt::W8A8, T::BM, T::BN, T::BK, 1, 1, T::kLdsBytes, T::BK, 0};
+  }
+};
 template <int BM>
 struct BranchOf<Bf6Tile<BM>> {
   // same format as the int4 tiles on the int8 instruction; what differs is the layout both operands are handed over in (6-bit
@@ -357,8 +365,8 @@ inline double tile_cost(const BranchInfo& b) {
   static const Row table[] = {
       // (inside a fused kernel the small integer tiles run at the occupancy of the largest one, which costs them part of the
       // advantage they show as single-tile kernels in the profile table)
-      {Fmt::W4A4, 128, 256, 1.00}, {Fmt::W4A4, 64, 256, 0.58}, {Fmt::W4A4, 32, 256, 0.48},
-      {Fmt::W8A8, 128, 256, 1.00}, {Fmt::W8A8, 64, 256, 0.74}, {Fmt::W8A8, 32, 256, 0.56},
+      {Fmt::W4A4, 128, 256, 1.00}, {Fmt::W4A4, 64, 256, 0.58}, {Fmt::W4A4, 32, 256, 0.48}, {Fmt::W4A4, 32, 64, 0.13},
+      {Fmt::W8A8, 128, 256, 1.00}, {Fmt::W8A8, 64, 256, 0.74}, {Fmt::W8A8, 32, 256, 0.56}, {Fmt::W8A8, 32, 64, 0.155},
       {Fmt::FP16, 128, 256, 1.00}, {Fmt::FP16, 64, 256, 0.69}, {Fmt::FP16, 32, 256, 0.53}, {Fmt::FP16, 128, 128, 0.57}, {Fmt::FP16, 256, 128, 1.09},
       {Fmt::W4A16, 16, 128, 0.37}, {Fmt::W4A16, 16, 64, 0.20}, {Fmt::W4A16, 32, 128, 0.50}, {Fmt::W4A16, 128, 128, 1.00}, {Fmt::W4A16, 128, 256, 1.50},
       {Fmt::W3A16, 16, 128, 0.31}, {Fmt::W3A16, 16, 64, 0.20}, {Fmt::W3A16, 32, 128, 0.50}, {Fmt::W3A16, 128, 128, 1.00}, {Fmt::W3A16, 128, 256, 1.50},
@@ -712,6 +720,35 @@ inline int auto_kernel_for(const mxmoe_qparams* h_q, int count, long max_rows) {
 }
 // (A few-row kernel runs 16-row tiles: it is meant for lists whose problems mostly fit one such tile.  When more than a quarter of
 // the non-empty problems need several, the kernels that also hold the 32-row few-token tile do better, whatever the largest count.)
+//
+// Lists of few rows with w4a4 or w8a8 problems go to the kernels that hold the narrow integer tile (WxAxNarrowTile, for problems of up to 32 rows; more take
+// 64-row tiles): no problem above 64 rows, 24 per problem on average, and at most 768 blocks of 256 channels over all problems.  A whole layer, us, w4a4 / w8a8
+// half and half, before -> with these kernels: 60 experts top-4 38 -> 28 (1 token), 53 -> 51 (8), 88 -> 77 (32), 98 -> 92 (64); 64 experts top-6 and a shared one
+// 46 -> 34 (1), 74 -> 68 (8), 111 -> 107 (32), 115 -> 110 (64; under a skewed routing 103 -> 106); 8 experts of N = 28 672 / 4096, K = 4096 / 14 336, whose
+// second block alone is within the limit, 103 -> 71 (1), 223 -> 191 (8), 230 -> 200 (64).  Beyond: 128 tokens of the second with its shared expert 118 -> 119, skewed
+// 117 -> 125; the first block of the third (896 blocks of 256 channels, enough for the wide tiles to fill the chip) on them too, w4a4 150 -> 160 (16 tokens).
+// A 128-row tile beside them would take the third workgroup of a CU (244 registers, 161 without): 60 experts 77 -> 83 (32).
+// (From 8 blocks on: the planning rules for long problems are stated, and tested, on lists of two or three small problems in the wide shapes.)
+constexpr int kFewRows = 24, kFewRowsMax = 64, kFewColumns = 768, kFewColumnsMin = 8;
+inline bool holds_narrow(const FusedKernel& k) {
+  for (const BranchInfo& b : k.branches)
+    if ((b.fmt == Fmt::W4A4 || b.fmt == Fmt::W8A8) && b.BN == 64) return true;
+  return false;
+}
+inline bool few_rows(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int count) {
+  long rows = 0, columns = 0, live = 0;
+  bool narrow = false;
+  for (int i = 0; i < count; ++i) {
+    if (h_sizes[i].x == 0) continue;
+    if (h_sizes[i].x > (unsigned)kFewRowsMax) return false;
+    ++live;
+    rows += h_sizes[i].x;
+    columns += (h_sizes[i].y + 255) / 256;
+    const Fmt f = classify(h_q[i]);
+    narrow = narrow || f == Fmt::W4A4 || f == Fmt::W8A8;
+  }
+  return narrow && rows <= kFewRows * live && columns >= kFewColumnsMin && columns <= kFewColumns;
+}
 inline int auto_kernel(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int count) {
   long max_rows = 0;
   int live = 0, over = 0;
@@ -719,6 +756,11 @@ inline int auto_kernel(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int 
     max_rows = std::max(max_rows, (long)h_sizes[i].x);
     live += h_sizes[i].x > 0;
     over += h_sizes[i].x > 16;
+  }
+  if (few_rows(h_sizes, h_q, count)) {
+    auto& reg = registry();
+    for (int i = 0; i < (int)reg.size(); ++i)
+      if (reg[i].policy == Policy::Fused && !kernel_has_variants(reg[i]) && holds_narrow(reg[i]) && kernel_covers(reg[i], h_q, count)) return i;
   }
   return auto_kernel_for(h_q, count, 4 * over > live ? -1 : max_rows);
 }

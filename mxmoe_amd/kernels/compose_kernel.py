@@ -26,7 +26,7 @@ from pathlib import Path
 
 from .. import build as _build
 from .kernel_sketch import ABI_TU, DEFAULT_ORDER_TEMPLATE, KERNEL_DECLARATION_TEMPLATE, KERNEL_DEFERRED_TEMPLATE, KERNEL_DEFINITION_TEMPLATE
-from .tile_config import QCFG_MAP, SUPPORTED_QCFG, TileConfig, get_gpu_info, get_info_from_qcfg_str, get_possible_tile_list  # noqa: F401
+from .tile_config import QCFG_MAP, SUPPORTED_QCFG, TileConfig, get_gpu_info, get_info_from_qcfg_str, get_possible_tile_list, narrow_tile  # noqa: F401
 
 
 class KernelType(str, enum.Enum):
@@ -202,6 +202,10 @@ def default_kernel_specs(arch: str = "gfx950"):
         ("groupgemm_hz_fused_wxax_b6", KernelType.Fused, OrderedDict([(w4, _pick(arch, w4, (128, 256), (64, 256), (32, 256), bf6=True)), (w8, _pick(arch, w8, (128, 256), (64, 256), (32, 256)))])),
         ("groupgemm_hz_fused_all_b6", KernelType.Fused, everything_b6),
         ("groupgemm_hz_fused_all_e4m3", KernelType.Fused, everything_e4m3),
+        # launches with few workgroups (decode batches on a few experts), asked for by name: narrow integer tiles, alone and next to the few-token weight-only ones
+        ("groupgemm_hz_fused_wxax_few", KernelType.Fused, OrderedDict((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8))),
+        ("groupgemm_hz_fused_all_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8)), *wo_all.items(),
+                                                                       ("w8a16_g128_asym", _pick(arch, "w8a16_g128_asym", (16, 128), (32, 128), (128, 128)))])),
         # bfloat16 operands and outputs (the reference's "bf16"): the QParams of fp16 problems, so by name only
         ("groupgemm_hz_fused_bf16", KernelType.Fused, OrderedDict([("bf16", _pick(arch, "bf16", (128, 256), (64, 256), (32, 256)))])),
     ]

@@ -190,6 +190,10 @@ class TileConfig:
         """int4 operands handed over as bf6 fragments (both activations and weights; the quantisers write them, tag 4)."""
         return self.MMA == BF6_MMA
 
+    def is_narrow(self) -> bool:
+        """Integer tile of 32 tokens x 64 channels whose four waves share K (few-workgroup launches)."""
+        return self.WK == 4 and self.BN == 64
+
     def is_group_wa(self) -> bool:
         """Both operands int4 with a scale per 128-wide K group (w4a4_g128_sym)."""
         return self.MMA == "MFMA_I32_32x32x32_I8_FROM_I4" and getattr(self.QCFGA, "GSIZE", -1) == 128
@@ -204,6 +208,8 @@ class TileConfig:
             return 4 * (self.BN // 16) * (64 * 16 * (self.BM // 16) + kp * 64)
         if self.is_weight_only():
             return 2 * self.BM * 256  # two stages of BM activation rows x one 128-wide k block
+        if self.is_narrow():
+            return 4 * 2 * 4 * 64 * 16  # the waves' partial sums
         if self.is_group_wa():
             return self.STAGE * self.BM * 64
         if self.is_bf6():  # four stages of the tile's token fragments (1536 bytes per 32 rows, rounded up to 1 KB pieces), or the epilogue patch
@@ -224,6 +230,8 @@ class TileConfig:
         if self.is_bf6():
             return f"Bf6Tile<{self.BM}>"
         op = {"MFMA_F32_32x32x16_F16": "Op::F16", "MFMA_F32_32x32x16_BF16": "Op::BF16", "MFMA_I32_32x32x32_I8": "Op::I8", "MFMA_I32_32x32x32_I8_FROM_I4": "Op::I4", "MFMA_F32_32x32x16_FP8": "Op::F8"}[self.MMA]
+        if self.is_narrow():
+            return f"WxAxNarrowTile<{op}>"
         if self.is_group_wa():
             return f"WxAxGTile<{self.BM}>"
         if op not in ("Op::F16", "Op::BF16"):
@@ -242,6 +250,10 @@ class TileConfig:
                 raise ValueError(f"{self!r}: bf6 tiles are BM x 256 x 64 with 1 x 4 waves and 4 stages, BM in 32 / 64 / 128")
             return
         k_elems = {"MFMA_F32_32x32x16_F16": 32, "MFMA_F32_32x32x16_BF16": 32, "MFMA_I32_32x32x32_I8": 64, "MFMA_I32_32x32x32_I8_FROM_I4": 128, "MFMA_F32_32x32x16_FP8": 64}[self.MMA]
+        if self.is_narrow() and self.MMA in ("MFMA_I32_32x32x32_I8", "MFMA_I32_32x32x32_I8_FROM_I4") and not self.is_group_wa():
+            if (self.BM, self.WM, self.WN, self.BK) != (32, 1, 1, k_elems):
+                raise ValueError(f"{self!r}: tiles whose waves share K are 32 x 64 x {k_elems}")
+            return
         if self.BK != k_elems or self.STAGE != 3 or self.WK != 1 or (self.BM // self.WM) % 32 or (self.BN // self.WN) % 32:
             raise ValueError(f"{self!r}: unsupported shape for {self.MMA} (BK must be {k_elems}, STAGE 3, wave tile a multiple of 32x32)")
         if self.is_group_wa() and self.BM not in (32, 64):
@@ -306,6 +318,11 @@ def get_possible_tile_list(arch: str, qcfg: str) -> list:
     if qcfg == "w4a4_g-1_sym":  # the same shapes on the 6-bit float path (operands as bf6 fragments): never mixed with the tiles above in one kernel
         tiles += [_with_q(TileConfig(BM=bm, BN=256, BK=64, WM=1, WN=4, WK=1, STAGE=4, MMA=BF6_MMA), qcfg) for bm in (128, 64, 32)]
     return tiles
+
+
+def narrow_tile(qcfg: str) -> TileConfig:
+    """The w4a4 / w8a8 tile for launches with few workgroups (not among the candidates of get_possible_tile_list: its kernels are chosen by launch)."""
+    return _with_q(TileConfig(BM=32, BN=64, BK=128 if qcfg == "w4a4_g-1_sym" else 64, WM=1, WN=1, WK=4, STAGE=3, MMA=QCFG_TO_MMA[qcfg]), qcfg)
 
 
 _FIELD = re.compile(r"(BM|BN|BK|WM|WN|WK|STAGE|SPLITK)=(-?\d+)")

@@ -151,6 +151,16 @@ class MxMoELayer:
             few = lib.mxmoe_find_kernel(b"groupgemm_hz_fused_wo_skinny")
             if few >= 0 and lib.mxmoe_plan_select_kernel(few, h, et) == few:
                 kid = few
+        if t <= 64 and any(d.a_bits < 16 for d in h):
+            # the launcher's rule for lists of few rows (mxmoe_launch.hpp, few_rows), with the experts that may have any
+            e_cnt, shared = self.cfg.num_experts, self.cfg.num_shared > 0
+            live = min(e_cnt, t * topk)
+            cols = sorted((-(-int(d.N) // 256) for d in h[:e_cnt]), reverse=True)
+            if t * topk + t * shared <= 24 * (live + shared) and 8 <= sum(cols[:live]) + shared * -(-int(h[et - 1].N) // 256) <= 768:
+                for name in (b"groupgemm_hz_fused_wxax_few", b"groupgemm_hz_fused_all_few"):
+                    few = lib.mxmoe_find_kernel(name)
+                    if few >= 0 and lib.mxmoe_plan_select_kernel(few, h, et) == few:
+                        return few
         return kid
 
     def _planned_setup(self, t: int, topk: int):

@@ -314,3 +314,32 @@ def test_layer_run_wants_aligned_tokens_where_tiles_read_them_in_place(lib, a_bi
         assert lib.mxmoe_layer_run(handle, None, some, some, some, None) == 5
     finally:
         lib.mxmoe_layer_destroy(handle)
+
+
+def test_lists_of_few_rows_take_the_kernels_with_narrow_tiles():
+    """Up to 64 rows per problem, 24 on average and 768 blocks of 256 channels: on and past each limit; formats those kernels have no tile for; empty problems
+    count for nothing."""
+    from mxmoe_amd import _lib
+
+    lib = _lib.load()
+    w4, w8, wo, fp = (4, 4, -1, True), (8, 8, -1, True), (16, 4, 128, False), (16, 16, -1, True)
+
+    def picked(*probs):
+        sizes = (_lib.Dim3 * len(probs))(*[_lib.Dim3(m, n, 2048) for m, n, _ in probs])
+        qs = (_lib.QParams * len(probs))(*[_lib.QParams(q[0], q[1], q[2], int(q[3])) for *_, q in probs])
+        rc = lib.mxmoe_group_gemm_plan(-1, sizes, qs, len(probs), None, None)
+        assert rc >= 1000, lib.mxmoe_last_error()
+        return lib.mxmoe_kernel_name(rc - 1000).decode().split("groupgemm_")[-1]
+
+    few = [(5, 2816, w4), (1, 2816, w8)]
+    assert picked(*few) == "hz_fused_wxax_few"
+    assert picked(*few, (3, 2816, wo)) == "hz_fused_all_few"
+    assert picked(*few, (0, 2816, fp)) != "hz_fused_wxax_few"          # (its format still has to be covered)
+    assert picked(*few, (3, 2816, fp)) == "hz_fused_all"
+    assert picked((3, 2816, wo), (2, 2816, wo)) == "hz_fused_wo_skinny"
+    assert picked((64, 2816, w4), (1, 2816, w8), (7, 2816, w8)) == "hz_fused_wxax_few"
+    assert picked((65, 2816, w4), *[(1, 2816, w8)] * 9) == "hz_fused_wxax"
+    assert picked((24, 2816, w4), (24, 2816, w8)) == "hz_fused_wxax_few"
+    assert picked((24, 2816, w4), (25, 2816, w8)) == "hz_fused_wxax"
+    assert picked(*[(1, 256, w4)] * 7) == "hz_fused_wxax" and picked(*[(1, 256, w4)] * 8) == "hz_fused_wxax_few"
+    assert picked(*[(1, 2048, w4)] * 96) == "hz_fused_wxax_few" and picked(*[(1, 2048, w4)] * 97) == "hz_fused_wxax"

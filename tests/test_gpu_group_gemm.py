@@ -289,6 +289,24 @@ def test_bf16_group_gemm():
     assert np.array_equal(got.view(np.uint32), exact.view(np.uint32))
 
 
+@pytest.mark.parametrize("kernel", ["groupgemm_hz_fused_wxax_few", "groupgemm_hz_fused_all_few"])
+def test_narrow_integer_tiles_bit_exact(kernel):
+    """32 x 64 tiles whose waves share K: accumulators and outputs bit for bit; K of fewer slices than waves, of a slice more than the waves' loads in flight cover
+    and of many, rows past one tile, channel counts that end inside a block and inside a tile."""
+    from mxmoe_amd import _lib
+
+    rng = np.random.default_rng(77)
+    shapes = [(1, 64, 128, 4), (31, 72, 128, 8), (32, 144, 256, 4), (33, 256, 1408, 4), (2, 200, 64, 8), (17, 320, 1408, 8), (70, 128, 2048, 8),
+              (5, 2816, 2048, 4), (3, 64, 14336, 8), (16, 96, 14336, 4), (1, 128, 2176, 4), (4, 128, 1088, 8)]
+    probs = [_wxax_problem(rng, m, n, k, b) for (m, n, k, b) in shapes]
+    kid = _lib.load().mxmoe_find_kernel(kernel.encode())
+    assert kid >= 0
+    _, outs, accs = _launch(probs, kernel_id=kid)
+    for p, out, acc in zip(probs, outs, accs):
+        assert np.array_equal(acc, p["acc"]), p["size"]
+        assert np.array_equal(out.view(np.uint16), p["out"].view(np.uint16)), p["size"]
+
+
 def test_weight_only_skinny():
     from mxmoe_amd.weights import quantize_and_pack
 
