@@ -749,11 +749,23 @@ inline bool few_rows(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int co
   }
   return narrow && rows <= kFewRows * live && columns >= kFewColumnsMin && columns <= kFewColumns;
 }
+// The kernel of few-token weight-only tiles of 64 channels, against those of 128: twice the workgroups, 125 registers (four workgroups per CU) against 164.
+// Up to 6 rows per problem on average; the activations, read once per tile, weigh more with more.  A whole layer, us, 128 -> 64 channels: 64 experts top-6 and
+// a shared one, w4a16 / w3a16, 30.2 -> 28.2 (1 token), 42.7 -> 39.2 (4), 64 -> 61 (16), 75 -> 73 (64); 60 experts top-4 and a shared one 33.6 -> 29.0 (1),
+// 58 -> 51 (16); 8 experts of N = 28 672 / 4096 61.6 -> 52.1 (1), 144 -> 140 (16), but 144 -> 150 (32: 8 rows each).
+constexpr int kFewTokenRows = 6;
+inline bool only_narrow_few_token(const FusedKernel& k) {
+  for (const BranchInfo& b : k.branches)
+    if (!is_weight_only(b.fmt) || b.BN != 64) return false;
+  return true;
+}
 inline int auto_kernel(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int count) {
-  long max_rows = 0;
+  long max_rows = 0, rows = 0, columns = 0;
   int live = 0, over = 0;
   for (int i = 0; i < count; ++i) {
     max_rows = std::max(max_rows, (long)h_sizes[i].x);
+    rows += h_sizes[i].x;
+    columns += h_sizes[i].x > 0 ? (h_sizes[i].y + 255) / 256 : 0;
     live += h_sizes[i].x > 0;
     over += h_sizes[i].x > 16;
   }
@@ -762,7 +774,13 @@ inline int auto_kernel(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int 
     for (int i = 0; i < (int)reg.size(); ++i)
       if (reg[i].policy == Policy::Fused && !kernel_has_variants(reg[i]) && holds_narrow(reg[i]) && kernel_covers(reg[i], h_q, count)) return i;
   }
-  return auto_kernel_for(h_q, count, 4 * over > live ? -1 : max_rows);
+  const int kid = auto_kernel_for(h_q, count, 4 * over > live ? -1 : max_rows);
+  if (kid >= 0 && registry()[kid].max_rows_hint > 0 && rows <= kFewTokenRows * live && columns >= kFewColumnsMin) {
+    auto& reg = registry();
+    for (int i = 0; i < (int)reg.size(); ++i)
+      if (reg[i].policy == Policy::Fused && only_narrow_few_token(reg[i]) && kernel_covers(reg[i], h_q, count)) return i;
+  }
+  return kid;
 }
 
 // K a multiple of the tile's K step, N a multiple of 8 (16 for the weight-only layouts)

@@ -202,7 +202,10 @@ def default_kernel_specs(arch: str = "gfx950"):
         ("groupgemm_hz_fused_wxax_b6", KernelType.Fused, OrderedDict([(w4, _pick(arch, w4, (128, 256), (64, 256), (32, 256), bf6=True)), (w8, _pick(arch, w8, (128, 256), (64, 256), (32, 256)))])),
         ("groupgemm_hz_fused_all_b6", KernelType.Fused, everything_b6),
         ("groupgemm_hz_fused_all_e4m3", KernelType.Fused, everything_e4m3),
-        # launches with few workgroups (decode batches on a few experts), asked for by name: narrow integer tiles, alone and next to the few-token weight-only ones
+        # launches with few workgroups (decode batches on a few experts): the few-token tiles of 64 channels; narrow integer tiles, alone and next to the few-token
+        # weight-only ones
+        ("groupgemm_hz_fused_wo_few", KernelType.Fused,
+         OrderedDict((f"w{b}a16_g128_asym", _pick(arch, f"w{b}a16_g128_asym", (16, 64), few_registers=True)) for b in (4, 3, 2))),
         ("groupgemm_hz_fused_wxax_few", KernelType.Fused, OrderedDict((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8))),
         ("groupgemm_hz_fused_all_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8)), *wo_all.items(),
                                                                        ("w8a16_g128_asym", _pick(arch, "w8a16_g128_asym", (16, 128), (32, 128), (128, 128)))])),

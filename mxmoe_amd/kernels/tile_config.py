@@ -302,7 +302,7 @@ def get_possible_tile_list(arch: str, qcfg: str) -> list:
         skinny = [_with_q(TileConfig(BM=16, BN=bn, BK=128, WM=1, WN=4, WK=1, STAGE=2, MMA=mma), qcfg) for bn in (128, 64)]
         skinny.append(_with_q(TileConfig(BM=32, BN=128, BK=128, WM=1, WN=4, WK=1, STAGE=2, MMA=mma), qcfg))  # experts with 17 .. 32 (.. 64) tokens
         if QCFG_MAP[qcfg].QCFGB.QBITS != 8:  # compiled for 3 waves per SIMD, for kernels made of few-token tiles alone (three workgroups per CU)
-            skinny.append(_with_q(TileConfig(BM=16, BN=128, BK=128, WM=1, WN=4, WK=1, STAGE=4, MMA=mma), qcfg))
+            skinny += [_with_q(TileConfig(BM=16, BN=bn, BK=128, WM=1, WN=4, WK=1, STAGE=4, MMA=mma), qcfg) for bn in (128, 64)]
         # (8-bit weights: the ring of packed blocks is twice as large, which leaves room for the 2 x 2 shape's accumulators only)
         shapes = ((128, 2, 2),) if QCFG_MAP[qcfg].QCFGB.QBITS == 8 else ((128, 2, 2), (256, 1, 4))
         big = [_with_q(TileConfig(BM=128, BN=bn, BK=128, WM=wm, WN=wn, WK=1, STAGE=2, MMA=mma), qcfg) for bn, wm, wn in shapes]

@@ -148,7 +148,7 @@ class MxMoELayer:
         if kid < 0:
             raise RuntimeError(lib.mxmoe_last_error().decode())
         if t <= 64 and t * topk <= 12 * self.cfg.num_experts:  # few tokens, and on average well under one 16-row tile per expert: a kernel made of 16-row few-token tiles alone, if one covers the formats
-            few = lib.mxmoe_find_kernel(b"groupgemm_hz_fused_wo_skinny")
+            few = lib.mxmoe_find_kernel(b"groupgemm_hz_fused_wo_few" if t * topk <= 6 * min(self.cfg.num_experts, t * topk) else b"groupgemm_hz_fused_wo_skinny")
             if few >= 0 and lib.mxmoe_plan_select_kernel(few, h, et) == few:
                 kid = few
         if t <= 64 and any(d.a_bits < 16 for d in h):

@@ -336,7 +336,8 @@ def test_lists_of_few_rows_take_the_kernels_with_narrow_tiles():
     assert picked(*few, (3, 2816, wo)) == "hz_fused_all_few"
     assert picked(*few, (0, 2816, fp)) != "hz_fused_wxax_few"          # (its format still has to be covered)
     assert picked(*few, (3, 2816, fp)) == "hz_fused_all"
-    assert picked((3, 2816, wo), (2, 2816, wo)) == "hz_fused_wo_skinny"
+    assert picked((3, 2816, wo), (2, 2816, wo)) == "hz_fused_wo_few"    # (64-channel tiles up to 6 rows on average)
+    assert picked((6, 2816, wo), (6, 2816, wo), (0, 2816, wo)) == "hz_fused_wo_few" and picked((6, 2816, wo), (7, 2816, wo)) == "hz_fused_wo_skinny"
     assert picked((64, 2816, w4), (1, 2816, w8), (7, 2816, w8)) == "hz_fused_wxax_few"
     assert picked((65, 2816, w4), *[(1, 2816, w8)] * 9) == "hz_fused_wxax"
     assert picked((24, 2816, w4), (24, 2816, w8)) == "hz_fused_wxax_few"
