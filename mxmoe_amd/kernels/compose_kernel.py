@@ -202,6 +202,8 @@ def default_kernel_specs(arch: str = "gfx950"):
         ("groupgemm_hz_fused_wxax_b6", KernelType.Fused, OrderedDict([(w4, _pick(arch, w4, (128, 256), (64, 256), (32, 256), bf6=True)), (w8, _pick(arch, w8, (128, 256), (64, 256), (32, 256)))])),
         ("groupgemm_hz_fused_all_b6", KernelType.Fused, everything_b6),
         ("groupgemm_hz_fused_all_e4m3", KernelType.Fused, everything_e4m3),
+        # bfloat16 operands and outputs (the reference's "bf16"): the QParams of fp16 problems, so by name only
+        ("groupgemm_hz_fused_bf16", KernelType.Fused, OrderedDict([("bf16", _pick(arch, "bf16", (128, 256), (64, 256), (32, 256)))])),
         # launches with few workgroups (decode batches on a few experts): the few-token tiles of 64 channels; narrow integer tiles, alone and next to the few-token
         # weight-only ones
         ("groupgemm_hz_fused_wo_few", KernelType.Fused,
@@ -209,8 +211,6 @@ def default_kernel_specs(arch: str = "gfx950"):
         ("groupgemm_hz_fused_wxax_few", KernelType.Fused, OrderedDict((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8))),
         ("groupgemm_hz_fused_all_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8)), *wo_all.items(),
                                                                        ("w8a16_g128_asym", _pick(arch, "w8a16_g128_asym", (16, 128), (32, 128), (128, 128)))])),
-        # bfloat16 operands and outputs (the reference's "bf16"): the QParams of fp16 problems, so by name only
-        ("groupgemm_hz_fused_bf16", KernelType.Fused, OrderedDict([("bf16", _pick(arch, "bf16", (128, 256), (64, 256), (32, 256)))])),
     ]
 
 
