@@ -94,6 +94,13 @@ def sweep_entry(tile: TileConfig, qcfg: str, k: int, waves: int, cus: int = 256)
     return {"shape": [m, n, k], "w_bits": w_bits, "a_bits": a_bits, "gsize": gsize, "sym": sym}
 
 
+def sweep_problem(tile: TileConfig, qcfg: str, k: int, waves: int, cus: int = 256, device: str = "cuda") -> dict:
+    """The operands of that workload, laid out as `tile` reads them (bf6 fragments take more bytes than packed int4 codes; fp8 codes)."""
+    from . import harness
+
+    return harness.make_problem(sweep_entry(tile, qcfg, k, waves, cus), None, device, bf6=tile.is_bf6(), fp8=qcfg.endswith("_E4M3"))
+
+
 def build_qcfg_lib(qcfg: str, arch: str = "gfx950", rebuild: bool = False):
     """One library of single-tile kernels (one per candidate tile of `qcfg`); returns (library path, tiles in kernel order).
     An existing library is reused unless `rebuild`, so it can be compiled on a machine without a GPU beforehand."""
@@ -122,7 +129,7 @@ def profile_qcfg(qcfg: str, arch: str = "gfx950", slots=SLOTS, waves=WAVES, rebu
         for kid, tile in enumerate(tiles):
             ts = []
             for w in waves:
-                prob = harness.make_problem(sweep_entry(tile, qcfg, k, w, cus), None)
+                prob = sweep_problem(tile, qcfg, k, w, cus)
                 launch = harness._launch_of([prob], lib, kid)
                 ts.append(harness.bench_func(launch.run, warmup=5, iters=20)["median"])
                 del prob, launch

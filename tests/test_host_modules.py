@@ -234,6 +234,25 @@ def test_perf_table_alias_and_weight_only_slot():
     assert cost == [[[[0.013920000000000002 * 4]]]]
 
 
+@pytest.mark.parametrize("qcfg", ["w4a4_g-1_sym", "w8a8_g-1_sym_E4M3", "w8a8_g-1_sym"])
+def test_perf_table_operands_have_the_layout_of_their_tile(qcfg):
+    """The operands of a timed single-tile kernel: w4a4 codes packed in half a byte, or as the 1536-byte fragments of 32 rows x 64 values that
+    the 6-bit float tiles read (an int4 store is too short for them); fp8 tiles get e4m3 codes, whose largest is 448."""
+    from mxmoe_amd.kernels.tile_config import get_possible_tile_list
+    from mxmoe_amd.perf_table import sweep_problem
+
+    k = 256
+    for tile in get_possible_tile_list("gfx950", qcfg):
+        p = sweep_problem(tile, qcfg, k, waves=1, cus=8, device="cpu")
+        m, n, _ = p["size"]
+        for name, rows in (("A", m), ("B", n)):
+            size = p[name].numel() * p[name].element_size()
+            assert size == (rows // 32 * (k // 64) * 1536 if tile.is_bf6() else rows * k * tile.a_bits() // 8), (name, tile)
+        if qcfg.endswith("E4M3"):
+            codes = p["A"].view(torch.uint8).view(torch.float8_e4m3fn).float()
+            assert bool((codes.reshape(m, k).abs().amax(dim=1) == 448).all())
+
+
 def test_perf_table_fit_and_sweep_shapes():
     from mxmoe_amd.kernels.tile_config import get_possible_tile_list
     from mxmoe_amd.perf_table import ProblemShape, linear_fit, sweep_entry
