@@ -103,14 +103,15 @@ def sweep_problem(tile: TileConfig, qcfg: str, k: int, waves: int, cus: int = 25
 
 def build_qcfg_lib(qcfg: str, arch: str = "gfx950", rebuild: bool = False):
     """One library of single-tile kernels (one per candidate tile of `qcfg`); returns (library path, tiles in kernel order).
-    An existing library is reused unless `rebuild`, so it can be compiled on a machine without a GPU beforehand."""
+    An existing library is reused unless `rebuild`, so it can be compiled on a machine without a GPU beforehand; its name carries a digest of its
+    kernels, so one of another candidate list is not taken for it (kernel ids would name other tiles)."""
     from .kernels.compose_kernel import GEN_DIR
 
     gen = TemplateGenerator(arch, [qcfg], KernelType.Fused, out_dir=GEN_DIR / f"perf_{qcfg}")  # one qcfg: one single-tile kernel per candidate
     gen.generate_source_code()
-    so = gen.out_dir / f"libmxmoe_{gen.kernel_type}.so"
+    so = gen.library_path()
     if rebuild or not so.exists():
-        gen.build(so)
+        gen.build()
     return so, [next(iter(c.values())) for c in gen.combos]
 
 

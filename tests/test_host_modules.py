@@ -253,6 +253,28 @@ def test_perf_table_operands_have_the_layout_of_their_tile(qcfg):
             assert bool((codes.reshape(m, k).abs().amax(dim=1) == 448).all())
 
 
+def test_perf_table_library_of_another_candidate_list_is_not_reused(tmp_path, monkeypatch):
+    from mxmoe_amd import perf_table as PT
+    from mxmoe_amd.kernels import compose_kernel as CK
+
+    built = []
+
+    def build(self, out=None):
+        path = Path(out) if out else self.library_path()
+        built.append(path)
+        path.write_bytes(b"")
+        return path
+
+    monkeypatch.setattr(CK, "GEN_DIR", tmp_path)
+    monkeypatch.setattr(CK.TemplateGenerator, "build", build)
+    tiles = CK.get_possible_tile_list("gfx950", "w4a16_g128_asym")
+    first, names = PT.build_qcfg_lib("w4a16_g128_asym")
+    assert PT.build_qcfg_lib("w4a16_g128_asym")[0] == first and len(built) == 1 and names == tiles
+    monkeypatch.setattr(CK, "get_possible_tile_list", lambda arch, q: tiles[1:])
+    second, names = PT.build_qcfg_lib("w4a16_g128_asym")
+    assert second != first and len(built) == 2 and names == tiles[1:]
+
+
 def test_perf_table_fit_and_sweep_shapes():
     from mxmoe_amd.kernels.tile_config import get_possible_tile_list
     from mxmoe_amd.perf_table import ProblemShape, linear_fit, sweep_entry
