@@ -144,7 +144,8 @@ def profile_qcfg(qcfg: str, arch: str = "gfx950", slots=SLOTS, waves=WAVES, rebu
 
 def main(argv=None) -> int:
     ap = argparse.ArgumentParser(description="Regenerate the kernel-profile table on this GPU")
-    ap.add_argument("--qcfgs", nargs="+", default=["w4a4_g-1_sym", "w8a8_g-1_sym", "w4a16_g128_asym", "w3a16_g128_asym", "w2a16_g128_asym", "w4a4_g128_sym", "fp16"])
+    ap.add_argument("--qcfgs", nargs="+", default=["w4a4_g-1_sym", "w8a8_g-1_sym", "w4a16_g128_asym", "w3a16_g128_asym", "w2a16_g128_asym", "w4a4_g128_sym", "fp16", "w8a16_g128_asym",
+                                                      "w4a16_g-1_asym", "w8a8_g-1_sym_E4M3"])
     ap.add_argument("--slots", nargs="+", default=list(SLOTS))
     ap.add_argument("--out", default="perf/performance_table.json")
     ap.add_argument("--build-only", action="store_true", help="compile the single-tile kernel libraries and stop (needs no GPU)")
@@ -158,6 +159,7 @@ def main(argv=None) -> int:
     table = json.loads(out.read_text()) if out.exists() else {}
     for q in a.qcfgs:
         table[q] = profile_qcfg(q, slots=a.slots, rebuild=a.rebuild)
+        table[table_key(q)] = table[q]
         out.parent.mkdir(parents=True, exist_ok=True)
         out.write_text(json.dumps(table, indent=1))
     return 0

@@ -275,6 +275,17 @@ def test_perf_table_library_of_another_candidate_list_is_not_reused(tmp_path, mo
     assert second != first and len(built) == 2 and names == tiles[1:]
 
 
+@pytest.mark.parametrize("strategies", [["w4a4_g-1_sym", "w8a8_g-1_sym"], ["w4a16_g128_asym", "w3a16_g128_asym", "w2a16_g128_asym"], ["w8a16_g128_asym", "fp16"],
+                                        ["w4a16_g-1_asym", "w4a4_g128_sym"], ["w8a8_g-1_sym_E4M3", "w4a4_g-1_sym"]])
+def test_shipped_profile_prices_every_candidate_tile(strategies):
+    """The allocator without hand-picked tiles asks the profile for every candidate of a format; w2a16 is looked up under its other name."""
+    from mxmoe_amd.perf_table import ProblemShape, get_runtime_cost
+
+    table = json.loads((Path(__file__).resolve().parent.parent / "perf" / "performance_table.json").read_text())
+    combos, cost = get_runtime_cost([[ProblemShape(37, 2816, 2048)]], strategies, table)
+    assert combos and all(c > 0 for per_strategy in cost[0][0] for c in per_strategy)
+
+
 def test_perf_table_fit_and_sweep_shapes():
     from mxmoe_amd.kernels.tile_config import get_possible_tile_list
     from mxmoe_amd.perf_table import ProblemShape, linear_fit, sweep_entry
