@@ -223,7 +223,11 @@ int mxmoe_unpermute_combine(const void* down_out, const void* shared_out, const 
  *                                  (A, B, scale_a, scale_b, C), 3 two int64 {rows routed, address of the shared expert's output rows},
  *                                  4 the sizes mxmoe_dim3 [P];
  *   mxmoe_plan_select_kernel       the kernel (>= 0) that mxmoe_plan_block / mxmoe_plan_grid_bound use for these formats when given -1, after
- *                                  checking formats and shapes; negative on error;
+ *                                  checking formats and shapes; negative on error.  It knows no row counts, so it never names a kernel made
+ *                                  for few rows;
+ *   mxmoe_plan_select_kernel_rows  the same for a batch of num_tokens tokens (shared_rows of them for the shared expert, 0 without one): a
+ *                                  kernel made for few rows where one is better, as the launcher would choose it for an even routing.
+ *                                  Pass the id to mxmoe_plan_grid_bound and to the calls that take a kernel_id;
  *   mxmoe_plan_grid_bound          workgroups that cover the launch whatever the routing, for at most routed_rows_max routed rows
  *                                  (tokens x top-k): per expert tiles(M) <= tiles(1) + slope * (M - 1), summed over the non-empty experts
  *                                  (workgroups past the planned tiles cost about 10 - 20 ns each, so the bound is kept tight);
@@ -241,6 +245,7 @@ int mxmoe_unpermute_combine(const void* down_out, const void* shared_out, const 
 size_t mxmoe_plan_bytes(int num_problems);
 size_t mxmoe_plan_offset(int which, int num_problems);
 int mxmoe_plan_select_kernel(int kernel_id, const mxmoe_block_desc* h_desc, int num_problems);
+int mxmoe_plan_select_kernel_rows(const mxmoe_block_desc* h_desc, int num_experts, int num_tokens, int topk, int shared_rows);
 int mxmoe_plan_grid_bound(int kernel_id, const mxmoe_block_desc* h_desc, int num_experts, int routed_rows_max, int shared_rows);
 int mxmoe_plan_block(int kernel_id, const int64_t* d_recv_tokens_per_exp, int num_experts, int shared_rows, const mxmoe_block_desc* d_desc,
                      const mxmoe_block_desc* h_desc, const void* inp_store, const void* scale_store, void* out_store, void* d_plan, void* stream);
@@ -301,7 +306,7 @@ int mxmoe_upload(void* dst, const void* host_src, size_t bytes, void* stream);
  *   plan_*         mxmoe_plan_bytes() each;
  *   dst_exp, token_of_row, row_of_slot   int32 [R]; iota   int32 [num_tokens] = 0, 1, 2, ...; recv   int64 [num_experts];
  *   workspace      mxmoe_permute_workspace_bytes(R, num_experts), 16-byte aligned.
- * grid_*: mxmoe_plan_grid_bound of each block.  rotate, had_*: of the intermediate rows, as for mxmoe_silu_mul_quant (bits 0 - 1 only).
+ * kernel_*: from mxmoe_plan_select_kernel_rows (or -1: as mxmoe_plan_select_kernel).  grid_*: mxmoe_plan_grid_bound of each block with that kernel.  rotate, had_*: of the intermediate rows, as for mxmoe_silu_mul_quant (bits 0 - 1 only).
  *
  * mxmoe_layer_supported   1 when the short form takes the layer: hidden 512, 1024, 2048 or 4096; at most 512 experts; inter a
  *                         multiple of 32; no bf6 operands; token stores and fp16 weights below 2 GiB; and R <= 65536, or

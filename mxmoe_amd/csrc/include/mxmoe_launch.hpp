@@ -703,23 +703,29 @@ inline bool kernel_covers(const FusedKernel& k, const mxmoe_qparams* q, int coun
   return true;
 }
 
-// The kernel the launcher picks when the caller names none: the first fused kernel without operand variants that has a tile for every
-// format; a kernel made for few rows per problem wins when no problem has more (`max_rows` < 0: row counts unknown, none of those).
-inline int auto_kernel_for(const mxmoe_qparams* h_q, int count, long max_rows) {
-  auto& reg = registry();
-  int plain = -1;
-  for (int i = 0; i < (int)reg.size(); ++i) {
-    if (reg[i].policy != Policy::Fused || kernel_has_variants(reg[i]) || !kernel_covers(reg[i], h_q, count)) continue;
-    if (reg[i].max_rows_hint > 0) {
-      if (max_rows >= 0 && max_rows <= reg[i].max_rows_hint) return i;
-    } else if (plain < 0) {
-      plain = i;
-    }
+// The problems of a launch that have rows, as far as the choice of a kernel for few rows looks at them.  The launcher fills it from its list; the planned
+// forward, which does not know its routing on the host, with what an even routing would give (mxmoe_plan_select_kernel_rows).
+struct RowSummary {
+  int live = 0, tall = 0;         // problems; those of more than 16 rows
+  long rows = 0, max_rows = 0;
+  long blocks = 0;                // of 256 channels
+  bool integer = false;           // w4a4 or w8a8 among them
+  void add(Fmt f, long m, uint32_t N) {
+    if (m == 0) return;
+    ++live;
+    tall += m > 16;
+    rows += m;
+    max_rows = std::max(max_rows, m);
+    blocks += (N + 255) / 256;
+    integer = integer || f == Fmt::W4A4 || f == Fmt::W8A8;
   }
-  return plain;
+};
+inline RowSummary row_summary(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int count) {
+  RowSummary s;
+  for (int i = 0; i < count; ++i) s.add(classify(h_q[i]), h_sizes[i].x, h_sizes[i].y);
+  return s;
 }
-// (A few-row kernel runs 16-row tiles: it is meant for lists whose problems mostly fit one such tile.  When more than a quarter of
-// the non-empty problems need several, the kernels that also hold the 32-row few-token tile do better, whatever the largest count.)
+
 //
 // Lists of few rows with w4a4 or w8a8 problems go to the kernels that hold the narrow integer tile (WxAxNarrowTile, for problems of up to 32 rows; more take
 // 64-row tiles): no problem above 64 rows, 24 per problem on average, and at most 768 blocks of 256 channels over all problems.  A whole layer, us, w4a4 / w8a8
@@ -729,27 +735,18 @@ inline int auto_kernel_for(const mxmoe_qparams* h_q, int count, long max_rows) {
 // 117 -> 125; the first block of the third (896 blocks of 256 channels, enough for the wide tiles to fill the chip) on them too, w4a4 150 -> 160 (16 tokens).
 // A 128-row tile beside them would take the third workgroup of a CU (244 registers, 161 without): 60 experts 77 -> 83 (32).
 // (From 8 blocks on: the planning rules for long problems are stated, and tested, on lists of two or three small problems in the wide shapes.)
-constexpr int kFewRows = 24, kFewRowsMax = 64, kFewColumns = 768, kFewColumnsMin = 8;
+constexpr int kFewRows = 24, kFewRowsMax = 64, kFewBlocks = 768, kFewBlocksMin = 8;
 inline bool holds_narrow(const FusedKernel& k) {
   for (const BranchInfo& b : k.branches)
     if ((b.fmt == Fmt::W4A4 || b.fmt == Fmt::W8A8) && b.BN == 64) return true;
   return false;
 }
-inline bool few_rows(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int count) {
-  long rows = 0, columns = 0, live = 0;
-  bool narrow = false;
-  for (int i = 0; i < count; ++i) {
-    if (h_sizes[i].x == 0) continue;
-    if (h_sizes[i].x > (unsigned)kFewRowsMax) return false;
-    ++live;
-    rows += h_sizes[i].x;
-    columns += (h_sizes[i].y + 255) / 256;
-    const Fmt f = classify(h_q[i]);
-    narrow = narrow || f == Fmt::W4A4 || f == Fmt::W8A8;
-  }
-  return narrow && rows <= kFewRows * live && columns >= kFewColumnsMin && columns <= kFewColumns;
+inline bool few_rows(const RowSummary& s) {
+  return s.integer && s.max_rows <= kFewRowsMax && s.rows <= kFewRows * s.live && s.blocks >= kFewBlocksMin && s.blocks <= kFewBlocks;
 }
-// The kernel of few-token weight-only tiles of 64 channels, against those of 128: twice the workgroups, 125 registers (four workgroups per CU) against 164.
+// A list of weight-only problems of few rows takes a kernel made of 16-row few-token tiles (FusedKernel::max_rows_hint), unless more than a quarter of its
+// problems need several of them: then the kernels that also hold the 32-row few-token tile do better, whatever the largest count.
+// Of those kernels, the one of 64-channel tiles against that of 128: twice the workgroups, 125 registers (four workgroups per CU) against 164.
 // Up to 6 rows per problem on average; the activations, read once per tile, weigh more with more.  A whole layer, us, 128 -> 64 channels: 64 experts top-6 and
 // a shared one, w4a16 / w3a16, 30.2 -> 28.2 (1 token), 42.7 -> 39.2 (4), 64 -> 61 (16), 75 -> 73 (64); 60 experts top-4 and a shared one 33.6 -> 29.0 (1),
 // 58 -> 51 (16); 8 experts of N = 28 672 / 4096 61.6 -> 52.1 (1), 144 -> 140 (16), but 144 -> 150 (32: 8 rows each).
@@ -759,28 +756,40 @@ inline bool only_narrow_few_token(const FusedKernel& k) {
     if (!is_weight_only(b.fmt) || b.BN != 64) return false;
   return true;
 }
-inline int auto_kernel(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int count) {
-  long max_rows = 0, rows = 0, columns = 0;
-  int live = 0, over = 0;
-  for (int i = 0; i < count; ++i) {
-    max_rows = std::max(max_rows, (long)h_sizes[i].x);
-    rows += h_sizes[i].x;
-    columns += h_sizes[i].x > 0 ? (h_sizes[i].y + 255) / 256 : 0;
-    live += h_sizes[i].x > 0;
-    over += h_sizes[i].x > 16;
-  }
-  if (few_rows(h_sizes, h_q, count)) {
-    auto& reg = registry();
+
+// The kernel made for the few rows of a launch, or -1 where there is none or the plain kernels do better.  `covers(k)`: whether kernel k has a tile for every
+// problem's format (and operand layout).  The one place of this choice: the launcher and the planned forward both come here.
+template <class Covers>
+int few_row_kernel(const RowSummary& s, Covers&& covers) {
+  auto& reg = registry();
+  auto first = [&](auto&& wanted) {
     for (int i = 0; i < (int)reg.size(); ++i)
-      if (reg[i].policy == Policy::Fused && !kernel_has_variants(reg[i]) && holds_narrow(reg[i]) && kernel_covers(reg[i], h_q, count)) return i;
+      if (reg[i].policy == Policy::Fused && wanted(reg[i]) && covers(reg[i])) return i;
+    return -1;
+  };
+  if (few_rows(s)) {
+    const int kid = first(holds_narrow);
+    if (kid >= 0) return kid;
   }
-  const int kid = auto_kernel_for(h_q, count, 4 * over > live ? -1 : max_rows);
-  if (kid >= 0 && registry()[kid].max_rows_hint > 0 && rows <= kFewTokenRows * live && columns >= kFewColumnsMin) {
-    auto& reg = registry();
-    for (int i = 0; i < (int)reg.size(); ++i)
-      if (reg[i].policy == Policy::Fused && only_narrow_few_token(reg[i]) && kernel_covers(reg[i], h_q, count)) return i;
+  if (4 * s.tall > s.live) return -1;
+  const int kid = first([&](const FusedKernel& k) { return k.max_rows_hint > 0 && s.max_rows <= k.max_rows_hint; });
+  if (kid >= 0 && s.rows <= kFewTokenRows * s.live && s.blocks >= kFewBlocksMin) {
+    const int narrow = first(only_narrow_few_token);
+    if (narrow >= 0) return narrow;
   }
   return kid;
+}
+
+// The kernel the launcher picks when the caller names none: one made for few rows, or the first fused kernel without operand variants that has a tile for every
+// format.
+inline int auto_kernel(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int count) {
+  auto covers = [&](const FusedKernel& k) { return !kernel_has_variants(k) && kernel_covers(k, h_q, count); };
+  const int few = few_row_kernel(row_summary(h_sizes, h_q, count), covers);
+  if (few >= 0) return few;
+  auto& reg = registry();
+  for (int i = 0; i < (int)reg.size(); ++i)
+    if (reg[i].policy == Policy::Fused && reg[i].max_rows_hint == 0 && covers(reg[i])) return i;
+  return -1;
 }
 
 // K a multiple of the tile's K step, N a multiple of 8 (16 for the weight-only layouts)

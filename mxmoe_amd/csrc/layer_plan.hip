@@ -92,22 +92,25 @@ __global__ void __launch_bounds__(kPlanThreads) perm_scatter_plan_kernel(const P
   plan_block_body(pair.p[b / pair.chunks], chunk, pair.chunks, counts, d, sh, true);
 }
 
+// Whether a kernel has a tile for the format and operand layout of every block.
+static bool covers_blocks(const FusedKernel& k, const mxmoe_block_desc* h_desc, int et) {
+  for (int i = 0; i < et; ++i) {
+    Segment sg[2];
+    const int f = fmt_of(h_desc[i].q);
+    if (f == (int)Fmt::UNSUPPORTED || plan_segments(plan_of(k), f, 1, 256, 0, sg) < 0) return false;
+    // a kernel's w4a4 tiles take packed int4 rows or bf6 fragments, never both: the descriptor says which the block will get
+    if (f == (int)Fmt::W4A4 && kernel_takes_bf6(k) != wants_bf6(h_desc[i].q)) return false;
+    if (f == (int)Fmt::W8A8 && (kernel_variant(k, Fmt::W8A8) == kVariantFp8) != wants_fp8(h_desc[i].q)) return false;
+    // 16-bit float blocks of a layer are fp16 (the activation step between the launches computes in fp16): no bfloat16 kernel here
+    if (f == (int)Fmt::FP16 && kernel_variant(k, Fmt::FP16) != 0) return false;
+  }
+  return true;
+}
+
 // Kernel for the formats of `h_desc`, checked once on the host: every problem's format has a branch and its shape fits it.
 int resolve_kernel(int kernel_id, const mxmoe_block_desc* h_desc, int et) {
   auto& reg = registry();
-  auto covers = [&](const FusedKernel& k) {
-    for (int i = 0; i < et; ++i) {
-      Segment sg[2];
-      const int f = fmt_of(h_desc[i].q);
-      if (f == (int)Fmt::UNSUPPORTED || plan_segments(plan_of(k), f, 1, 256, 0, sg) < 0) return false;
-      // a kernel's w4a4 tiles take packed int4 rows or bf6 fragments, never both: the descriptor says which the block will get
-      if (f == (int)Fmt::W4A4 && kernel_takes_bf6(k) != wants_bf6(h_desc[i].q)) return false;
-      if (f == (int)Fmt::W8A8 && (kernel_variant(k, Fmt::W8A8) == kVariantFp8) != wants_fp8(h_desc[i].q)) return false;
-      // 16-bit float blocks of a layer are fp16 (the activation step between the launches computes in fp16): no bfloat16 kernel here
-      if (f == (int)Fmt::FP16 && kernel_variant(k, Fmt::FP16) != 0) return false;
-    }
-    return true;
-  };
+  auto covers = [&](const FusedKernel& k) { return covers_blocks(k, h_desc, et); };
   if (kernel_id < 0) {
     for (int i = 0; i < (int)reg.size() && kernel_id < 0; ++i)
       if (reg[i].policy == Policy::Fused && reg[i].max_rows_hint == 0 && covers(reg[i])) kernel_id = i;  // (row counts are not known here: no few-row kernel)
@@ -169,6 +172,34 @@ int mxmoe_plan_select_kernel(int kernel_id, const mxmoe_block_desc* h_desc, int 
     return -3;
   }
   return resolve_kernel(kernel_id, h_desc, num_problems);
+}
+
+int mxmoe_plan_select_kernel_rows(const mxmoe_block_desc* h_desc, int num_experts, int num_tokens, int topk, int shared_rows) {
+  const int et = num_experts + (shared_rows > 0 ? 1 : 0);
+  const int plain = mxmoe_plan_select_kernel(-1, h_desc, et);
+  if (plain < 0) return plain;
+  if (num_experts <= 0 || num_tokens <= 0 || topk <= 0 || shared_rows < 0) {
+    last_error() = "experts, tokens and top-k must be positive";
+    return -3;
+  }
+  // an even routing over the widest experts: every one of them gets a row before any gets two
+  const long routed = (long)num_tokens * topk;
+  const int live = (int)std::min<long>(num_experts, routed);
+  std::vector<int> widest(num_experts);
+  for (int i = 0; i < num_experts; ++i) widest[i] = i;
+  std::stable_sort(widest.begin(), widest.end(), [&](int x, int y) { return h_desc[x].N > h_desc[y].N; });
+  RowSummary s;
+  for (int i = 0; i < num_experts; ++i) {
+    const mxmoe_block_desc& d = h_desc[widest[i]];
+    s.add((Fmt)fmt_of(d.q), i < live ? routed / live + (i < routed % live) : 0, d.N);
+    s.integer = s.integer || fmt_of(d.q) == (int)Fmt::W4A4 || fmt_of(d.q) == (int)Fmt::W8A8;  // (any of them may get rows)
+  }
+  if (shared_rows > 0) s.add((Fmt)fmt_of(h_desc[num_experts].q), shared_rows, h_desc[num_experts].N);
+  s.max_rows = std::max<long>(s.max_rows, num_tokens);  // one expert may get them all
+  // an uneven routing has problems of several 16-row tiles well before the average reaches 16
+  if (routed > 12l * num_experts) s.tall = s.live;
+  const int few = few_row_kernel(s, [&](const FusedKernel& k) { return covers_blocks(k, h_desc, et); });
+  return few >= 0 && resolve_kernel(few, h_desc, et) == few ? few : plain;
 }
 
 int mxmoe_plan_grid_bound(int kernel_id, const mxmoe_block_desc* h_desc, int num_experts, int routed_rows_max, int shared_rows) {

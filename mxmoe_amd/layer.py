@@ -143,24 +143,10 @@ class MxMoELayer:
 
     def _planned_kernel(self, h, t: int, topk: int) -> int:
         """The kernel that a block's planned launch runs on for t tokens."""
-        lib, et = _lib.load(), len(h)
-        kid = lib.mxmoe_plan_select_kernel(-1, h, et)
+        lib = _lib.load()
+        kid = lib.mxmoe_plan_select_kernel_rows(h, self.cfg.num_experts, t, topk, t if self.cfg.num_shared else 0)
         if kid < 0:
             raise RuntimeError(lib.mxmoe_last_error().decode())
-        if t <= 64 and t * topk <= 12 * self.cfg.num_experts:  # few tokens, and on average well under one 16-row tile per expert: a kernel made of 16-row few-token tiles alone, if one covers the formats
-            few = lib.mxmoe_find_kernel(b"groupgemm_hz_fused_wo_few" if t * topk <= 6 * min(self.cfg.num_experts, t * topk) else b"groupgemm_hz_fused_wo_skinny")
-            if few >= 0 and lib.mxmoe_plan_select_kernel(few, h, et) == few:
-                kid = few
-        if t <= 64 and any(d.a_bits < 16 for d in h):
-            # the launcher's rule for lists of few rows (mxmoe_launch.hpp, few_rows), with the experts that may have any
-            e_cnt, shared = self.cfg.num_experts, self.cfg.num_shared > 0
-            live = min(e_cnt, t * topk)
-            cols = sorted((-(-int(d.N) // 256) for d in h[:e_cnt]), reverse=True)
-            if t * topk + t * shared <= 24 * (live + shared) and 8 <= sum(cols[:live]) + shared * -(-int(h[et - 1].N) // 256) <= 768:
-                for name in (b"groupgemm_hz_fused_wxax_few", b"groupgemm_hz_fused_all_few"):
-                    few = lib.mxmoe_find_kernel(name)
-                    if few >= 0 and lib.mxmoe_plan_select_kernel(few, h, et) == few:
-                        return few
         return kid
 
     def _planned_setup(self, t: int, topk: int):

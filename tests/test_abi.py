@@ -344,3 +344,43 @@ def test_lists_of_few_rows_take_the_kernels_with_narrow_tiles():
     assert picked((24, 2816, w4), (25, 2816, w8)) == "hz_fused_wxax"
     assert picked(*[(1, 256, w4)] * 7) == "hz_fused_wxax" and picked(*[(1, 256, w4)] * 8) == "hz_fused_wxax_few"
     assert picked(*[(1, 2048, w4)] * 96) == "hz_fused_wxax_few" and picked(*[(1, 2048, w4)] * 97) == "hz_fused_wxax"
+
+
+def _blocks(formats, n, k, shared=None):
+    """Host block descriptors: experts of the given formats, and a shared expert (format, N, K)."""
+    from mxmoe_amd import _lib
+
+    rows = [(q, n, k) for q in formats] + ([shared] if shared else [])
+    return (_lib.BlockDesc * len(rows))(*[_lib.BlockDesc(q[0], q[1], q[2], int(q[3]), (C.c_uint8 * 3)(), nn, kk, 0, 0) for q, nn, kk in rows])
+
+
+W4, W8, WO4, WO3, FP = (4, 4, -1, True), (8, 8, -1, True), (16, 4, 128, False), (16, 3, 128, False), (16, 16, -1, True)
+
+
+@pytest.mark.parametrize("formats", [[W4], [W8], [W4, W8], [WO4, WO3], [W4, W8, WO4], [FP], [W4, FP]])
+@pytest.mark.parametrize("experts,topk,n,k,shared_n,shared_k", [(60, 4, 2816, 2048, 0, 0), (60, 4, 2048, 1408, 2048, 5632), (64, 6, 2816, 2048, 5632, 2048),
+                                                                (8, 2, 4096, 14336, 0, 0), (8, 2, 28672, 4096, 0, 0), (4, 1, 256, 512, 0, 0)])
+def test_planned_batches_take_the_kernel_that_the_launcher_takes_for_an_even_routing(lib, formats, experts, topk, n, k, shared_n, shared_k):
+    """One rule for few rows, whoever asks: mxmoe_plan_select_kernel_rows against the automatic choice for a list with as even a routing as the batch has, up to
+    the largest batch that any of those kernels is meant for, and the kernel by formats alone beyond."""
+    qs = [formats[e % len(formats)] for e in range(experts)]
+    shared = (formats[0], shared_n, shared_k) if shared_n else None
+    desc = _blocks(qs, n, k, shared)
+    for t in (1, 2, 3, 5, 8, 13, 16, 24, 32, 33, 48, 64, 65, 200):
+        kid = lib.mxmoe_plan_select_kernel_rows(desc, experts, t, topk, t if shared else 0)
+        live = min(experts, t * topk)
+        counts = [t * topk // live + (e < t * topk % live) for e in range(live)] + [0] * (experts - live)
+        assert kid >= 0, lib.mxmoe_last_error()
+        if t > 64 or t * topk > 12 * experts and formats[0][0] == 16:
+            assert kid == lib.mxmoe_plan_select_kernel(-1, desc, experts + (1 if shared else 0)), t
+            continue
+        rc, _, _ = _plan(lib, -1, [((c, n, k), q) for c, q in zip(counts, qs)] + ([((t, shared_n, shared_k), shared[0])] if shared else []))
+        assert rc - 1000 == kid, (t, lib.mxmoe_kernel_name(rc - 1000), lib.mxmoe_kernel_name(kid))
+
+
+def test_planned_batches_refuse_what_is_no_batch(lib):
+    desc = _blocks([W4, W4], 256, 512)
+    for args in ((0, 1, 1, 0), (2, 0, 1, 0), (2, 1, 0, 0), (2, 1, 1, -1)):
+        assert lib.mxmoe_plan_select_kernel_rows(desc, *args) < 0
+    assert lib.mxmoe_plan_select_kernel_rows(None, 2, 1, 1, 0) < 0
+    assert lib.mxmoe_plan_select_kernel_rows(_blocks([(4, 2, -1, True)] * 2, 256, 512), 2, 1, 1, 0) < 0
