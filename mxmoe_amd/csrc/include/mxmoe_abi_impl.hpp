@@ -91,10 +91,10 @@ int mxmoe_group_gemm_plan(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_
     }
     const Fmt f = classify(h_q[i]);
     Segment sg[2];
-    const int ns = f == Fmt::UNSUPPORTED ? -1 : plan_segments(plan_of(k), (int)f, (int)h_sizes[i].x, (int)h_sizes[i].y, scope.long_tiles_of(h_sizes[i]), sg);
+    const int ns = f == Fmt::UNSUPPORTED ? -1 : plan_segments(plan_of(k), (int)f, (int)h_sizes[i].x, (int)h_sizes[i].y, scope.long_tiles_of(h_sizes[i]), scope.few_blocks, sg);
     if (ns < 0) { last_error() = "quant type not supported"; return 1; }
     if (branch_out) {  // (an empty problem: the branch one row would take)
-      if (ns == 0) plan_segments(plan_of(k), (int)f, 1, (int)h_sizes[i].y, scope.long_tiles_of(h_sizes[i]), sg);
+      if (ns == 0) plan_segments(plan_of(k), (int)f, 1, (int)h_sizes[i].y, scope.long_tiles_of(h_sizes[i]), scope.few_blocks, sg);
       branch_out[i] = sg[0].branch;
     }
     for (int j = 0; j < ns; ++j) {

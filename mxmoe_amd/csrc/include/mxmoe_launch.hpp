@@ -403,6 +403,8 @@ __host__ __device__ inline int tiles_over(int x, int lg) { return (x + (1 << lg)
 constexpr int kNumFmts = (int)Fmt::UNSUPPORTED;
 struct PlanInfo {
   int nb;                       // branches
+  // Narrow integer tiles among them; and, where a launch is planned with them, whether it has few blocks of channels (kPoleBlocks).
+  int narrow, few_blocks;
   uint8_t order[kMaxBranches];  // positions in b, most expensive tile first (branch_cost); ties keep the registration order
   uint8_t fmt_start[kNumFmts + 4];
   // by format, in registration order inside a format: those of format f are b[fmt_start[f]] .. b[fmt_start[f + 1] - 1], and the planners
@@ -414,6 +416,14 @@ static_assert(sizeof(PlanInfo) % 8 == 0, "copied word by word");
 struct Segment {
   int row0, rows, branch, tiles;
 };
+
+// Blocks of 256 channels, over all problems of a launch, up to which a 64-row integer tile sets the launch's time when it runs beside narrow ones: they stream
+// their weights at the rate of the machine and are done in less than half of its time, during which it shares its CU with them.  There, problems of 33 .. 64 rows
+// (and up to 128) take narrow tiles too (same sums: integers).  Eight problems of 45 .. 2 rows, K = 2048 / 14 336, us, 64-row tiles / narrow ones / a kernel of wide tiles
+// alone: 128 blocks w4a4 16.6 / 13.5 / 13.4, 82 / 63 / 60, w8a8 26.5 / 21.8 / 19.9, 146 / 118 / 107; 64 blocks w4a4 13.9 / 10.0 / 13.0, 60 / 40 / 56.  Beyond, the
+// narrow tiles lose what they gain: 256 blocks 22.1 / 19.9 / 17.8; 512 blocks (64 problems) 31.8 / 32.2 / 32.0, half of them of 40 rows 33.6 / 39.0 / 31.8.
+constexpr int kPoleBlocks = 128;
+__host__ __device__ inline bool integer_sums(int f) { return f == (int)Fmt::W4A4 || f == (int)Fmt::W8A8; }
 
 // Tiles of a launch's long-K problems, all of them together, from which on it is as busy with them as with the rest (a quarter of the 512
 // workgroups that run at a time).
@@ -522,10 +532,11 @@ __host__ __device__ inline int plan_split(const PlanInfo& k, int f, int M, int N
   return 2;
 }
 
-// Both steps: the number of segments (0 for M == 0), or -1 when the kernel has no tile for `f`.
-inline int plan_segments(const PlanInfo& k, int f, int M, int N, int long_tiles, Segment out[2]) {
+// Both steps: the number of segments (0 for M == 0), or -1 when the kernel has no tile for `f`.  `pole`: the problem is in a launch of few blocks (kPoleBlocks).
+inline int plan_segments(const PlanInfo& k, int f, int M, int N, int long_tiles, bool pole, Segment out[2]) {
   PlanChoice c;
   const int rc = plan_choose(k, f, M, N, c);
+  if (pole && long_tiles == 0 && integer_sums(f)) long_tiles = c.large_tiles;
   return rc <= 0 ? rc : plan_split(k, f, M, N, c, long_tiles, out);
 }
 
@@ -533,6 +544,7 @@ inline PlanInfo make_plan_info(const std::vector<BranchInfo>& branches) {
   PlanInfo k;
   std::memset(&k, 0, sizeof k);
   k.nb = std::min((int)branches.size(), kMaxBranches);
+  for (int i = 0; i < k.nb; ++i) k.narrow |= integer_sums((int)branches[i].fmt) && branches[i].BN == 64;
   auto log2_of = [](int v) {
     int lg = 0;
     while ((1 << lg) < v) ++lg;
@@ -698,7 +710,7 @@ inline bool kernel_covers(const FusedKernel& k, const mxmoe_qparams* q, int coun
   for (int i = 0; i < count; ++i) {
     const Fmt f = classify(q[i]);
     Segment sg[2];
-    if (f == Fmt::UNSUPPORTED || plan_segments(plan_of(k), (int)f, 1, 256, 0, sg) < 0) return false;
+    if (f == Fmt::UNSUPPORTED || plan_segments(plan_of(k), (int)f, 1, 256, 0, false, sg) < 0) return false;
   }
   return true;
 }
@@ -736,11 +748,7 @@ inline RowSummary row_summary(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_
 // A 128-row tile beside them would take the third workgroup of a CU (244 registers, 161 without): 60 experts 77 -> 83 (32).
 // (From 8 blocks on: the planning rules for long problems are stated, and tested, on lists of two or three small problems in the wide shapes.)
 constexpr int kFewRows = 24, kFewRowsMax = 64, kFewBlocks = 768, kFewBlocksMin = 8;
-inline bool holds_narrow(const FusedKernel& k) {
-  for (const BranchInfo& b : k.branches)
-    if ((b.fmt == Fmt::W4A4 || b.fmt == Fmt::W8A8) && b.BN == 64) return true;
-  return false;
-}
+inline bool holds_narrow(const FusedKernel& k) { return plan_of(k).narrow; }
 inline bool few_rows(const RowSummary& s) {
   return s.integer && s.max_rows <= kFewRowsMax && s.rows <= kFewRows * s.live && s.blocks >= kFewBlocksMin && s.blocks <= kFewBlocks;
 }
@@ -798,17 +806,23 @@ inline bool shape_ok(const BranchInfo& bi, const mxmoe_dim3& sz) {
   return sz.z != 0 && sz.z % bi.k_multiple == 0 && (int)sz.z >= bi.k_min && sz.y % 8 == 0 && !(wo && sz.y % 16 != 0);
 }
 
-// What the planning of one launch's problems has in common: its smallest K, and the large tiles of its long problems.  Problems without rows
+// What the planning of one launch's problems has in common: its smallest K, the large tiles of its long problems, whether it has few blocks.  Problems without rows
 // have no part in it: a list plans the same with and without them (the device planner sees every expert, the operators leave out empty ones).
 struct LaunchScope {
   int kmin = 0x7fffffff, long_tiles = 0;
+  bool few_blocks = false;
   // the `long_tiles` argument of a problem's plan
   int long_tiles_of(const mxmoe_dim3& sz) const { return runs_long((int)sz.z, kmin) ? long_tiles : 0; }
 };
 inline LaunchScope launch_scope(const PlanInfo& pi, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int n) {
   LaunchScope s;
+  long blocks = 0;
   for (int i = 0; i < n; ++i)
-    if (h_sizes[i].x != 0) s.kmin = std::min(s.kmin, (int)h_sizes[i].z);
+    if (h_sizes[i].x != 0) {
+      s.kmin = std::min(s.kmin, (int)h_sizes[i].z);
+      blocks += (h_sizes[i].y + 255) / 256;
+    }
+  s.few_blocks = pi.narrow && blocks <= kPoleBlocks;
   for (int i = 0; i < n; ++i) {
     const Fmt f = classify(h_q[i]);
     PlanChoice c;
@@ -834,7 +848,7 @@ inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, c
     const mxmoe_dim3& sz = h_sizes[base + i];
     const Fmt f = classify(h_q[base + i]);
     Segment sg[2];
-    const int ns = f == Fmt::UNSUPPORTED ? -1 : plan_segments(pi, (int)f, (int)sz.x, (int)sz.y, scope.long_tiles_of(sz), sg);
+    const int ns = f == Fmt::UNSUPPORTED ? -1 : plan_segments(pi, (int)f, (int)sz.x, (int)sz.y, scope.long_tiles_of(sz), scope.few_blocks, sg);
     if (ns < 0) {
       last_error() = "quant type not supported";
       return 1;

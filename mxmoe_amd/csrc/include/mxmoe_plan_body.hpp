@@ -56,6 +56,15 @@ struct PlanParams {
   PlanInfo info;
 };
 
+// The branch table a block is planned with.  Which experts get rows is not known here, so all of them count as blocks of the launch.
+inline PlanInfo plan_info_of_block(const FusedKernel& k, const mxmoe_block_desc* h_desc, int et) {
+  PlanInfo info = plan_of(k);
+  long blocks = 0;
+  for (int i = 0; i < et; ++i) blocks += (h_desc[i].N + 255) / 256;
+  info.few_blocks = info.narrow && blocks <= kPoleBlocks;
+  return info;
+}
+
 constexpr int kPlanThreads = 128;
 constexpr int kMaxPlannedProblems = 4096;  // experts of a planned block (run as launches of kMaxProblems experts each)
 static_assert(kMaxProblems <= kPlanThreads, "one thread per problem");
@@ -200,7 +209,7 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
   const bool long_k = mine && K > kmin;
   const int long_tiles = sh.long_tiles[0] - (sh.kmin[0] == kmin ? sh.long_tiles_kmin[0] : 0) + sh.long_tiles[1] - (sh.kmin[1] == kmin ? sh.long_tiles_kmin[1] : 0);
   Segment sg[2];
-  const int ns = have > 0 ? plan_split(info, fmt, (int)rows, N, choice, runs_long(K, kmin) ? min(long_tiles, kLongTiles) : 0, sg) : 0;
+  const int ns = have > 0 ? plan_split(info, fmt, (int)rows, N, choice, runs_long(K, kmin) ? min(long_tiles, kLongTiles) : info.few_blocks && integer_sums(fmt) ? choice.large_tiles : 0, sg) : 0;
   const PlanBranch& my_branch = info.b[info.order[min(lane, kMaxBranches - 1)]];  // lane r: the branch of rank r
   const int my_order = my_branch.index;
   int seg_rank[2] = {-1, -1}, seg_pos[2] = {0, 0}, seg_first[2] = {0, 0};

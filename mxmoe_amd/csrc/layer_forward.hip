@@ -409,7 +409,7 @@ int mxmoe_layer_create(const mxmoe_layer_desc* d, void** handle) {
     p.E = d->num_experts;
     p.Et = et;
     p.shared_rows = shared_rows;
-    p.info = plan_of(registry()[kid]);
+    p.info = plan_info_of_block(registry()[kid], h_desc, et);
     return kid;
   };
   f->d.kernel_gate_up = fill(f->pair.p[0], d->kernel_gate_up, d->d_gate_up, d->h_gate_up, d->act, d->plan_gate_up);

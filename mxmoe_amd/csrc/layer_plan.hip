@@ -97,7 +97,7 @@ static bool covers_blocks(const FusedKernel& k, const mxmoe_block_desc* h_desc, 
   for (int i = 0; i < et; ++i) {
     Segment sg[2];
     const int f = fmt_of(h_desc[i].q);
-    if (f == (int)Fmt::UNSUPPORTED || plan_segments(plan_of(k), f, 1, 256, 0, sg) < 0) return false;
+    if (f == (int)Fmt::UNSUPPORTED || plan_segments(plan_of(k), f, 1, 256, 0, false, sg) < 0) return false;
     // a kernel's w4a4 tiles take packed int4 rows or bf6 fragments, never both: the descriptor says which the block will get
     if (f == (int)Fmt::W4A4 && kernel_takes_bf6(k) != wants_bf6(h_desc[i].q)) return false;
     if (f == (int)Fmt::W8A8 && (kernel_variant(k, Fmt::W8A8) == kVariantFp8) != wants_fp8(h_desc[i].q)) return false;
@@ -206,11 +206,11 @@ int mxmoe_plan_grid_bound(int kernel_id, const mxmoe_block_desc* h_desc, int num
   const int et = num_experts + (shared_rows > 0 ? 1 : 0);
   const int kid = mxmoe_plan_select_kernel(kernel_id, h_desc, et);
   if (kid < 0) return kid;
-  const PlanInfo& pi = plan_of(registry()[kid]);
+  const PlanInfo pi = plan_info_of_block(registry()[kid], h_desc, et);
   // For every routed expert tiles(M) <= first + slope * (M - 1) for all M >= 1, with first = tiles(1) and slope the steepest rise
   // found by walking M over 64 rows of the format's largest tile (the planner's decisions repeat with that tile's period).  With at
   // most n = min(experts, rows) experts non-empty, the launch has at most (sum of the n largest `first`) + max slope * (rows - n) tiles.
-  // A block that is long against the smallest K may be so in its launch (or not, when the block is run as several launches), beside
+  // A block that is long against the smallest K, or an integer one of few blocks of channels, may be planned as such in its launch (or not, when the block is run as several launches), beside
   // any number of others: the larger count holds, and with more of the others it takes shapes of less total cost and more each,
   // hence fewer tiles, so it is enough to look at the block with none.
   auto tiles_of = [&](int f, int m, int n, bool maybe_long) {
@@ -238,7 +238,7 @@ int mxmoe_plan_grid_bound(int kernel_id, const mxmoe_block_desc* h_desc, int num
   std::vector<Seen> seen;
   for (int e = 0; e < et; ++e) {
     const int f = fmt_of(h_desc[e].q), n = (int)h_desc[e].N;
-    const bool maybe_long = runs_long((int)h_desc[e].K, (int)kmin);
+    const bool maybe_long = runs_long((int)h_desc[e].K, (int)kmin) || (pi.few_blocks && integer_sums(f));
     if (e >= num_experts) {  // the shared expert's row count is known
       shared_tiles += tiles_of(f, shared_rows, n, maybe_long);
       continue;
@@ -248,7 +248,7 @@ int mxmoe_plan_grid_bound(int kernel_id, const mxmoe_block_desc* h_desc, int num
       if (sn.f == f && sn.n == n && sn.maybe_long == maybe_long) hit = &sn;
     if (!hit) {
       Segment sg[2];
-      plan_segments(pi, f, 1 << 20, n, 0, sg);
+      plan_segments(pi, f, 1 << 20, n, 0, false, sg);
       const BranchInfo& bi = registry()[kid].branches[sg[0].branch];
       const int bm = bi.BM, cols = (n + bi.BN - 1) / bi.BN;
       Seen sn{f, n, maybe_long, tiles_of(f, 1, n, maybe_long), 0, 0.0, (double)cols / bm};
@@ -301,7 +301,7 @@ static int fill_plan_params(PlanParams& p, int kernel_id, const int64_t* d_recv,
   p.Et = et;
   p.shared_rows = shared_rows;
   p.form = LayerForm{};
-  p.info = plan_of(registry()[kid]);
+  p.info = plan_info_of_block(registry()[kid], h_desc, et);
   return 0;
 }
 

@@ -384,3 +384,63 @@ def test_planned_batches_refuse_what_is_no_batch(lib):
         assert lib.mxmoe_plan_select_kernel_rows(desc, *args) < 0
     assert lib.mxmoe_plan_select_kernel_rows(None, 2, 1, 1, 0) < 0
     assert lib.mxmoe_plan_select_kernel_rows(_blocks([(4, 2, -1, True)] * 2, 256, 512), 2, 1, 1, 0) < 0
+
+
+@pytest.mark.parametrize("kernel", ["groupgemm_hz_fused_wxax_few", "groupgemm_hz_fused_all_few"])
+def test_few_blocks_take_narrow_tiles_beyond_32_rows(lib, kernel):
+    """Launches of up to 128 blocks of 256 channels with narrow tiles: problems of 33 .. 128 rows take them too (a 64-row tile would be what the launch waits
+    for); one block more, or a weight-only problem, and they do not.  Problems without rows are no blocks of the launch."""
+    kid = lib.mxmoe_find_kernel(kernel.encode())
+
+    def tile(rows, probs):
+        rc, br, _ = _plan(lib, kid, probs)
+        assert rc == 1000 + kid
+        info = (C.c_int32 * 8)()
+        at = next(i for i, p in enumerate(probs) if p[0][0] == rows)
+        assert lib.mxmoe_kernel_branch(kid, br[at], info) == 0
+        return info[1], info[2]                                          # rows, channels of the tile
+
+    def few(rows, q, blocks, empty=0):
+        return [((rows, 4096, 14336), q)] + [((5, 4096, 14336), W4 if i % 2 else W8) for i in range(blocks // 16 - 1)] + [((7, 256, 14336), W4)] * (blocks % 16) \
+            + [((0, 4096, 14336), W8)] * empty
+
+    for q in (W4, W8):
+        for rows in (33, 45, 64, 65, 100, 128):
+            assert tile(rows, few(rows, q, 128, empty=4)) == (32, 64), (q, rows)
+        assert tile(45, few(45, q, 129))[1] == 256 and tile(64, few(64, q, 129))[1] == 256 and tile(129, few(129, q, 64))[1] == 256
+        assert tile(32, few(32, q, 128)) == (32, 64) and tile(32, few(32, q, 160)) == (32, 64)
+    wide = lib.mxmoe_find_kernel(kernel.replace("_few", "").encode())
+    rc, br, _ = _plan(lib, wide, few(45, W4, 64))                         # kernels without narrow tiles: as before
+    assert rc == 1000 + wide
+    if "all" in kernel:
+        assert tile(45, few(45, WO4, 64)) == (128, 256)
+
+
+def test_planned_grid_bound_with_narrow_tiles(lib):
+    """The worst-case grid of planned launches on the kernels with narrow tiles against the tiles of the same launches planned on the host; few blocks count
+    over all experts there (they are not known to be empty), so a list of all of them decides alike."""
+    import random
+
+    rnd = random.Random(5)
+    for kernel, n, k, e, shared_rows, fmts in (("groupgemm_hz_fused_wxax_few", 4096, 14336, 8, 0, [W4, W8]), ("groupgemm_hz_fused_all_few", 4096, 14336, 8, 0, [W4, W8, WO4]),
+                                               ("groupgemm_hz_fused_wxax_few", 512, 1024, 40, 64, [W4, W8]), ("groupgemm_hz_fused_wxax_few", 2048, 1408, 60, 48, [W4])):
+        kid = lib.mxmoe_find_kernel(kernel.encode())
+        qs = [rnd.choice(fmts) for _ in range(e)]
+        desc = _blocks(qs, n, k, (fmts[0], n, 2 * k) if shared_rows else None)
+        for routed in (1, 7, 64, 128, 200, 512):
+            bound = lib.mxmoe_plan_grid_bound(kid, desc, e, routed, shared_rows)
+            assert bound > 0, lib.mxmoe_last_error()
+            for trial in range(60):
+                counts = [0] * e
+                if trial % 3 == 0:
+                    unit = rnd.choice([1, 17, 32, 33, 40, 64, 65])
+                    left = routed
+                    for i in range(e):
+                        counts[i] = min(unit, left)
+                        left -= counts[i]
+                    counts[rnd.randrange(e)] += left
+                else:
+                    for _ in range(routed):
+                        counts[min(int(rnd.paretovariate(0.7 if trial % 3 == 1 else 3.0)) - 1, e - 1)] += 1
+                rc, _, tiles = _plan(lib, kid, [((m, n, k), q) for m, q in zip(counts, qs)] + ([((shared_rows, n, 2 * k), fmts[0])] if shared_rows else []))
+                assert rc == 1000 + kid and tiles + 8 * 9 <= bound, (kernel, n, routed, counts, tiles, bound)

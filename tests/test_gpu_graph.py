@@ -41,3 +41,26 @@ def test_captured_launches_replay_the_eager_result():
         torch.cuda.synchronize()
         assert torch.equal(st["mid_store"].view(torch.int16), want_mid.view(torch.int16)), f"gate_up outputs, replay {replay}"
         assert torch.equal(st["out_store"].view(torch.int16), want_out.view(torch.int16)), f"down outputs, replay {replay}"
+
+
+@pytest.mark.parametrize("mix", ["wxax", "all"])
+def test_captured_layer_on_the_kernels_for_few_rows(mix):
+    """A whole captured forward on kernels with narrow tiles: every replay the eager result, with routings that the capture has not seen and
+    eager work between the replays."""
+    from test_gpu_short_forward import _few_layer
+
+    cfg, layer, hidden, ids, w = _few_layer(48, mix, 512)
+    captured = layer.capture(cfg.tokens)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    for replay in range(5):
+        want = layer.call_with_host_tables(hidden, ids, w)
+        captured.hidden.copy_(hidden)
+        captured.topk_ids.copy_(ids)
+        captured.topk_weights.copy_(w)
+        captured.out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        got = captured.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want), f"replay {replay}"
+        ids = torch.randint(0, cfg.num_experts + (replay == 2), ids.shape, generator=gen, device="cuda", dtype=torch.int32)  # (one with dropped entries)
+        hidden = torch.randn(hidden.shape, generator=gen, device="cuda", dtype=torch.float16)

@@ -196,6 +196,35 @@ def test_device_planner_agrees_on_lists_of_long_problems(case):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kernel", ["groupgemm_hz_fused_wxax_few", "groupgemm_hz_fused_all_few"])
+@pytest.mark.parametrize("n,experts,shared", [(4096, 8, 0), (4096, 9, 0), (2048, 7, 100), (512, 63, 33)])
+def test_device_planner_agrees_on_launches_of_few_blocks(kernel, n, experts, shared):
+    """The same comparison on the kernels with narrow tiles, at and past 128 blocks of 256 channels: problems of more than 32 rows."""
+    from mxmoe_amd import _lib
+
+    lib = _lib.load()
+    kid = lib.mxmoe_find_kernel(kernel.encode())
+    fmts = [(4, 4, -1, True), (8, 8, -1, True)] + ([(16, 4, 128, False)] if "all" in kernel else [])
+    rows = [(45, 30, 64, 1, 129, 33, 16, 100)[i % 8] for i in range(experts)]
+    qs = [fmts[i % len(fmts)] for i in range(experts + (shared > 0))]
+    ks = [2048] * experts + [4096] * (shared > 0)
+    et = len(ks)
+    desc = (_lib.BlockDesc * et)(*[_lib.BlockDesc(q[0], q[1], q[2], int(q[3]), (C.c_uint8 * 3)(), n, k, 0, 0) for q, k in zip(qs, ks)])
+    d_desc = torch.frombuffer(bytearray(bytes(desc)), dtype=torch.uint8).cuda()
+    recv = torch.tensor(rows, dtype=torch.int64, device="cuda")
+    plan = torch.zeros(lib.mxmoe_plan_bytes(et), dtype=torch.uint8, device="cuda")
+    some = torch.zeros(16, dtype=torch.uint8, device="cuda")
+    _lib.check(lib, lib.mxmoe_plan_block(kid, recv.data_ptr(), experts, shared, d_desc.data_ptr(), desc, some.data_ptr(), some.data_ptr(), some.data_ptr(), plan.data_ptr(),
+                                         torch.cuda.current_stream().cuda_stream))
+    _, host = _tables(lib, kid, [((m, n, k), q) for m, k, q in zip(rows + [shared] * (shared > 0), ks, qs)])
+    ne, tiles, nph, grid = host[:4]
+    hdr = plan.cpu().numpy()[:4096].view(np.int32)[14:]
+    assert list(hdr[:4]) == [0, ne, tiles, nph] and grid <= lib.mxmoe_plan_grid_bound(kid, desc, experts, sum(rows), shared)
+    assert np.array_equal(hdr[4:5 + nph], host[4:5 + nph]) and np.array_equal(hdr[13:14 + nph], host[13:14 + nph])
+    assert np.array_equal(hdr[23:23 + 4 * ne], host[22:22 + 4 * ne])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("routed", [False, True])
 def test_layer_whose_tokens_all_go_to_its_shared_expert(routed):
     """No expert id in range (or of one slot only): the shared expert is alone in its launches, in the device's plan and in the host's."""

@@ -49,6 +49,38 @@ def test_short_forward_equals_the_forward_with_host_tables(tokens, mix):
     _check(cfg, layer, drop=tokens > 1)
 
 
+def _few_layer(tokens, mix, inter, hidden=512):
+    """A layer of ten to twelve experts and a shared one on the kernels made for few rows, its routing drawn to one expert (up to all of the tokens: several narrow row tiles)."""
+    from mxmoe_amd import _lib
+    from mxmoe_amd import synth as S
+
+    fm = {"wxax": [(S.W4A4, S.W8A8), (S.W8A8, S.W4A4), (S.W4A4, S.W4A4), (S.W8A8, S.W8A8)],
+          "all": [(S.W4A4, S.W8A8), (S.W8A8, S.W4A16), (S.W4A16, S.W4A4), (S.W3A16, S.W8A8), (W8A16, S.W2A16)]}[mix]
+    fm = fm * (12 // len(fm)) + fm[:1]
+    cfg, layer = _layer(tokens, 2, fm, hidden=hidden, inter=inter)
+    lib = _lib.load()
+    desc = layer._block_descs(layer.qp_gate_up, [2 * inter] * len(fm), [hidden] * len(fm), layer.w13, False)
+    kid = lib.mxmoe_plan_select_kernel_rows(desc, cfg.num_experts, tokens, cfg.topk, tokens)
+    assert lib.mxmoe_kernel_name(kid).decode().endswith(f"groupgemm_hz_fused_{mix}_few")
+    hidden_t = S.make_hidden(cfg).cuda()
+    ids, w = S.make_routing(cfg)
+    ids = ids.cuda()
+    ids[:, 0] = 1                                                       # (expert 1 may be in a token's list twice: it gets both rows)
+    ids[:tokens // 4, 0] = 0
+    return cfg, layer, hidden_t, ids, w.cuda()
+
+
+# tokens: one row; the last that fits one narrow row tile; one more (two row tiles of narrow tiles: few blocks); the most those kernels take
+@pytest.mark.parametrize("tokens,inter", [(1, 1408), (24, 1408), (32, 1408), (33, 512), (64, 512)])
+@pytest.mark.parametrize("mix", ["wxax", "all"])
+def test_short_forward_on_the_kernels_for_few_rows(tokens, inter, mix):
+    """Their gate_up form (rows gathered by token, silu(gate) * up as output) with every format that they hold beside each other."""
+    cfg, layer, hidden, ids, w = _few_layer(tokens, mix, inter)
+    assert layer._short_setup(cfg.tokens, cfg.topk) is not None
+    want = layer.call_with_host_tables(hidden, ids, w)
+    assert torch.equal(layer(hidden, ids, w), want)
+
+
 @pytest.mark.parametrize("hidden,inter,num_shared,rotate", [(1024, 224, 0, 2), (2048, 64, 2, 0), (4096, 96, 1, 0), (512, 32, 0, 0)])
 def test_short_forward_row_lengths_and_rotations(hidden, inter, num_shared, rotate):
     """Every row length of the head's token kernel; intermediate sizes that end inside a tile's gate half."""
