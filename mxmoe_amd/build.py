@@ -28,7 +28,7 @@ HIPCC_FLAGS = [
 
 
 def check_no_spills(remarks: str) -> None:
-    """Refuse a build in which a WxAxTile kernel spills vector registers.
+    """Refuse a build in which a kernel of a tile with hand-tracked loads (WxAxTile, WxAxNarrowTile, Bf6Tile) spills vector registers.
 
     Those tiles load weight fragments with loads the compiler does not track (the waits are placed by hand): a fragment register
     that the compiler spills or re-uses while its load is in flight is overwritten when the load lands, and when that register
@@ -40,7 +40,7 @@ def check_no_spills(remarks: str) -> None:
             name = m.group(1)
             continue
         m = re.search(r"remark:\s+VGPRs Spill: (\d+)", line)
-        if m and name and ("WxAxTile" in name or "Bf6Tile" in name) and int(m.group(1)) > 0:
+        if m and name and any(t in name for t in ("WxAxTile", "WxAxNarrowTile", "Bf6Tile")) and int(m.group(1)) > 0:
             raise RuntimeError(f"{name}: {m.group(1)} vector registers spilled in a kernel with hand-tracked loads; shrink the tile's "
                                f"register ring or lower its waves per SIMD")
 

@@ -313,6 +313,17 @@ def test_build_refuses_spilling_wxax_kernels():
         check_no_spills(fmt.format("_ZN5mxmoe8WxAxTileILi1EEE", 45))
 
 
+@pytest.mark.parametrize("tile", ["14WxAxNarrowTileILNS_2OpE0EEE", "8Bf6TileILi64EEE"])
+def test_build_refuses_spilling_kernels_of_every_tile_with_hand_tracked_loads(tile):
+    """A single-tile kernel names no other tile that would have it checked."""
+    from mxmoe_amd.build import check_no_spills
+
+    fmt = "t.hpp:1:1: remark: Function Name: _ZN5mxmoe{} [-Rpass-analysis=kernel-resource-usage]\nt.hpp:1:1: remark:     VGPRs Spill: {} [-Rpass-analysis=kernel-resource-usage]\n"
+    check_no_spills(fmt.format(tile, 0))
+    with pytest.raises(RuntimeError, match="spilled"):
+        check_no_spills(fmt.format(tile, 1))
+
+
 def test_build_refuses_moves_of_registers_with_loads_in_flight():
     """The build's ISA check: a register written by a hand-tracked (inline-assembly) load may not be moved before the wait that names it."""
     from mxmoe_amd.build import check_untracked_load_copies as chk
