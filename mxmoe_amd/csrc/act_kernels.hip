@@ -1314,15 +1314,18 @@ __global__ void __launch_bounds__(256) row_quant_dense_kernel(const RowArgs a) {
 // them to fill the chip.  The Sylvester part runs in registers (a k row is at most 16 lanes long).  The snapped row goes to LDS as it is, [block of kb k
 // rows][k][column]; a wave gathers the second operand of 16 columns from there, two bytes per read, multiplies B (first operand, in LDS in operand
 // order) into them, and the results return through LDS in row order.  Arithmetic of the other row kernels, bit for bit.
+// (a k row's pitch is 8 modulo 16 for m > 8, so its chunks are 8-byte aligned and no more)
+typedef v8h RowChunk __attribute__((aligned(8)));
 struct BlockRows {  // LDS of a workgroup, in bytes
   int kb, m, f, ksteps, mblocks;
   int pitch;   // k row of m values.  m > 8: 8 k rows are 64 bytes modulo 256, so the lane groups of a gather touch different banks
+  __host__ __device__ static constexpr int pitch_of(int m) { return m > 8 ? 2 * m + 8 : 16; }
   int blk;     // block of kb k rows of the snapped row, padded to whole k steps
   int snapped, rotated, codes;
   __host__ __device__ explicit BlockRows(const RotPlan& p) {
     kb = p.kb, m = p.m, f = p.f;
     ksteps = (kb + 31) >> 5, mblocks = (kb + 15) >> 4;
-    pitch = m > 8 ? 2 * m + 8 : 16;
+    pitch = pitch_of(m);
     blk = ksteps * 32 * pitch + (m > 8 ? 0 : 32);
     snapped = (m > 8 || f > 2 ? f : 2) * blk;  // (H_8: 16 columns are two blocks)
     rotated = f * kb * pitch + 16;             // (a slot for discarded values at the end)
@@ -1330,6 +1333,12 @@ struct BlockRows {  // LDS of a workgroup, in bytes
   }
   __host__ __device__ int lds() const { return codes + ((snapped + 15) & ~15) + ((rotated + 15) & ~15) + 2 * 12 * 4; }
 };
+constexpr bool chunks_aligned() {
+  for (int m = 8; m <= 128; m *= 2)
+    if (BlockRows::pitch_of(m) % alignof(RowChunk)) return false;
+  return true;
+}
+static_assert(chunks_aligned(), "a chunk of any k row is read and written at the alignment its type promises");
 template <int NT, int MAXC, bool SILU, bool EXT>
 __device__ __forceinline__ void row_quant_block_body(const RowArgs& a, const int wg, const int wgs, uint8_t* const lds) {
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1475,7 +1484,7 @@ __device__ __forceinline__ void row_quant_block_body(const RowArgs& a, const int
           v8h q;
 #pragma unroll
           for (int j = 0; j < 8; ++j) q[j] = (_Float16)(rintf(v[i][j] * grid.to_grid) * 0.0625f);
-          *reinterpret_cast<v8h*>(xt + at_x(c)) = q;
+          *reinterpret_cast<RowChunk*>(xt + at_x(c)) = q;
         }
       }
       __syncthreads();
@@ -1576,7 +1585,7 @@ __device__ __forceinline__ void row_quant_block_body(const RowArgs& a, const int
       for (int i = 0; i < MAXC; ++i) {
         const int c = tid + NT * i;
         if (c < nchunks) {
-          const v8h y = *reinterpret_cast<const v8h*>(yrow + at_y(c));
+          const v8h y = *reinterpret_cast<const RowChunk*>(yrow + at_y(c));
 #pragma unroll
           for (int j = 0; j < 8; ++j) v[i][j] = (float)y[j];
         }
