@@ -16,6 +16,8 @@
 #include <type_traits>
 #include <stdint.h>
 
+#include <algorithm>
+#include <climits>
 #include <cmath>
 #include <string>
 
@@ -1611,7 +1613,7 @@ __global__ void __launch_bounds__(256) row_quant_pair_kernel(const RowArgs route
   else row_quant_dense_body<MAXC, SILU, EXT>(routed, wg - shared_wgs, (int)gridDim.x - shared_wgs, plds);
 }
 // The same for few rows, one of either kind per workgroup: the chain of one row's steps is all there is.  64 shared rows of 5632 values and 256 routed ones
-// of 1408: 15.6 us in row_quant_kernel, 11.3 / 9.4 / 11.5 here with 256 / 384 / 768 threads.
+// of 1408: 15.6 us in row_quant_kernel, 11.3 / 9.4 / 11.5 here with 256 / 384 / 768 threads (row_quant_pair_kernel from there on: launch_rows_as).
 constexpr int kFewThreads = 384;
 template <int NT, int MAXC, bool SILU, bool EXT>
 __global__ void __launch_bounds__(NT) row_quant_few_kernel(const RowArgs routed, const RowArgs shared, const int shared_wgs) {
@@ -1911,10 +1913,22 @@ static bool wide_rows(const RowArgs& a) {
   return a.plan.kb > 1 && a.plan.kb <= 32 && a.plan.m == 512 && a.plan.f == 1 && a.plan_shared.n == a.plan.n && a.plan_shared.kb == a.plan.kb && a.rotate != 0;
 }
 
-// Rows that row_quant_block_kernel takes: one length of at most 6144 values (three chunks per thread).
+// Rows that row_quant_block_kernel can take: one length of at most 6144 values (three chunks per thread).
 static bool block_rows(const RowArgs& a) {
   return a.plan.kb > 1 && a.plan.kb <= 64 && a.plan.n <= 8 * 256 * 3 && a.plan.f <= 4 && a.plan.m <= 128 &&
          a.plan_shared.n == a.plan.n && a.plan_shared.kb == a.plan.kb && a.rotate != 0;
+}
+// Up to how many of such rows it is the fastest kernel.  A row costs it much the same whatever its length and kb, while the kernels that it replaces pay for both: one row
+// per wave (m = 8) and the general kernel (m > 8, n kb operations on the vector ALU).  us, older kernel -> this one, by rows:
+//   m = 8:  224 = 28 x 8, 256 rows 5.0 -> 5.1, 512 5.3 -> 6.2;  480 = 60 x 8, 256 6.3 -> 5.7, 320 6.3 -> 6.9;  1408, 256 8.0 -> 5.9, 512 8.1 -> 7.0
+//   kb 12:  192 and 1536, 256 rows 5.1 -> 5.2 and 5.8 -> 5.9, 512 5.4 -> 6.2 and 6.5 -> 7.2, 2048 7.4 -> 12.0 and 10.9 -> 14.4
+//   kb 20:  640, 512 rows 6.9 -> 6.5, 1024 7.1 -> 8.2;  2560, 512 10.0 -> 9.0, 1024 11.8 -> 12.4
+//   kb 28:  448, 512 rows 6.6 -> 6.3, 1024 7.1 -> 8.1;  896, 512 7.2 -> 6.7, 1024 7.7 -> 8.9;  1792, 1024 10.0 -> 9.5, 4096 28.9 -> 24.5
+//   above:  960 = 60 x 16, 1024 rows 11.2 -> 10.0, 4096 24.8 -> 22.9;  2816 = 4 x 44 x 16, 512 13.8 -> 9.7, 16 384 191 -> 127;  5632, 16 384 327 -> 215
+static int block_row_limit(const RotPlan& p) {
+  if (p.m == 8) return p.n > 512 ? 512 : p.kb > 32 ? 256 : 0;
+  if (p.kb < 16) return 256;
+  return p.kb < 24 || p.n * p.kb < 48 * 1024 ? 512 : INT_MAX;
 }
 
 static int rows_launched() {
@@ -1949,9 +1963,6 @@ static int launch_pair(const RowArgs& routed, const RowArgs& shared, bool dense,
   return rows_launched();
 }
 
-// Routed rows up to which one row per workgroup beats one row per wave (rows of 1408 values: 32 rows 7.8 -> 6.2 us).
-constexpr int kBlockRowsMax = 512;
-
 template <bool SILU, bool EXT>
 static int launch_rows_as(const RowArgs& a, int lds_bytes, hipStream_t s) {
   // Shared rows of another length keep the routed rows out of the kernels made for one length: both lengths' kernels side by side in one launch, or one launch
@@ -1963,9 +1974,14 @@ static int launch_rows_as(const RowArgs& a, int lds_bytes, hipStream_t s) {
     shared.R = 0;
     shared.rows = a.rows - a.R;
     shared.plan = a.plan_shared;
-    if (a.R > 0 && shared.rows <= kPairSharedRows && dense_rows(routed) && block_rows(shared)) {
-      const bool few = a.R <= kBlockRowsMax;
-      if (!few || block_rows(routed)) return launch_pair<SILU, EXT>(routed, shared, !few, s);
+    // Shared rows beside routed ones: up to 512, or 2304 of those that row_quant_block_kernel is fastest for in any number (us, one after the other -> side by
+    // side: 2 x 480 values 512 tokens top-6 19.1 -> 13.0, 1024 24.0 -> 21.7; 2 x 224, 512 13.3 -> 10.9, 1024 16.8 -> 18.4).  One row of either kind per workgroup up
+    // to 256 rows in all (1408 values and 4 x 1408, routed rows one per wave -> per workgroup: 252 rows 9.7 -> 8.9, 280 9.7 -> 9.8; and 2 x 1408: 280 8.2 -> 9.4, 511
+    // 8.4 -> 9.6).  Short routed rows are below kSplitSharedRows best off in the general kernel (2 x 224, 32 tokens 6.1, side by side 6.8).
+    if (a.R > 0 && dense_rows(routed) && block_rows(shared) && shared.rows <= std::min(std::max(block_row_limit(shared.plan), 512), kPairSharedRows)) {
+      const int limit = block_row_limit(routed.plan);  // (dense_rows: block_rows as well)
+      const bool few = a.R <= limit && a.rows <= 256;
+      if (few || limit > 0 || a.R >= kSplitSharedRows) return launch_pair<SILU, EXT>(routed, shared, !few, s);
     }
     if (a.R >= kSplitSharedRows || (a.R == 0 && block_rows(shared))) {
       const int rc = a.R ? launch_rows_as<SILU, EXT>(routed, lds_bytes, s) : 0;
@@ -2000,7 +2016,7 @@ static int launch_rows_as(const RowArgs& a, int lds_bytes, hipStream_t s) {
     }
     return 0;
   }
-  if (block_rows(a) && (!dense_rows(a) || a.rows <= kBlockRowsMax) && !wide_rows(a)) {
+  if (block_rows(a) && a.rows <= block_row_limit(a.plan) && !wide_rows(a)) {
     const int blds = BlockRows(a.plan).lds();
     switch ((n / 8 + 255) / 256) {
       case 1: hipLaunchKernelGGL((row_quant_block_kernel<1, SILU, EXT>), dim3(grid), dim3(256), blds, s, a); break;

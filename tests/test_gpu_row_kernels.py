@@ -62,11 +62,11 @@ def _quant_inp(k, t, topk, variant, n_sh=0):
         _check(inp[ex], sc[ex], (y if qp[ex][0] < 16 else x)[rows], qp[ex], variant, ex)
 
 
-def _silu(n, n_sh, t, variant):
+def _silu(n, n_sh, t, variant, topk=2):
     from mxmoe_amd import ops
 
     rng = np.random.default_rng(n + n_sh + t)
-    e, topk = 4, 2
+    e = 4
     ids = _ids(rng, t, e, topk)
     o_dst, _, _, o_recv = O.permute_by_expert(ids, e)
     gu = (rng.standard_normal((t * topk, 2 * n)) * 2).astype(F16)
@@ -105,6 +105,19 @@ def test_rows_by_waves_beside_shared_rows_bit_exact(n, order, variant, monkeypat
     if variant == "bf6" and n % 64:
         pytest.skip("bf6 fragments are 64 values long")
     _silu(n, 2, 270, variant)
+
+
+# the last row count of the kernel with one row per workgroup and the first of its neighbour, for each limit that row lengths lead to
+@pytest.mark.parametrize("k,rows", [(192, 256), (192, 257), (448, 512), (448, 513), (480, 256), (480, 257), (224, 16), (1408, 512), (1408, 513)])
+def test_rows_at_the_limits_between_kernels_bit_exact(k, rows):
+    _quant_inp(k, rows, 1, "")
+    _silu(k, 0, rows, "", topk=1)
+
+
+# tokens of two routed rows and a shared one of twice the length: one row of either kind per workgroup, routed rows by waves, launches after each other, any row
+@pytest.mark.parametrize("n,t", [(1408, 85), (1408, 86), (480, 85), (480, 86), (480, 129), (224, 20), (224, 256), (224, 513), (448, 256)])
+def test_shared_rows_at_the_limits_between_kernels_bit_exact(n, t):
+    _silu(n, 2, t, "")
 
 
 # table orders times H_64 and H_256, in the kernel that takes any row
