@@ -721,36 +721,57 @@ struct RowSummary {
   int live = 0, tall = 0;         // problems; those of more than 16 rows
   long rows = 0, max_rows = 0;
   long blocks = 0;                // of 256 channels
-  bool integer = false;           // w4a4 or w8a8 among them
-  void add(Fmt f, long m, uint32_t N) {
+  uint32_t max_k = 0;
+  bool w4a4 = false, w8a8 = false, other = false;  // formats among them
+  void add_format(Fmt f) { (f == Fmt::W4A4 ? w4a4 : f == Fmt::W8A8 ? w8a8 : other) = true; }
+  void add(Fmt f, long m, uint32_t N, uint32_t K) {
     if (m == 0) return;
+    add_format(f);
     ++live;
     tall += m > 16;
     rows += m;
     max_rows = std::max(max_rows, m);
     blocks += (N + 255) / 256;
-    integer = integer || f == Fmt::W4A4 || f == Fmt::W8A8;
+    max_k = std::max(max_k, K);
   }
 };
 inline RowSummary row_summary(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int count) {
   RowSummary s;
-  for (int i = 0; i < count; ++i) s.add(classify(h_q[i]), h_sizes[i].x, h_sizes[i].y);
+  for (int i = 0; i < count; ++i) s.add(classify(h_q[i]), h_sizes[i].x, h_sizes[i].y, h_sizes[i].z);
   return s;
 }
 
-//
 // Lists of few rows with w4a4 or w8a8 problems go to the kernels that hold the narrow integer tile (WxAxNarrowTile, for problems of up to 32 rows; more take
-// 64-row tiles): no problem above 64 rows, 24 per problem on average, and at most 768 blocks of 256 channels over all problems.  A whole layer, us, w4a4 / w8a8
-// half and half, before -> with these kernels: 60 experts top-4 38 -> 28 (1 token), 53 -> 51 (8), 88 -> 77 (32), 98 -> 92 (64); 64 experts top-6 and a shared one
-// 46 -> 34 (1), 74 -> 68 (8), 111 -> 107 (32), 115 -> 110 (64; under a skewed routing 103 -> 106); 8 experts of N = 28 672 / 4096, K = 4096 / 14 336, whose
-// second block alone is within the limit, 103 -> 71 (1), 223 -> 191 (8), 230 -> 200 (64).  Beyond: 128 tokens of the second with its shared expert 118 -> 119, skewed
-// 117 -> 125; the first block of the third (896 blocks of 256 channels, enough for the wide tiles to fill the chip) on them too, w4a4 150 -> 160 (16 tokens).
+// 64-row tiles): no problem above 64 rows, at most 768 blocks of 256 channels over all problems, and few rows per problem on average.  A narrow tile reads the rows
+// of its problem as often as there are 64-channel columns, so it loses with rows what it gains where the wide tiles leave the chip idle: by blocks, in rounds of 256 or 512
+// workgroups.  One launch over weights from memory, time against the wide kernel's (w4a4 / w8a8 / half and half, then a third weight-only):
+//   64 .. 128 blocks:              2 .. 24 rows 0.43 .. 0.96;  one problem of 48 rows 0.58 .. 0.97
+//   132 .. 256 blocks:             8 rows 0.83 .. 1.05, 12 0.84 .. 1.08, 24 0.89 .. 1.20;  one problem of 36 rows 1.04 .. 1.45 (its 64-row tile is what the launch waits for)
+//   K = 1408, 320 blocks:          8 rows 0.95 / 0.86 / 0.93, 12 0.95 / 0.90 / 0.95, 24 1.04 / 1.01 / 1.06;  with weight-only 192 and 256 blocks, 16 rows 0.90 and 0.95
+//   K = 1408, 480 and 512 blocks:  4 rows 1.03, 1.06 / 0.97, 0.97 / 1.01, 1.01, 8 1.05, 1.09 / 1.03, 1.05 / 1.05, 1.06, 24 1.20 .. 1.26;  with weight-only 1.07 .. 1.11 at 1 .. 24
+//   K = 2048, 660 blocks:          8 rows 0.97 / 0.96 / 0.93, 12 1.00 / 1.00 / 0.96, 16 1.03 / 1.03 / 0.98, 24 1.11 / 1.11 / 1.02;  with weight-only, 16 rows 0.98, 24 1.10
+//   K = 4096, 448 blocks:          8 rows 0.97 / 0.94 / 0.99, 12 1.01 / 0.94 / 0.98, 16 1.05 / 0.96 / 1.00, 24 1.11 / 1.02 / 1.06;  with weight-only, 16 rows 0.99, 24 1.06
+// Whole layers, planned, us, wide -> as chosen here: 60 experts top-4, w4a4 / w8a8 half and half 45 -> 35 (1 token), 65 -> 58 (8), 99 -> 89 (32), 106 -> 97 (64); with a shared
+// expert of four times the width 58 -> 42 (1), 80 -> 70 (8), 122 -> 120 (64), under a skewed routing 93 -> 98 (32), 113 -> 114 (64); 64 experts top-6 and a shared one 50 -> 41 (1), 81 -> 74 (8),
+// 117 -> 110 (32), 121 -> 117 (64), skewed 112 -> 119 (64: the planned forward does not know its routing); 8 experts of N = 28 672 / 4096, K = 4096 / 14 336, whose second
+// block alone is within the limit of blocks, 126 -> 94 (1), 230 -> 199 (8), 240 -> 209 (64).  More than 768 blocks: lists of 770 .. 902 at 8 rows 0.91 .. 1.01, but the gate_up form of those 8
+// experts' first block (896) 1.00 .. 1.05 in w4a4 layers of 1 .. 32 tokens, 1.12 skewed.
 // A 128-row tile beside them would take the third workgroup of a CU (244 registers, 161 without): 60 experts 77 -> 83 (32).
-// (From 8 blocks on: the planning rules for long problems are stated, and tested, on lists of two or three small problems in the wide shapes.)
-constexpr int kFewRows = 24, kFewRowsMax = 64, kFewBlocks = 768, kFewBlocksMin = 8;
+// (Launches of fewer than 8 blocks would run at 0.35 .. 0.6 of the wide kernel's time as well; the planning rules for long problems are stated, and tested, on lists of two or three
+// small problems in the wide shapes.)
+constexpr int kFewRowsMax = 64, kFewBlocks = 768, kFewBlocksMin = 8;
 inline bool holds_narrow(const FusedKernel& k) { return plan_of(k).narrow; }
+// Rows per problem, on average, up to which those kernels are chosen.
+inline int few_rows_limit(const RowSummary& s) {
+  if (s.blocks <= kPoleBlocks) return 24;
+  if (s.max_k < 2048 && s.blocks > 384) return s.other ? 2 : 5;
+  if (s.other || (s.w4a4 && s.w8a8 && s.max_k >= 2048)) return 16;
+  return s.max_k < 2048 ? 8 : 12;
+}
 inline bool few_rows(const RowSummary& s) {
-  return s.integer && s.max_rows <= kFewRowsMax && s.rows <= kFewRows * s.live && s.blocks >= kFewBlocksMin && s.blocks <= kFewBlocks;
+  if (!(s.w4a4 || s.w8a8) || s.max_rows > kFewRowsMax || s.blocks < kFewBlocksMin || s.blocks > kFewBlocks) return false;
+  if (s.blocks > kPoleBlocks && s.blocks <= 256 && s.max_rows > 32) return false;
+  return s.rows <= few_rows_limit(s) * s.live;
 }
 // A list of weight-only problems of few rows takes a kernel made of 16-row few-token tiles (FusedKernel::max_rows_hint), unless more than a quarter of its
 // problems need several of them: then the kernels that also hold the 32-row few-token tile do better, whatever the largest count.

@@ -191,10 +191,10 @@ int mxmoe_plan_select_kernel_rows(const mxmoe_block_desc* h_desc, int num_expert
   RowSummary s;
   for (int i = 0; i < num_experts; ++i) {
     const mxmoe_block_desc& d = h_desc[widest[i]];
-    s.add((Fmt)fmt_of(d.q), i < live ? routed / live + (i < routed % live) : 0, d.N);
-    s.integer = s.integer || fmt_of(d.q) == (int)Fmt::W4A4 || fmt_of(d.q) == (int)Fmt::W8A8;  // (any of them may get rows)
+    s.add((Fmt)fmt_of(d.q), i < live ? routed / live + (i < routed % live) : 0, d.N, d.K);
+    s.add_format((Fmt)fmt_of(d.q));  // (any of them may get rows)
   }
-  if (shared_rows > 0) s.add((Fmt)fmt_of(h_desc[num_experts].q), shared_rows, h_desc[num_experts].N);
+  if (shared_rows > 0) s.add((Fmt)fmt_of(h_desc[num_experts].q), shared_rows, h_desc[num_experts].N, h_desc[num_experts].K);
   s.max_rows = std::max<long>(s.max_rows, num_tokens);  // one expert may get them all
   // an uneven routing has problems of several 16-row tiles well before the average reaches 16
   if (routed > 12l * num_experts) s.tall = s.live;

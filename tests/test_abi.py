@@ -346,15 +346,33 @@ def test_lists_of_few_rows_take_the_kernels_with_narrow_tiles():
     assert picked(*[(1, 2048, w4)] * 96) == "hz_fused_wxax_few" and picked(*[(1, 2048, w4)] * 97) == "hz_fused_wxax"
 
 
+W4, W8, WO4, WO3, FP = (4, 4, -1, True), (8, 8, -1, True), (16, 4, 128, False), (16, 3, 128, False), (16, 16, -1, True)
+
+
+# (problems, channels, K), formats, the most rows per problem that go to the narrow tiles
+@pytest.mark.parametrize("count,n,k,formats,most", [
+    (16, 2048, 1408, "48", 24), (17, 2048, 1408, "48", 8), (48, 2048, 1408, "4", 8), (49, 2048, 1408, "4", 5), (60, 2048, 1408, "48", 5), (48, 2048, 1408, "48o", 16), (60, 2048, 1408, "48o", 2),
+    (60, 2816, 2048, "4", 12), (60, 2816, 2048, "8", 12), (60, 2816, 2048, "48", 16), (60, 2816, 2048, "48o", 16), (8, 14336, 4096, "8", 12), (8, 4096, 14336, "4", 24)])
+def test_rows_up_to_which_lists_take_the_kernels_with_narrow_tiles(lib, count, n, k, formats, most):
+    qs = [{"4": W4, "8": W8, "o": WO4}[f] for f in formats]
+
+    def picked(rows):
+        rc, _, _ = _plan(lib, -1, [((m, n, k), qs[i % len(qs)]) for i, m in enumerate(rows)])
+        return lib.mxmoe_kernel_name(rc - 1000).decode().endswith("_few")
+
+    assert picked([most] * count)
+    assert not picked([most] * (count - 1) + [most + 1])
+    if most < 24:                                                       # one problem above 32 rows: not among the launches that a 64-row tile would hold up
+        few_blocks = count * -(-n // 256) <= 256
+        assert picked([33] + [1] * (count - 1)) is not few_blocks and picked([32] + [1] * (count - 1))
+
+
 def _blocks(formats, n, k, shared=None):
     """Host block descriptors: experts of the given formats, and a shared expert (format, N, K)."""
     from mxmoe_amd import _lib
 
     rows = [(q, n, k) for q in formats] + ([shared] if shared else [])
     return (_lib.BlockDesc * len(rows))(*[_lib.BlockDesc(q[0], q[1], q[2], int(q[3]), (C.c_uint8 * 3)(), nn, kk, 0, 0) for q, nn, kk in rows])
-
-
-W4, W8, WO4, WO3, FP = (4, 4, -1, True), (8, 8, -1, True), (16, 4, 128, False), (16, 3, 128, False), (16, 16, -1, True)
 
 
 @pytest.mark.parametrize("formats", [[W4], [W8], [W4, W8], [WO4, WO3], [W4, W8, WO4], [FP], [W4, FP]])
