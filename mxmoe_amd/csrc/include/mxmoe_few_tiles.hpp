@@ -2,8 +2,8 @@
 //
 // 32 tokens x 64 channels per workgroup, K dealt to the four waves in contiguous quarters, against 32 x 256 with all of K per wave (WxAxTile): four times the
 // workgroups and a quarter of the steps in each, for problems whose weight stream is all there is.  The 128 workgroups that the wide tile makes of eight
-// experts of N = 4096, K = 14336 leave half of the CUs idle and take 82 us in w8a8, whatever the number of tokens; whole layers with either tile: few_rows in
-// mxmoe_launch.hpp.  The partial sums are integers: the same result in any order.
+// experts of N = 4096, K = 14336 leave half of the CUs idle: w4a4 and w8a8 half and half 90 us whatever the number of tokens, 62 here (w8a8 alone 97 -> 82, w4a4
+// 56 -> 44); by blocks, rows and formats, and for whole layers: few_rows in mxmoe_launch.hpp.  The partial sums are integers: the same result in any order.
 //
 // A wave streams the fragments of its channels (64 bytes of K of 32 channels are 2 KB, WxAxTile's layout) and of all 32 token rows straight into registers, kAhead
 // K slices ahead, without LDS or barriers; every load is an untracked one (gload16_untracked) awaited with the exact number of younger loads.  Rows past M
@@ -82,7 +82,7 @@ struct WxAxNarrowTile {
     };
     int sa_bits = 0;
     const int klast = max(k1 - 1, 0);
-    // (a wave without slices loads slice 0 of its tile and multiplies nothing)
+    // (a wave without slices loads the last slice of K and multiplies nothing)
     static_for<kAhead>([&](auto dc) {
       constexpr int d = decltype(dc)::value;
       load_w(dc, min(k0 + d, klast));

@@ -303,10 +303,10 @@ struct BranchOf<Bf6Tile<BM>> {
     return BranchInfo{Fmt::W4A4, BM, T::BN, T::BK, 1, 4, T::kLdsBytes, 128, 0, 256, kVariantBf6};
   }
 };
-template <int WBITS, int BN, int KP, int RING, int WAVES, int MB>
-struct BranchOf<SkinnyWoTile<WBITS, BN, KP, RING, WAVES, MB>> {
+template <int WBITS, int BN, int MB, int WAVES>
+struct BranchOf<SkinnyWoTile<WBITS, BN, MB, WAVES>> {
   static BranchInfo get() {
-    using T = SkinnyWoTile<WBITS, BN, KP, RING, WAVES, MB>;
+    using T = SkinnyWoTile<WBITS, BN, MB, WAVES>;
     return BranchInfo{WBITS == 8 ? Fmt::W8A16 : WBITS == 4 ? Fmt::W4A16 : WBITS == 3 ? Fmt::W3A16 : Fmt::W2A16, T::BM, BN, 128, 1, 4, T::kLdsBytes, 128, 0};
   }
 };
@@ -359,7 +359,8 @@ struct BranchOf<WoMfmaTile<WBITS, BM, BN>> {
 // well; the weight-only entries compare the skinny streaming tile with the 128 x 128 dequantise-to-fp16 tile (the 128 x 256
 // one, four waves side by side with twice the tokens each, does twice the work in 1.5 times the time).
 // The 32-token few-token tile costs the same for every bit width (it waits for memory, not for bytes), and two of them must not
-// look cheaper than one 128 x 256 tile, which runs half its loop for a problem of 33 .. 64 rows.
+// look cheaper than one 128 x 256 tile, which runs half its loop for a problem of 33 .. 64 rows.  (Its 4-, 3- and 2-bit entries are from before it walked K as
+// one stream, which took a fifth off its time: what 33 .. 128 rows run on has not been weighed again since.)
 inline double tile_cost(const BranchInfo& b) {
   struct Row { Fmt f; int bm, bn; double c; };
   static const Row table[] = {

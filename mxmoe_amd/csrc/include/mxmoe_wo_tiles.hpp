@@ -38,19 +38,19 @@ namespace mxmoe {
 // twice as long).
 // 4, 3 and 2 bits: a wave walks its K range as one stream (stream()), with as many packed blocks in flight as the tile has channel blocks.
 // 8 bits, whose packed blocks take twice the registers: in passes (pass()) of KP k blocks (128 wide), whose activations live in registers, with
-// RING packed blocks in flight; the activations of a pass take MB times the registers, which is why KP shrinks as MB grows.
+// kRing packed blocks in flight; the activations of a pass take MB times the registers, which is why both shrink as MB grows.
 // The stream replaced passes for every width but 8 (there it spills at 32 tokens and gains nothing at 16).  A pass starts with an empty ring and waits
 // out a memory latency, two or more times per tile.  64 problems of N = 2816, K = 2048, us, pass -> stream: 24 tokens w4 57 -> 45, w3 57 -> 44, w2
 // 53 -> 41; 16 tokens and fewer the same there, but 23 -> 20 at N = 2048, K = 1408 (w4, 3 tokens: waves of 3, 3, 3 and 2 k blocks).
-template <int WBITS_, int BN_, int KP_ = 4, int RING_ = (WBITS_ == 8 ? 6 : 12), int WAVES_ = 2, int MB_ = 1>
+template <int WBITS_, int BN_, int MB_ = 1, int WAVES_ = 2>
 struct SkinnyWoTile {
   static constexpr int WBITS = WBITS_, MB = MB_, BM = 16 * MB_, BN = BN_;
   static_assert(WBITS == 8 || WBITS == 4 || WBITS == 3 || WBITS == 2, "w8 / w4 / w3 / w2");
   static_assert(BN % 64 == 0, "the final reduction deals 16-channel blocks to 4 waves");
   static constexpr int NB = BN / 16;                 // 16-channel blocks per tile
-  static constexpr int KP = KP_;                     // k blocks (128 wide) per pass of a wave: their activations live in registers
   static constexpr int kRedBytes = kWaves * NB * MB * 64 * 16;  // per-wave partial sums for the final reduction
   static constexpr bool kStream = WBITS != 8;                 // stream() instead of pass()
+  static constexpr int KP = MB == 1 ? 4 : 2, kRing = MB == 1 ? 6 : 4;  // of pass()
   static constexpr int kChunk = kStream ? 4 : KP;              // k blocks whose (scale, zero) pairs a wave holds at a time
   static constexpr int kScaleBytes = NB * kChunk * 64;        // its patch for them
   static constexpr int kLdsBytes = kRedBytes + kWaves * kScaleBytes;
@@ -59,7 +59,6 @@ struct SkinnyWoTile {
   static constexpr int kABits = 16, kWBits = WBITS;  // fp16 activations, packed weights
   static constexpr int kLaneBytes = WBITS * 4;       // packed bytes per lane per (channel block, k block)
   static constexpr int kBlockBytes = 64 * kLaneBytes;
-  static constexpr int kRing = RING_;                // packed blocks in flight per wave (12 KB by default)
 
   struct WReg {
     int d[WBITS];
@@ -145,7 +144,7 @@ struct SkinnyWoTile {
   // One pass of a wave: NKB (<= KP) consecutive k blocks starting at kb0, against all NB channel blocks of the tile.
   // The wave's activations of these k blocks are loaded once into registers and its (scale, zero) pairs into a private LDS
   // patch; the packed weight blocks then stream through a ring of kRing register buffers with no barrier in the loop, so
-  // kRing KB per wave are always in flight.  The sums: see stream().
+  // kRing blocks of 2 KB per wave are always in flight.  The sums: see stream().
   template <bool GU, int NKB>
   __device__ static __forceinline__ void pass(const TileArgs& t, int kb0, int m0, int n0, int nbv, int lane, const int (&src)[MB], uint8_t* __restrict__ spatch, v4f (&acc)[NB][MB]) {
     const int K = t.K, KB = K / 128;

@@ -221,10 +221,8 @@ class TileConfig:
     def cpp_type(self) -> str:
         """The C++ tile type this descriptor instantiates."""
         if self.is_skinny():
-            if self.BM == 32:  # two blocks of 16 tokens against every unpacked weight: 2 k blocks per pass, 8 (8-bit: 4) packed blocks in flight
-                return f"SkinnyWoTile<{self.QCFGB.QBITS}, {self.BN}, 2, {4 if self.QCFGB.QBITS == 8 else 8}, 2, 2>"
-            # STAGE 4: compiled for 3 waves per SIMD (the two numbers in front count for 8-bit weights only)
-            return f"SkinnyWoTile<{self.QCFGB.QBITS}, {self.BN}, 2, 4, 3>" if self.STAGE == 4 else f"SkinnyWoTile<{self.QCFGB.QBITS}, {self.BN}>"
+            # <bits, channels, blocks of 16 tokens, waves per SIMD it is compiled for (STAGE 4: 3)>
+            return f"SkinnyWoTile<{self.QCFGB.QBITS}, {self.BN}, {self.BM // 16}, {3 if self.STAGE == 4 else 2}>"
         if self.is_weight_only():
             return f"WoMfmaTile<{self.QCFGB.QBITS}, {self.BM}, {self.BN}>"
         if self.is_bf6():

@@ -165,9 +165,9 @@ def test_layers_the_short_form_does_not_take():
         assert torch.equal(layer(hidden_t, ids, w), layer.call_with_host_tables(hidden_t, ids, w))
 
 
-@pytest.mark.parametrize("num_bytes", [4, 3584, 3588, 10000])
+@pytest.mark.parametrize("num_bytes", [4, 3584, 3588, 4032, 4036, 8064, 10000])
 def test_upload_in_kernel_arguments(num_bytes):
-    """Host tables of less than one, exactly one and several launches' arguments; the bytes behind them stay as they were."""
+    """Host tables of less than one, exactly one (4032 bytes) and several launches' arguments; the bytes behind them stay as they were."""
     import numpy as np
 
     from mxmoe_amd import _lib
