@@ -1613,7 +1613,7 @@ __global__ void __launch_bounds__(256) row_quant_pair_kernel(const RowArgs route
   else row_quant_dense_body<MAXC, SILU, EXT>(routed, wg - shared_wgs, (int)gridDim.x - shared_wgs, plds);
 }
 // The same for few rows, one of either kind per workgroup: the chain of one row's steps is all there is.  64 shared rows of 5632 values and 256 routed ones
-// of 1408: 15.6 us in row_quant_kernel, 11.3 / 9.4 / 11.5 here with 256 / 384 / 768 threads (row_quant_pair_kernel from there on: launch_rows_as).
+// of 1408: 15.6 us in row_quant_kernel, 11.3 / 9.4 / 11.5 here with 256 / 384 / 768 threads.
 constexpr int kFewThreads = 384;
 template <int NT, int MAXC, bool SILU, bool EXT>
 __global__ void __launch_bounds__(NT) row_quant_few_kernel(const RowArgs routed, const RowArgs shared, const int shared_wgs) {
@@ -1976,11 +1976,12 @@ static int launch_rows_as(const RowArgs& a, int lds_bytes, hipStream_t s) {
     shared.plan = a.plan_shared;
     // Shared rows beside routed ones: up to 512, or 2304 of those that row_quant_block_kernel is fastest for in any number (us, one after the other -> side by
     // side: 2 x 480 values 512 tokens top-6 19.1 -> 13.0, 1024 24.0 -> 21.7; 2 x 224, 512 13.3 -> 10.9, 1024 16.8 -> 18.4).  One row of either kind per workgroup up
-    // to 256 rows in all (1408 values and 4 x 1408, routed rows one per wave -> per workgroup: 252 rows 9.7 -> 8.9, 280 9.7 -> 9.8; and 2 x 1408: 280 8.2 -> 9.4, 511
-    // 8.4 -> 9.6).  Short routed rows are below kSplitSharedRows best off in the general kernel (2 x 224, 32 tokens 6.1, side by side 6.8).
+    // to 512 rows in all, 256 with the SiLU (routed rows one per wave -> per workgroup: finished rows inside a planned forward, 4 x 1408 values beside, 280 rows 10.9 -> 10.0,
+    // 500 11.3 -> 10.1, 600 11.3 -> 11.7; 2 x 1408, 448 9.7 -> 9.2, 560 9.9 -> 11.3; with the SiLU, launches back to back, 4 x 1408 252 9.7 -> 8.9, 280 9.7 -> 9.8; 2 x 1408
+    // 280 8.2 -> 9.4, 511 8.4 -> 9.6).  Short routed rows are below kSplitSharedRows best off in the general kernel (2 x 224, 32 tokens 6.1, side by side 6.8).
     if (a.R > 0 && dense_rows(routed) && block_rows(shared) && shared.rows <= std::min(std::max(block_row_limit(shared.plan), 512), kPairSharedRows)) {
       const int limit = block_row_limit(routed.plan);  // (dense_rows: block_rows as well)
-      const bool few = a.R <= limit && a.rows <= 256;
+      const bool few = a.R <= limit && a.rows <= (SILU ? 256 : 512);
       if (few || limit > 0 || a.R >= kSplitSharedRows) return launch_pair<SILU, EXT>(routed, shared, !few, s);
     }
     if (a.R >= kSplitSharedRows || (a.R == 0 && block_rows(shared))) {
