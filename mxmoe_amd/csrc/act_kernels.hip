@@ -1887,7 +1887,9 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
 }
 
 constexpr int kSplitSharedRows = 512;
-constexpr int kPairSharedRows = 2304;  // (row_quant_pair_kernel)
+// Shared rows up to which row_quant_pair_kernel takes them (us, 2304 in it / 2305 in launches after one another, six routed rows of 1408 values each: 2 x 1408 65.5 / 65.3,
+// 4 x 1408 71.0 / 80.2; side by side beyond it has been timed with older shared-row code only).
+constexpr int kPairSharedRows = 2304;
 
 static int make_plan(int n, int had_k, int had_f, bool rotate, RotPlan* p) {
   p->n = n;
