@@ -779,7 +779,8 @@ inline bool few_rows(const RowSummary& s) {
 // Of those kernels, the one of 64-channel tiles against that of 128: twice the workgroups, 125 registers (four workgroups per CU) against 164.
 // Up to 6 rows per problem on average; the activations, read once per tile, weigh more with more.  A whole layer, us, 128 -> 64 channels: 64 experts top-6 and
 // a shared one, w4a16 / w3a16, 30.2 -> 28.2 (1 token), 42.7 -> 39.2 (4), 64 -> 61 (16), 75 -> 73 (64); 60 experts top-4 and a shared one 33.6 -> 29.0 (1),
-// 58 -> 51 (16); 8 experts of N = 28 672 / 4096 61.6 -> 52.1 (1), 144 -> 140 (16), but 144 -> 150 (32: 8 rows each).
+// 58 -> 51 (16); 8 experts of N = 28 672 / 4096 61.6 -> 52.1 (1), 144 -> 140 (16), but 144 -> 150 (32: 8 rows each).  (Launches of fewer than 8 blocks
+// would take 0.73 .. 0.81 of the time as well: 7 blocks of K = 2048, 1 row, 7.6 -> 5.9.)
 constexpr int kFewTokenRows = 6;
 inline bool only_narrow_few_token(const FusedKernel& k) {
   for (const BranchInfo& b : k.branches)

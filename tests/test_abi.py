@@ -317,7 +317,7 @@ def test_layer_run_wants_aligned_tokens_where_tiles_read_them_in_place(lib, a_bi
 
 
 def test_lists_of_few_rows_take_the_kernels_with_narrow_tiles():
-    """Up to 64 rows per problem, 24 on average and 768 blocks of 256 channels: on and past each limit; formats those kernels have no tile for; empty problems
+    """Up to 64 rows per problem, 24 on average (in launches of few blocks) and 768 blocks of 256 channels: on and past each limit; formats those kernels have no tile for; empty problems
     count for nothing."""
     from mxmoe_amd import _lib
 
