@@ -104,8 +104,8 @@ int mxmoe_last_status(void);
 int mxmoe_group_gemm_plan(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int problem_count, int32_t* branch_out, int32_t* tiles_out);
 
 /* The tile tables themselves (host-only; what the generated launcher keeps in its prefix-sum array, kernel_sketch.py:89-104): out receives
- * {entries, tiles, phases, workgroups}, phase_tile0[9], phase_wg0[9], then per entry {first tile, first row, rows, problem | branch << 16}.
- * At most 120 problems; used by the tests that compare the device-side planner with the host launcher. */
+ * {entries, tiles, phases, workgroups}, phase_tile0[9], phase_wg0[9], then per entry {first tile, first row, rows, problem | branch << 16 |
+ * what a pair of entries carries (bits 21 .. 31: mxmoe_launch.hpp, pair_word)}.  At most 120 problems; used by the tests that compare the device-side planner with the host launcher. */
 int mxmoe_group_gemm_plan_tables(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int problem_count, int32_t* out, int out_ints);
 
 /* The tile each workgroup of such a launch runs when the grid holds `grid` workgroups (host-only; the role of the block -> tile walk of
@@ -113,6 +113,10 @@ int mxmoe_group_gemm_plan_tables(int kernel_id, const mxmoe_dim3* h_sizes, const
  * launch is enqueued with a grid sized for the worst routing, so `grid` may exceed the workgroups the tables need; the function the
  * kernels call to find their tile is the one evaluated here. */
 int mxmoe_group_gemm_plan_tile_map(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int problem_count, int grid, int32_t* tile_of_wg);
+
+/* What each of those workgroups computes (host-only): area[5 w ..] = {problem, first row, end row, first column, end column}, or {-1, ...}
+ * for a workgroup without a tile.  The order of the tiles inside a problem is the one the kernels follow. */
+int mxmoe_group_gemm_plan_tile_area(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int problem_count, int grid, int32_t* area);
 
 /* ---- routing: what the models' gates compute between the router's logits and this layer (mxmoe/quant/moe_tracer.py:79-86:
  *      F.softmax(router_logits, dim=1, dtype=float) -> torch.topk -> optional division by the sum of the k weights) ----

@@ -80,6 +80,7 @@ SIGNATURES = {
     "mxmoe_unpermute_combine_planned": (_I, [_P, _P, _I, _P, _P, _I, _I, _I, _P, _P, _P]),
     "mxmoe_group_gemm_plan_tables": (_I, [_I, C.POINTER(Dim3), C.POINTER(QParams), _I, C.POINTER(C.c_int32), _I]),
     "mxmoe_group_gemm_plan_tile_map": (_I, [_I, C.POINTER(Dim3), C.POINTER(QParams), _I, _I, C.POINTER(C.c_int32)]),
+    "mxmoe_group_gemm_plan_tile_area": (_I, [_I, C.POINTER(Dim3), C.POINTER(QParams), _I, _I, C.POINTER(C.c_int32)]),
     "mxmoe_upload": (_I, [_P, _P, C.c_size_t, _P]),
     "mxmoe_combine_sorted": (_I, [_P, _P, _I, _I, _P, _P, _I, _I, _I, _P, _P]),
     "mxmoe_layer_supported": (_I, [_P]),
@@ -94,7 +95,7 @@ _cached = {}
 
 
 GEMM_ONLY = ("mxmoe_last_error", "mxmoe_num_kernels", "mxmoe_kernel_name", "mxmoe_find_kernel", "mxmoe_kernel_num_branches", "mxmoe_kernel_branch",
-             "mxmoe_group_gemm", "mxmoe_group_gemm_plan", "mxmoe_group_gemm_plan_tables", "mxmoe_group_gemm_plan_tile_map", "mxmoe_kernel_func", "mxmoe_get_kernel", "mxmoe_kernel_policy", "mxmoe_set_stream", "mxmoe_get_stream",
+             "mxmoe_group_gemm", "mxmoe_group_gemm_plan", "mxmoe_group_gemm_plan_tables", "mxmoe_group_gemm_plan_tile_map", "mxmoe_group_gemm_plan_tile_area", "mxmoe_kernel_func", "mxmoe_get_kernel", "mxmoe_kernel_policy", "mxmoe_set_stream", "mxmoe_get_stream",
              "mxmoe_last_status")
 
 # the reference's FuncType (registry.cuh:28-39): 15 arguments, no return value

@@ -151,4 +151,45 @@ int mxmoe_group_gemm_plan_tile_map(int kernel_id, const mxmoe_dim3* h_sizes, con
   return 0;
 }
 
+int mxmoe_group_gemm_plan_tile_area(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int problem_count, int grid, int32_t* area) {
+  auto& reg = registry();
+  if (problem_count <= 0 || problem_count > kMaxProblems || !h_sizes || !h_q || !area || grid < 0 || kernel_id < 0 || kernel_id >= (int)reg.size()) {
+    last_error() = "bad argument";
+    return 5;
+  }
+  const FusedKernel& k = reg[kernel_id];
+  FusedArgs a;
+  std::memset(&a, 0, sizeof a);
+  int planned = 0;
+  if (const int rc = build_fused_tables(k, h_sizes, h_q, 0, problem_count, a, &planned)) return rc;
+  for (int wg = 0; wg < grid; ++wg) {
+    int32_t* o = area + 5 * wg;
+    o[0] = -1;
+    const int tile = tile_of_workgroup(&a, wg);
+    if (tile < 0) continue;
+    int i = 0;
+    while (i + 1 < a.num_entries && a.entry[i + 1].first <= tile) ++i;
+    if ((unsigned)a.entry[i].problem_branch & kPairSecond) --i;
+    const int pb = a.entry[i].problem_branch, p = entry_problem(pb);
+    auto locate = [&](int local, int rows, const BranchInfo& b, int word) {
+      const int w_bits = b.fmt == Fmt::W8A16 || b.fmt == Fmt::W8A8 ? 8 : b.fmt == Fmt::FP16 ? 16 : b.fmt == Fmt::W3A16 ? 3 : b.fmt == Fmt::W2A16 ? 2 : 4;
+      return locate_tile(local, rows, (int)h_sizes[p].y, (int)h_sizes[p].z, b.BM, b.BN, is_weight_only(b.fmt) ? 16 : w_bits, w_bits, word);
+    };
+    const BranchInfo* b = &k.branches[entry_branch(pb)];
+    TileAt at = locate(tile - a.entry[i].first, a.entry[i].rows, *b, pb);
+    if (at.second) {  // as the kernels do: counted inside its own segment
+      ++i;
+      b = &k.branches[entry_branch(a.entry[i].problem_branch)];
+      at = locate(at.n * (pair_width(pb) >> ((unsigned)pb >> 30)) + at.m, a.entry[i].rows, *b, 0);
+    }
+    const FusedArgs::Entry& e = a.entry[i];
+    o[0] = p;
+    o[1] = e.row0 + at.m * b->BM;
+    o[2] = std::min(o[1] + b->BM, e.row0 + e.rows);
+    o[3] = at.n * b->BN;
+    o[4] = std::min(o[3] + b->BN, (int)h_sizes[p].y);
+  }
+  return 0;
+}
+
 }  // extern "C"

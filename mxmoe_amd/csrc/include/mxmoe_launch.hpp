@@ -57,7 +57,7 @@ struct FusedArgs {
   int phase_flat;
   // One entry per row segment of a problem, 16 bytes so that a workgroup fetches its entry with one scalar load: first tile of the
   // entry (exclusive prefix sum of tiles), first row of the segment inside its problem, rows of the segment, and
-  // problem (relative to problem_offset) | tile type << 16.
+  // problem (relative to problem_offset) | tile type << 16 | the fields of a pair (pair_word).
   struct Entry {
     int first, row0, rows, problem_branch;
   };
@@ -66,51 +66,81 @@ struct FusedArgs {
 };
 static_assert(sizeof(FusedArgs) <= 4096, "kernel arguments are limited to 4 KB");
 
-// Activation bytes that a group of row tiles may hold (see Dispatch::go): half of an XCD's 4 MB L2.
+// Activation bytes that a group of row tiles may hold (see locate_tile): half of an XCD's 4 MB L2.
 #ifndef MXMOE_GROUP_BYTES
 #define MXMOE_GROUP_BYTES (2 << 20)
 #endif
 
-template <int I, bool GU, class... Tiles>
-struct Dispatch;
-template <int I, bool GU>
-struct Dispatch<I, GU> {
-  __device__ static __forceinline__ void go(int, TileArgs&, int, uint8_t*) {}
+// A pair: the two row segments of one problem as neighbouring entries whose tiles are dealt out column by column, so that the tiles of both
+// shapes that read a block of weight rows run at the same time and the block is fetched once.  (As phases of their own, the launch went through
+// all of its weights a second time for the remainder tiles; with more weights than the caches hold, that was the launch's time.)
+// Fields of problem_branch, on both entries: bits 21 .. 28 the second segment's tiles per column tile of the first (0: no pair), bit 29 set on
+// the second entry, bits 30 .. 31 log2 of the second's column tiles per column tile of the first.
+constexpr unsigned kPairSecond = 1u << 29;
+__host__ __device__ inline int entry_problem(int pb) { return pb & 0xFFFF; }
+__host__ __device__ inline int entry_branch(int pb) { return (int)((unsigned)pb >> 16 & 31u); }
+__host__ __device__ inline int pair_width(int pb) { return (int)((unsigned)pb >> 21 & 255u); }
+
+// Where a tile of an entry (of a pair: of both entries) lies.
+struct TileAt {
+  int m, n;
+  bool second;  // in the pair's second segment
 };
-template <int I, bool GU, class T, class... Rest>
-struct Dispatch<I, GU, T, Rest...> {
-  __device__ static __forceinline__ void go(int branch, TileArgs& t, int local, uint8_t* smem) {
-    if (branch == I) {
-      // local index -> (row tile, column tile) as tile_scheduler.cuh:40-49, but row tile fastest: neighbouring workgroups then share
-      // one block of weight rows and sweep the problem's activations.  The 64 workgroups that an XCD runs at a time only share
-      // what its 4 MB L2 still holds, and they drift apart along K, so a problem whose activations exceed the L2 ends up
-      // streaming them once per column tile.  Such a problem is walked in groups of row tiles holding at most 2 MB of
-      // activations, each group against all column tiles: the group's activations stay resident whatever the drift, and a block
-      // of weights is fetched once per group by row tiles that start together.  The plain order is kept where the estimate of
-      // its traffic (activations once per 64 / grid_m column tiles, weights once) is below half of the grouped order's (weights
-      // once per group, activations once): very long rows, of which only one or two row tiles fit.
-      const int grid_m = (t.M - t.row0 + T::BM - 1) / T::BM;
-      const int grid_n = (t.N + T::BN - 1) / T::BN;
-      const int tile_bytes = max(T::BM * (t.K / 8) * T::kABits, 1);
-      int rg = min(max(MXMOE_GROUP_BYTES / tile_bytes, 1), grid_m);  // row tiles per group
-      if (rg < grid_m) {
-        const float a_bytes = (float)grid_m * (float)tile_bytes;
-        const float b_bytes = (float)t.N * (float)(t.K / 8) * (float)T::kWBits;
-        const float grouped = (float)((grid_m + rg - 1) / rg) * b_bytes + a_bytes;
-        const float plain = fmaxf((float)grid_n * (float)grid_m * (1.0f / 64.0f), 1.0f) * a_bytes + b_bytes;
-        if (grouped >= 2.0f * plain || tile_bytes > MXMOE_GROUP_BYTES) rg = grid_m;  // (a single row tile beyond the budget cannot stay resident either)
-      }
-      const int per_group = rg * grid_n;
-      const int g = local / per_group, r = local - g * per_group;
-      const int rows_g = min(rg, grid_m - g * rg);
-      t.tile_n = r / rows_g;
-      t.tile_m = g * rg + (r - t.tile_n * rows_g);
-      T::template run<GU>(t, smem);
-    } else {
-      Dispatch<I + 1, GU, Rest...>::go(branch, t, local, smem);
+// Local index -> (row tile, column tile) as tile_scheduler.cuh:40-49, but row tile fastest: neighbouring workgroups then share
+// one block of weight rows and sweep the problem's activations.  The 64 workgroups that an XCD runs at a time only share
+// what its 4 MB L2 still holds, and they drift apart along K, so a problem whose activations exceed the L2 ends up
+// streaming them once per column tile.  Such a problem is walked in groups of row tiles holding at most 2 MB of
+// activations, each group against all column tiles: the group's activations stay resident whatever the drift, and a block
+// of weights is fetched once per group by row tiles that start together.  The plain order is kept where the estimate of
+// its traffic (activations once per 64 / grid_m column tiles, weights once) is below half of the grouped order's (weights
+// once per group, activations once): very long rows, of which only one or two row tiles fit.
+// BM, BN, bits: of the entry's tile shape (of a pair: of its first segment, which the last group shares with the second).
+__host__ __device__ __forceinline__ TileAt locate_tile(int local, int rows, int N, int K, int BM, int BN, int a_bits, int w_bits, int problem_branch) {
+  const int grid_m = (rows + BM - 1) / BM;
+  const int beside = pair_width(problem_branch);
+  if (grid_m == 1 && beside == 0) return TileAt{0, local, false};
+  const int raw_bytes = BM * (K / 8) * a_bits, tile_bytes = raw_bytes > 1 ? raw_bytes : 1;
+  int g = 0, r = local, rows_g = grid_m;  // group, index inside it, its row tiles
+  bool last = true;
+  if ((long)grid_m * tile_bytes > MXMOE_GROUP_BYTES && tile_bytes <= MXMOE_GROUP_BYTES) {  // (a single row tile beyond the budget cannot stay resident either)
+    const int rg = MXMOE_GROUP_BYTES / tile_bytes, groups = (grid_m + rg - 1) / rg;
+    const int grid_n = (N + BN - 1) / BN;
+    const float a_bytes = (float)grid_m * (float)tile_bytes;
+    const float b_bytes = (float)N * (float)(K / 8) * (float)w_bits;
+    const float cols = (float)grid_n * (float)grid_m * (1.0f / 64.0f);
+    if ((float)groups * b_bytes + a_bytes < 2.0f * ((cols > 1.0f ? cols : 1.0f) * a_bytes + b_bytes)) {
+      g = local / (rg * grid_n);
+      g = g < groups ? g : groups - 1;
+      r = local - g * (rg * grid_n);
+      last = g == groups - 1;
+      rows_g = last ? grid_m - g * rg : rg;
+      g *= rg;
     }
   }
+  const int width = rows_g + (last ? beside : 0);
+  const int col = r / width, at = r - col * width;
+  if (beside == 0 || at < rows_g) return TileAt{g + at, col, false};
+  const int lg = (int)((unsigned)problem_branch >> 30), sub = at - rows_g;
+  return TileAt{sub >> lg, (col << lg) + (sub & ((1 << lg) - 1)), true};
+}
+
+// Whether a kernel of these tiles may be given pairs: two of its shapes are of one format that has them (pairs_pay; weight-only tiles have 16-bit
+// activations and less than 16 bits a weight).
+template <class... Tiles>
+constexpr bool kMayPair = ((Tiles::kABits == Tiles::kWBits) || ...);
+
+// f(TileType<T>{}) with T the tile of branch `branch`: the compile-time dispatch over a kernel's tiles.
+template <class T>
+struct TileType {
+  using type = T;
 };
+template <int I, class F>
+__device__ __forceinline__ void with_branch(std::integral_constant<int, I>, int, F&&) {}
+template <class T, class... Rest, int I, class F>
+__device__ __forceinline__ void with_branch(std::integral_constant<int, I>, int branch, F&& f) {
+  if (branch == I) f(TileType<T>{});
+  else with_branch<Rest...>(std::integral_constant<int, I + 1>{}, branch, f);
+}
 
 // Waves per SIMD the register allocator should aim for: 2 (two co-resident workgroups per CU, 256 registers per lane) unless a
 // tile keeps more than 128 accumulator registers per lane, which needs the full 512-register budget of a lone wave.
@@ -169,9 +199,15 @@ __device__ __forceinline__ void fused_body(ArgsPtr args, uint8_t* smem) {
     const int mid = (lo + hi + 1) >> 1;
     if (uni(args->entry[mid].first) <= tile) lo = mid; else hi = mid - 1;
   }
-  const int en_first = uni(args->entry[lo].first), en_row0 = uni(args->entry[lo].row0), en_rows = uni(args->entry[lo].rows), en_pb = uni(args->entry[lo].problem_branch);
-  const int local = tile - en_first;
-  const int gp = uni(args->problem_offset) + (en_pb & 0xFFFF);
+  int en_first = uni(args->entry[lo].first), en_row0 = uni(args->entry[lo].row0), en_rows = uni(args->entry[lo].rows), en_pb = uni(args->entry[lo].problem_branch);
+  if (kMayPair<Tiles...> && ((unsigned)en_pb & kPairSecond)) {  // found by its index among the second segment's: a pair's tiles are counted from the first segment on
+    --lo;
+    en_first = uni(args->entry[lo].first);
+    en_row0 = uni(args->entry[lo].row0);
+    en_rows = uni(args->entry[lo].rows);
+    en_pb = uni(args->entry[lo].problem_branch);
+  }
+  const int gp = uni(args->problem_offset) + entry_problem(en_pb);
   const mxmoe_dim3* sizes = args->sizes;
   const uint8_t* const* As = args->As;
   const uint8_t* const* Bs = args->Bs;
@@ -186,14 +222,39 @@ __device__ __forceinline__ void fused_body(ArgsPtr args, uint8_t* smem) {
   t.sb = sb ? cload(sb + gp) : nullptr;
   t.C = cload(Cs + gp);
   t.acc_dump = acc ? cload(acc + gp) : nullptr;
-  t.row0 = en_row0;
-  t.M = t.row0 + en_rows;  // rows past the segment are treated like rows past the problem
   t.N = uni((int)cload(&sizes[gp].y));
   t.K = uni((int)cload(&sizes[gp].z));
-  t.tile_m = t.tile_n = 0;
   t.rows = nullptr;
   if constexpr (GU) t.rows = cload(args->rows + gp);
-  Dispatch<0, GU, Tiles...>::go(en_pb >> 16, t, local, smem);
+  int branch = entry_branch(en_pb), local = tile - en_first;
+  if (kMayPair<Tiles...> && pair_width(en_pb) != 0) {  // which of the two shapes it is comes out of the place; from here on a tile like any other
+    TileAt at{0, 0, false};
+    int bm = 0;
+    with_branch<Tiles...>(std::integral_constant<int, 0>{}, branch, [&](auto tile_type) {
+      using T = typename decltype(tile_type)::type;
+      at = locate_tile(local, en_rows, t.N, t.K, T::BM, T::BN, T::kABits, T::kWBits, en_pb);
+      bm = T::BM;
+    });
+    if (uni(at.second)) {
+      en_row0 = uni(args->entry[lo + 1].row0);
+      en_rows = uni(args->entry[lo + 1].rows);
+      branch = entry_branch(uni(args->entry[lo + 1].problem_branch));
+      local = uni(at.n * (int)(pair_width(en_pb) >> ((unsigned)en_pb >> 30)) + at.m);
+    } else {  // (the first segment is whole tiles) as the one row tile of its own segment
+      en_row0 += uni(at.m * bm);
+      en_rows = uni(bm);
+      local = uni(at.n);
+    }
+  }
+  t.row0 = en_row0;
+  t.M = t.row0 + en_rows;  // rows past the segment are treated like rows past the problem
+  with_branch<Tiles...>(std::integral_constant<int, 0>{}, branch, [&](auto tile_type) {
+    using T = typename decltype(tile_type)::type;
+    const TileAt at = locate_tile(local, en_rows, t.N, t.K, T::BM, T::BN, T::kABits, T::kWBits, 0);
+    t.tile_m = at.m;
+    t.tile_n = at.n;
+    T::template run<GU>(t, smem);
+  });
 }
 
 template <class... Tiles>
@@ -406,6 +467,7 @@ struct PlanInfo {
   int nb;                       // branches
   // Narrow integer tiles among them; and, where a launch is planned with them, whether it has few blocks of channels (kPoleBlocks).
   int narrow, few_blocks;
+  int may_pair;  // a format that has pairs (pairs_pay) comes in several shapes
   uint8_t order[kMaxBranches];  // positions in b, most expensive tile first (branch_cost); ties keep the registration order
   uint8_t fmt_start[kNumFmts + 4];
   // by format, in registration order inside a format: those of format f are b[fmt_start[f]] .. b[fmt_start[f + 1] - 1], and the planners
@@ -416,6 +478,7 @@ static_assert(sizeof(PlanInfo) % 8 == 0, "copied word by word");
 
 struct Segment {
   int row0, rows, branch, tiles;
+  int bm_log2, bn_log2;  // of two segments: their tiles
 };
 
 // Blocks of 256 channels, over all problems of a launch, up to which a 64-row integer tile sets the launch's time when it runs beside narrow ones: they stream
@@ -434,14 +497,37 @@ constexpr int kLongTiles = 128;
 constexpr int kLongK = 2048;
 __host__ __device__ inline bool runs_long(int K, int kmin) { return K > kmin && K >= kLongK; }
 
+// The fields of a pair of segments (FusedArgs::Entry); 0 where their column tiles do not come out even.
+__host__ __device__ inline unsigned pair_word(const Segment (&s)[2], int N) {
+  const int lg = s[0].bn_log2 - s[1].bn_log2;
+  if (lg < 0 || lg > 3 || tiles_over(N, s[1].bn_log2) != tiles_over(N, s[0].bn_log2) << lg) return 0;
+  const unsigned width = (unsigned)tiles_over(s[1].rows, s[1].bm_log2) << lg;
+  return width <= 255 ? width << 21 | (unsigned)lg << 30 : 0;
+}
+// Whether the two row segments of a problem are dealt out as a pair.  What a pair saves is the second trip of its weights from memory;
+// what it costs is that cheap tiles no longer come last, where they fill the end of the launch, so a launch has to have many tiles for it: `launch_tiles`
+// counts them in the shapes that are cheapest per row (launch_tiles_of).  At most 512 run at a time, together with those they share weights with; and there
+// large tiles that come first get a CU each.  Weights from memory, us, phases / pairs: 64 problems of N = 2816, K = 2048: w8a8 144 rows 146 / 102, 192 rows
+// 155 / 114, 546 rows 297 / 247 (N = 2048, K = 1408: 74 / 61, 78 / 68, 160 / 145), fp16 301 / 219, 310 / 232, 583 / 510; fp8 267 rows 210 / 190.  8 problems of
+// N = 28 672, K = 4096: w8a8 160 rows 363 / 247, 575 rows 678 / 580; of N = 4096, K = 14 336: 575 rows (640 tiles) 347 / 319, but 300 rows (384 tiles) 184 / 247.
+// int4 operands take half the time to fetch and as long to multiply: 144 rows 79 / 86, 192 rows 87 / 90, 546 rows 201 / 200, but with
+// N = 28 672, K = 4096 160 rows 205 / 194, 300 rows 294 / 260, 575 rows 472 / 438.  Weight-only tiles are bound by their arithmetic: 135 rows 134 / 149, 267 rows 209 / 273.
+// (launch_cols: the launch's blocks of 256 channels, each counted K / 4096 times: how much there is to fetch.)
+constexpr int kPairTiles = 512, kPairColsInt4 = 768;
+__host__ __device__ inline bool pairs_pay(int f, int launch_tiles, int launch_cols) {
+  return launch_tiles > kPairTiles && (f == (int)Fmt::W8A8 || f == (int)Fmt::FP16 || (f == (int)Fmt::W4A4 && launch_cols > kPairColsInt4));
+}
+
 // The choice of tile shapes for an M x N problem, as far as it does not depend on the rest of the launch.
 struct PlanPick {
-  int branch = -1, bm = 0, tiles = 0;
+  int branch = -1, bm = 0, tiles = 0, bm_log2 = 0, bn_log2 = 0;
   double cost = 0;
   __host__ __device__ void offer(const PlanBranch& b, int t, double c, double eps) {
     if (branch < 0 || c < cost - eps || (c < cost + eps && b.BM > bm)) {
       branch = b.index;
       bm = b.BM;
+      bm_log2 = b.bm_log2;
+      bn_log2 = b.bn_log2;
       tiles = t;
       cost = c;
     }
@@ -455,6 +541,15 @@ struct PlanChoice {
   // when it takes a shorter shape anyway or there is no other.
   int large_tiles = 0;
 };
+
+// What a problem adds to its launch's `launch_tiles` (upper half) and `launch_cols` (lower half).  Clamped where more makes no difference: the sums over a wave's
+// problems stay within 16 bits each.
+__host__ __device__ inline unsigned launch_load_of(const PlanChoice& c, int M, int N, int K) {
+  const unsigned tm = tiles_over(M, c.unit.bm_log2), tn = tiles_over(N, c.unit.bn_log2), blocks = tiles_over(N, 8);
+  const unsigned tiles = tm > kPairTiles || tn > kPairTiles || tm * tn > kPairTiles ? kPairTiles + 1 : tm * tn;
+  const unsigned cols = blocks > kPairColsInt4 || K > (kPairColsInt4 << 12) || blocks * (unsigned)K > (kPairColsInt4 << 12) ? kPairColsInt4 + 1 : blocks * (unsigned)K >> 12;
+  return tiles << 16 | cols;
+}
 
 // Returns 1, or 0 for M == 0, or -1 when the kernel has no tile for `f`.  Rolled loops here and below on purpose: the device planner runs
 // this once per launch, when none of its code is in the instruction cache, and what it costs there is the fetching of its instructions.
@@ -507,12 +602,12 @@ __host__ __device__ inline int plan_split(const PlanInfo& k, int f, int M, int N
       quick.offer(b, tiles, all > one ? all : one, 1e-9);
     }
     if (quick.branch != c.unit.branch) {
-      out[0] = Segment{0, M, quick.branch, quick.tiles};
+      out[0] = Segment{0, M, quick.branch, quick.tiles, 0, 0};
       return 1;
     }
   }
   const int rem = M - c.full;
-  out[0] = Segment{0, M, c.whole.branch, c.whole.tiles};
+  out[0] = Segment{0, M, c.whole.branch, c.whole.tiles, 0, 0};
   if (rem == 0 || c.full == 0) return 1;
   PlanPick rest;
   int all_unit = 0;  // tiles of the whole problem in the shape that is cheapest per row
@@ -524,12 +619,12 @@ __host__ __device__ inline int plan_split(const PlanInfo& k, int f, int M, int N
     if (b.index == c.unit.branch) all_unit = tiles_over(M, b.bm_log2) * tn;
   }
   if (rest.branch == c.unit.branch) {
-    out[0] = Segment{0, M, c.unit.branch, all_unit};
+    out[0] = Segment{0, M, c.unit.branch, all_unit, 0, 0};
     return 1;
   }
   if (c.whole.cost <= c.full_cost + rest.cost + 1e-9) return 1;
-  out[0] = Segment{0, c.full, c.unit.branch, c.unit.tiles};
-  out[1] = Segment{c.full, rem, rest.branch, rest.tiles};
+  out[0] = Segment{0, c.full, c.unit.branch, c.unit.tiles, c.unit.bm_log2, c.unit.bn_log2};
+  out[1] = Segment{c.full, rem, rest.branch, rest.tiles, rest.bm_log2, rest.bn_log2};
   return 2;
 }
 
@@ -545,6 +640,8 @@ inline PlanInfo make_plan_info(const std::vector<BranchInfo>& branches) {
   PlanInfo k;
   std::memset(&k, 0, sizeof k);
   k.nb = std::min((int)branches.size(), kMaxBranches);
+  for (int i = 0; i < k.nb; ++i)
+    for (int j = 0; j < i; ++j) k.may_pair |= branches[i].fmt == branches[j].fmt && !is_weight_only(branches[i].fmt) && branches[i].fmt != Fmt::W4A4G128;
   for (int i = 0; i < k.nb; ++i) k.narrow |= integer_sums((int)branches[i].fmt) && branches[i].BN == 64;
   auto log2_of = [](int v) {
     int lg = 0;
@@ -829,10 +926,10 @@ inline bool shape_ok(const BranchInfo& bi, const mxmoe_dim3& sz) {
   return sz.z != 0 && sz.z % bi.k_multiple == 0 && (int)sz.z >= bi.k_min && sz.y % 8 == 0 && !(wo && sz.y % 16 != 0);
 }
 
-// What the planning of one launch's problems has in common: its smallest K, the large tiles of its long problems, whether it has few blocks.  Problems without rows
+// What the planning of one launch's problems has in common: its smallest K, its tiles, the large tiles of its long problems, whether it has few blocks.  Problems without rows
 // have no part in it: a list plans the same with and without them (the device planner sees every expert, the operators leave out empty ones).
 struct LaunchScope {
-  int kmin = 0x7fffffff, long_tiles = 0;
+  int kmin = 0x7fffffff, long_tiles = 0, launch_tiles = 0, launch_cols = 0;
   bool few_blocks = false;
   // the `long_tiles` argument of a problem's plan
   int long_tiles_of(const mxmoe_dim3& sz) const { return runs_long((int)sz.z, kmin) ? long_tiles : 0; }
@@ -849,8 +946,11 @@ inline LaunchScope launch_scope(const PlanInfo& pi, const mxmoe_dim3* h_sizes, c
   for (int i = 0; i < n; ++i) {
     const Fmt f = classify(h_q[i]);
     PlanChoice c;
-    if (f != Fmt::UNSUPPORTED && runs_long((int)h_sizes[i].z, s.kmin) && plan_choose(pi, (int)f, (int)h_sizes[i].x, (int)h_sizes[i].y, c) > 0)
-      s.long_tiles = std::min(s.long_tiles + c.large_tiles, kLongTiles);
+    if (f == Fmt::UNSUPPORTED || plan_choose(pi, (int)f, (int)h_sizes[i].x, (int)h_sizes[i].y, c) <= 0) continue;
+    const unsigned load = launch_load_of(c, (int)h_sizes[i].x, (int)h_sizes[i].y, (int)h_sizes[i].z);
+    s.launch_tiles += (int)(load >> 16);
+    s.launch_cols += (int)(load & 0xFFFF);
+    if (runs_long((int)h_sizes[i].z, s.kmin)) s.long_tiles = std::min(s.long_tiles + c.large_tiles, kLongTiles);
   }
   return s;
 }
@@ -863,6 +963,8 @@ inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, c
   const PlanInfo& pi = plan_of(k);
   struct Entry {
     int row0, rows, problem, branch, tiles;
+    unsigned pair;
+    int phase_branch;  // whose phase it runs in: its own, or that of the pair's first segment
   };
   Entry entries[kMaxEntries];
   int nent = 0;
@@ -884,7 +986,8 @@ inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, c
         last_error() = buf;
         return 3;
       }
-      entries[nent++] = Entry{sg[j].row0, sg[j].rows, i, sg[j].branch, sg[j].tiles};
+      const unsigned pair = ns == 2 && pairs_pay((int)f, scope.launch_tiles, scope.launch_cols) ? pair_word(sg, (int)sz.y) : 0;
+      entries[nent++] = Entry{sg[j].row0, sg[j].rows, i, sg[j].branch, sg[j].tiles, pair | (pair && j ? kPairSecond : 0u), sg[pair ? 0 : j].branch};
     }
   }
   // Most expensive tile shape first.  Inside a shape, the problems whose K is above the launch's smallest K go first (their tiles
@@ -899,8 +1002,8 @@ inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, c
     for (int pass = 0; pass < 2; ++pass)
       for (int ei = 0; ei < nent; ++ei) {
         const Entry& en = entries[ei];
-        if (en.branch != b || en.tiles == 0 || ((int)h_sizes[base + en.problem].z > scope.kmin) != (pass == 0)) continue;
-        a.entry[ne] = FusedArgs::Entry{total, en.row0, en.rows, en.problem | (en.branch << 16)};
+        if (en.phase_branch != b || en.tiles == 0 || ((int)h_sizes[base + en.problem].z > scope.kmin) != (pass == 0)) continue;
+        a.entry[ne] = FusedArgs::Entry{total, en.row0, en.rows, (int)((unsigned)(en.problem | (en.branch << 16)) | en.pair)};
         total += en.tiles;
         ++ne;
       }

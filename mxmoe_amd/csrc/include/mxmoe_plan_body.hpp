@@ -92,6 +92,7 @@ struct PlanShared {
   int cnt[kMaxBranches][2], til[kMaxBranches][2];    // per run-order rank and wave: entries, tiles
   int cnt_long[kMaxBranches][2], til_long[kMaxBranches][2];  // ... of which belong to long-K problems
   int kmin[2];
+  unsigned load[2];                                  // launch_load_of, per wave
   int long_tiles[2], long_tiles_kmin[2];             // large tiles of the wave's problems with K >= kLongK; of those with K = kmin
   // the kernel's branch table, from the kernel arguments: the planning functions walk it entry by entry, and each step of such a
   // walk through the argument segment costs a trip to the scalar cache
@@ -193,6 +194,10 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
     // what this problem's tile shapes are, as far as the rest of the launch has no say in it, and the large tiles of the long problems
     // (launch_scope): whether one of K >= kLongK is above the launch's smallest is known behind the barrier
     have = mine ? plan_choose(info, fmt, (int)rows, N, choice) : 0;
+    if (info.may_pair) {
+      const unsigned load = (unsigned)wave_last(wave_inclusive_scan(have > 0 ? (int)launch_load_of(choice, (int)rows, N, K) : 0));
+      if (lane == 0) sh.load[wave] = load;
+    }
     const int large = have > 0 && K >= kLongK ? choice.large_tiles : 0;
     if (__ballot(large > 0) != 0) {
       const int all = wave_last(wave_inclusive_scan(large)), at_km = wave_last(wave_inclusive_scan(K == km ? large : 0));
@@ -212,6 +217,8 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
   const int ns = have > 0 ? plan_split(info, fmt, (int)rows, N, choice, runs_long(K, kmin) ? min(long_tiles, kLongTiles) : info.few_blocks && integer_sums(fmt) ? choice.large_tiles : 0, sg) : 0;
   const PlanBranch& my_branch = info.b[info.order[min(lane, kMaxBranches - 1)]];  // lane r: the branch of rank r
   const int my_order = my_branch.index;
+  unsigned pair = 0;  // the second segment goes beside the first: one item of two entries
+  if (info.may_pair && ns == 2 && pairs_pay(fmt, (int)((sh.load[0] >> 16) + (sh.load[1] >> 16)), (int)((sh.load[0] & 0xFFFF) + (sh.load[1] & 0xFFFF)))) pair = pair_word(sg, N);
   int seg_rank[2] = {-1, -1}, seg_pos[2] = {0, 0}, seg_first[2] = {0, 0};
   // per branch in run order, this wave's entries and tiles
   for (int r = 0; active && r < info.nb; ++r) {
@@ -219,14 +226,14 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
     int mine_tiles = 0, which = -1;
 #pragma unroll
     for (int j = 0; j < 2; ++j)
-      if (j < ns && sg[j].branch == b && sg[j].tiles > 0) {
-        mine_tiles = sg[j].tiles;
+      if (j < ns && sg[j].branch == b && sg[j].tiles > 0 && !(j == 1 && pair)) {
+        mine_tiles = sg[j].tiles + (pair ? sg[1].tiles : 0);
         which = j;
       }
     // entries of this branch in this wave, long-K problems first: position = matching lanes that run earlier, first tile = their tiles
     const uint64_t has = __ballot(which >= 0);
     if (has == 0) continue;  // (most branches of a kernel are not used by a given launch: their counters stay zero)
-    const uint64_t has_long = __ballot(which >= 0 && long_k);
+    const uint64_t has_long = __ballot(which >= 0 && long_k), two = __ballot(which >= 0 && pair);
     const int inc_long = wave_inclusive_scan(long_k ? mine_tiles : 0), inc_rest = wave_inclusive_scan(long_k ? 0 : mine_tiles);
     const int tt_long = wave_last(inc_long), tt = tt_long + wave_last(inc_rest);
     const uint64_t before = (1ull << lane) - 1;
@@ -235,15 +242,21 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
       if (which == j) {
         seg_rank[j] = r;
         // position / first tile inside this wave's entries of its own class; the other wave's and the other class's are added below
-        seg_pos[j] = long_k ? __popcll(has_long & before) : __popcll(has & ~has_long & before);
+        const uint64_t here = (long_k ? has_long : ~has_long) & before;
+        seg_pos[j] = __popcll(has & here) + __popcll(two & here);
         seg_first[j] = long_k ? inc_long - mine_tiles : inc_rest - mine_tiles;
       }
     if (lane == 0) {
-      sh.cnt[r][wave] = __popcll(has);
+      sh.cnt[r][wave] = __popcll(has) + __popcll(two);
       sh.til[r][wave] = tt;
-      sh.cnt_long[r][wave] = __popcll(has_long);
+      sh.cnt_long[r][wave] = __popcll(has_long) + __popcll(has_long & two);
       sh.til_long[r][wave] = tt_long;
     }
+  }
+  if (pair) {
+    seg_rank[1] = seg_rank[0];
+    seg_pos[1] = seg_pos[0] + 1;
+    seg_first[1] = seg_first[0] + sg[0].tiles;
   }
   __syncthreads();
   if (!active) return;
@@ -298,7 +311,7 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
           first += sh.til[r][0] - sh.til_long[r][0];
         }
       }
-      fa->entry[pos] = FusedArgs::Entry{first, sg[j].row0, sg[j].rows, e | (sg[j].branch << 16)};  // problem index relative to the launch's first
+      fa->entry[pos] = FusedArgs::Entry{first, sg[j].row0, sg[j].rows, (int)((unsigned)(e | (sg[j].branch << 16)) | pair | (pair && j ? kPairSecond : 0u))};  // problem index relative to the launch's first
     }
   }
   if (wave == 0) {

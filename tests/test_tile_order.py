@@ -1,0 +1,98 @@
+"""The order of a launch's tiles: which part of which problem each workgroup computes, on the host, through the functions the kernels call."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+W4, W8, FP, WO = (4, 4, -1, True), (8, 8, -1, True), (16, 16, -1, True), (16, 4, 128, False)
+
+
+def _launch(lib, probs, kid=-1):
+    from mxmoe_amd import _lib
+
+    n = len(probs)
+    sizes = (_lib.Dim3 * n)(*[_lib.Dim3(*p[:3]) for p in probs])
+    qs = (_lib.QParams * n)(*[_lib.QParams(q[0], q[1], q[2], int(q[3])) for *_, q in probs])
+    if kid < 0:
+        kid = lib.mxmoe_group_gemm_plan(-1, sizes, qs, n, None, None) - 1000
+        assert kid >= 0, lib.mxmoe_last_error()
+    out = (C.c_int32 * 1200)()
+    assert lib.mxmoe_group_gemm_plan_tables(kid, sizes, qs, n, out, 1200) == 0, lib.mxmoe_last_error()
+    tab = np.array(out[:], np.int64)
+    grid = int(tab[3]) + 64
+    area = (C.c_int32 * (5 * grid))()
+    assert lib.mxmoe_group_gemm_plan_tile_area(kid, sizes, qs, n, grid, area) == 0, lib.mxmoe_last_error()
+    return tab, np.array(area[:], np.int64).reshape(grid, 5)
+
+
+def _pairs(tab):
+    entries = tab[22:22 + 4 * tab[0]].reshape(-1, 4)
+    return [int(e[3]) & 0xFFFF for e in entries if (int(e[3]) >> 29) & 1]  # problems whose second segment runs beside the first
+
+
+@pytest.mark.parametrize("q,rows,n,k", [
+    (W8, 144, 2816, 2048), (W8, 192, 2816, 2048), (W8, 129, 2816, 2048), (W8, 546, 2048, 1408), (FP, 144, 2816, 2048), (FP, 300, 1288, 4096),
+    (W4, 300, 28672, 4096), (W8, 1060, 28672, 4096),                  # activations of several groups of row tiles: the second segment goes with the last
+    (W8, 160, 2824, 2048),                                            # the last column tile is 8 wide
+    (WO, 140, 2816, 2048), (W4, 144, 2816, 2048),                     # two segments, no pairs
+])
+def test_every_output_is_computed_once(lib, q, rows, n, k):
+    """Every element of every output in exactly one workgroup's tile, for problems of two row segments next to empty and small ones."""
+    probs = [((rows, rows + 1, rows - 1, 0, 7, 128)[i % 6], n, k, q) for i in range(60)]
+    tab, area = _launch(lib, probs)
+    assert bool(_pairs(tab)) == (q is W8 or q is FP or n == 28672)
+    area = area[area[:, 0] >= 0]
+    for p, (m, *_rest) in enumerate(probs[:6]):
+        cover = np.zeros((m, n), np.int8)
+        for _, r0, r1, c0, c1 in area[area[:, 0] == p]:
+            cover[r0:r1, c0:c1] += 1
+        assert (cover == 1).all(), (p, m)
+
+
+def test_tiles_of_a_pair_that_share_weights_are_neighbours(lib):
+    """All row tiles of both shapes against one block of channels come one after the other on an XCD (workgroup w runs on XCD w mod 8)."""
+    tab, area = _launch(lib, [(192, 2816, 2048, W8)] * 64)
+    assert len(_pairs(tab)) == 64
+    area = area[area[:, 0] >= 0]
+    order = np.concatenate([area[x::8] for x in range(8)])
+    first = order[::2]
+    assert (order[1::2, [0, 3, 4]] == first[:, [0, 3, 4]]).all() and set(map(tuple, first[:, 1:3])) == {(0, 128)} and set(map(tuple, order[1::2, 1:3])) == {(128, 192)}
+
+
+@pytest.mark.parametrize("q,count,rows,n,k,pairs", [
+    (W8, 64, 192, 2048, 1408, True), (W8, 8, 300, 4096, 14336, False),     # 1024 and 384 tiles: past and within what runs at a time
+    (W4, 64, 192, 2816, 2048, False), (W4, 8, 300, 28672, 4096, True),     # int4: by what there is to fetch
+    (WO, 64, 140, 28672, 4096, False), ((4, 4, 128, True), 64, 90, 28672, 4096, False),
+])
+def test_when_segments_are_paired(lib, q, count, rows, n, k, pairs):
+    tab, _ = _launch(lib, [(rows, n, k, q)] * count)
+    assert (len(_pairs(tab)) == count) == pairs and (pairs or not _pairs(tab))
+    # a problem without rows changes nothing
+    tab2, _ = _launch(lib, [(rows, n, k, q)] * count + [(0, n, k, q)] * 8)
+    assert (tab[:22] == tab2[:22]).all() and (tab[22:22 + 4 * tab[0]] == tab2[22:22 + 4 * tab[0]]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("q,rows,n,k", [(W8, 192, 2816, 2048), (W4, 185, 28672, 4096), (FP, 150, 2048, 1408)])
+def test_device_planner_makes_the_same_pairs(lib, q, rows, n, k):
+    import torch
+
+    from mxmoe_amd import _lib
+
+    e = 8 if n == 28672 else 60
+    counts = [(rows, rows + 1, rows - 1, 0, 7, 128)[i % 6] for i in range(e)]
+    desc = (_lib.BlockDesc * e)(*[_lib.BlockDesc(q[0], q[1], q[2], int(q[3]), (C.c_uint8 * 3)(), n, k, 0, 0)] * e)
+    kid = lib.mxmoe_plan_select_kernel(-1, desc, e)
+    d_desc = torch.frombuffer(bytearray(bytes(desc)), dtype=torch.uint8).cuda()
+    recv = torch.tensor(counts, dtype=torch.int64, device="cuda")
+    plan = torch.zeros(lib.mxmoe_plan_bytes(e), dtype=torch.uint8, device="cuda")
+    some = torch.zeros(16, dtype=torch.uint8, device="cuda")
+    _lib.check(lib, lib.mxmoe_plan_block(kid, recv.data_ptr(), e, 0, d_desc.data_ptr(), desc, some.data_ptr(), some.data_ptr(), some.data_ptr(), plan.data_ptr(),
+                                         torch.cuda.current_stream().cuda_stream))
+    tab, _ = _launch(lib, [(m, n, k, q) for m in counts], kid)
+    assert _pairs(tab)
+    ne, tiles, nph, grid = tab[:4]
+    hdr = plan.cpu().numpy()[:4096].view(np.int32)[14:]
+    assert list(hdr[:4]) == [0, ne, tiles, nph] and grid <= lib.mxmoe_plan_grid_bound(kid, desc, e, sum(counts), 0)
+    assert np.array_equal(hdr[4:5 + nph], tab[4:5 + nph]) and np.array_equal(hdr[13:14 + nph], tab[13:14 + nph])
+    assert np.array_equal(hdr[23:23 + 4 * ne], tab[22:22 + 4 * ne].astype(np.int32))
