@@ -3,6 +3,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import torch
 
 W4, W8, FP, WO = (4, 4, -1, True), (8, 8, -1, True), (16, 16, -1, True), (16, 4, 128, False)
 
@@ -75,8 +76,6 @@ def test_when_segments_are_paired(lib, q, count, rows, n, k, pairs):
 @pytest.mark.gpu
 @pytest.mark.parametrize("q,rows,n,k", [(W8, 192, 2816, 2048), (W4, 185, 28672, 4096), (FP, 150, 2048, 1408)])
 def test_device_planner_makes_the_same_pairs(lib, q, rows, n, k):
-    import torch
-
     from mxmoe_amd import _lib
 
     e = 8 if n == 28672 else 60
