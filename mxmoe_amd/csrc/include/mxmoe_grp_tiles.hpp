@@ -8,9 +8,16 @@
 // Operands: activations int4 rows [M, K/2] with scales [M, K/128]; weights in MFMA fragment order as for w4a4 (mxmoe_tiles.hpp,
 // WxAxTile) with scales stored group-major [K/128, N], so that the scales of a tile's channels for one group are contiguous.
 // BM x 256 outputs per workgroup, 4 waves x 64 channels.  Activations go global -> registers -> LDS (3-stage ring, one barrier
-// per slice), weights global -> registers two slices ahead, a group's scales global -> registers at the start of its slice; every load is an ordinary
-// load whose waits the compiler places.  Indices past the ends (rows past M, channel blocks past N, slices past K) are clamped
+// per slice), weights global -> registers one slice ahead, a group's scales global -> registers as soon as the last group's are used; every load is an
+// ordinary load whose waits the compiler places.  Indices past the ends (rows past M, channel blocks past N, slices past K) are clamped
 // to the last valid one: such results are computed and never stored.
+//
+// Bound: the vector ALU.  A 32 x 32 block of a slice is four matrix instructions (128 cycles of the matrix pipe) and, written out, 80 vector ones to rescale
+// it (320 cycles), besides the widening of its operands.  The products of the scales, 32 of those 80, therefore come out of the matrix pipe too, which
+// has the time: the outer product of 32 channel scales and 32 token scales is one more matrix instruction, exact (22 bits of product, everything else
+// it adds is zero) and in the layout of the sums.  Every block is then 16 conversions, multiplications and additions, and the operands of the blocks to come
+// are widened between the matrix instructions.  64 problems of N = 2816, K = 2048, weights from memory, us: 30 rows 65 -> 54, 192 rows 175 -> 151,
+// 546 rows 431 -> 363.  (The order alone, blocks rescaled beside the next block's matrix instructions, changed nothing: the other wave of the SIMD fills the gaps.)
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -70,10 +77,6 @@ struct WxAxGTile {
     };
     const int fa = lrow * kRowBytes;
     const int sw = lds_swizzle(lrow);
-    auto a_sread = [&](int stage, int step, int i) {
-      return *reinterpret_cast<const v4i*>(smem + stage * kStageBytes + fa + i * 32 * kRowBytes + ((((lane >> 5) + 2 * step) ^ sw) << 4));
-    };
-
     // ---- weights: fragment (block j, k-step s) of slice kt at ((nb * G + kt) * 2 + s) * 1 KB ----
     const int nblk = (N + 31) / 32;
     const uint8_t* bptr[FN];
@@ -82,24 +85,25 @@ struct WxAxGTile {
       bptr[j] = t.B + (long)(GU ? min(n0 / 32 + wave, nblk - 1) + j * nblk : min(n0 / 32 + wave * FN + j, nblk - 1)) * G * 2048 + lane * 16;
     auto b_gload = [&](int j, int s, int kt) { return gload<v4i>(bptr[j] + ((long)min(kt, G - 1) * 2 + s) * 1024); };
 
-    // ---- scales of one group: token scales of the lane's rows, channel scales of its 4-channel runs ----
+    // ---- scales of one group.  Their products come out of the matrix pipe in the layout of the sums: channel scales as a 32 x 16 operand with all but its
+    // first column zero, token scales likewise, so a lane loads one of each per block (lanes 32 .. 63 hold columns 8 .. 15 and mask what they load)
     const _Float16* sa_ptr[FM];
 #pragma unroll
     for (int i = 0; i < FM; ++i) sa_ptr[i] = t.sa + (long)row_of(m0 + i * 32 + lrow) * G;
-    // channel scales: the lane's first run of 4 channels; the others sit 8 channels (16 bytes) apart and are clamped one by one
-    const int nbase = n0 + wave * (GU ? 32 : 64) + nq;
-    auto s_gload = [&](int kt, _Float16 (&sa_h)[FM], v4h (&sb_h)[FN][4]) {
+    int sb_at[FN];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) sb_at[j] = GU ? j * N + min(n0 + wave * 32 + lrow, N - 1) : min(n0 + wave * 64 + j * 32 + lrow, N - 1);
+    const int first_column = lane < 32 ? 0xFFFF : 0;
+    int sa_next[FM], sb_next[FN];  // of the next group, as bits
+    auto s_load = [&](int kt) {
       const int g = min(kt, G - 1);
 #pragma unroll
-      for (int i = 0; i < FM; ++i) sa_h[i] = gload<_Float16>(sa_ptr[i] + g);
-      const _Float16* sbg = t.sb + (long)g * t.N;
+      for (int i = 0; i < FM; ++i) sa_next[i] = gload<unsigned short>(sa_ptr[i] + g);
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) sb_h[j][q] = gload<v4h>(sbg + (GU ? j * N + min(nbase + q * 8, N - 4) : min(nbase + j * 32 + q * 8, N - 4)));
+      for (int j = 0; j < FN; ++j) sb_next[j] = gload<unsigned short>(t.sb + (long)g * t.N + sb_at[j]);
     };
 
-    v16f facc[FM][FN];
+    v16f facc[FM][FN];    // 256 times the outputs: the integer sums are of 16 * code products (int4 widened in place), a power of two either way
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -107,84 +111,99 @@ struct WxAxGTile {
 #pragma unroll
         for (int r = 0; r < 16; ++r) facc[i][j][r] = 0.0f;
 
-    v4i stg[2][kQ];       // activation slices kt+1 / kt+2 on their way to LDS
-    v4i wb[2][FN][2];     // packed weight fragments of slices kt, kt+1 (slot = slice parity)
-
-    a_gload(0, stg[0]);
+    v4i stg[kQ];          // activation slice kt+2 on its way to LDS
+    v4i wb[FN][2];        // packed weight fragments, each loaded for the next slice when it has been widened for this one
+    v4i pa[2];            // packed activation fragments of one block
+    v4i aop[FM][2][2];    // operands of a slice: [block][k-step][low / high nibbles]
+    v4i bop[FN][2][2];
+    v4i sa_op[FM], sb_op[FN];
 #pragma unroll
-    for (int d = 0; d < 2; ++d)
+    for (int i = 0; i < FM; ++i) sa_op[i] = v4i{};
+#pragma unroll
+    for (int j = 0; j < FN; ++j) sb_op[j] = v4i{};
+
+    // nibble n of a byte -> int8 holding 16 * signed(n): quarter x of a block's fragments
+    auto widen = [](const v4i (&p)[2], v4i (&o)[2][2], int x) {
+      if (x & 1) o[x >> 1][1] = p[x >> 1] & (int)0xF0F0F0F0;
+      else o[x >> 1][0] = (p[x >> 1] << 4) & (int)0xF0F0F0F0;
+    };
+    auto a_sread = [&](int stage, int i) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+        pa[s] = *reinterpret_cast<const v4i*>(smem + stage * kStageBytes + fa + i * 32 * kRowBytes + ((((lane >> 5) + 2 * s) ^ sw) << 4));
+    };
+    auto b_load = [&](int j, int kt) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) wb[j][s] = b_gload(j, s, kt);
+    };
+
+    a_gload(0, stg);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) b_load(j, 0);
+    s_load(0);
+    a_swrite(0, stg);
+    a_gload(1, stg);
+    __syncthreads();
+    a_sread(0, 0);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      widen(pa, aop[0], x);
+      widen(wb[0], bop[0], x);
+    }
+    b_load(0, 1);
+
+    constexpr int kBlocks = FM * FN;  // block b of a slice: token block b / FN, channel block b % FN
+    int stage = 0;
+#pragma unroll 1
+    for (int kt = 0; kt < G; ++kt) {
+      const int nstage = stage == kStages - 1 ? 0 : stage + 1;
+#pragma unroll
+      for (int i = 0; i < FM; ++i) sa_op[i][0] = sa_next[i] & first_column;
+#pragma unroll
+      for (int j = 0; j < FN; ++j) sb_op[j][0] = sb_next[j] & first_column;
+      s_load(kt + 1);
+      a_swrite(nstage, stg);  // slice kt+1, fetched during the previous slice
+      a_gload(kt + 2, stg);
+      static_for<kBlocks>([&](auto bc) {
+        constexpr int b = decltype(bc)::value, i = b / FN, j = b % FN;
+        if constexpr (b == 0 && FM == 2) a_sread(stage, 1);
+        if constexpr (b == kBlocks - 2) {
+          __syncthreads();  // slice kt+1 is in LDS for everybody (and everybody is done with the stage that slice kt+2 will overwrite)
+          a_sread(nstage, 0);
+        }
+        const v16f sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, sb_op[j]), __builtin_bit_cast(v8h, sa_op[i]), v16f{}, 0, 0, 0);
+        v16i c;
+        // four matrix instructions, and the operands whose registers are free widened beside them
+        static_for<4>([&](auto xc) {
+          constexpr int x = decltype(xc)::value;
+          if constexpr (x == 0) c = __builtin_amdgcn_mfma_i32_32x32x32_i8(bop[j][0][0], aop[i][0][0], v16i{}, 0, 0, 0);
+          else c = __builtin_amdgcn_mfma_i32_32x32x32_i8(bop[j][x >> 1][x & 1], aop[i][x >> 1][x & 1], c, 0, 0, 0);
+          if constexpr (b == 0) widen(wb[1], bop[1], x);
+          if constexpr (FM == 2 && b == 1) widen(pa, aop[1], x);
+          if constexpr (FM == 2 && b == 2) widen(pa, aop[0], x);
+          __builtin_amdgcn_sched_barrier(0);
+        });
+        if constexpr (b == 0) b_load(1, kt + 1);
+        if constexpr (b == kBlocks - 1) {
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            if constexpr (FM == 1) widen(pa, aop[0], x);
+            widen(wb[0], bop[0], x);
+          }
+          b_load(0, kt + 2);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) facc[i][j][r] = facc[i][j][r] + (float)c[r] * sc[r];
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      stage = nstage;
+    }
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int j = 0; j < FN; ++j)
 #pragma unroll
-        for (int s = 0; s < 2; ++s) wb[d][j][s] = b_gload(j, s, d);
-    a_swrite(0, stg[0]);
-    a_gload(1, stg[1]);
-    __syncthreads();
-
-    auto slice = [&](auto dc, int kt, int stage) {
-      constexpr int d = decltype(dc)::value;
-      const int nstage = stage == kStages - 1 ? 0 : stage + 1;
-      a_swrite(nstage, stg[(d + 1) & 1]);  // slice kt+1, fetched during the previous slice
-      a_gload(kt + 2, stg[d & 1]);
-      // this group's scales: used after the slice's MFMAs, which cover the load
-      _Float16 sa_c[FM];
-      v4h sb_c[FN][4];
-      s_gload(kt, sa_c, sb_c);
-      v16i iacc[FM][FN];
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) iacc[i][j][r] = 0;
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        v4i alo[FM], ahi[FM];
-#pragma unroll
-        for (int i = 0; i < FM; ++i) {
-          const v4i p = a_sread(stage, s, i);
-          alo[i] = (p << 4) & (int)0xF0F0F0F0;
-          ahi[i] = p & (int)0xF0F0F0F0;
-        }
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const v4i p = wb[d][j][s];
-          const v4i blo = (p << 4) & (int)0xF0F0F0F0, bhi = p & (int)0xF0F0F0F0;
-          wb[d][j][s] = b_gload(j, s, kt + 2);
-#pragma unroll
-          for (int i = 0; i < FM; ++i) {
-            iacc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(blo, alo[i], iacc[i][j], 0, 0, 0);
-            iacc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bhi, ahi[i], iacc[i][j], 0, 0, 0);
-          }
-        }
-      }
-      // this group's contribution: float(acc) * (sa * sb), the accumulator holding 256 * sum (2^-8 folded into sa, exact)
-#pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const float sa_f = (float)sa_c[i] * 0.00390625f;
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float sc = sa_f * (float)sb_c[j][q][e];
-              facc[i][j][q * 4 + e] = facc[i][j][q * 4 + e] + keep_f32((float)iacc[i][j][q * 4 + e] * sc);
-            }
-      }
-      __syncthreads();  // slice kt+1 is in LDS for everybody, and everybody is done with the stage that slice kt+2 will overwrite
-    };
-
-    int stage = 0;
-#pragma unroll 1
-    for (int kt0 = 0; kt0 < G; kt0 += 2) {
-      slice(std::integral_constant<int, 0>{}, kt0, stage);
-      stage = stage == kStages - 1 ? 0 : stage + 1;
-      if (kt0 + 1 < G) {
-        slice(std::integral_constant<int, 1>{}, kt0 + 1, stage);
-        stage = stage == kStages - 1 ? 0 : stage + 1;
-      }
-    }
+        for (int r = 0; r < 16; ++r) facc[i][j][r] *= 0.00390625f;  // exact
 
     // ---- epilogue: lane holds token lane & 31 and channels 8*(r/4) + 4*(lane >> 5) + (r & 3) of each 32 x 32 block ----
 #pragma unroll
