@@ -477,6 +477,10 @@ struct WoMfmaTile {
   static constexpr int kABits = 16, kWBits = WBITS;  // fp16 activations, packed weights
   static constexpr int kLaneBytes = Sk::kLaneBytes, kBlockBytes = Sk::kBlockBytes;
   static constexpr int kDma = kStageBytes / 1024 / kWaves;  // direct-to-LDS loads per wave per stage
+  // 8-bit weights beside 128 accumulator registers: a ring of two k blocks has no room, so a wave holds one, in halves.  The half that sub-blocks 0 and 1
+  // read is loaded again for the next k block when they are done, the other half at the end.  Against the 2 x 2 shape, whose waves unpack every weight
+  // twice: 64 problems of N = 2816, K = 2048, weights from memory, us, 48 rows 127 -> 88, 96 rows 133 -> 109, 192 rows 224 -> 184, 546 rows 539 -> 412.
+  static constexpr bool kHalves = WBITS == 8 && MB == 8;
 
   template <bool GU>
   __device__ static __forceinline__ void run(const TileArgs& t, uint8_t* __restrict__ smem) {
@@ -531,7 +535,12 @@ struct WoMfmaTile {
     const uint8_t* sb = reinterpret_cast<const uint8_t*>(t.sb) + ((long)nb0 * KB) * 64 + lm * 4;
     auto w_of = [&](int nb, int kb) { return Sk::load_w(wb + ((long)block_of(nb) * KB + min(kb, KB - 1)) * kBlockBytes); };
     auto s_of = [&](int nb, int kb) { return gload<int>(sb + ((long)block_of(nb) * KB + min(kb, KB - 1)) * 64); };
-    typename Sk::WReg wr[8];
+    auto half_of = [&](typename Sk::WReg& w, int h, int nb, int kb) {
+      const v4i v = gload<v4i>(wb + ((long)block_of(nb) * KB + min(kb, KB - 1)) * kBlockBytes + 16 * h);
+#pragma unroll
+      for (int d = 0; d < 4; ++d) w.d[(4 * h + d) % WBITS] = v[d];
+    };
+    typename Sk::WReg wr[kHalves ? 4 : 8];
     int sr[8];
 
     v4f acc[4][MB];  // [channel block][token block]
@@ -541,18 +550,30 @@ struct WoMfmaTile {
       for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = v4f{0.f, 0.f, 0.f, 0.f};
 
     {
-      // prologue: exactly 8 ring loads are younger than the loads of the first activation stage, as in every later iteration
+      // prologue: exactly kYounger loads are younger than the loads of the first activation stage, as in every later iteration
+      constexpr int kYounger = kHalves ? 12 : 8;
+      if constexpr (kHalves) {
+        dma_x(0, 0);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        wr[q] = w_of(q, 0);
-        sr[q] = s_of(q, 0);
-      }
-      asm volatile("" ::: "memory");
-      dma_x(0, 0);
+        for (int q = 0; q < 4; ++q) {
+          half_of(wr[q], 0, q, 0);
+          sr[q] = s_of(q, 0);
+        }
 #pragma unroll
-      for (int q = 4; q < 8; ++q) {
-        wr[q] = w_of(q - 4, 1);
-        sr[q] = s_of(q - 4, 1);
+        for (int q = 0; q < 4; ++q) half_of(wr[q], 1, q, 0);
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          wr[q] = w_of(q, 0);
+          sr[q] = s_of(q, 0);
+        }
+        asm volatile("" ::: "memory");
+        dma_x(0, 0);
+#pragma unroll
+        for (int q = 4; q < 8; ++q) {
+          wr[q % (kHalves ? 4 : 8)] = w_of(q - 4, 1);
+          sr[q] = s_of(q - 4, 1);
+        }
       }
       asm volatile("" ::: "memory");
       const v8h bias = Sk::bias8();
@@ -565,12 +586,13 @@ struct WoMfmaTile {
       auto step = [&](auto parc, int kb, auto livec) {
         constexpr int st = decltype(parc)::value;
         constexpr int LIVE = decltype(livec)::value;
-        // the activation stage of this k block has landed: the only younger loads are the 8 ring refills of the last iteration
-        // (or the 8 ring loads of the prologue)
-        vm_wait<8>();
+        // the activation stage of this k block has landed: the only younger loads are the refills of the last iteration (or the loads of
+        // the prologue)
+        vm_wait<kYounger>();
         __syncthreads();  // ... for every wave; and every wave holds the previous stage's fragments in registers by now
-        if (kb + 1 < KB) dma_x(kb + 1, st ^ 1);
-        constexpr int base = st * 4;
+        if constexpr (!kHalves)
+          if (kb + 1 < KB) dma_x(kb + 1, st ^ 1);
+        constexpr int base = st * 4, wbase = kHalves ? 0 : base;
         // k sub-block by k sub-block: its token fragments, then every channel block's 8 weights per lane against all of them
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -580,7 +602,7 @@ struct WoMfmaTile {
 #pragma unroll
           for (int nb = 0; nb < 4; ++nb) {
             v8h wf[4];
-            Sk::unpack(wr[base + nb], wf);  // only wf[j] is used: the rest folds away
+            Sk::unpack(wr[wbase + nb], wf);  // only wf[j] is used: the rest folds away
             const v2h sz = __builtin_bit_cast(v2h, sr[base + nb]);
             const v8h s8 = {sz[0], sz[0], sz[0], sz[0], sz[0], sz[0], sz[0], sz[0]};
             const v8h z8 = {sz[1], sz[1], sz[1], sz[1], sz[1], sz[1], sz[1], sz[1]};
@@ -591,11 +613,33 @@ struct WoMfmaTile {
           // keeps the scheduler from starting the next sub-block's unpacking and fragment reads early: that costs no time (the
           // other wave of the SIMD fills the gap) and without it the 3-bit tile runs out of registers
           __builtin_amdgcn_sched_barrier(0);
-        }
+          if constexpr (kHalves) {
+            if (j == 1) {
+              // The compiler's waits count its own loads only.  The second halves are awaited here, in front of the activation loads: behind them, a
+              // wait for the halves would be one for these as well.
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
-          wr[base + nb] = w_of(nb, kb + 2);
-          sr[base + nb] = s_of(nb, kb + 2);
+              for (int nb = 0; nb < 4; ++nb) asm volatile("" : "+v"(wr[nb].d[4 % WBITS]), "+v"(wr[nb].d[5 % WBITS]), "+v"(wr[nb].d[6 % WBITS]), "+v"(wr[nb].d[7 % WBITS]));
+              asm volatile("" ::: "memory");
+              dma_x(min(kb + 1, KB - 1), st ^ 1);  // (behind the end of K: the last block once more, into the stage that nobody reads)
+#pragma unroll
+              for (int nb = 0; nb < 4; ++nb) {
+                half_of(wr[nb], 0, nb, kb + 1);
+                sr[(base ^ 4) + nb] = s_of(nb, kb + 1);
+              }
+              asm volatile("" ::: "memory");
+            }
+          }
+        }
+        if constexpr (kHalves) {
+#pragma unroll
+          for (int nb = 0; nb < 4; ++nb) half_of(wr[nb], 1, nb, kb + 1);
+          asm volatile("" ::: "memory");
+        } else {
+#pragma unroll
+          for (int nb = 0; nb < 4; ++nb) {
+            wr[wbase + nb] = w_of(nb, kb + 2);
+            sr[base + nb] = s_of(nb, kb + 2);
+          }
         }
       };
       if (mbv > MB / 2) {

@@ -301,9 +301,7 @@ def get_possible_tile_list(arch: str, qcfg: str) -> list:
         skinny.append(_with_q(TileConfig(BM=32, BN=128, BK=128, WM=1, WN=4, WK=1, STAGE=2, MMA=mma), qcfg))  # experts with 17 .. 32 (.. 64) tokens
         if QCFG_MAP[qcfg].QCFGB.QBITS != 8:  # compiled for 3 waves per SIMD, for kernels made of few-token tiles alone (three workgroups per CU)
             skinny += [_with_q(TileConfig(BM=16, BN=bn, BK=128, WM=1, WN=4, WK=1, STAGE=4, MMA=mma), qcfg) for bn in (128, 64)]
-        # (8-bit weights: the ring of packed blocks is twice as large, which leaves room for the 2 x 2 shape's accumulators only)
-        shapes = ((128, 2, 2),) if QCFG_MAP[qcfg].QCFGB.QBITS == 8 else ((128, 2, 2), (256, 1, 4))
-        big = [_with_q(TileConfig(BM=128, BN=bn, BK=128, WM=wm, WN=wn, WK=1, STAGE=2, MMA=mma), qcfg) for bn, wm, wn in shapes]
+        big = [_with_q(TileConfig(BM=128, BN=bn, BK=128, WM=wm, WN=wn, WK=1, STAGE=2, MMA=mma), qcfg) for bn, wm, wn in ((128, 2, 2), (256, 1, 4))]
         return skinny + big
     bk = {"MFMA_F32_32x32x16_F16": 32, "MFMA_F32_32x32x16_BF16": 32, "MFMA_I32_32x32x32_I8": 64, "MFMA_I32_32x32x32_I8_FROM_I4": 128, "MFMA_F32_32x32x16_FP8": 64}[mma]
     if mma in ("MFMA_F32_32x32x16_F16", "MFMA_F32_32x32x16_BF16"):
