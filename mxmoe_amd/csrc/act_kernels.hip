@@ -227,11 +227,10 @@ typedef unsigned v4u __attribute__((ext_vector_type(4)));
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
 
 // the eight codes of a chunk: v / scale rounded to fp16, clamped to +-7, rounded to the nearest integer (ties to even)
-template <class Div>
-__device__ __forceinline__ v8h bf6_chunk_codes(const float (&v)[8], const Div& div) {
+__device__ __forceinline__ v8h bf6_chunk_codes(const v8h& h, const ScaleDiv& div) {
   v8h o;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) o[j] = (_Float16)rintf(fminf(fmaxf(round_h(div(v[j])), -7.0f), 7.0f));
+  for (int j = 0; j < 8; ++j) o[j] = (_Float16)rintf(fminf(fmaxf(round_h(div((float)h[j])), -7.0f), 7.0f));
   return o;
 }
 
@@ -265,11 +264,11 @@ __device__ __forceinline__ void bf6_emit_row(const uint8_t* codes, int row_elems
 // that is a multiple of 64.
 __device__ __forceinline__ int xcd_row_group(int wg) { return (wg & ~63) | ((wg & 7) << 3) | ((wg >> 3) & 7); }
 
-// What every kernel of one row per workgroup does with a finished row, chunk tid + NT i of it in v[i]: fp16 copy or symmetric quantisation.  `red`: one slot per
+// What every kernel of one row per workgroup does with a finished row, chunk tid + NT i of it in h[i]: fp16 copy or symmetric quantisation.  `red`: one slot per
 // wave; `codes`: LDS for the row as fp16 (tag 4).  Passes barriers only where `tag` is
 // neither 0 nor 3.
 template <int MAXC, int NT, bool EXT>
-__device__ __forceinline__ void store_row(const float (&v)[MAXC][8], int n, int tag, long lrow, long inp_off, long scale_off, uint8_t* inp_store, _Float16* scale_store,
+__device__ __forceinline__ void store_row(const v8h (&h)[MAXC], int n, int tag, long lrow, long inp_off, long scale_off, uint8_t* inp_store, _Float16* scale_store,
                                           float* red, uint8_t* codes) {
   const int tid = threadIdx.x, nchunks = n >> 3;
   if (tag == 0) {
@@ -278,10 +277,7 @@ __device__ __forceinline__ void store_row(const float (&v)[MAXC][8], int n, int 
     for (int i = 0; i < MAXC; ++i) {
       const int c = tid + i * NT;
       if (c < nchunks) {
-        v8h o;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) o[j] = (_Float16)v[i][j];
-        *reinterpret_cast<v8h*>(out + c * 8) = o;
+        *reinterpret_cast<v8h*>(out + c * 8) = h[i];
       }
     }
     return;
@@ -296,38 +292,22 @@ __device__ __forceinline__ void store_row(const float (&v)[MAXC][8], int n, int 
     for (int i = 0; i < MAXC; ++i) {
       const int c = tid + i * NT;
       const bool live = c < nchunks;  // whole lane groups are live or not: n is a multiple of 128
-      float gmax = 0.0f;
-      if (live) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) gmax = fmaxf(gmax, fabsf(v[i][j]));
-      }
-      gmax = row16_max(gmax);
-      float scale = round_h(gmax / 7.0f);
+      HalfMax gmax;
+      if (live) gmax.add(h[i]);
+      float scale = round_h(row16_max_abs(gmax.get()) / 7.0f);
       if (scale == 0.0f) scale = 1.0f;
-      const ScaleDiv div(scale);
       if (live) {
         if ((c & 15) == 0) sout[c >> 4] = (_Float16)scale;
-        unsigned w = 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float r = round_h(div(v[i][j]));
-          w = push_code<4>(w, code_word(fminf(fmaxf(r, -7.0f), 7.0f)));
-        }
-        *reinterpret_cast<unsigned*>(out + c * 4) = w;
+        *reinterpret_cast<unsigned*>(out + c * 4) = HalfDiv(scale).int4(h[i]);
       }
     }
     return;
   }
-  float amax = 0.0f;
+  HalfMax half_max;
 #pragma unroll
-  for (int i = 0; i < MAXC; ++i) {
-    const int c = tid + i * NT;
-    if (c < nchunks) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[i][j]));
-    }
-  }
-  amax = wave_max(amax);
+  for (int i = 0; i < MAXC; ++i)
+    if (tid + i * NT < nchunks) half_max.add(h[i]);
+  float amax = wave_max_abs(half_max.get());
   __syncthreads();
   if ((tid & 63) == 0) red[tid >> 6] = amax;
   __syncthreads();
@@ -337,47 +317,30 @@ __device__ __forceinline__ void store_row(const float (&v)[MAXC][8], int n, int 
   const float upper = tag == 1 ? 127.0f : (EXT && tag == 5 ? 448.0f : 7.0f);
   float scale = round_h(amax / upper);   // fp16 division: fp32 quotient of two fp16 values, rounded to fp16
   if (scale == 0.0f) scale = 1.0f;       // quantize.cuh:258
-  const ScaleDiv div(scale);
+  const ScaleDiv div(scale);  // (fp8 and bf6 codes)
+  const HalfDiv half(scale);
   if (tid == 0) scale_store[scale_off + lrow] = (_Float16)scale;
   if (EXT && tag == 4) {  // the row's codes as fp16 in LDS (in place of the row itself, which every thread is done reading), then fragments
 #pragma unroll
     for (int i = 0; i < MAXC; ++i) {
       const int c = tid + i * NT;
-      if (c < nchunks) *reinterpret_cast<v8h*>(codes + c * 16) = bf6_chunk_codes(v[i], div);
+      if (c < nchunks) *reinterpret_cast<v8h*>(codes + c * 16) = bf6_chunk_codes(h[i], div);
     }
     __syncthreads();
     bf6_emit_row(codes, n, 0, n, inp_store + 2 * inp_off, lrow, tid, NT);
     return;  // (the next row begins with a barrier before it touches LDS)
   }
-  uint8_t* out = inp_store + 2 * (inp_off + lrow * (tag == 1 || (EXT && tag == 5) ? n / 2 : n / 4));
+  uint8_t* out = inp_store + 2 * (inp_off + lrow * (n >> (tag == 1 || (EXT && tag == 5) ? 1 : 2)));
 #pragma unroll
   for (int i = 0; i < MAXC; ++i) {
     const int c = tid + i * NT;
     if (c < nchunks) {
       if (EXT && tag == 5) {
-        *reinterpret_cast<uint2*>(out + c * 8) = fp8_chunk_codes(v[i], div);
+        *reinterpret_cast<uint2*>(out + c * 8) = fp8_chunk_codes(h[i], div);
         continue;
       }
-      unsigned q[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float r = round_h(div(v[i][j]));
-        q[j] = code_word(fminf(fmaxf(r, -upper), upper));
-      }
-      if (tag == 1) {
-        uint2 w{0, 0};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          w.x = push_code<8>(w.x, q[j]);
-          w.y = push_code<8>(w.y, q[j + 4]);
-        }
-        *reinterpret_cast<uint2*>(out + c * 8) = w;
-      } else {
-        unsigned w = 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) w = push_code<4>(w, q[j]);
-        *reinterpret_cast<unsigned*>(out + c * 4) = w;
-      }
+      if (tag == 1) *reinterpret_cast<uint2*>(out + c * 8) = half.int8(h[i]);
+      else *reinterpret_cast<unsigned*>(out + c * 4) = half.int4(h[i]);
     }
   }
 }
@@ -583,7 +546,7 @@ __device__ __forceinline__ void row_quant_body(const RowArgs& a, const int wg, c
             for (int j = 0; j < 8; ++j) mx = fmaxf(mx, fabsf(v[i][j]));
           }
         }
-        mx = wave_max(mx);
+        mx = wave_max_abs(mx);
         if ((tid & 63) == 0) red[tid >> 6] = mx;
         __syncthreads();
         mx = red[0];
@@ -655,7 +618,12 @@ __device__ __forceinline__ void row_quant_body(const RowArgs& a, const int wg, c
       }
     }
 
-    store_row<MAXC, NT, EXT>(v, n, tag, lrow, inp_off, scale_off, a.inp_store, a.scale_store, red, reinterpret_cast<uint8_t*>(x));
+    v8h h[MAXC];
+#pragma unroll
+    for (int i = 0; i < MAXC; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) h[i][j] = (_Float16)v[i][j];
+    store_row<MAXC, NT, EXT>(h, n, tag, lrow, inp_off, scale_off, a.inp_store, a.scale_store, red, reinterpret_cast<uint8_t*>(x));
   }
 }
 
@@ -693,33 +661,25 @@ __global__ void __launch_bounds__(256) row_quant_wave_kernel(const RowArgs a) {
     } else {
       srow = (shared_row ? src_shared : a.src) + (shared_row ? (long)(row - a.R) : source_row(a, row)) * n;
     }
-    float v[NI][8];
+    v8h h[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int c = lane + 64 * i;
-      const v8h g = *reinterpret_cast<const v8h*>(srow + c * 8);
+      h[i] = *reinterpret_cast<const v8h*>(srow + c * 8);
       if (SILU) {
         const v8h u = *reinterpret_cast<const v8h*>(srow + n + c * 8);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float gf = (float)g[j];
-          const float s = silu_fixed(gf);
-          v[i][j] = round_h(keep_f32(s * (float)u[j]));
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[i][j] = (float)g[j];
+        for (int j = 0; j < 8; ++j) h[i][j] = silu_mul_half(h[i][j], u[j]);
+      } else if (!rot) {
+        h[i] = quiet(h[i]);
       }
     }
-    if (rot) wave_rotate<NI>(v, lane, a.plan.scale);
+    if (rot) wave_rotate<NI>(h, lane, a.plan.scale);
     if (tag == 0) {
       _Float16* out = reinterpret_cast<_Float16*>(a.inp_store) + inp_off + lrow * n;
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
-        v8h o;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) o[j] = (_Float16)v[i][j];
-        *reinterpret_cast<v8h*>(out + (lane + 64 * i) * 8) = o;
+        *reinterpret_cast<v8h*>(out + (lane + 64 * i) * 8) = h[i];
       }
       continue;
     }
@@ -729,39 +689,29 @@ __global__ void __launch_bounds__(256) row_quant_wave_kernel(const RowArgs a) {
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
         const int c = lane + 64 * i;
-        float gmax = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) gmax = fmaxf(gmax, fabsf(v[i][j]));
-        gmax = row16_max(gmax);
-        float scale = round_h(gmax / 7.0f);
+        HalfMax gmax;
+        gmax.add(h[i]);
+        float scale = round_h(row16_max_abs(gmax.get()) / 7.0f);
         if (scale == 0.0f) scale = 1.0f;
-        const ScaleDiv div(scale);
-        if ((c & 15) == 0) sout[c >> 4] = (_Float16)scale;
-        unsigned w = 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float r = round_h(div(v[i][j]));
-          w = push_code<4>(w, code_word(fminf(fmaxf(r, -7.0f), 7.0f)));
-        }
-        *reinterpret_cast<unsigned*>(out + c * 4) = w;
+          if ((c & 15) == 0) sout[c >> 4] = (_Float16)scale;
+        *reinterpret_cast<unsigned*>(out + c * 4) = HalfDiv(scale).int4(h[i]);
       }
       continue;
     }
-    float amax = 0.0f;
+    HalfMax half_max;
 #pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[i][j]));
-    amax = wave_max(amax);
+    for (int i = 0; i < NI; ++i) half_max.add(h[i]);
+    float amax = wave_max_abs(half_max.get());
     const float upper = tag == 1 ? 127.0f : (EXT && tag == 5 ? 448.0f : 7.0f);
     float scale = round_h(amax / upper);   // fp16 division: fp32 quotient of two fp16 values, rounded to fp16
     if (scale == 0.0f) scale = 1.0f;       // quantize.cuh:258
-    const ScaleDiv div(scale);
+    const ScaleDiv div(scale);  // (fp8 and bf6 codes)
+    const HalfDiv half(scale);
     if (lane == 0) a.scale_store[scale_off + lrow] = (_Float16)scale;
     if (EXT && tag == 4) {
       uint8_t* codes = wave_codes + wave * (n * 2);
 #pragma unroll
-      for (int i = 0; i < NI; ++i) *reinterpret_cast<v8h*>(codes + (lane + 64 * i) * 16) = bf6_chunk_codes(v[i], div);
+      for (int i = 0; i < NI; ++i) *reinterpret_cast<v8h*>(codes + (lane + 64 * i) * 16) = bf6_chunk_codes(h[i], div);
       asm volatile("" ::: "memory");
       __builtin_amdgcn_wave_barrier();
       bf6_emit_row(codes, n, 0, n, a.inp_store + 2 * inp_off, lrow, lane, 64);
@@ -769,34 +719,16 @@ __global__ void __launch_bounds__(256) row_quant_wave_kernel(const RowArgs a) {
       __builtin_amdgcn_wave_barrier();  // the next row's codes come after these reads
       continue;
     }
-    uint8_t* out = a.inp_store + 2 * (inp_off + lrow * (tag == 1 || (EXT && tag == 5) ? n / 2 : n / 4));
+    uint8_t* out = a.inp_store + 2 * (inp_off + lrow * (n >> (tag == 1 || (EXT && tag == 5) ? 1 : 2)));
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int c = lane + 64 * i;
       if (EXT && tag == 5) {
-        *reinterpret_cast<uint2*>(out + c * 8) = fp8_chunk_codes(v[i], div);
+        *reinterpret_cast<uint2*>(out + c * 8) = fp8_chunk_codes(h[i], div);
         continue;
       }
-      unsigned q[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float r = round_h(div(v[i][j]));
-        q[j] = code_word(fminf(fmaxf(r, -upper), upper));
-      }
-      if (tag == 1) {
-        uint2 w{0, 0};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          w.x = push_code<8>(w.x, q[j]);
-          w.y = push_code<8>(w.y, q[j + 4]);
-        }
-        *reinterpret_cast<uint2*>(out + c * 8) = w;
-      } else {
-        unsigned w = 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) w = push_code<4>(w, q[j]);
-        *reinterpret_cast<unsigned*>(out + c * 4) = w;
-      }
+      if (tag == 1) *reinterpret_cast<uint2*>(out + c * 8) = half.int8(h[i]);
+      else *reinterpret_cast<unsigned*>(out + c * 4) = half.int4(h[i]);
     }
   }
 }
@@ -849,12 +781,12 @@ __global__ void __launch_bounds__(256) token_quant_wave_kernel(const TokenArgs a
     }
     if (present == 0) continue;
     const _Float16* srow = a.src + (long)t * n;
-    float v[NI][8];
+    v8h h[NI];
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const v8h g = *reinterpret_cast<const v8h*>(srow + (lane + 64 * i) * 8);
+    for (int i = 0; i < NI; ++i) h[i] = *reinterpret_cast<const v8h*>(srow + (lane + 64 * i) * 8);
+    if (a.rotate == 0 || (present & 1u)) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[i][j] = (float)g[j];
+      for (int i = 0; i < NI; ++i) h[i] = quiet(h[i]);
     }
     // fp16 copies (tag 0): of the row as it is unless every row is rotated
     auto store_copies = [&]() {
@@ -864,37 +796,26 @@ __global__ void __launch_bounds__(256) token_quant_wave_kernel(const TokenArgs a
           _Float16* out = reinterpret_cast<_Float16*>(a.inp_store) + const_load(a.table + 2 * a.Et + e_of[k]) + lrow_of[k] * n;
 #pragma unroll
           for (int i = 0; i < NI; ++i) {
-            v8h o;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) o[j] = (_Float16)v[i][j];
-            *reinterpret_cast<v8h*>(out + (lane + 64 * i) * 8) = o;
+            *reinterpret_cast<v8h*>(out + (lane + 64 * i) * 8) = h[i];
           }
         }
       }
     };
     if ((present & 1u) && a.rotate != 2) store_copies();
     if ((present & ~1u) == 0 && a.rotate != 2) continue;
-    if (a.rotate != 0) wave_rotate<NI>(v, lane, a.scale);
+    if (a.rotate != 0) wave_rotate<NI>(h, lane, a.scale);
     if ((present & 1u) && a.rotate == 2) store_copies();
     if (present & 0x8u) {  // tag 3: int4, one scale per 128 values = the 16 chunks held by an aligned group of 16 lanes
       unsigned w[NI];
       float gscale[NI];
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
-        float gmax = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) gmax = fmaxf(gmax, fabsf(v[i][j]));
-        gmax = row16_max(gmax);
-        float scale = round_h(gmax / 7.0f);
+        HalfMax gmax;
+        gmax.add(h[i]);
+        float scale = round_h(row16_max_abs(gmax.get()) / 7.0f);
         if (scale == 0.0f) scale = 1.0f;
-        const ScaleDiv div(scale);
         gscale[i] = scale;
-        w[i] = 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float r = round_h(div(v[i][j]));
-          w[i] = push_code<4>(w[i], code_word(fminf(fmaxf(r, -7.0f), 7.0f)));
-        }
+        w[i] = HalfDiv(scale).int4(h[i]);
       }
 #pragma unroll
       for (int k = 0; k < KD; ++k) {
@@ -911,26 +832,17 @@ __global__ void __launch_bounds__(256) token_quant_wave_kernel(const TokenArgs a
       }
     }
     if ((present & 0x6u) == 0) continue;
-    float amax = 0.0f;
+    HalfMax half_max;
 #pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[i][j]));
-    amax = wave_max(amax);
+    for (int i = 0; i < NI; ++i) half_max.add(h[i]);
+    float amax = wave_max_abs(half_max.get());
     if (present & 0x2u) {  // tag 1: int8 per token
       float scale = round_h(amax / 127.0f);  // fp16 division: fp32 quotient of two fp16 values, rounded to fp16
       if (scale == 0.0f) scale = 1.0f;       // quantize.cuh:258
-      const ScaleDiv div(scale);
+      const HalfDiv half(scale);
       uint2 w[NI];
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        w[i] = uint2{0, 0};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          w[i].x = push_code<8>(w[i].x, code_word(fminf(fmaxf(round_h(div(v[i][j])), -127.0f), 127.0f)));
-          w[i].y = push_code<8>(w[i].y, code_word(fminf(fmaxf(round_h(div(v[i][j + 4])), -127.0f), 127.0f)));
-        }
-      }
+      for (int i = 0; i < NI; ++i) w[i] = half.int8(h[i]);
 #pragma unroll
       for (int k = 0; k < KD; ++k) {
         if (k < ndst && tag_of[k] == 1) {
@@ -944,14 +856,10 @@ __global__ void __launch_bounds__(256) token_quant_wave_kernel(const TokenArgs a
     if (present & 0x4u) {  // tag 2: int4 per token
       float scale = round_h(amax / 7.0f);
       if (scale == 0.0f) scale = 1.0f;
-      const ScaleDiv div(scale);
+      const HalfDiv half(scale);
       unsigned w[NI];
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        w[i] = 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) w[i] = push_code<4>(w[i], code_word(fminf(fmaxf(round_h(div(v[i][j])), -7.0f), 7.0f)));
-      }
+      for (int i = 0; i < NI; ++i) w[i] = half.int4(h[i]);
 #pragma unroll
       for (int k = 0; k < KD; ++k) {
         if (k < ndst && tag_of[k] == 2) {
@@ -1054,26 +962,13 @@ __device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int
     const RowMeta cur = next_meta;
     const bool has_next = row + stride_rows < a.rows;
     if (has_next) next_meta = load_meta(row + stride_rows);
-    float v[MAXC][8];
+    v8h h[MAXC];
 #pragma unroll
     for (int i = 0; i < MAXC; ++i) {
-      const bool live = lane + 64 * i < nchunks;
-      const v8h g = row_g[i];
+      h[i] = row_g[i];  // (lanes past the row hold its last chunk again: its maxima stay what they are, and it is never stored)
       if (SILU) {
-        const v8h u = row_u[i];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float gf = (float)g[j];
-          const float sl = silu_fixed(gf);
-          v[i][j] = round_h(keep_f32(sl * (float)u[j]));
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[i][j] = (float)g[j];
-      }
-      if (!live) {  // chunks past the row count as zeros (in the row's maxima) and are never stored
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[i][j] = 0.0f;
+        for (int j = 0; j < 8; ++j) h[i][j] = silu_mul_half(row_g[i][j], row_u[i][j]);
       }
     }
     if (has_next) load_data(next_meta, row_g, row_u);
@@ -1086,24 +981,11 @@ __device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int
       float mx = 0.0f;
 #pragma unroll
       for (int i = 0; i < MAXC; ++i) {
-#pragma unroll
-        for (int h = 1; h < 8; h <<= 1)
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (!(j & h)) {
-              const float p = v[i][j], q = v[i][j + h];
-              v[i][j] = p + q;
-              v[i][j + h] = p - q;
-            }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          v[i][j] = round_h(keep_f32(v[i][j] * pl.scale));
-          mx = fmaxf(mx, fabsf(v[i][j]));
-        }
+        float v[8];
+        chunk_h8(h[i], v);
+        h[i] = scale_chunk(v, pl.scale, mx);
       }
-      mx = wave_max(mx);
-      const DenseGrid grid(mx);
-      const float to16 = grid.to_grid * 0.0625f;  // exact (a power of two well inside the range); rint(v * to_grid) / 16 below
+      const DenseGrid grid(round_h(wave_max_abs(mx)));
       // transposed write: chunk c = blk * kb + b' -> columns blk * 8 + j, position b'
 #pragma unroll
       for (int i = 0; i < MAXC; ++i) {
@@ -1111,11 +993,11 @@ __device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int
         if (c < nchunks) {
           const int blk = c / kb, bp = c - blk * kb;
           uint8_t* dst = xt + (blk * 8) * kDensePitch + bp * 2;
+          const v8h q = snap_chunk(h[i], grid.to_grid);
 #pragma unroll
-          for (int j = 0; j < 8; ++j) *reinterpret_cast<_Float16*>(dst + j * kDensePitch) = (_Float16)(rintf(v[i][j] * grid.to_grid) * 0.0625f);
+          for (int j = 0; j < 8; ++j) *reinterpret_cast<_Float16*>(dst + j * kDensePitch) = q[j];
         }
       }
-      (void)to16;
       asm volatile("" ::: "memory");
       __builtin_amdgcn_wave_barrier();
       // lane holds column col = 16 nb + (lane & 15), i.e. blk = 2 nb + ((lane >> 3) & 1), j = lane & 7, and rows b = 16 mb + 4 (lane >> 4) + r
@@ -1196,13 +1078,13 @@ __device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int
 #pragma unroll
       for (int i = 0; i < MAXC; ++i) {
         const int c = min(lane + 64 * i, nchunks - 1);
-        const bool live = lane + 64 * i < nchunks;
-        const v8h y = *reinterpret_cast<const v8h*>(yrow + c * 16);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[i][j] = live ? (float)y[j] : 0.0f;
+        h[i] = *reinterpret_cast<const v8h*>(yrow + c * 16);
       }
       asm volatile("" ::: "memory");
       __builtin_amdgcn_wave_barrier();  // the next row's writes come after these reads
+    } else if (!SILU) {
+#pragma unroll
+      for (int i = 0; i < MAXC; ++i) h[i] = quiet(h[i]);
     }
 
     // ---- store: fp16 copy or symmetric quantisation (as in the other row kernels) ----
@@ -1213,10 +1095,7 @@ __device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int
       for (int i = 0; i < MAXC; ++i) {
         const int c = lane + 64 * i;
         if (c < nchunks) {
-          v8h o;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) o[j] = (_Float16)v[i][j];
-          *reinterpret_cast<v8h*>(out + c * 8) = o;
+          *reinterpret_cast<v8h*>(out + c * 8) = h[i];
         }
       }
       continue;
@@ -1228,42 +1107,32 @@ __device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int
       for (int i = 0; i < MAXC; ++i) {
         const int c = lane + 64 * i;
         const bool live = c < nchunks;  // whole lane groups are live or not: n is a multiple of 128
-        float gmax = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) gmax = fmaxf(gmax, fabsf(v[i][j]));
-        gmax = row16_max(gmax);
-        float scale = round_h(gmax / 7.0f);
+        HalfMax gmax;
+        gmax.add(h[i]);
+        float scale = round_h(row16_max_abs(gmax.get()) / 7.0f);
         if (scale == 0.0f) scale = 1.0f;
-        const ScaleDiv div(scale);
-        if (live) {
+          if (live) {
           if ((c & 15) == 0) sout[c >> 4] = (_Float16)scale;
-          unsigned w = 0;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const float r = round_h(div(v[i][j]));
-            w = push_code<4>(w, code_word(fminf(fmaxf(r, -7.0f), 7.0f)));
-          }
-          *reinterpret_cast<unsigned*>(out + c * 4) = w;
+          *reinterpret_cast<unsigned*>(out + c * 4) = HalfDiv(scale).int4(h[i]);
         }
       }
       continue;
     }
-    float amax = 0.0f;
+    HalfMax half_max;
 #pragma unroll
-    for (int i = 0; i < MAXC; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[i][j]));  // chunks past the row hold zeros
-    amax = wave_max(amax);
+    for (int i = 0; i < MAXC; ++i) half_max.add(h[i]);
+    float amax = wave_max_abs(half_max.get());
     const float upper = tag == 1 ? 127.0f : (EXT && tag == 5 ? 448.0f : 7.0f);
     float scale = round_h(amax / upper);   // fp16 division: fp32 quotient of two fp16 values, rounded to fp16
     if (scale == 0.0f) scale = 1.0f;       // quantize.cuh:258
-    const ScaleDiv div(scale);
+    const ScaleDiv div(scale);  // (fp8 and bf6 codes)
+    const HalfDiv half(scale);
     if (lane == 0) a.scale_store[scale_off + lrow] = (_Float16)scale;
     if (EXT && tag == 4) {  // codes into the wave's row buffer (its reads of the rotated row are behind a wave barrier), then fragments
 #pragma unroll
       for (int i = 0; i < MAXC; ++i) {
         const int c = lane + 64 * i;
-        if (c < nchunks) *reinterpret_cast<v8h*>(yrow + c * 16) = bf6_chunk_codes(v[i], div);
+        if (c < nchunks) *reinterpret_cast<v8h*>(yrow + c * 16) = bf6_chunk_codes(h[i], div);
       }
       asm volatile("" ::: "memory");
       __builtin_amdgcn_wave_barrier();
@@ -1272,35 +1141,17 @@ __device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int
       __builtin_amdgcn_wave_barrier();  // the next row's writes come after these reads
       continue;
     }
-    uint8_t* out = a.inp_store + 2 * (inp_off + lrow * (tag == 1 || (EXT && tag == 5) ? n / 2 : n / 4));
+    uint8_t* out = a.inp_store + 2 * (inp_off + lrow * (n >> (tag == 1 || (EXT && tag == 5) ? 1 : 2)));
 #pragma unroll
     for (int i = 0; i < MAXC; ++i) {
       const int c = lane + 64 * i;
       if (c < nchunks) {
         if (EXT && tag == 5) {
-          *reinterpret_cast<uint2*>(out + c * 8) = fp8_chunk_codes(v[i], div);
+          *reinterpret_cast<uint2*>(out + c * 8) = fp8_chunk_codes(h[i], div);
           continue;
         }
-        unsigned q[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float r = round_h(div(v[i][j]));
-          q[j] = code_word(fminf(fmaxf(r, -upper), upper));
-        }
-        if (tag == 1) {
-          uint2 w{0, 0};
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            w.x = push_code<8>(w.x, q[j]);
-            w.y = push_code<8>(w.y, q[j + 4]);
-          }
-          *reinterpret_cast<uint2*>(out + c * 8) = w;
-        } else {
-          unsigned w = 0;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) w = push_code<4>(w, q[j]);
-          *reinterpret_cast<unsigned*>(out + c * 4) = w;
-        }
+        if (tag == 1) *reinterpret_cast<uint2*>(out + c * 8) = half.int8(h[i]);
+        else *reinterpret_cast<unsigned*>(out + c * 4) = half.int4(h[i]);
       }
     }
   }
@@ -1428,15 +1279,13 @@ __device__ __forceinline__ void row_quant_block_body(const RowArgs& a, const int
     const RowMeta cur = next_meta;
     const bool has_next = row + wgs < a.rows;
     if (has_next) next_meta = load_meta(row + wgs);
-    float v[MAXC][8];
+    v8h h[MAXC];
 #pragma unroll
     for (int i = 0; i < MAXC; ++i) {
-      const bool live = tid + NT * i < nchunks;
+      h[i] = row_g[i];  // (threads past the row hold its last chunk again: its maxima stay what they are, and it is never stored)
+      if constexpr (SILU) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float x = (float)row_g[i][j];
-        const float y = SILU ? round_h(keep_f32(silu_fixed(x) * (float)row_u[i][j])) : x;
-        v[i][j] = live ? y : 0.0f;  // (chunks past the row count as zeros in its maxima and are never stored)
+        for (int j = 0; j < 8; ++j) h[i][j] = silu_mul_half(row_g[i][j], row_u[i][j]);
       }
     }
     if (has_next) load_data(next_meta, row_g, row_u);
@@ -1448,46 +1297,31 @@ __device__ __forceinline__ void row_quant_block_body(const RowArgs& a, const int
       float mx = 0.0f;
 #pragma unroll
       for (int i = 0; i < MAXC; ++i) {
+        float v[8];
+        v8h x = h[i];
+        if (tid + NT * i >= nchunks) {  // (the lane stages would add up what threads past the row hold)
 #pragma unroll
-        for (int h = 1; h < 8; h <<= 1)
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (!(j & h)) {
-              const float p = v[i][j], q = v[i][j + h];
-              v[i][j] = p + q;
-              v[i][j + h] = p - q;
-            }
-        // strides 8 .. m / 2: the partner chunk is 1 .. 8 lanes away
-        auto stage = [&](auto dc) {
-#pragma unroll
-          for (int j = 0; j < 8; j += 2) lane_butterfly<decltype(dc)::value>(v[i][j], v[i][j + 1], lane);
-        };
-        if (mc > 1) stage(std::integral_constant<int, 1>{});
-        if (mc > 2) stage(std::integral_constant<int, 2>{});
-        if (mc > 4) stage(std::integral_constant<int, 4>{});
-        if (mc > 8) stage(std::integral_constant<int, 8>{});
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          v[i][j] = round_h(keep_f32(v[i][j] * pl.scale));
-          mx = fmaxf(mx, fabsf(v[i][j]));
+          for (int j = 0; j < 8; ++j) x[j] = (_Float16)0.0f;
         }
+        chunk_h8(x, v);
+        // strides 8 .. m / 2: the partner chunk is 1 .. 8 lanes away
+        if (mc > 1) lane_stage<1>(v, lane);
+        if (mc > 2) lane_stage<2>(v, lane);
+        if (mc > 4) lane_stage<4>(v, lane);
+        if (mc > 8) lane_stage<8>(v, lane);
+        h[i] = scale_chunk(v, pl.scale, mx);
       }
-      mx = wave_max(mx);
+      mx = wave_max_abs(mx);
       if (lane == 0) red[wave] = mx;
       __syncthreads();
       mx = red[0];
 #pragma unroll
       for (int w = 1; w < kW; ++w) mx = fmaxf(mx, red[w]);
-      const DenseGrid grid(mx);
+      const DenseGrid grid(round_h(mx));
 #pragma unroll
       for (int i = 0; i < MAXC; ++i) {
         const int c = tid + NT * i;
-        if (c < nchunks) {
-          v8h q;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) q[j] = (_Float16)(rintf(v[i][j] * grid.to_grid) * 0.0625f);
-          *reinterpret_cast<RowChunk*>(xt + at_x(c)) = q;
-        }
+        if (c < nchunks) *reinterpret_cast<RowChunk*>(xt + at_x(c)) = snap_chunk(h[i], grid.to_grid);
       }
       __syncthreads();
       const float back = grid.from_grid * 16.0f;
@@ -1586,14 +1420,13 @@ __device__ __forceinline__ void row_quant_block_body(const RowArgs& a, const int
 #pragma unroll
       for (int i = 0; i < MAXC; ++i) {
         const int c = tid + NT * i;
-        if (c < nchunks) {
-          const v8h y = *reinterpret_cast<const RowChunk*>(yrow + at_y(c));
-#pragma unroll
-          for (int j = 0; j < 8; ++j) v[i][j] = (float)y[j];
-        }
+        if (c < nchunks) h[i] = *reinterpret_cast<const RowChunk*>(yrow + at_y(c));
       }
+    } else if (!SILU) {
+#pragma unroll
+      for (int i = 0; i < MAXC; ++i) h[i] = quiet(h[i]);
     }
-    store_row<MAXC, NT, EXT>(v, n, tag, cur.lrow, cur.inp_off, cur.scale_off, a.inp_store, a.scale_store, red + kW, yrow);
+    store_row<MAXC, NT, EXT>(h, n, tag, cur.lrow, cur.inp_off, cur.scale_off, a.inp_store, a.scale_store, red + kW, yrow);
   }
 }
 template <int MAXC, bool SILU, bool EXT>
@@ -1678,28 +1511,23 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
     }
     // A k row past kb (the last of a wave's four when kb is not a multiple of 8: waves 4 .. 7 of a 28-row view) costs nothing: the
     // whole wave skips its loads, its SiLU and its butterflies, and the slot holds zeros.
-    float v[MAXC][8];
+    v8h h[MAXC];
 #pragma unroll
     for (int i = 0; i < MAXC; ++i) {
       const int kr = wave + 8 * i;
       if (kr < kb) {
         const int c = kr * 64 + lane;  // chunk index in the row
-        const v8h g = *reinterpret_cast<const v8h*>(srow + c * 8);
+        h[i] = *reinterpret_cast<const v8h*>(srow + c * 8);
         if (SILU) {
           const v8h u = *reinterpret_cast<const v8h*>(srow + n + c * 8);
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const float gf = (float)g[j];
-            const float sl = silu_fixed(gf);
-            v[i][j] = round_h(keep_f32(sl * (float)u[j]));
-          }
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) v[i][j] = (float)g[j];
+          for (int j = 0; j < 8; ++j) h[i][j] = silu_mul_half(h[i][j], u[j]);
+        } else if (!rot) {
+          h[i] = quiet(h[i]);
         }
       } else {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[i][j] = 0.0f;
+        for (int j = 0; j < 8; ++j) h[i][j] = (_Float16)0.0f;
       }
     }
     if (rot) {
@@ -1708,48 +1536,28 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
 #pragma unroll
       for (int i = 0; i < MAXC; ++i) {
         if (wave + 8 * i >= kb) continue;
-#pragma unroll
-        for (int h = 1; h < 8; h <<= 1)
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (!(j & h)) {
-              const float p = v[i][j], q = v[i][j + h];
-              v[i][j] = p + q;
-              v[i][j + h] = p - q;
-            }
-        auto lane_stage = [&](auto mc) {
-#pragma unroll
-          for (int j = 0; j < 8; j += 2) lane_butterfly<decltype(mc)::value>(v[i][j], v[i][j + 1], lane);
-        };
-        lane_stage(std::integral_constant<int, 1>{});
-        lane_stage(std::integral_constant<int, 2>{});
-        lane_stage(std::integral_constant<int, 4>{});
-        lane_stage(std::integral_constant<int, 8>{});
-        lane_stage(std::integral_constant<int, 16>{});
-        lane_stage(std::integral_constant<int, 32>{});
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          v[i][j] = round_h(keep_f32(v[i][j] * pl.scale));
-          mx = fmaxf(mx, fabsf(v[i][j]));
-        }
+        float v[8];
+        chunk_h8(h[i], v);
+        lane_stage<1>(v, lane);
+        lane_stage<2>(v, lane);
+        lane_stage<4>(v, lane);
+        lane_stage<8>(v, lane);
+        lane_stage<16>(v, lane);
+        lane_stage<32>(v, lane);
+        h[i] = scale_chunk(v, pl.scale, mx);
       }
-      mx = wave_max(mx);
+      mx = wave_max_abs(mx);
       if (lane == 0) red[wave] = mx;
       __syncthreads();  // (also: the previous row's readers of xt / yrow are done)
       mx = red[0];
 #pragma unroll
       for (int w = 1; w < 8; ++w) mx = fmaxf(mx, red[w]);
-      const DenseGrid grid(mx);
+      const DenseGrid grid(round_h(mx));
       // the snapped row, k row kr / chunk lane at its place
 #pragma unroll
       for (int i = 0; i < MAXC; ++i) {
         const int kr = wave + 8 * i;
-        if (kr < kb) {
-          v8h q;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) q[j] = (_Float16)(rintf(v[i][j] * grid.to_grid) * 0.0625f);
-          *reinterpret_cast<v8h*>(xt + kr * kWidePitch + lane * 16) = q;
-        }
+        if (kr < kb) *reinterpret_cast<v8h*>(xt + kr * kWidePitch + lane * 16) = snap_chunk(h[i], grid.to_grid);
       }
       __syncthreads();
       // this wave's 64 columns: 4 column blocks x 2 row blocks; the second operand of a lane is column col, k = 8 (lane >> 4) + 0..7
@@ -1776,9 +1584,7 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
       for (int i = 0; i < MAXC; ++i) {
         const int kr = wave + 8 * i;
         if (kr >= kb) continue;  // (still zeros)
-        const v8h y = *reinterpret_cast<const v8h*>(yrow + kr * kWidePitch + lane * 16);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[i][j] = (float)y[j];
+        h[i] = *reinterpret_cast<const v8h*>(yrow + kr * kWidePitch + lane * 16);
       }
     }
 
@@ -1789,10 +1595,7 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
       for (int i = 0; i < MAXC; ++i) {
         const int kr = wave + 8 * i;
         if (kr < kb) {
-          v8h o;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) o[j] = (_Float16)v[i][j];
-          *reinterpret_cast<v8h*>(out + (kr * 64 + lane) * 8) = o;
+          *reinterpret_cast<v8h*>(out + (kr * 64 + lane) * 8) = h[i];
         }
       }
       continue;
@@ -1805,30 +1608,19 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
         const int kr = wave + 8 * i;
         if (kr >= kb) continue;
         const int c = kr * 64 + lane;
-        float gmax = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) gmax = fmaxf(gmax, fabsf(v[i][j]));
-        gmax = row16_max(gmax);
-        float scale = round_h(gmax / 7.0f);
+        HalfMax gmax;
+        gmax.add(h[i]);
+        float scale = round_h(row16_max_abs(gmax.get()) / 7.0f);
         if (scale == 0.0f) scale = 1.0f;
-        const ScaleDiv div(scale);
-        if ((c & 15) == 0) sout[c >> 4] = (_Float16)scale;
-        unsigned w = 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float r = round_h(div(v[i][j]));
-          w = push_code<4>(w, code_word(fminf(fmaxf(r, -7.0f), 7.0f)));
-        }
-        *reinterpret_cast<unsigned*>(out + c * 4) = w;
+          if ((c & 15) == 0) sout[c >> 4] = (_Float16)scale;
+        *reinterpret_cast<unsigned*>(out + c * 4) = HalfDiv(scale).int4(h[i]);
       }
       continue;
     }
-    float amax = 0.0f;
+    HalfMax half_max;
 #pragma unroll
-    for (int i = 0; i < MAXC; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[i][j]));
-    amax = wave_max(amax);
+    for (int i = 0; i < MAXC; ++i) half_max.add(h[i]);
+    float amax = wave_max_abs(half_max.get());
     if (lane == 0) red[8 + wave] = amax;
     __syncthreads();
     amax = red[8];
@@ -1837,50 +1629,33 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
     const float upper = tag == 1 ? 127.0f : (EXT && tag == 5 ? 448.0f : 7.0f);
     float scale = round_h(amax / upper);   // fp16 division: fp32 quotient of two fp16 values, rounded to fp16
     if (scale == 0.0f) scale = 1.0f;       // quantize.cuh:258
-    const ScaleDiv div(scale);
+    const ScaleDiv div(scale);  // (fp8 and bf6 codes)
+    const HalfDiv half(scale);
     if (tid == 0) a.scale_store[scale_off + lrow] = (_Float16)scale;
     if (EXT && tag == 4) {  // codes into the rotated row's buffer, each wave over its own k rows, then fragments by the whole workgroup
       __syncthreads();  // (a row that was not rotated did not pass the barriers that order the previous row's readers of this buffer)
 #pragma unroll
       for (int i = 0; i < MAXC; ++i) {
         const int kr = wave + 8 * i;
-        if (kr < kb) *reinterpret_cast<v8h*>(yrow + kr * kWidePitch + lane * 16) = bf6_chunk_codes(v[i], div);
+        if (kr < kb) *reinterpret_cast<v8h*>(yrow + kr * kWidePitch + lane * 16) = bf6_chunk_codes(h[i], div);
       }
       __syncthreads();
       bf6_emit_row(yrow, 512, kWidePitch, n, a.inp_store + 2 * inp_off, lrow, tid, 512);
       __syncthreads();
       continue;
     }
-    uint8_t* out = a.inp_store + 2 * (inp_off + lrow * (tag == 1 || (EXT && tag == 5) ? n / 2 : n / 4));
+    uint8_t* out = a.inp_store + 2 * (inp_off + lrow * (n >> (tag == 1 || (EXT && tag == 5) ? 1 : 2)));
 #pragma unroll
     for (int i = 0; i < MAXC; ++i) {
       const int kr = wave + 8 * i;
       if (kr < kb) {
         const int c = kr * 64 + lane;
         if (EXT && tag == 5) {
-          *reinterpret_cast<uint2*>(out + c * 8) = fp8_chunk_codes(v[i], div);
+          *reinterpret_cast<uint2*>(out + c * 8) = fp8_chunk_codes(h[i], div);
           continue;
         }
-        unsigned q[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float r = round_h(div(v[i][j]));
-          q[j] = code_word(fminf(fmaxf(r, -upper), upper));
-        }
-        if (tag == 1) {
-          uint2 w{0, 0};
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            w.x = push_code<8>(w.x, q[j]);
-            w.y = push_code<8>(w.y, q[j + 4]);
-          }
-          *reinterpret_cast<uint2*>(out + c * 8) = w;
-        } else {
-          unsigned w = 0;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) w = push_code<4>(w, q[j]);
-          *reinterpret_cast<unsigned*>(out + c * 4) = w;
-        }
+        if (tag == 1) *reinterpret_cast<uint2*>(out + c * 8) = half.int8(h[i]);
+        else *reinterpret_cast<unsigned*>(out + c * 4) = half.int4(h[i]);
       }
     }
   }

@@ -17,15 +17,6 @@ __device__ __forceinline__ T const_load(const T* p) {
 
 __device__ __forceinline__ float round_h(float v) { return (float)(_Float16)v; }
 
-// Integer code of a value already clamped to the code range, as the low bits of a word: the addition of 1.5 * 2^23 rounds to an
-// integer by itself (to nearest, ties to even: rintf) and leaves its two's complement in the low mantissa bits.  push_code<BITS>
-// shifts a word of codes right by BITS and puts the new code on top: after 32 / BITS pushes the first code sits in the lowest bits.
-__device__ __forceinline__ unsigned code_word(float clamped) { return __float_as_uint(clamped + 12582912.0f); }
-template <int BITS>
-__device__ __forceinline__ unsigned push_code(unsigned w, unsigned code) {
-  return __builtin_amdgcn_alignbit(code, w, BITS);
-}
-
 // v / s in fp32 for fp16-valued v and s, given r = 1.0f / s: the rounded product v * r corrected once with its exact remainder.
 // With r the correctly rounded reciprocal this is the correctly rounded quotient, i.e. bit for bit what the division instruction
 // sequence returns, for every pair of fp16 values (checked with exact integer arithmetic over all 2^20 mantissa pairs in
@@ -40,6 +31,112 @@ struct ScaleDiv {
     return __builtin_fmaf(e, r, q0);
   }
 };
+
+// A finished row is held as what it is, fp16 values, eight to a chunk: half the registers of fp32 copies, and two values to an instruction in its maximum and its
+// codes.  (The quantisers are bound by their vector instructions; with fp32 copies a code took nine and a value of the maximum three.)
+
+// Largest magnitude: two values of a chunk per instruction, NaN ignored as fmaxf ignores it.
+struct HalfMax {
+  unsigned m = 0;  // an fp16 value in the low half
+  __device__ __forceinline__ void add(const v8h& h) {
+    const v4i w = __builtin_bit_cast(v4i, h);
+#pragma unroll
+    for (int d = 0; d < 4; ++d) asm("v_max3_f16 %0, |%1|, |%1|, %2 op_sel:[0,1,0,0]" : "=v"(m) : "v"(w[d]), "v"(m));
+  }
+  __device__ __forceinline__ float get() const { return (float)__builtin_bit_cast(_Float16, (unsigned short)m); }
+};
+// A row that goes on as it was read: signalling NaNs become quiet ones, as a trip through fp32 makes them.
+__device__ __forceinline__ v8h quiet(const v8h& h) { return __builtin_elementwise_canonicalize(h); }
+
+// Integer codes of a row whose scale is known: clamp(fp16(v / scale), +-UPPER) rounded to the nearest integer, ties to even.  Two values at a time in fp16: value and
+// scale times the power of two that brings the scale into 1 .. 2 (a scale below the normal numbers: into 2^-9 .. 1), the product with the reciprocal corrected
+// once with its remainder, and 1536 added, where fp16 numbers are integers, so that the code's two's complement is left in the low mantissa bits.  The same
+// code as from the fp32 quotient for every value and scale that a row can have (test_codes_from_packed_halves_are_those_of_the_fp32_quotient goes through all
+// of them).  An infinite scale (a row that holds an infinity) keeps the plain product: finite / inf = 0.
+struct HalfDiv {
+  v2h up, s, r;  // both halves alike
+  __device__ __forceinline__ explicit HalfDiv(float scale) {
+    const int e = (__float_as_int(scale) >> 23) - 127;  // scale > 0
+    const float f = __int_as_float((127 + min(max(-e, -15), 15)) << 23);
+    const _Float16 hu = (_Float16)f, hs = (_Float16)(__builtin_isinf(scale) ? 0.0f : scale * f), hr = (_Float16)__builtin_amdgcn_rcpf(scale * f);
+    up = v2h{hu, hu};
+    s = v2h{hs, hs};
+    r = v2h{hr, hr};
+  }
+  template <int UPPER>
+  __device__ __forceinline__ unsigned codes(v2h v) const {
+    const v2h x = v * up;
+    const v2h q0 = x * r;
+    v2h q = __builtin_elementwise_fma(__builtin_elementwise_fma(-q0, s, x), r, q0);
+    const _Float16 top = UPPER, magic = 1536;
+    q = __builtin_elementwise_min(__builtin_elementwise_max(q, v2h{-top, -top}), v2h{top, top});
+    return __builtin_bit_cast(unsigned, q + v2h{magic, magic});
+  }
+  template <int UPPER>
+  __device__ __forceinline__ void codes8(const v8h& h, unsigned (&w)[4]) const {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) w[d] = codes<UPPER>(v2h{h[2 * d], h[2 * d + 1]});
+  }
+  // eight int8 codes, the first in the lowest byte
+  __device__ __forceinline__ uint2 int8(const v8h& h) const {
+    unsigned w[4];
+    codes8<127>(h, w);
+    return make_uint2(__builtin_amdgcn_perm(w[1], w[0], 0x06040200), __builtin_amdgcn_perm(w[3], w[2], 0x06040200));
+  }
+  // eight int4 codes, the first in the lowest bits
+  __device__ __forceinline__ unsigned int4(const v8h& h) const {
+    unsigned w[4];
+    codes8<7>(h, w);
+    const unsigned a = __builtin_amdgcn_perm(w[1], w[0], 0x06020400), b = __builtin_amdgcn_perm(w[3], w[2], 0x06020400);  // codes 0 2 1 3, 4 6 5 7
+    const unsigned even = __builtin_amdgcn_perm(b, a, 0x05040100), odd = __builtin_amdgcn_perm(b, a, 0x07060302);
+    return (even & 0x0F0F0F0Fu) | (odd << 4 & 0xF0F0F0F0u);
+  }
+};
+
+// H_8 of a chunk of fp16 values, in fp32: strides 1, 2, 4.  The first stage takes the halves as they are (mixed-precision fused multiply-adds by one and minus one:
+// sums and differences rounded once, without conversions in front).
+__device__ __forceinline__ void chunk_h8(const v8h& h, float (&v)[8]) {
+  float one = 1.0f;
+  asm("" : "+s"(one));  // (a multiplication by a visible 1 would be folded away, and with it the mixed-precision form)
+#pragma unroll
+  for (int j = 0; j < 8; j += 2) {
+    v[j] = __builtin_fmaf((float)h[j + 1], one, (float)h[j]);
+    v[j + 1] = __builtin_fmaf((float)h[j + 1], -one, (float)h[j]);
+  }
+#pragma unroll
+  for (int st = 2; st < 8; st <<= 1)
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (!(j & st)) {
+        const float p = v[j], q = v[j + st];
+        v[j] = p + q;
+        v[j + st] = p - q;
+      }
+}
+
+// fp16(v * scale), the product rounded to fp32 first; `mx` follows the largest magnitude (of the products: their maximum, rounded, is that of the rounded ones)
+__device__ __forceinline__ v8h scale_chunk(const float (&v)[8], float scale, float& mx) {
+  v8h h;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float p = keep_f32(v[j] * scale);
+    h[j] = (_Float16)p;
+    mx = fmaxf(mx, fabsf(p));
+  }
+  return h;
+}
+
+// The chunk on the exact grid of the dense stage: rint(h * to_grid) / 16, a number of at most 2^13 in steps of 1/16.  One fused operation rounds to the grid
+// (beside 1.5 * 2^19 an fp32 number has steps of 1/16), one takes the offset off and converts; both are exact otherwise.
+__device__ __forceinline__ v8h snap_chunk(const v8h& h, float to_grid) {
+  const float to16 = to_grid * 0.0625f;
+  float one = 1.0f, off = 786432.0f;
+  asm("" : "+s"(one), "+s"(off));
+  v8h q;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) q[j] = (_Float16)__builtin_fmaf(__builtin_fmaf((float)h[j], to16, off), one, -off);
+  return q;
+}
 
 // Value of lane (l ^ M), M = 1 .. 8: data-parallel-primitive moves inside a row of 16 lanes, in the vector ALU (quad permutations;
 // l ^ 4 = mirror of 8 lanes, then of 4; l ^ 8 = a rotation of the row by 8).
@@ -88,6 +185,27 @@ __device__ __forceinline__ void lane_butterfly(float& a, float& b, int lane) {
   }
 }
 
+// The stage across lanes l ^ M for the eight values of a chunk.
+// M = 4: the partner is four lanes up for the even quads of a row of 16 lanes and four lanes down for the odd ones, so an addition with its exchange built in writes
+// the even quads and a subtraction the odd ones (bank masks): two instructions a value, where an exchange of that distance takes two by itself.  (Two wait
+// states are due between a vector write and a lane exchange that reads it: the compiler does not see into the block.)
+template <int M>
+__device__ __forceinline__ void lane_stage(float (&v)[8], int lane) {
+  if constexpr (M == 4) {
+    float o[8];
+#define MXMOE_XOR4(n, src) "\n\tv_add_f32_dpp %" #n ", %" #src ", %" #src " row_shl:4 row_mask:0xf bank_mask:0x5\n\tv_sub_f32_dpp %" #n ", %" #src ", %" #src " row_shr:4 row_mask:0xf bank_mask:0xa"
+    asm("s_nop 1" MXMOE_XOR4(0, 8) MXMOE_XOR4(1, 9) MXMOE_XOR4(2, 10) MXMOE_XOR4(3, 11) MXMOE_XOR4(4, 12) MXMOE_XOR4(5, 13) MXMOE_XOR4(6, 14) MXMOE_XOR4(7, 15) "\n\ts_nop 1"
+        : "=&v"(o[0]), "=&v"(o[1]), "=&v"(o[2]), "=&v"(o[3]), "=&v"(o[4]), "=&v"(o[5]), "=&v"(o[6]), "=&v"(o[7])
+        : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]));
+#undef MXMOE_XOR4
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = o[j];
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) lane_butterfly<M>(v[j], v[j + 1], lane);
+  }
+}
+
 // Largest value over the wave of values that are not negative (or NaN-free in general), in every lane; vector ALU only.
 __device__ __forceinline__ float wave_max(float v) {
   v = fmaxf(v, lane_xor<1>(v));
@@ -99,22 +217,32 @@ __device__ __forceinline__ float wave_max(float v) {
   const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
-// Largest value over each aligned group of 16 lanes.
-__device__ __forceinline__ float row16_max(float v) {
-  v = fmaxf(v, lane_xor<8>(v));
-  v = fmaxf(v, lane_xor<4>(v));
-  v = fmaxf(v, lane_xor<2>(v));
-  return fmaxf(v, lane_xor<1>(v));
+// The same of magnitudes (no NaN, no sign), whose bit patterns order like the values: one instruction a step, as the lane exchange is part of an integer
+// maximum and nothing has to be made canonical.
+__device__ __forceinline__ unsigned max_xor8421(unsigned x) {
+  auto dpp = [](unsigned v, auto ctrl) { return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, 0xF, 0xF, true); };
+  x = max(x, dpp(x, std::integral_constant<int, 0xB1>{}));         // quad_perm [1,0,3,2]
+  x = max(x, dpp(x, std::integral_constant<int, 0x4E>{}));         // quad_perm [2,3,0,1]: a quad is alike
+  x = max(x, dpp(x, std::integral_constant<int, 0x141>{}));        // row_half_mirror: the other quad of 8 lanes
+  return max(x, dpp(x, std::integral_constant<int, 0x128>{}));     // row_ror:8
 }
+__device__ __forceinline__ float wave_max_abs(float v) {
+  unsigned x = max_xor8421(__float_as_uint(v));
+  const auto a = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  x = max(a[0], a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  return __uint_as_float(max(b[0], b[1]));
+}
+// ... over each aligned group of 16 lanes.
+__device__ __forceinline__ float row16_max_abs(float v) { return __uint_as_float(max_xor8421(__float_as_uint(v))); }
 
 // ---- tag 5: per-token fp8 (OCP e4m3) codes for the kernels whose w8a8 tiles run the fp8 matrix instruction.  scale = max|x| / 448
 // (the largest e4m3 number) in fp16 like the integer scales; code = e4m3(clamp(fp16(x / scale), +-448)), round to nearest even; rows
 // are stored like int8 rows, one byte per value.
-template <class Div>
-__device__ __forceinline__ uint2 fp8_chunk_codes(const float (&v)[8], const Div& div) {
+__device__ __forceinline__ uint2 fp8_chunk_codes(const v8h& h, const ScaleDiv& div) {
   float r[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) r[j] = fminf(fmaxf(round_h(div(v[j])), -448.0f), 448.0f);
+  for (int j = 0; j < 8; ++j) r[j] = fminf(fmaxf(round_h(div((float)h[j])), -448.0f), 448.0f);
   int lo = 0, hi = 0;
   lo = __builtin_amdgcn_cvt_pk_fp8_f32(r[0], r[1], lo, false);
   lo = __builtin_amdgcn_cvt_pk_fp8_f32(r[2], r[3], lo, true);
@@ -127,30 +255,25 @@ __device__ __forceinline__ uint2 fp8_chunk_codes(const float (&v)[8], const Div&
 // to fp32 in ascending order of stride and the scaled result rounded to fp16: strides 1, 2, 4 inside a chunk, 8 .. 256 across
 // lanes, 512 and up across the chunks of a lane.
 template <int NI>
-__device__ __forceinline__ void wave_rotate(float (&v)[NI][8], int lane, float scale) {
+__device__ __forceinline__ void wave_rotate(v8h (&h)[NI], int lane, float scale) {
+  float v[NI][8];
 #pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int h = 1; h < 8; h <<= 1)
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (!(j & h)) {
-          const float p = v[i][j], q = v[i][j + h];
-          v[i][j] = p + q;
-          v[i][j + h] = p - q;
-        }
-  auto lane_stage = [&](auto mc) {
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; j += 2) lane_butterfly<decltype(mc)::value>(v[i][j], v[i][j + 1], lane);
+  for (int i = 0; i < NI; ++i) {  // (chunk by chunk: stage by stage over all of them takes more registers)
+    chunk_h8(h[i], v[i]);
+    lane_stage<1>(v[i], lane);
+    lane_stage<2>(v[i], lane);
+    lane_stage<4>(v[i], lane);
+    lane_stage<8>(v[i], lane);
+    lane_stage<16>(v[i], lane);
+    lane_stage<32>(v[i], lane);
+  }
+  // Chunk by chunk, stage by stage: the compiler otherwise follows single results through all the stages and keeps the operands of the others (178 registers
+  // instead of 119 for rows of 4096 values in the layer's first kernel; 8192 of them 54 us instead of 48).
+  auto formed = [](float (&x)[8]) {
+    asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]));
   };
-  lane_stage(std::integral_constant<int, 1>{});
-  lane_stage(std::integral_constant<int, 2>{});
-  lane_stage(std::integral_constant<int, 4>{});
-  lane_stage(std::integral_constant<int, 8>{});
-  lane_stage(std::integral_constant<int, 16>{});
-  lane_stage(std::integral_constant<int, 32>{});
+#pragma unroll
+  for (int i = 0; i < NI; ++i) formed(v[i]);
 #pragma unroll
   for (int hi = 1; hi < NI; hi <<= 1)
 #pragma unroll
@@ -162,11 +285,13 @@ __device__ __forceinline__ void wave_rotate(float (&v)[NI][8], int lane, float s
           v[i][j] = p + q;
           v[i + hi][j] = p - q;
         }
+        formed(v[i]);
+        formed(v[i + hi]);
       }
 #pragma unroll
   for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[i][j] = round_h(keep_f32(v[i][j] * scale));
+    for (int j = 0; j < 8; ++j) h[i][j] = (_Float16)keep_f32(v[i][j] * scale);
 }
 
 // The activation step behind a gate_up form (act_kernels.hip): rows that are already silu(gate) * up -> rotation, quantisation,

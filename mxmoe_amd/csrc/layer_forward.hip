@@ -175,32 +175,22 @@ __device__ __forceinline__ void head_scatter(const HeadArgs& a, int block, int32
 template <int NI>
 __device__ __forceinline__ void head_token(const HeadArgs& a, int t, int lane) {
   constexpr int n = 512 * NI;
+  asm volatile("" : "+v"(lane));  // (else every address below becomes a register pair of its own that the loop over tokens carries along)
   const _Float16* srow = a.hidden + (long)t * n;
-  float v[NI][8];
+  v8h h[NI];
 #pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const v8h g = *reinterpret_cast<const v8h*>(srow + (lane + 64 * i) * 8);
+  for (int i = 0; i < NI; ++i) h[i] = *reinterpret_cast<const v8h*>(srow + lane * 8 + 512 * i);
+  if (a.rotate != 0) {
+    wave_rotate<NI>(h, lane, a.scale);
+  } else {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[i][j] = (float)g[j];
+    for (int i = 0; i < NI; ++i) h[i] = quiet(h[i]);
   }
-  if (a.rotate != 0) wave_rotate<NI>(v, lane, a.scale);
   if (a.tags & 1u) {  // fp16: only when every row is rotated (else the GEMM reads the tokens where they are)
     _Float16* out = reinterpret_cast<_Float16*>(a.store[0]) + (long)t * n;
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      v8h o;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] = (_Float16)v[i][j];
-      *reinterpret_cast<v8h*>(out + (lane + 64 * i) * 8) = o;
-    }
+    for (int i = 0; i < NI; ++i) *reinterpret_cast<v8h*>(out + lane * 8 + 512 * i) = h[i];
   }
-  auto codes4 = [&](const float (&x)[8], float scale) {
-    const ScaleDiv div(scale);
-    unsigned w = 0;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) w = push_code<4>(w, code_word(fminf(fmaxf(round_h(div(x[j])), -7.0f), 7.0f)));
-    return w;
-  };
   // fp16 division: fp32 quotient of two fp16 values, rounded to fp16; a zero row gets 1 (quantize.cuh:258)
   auto scale_of = [](float amax, float upper) {
     const float scale = round_h(amax / upper);
@@ -210,52 +200,43 @@ __device__ __forceinline__ void head_token(const HeadArgs& a, int t, int lane) {
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int c = lane + 64 * i;
-      float gmax = 0.0f;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) gmax = fmaxf(gmax, fabsf(v[i][j]));
-      const float scale = scale_of(row16_max(gmax), 7.0f);
+      HalfMax gmax;
+      gmax.add(h[i]);
+      const float scale = scale_of(row16_max_abs(gmax.get()), 7.0f);
       if ((c & 15) == 0) a.scales[3][(long)t * (n >> 7) + (c >> 4)] = (_Float16)scale;
-      *reinterpret_cast<unsigned*>(a.store[3] + (long)t * (n / 2) + c * 4) = codes4(v[i], scale);
+      *reinterpret_cast<unsigned*>(a.store[3] + (long)t * (n / 2) + lane * 4 + 256 * i) = HalfDiv(scale).int4(h[i]);
     }
   }
   if ((a.tags & 0x26u) == 0) return;
-  float amax = 0.0f;
+  HalfMax half_max;
 #pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[i][j]));
-  amax = wave_max(amax);
+  for (int i = 0; i < NI; ++i) half_max.add(h[i]);
+  const float amax = wave_max_abs(half_max.get());
   if (a.tags & 2u) {  // tag 1: int8 per token
     const float scale = scale_of(amax, 127.0f);
-    const ScaleDiv div(scale);
+    const HalfDiv half(scale);
     if (lane == 0) a.scales[1][t] = (_Float16)scale;
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      uint2 w{0, 0};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        w.x = push_code<8>(w.x, code_word(fminf(fmaxf(round_h(div(v[i][j])), -127.0f), 127.0f)));
-        w.y = push_code<8>(w.y, code_word(fminf(fmaxf(round_h(div(v[i][j + 4])), -127.0f), 127.0f)));
-      }
-      *reinterpret_cast<uint2*>(a.store[1] + (long)t * n + (lane + 64 * i) * 8) = w;
-    }
+    for (int i = 0; i < NI; ++i) *reinterpret_cast<uint2*>(a.store[1] + (long)t * n + lane * 8 + 512 * i) = half.int8(h[i]);
   }
   if (a.tags & 0x20u) {  // tag 5: fp8 e4m3 per token
     const float scale = scale_of(amax, 448.0f);
     const ScaleDiv div(scale);
     if (lane == 0) a.scales[5][t] = (_Float16)scale;
 #pragma unroll
-    for (int i = 0; i < NI; ++i) *reinterpret_cast<uint2*>(a.store[5] + (long)t * n + (lane + 64 * i) * 8) = fp8_chunk_codes(v[i], div);
+    for (int i = 0; i < NI; ++i) *reinterpret_cast<uint2*>(a.store[5] + (long)t * n + lane * 8 + 512 * i) = fp8_chunk_codes(h[i], div);
   }
   if (a.tags & 4u) {  // tag 2: int4 per token
     const float scale = scale_of(amax, 7.0f);
+    const HalfDiv half(scale);
     if (lane == 0) a.scales[2][t] = (_Float16)scale;
 #pragma unroll
-    for (int i = 0; i < NI; ++i) *reinterpret_cast<unsigned*>(a.store[2] + (long)t * (n / 2) + (lane + 64 * i) * 4) = codes4(v[i], scale);
+    for (int i = 0; i < NI; ++i) *reinterpret_cast<unsigned*>(a.store[2] + (long)t * (n / 2) + lane * 4 + 256 * i) = half.int4(h[i]);
   }
 }
 
-// Workgroups: planning first (the longest chain of dependent steps), then the permutation's entries, then tokens, one per wave.
+// Workgroups: planning first (the longest chain of dependent steps), then the permutation's entries, then tokens, one per wave.  (Four waves per SIMD: left to
+// itself the compiler takes 178 registers for tokens of 4096 values, and 8192 of them 54 us instead of 48.)
 template <int NI, int TH>
 __global__ void __launch_bounds__(TH) layer_head_kernel(const HeadArgs a, const PlanPair pair) {
   extern __shared__ __align__(16) int32_t head_lds[];
