@@ -878,24 +878,24 @@ __global__ void __launch_bounds__(256) token_quant_wave_kernel(const TokenArgs a
 // (H_8) stays inside a chunk.  The dense stage t[b][col] = sum_b' B[b][b'] q[b'][col] over the 8 f columns col = blk * 8 + j runs on the
 // matrix cores: the row, snapped to integers of at most 18 bits (DenseGrid) and divided by 16 so that every value is an fp16 number,
 // is written to LDS transposed ([col][b'], b' contiguous), B (+-1, zero padded) is the first operand, kept in LDS in operand order
-// and read block by block, and the fp32 results are exact whatever order the hardware adds in.  Results return through LDS in row order, so
-// the quantise / pack / store code sees the same chunk-per-lane layout as in the other kernels and writes 16 bytes per lane.
-// Four independent rows per workgroup; no barrier (each wave owns its piece of LDS).
+// and read block by block, and the fp32 results are exact whatever order the hardware adds in.  Results take the place of the values they came from ([col][b],
+// four neighbouring ones of a lane in one write) and are gathered from there, so the quantise / pack / store code sees the same chunk-per-lane layout as in the
+// other kernels.  Four independent rows per workgroup; no barrier (each wave owns its piece of LDS).
+// Bound by the vector ALU and by how many waves cover each other's latencies: 32 768 rows of 1408 values take 58 us with six waves per SIMD (24 KiB of LDS a
+// workgroup, 71 registers), 67 with four (rotated row in a buffer of its own, one element a write: 36 KiB, 92 registers).
 constexpr int kDensePitch = 144;             // bytes per column of the transposed row: 64 fp16 + 16 (16 lanes read 16 distinct bank groups)
-// LDS of a workgroup: B as matrix operands (one KiB per 16 x 32 block), then per wave the transposed row and the rotated row in row
-// order (+ a slot of 8 values for discarded ones)
-__host__ __device__ constexpr int dense_wave_lds(int n) { return 32 * kDensePitch + (n + 8) * 2; }
-__host__ __device__ constexpr int dense_lds(int n, int kb) { return ((kb + 15) >> 4) * ((kb + 31) >> 5) * 1024 + 4 * dense_wave_lds(n); }
+// LDS of a workgroup: B as matrix operands (one KiB per 16 x 32 block), then per wave the transposed row
+constexpr int kDenseWaveLds = 32 * kDensePitch;
+__host__ __device__ constexpr int dense_lds(int kb) { return ((kb + 15) >> 4) * ((kb + 31) >> 5) * 1024 + 4 * kDenseWaveLds; }
 template <int MAXC, bool SILU, bool EXT>
 __device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int wg, const int wgs, uint8_t* const dlds) {
-  const int lane = threadIdx.x & 63;
+  const int lane0 = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lm = lane & 15, lg = lane >> 4;
+  const int lm = lane0 & 15, lg = lane0 >> 4;
   const RotPlan pl = a.plan;
   const int n = pl.n, nchunks = n >> 3, kb = pl.kb;
   const int ksteps = (kb + 31) >> 5, mblocks = (kb + 15) >> 4;
-  uint8_t* xt = dlds + mblocks * ksteps * 1024 + wave * dense_wave_lds(n);  // [32 columns][kDensePitch]
-  uint8_t* yrow = xt + 32 * kDensePitch;                                      // [n] fp16, then the discard slot
+  uint8_t* const xt = dlds + mblocks * ksteps * 1024 + wave * kDenseWaveLds;  // [32 columns][kDensePitch]
   // B as the first operand of v_mfma_f32_16x16x32_f16: lane holds row 16 mb + (lane & 15), k = 32 ks + 8 (lane >> 4) + 0..7.  Kept in
   // LDS (block (mb, ks) at (mb * ksteps + ks) KiB, 16 bytes per lane) and read per row: 32 registers fewer per lane.
   for (int blkid = wave; blkid < mblocks * ksteps; blkid += 4) {
@@ -909,10 +909,20 @@ __device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int
       const float sv = a.signs[min(b, kb - 1) * kb + min(bp, kb - 1)];
       bs[i] = (b < kb && bp < kb) ? (_Float16)sv : (_Float16)0.0f;
     }
-    *reinterpret_cast<v8h*>(dlds + blkid * 1024 + lane * 16) = bs;
+    *reinterpret_cast<v8h*>(dlds + blkid * 1024 + lane0 * 16) = bs;
   }
   // columns and k positions that no row ever writes must read as zero
-  for (int i = lane; i < 32 * kDensePitch / 16; i += 64) reinterpret_cast<v4i*>(xt)[i] = v4i{0, 0, 0, 0};
+  auto clear = [&]() {
+    for (int i = lane0; i < kDenseWaveLds / 16; i += 64) reinterpret_cast<v4i*>(xt)[i] = v4i{0, 0, 0, 0};
+  };
+  clear();
+  // place of the lane's chunks: chunk c = blk * kb + b' is columns blk * 8 + j, position b' (lanes past the row: its last chunk, whose values they hold too)
+  int place[MAXC];
+#pragma unroll
+  for (int i = 0; i < MAXC; ++i) {
+    const int c = min(lane0 + 64 * i, nchunks - 1), blk = c / kb;
+    place[i] = blk * 8 * kDensePitch + (c - blk * kb) * 2;
+  }
   __syncthreads();
 
   struct RowMeta {
@@ -943,7 +953,7 @@ __device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int
   auto load_data = [&](const RowMeta& m, v8h (&g)[MAXC], v8h (&u)[MAXC]) {
 #pragma unroll
     for (int i = 0; i < MAXC; ++i) {
-      const int c = min(lane + 64 * i, nchunks - 1);  // lanes past the row re-read its last chunk (never used)
+      const int c = min(lane0 + 64 * i, nchunks - 1);  // lanes past the row re-read its last chunk (never used)
       g[i] = *reinterpret_cast<const v8h*>(m.srow + c * 8);
       if (SILU) u[i] = *reinterpret_cast<const v8h*>(m.srow + n + c * 8);
     }
@@ -960,6 +970,8 @@ __device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int
   }
   for (int row = row0; row < a.rows; row += stride_rows) {
     const RowMeta cur = next_meta;
+    int lane = lane0;  // (as something that changes from row to row: else every address below is kept in registers of its own for the whole kernel)
+    asm volatile("" : "+v"(lane));
     const bool has_next = row + stride_rows < a.rows;
     if (has_next) next_meta = load_meta(row + stride_rows);
     v8h h[MAXC];
@@ -986,87 +998,63 @@ __device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int
         h[i] = scale_chunk(v, pl.scale, mx);
       }
       const DenseGrid grid(round_h(wave_max_abs(mx)));
-      // transposed write: chunk c = blk * kb + b' -> columns blk * 8 + j, position b'
 #pragma unroll
       for (int i = 0; i < MAXC; ++i) {
-        const int c = lane + 64 * i;
-        if (c < nchunks) {
-          const int blk = c / kb, bp = c - blk * kb;
-          uint8_t* dst = xt + (blk * 8) * kDensePitch + bp * 2;
-          const v8h q = snap_chunk(h[i], grid.to_grid);
+        const v8h q = snap_chunk(h[i], grid.to_grid);
 #pragma unroll
-          for (int j = 0; j < 8; ++j) *reinterpret_cast<_Float16*>(dst + j * kDensePitch) = q[j];
-        }
+        for (int j = 0; j < 8; ++j) *reinterpret_cast<_Float16*>(xt + place[i] + j * kDensePitch) = q[j];
       }
       asm volatile("" ::: "memory");
       __builtin_amdgcn_wave_barrier();
       // lane holds column col = 16 nb + (lane & 15), i.e. blk = 2 nb + ((lane >> 3) & 1), j = lane & 7, and rows b = 16 mb + 4 (lane >> 4) + r
-      // of every 16 x 16 block.  One block of 16 rows of B at a time (8 accumulator registers live, the second operand re-read
-      // from LDS), each followed by its way back: S_f butterflies across blk (bit 0 = lane bit 3, bit 1 = the column block;
-      // ascending), back to the row's scale (a power of two: exact wherever it is applied) with the one rounding to fp16, and the
-      // value goes to its place in the row (values of rows or blocks that do not exist go to the discard slot).  Compiled once per
-      // order f of the Sylvester factor, so that nothing in it branches on f.
+      // of every 16 x 16 block.  Then the way back: S_f butterflies across blk (bit 0 = lane bit 3, bit 1 = the column block; ascending), back to the
+      // row's scale (a power of two: exact wherever it is applied) with the one rounding to fp16.  A lane's four rows exist or not together: kb is a
+      // multiple of four.  Compiled once per order f of the Sylvester factor, so that nothing in it branches on f.
       const float back = grid.from_grid * 16.0f;
-      // (positions from a lane number the compiler must take as changing from row to row: otherwise it keeps every position of
-      // every row block in a register of its own for the whole kernel)
-      int lane_now = lane;
-      asm volatile("" : "+v"(lane_now));
+      const int lm = lane & 15, lg = lane >> 4;
       auto dense_stage = [&](auto f_const) {
         constexpr int F = decltype(f_const)::value;
         constexpr int NCOLS = F > 2 ? 2 : 1;
-        const float sgn8 = (lane_now & 8) ? -1.0f : 1.0f;
-        const int blk0 = (lane_now >> 3) & 1, jj = lane_now & 7;
-        // row 16 mb + 4 (lane >> 4) + r of B exists, and the lane's column block too, when 16 mb + r < lim
-        const int lim = blk0 < F ? kb - 4 * (lane_now >> 4) : 0;
-        uint8_t* const y0 = yrow + 2 * (((blk0 * kb + 4 * (lane_now >> 4)) << 3) + jj);  // place of row block 0, r = 0, in the row
-        uint8_t* const y1 = y0 + 2 * ((2 * kb) << 3);                                      // the same, two column blocks on
-        uint8_t* const ydiscard = yrow + 2 * n;
-        constexpr int kStep = 2 * 8;  // bytes between the places of consecutive rows of B
+        const float sgn8 = (lane & 8) ? -1.0f : 1.0f;
+        uint8_t* const col = xt + lm * kDensePitch + lg * 8;
+        v8h xf[2][NCOLS];
 #pragma unroll
-        for (int mb = 0; mb < 4; ++mb) {
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+          for (int nb = 0; nb < NCOLS; ++nb) xf[ks][nb] = *reinterpret_cast<const v8h*>(xt + (nb * 16 + lm) * kDensePitch + ks * 64 + lg * 16);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();  // (the results go where the operands were)
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb)
           if (mb < mblocks) {
             v4f acc[NCOLS];
+            const v8h b0 = *reinterpret_cast<const v8h*>(dlds + mb * ksteps * 1024 + lane * 16);
 #pragma unroll
-            for (int nb = 0; nb < NCOLS; ++nb) acc[nb] = v4f{0.f, 0.f, 0.f, 0.f};
+            for (int nb = 0; nb < NCOLS; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b0, xf[0][nb], v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            if (ksteps > 1) {
+              const v8h b1 = *reinterpret_cast<const v8h*>(dlds + (mb * ksteps + 1) * 1024 + lane * 16);
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-              if (ks < ksteps) {
-                const v8h bs = *reinterpret_cast<const v8h*>(dlds + (mb * ksteps + ks) * 1024 + lane * 16);
-#pragma unroll
-                for (int nb = 0; nb < NCOLS; ++nb) {
-                  const v8h xf = *reinterpret_cast<const v8h*>(xt + (nb * 16 + lm) * kDensePitch + ks * 64 + lg * 16);
-                  acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bs, xf, acc[nb], 0, 0, 0);
-                }
-              }
+              for (int nb = 0; nb < NCOLS; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b1, xf[1][nb], acc[nb], 0, 0, 0);
             }
-            // a block whose 16 rows all exist, in a column block that exists for every lane, needs no test per value
-            const bool whole = F > 1 && 16 * mb + 16 <= kb;
-            auto emit = [&](auto whole_const) {
+            v4h o[NCOLS];
 #pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                constexpr bool kWhole = decltype(whole_const)::value;
-                const int off = (16 * mb + r) * kStep;
-                const bool ok = kWhole || 16 * mb + r < lim;
-                float t0 = acc[0][r], t1 = 0.0f;
-                if constexpr (F > 1) t0 = __builtin_fmaf(sgn8, t0, lane_xor<8>(t0));
-                if constexpr (F > 2) {
-                  t1 = acc[NCOLS - 1][r];
-                  t1 = __builtin_fmaf(sgn8, t1, lane_xor<8>(t1));
-                  const float p = t0, q = t1;
-                  t0 = p + q;
-                  t1 = p - q;
-                }
-                *reinterpret_cast<_Float16*>((ok ? y0 : ydiscard - off) + off) = (_Float16)(t0 * back);
-                if constexpr (F > 2) *reinterpret_cast<_Float16*>((ok ? y1 : ydiscard - off) + off) = (_Float16)(t1 * back);
+            for (int r = 0; r < 4; ++r) {
+              float t0 = acc[0][r];
+              if constexpr (F > 1) t0 = __builtin_fmaf(sgn8, t0, lane_xor<8>(t0));
+              if constexpr (F > 2) {
+                float t1 = acc[NCOLS - 1][r];
+                t1 = __builtin_fmaf(sgn8, t1, lane_xor<8>(t1));
+                const float p = t0, q = t1;
+                t0 = p + q;
+                o[NCOLS - 1][r] = (_Float16)((p - q) * back);
               }
-            };
-            if (whole) {
-              emit(std::true_type{});
-            } else {
-              emit(std::false_type{});
+              o[0][r] = (_Float16)(t0 * back);
+            }
+            if (16 * mb + 4 * lg < kb && (F > 1 || lm < 8)) {
+#pragma unroll
+              for (int nb = 0; nb < NCOLS; ++nb) *reinterpret_cast<v4h*>(col + nb * 16 * kDensePitch + mb * 32) = o[nb];
             }
           }
-        }
       };
       switch (pl.f) {
         case 1: dense_stage(std::integral_constant<int, 1>{}); break;
@@ -1076,10 +1064,9 @@ __device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int
       asm volatile("" ::: "memory");
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
-      for (int i = 0; i < MAXC; ++i) {
-        const int c = min(lane + 64 * i, nchunks - 1);
-        h[i] = *reinterpret_cast<const v8h*>(yrow + c * 16);
-      }
+      for (int i = 0; i < MAXC; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) h[i][j] = *reinterpret_cast<const _Float16*>(xt + place[i] + j * kDensePitch);
       asm volatile("" ::: "memory");
       __builtin_amdgcn_wave_barrier();  // the next row's writes come after these reads
     } else if (!SILU) {
@@ -1128,17 +1115,18 @@ __device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int
     const ScaleDiv div(scale);  // (fp8 and bf6 codes)
     const HalfDiv half(scale);
     if (lane == 0) a.scale_store[scale_off + lrow] = (_Float16)scale;
-    if (EXT && tag == 4) {  // codes into the wave's row buffer (its reads of the rotated row are behind a wave barrier), then fragments
+    if (EXT && tag == 4) {  // codes in row order in the wave's piece of LDS (its reads of the rotated row are behind a wave barrier), then fragments
 #pragma unroll
       for (int i = 0; i < MAXC; ++i) {
         const int c = lane + 64 * i;
-        if (c < nchunks) *reinterpret_cast<v8h*>(yrow + c * 16) = bf6_chunk_codes(h[i], div);
+        if (c < nchunks) *reinterpret_cast<v8h*>(xt + c * 16) = bf6_chunk_codes(h[i], div);
       }
       asm volatile("" ::: "memory");
       __builtin_amdgcn_wave_barrier();
-      bf6_emit_row(yrow, n, 0, n, a.inp_store + 2 * inp_off, lrow, lane, 64);
+      bf6_emit_row(xt, n, 0, n, a.inp_store + 2 * inp_off, lrow, lane, 64);
       asm volatile("" ::: "memory");
-      __builtin_amdgcn_wave_barrier();  // the next row's writes come after these reads
+      __builtin_amdgcn_wave_barrier();  // what follows comes after these reads
+      clear();
       continue;
     }
     uint8_t* out = a.inp_store + 2 * (inp_off + lrow * (n >> (tag == 1 || (EXT && tag == 5) ? 1 : 2)));
@@ -1157,7 +1145,7 @@ __device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int
   }
 }
 template <int MAXC, bool SILU, bool EXT>
-__global__ void __launch_bounds__(256) row_quant_dense_kernel(const RowArgs a) {
+__global__ void __launch_bounds__(256, SILU || EXT || MAXC > 3 ? 1 : 6) row_quant_dense_kernel(const RowArgs a) {
   extern __shared__ __align__(16) uint8_t dlds[];
   row_quant_dense_body<MAXC, SILU, EXT>(a, blockIdx.x, gridDim.x, dlds);
 }
@@ -1194,9 +1182,9 @@ constexpr bool chunks_aligned() {
 static_assert(chunks_aligned(), "a chunk of any k row is read and written at the alignment its type promises");
 template <int NT, int MAXC, bool SILU, bool EXT>
 __device__ __forceinline__ void row_quant_block_body(const RowArgs& a, const int wg, const int wgs, uint8_t* const lds) {
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lm = lane & 15, lg = lane >> 4;
+  const int tid0 = threadIdx.x, lane0 = tid0 & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid0 >> 6);
+  const int lm = lane0 & 15, lg = lane0 >> 4;
   constexpr int kW = NT / 64;
   const RotPlan pl = a.plan;
   const BlockRows g(pl);
@@ -1227,11 +1215,11 @@ __device__ __forceinline__ void row_quant_block_body(const RowArgs& a, const int
     v8h bs;
 #pragma unroll
     for (int i = 0; i < 8; ++i) bs[i] = (16 * mb + lm < kb && 32 * ks + 8 * lg + i < kb) ? (_Float16)sv[i] : (_Float16)0.0f;
-    *reinterpret_cast<v8h*>(lds + blkid * 1024 + lane * 16) = bs;
+    *reinterpret_cast<v8h*>(lds + blkid * 1024 + lane0 * 16) = bs;
   };
   load_signs(min(wave, mblocks * ksteps - 1));
   // columns and k positions that no row ever writes must read as zero
-  for (int i = tid; i < g.snapped / 8; i += NT) reinterpret_cast<uint2*>(xt)[i] = make_uint2(0, 0);
+  for (int i = tid0; i < g.snapped / 8; i += NT) reinterpret_cast<uint2*>(xt)[i] = make_uint2(0, 0);
 
   struct RowMeta {
     int tag;
@@ -1259,7 +1247,7 @@ __device__ __forceinline__ void row_quant_block_body(const RowArgs& a, const int
   auto load_data = [&](const RowMeta& m, v8h (&gt)[MAXC], v8h (&up)[MAXC]) {
 #pragma unroll
     for (int i = 0; i < MAXC; ++i) {
-      const int c = min(tid + NT * i, nchunks - 1);  // threads past the row re-read its last chunk (never used)
+      const int c = min(tid0 + NT * i, nchunks - 1);  // threads past the row re-read its last chunk (never used)
       gt[i] = gload<v8h>(m.srow + c * 8);
       if (SILU) up[i] = gload<v8h>(m.srow + n + c * 8);
     }
@@ -1277,6 +1265,9 @@ __device__ __forceinline__ void row_quant_block_body(const RowArgs& a, const int
 
   for (int row = wg; row < a.rows; row += wgs) {
     const RowMeta cur = next_meta;
+    int tid = tid0;  // (as something that changes from row to row: else every address below is kept in registers of its own for the whole kernel)
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, lm = lane & 15, lg = lane >> 4;
     const bool has_next = row + wgs < a.rows;
     if (has_next) next_meta = load_meta(row + wgs);
     v8h h[MAXC];
@@ -1439,7 +1430,7 @@ __global__ void __launch_bounds__(256) row_quant_block_kernel(const RowArgs a) {
 // leaves most of the chip idle when it is short.  The first `shared_wgs` workgroups (a multiple of 64: xcd_row_group) take the shared rows, which run longest,
 // by row_quant_block_kernel's code, the others the routed rows by row_quant_dense_kernel's.
 template <int MAXC, bool SILU, bool EXT>
-__global__ void __launch_bounds__(256) row_quant_pair_kernel(const RowArgs routed, const RowArgs shared, const int shared_wgs) {
+__global__ void __launch_bounds__(256, SILU ? 1 : 4) row_quant_pair_kernel(const RowArgs routed, const RowArgs shared, const int shared_wgs) {
   extern __shared__ __align__(16) uint8_t plds[];
   const int wg = blockIdx.x;
   if (wg < shared_wgs) row_quant_block_body<256, 3, SILU, EXT>(shared, wg, shared_wgs, plds);
@@ -1462,39 +1453,42 @@ __global__ void __launch_bounds__(NT) row_quant_few_kernel(const RowArgs routed,
 // same exact integer sum as in row_quant_dense_kernel, on the matrix cores: the snapped row goes to LDS as it is ([k][column], one
 // 16-byte write per chunk), every wave gathers the second operand of its 64 columns from there (two bytes per read, each landing in
 // its half of the operand register) and multiplies B (first operand, in registers) into them, and the results return through LDS in
-// row order for the quantise / pack / store code.  Four barriers per row; two workgroups share a CU.
+// row order for the quantise / pack / store code.  Four barriers per row; three workgroups share a CU: 16 384 rows of 14 336 values 312 us, 354 with two (a buffer
+// for the rotated row, 104 registers).  The next row's loads under this one's rotation: 16 more registers, 359.
 constexpr int kWidePitch = 1024 + 8;                                 // bytes per k row of 512 fp16 in LDS: the 4 k groups (or row groups) that the
                                                                      // lanes of a wave touch together land 8 or 16 banks apart
-constexpr int kWideLds = 2 * 32 * kWidePitch + 64;                   // snapped row, rotated row, reduction slots
+constexpr int kWideLds = 32 * kWidePitch + 64 + 2048;                // the row, reduction slots, B
 template <bool SILU, bool EXT>
-__global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
+__global__ void __launch_bounds__(512, 6) row_quant_wide_kernel(const RowArgs a) {
   extern __shared__ __align__(16) uint8_t wlds[];
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // in a scalar register: "is k row wave + 8 i live" is then a scalar branch
-  const int lm = lane & 15, lg = lane >> 4;
-  uint8_t* xt = wlds;                                   // [32 k rows][kWidePitch]: the snapped row
-  uint8_t* yrow = xt + 32 * kWidePitch;                 // [32 rows][kWidePitch]: the rotated row
-  float* red = reinterpret_cast<float*>(yrow + 32 * kWidePitch);  // [8] + [8]
+  uint8_t* const xt = wlds;                             // [32 k rows][kWidePitch]: the snapped row, then in its place the rotated one
+  float* red = reinterpret_cast<float*>(xt + 32 * kWidePitch);  // [8] + [8]
   const RotPlan pl = a.plan;
   const int n = pl.n, kb = pl.kb;
   constexpr int MAXC = 4;
-  // B as the first operand of v_mfma_f32_16x16x32_f16: lane holds row 16 mb + (lane & 15), k = 8 (lane >> 4) + 0..7
-  v8h bsign[2];
-#pragma unroll
-  for (int mb = 0; mb < 2; ++mb) {
-    const int b = 16 * mb + lm;
+  // B as the first operand of v_mfma_f32_16x16x32_f16: lane holds row 16 mb + (lane & 15), k = 8 (lane >> 4) + 0..7.  In LDS, one KiB per block of 16 rows: eight
+  // registers fewer per lane.
+  uint8_t* const signs = reinterpret_cast<uint8_t*>(red + 16);
+  if (wave < 2) {
+    const int lane = tid & 63, b = 16 * wave + (lane & 15);
+    v8h bs;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const int bp = 8 * lg + i;
+      const int bp = 8 * (lane >> 4) + i;
       const float sv = a.signs[min(b, kb - 1) * kb + min(bp, kb - 1)];
-      bsign[mb][i] = (b < kb && bp < kb) ? (_Float16)sv : (_Float16)0.0f;
+      bs[i] = (b < kb && bp < kb) ? (_Float16)sv : (_Float16)0.0f;
     }
+    *reinterpret_cast<v8h*>(signs + wave * 1024 + lane * 16) = bs;
   }
   // k rows kb .. 31 are never written and must read as zero
   for (int i = tid; i < 32 * kWidePitch / 8; i += 512) reinterpret_cast<uint2*>(xt)[i] = make_uint2(0, 0);
   const _Float16* const src_shared = shared_src(a);
   for (int row = blockIdx.x; row < a.rows; row += gridDim.x) {
     if (!row_exists(a, row)) continue;
+    int lane = tid & 63;  // (as something that changes from row to row: else every address below is kept in registers of its own for the whole kernel)
+    asm volatile("" : "+v"(lane));
     const bool shared_row = row >= a.R;
     const int e = shared_row ? a.E : a.dst_exp[row];
     const int tag = (int)a.table[e];
@@ -1560,23 +1554,28 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
         if (kr < kb) *reinterpret_cast<v8h*>(xt + kr * kWidePitch + lane * 16) = snap_chunk(h[i], grid.to_grid);
       }
       __syncthreads();
-      // this wave's 64 columns: 4 column blocks x 2 row blocks; the second operand of a lane is column col, k = 8 (lane >> 4) + 0..7
+      // this wave's 64 columns: 4 column blocks x 2 row blocks; the second operand of a lane is column 16 nb + (lane & 15), k = 8 (lane >> 4) + 0..7
       const float back = grid.from_grid * 16.0f;
+      const int lm = lane & 15, lg = lane >> 4;
+      uint8_t* const col = xt + (wave * 64 + lm) * 2;
+      v8h xf[4];
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb) {
-        const int col = wave * 64 + nb * 16 + lm;
-        v8h xf;
+      for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) xf[i] = *reinterpret_cast<const _Float16*>(xt + (8 * lg + i) * kWidePitch + col * 2);
+        for (int i = 0; i < 8; ++i) xf[nb][i] = *reinterpret_cast<const _Float16*>(col + (8 * lg + i) * kWidePitch + nb * 32);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_wave_barrier();  // (the results go where the operands were: no other wave reads or writes these columns)
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb) {
-          v4f acc = {0.f, 0.f, 0.f, 0.f};
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(bsign[mb], xf, acc, 0, 0, 0);
+      for (int mb = 0; mb < 2; ++mb) {
+        v4f acc[4];
+        const v8h bs = *reinterpret_cast<const v8h*>(signs + mb * 1024 + lane * 16);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int b = 16 * mb + 4 * lg + r;  // lane holds column col and rows b of the block (rows kb .. 31 are never read back)
-            *reinterpret_cast<_Float16*>(yrow + b * kWidePitch + col * 2) = (_Float16)(acc[r] * back);
-          }
+        for (int nb = 0; nb < 4; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bs, xf[nb], v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        if (16 * mb + 4 * lg < kb) {  // (rows kb .. 31 stay zero; a lane's four rows exist or not together: kb is a multiple of four)
+#pragma unroll
+          for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) *reinterpret_cast<_Float16*>(col + (16 * mb + 4 * lg + r) * kWidePitch + nb * 32) = (_Float16)(acc[nb][r] * back);
         }
       }
       __syncthreads();
@@ -1584,7 +1583,7 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
       for (int i = 0; i < MAXC; ++i) {
         const int kr = wave + 8 * i;
         if (kr >= kb) continue;  // (still zeros)
-        h[i] = *reinterpret_cast<const v8h*>(yrow + kr * kWidePitch + lane * 16);
+        h[i] = *reinterpret_cast<const v8h*>(xt + kr * kWidePitch + lane * 16);
       }
     }
 
@@ -1637,10 +1636,10 @@ __global__ void __launch_bounds__(512) row_quant_wide_kernel(const RowArgs a) {
 #pragma unroll
       for (int i = 0; i < MAXC; ++i) {
         const int kr = wave + 8 * i;
-        if (kr < kb) *reinterpret_cast<v8h*>(yrow + kr * kWidePitch + lane * 16) = bf6_chunk_codes(h[i], div);
+        if (kr < kb) *reinterpret_cast<v8h*>(xt + kr * kWidePitch + lane * 16) = bf6_chunk_codes(h[i], div);
       }
       __syncthreads();
-      bf6_emit_row(yrow, 512, kWidePitch, n, a.inp_store + 2 * inp_off, lrow, tid, 512);
+      bf6_emit_row(xt, 512, kWidePitch, n, a.inp_store + 2 * inp_off, lrow, tid, 512);
       __syncthreads();
       continue;
     }
@@ -1684,10 +1683,10 @@ static int make_plan(int n, int had_k, int had_f, bool rotate, RotPlan* p) {
 
 // Rows that row_quant_dense_kernel and row_quant_wide_kernel take: one length, a table-driven factor times H_8 / times H_512.
 static bool dense_rows(const RowArgs& a) {
-  return a.plan.kb > 1 && a.plan.m == 8 && a.plan.f <= 4 && a.plan.kb <= 64 && a.plan.n <= 2048 && a.plan_shared.n == a.plan.n && a.plan_shared.kb == a.plan.kb && a.rotate != 0;
+  return a.plan.kb > 1 && a.plan.kb % 4 == 0 && a.plan.m == 8 && a.plan.f <= 4 && a.plan.kb <= 64 && a.plan.n <= 2048 && a.plan_shared.n == a.plan.n && a.plan_shared.kb == a.plan.kb && a.rotate != 0;
 }
 static bool wide_rows(const RowArgs& a) {
-  return a.plan.kb > 1 && a.plan.kb <= 32 && a.plan.m == 512 && a.plan.f == 1 && a.plan_shared.n == a.plan.n && a.plan_shared.kb == a.plan.kb && a.rotate != 0;
+  return a.plan.kb > 1 && a.plan.kb % 4 == 0 && a.plan.kb <= 32 && a.plan.m == 512 && a.plan.f == 1 && a.plan_shared.n == a.plan.n && a.plan_shared.kb == a.plan.kb && a.rotate != 0;
 }
 
 // Rows that row_quant_block_kernel can take: one length of at most 6144 values (three chunks per thread).
@@ -1721,15 +1720,15 @@ static int launch_pair(const RowArgs& routed, const RowArgs& shared, bool dense,
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   // (dense_rows and block_rows: at most 64 KiB of LDS)
-  // (workgroups per CU: 2049 shared rows of 2816 values and 12 294 routed ones of 1408, us, shared + routed per CU: 1 + 2 46, 1 + 3 50, 2 + 3 52, 2 + 4 48, 3 + 2 55;
-  // with the shared rows by row_quant_kernel's code 56)
-  const int lds = std::max(BlockRows(shared.plan).lds(), dense ? dense_lds(routed.plan.n, routed.plan.kb) : BlockRows(routed.plan).lds());
-  const int shared_wgs = std::min(shared.rows, cus) + 63 & ~63;
+  // (workgroups per CU: 2049 shared rows of 2816 values and 12 294 routed ones of 1408, us, shared + routed per CU, of which four are resident: 1 + 2 44.2, 1 + 3 46.0,
+  // 2 + 2 42.6, 1.5 + 2.5 40.8, 2 + 3 43.7, 1 + 4 43.8.  With the SiLU three are: 1 + 2.)
+  const int lds = std::max(BlockRows(shared.plan).lds(), dense ? dense_lds(routed.plan.kb) : BlockRows(routed.plan).lds());
+  const int shared_wgs = std::min(shared.rows, SILU ? cus : cus * 3 / 2) + 63 & ~63;
   if (!dense) {
     hipLaunchKernelGGL((row_quant_few_kernel<kFewThreads, 2, SILU, EXT>), dim3(shared.rows + routed.rows), dim3(kFewThreads), lds, s, routed, shared, shared.rows);
     return rows_launched();
   }
-  const int routed_wgs = std::min((routed.rows + 3) / 4, cus * 2) + 63 & ~63;
+  const int routed_wgs = std::min((routed.rows + 3) / 4, SILU ? cus * 2 : cus * 5 / 2) + 63 & ~63;
   const dim3 grid(shared_wgs + routed_wgs);
   switch ((routed.plan.n / 8 + 63) / 64) {
     case 1: hipLaunchKernelGGL((row_quant_pair_kernel<1, SILU, EXT>), grid, dim3(256), lds, s, routed, shared, shared_wgs); break;
@@ -1805,7 +1804,7 @@ static int launch_rows_as(const RowArgs& a, int lds_bytes, hipStream_t s) {
   }
   // table-driven factor times H_8, one size of row: one row per wave, dense stage on the matrix cores
   if (dense_rows(a)) {
-    const int dlds = dense_lds(n, a.plan.kb);
+    const int dlds = dense_lds(a.plan.kb);
     // as many workgroups as stay resident together (registers and LDS decide how many share a CU), each looping over its rows
     auto launch = [&](auto kernel, int which) {
       static int asked_lds[4][64] = {}, answer[4][64] = {};  // per kernel size and device: the last LDS size asked about
