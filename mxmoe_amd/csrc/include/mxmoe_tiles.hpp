@@ -552,7 +552,9 @@ struct MfmaTile {
 //     slice kt+kDepth (its registers are free again): kDepth * 4 KB of weights per wave are always in flight;
 //   - at the first unit of a k-step reads the activation fragments of the next k-step from LDS;
 //   - int4: widens the weight fragment of unit u+1, and on the last unit of a k-step the activation fragments of the next
-//     k-step, each right after its last use.
+//     k-step, each right after its last use;
+//   - fp8: both k-steps of a block are one matrix instruction, at the block's second unit, and the activation fragments of the next slice are read at
+//     the last unit.
 // Waits: vmcnt counts the direct-to-LDS loads and the weight loads together, in issue order; the barrier unit (2) waits until
 // only the loads issued after this wave's activation loads of slice kt+1 are outstanding (a fixed count, see kYounger).
 template <Op OP, int BM_, int BN_>
@@ -577,6 +579,11 @@ struct WxAxTile {
   static constexpr int kABits = OpTraits<OP>::kBitsPerElem, kWBits = kABits;  // bits per activation / weight element
   static constexpr int kOps = OP == Op::I4 ? 2 : 1;
   static constexpr int U = 4;                                    // units per K slice
+  // Fragment uf of a slice is (block, k-step).  fp8 takes both k-steps of a block together, at the second of the block's two units, so its fragments are block
+  // major, and a fragment is re-loaded two units after its own (kReload) instead of one.
+  static constexpr int block_of(int uf) { return OP == Op::F8 ? uf / 2 : uf % FN; }
+  static constexpr int step_of(int uf) { return OP == Op::F8 ? uf % 2 : uf / FN; }
+  static constexpr int kReload = OP == Op::F8 ? 2 : 1;
   static constexpr int kDmaTotal = BM / 16;                      // 1 KB pieces of one activation slice
   // Activation loads per wave and slice.  Every wave issues the same number of loads, because the hand-placed waits count them: a
   // tile with fewer pieces than waves (BM = 32) has the spare waves fetch a piece a second time (same bytes to the same LDS
@@ -591,19 +598,20 @@ struct WxAxTile {
   static constexpr int kDepth = OP == Op::I4 ? 2 : 4;
   using Acc = typename OpTraits<OP>::Acc;
 
-  // One 16-byte fragment pair of the byte formats.  int8: one instruction over the 32 k of the pair.  fp8 (e4m3): two instructions of
-  // 16 k, the first on the low 8 bytes of both lanes' fragments, the second on the high 8; which k a byte stands for is the same on
-  // both sides, and the sum runs over all of them either way (w8a8_g-1_sym_E4M3 of the reference: MMA_E4M3_K32,
-  // mxmoe/kernels/src/include/mm_tile.cuh:696-697).
+  // One 16-byte fragment pair of int8: one instruction over the 32 k of the pair.
   __device__ static __forceinline__ void mma_bytes(Acc& c, const v4i& w, const v4i& a) {
-    if constexpr (OP == Op::F8) {
-      typedef long v2l __attribute__((ext_vector_type(2)));
-      const v2l wl = __builtin_bit_cast(v2l, w), al = __builtin_bit_cast(v2l, a);
-      c = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(wl[0], al[0], c, 0, 0, 0);
-      c = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(wl[1], al[1], c, 0, 0, 0);
-    } else {
-      c = __builtin_amdgcn_mfma_i32_32x32x32_i8(w, a, c, 0, 0, 0);
-    }
+    if constexpr (OP != Op::F8) c = __builtin_amdgcn_mfma_i32_32x32x32_i8(w, a, c, 0, 0, 0);
+  }
+  // fp8 (e4m3): the fragment pairs of both k-steps of a block in one instruction over the 64 k of the slice (unit scales), at twice the rate of the 16-deep
+  // one.  (Half w4a4, half fp8, 60 experts of N = 2816, K = 2048 and N = 2048, K = 1408, 8192 tokens: both launches 350 -> 321 us; a Mixtral layer of 2000 tokens 837 ->
+  // 751.  The sums are as far from the float64 ones as they were: 1.2e-5 .. 5.1e-5 of their 2-norm.)  Which k a byte stands for is the same on both sides, and the sum runs over all of them either way (w8a8_g-1_sym_E4M3 of the reference: MMA_E4M3_K32,
+  // mxmoe/kernels/src/include/mm_tile.cuh:696-697).
+  __device__ static __forceinline__ void mma_slice(Acc& c, const v4i& w0, const v4i& w1, const v4i& a0, const v4i& a1) {
+    typedef int v8i __attribute__((ext_vector_type(8)));
+    constexpr int kUnit = 0x7F7F7F7F;
+    if constexpr (OP == Op::F8)
+      c = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(__builtin_shufflevector(w0, w1, 0, 1, 2, 3, 4, 5, 6, 7), __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7), c,
+                                                          0, 0, 0, kUnit, 0, kUnit);
   }
 
   // Vector-memory loads a wave issues in units a..b of one iteration: one weight fragment per unit, plus one activation load in
@@ -613,12 +621,12 @@ struct WxAxTile {
     for (int u = a; u <= b; ++u) n += 1 + (u < nd ? 1 : 0);
     return n;
   }
-  // Loads issued after the load of fragment `uf` (= k-step * FN + block) of a slice, up to and including the unit that first
-  // uses it: the fragment of unit uf is (re)loaded at unit uf+1 kDepth slices earlier and first used at unit uf-1 (int4: widened
-  // one unit ahead) or uf (int8).
+  // Loads issued after the load of fragment `uf` of a slice, up to and including the unit that first uses it: the fragment of unit uf
+  // is (re)loaded at unit uf+kReload kDepth slices earlier and first used at unit uf-1 (int4: widened one unit ahead), uf (int8) or at
+  // the second unit of its block (fp8).
   static constexpr int younger_than_fragment(int uf, int nd) {
-    const int ul = (uf + 1) % U, kl = -kDepth + (uf == U - 1 ? 1 : 0);
-    const int uc = OP == Op::I4 ? (uf + U - 1) % U : uf, kc = OP == Op::I4 && uf == 0 ? -1 : 0;
+    const int ul = (uf + kReload) % U, kl = -kDepth + (uf + kReload >= U ? 1 : 0);
+    const int uc = OP == Op::I4 ? (uf + U - 1) % U : OP == Op::F8 ? uf | 1 : uf, kc = OP == Op::I4 && uf == 0 ? -1 : 0;
     return ops_in(ul + 1, U - 1, nd) + ops_in(0, U - 1, nd) * (kc - kl - 1) + ops_in(0, uc, nd);
   }
 
@@ -699,7 +707,7 @@ struct WxAxTile {
 
     v4i pbq[kDepth][FN][2];  // packed weight fragments [slice % kDepth][block][k-step]
     v4i bop[2][kOps];        // int4: widened weight operands of units u, u+1
-    v4i aop[2][FM][kOps];    // activation operands; int8 double-buffers them by k-step parity, int4 widens in place (buffer 0)
+    v4i aop[2][FM][kOps];    // activation operands; int8 double-buffers them by k-step parity, int4 widens in place (buffer 0), fp8 holds both k-steps of a slice
     v4i pa[FM];              // int4: packed activation fragments of the next k-step
 
     auto mma = [&](Acc& c, const v4i* a, const v4i* b) {
@@ -746,8 +754,9 @@ struct WxAxTile {
       constexpr int u = decltype(uc)::value;
       if constexpr (u < kDma) dma_a(u, 1, 1);
       asm volatile("" ::: "memory");
-      if constexpr (u == 0) pbq[kDepth - 2][1][1] = load_b(1, 1, kDepth - 2);  // in place of "fragment of the previous iteration's last unit"
-      else pbq[kDepth - 1][(u - 1) % FN][(u - 1) / FN] = load_b((u - 1) % FN, (u - 1) / FN, kDepth - 1);
+      // (the first kReload units: in place of fragments of the previous iteration's last units)
+      constexpr int uf = (u + U - kReload) % U, d = u < kReload ? kDepth - 2 : kDepth - 1;
+      pbq[d][block_of(uf)][step_of(uf)] = load_b(block_of(uf), step_of(uf), d);
       asm volatile("" ::: "memory");
     });
 #pragma unroll
@@ -757,6 +766,7 @@ struct WxAxTile {
         widen(p, aop[0][i]);
       } else {
         aop[0][i][0] = lds_a(smem, 0, i);
+        if constexpr (OP == Op::F8) aop[1][i][0] = lds_a(smem, 1, i);
       }
     }
     if constexpr (OP == Op::I4) widen(pbq[0][0][0], bop[0]);
@@ -780,18 +790,38 @@ struct WxAxTile {
         }
         if constexpr (u < kDma) dma_a(u, kt + 2, nstage);
         asm volatile("" ::: "memory");
-        // re-load the fragment that unit u-1 used, kDepth slices ahead
-        if constexpr (u == 0) pbq[Pprev][1][1] = load_b(1, 1, kt - 1 + kDepth);
-        else pbq[P][(u - 1) % FN][(u - 1) / FN] = load_b((u - 1) % FN, (u - 1) / FN, kt + kDepth);
+        // re-load the fragment that unit u-1 used (fp8: of unit u-2, used at u-1 or u-2), kDepth slices ahead
+        constexpr int uf = (u + U - kReload) % U;
+        if constexpr (u < kReload) pbq[Pprev][block_of(uf)][step_of(uf)] = load_b(block_of(uf), step_of(uf), kt - 1 + kDepth);
+        else pbq[P][block_of(uf)][step_of(uf)] = load_b(block_of(uf), step_of(uf), kt + kDepth);
         asm volatile("" ::: "memory");
         if constexpr (OP == Op::I4) {
           // weight operands of unit u+1
           if constexpr (u + 1 < U) ready(std::integral_constant<int, u + 1>{}, pbq[P][(u + 1) % FN][(u + 1) / FN]);
           else ready(std::integral_constant<int, 0>{}, pbq[Pnext][0][0]);
+        } else if constexpr (OP == Op::F8) {
+          if constexpr (u % 2 == 1) {
+            ready(std::integral_constant<int, u - 1>{}, pbq[P][u / 2][0]);
+            ready(uc, pbq[P][u / 2][1]);
+          }
         } else {
           ready(uc, pbq[P][j][step]);
         }
-        if (live) {
+        if constexpr (OP == Op::F8) {
+          // both k-steps of block u / 2; the activation fragments of the next slice (behind the barrier of unit 2) each right after the last use of this one's
+          if (u % 2 == 1 && live) {
+#pragma unroll
+            for (int i = 0; i < FM; ++i) {
+              mma_slice(acc[i][u / 2], pbq[P][u / 2][0], pbq[P][u / 2][1], aop[0][i][0], aop[1][i][0]);
+              // (the product stays here: moved past a branch, its fragments would be copied while loads into them are in flight)
+              asm volatile("" : "+v"(acc[i][u / 2]) : : "memory");
+              if (u == U - 1) {
+                aop[0][i][0] = lds_a(sn, 0, i);
+                aop[1][i][0] = lds_a(sn, 1, i);
+              }
+            }
+          }
+        } else if (live) {
           // activation fragments of the next k-step
           if (j == 0) {
 #pragma unroll

@@ -61,6 +61,7 @@ MMA_SHAPE = {
     # int4 values held as 6-bit floats (bf6, e3m2: every integer -8 .. 8 is one) on v_mfma_scale_f32_32x32x64_f8f6f4 with unit
     # scales: the fp32 accumulators are the exact integer sums, at twice the int8 instruction's rate
     "MFMA_F32_32x32x64_BF6_FROM_I4": (32, 32, 64),
+    # (the name is that of the format's entry in the kernel profile; the tile multiplies 64 deep, both k-steps of a slice at once)
     "MFMA_F32_32x32x16_FP8": (32, 32, 16),
 }
 MMA_TO_ACC_TYPE = {"MFMA_F32_32x32x16_F16": "float", "MFMA_F32_32x32x16_BF16": "float", "MFMA_I32_32x32x32_I8": "int32_t", "MFMA_I32_32x32x32_I8_FROM_I4": "int32_t", "MFMA_F32_16x16x32_F16": "float",
