@@ -12,6 +12,7 @@
 // intermediate value are neither written nor read.  The same kernels' arithmetic, bit for bit.  Measured, that form -> this one, us a
 // pass: DeepSeek-V2-Lite w4a16 / w3a16 47.7 -> 35.2 (1 token), 98.7 -> 84.9 (32), 163 -> 139 (201); Qwen1.5-MoE w4a4 456 -> 402 (8192,
 // of which the head 47 -> 24, the activation step 107 -> 72); Mixtral w4a4 / w8a8 / w4a16 3368 -> 3249 (8192).
+#include <climits>
 #include <hip/hip_runtime.h>
 
 #include <memory>
@@ -391,6 +392,11 @@ int mxmoe_layer_create(const mxmoe_layer_desc* d, void** handle) {
     p.Et = et;
     p.shared_rows = shared_rows;
     p.info = plan_info_of_block(registry()[kid], h_desc, et);
+    // a problem has two row segments only with more rows than its format's lowest shape: for a handful of tokens the planner need not look for pairs
+    int low = INT_MAX;
+    for (const BranchInfo& b : registry()[kid].branches)
+      if (!is_weight_only(b.fmt)) low = std::min(low, b.BM);
+    if ((long)d->num_tokens * d->topk <= low) p.info.may_pair = 0;
     return kid;
   };
   f->d.kernel_gate_up = fill(f->pair.p[0], d->kernel_gate_up, d->d_gate_up, d->h_gate_up, d->act, d->plan_gate_up);
