@@ -172,8 +172,7 @@ int mxmoe_group_gemm_plan_tile_area(int kernel_id, const mxmoe_dim3* h_sizes, co
     if ((unsigned)a.entry[i].problem_branch & kPairSecond) --i;
     const int pb = a.entry[i].problem_branch, p = entry_problem(pb);
     auto locate = [&](int local, int rows, const BranchInfo& b, int word) {
-      const int w_bits = b.fmt == Fmt::W8A16 || b.fmt == Fmt::W8A8 ? 8 : b.fmt == Fmt::FP16 ? 16 : b.fmt == Fmt::W3A16 ? 3 : b.fmt == Fmt::W2A16 ? 2 : 4;
-      return locate_tile(local, rows, (int)h_sizes[p].y, (int)h_sizes[p].z, b.BM, b.BN, is_weight_only(b.fmt) ? 16 : w_bits, w_bits, word);
+      return locate_tile(local, rows, (int)h_sizes[p].y, (int)h_sizes[p].z, b.BM, b.BN, b.a_bits, b.w_bits, word);
     };
     const BranchInfo* b = &k.branches[entry_branch(pb)];
     TileAt at = locate(tile - a.entry[i].first, a.entry[i].rows, *b, pb);

@@ -310,6 +310,7 @@ inline const char* fmt_name(Fmt f, bool sym) {
 
 struct BranchInfo {
   Fmt fmt;
+  int a_bits, w_bits;  // of an element of either operand as the tile reads it (kABits, kWBits: what the order of a problem's tiles goes by)
   int BM, BN, BK, WGM, WGN;
   int lds_bytes;
   int k_multiple;  // K must be a multiple of this
@@ -331,28 +332,28 @@ struct BranchOf<MfmaTile<OP, BM, BN, WGM, WGN>> {
     using T = MfmaTile<OP, BM, BN, WGM, WGN>;
     const Fmt f = OP == Op::I8 ? Fmt::W8A8 : (OP == Op::I4 ? Fmt::W4A4 : Fmt::FP16);
     // bfloat16 problems carry the QParams of fp16 ones (16 / 16 bits): which of the two a kernel computes is the kernel's variant
-    return BranchInfo{f, BM, BN, T::BK, WGM, WGN, T::kLdsBytes, T::BK, 0, 0, OP == Op::BF16 ? kVariantBf16 : 0};
+    return BranchInfo{f, T::kABits, T::kWBits, BM, BN, T::BK, WGM, WGN, T::kLdsBytes, T::BK, 0, 0, OP == Op::BF16 ? kVariantBf16 : 0};
   }
 };
 template <int BM>
 struct BranchOf<WxAxGTile<BM>> {
   static BranchInfo get() {
     using T = WxAxGTile<BM>;
-    return BranchInfo{Fmt::W4A4G128, BM, T::BN, T::BK, 1, 4, T::kLdsBytes, T::BK, 0};
+    return BranchInfo{Fmt::W4A4G128, T::kABits, T::kWBits, BM, T::BN, T::BK, 1, 4, T::kLdsBytes, T::BK, 0};
   }
 };
 template <Op OP, int BM, int BN>
 struct BranchOf<WxAxTile<OP, BM, BN>> {
   static BranchInfo get() {
     using T = WxAxTile<OP, BM, BN>;
-    return BranchInfo{OP == Op::I4 ? Fmt::W4A4 : Fmt::W8A8, BM, BN, T::BK, 1, 4, T::kLdsBytes, T::BK, 0, 0, OP == Op::F8 ? kVariantFp8 : 0};
+    return BranchInfo{OP == Op::I4 ? Fmt::W4A4 : Fmt::W8A8, T::kABits, T::kWBits, BM, BN, T::BK, 1, 4, T::kLdsBytes, T::BK, 0, 0, OP == Op::F8 ? kVariantFp8 : 0};
   }
 };
 template <Op OP>
 struct BranchOf<WxAxNarrowTile<OP>> {
   static BranchInfo get() {
     using T = WxAxNarrowTile<OP>;
-    return BranchInfo{OP == Op::I4 ? Fmt::W4A4 : Fmt::W8A8, T::BM, T::BN, T::BK, 1, 1, T::kLdsBytes, T::BK, 0};
+    return BranchInfo{OP == Op::I4 ? Fmt::W4A4 : Fmt::W8A8, T::kABits, T::kWBits, T::BM, T::BN, T::BK, 1, 1, T::kLdsBytes, T::BK, 0};
   }
 };
 template <int BM>
@@ -361,14 +362,14 @@ struct BranchOf<Bf6Tile<BM>> {
   // fragments), so the two kinds never share a kernel: the kernel a caller picks says which layout its operands have
   static BranchInfo get() {
     using T = Bf6Tile<BM>;
-    return BranchInfo{Fmt::W4A4, BM, T::BN, T::BK, 1, 4, T::kLdsBytes, 128, 0, 256, kVariantBf6};
+    return BranchInfo{Fmt::W4A4, T::kABits, T::kWBits, BM, T::BN, T::BK, 1, 4, T::kLdsBytes, 128, 0, 256, kVariantBf6};
   }
 };
 template <int WBITS, int BN, int MB, int WAVES>
 struct BranchOf<SkinnyWoTile<WBITS, BN, MB, WAVES>> {
   static BranchInfo get() {
     using T = SkinnyWoTile<WBITS, BN, MB, WAVES>;
-    return BranchInfo{WBITS == 8 ? Fmt::W8A16 : WBITS == 4 ? Fmt::W4A16 : WBITS == 3 ? Fmt::W3A16 : Fmt::W2A16, T::BM, BN, 128, 1, 4, T::kLdsBytes, 128, 0};
+    return BranchInfo{WBITS == 8 ? Fmt::W8A16 : WBITS == 4 ? Fmt::W4A16 : WBITS == 3 ? Fmt::W3A16 : Fmt::W2A16, T::kABits, T::kWBits, T::BM, BN, 128, 1, 4, T::kLdsBytes, 128, 0};
   }
 };
 
@@ -411,7 +412,7 @@ template <int WBITS, int BM, int BN>
 struct BranchOf<WoMfmaTile<WBITS, BM, BN>> {
   static BranchInfo get() {
     using T = WoMfmaTile<WBITS, BM, BN>;
-    return BranchInfo{WBITS == 8 ? Fmt::W8A16 : WBITS == 4 ? Fmt::W4A16 : WBITS == 3 ? Fmt::W3A16 : Fmt::W2A16, BM, BN, 128, T::WM, 4 / T::WM, T::kLdsBytes, 128, 0};
+    return BranchInfo{WBITS == 8 ? Fmt::W8A16 : WBITS == 4 ? Fmt::W4A16 : WBITS == 3 ? Fmt::W3A16 : Fmt::W2A16, T::kABits, T::kWBits, BM, BN, 128, T::WM, 4 / T::WM, T::kLdsBytes, 128, 0};
   }
 };
 

@@ -95,3 +95,11 @@ def test_device_planner_makes_the_same_pairs(lib, q, rows, n, k):
     assert list(hdr[:4]) == [0, ne, tiles, nph] and grid <= lib.mxmoe_plan_grid_bound(kid, desc, e, sum(counts), 0)
     assert np.array_equal(hdr[4:5 + nph], tab[4:5 + nph]) and np.array_equal(hdr[13:14 + nph], tab[13:14 + nph])
     assert np.array_equal(hdr[23:23 + 4 * ne], tab[22:22 + 4 * ne].astype(np.int32))
+
+
+@pytest.mark.parametrize("kernel,tiles", [("groupgemm_hz_fused_wxax", 8), ("groupgemm_hz_fused_wxax_b6", 5), ("groupgemm_hz_fused_all_b6", 5)])
+def test_groups_of_row_tiles_by_the_bits_that_the_tile_reads(lib, kernel, tiles):
+    """2 MB of activations to a group: 128 rows of 4096 values are 256 KB of int4 codes, 384 KB of bf6 fragments."""
+    _, area = _launch(lib, [(1280, 28672, 4096, W4)] * 8, lib.mxmoe_find_kernel(kernel.encode()))
+    first = area[::8][:tiles + 1]  # the first tiles of XCD 0
+    assert first[:, 1].tolist() == [128 * i for i in range(tiles)] + [0] and first[:, 3].tolist() == [0] * tiles + [256]
