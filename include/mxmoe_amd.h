@@ -105,7 +105,7 @@ int mxmoe_group_gemm_plan(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_
 
 /* The tile tables themselves (host-only; what the generated launcher keeps in its prefix-sum array, kernel_sketch.py:89-104): out receives
  * {entries, tiles, phases, workgroups}, phase_tile0[9], phase_wg0[9], then per entry {first tile, first row, rows, problem | branch << 16 |
- * what a pair of entries carries (bits 21 .. 31: mxmoe_launch.hpp, pair_word)}.  At most 120 problems; used by the tests that compare the device-side planner with the host launcher. */
+ * what a pair of entries carries (bits 21 .. 29: mxmoe_launch.hpp, pair_word)}.  At most 120 problems; used by the tests that compare the device-side planner with the host launcher. */
 int mxmoe_group_gemm_plan_tables(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int problem_count, int32_t* out, int out_ints);
 
 /* The tile each workgroup of such a launch runs when the grid holds `grid` workgroups (host-only; the role of the block -> tile walk of

@@ -179,7 +179,7 @@ int mxmoe_group_gemm_plan_tile_area(int kernel_id, const mxmoe_dim3* h_sizes, co
     if (at.second) {  // as the kernels do: counted inside its own segment
       ++i;
       b = &k.branches[entry_branch(a.entry[i].problem_branch)];
-      at = locate(at.n * (pair_width(pb) >> ((unsigned)pb >> 30)) + at.m, a.entry[i].rows, *b, 0);
+      at = locate(at.n * pair_width(pb) + at.m, a.entry[i].rows, *b, 0);
     }
     const FusedArgs::Entry& e = a.entry[i];
     o[0] = p;

@@ -74,8 +74,8 @@ static_assert(sizeof(FusedArgs) <= 4096, "kernel arguments are limited to 4 KB")
 // A pair: the two row segments of one problem as neighbouring entries whose tiles are dealt out column by column, so that the tiles of both
 // shapes that read a block of weight rows run at the same time and the block is fetched once.  (As phases of their own, the launch went through
 // all of its weights a second time for the remainder tiles; with more weights than the caches hold, that was the launch's time.)
-// Fields of problem_branch, on both entries: bits 21 .. 28 the second segment's tiles per column tile of the first (0: no pair), bit 29 set on
-// the second entry, bits 30 .. 31 log2 of the second's column tiles per column tile of the first.
+// Both shapes' column tiles are equally wide.  Fields of problem_branch, on both entries: bits 21 .. 28 the second segment's row tiles (0: no pair), bit 29 set on
+// the second entry.
 constexpr unsigned kPairSecond = 1u << 29;
 __host__ __device__ inline int entry_problem(int pb) { return pb & 0xFFFF; }
 __host__ __device__ inline int entry_branch(int pb) { return (int)((unsigned)pb >> 16 & 31u); }
@@ -120,14 +120,22 @@ __host__ __device__ __forceinline__ TileAt locate_tile(int local, int rows, int 
   const int width = rows_g + (last ? beside : 0);
   const int col = r / width, at = r - col * width;
   if (beside == 0 || at < rows_g) return TileAt{g + at, col, false};
-  const int lg = (int)((unsigned)problem_branch >> 30), sub = at - rows_g;
-  return TileAt{sub >> lg, (col << lg) + (sub & ((1 << lg) - 1)), true};
+  return TileAt{at - rows_g, col, true};
 }
 
-// Whether a kernel of these tiles may be given pairs: two of its shapes are of one format that has them (pairs_pay; weight-only tiles have 16-bit
-// activations and less than 16 bits a weight).
+// Whether a kernel of these tiles may be given pairs (PlanInfo::may_pair): some of them are of a format that has them (weight-only tiles have 16-bit activations and
+// less than 16 bits a weight, group-scaled ones are bound by their arithmetic), and it is not one of those for few rows.  Those run lists of at most 64 rows, which
+// have nothing to pair, in a few microseconds, of which the looking for pairs was a part.
+template <class T>
+constexpr bool kPairs = T::kABits == T::kWBits;
+template <int BM>
+constexpr bool kPairs<WxAxGTile<BM>> = false;
+template <class T>
+constexpr bool kNarrow = false;
+template <Op OP>
+constexpr bool kNarrow<WxAxNarrowTile<OP>> = true;
 template <class... Tiles>
-constexpr bool kMayPair = ((Tiles::kABits == Tiles::kWBits) || ...);
+constexpr bool kMayPair = (kPairs<Tiles> || ...) && !(kNarrow<Tiles> || ...);
 
 // f(TileType<T>{}) with T the tile of branch `branch`: the compile-time dispatch over a kernel's tiles.
 template <class T>
@@ -239,7 +247,7 @@ __device__ __forceinline__ void fused_body(ArgsPtr args, uint8_t* smem) {
       en_row0 = uni(args->entry[lo + 1].row0);
       en_rows = uni(args->entry[lo + 1].rows);
       branch = entry_branch(uni(args->entry[lo + 1].problem_branch));
-      local = uni(at.n * (int)(pair_width(en_pb) >> ((unsigned)en_pb >> 30)) + at.m);
+      local = uni(at.n * pair_width(en_pb) + at.m);
     } else {  // (the first segment is whole tiles) as the one row tile of its own segment
       en_row0 += uni(at.m * bm);
       en_rows = uni(bm);
@@ -468,7 +476,7 @@ struct PlanInfo {
   int nb;                       // branches
   // Narrow integer tiles among them; and, where a launch is planned with them, whether it has few blocks of channels (kPoleBlocks).
   int narrow, few_blocks;
-  int may_pair;  // a format that has pairs (pairs_pay) comes in several shapes
+  int may_pair;  // a format that has pairs (pairs_pay) comes in several shapes, and it is no kernel for few rows
   uint8_t order[kMaxBranches];  // positions in b, most expensive tile first (branch_cost); ties keep the registration order
   uint8_t fmt_start[kNumFmts + 4];
   // by format, in registration order inside a format: those of format f are b[fmt_start[f]] .. b[fmt_start[f + 1] - 1], and the planners
@@ -498,12 +506,11 @@ constexpr int kLongTiles = 128;
 constexpr int kLongK = 2048;
 __host__ __device__ inline bool runs_long(int K, int kmin) { return K > kmin && K >= kLongK; }
 
-// The fields of a pair of segments (FusedArgs::Entry); 0 where their column tiles do not come out even.
-__host__ __device__ inline unsigned pair_word(const Segment (&s)[2], int N) {
-  const int lg = s[0].bn_log2 - s[1].bn_log2;
-  if (lg < 0 || lg > 3 || tiles_over(N, s[1].bn_log2) != tiles_over(N, s[0].bn_log2) << lg) return 0;
-  const unsigned width = (unsigned)tiles_over(s[1].rows, s[1].bm_log2) << lg;
-  return width <= 255 ? width << 21 | (unsigned)lg << 30 : 0;
+// The fields of a pair of segments (FusedArgs::Entry); 0 where their column tiles differ.
+__host__ __device__ inline unsigned pair_word(const Segment (&s)[2]) {
+  if (s[0].bn_log2 != s[1].bn_log2) return 0;
+  const unsigned width = (unsigned)tiles_over(s[1].rows, s[1].bm_log2);
+  return width <= 255 ? width << 21 : 0;
 }
 // Whether the two row segments of a problem are dealt out as a pair.  What a pair saves is the second trip of its weights from memory;
 // what it costs is that cheap tiles no longer come last, where they fill the end of the launch, so a launch has to have many tiles for it: `launch_tiles`
@@ -641,9 +648,9 @@ inline PlanInfo make_plan_info(const std::vector<BranchInfo>& branches) {
   PlanInfo k;
   std::memset(&k, 0, sizeof k);
   k.nb = std::min((int)branches.size(), kMaxBranches);
-  for (int i = 0; i < k.nb; ++i)
-    for (int j = 0; j < i; ++j) k.may_pair |= branches[i].fmt == branches[j].fmt && !is_weight_only(branches[i].fmt) && branches[i].fmt != Fmt::W4A4G128;
   for (int i = 0; i < k.nb; ++i) k.narrow |= integer_sums((int)branches[i].fmt) && branches[i].BN == 64;
+  for (int i = 0; i < k.nb && !k.narrow; ++i)  // (kMayPair)
+    for (int j = 0; j < i; ++j) k.may_pair |= branches[i].fmt == branches[j].fmt && !is_weight_only(branches[i].fmt) && branches[i].fmt != Fmt::W4A4G128;
   auto log2_of = [](int v) {
     int lg = 0;
     while ((1 << lg) < v) ++lg;
@@ -987,7 +994,7 @@ inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, c
         last_error() = buf;
         return 3;
       }
-      const unsigned pair = ns == 2 && pairs_pay((int)f, scope.launch_tiles, scope.launch_cols) ? pair_word(sg, (int)sz.y) : 0;
+      const unsigned pair = ns == 2 && pairs_pay((int)f, scope.launch_tiles, scope.launch_cols) ? pair_word(sg) : 0;
       entries[nent++] = Entry{sg[j].row0, sg[j].rows, i, sg[j].branch, sg[j].tiles, pair | (pair && j ? kPairSecond : 0u), sg[pair ? 0 : j].branch};
     }
   }

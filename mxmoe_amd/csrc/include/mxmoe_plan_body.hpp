@@ -218,7 +218,7 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
   const PlanBranch& my_branch = info.b[info.order[min(lane, kMaxBranches - 1)]];  // lane r: the branch of rank r
   const int my_order = my_branch.index;
   unsigned pair = 0;  // the second segment goes beside the first: one item of two entries
-  if (info.may_pair && ns == 2 && pairs_pay(fmt, (int)((sh.load[0] >> 16) + (sh.load[1] >> 16)), (int)((sh.load[0] & 0xFFFF) + (sh.load[1] & 0xFFFF)))) pair = pair_word(sg, N);
+  if (info.may_pair && ns == 2 && pairs_pay(fmt, (int)((sh.load[0] >> 16) + (sh.load[1] >> 16)), (int)((sh.load[0] & 0xFFFF) + (sh.load[1] & 0xFFFF)))) pair = pair_word(sg);
   int seg_rank[2] = {-1, -1}, seg_pos[2] = {0, 0}, seg_first[2] = {0, 0};
   // per branch in run order, this wave's entries and tiles
   for (int r = 0; active && r < info.nb; ++r) {

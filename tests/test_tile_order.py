@@ -103,3 +103,11 @@ def test_groups_of_row_tiles_by_the_bits_that_the_tile_reads(lib, kernel, tiles)
     _, area = _launch(lib, [(1280, 28672, 4096, W4)] * 8, lib.mxmoe_find_kernel(kernel.encode()))
     first = area[::8][:tiles + 1]  # the first tiles of XCD 0
     assert first[:, 1].tolist() == [128 * i for i in range(tiles)] + [0] and first[:, 3].tolist() == [0] * tiles + [256]
+
+
+@pytest.mark.parametrize("kernel", ["groupgemm_hz_fused_wxax_few", "groupgemm_hz_fused_all_few"])
+@pytest.mark.parametrize("q", [W8, W4])
+def test_kernels_for_few_rows_make_no_pairs(lib, kernel, q):
+    """More rows than such a kernel is chosen for: its two shapes one after the other."""
+    tab, _ = _launch(lib, [(96, 28672, 4096, q)] * 12, lib.mxmoe_find_kernel(kernel.encode()))
+    assert tab[2] == 2 and not _pairs(tab)
