@@ -83,18 +83,20 @@ int mxmoe_group_gemm_plan(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_
   if (kernel_id >= (int)reg.size()) { last_error() = "kernel id out of range"; return 2; }
   const FusedKernel& k = reg[kernel_id];
   int total = 0;
-  LaunchScope scope;  // of the launch that holds the problem
-  for (int i = 0, next = 0; i < problem_count; ++i) {
+  LaunchScope scope;  // of the launch that holds the problem, whose first is problem `base`
+  for (int i = 0, base = 0, next = 0; i < problem_count; ++i) {
     if (i == next) {
+      base = i;
       next = i + launch_length(k, h_q, i, problem_count);
-      scope = launch_scope(plan_of(k), h_sizes + i, h_q + i, next - i);
+      launch_scope(plan_of(k), h_sizes + i, h_q + i, next - i, scope);
     }
     const Fmt f = classify(h_q[i]);
     Segment sg[2];
-    const int ns = f == Fmt::UNSUPPORTED ? -1 : plan_segments(plan_of(k), (int)f, (int)h_sizes[i].x, (int)h_sizes[i].y, scope.long_tiles_of(h_sizes[i]), scope.few_blocks, sg);
+    const int ns = scope.segments(plan_of(k), i - base, h_sizes[i], (int)f, sg);
     if (ns < 0) { last_error() = "quant type not supported"; return 1; }
     if (branch_out) {  // (an empty problem: the branch one row would take)
-      if (ns == 0) plan_segments(plan_of(k), (int)f, 1, (int)h_sizes[i].y, scope.long_tiles_of(h_sizes[i]), scope.few_blocks, sg);
+      PlanChoice c;
+      if (ns == 0 && plan_choose(plan_of(k), (int)f, 1, (int)h_sizes[i].y, c) > 0) scope.split(plan_of(k), (int)f, 1, h_sizes[i], c, sg);
       branch_out[i] = sg[0].branch;
     }
     for (int j = 0; j < ns; ++j) {

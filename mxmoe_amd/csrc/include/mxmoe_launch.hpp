@@ -636,12 +636,11 @@ __host__ __device__ inline int plan_split(const PlanInfo& k, int f, int M, int N
   return 2;
 }
 
-// Both steps: the number of segments (0 for M == 0), or -1 when the kernel has no tile for `f`.  `pole`: the problem is in a launch of few blocks (kPoleBlocks).
-inline int plan_segments(const PlanInfo& k, int f, int M, int N, int long_tiles, bool pole, Segment out[2]) {
+// Both steps for a problem by itself: the number of segments (0 for M == 0), or -1 when the kernel has no tile for `f`.
+inline int plan_segments(const PlanInfo& k, int f, int M, int N, Segment out[2]) {
   PlanChoice c;
   const int rc = plan_choose(k, f, M, N, c);
-  if (pole && long_tiles == 0 && integer_sums(f)) long_tiles = c.large_tiles;
-  return rc <= 0 ? rc : plan_split(k, f, M, N, c, long_tiles, out);
+  return rc <= 0 ? rc : plan_split(k, f, M, N, c, 0, out);
 }
 
 inline PlanInfo make_plan_info(const std::vector<BranchInfo>& branches) {
@@ -816,7 +815,7 @@ inline bool kernel_covers(const FusedKernel& k, const mxmoe_qparams* q, int coun
   for (int i = 0; i < count; ++i) {
     const Fmt f = classify(q[i]);
     Segment sg[2];
-    if (f == Fmt::UNSUPPORTED || plan_segments(plan_of(k), (int)f, 1, 256, 0, false, sg) < 0) return false;
+    if (f == Fmt::UNSUPPORTED || plan_segments(plan_of(k), (int)f, 1, 256, sg) < 0) return false;
   }
   return true;
 }
@@ -934,16 +933,29 @@ inline bool shape_ok(const BranchInfo& bi, const mxmoe_dim3& sz) {
   return sz.z != 0 && sz.z % bi.k_multiple == 0 && (int)sz.z >= bi.k_min && sz.y % 8 == 0 && !(wo && sz.y % 16 != 0);
 }
 
-// What the planning of one launch's problems has in common: its smallest K, its tiles, the large tiles of its long problems, whether it has few blocks.  Problems without rows
+// What the planning of one launch's problems has in common: its smallest K, its tiles (where it may have pairs), the large tiles of its long problems, whether it has
+// few blocks; and what was chosen for each problem on the way, so that the tables do not choose again.  Problems without rows
 // have no part in it: a list plans the same with and without them (the device planner sees every expert, the operators leave out empty ones).
 struct LaunchScope {
   int kmin = 0x7fffffff, long_tiles = 0, launch_tiles = 0, launch_cols = 0;
   bool few_blocks = false;
-  // the `long_tiles` argument of a problem's plan
-  int long_tiles_of(const mxmoe_dim3& sz) const { return runs_long((int)sz.z, kmin) ? long_tiles : 0; }
+  int8_t have[kMaxProblems];          // plan_choose's answer for each problem (-1 too where its format is not supported)
+  union {
+    PlanChoice choice[kMaxProblems];  // where that is 1
+  };
+  LaunchScope() {}  // (leaves the arrays alone)
+  // A problem of `M` rows, N and K of `sz`, whose shapes are `c`: plan_split in this launch.
+  int split(const PlanInfo& pi, int f, int M, const mxmoe_dim3& sz, const PlanChoice& c, Segment out[2]) const {
+    return plan_split(pi, f, M, (int)sz.y, c, runs_long((int)sz.z, kmin) ? long_tiles : few_blocks && integer_sums(f) ? c.large_tiles : 0, out);
+  }
+  // The number of segments of problem i (0 without rows), or -1 when the kernel has no tile for it.
+  int segments(const PlanInfo& pi, int i, const mxmoe_dim3& sz, int f, Segment out[2]) const {
+    return have[i] <= 0 ? have[i] : split(pi, f, (int)sz.x, sz, choice[i], out);
+  }
 };
-inline LaunchScope launch_scope(const PlanInfo& pi, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int n) {
-  LaunchScope s;
+inline void launch_scope(const PlanInfo& pi, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int n, LaunchScope& s) {
+  s.kmin = 0x7fffffff;
+  s.long_tiles = s.launch_tiles = s.launch_cols = 0;
   long blocks = 0;
   for (int i = 0; i < n; ++i)
     if (h_sizes[i].x != 0) {
@@ -953,14 +965,17 @@ inline LaunchScope launch_scope(const PlanInfo& pi, const mxmoe_dim3* h_sizes, c
   s.few_blocks = pi.narrow && blocks <= kPoleBlocks;
   for (int i = 0; i < n; ++i) {
     const Fmt f = classify(h_q[i]);
-    PlanChoice c;
-    if (f == Fmt::UNSUPPORTED || plan_choose(pi, (int)f, (int)h_sizes[i].x, (int)h_sizes[i].y, c) <= 0) continue;
-    const unsigned load = launch_load_of(c, (int)h_sizes[i].x, (int)h_sizes[i].y, (int)h_sizes[i].z);
-    s.launch_tiles += (int)(load >> 16);
-    s.launch_cols += (int)(load & 0xFFFF);
+    PlanChoice& c = s.choice[i];
+    c = PlanChoice{};
+    s.have[i] = f == Fmt::UNSUPPORTED ? -1 : (int8_t)plan_choose(pi, (int)f, (int)h_sizes[i].x, (int)h_sizes[i].y, c);
+    if (s.have[i] <= 0) continue;
+    if (pi.may_pair) {
+      const unsigned load = launch_load_of(c, (int)h_sizes[i].x, (int)h_sizes[i].y, (int)h_sizes[i].z);
+      s.launch_tiles += (int)(load >> 16);
+      s.launch_cols += (int)(load & 0xFFFF);
+    }
     if (runs_long((int)h_sizes[i].z, s.kmin)) s.long_tiles = std::min(s.long_tiles + c.large_tiles, kLongTiles);
   }
-  return s;
 }
 
 // Tile tables of one launch over problems [base, base + n) (n <= kMaxProblems): entries, phases, totals of `a`; *grid receives the
@@ -976,12 +991,13 @@ inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, c
   };
   Entry entries[kMaxEntries];
   int nent = 0;
-  const LaunchScope scope = launch_scope(pi, h_sizes + base, h_q + base, n);
+  LaunchScope scope;
+  launch_scope(pi, h_sizes + base, h_q + base, n, scope);
   for (int i = 0; i < n; ++i) {
     const mxmoe_dim3& sz = h_sizes[base + i];
     const Fmt f = classify(h_q[base + i]);
     Segment sg[2];
-    const int ns = f == Fmt::UNSUPPORTED ? -1 : plan_segments(pi, (int)f, (int)sz.x, (int)sz.y, scope.long_tiles_of(sz), scope.few_blocks, sg);
+    const int ns = scope.segments(pi, i, sz, (int)f, sg);
     if (ns < 0) {
       last_error() = "quant type not supported";
       return 1;
@@ -994,7 +1010,7 @@ inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, c
         last_error() = buf;
         return 3;
       }
-      const unsigned pair = ns == 2 && pairs_pay((int)f, scope.launch_tiles, scope.launch_cols) ? pair_word(sg) : 0;
+      const unsigned pair = ns == 2 && pi.may_pair && pairs_pay((int)f, scope.launch_tiles, scope.launch_cols) ? pair_word(sg) : 0;
       entries[nent++] = Entry{sg[j].row0, sg[j].rows, i, sg[j].branch, sg[j].tiles, pair | (pair && j ? kPairSecond : 0u), sg[pair ? 0 : j].branch};
     }
   }

@@ -97,7 +97,7 @@ static bool covers_blocks(const FusedKernel& k, const mxmoe_block_desc* h_desc, 
   for (int i = 0; i < et; ++i) {
     Segment sg[2];
     const int f = fmt_of(h_desc[i].q);
-    if (f == (int)Fmt::UNSUPPORTED || plan_segments(plan_of(k), f, 1, 256, 0, false, sg) < 0) return false;
+    if (f == (int)Fmt::UNSUPPORTED || plan_segments(plan_of(k), f, 1, 256, sg) < 0) return false;
     // a kernel's w4a4 tiles take packed int4 rows or bf6 fragments, never both: the descriptor says which the block will get
     if (f == (int)Fmt::W4A4 && kernel_takes_bf6(k) != wants_bf6(h_desc[i].q)) return false;
     if (f == (int)Fmt::W8A8 && (kernel_variant(k, Fmt::W8A8) == kVariantFp8) != wants_fp8(h_desc[i].q)) return false;
@@ -248,7 +248,7 @@ int mxmoe_plan_grid_bound(int kernel_id, const mxmoe_block_desc* h_desc, int num
       if (sn.f == f && sn.n == n && sn.maybe_long == maybe_long) hit = &sn;
     if (!hit) {
       Segment sg[2];
-      plan_segments(pi, f, 1 << 20, n, 0, false, sg);
+      plan_segments(pi, f, 1 << 20, n, sg);
       const BranchInfo& bi = registry()[kid].branches[sg[0].branch];
       const int bm = bi.BM, cols = (n + bi.BN - 1) / bi.BN;
       Seen sn{f, n, maybe_long, tiles_of(f, 1, n, maybe_long), 0, 0.0, (double)cols / bm};
