@@ -23,15 +23,16 @@ __device__ __forceinline__ uint64_t match_same(int e, int nbits) {
 // crossbar costs an LDS round trip each.
 template <int CTRL, int ROWS>
 __device__ __forceinline__ int dpp_or_zero(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false); }
-__device__ __forceinline__ int wave_inclusive_scan(int v) {
-  v += dpp_or_zero<0x111, 0xF>(v);
-  v += dpp_or_zero<0x112, 0xF>(v);
-  v += dpp_or_zero<0x114, 0xF>(v);
-  v += dpp_or_zero<0x118, 0xF>(v);
-  v += dpp_or_zero<0x142, 0xA>(v);
-  v += dpp_or_zero<0x143, 0xC>(v);
+__device__ __forceinline__ unsigned wave_inclusive_scan(unsigned v) {
+  v += (unsigned)dpp_or_zero<0x111, 0xF>((int)v);
+  v += (unsigned)dpp_or_zero<0x112, 0xF>((int)v);
+  v += (unsigned)dpp_or_zero<0x114, 0xF>((int)v);
+  v += (unsigned)dpp_or_zero<0x118, 0xF>((int)v);
+  v += (unsigned)dpp_or_zero<0x142, 0xA>((int)v);
+  v += (unsigned)dpp_or_zero<0x143, 0xC>((int)v);
   return v;
 }
+__device__ __forceinline__ int wave_inclusive_scan(int v) { return (int)wave_inclusive_scan((unsigned)v); }
 template <int CTRL, int ROWS>
 __device__ __forceinline__ long dpp_or_zero(long v) {
   const unsigned lo = (unsigned)dpp_or_zero<CTRL, ROWS>((int)v), hi = (unsigned)dpp_or_zero<CTRL, ROWS>((int)((unsigned long)v >> 32));

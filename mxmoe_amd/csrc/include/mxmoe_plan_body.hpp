@@ -195,7 +195,7 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
     // (launch_scope): whether one of K >= kLongK is above the launch's smallest is known behind the barrier
     have = mine ? plan_choose(info, fmt, (int)rows, N, choice) : 0;
     if (info.may_pair) {
-      const unsigned load = (unsigned)wave_last(wave_inclusive_scan(have > 0 ? (int)launch_load_of(choice, (int)rows, N, K) : 0));
+      const unsigned load = (unsigned)wave_last((int)wave_inclusive_scan(have > 0 ? launch_load_of(choice, (int)rows, N, K) : 0u));  // (unsigned: the upper half takes all 16 bits)
       if (lane == 0) sh.load[wave] = load;
     }
     const int large = have > 0 && K >= kLongK ? choice.large_tiles : 0;

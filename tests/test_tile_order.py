@@ -73,13 +73,11 @@ def test_when_segments_are_paired(lib, q, count, rows, n, k, pairs):
     assert (tab[:22] == tab2[:22]).all() and (tab[22:22 + 4 * tab[0]] == tab2[22:22 + 4 * tab[0]]).all()
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("q,rows,n,k", [(W8, 192, 2816, 2048), (W4, 185, 28672, 4096), (FP, 150, 2048, 1408)])
-def test_device_planner_makes_the_same_pairs(lib, q, rows, n, k):
+def _device_plan_is_the_hosts(lib, q, counts, n, k):
+    """Entries and phases of a block as the device planner leaves them against the host's; the host's tables."""
     from mxmoe_amd import _lib
 
-    e = 8 if n == 28672 else 60
-    counts = [(rows, rows + 1, rows - 1, 0, 7, 128)[i % 6] for i in range(e)]
+    e = len(counts)
     desc = (_lib.BlockDesc * e)(*[_lib.BlockDesc(q[0], q[1], q[2], int(q[3]), (C.c_uint8 * 3)(), n, k, 0, 0)] * e)
     kid = lib.mxmoe_plan_select_kernel(-1, desc, e)
     d_desc = torch.frombuffer(bytearray(bytes(desc)), dtype=torch.uint8).cuda()
@@ -89,12 +87,27 @@ def test_device_planner_makes_the_same_pairs(lib, q, rows, n, k):
     _lib.check(lib, lib.mxmoe_plan_block(kid, recv.data_ptr(), e, 0, d_desc.data_ptr(), desc, some.data_ptr(), some.data_ptr(), some.data_ptr(), plan.data_ptr(),
                                          torch.cuda.current_stream().cuda_stream))
     tab, _ = _launch(lib, [(m, n, k, q) for m in counts], kid)
-    assert _pairs(tab)
     ne, tiles, nph, grid = tab[:4]
     hdr = plan.cpu().numpy()[:4096].view(np.int32)[14:]
     assert list(hdr[:4]) == [0, ne, tiles, nph] and grid <= lib.mxmoe_plan_grid_bound(kid, desc, e, sum(counts), 0)
     assert np.array_equal(hdr[4:5 + nph], tab[4:5 + nph]) and np.array_equal(hdr[13:14 + nph], tab[13:14 + nph])
     assert np.array_equal(hdr[23:23 + 4 * ne], tab[22:22 + 4 * ne].astype(np.int32))
+    return tab
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("q,rows,n,k", [(W8, 192, 2816, 2048), (W4, 185, 28672, 4096), (FP, 150, 2048, 1408)])
+def test_device_planner_makes_the_same_pairs(lib, q, rows, n, k):
+    e = 8 if n == 28672 else 60
+    counts = [(rows, rows + 1, rows - 1, 0, 7, 128)[i % 6] for i in range(e)]
+    assert _pairs(_device_plan_is_the_hosts(lib, q, counts, n, k))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("q,k", [(W8, 128), (W4, 4096)])
+def test_device_planner_with_as_many_tiles_as_its_sums_hold(lib, q, k):
+    """64 problems of one wave, each with more tiles and columns than are told apart: the packed sum passes 2^31."""
+    assert len(_pairs(_device_plan_is_the_hosts(lib, q, [1160] * 64, 28672 * 2, k))) == 64
 
 
 @pytest.mark.parametrize("kernel,tiles", [("groupgemm_hz_fused_wxax", 8), ("groupgemm_hz_fused_wxax_b6", 5), ("groupgemm_hz_fused_all_b6", 5)])
