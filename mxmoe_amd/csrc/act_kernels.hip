@@ -227,7 +227,8 @@ typedef unsigned v4u __attribute__((ext_vector_type(4)));
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
 
 // the eight codes of a chunk: v / scale rounded to fp16, clamped to +-7, rounded to the nearest integer (ties to even)
-__device__ __forceinline__ v8h bf6_chunk_codes(const v8h& h, const ScaleDiv& div) {
+template <class Chunk>
+__device__ __forceinline__ v8h bf6_chunk_codes(const Chunk& h, const ScaleDiv& div) {
   v8h o;
 #pragma unroll
   for (int j = 0; j < 8; ++j) o[j] = (_Float16)rintf(fminf(fmaxf(round_h(div((float)h[j])), -7.0f), 7.0f));
@@ -267,8 +268,8 @@ __device__ __forceinline__ int xcd_row_group(int wg) { return (wg & ~63) | ((wg 
 // What every kernel of one row per workgroup does with a finished row, chunk tid + NT i of it in h[i]: fp16 copy or symmetric quantisation.  `red`: one slot per
 // wave; `codes`: LDS for the row as fp16 (tag 4).  Passes barriers only where `tag` is
 // neither 0 nor 3.
-template <int MAXC, int NT, bool EXT>
-__device__ __forceinline__ void store_row(const v8h (&h)[MAXC], int n, int tag, long lrow, long inp_off, long scale_off, uint8_t* inp_store, _Float16* scale_store,
+template <int MAXC, int NT, bool EXT, class Chunk>
+__device__ __forceinline__ void store_row(const Chunk (&h)[MAXC], int n, int tag, long lrow, long inp_off, long scale_off, uint8_t* inp_store, _Float16* scale_store,
                                           float* red, uint8_t* codes) {
   const int tid = threadIdx.x, nchunks = n >> 3;
   if (tag == 0) {
@@ -277,7 +278,7 @@ __device__ __forceinline__ void store_row(const v8h (&h)[MAXC], int n, int tag, 
     for (int i = 0; i < MAXC; ++i) {
       const int c = tid + i * NT;
       if (c < nchunks) {
-        *reinterpret_cast<v8h*>(out + c * 8) = h[i];
+        *reinterpret_cast<v8h*>(out + c * 8) = as_half(h[i]);
       }
     }
     return;
@@ -292,22 +293,22 @@ __device__ __forceinline__ void store_row(const v8h (&h)[MAXC], int n, int tag, 
     for (int i = 0; i < MAXC; ++i) {
       const int c = tid + i * NT;
       const bool live = c < nchunks;  // whole lane groups are live or not: n is a multiple of 128
-      HalfMax gmax;
+      AbsMax<Chunk> gmax;
       if (live) gmax.add(h[i]);
       float scale = round_h(row16_max_abs(gmax.get()) / 7.0f);
       if (scale == 0.0f) scale = 1.0f;
       if (live) {
         if ((c & 15) == 0) sout[c >> 4] = (_Float16)scale;
-        *reinterpret_cast<unsigned*>(out + c * 4) = HalfDiv(scale).int4(h[i]);
+        *reinterpret_cast<unsigned*>(out + c * 4) = HalfDiv(scale).int4(as_half(h[i]));
       }
     }
     return;
   }
-  HalfMax half_max;
+  AbsMax<Chunk> row_max;
 #pragma unroll
   for (int i = 0; i < MAXC; ++i)
-    if (tid + i * NT < nchunks) half_max.add(h[i]);
-  float amax = wave_max_abs(half_max.get());
+    if (tid + i * NT < nchunks) row_max.add(h[i]);
+  float amax = wave_max_abs(row_max.get());
   __syncthreads();
   if ((tid & 63) == 0) red[tid >> 6] = amax;
   __syncthreads();
@@ -339,8 +340,8 @@ __device__ __forceinline__ void store_row(const v8h (&h)[MAXC], int n, int tag, 
         *reinterpret_cast<uint2*>(out + c * 8) = fp8_chunk_codes(h[i], div);
         continue;
       }
-      if (tag == 1) *reinterpret_cast<uint2*>(out + c * 8) = half.int8(h[i]);
-      else *reinterpret_cast<unsigned*>(out + c * 4) = half.int4(h[i]);
+      if (tag == 1) *reinterpret_cast<uint2*>(out + c * 8) = half.int8(as_half(h[i]));
+      else *reinterpret_cast<unsigned*>(out + c * 4) = half.int4(as_half(h[i]));
     }
   }
 }
@@ -618,12 +619,16 @@ __device__ __forceinline__ void row_quant_body(const RowArgs& a, const int wg, c
       }
     }
 
-    v8h h[MAXC];
+    // With the operand variants the row stays in fp32, whose codes are formed from that: packed halves, and the fp32 values that the compiler keeps beside them
+    // for those codes, take 143 registers instead of 122 (three chunks a thread), and 8192 rows of 10 240 values with the SiLU 148 us instead of 105 (fp8; bf6 184 and 131).
+    if constexpr (EXT) {
+      store_row<MAXC, NT, EXT>(v, n, tag, lrow, inp_off, scale_off, a.inp_store, a.scale_store, red, reinterpret_cast<uint8_t*>(x));
+    } else {
+      v8h h[MAXC];
 #pragma unroll
-    for (int i = 0; i < MAXC; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) h[i][j] = (_Float16)v[i][j];
-    store_row<MAXC, NT, EXT>(h, n, tag, lrow, inp_off, scale_off, a.inp_store, a.scale_store, red, reinterpret_cast<uint8_t*>(x));
+      for (int i = 0; i < MAXC; ++i) h[i] = as_half(v[i]);
+      store_row<MAXC, NT, EXT>(h, n, tag, lrow, inp_off, scale_off, a.inp_store, a.scale_store, red, reinterpret_cast<uint8_t*>(x));
+    }
   }
 }
 

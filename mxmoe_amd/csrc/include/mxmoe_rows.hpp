@@ -45,6 +45,25 @@ struct HalfMax {
   }
   __device__ __forceinline__ float get() const { return (float)__builtin_bit_cast(_Float16, (unsigned short)m); }
 };
+// The same of a row held in fp32.
+struct FloatMax {
+  float m = 0.0f;
+  __device__ __forceinline__ void add(const float (&v)[8]) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf(v[j]));
+  }
+  __device__ __forceinline__ float get() const { return m; }
+};
+template <class Chunk>
+using AbsMax = std::conditional_t<std::is_same_v<Chunk, v8h>, HalfMax, FloatMax>;
+// A chunk as packed halves: of a row that is held so, or of one held in fp32 (values that are fp16 numbers).
+__device__ __forceinline__ const v8h& as_half(const v8h& h) { return h; }
+__device__ __forceinline__ v8h as_half(const float (&v)[8]) {
+  v8h h;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) h[j] = (_Float16)v[j];
+  return h;
+}
 // A row that goes on as it was read: signalling NaNs become quiet ones, as a trip through fp32 makes them.
 __device__ __forceinline__ v8h quiet(const v8h& h) { return __builtin_elementwise_canonicalize(h); }
 
@@ -239,7 +258,8 @@ __device__ __forceinline__ float row16_max_abs(float v) { return __uint_as_float
 // ---- tag 5: per-token fp8 (OCP e4m3) codes for the kernels whose w8a8 tiles run the fp8 matrix instruction.  scale = max|x| / 448
 // (the largest e4m3 number) in fp16 like the integer scales; code = e4m3(clamp(fp16(x / scale), +-448)), round to nearest even; rows
 // are stored like int8 rows, one byte per value.
-__device__ __forceinline__ uint2 fp8_chunk_codes(const v8h& h, const ScaleDiv& div) {
+template <class Chunk>
+__device__ __forceinline__ uint2 fp8_chunk_codes(const Chunk& h, const ScaleDiv& div) {
   float r[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) r[j] = fminf(fmaxf(round_h(div((float)h[j])), -448.0f), 448.0f);
