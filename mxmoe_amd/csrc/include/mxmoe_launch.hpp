@@ -154,11 +154,8 @@ __device__ __forceinline__ void with_branch(std::integral_constant<int, I>, int 
 // tile keeps more than 128 accumulator registers per lane, which needs the full 512-register budget of a lone wave.
 // A kernel made only of tiles that ask for more waves (the few-token weight-only tiles: latency-bound streams that gain from every
 // further workgroup in flight) is compiled for the smallest number any of its tiles asks for.
-constexpr int min_of(int a) { return a; }
-template <class... R>
-constexpr int min_of(int a, R... r) { return a < min_of(r...) ? a : min_of(r...); }
 template <class... Tiles>
-constexpr int kWavesPerSimd = ((Tiles::kAccRegs > 128) || ...) ? 1 : min_of(Tiles::kWavesWanted...);
+constexpr int kWavesPerSimd = ((Tiles::kAccRegs > 128) || ...) ? 1 : std::min({Tiles::kWavesWanted...});
 
 // Tables are read through the constant address space: what a workgroup reads from them is the same for all lanes and is not
 // written while the kernel runs (a planned launch's tables were written by the planning kernel before it), so every read is a
@@ -477,6 +474,9 @@ struct PlanInfo {
   // Narrow integer tiles among them; and, where a launch is planned with them, whether it has few blocks of channels (kPoleBlocks).
   int narrow, few_blocks;
   int may_pair;  // a format that has pairs (pairs_pay) comes in several shapes, and it is no kernel for few rows
+  // A 128 x 256 tile that has a 128 x 128 one for launches of few tiles (kSlimTiles): branches, and whether there is such a pair of shapes.  The slim one stands behind
+  // the formats' branches in b: problems are planned without it.
+  int wide, slim, has_slim;
   uint8_t order[kMaxBranches];  // positions in b, most expensive tile first (branch_cost); ties keep the registration order
   uint8_t fmt_start[kNumFmts + 4];
   // by format, in registration order inside a format: those of format f are b[fmt_start[f]] .. b[fmt_start[f + 1] - 1], and the planners
@@ -526,6 +526,16 @@ __host__ __device__ inline bool pairs_pay(int f, int launch_tiles, int launch_co
   return launch_tiles > kPairTiles && (f == (int)Fmt::W8A8 || f == (int)Fmt::FP16 || (f == (int)Fmt::W4A4 && launch_cols > kPairColsInt4));
 }
 
+// Large tiles of a launch's problems of one length (the smallest K; any longer one) up to which the 128 x 128 tile of 8-bit weights runs in the place of the 128 x 256
+// one: twice as many find a CU each, and one takes 0.8 of the time; with more, what counts is the work, of which the wide tile does twice as much in 1.5 times the
+// time.  us, slim / wide, weights from memory, by wide tiles: N = 2048, K = 1408 96 rows 18.3 / 24.8 (8), 25.4 / 28.7 (128), 36.2 / 32.7 (256); N = 4096, K = 4096 96 rows
+// 44.7 / 59.4 (16), 58.3 / 65.3 (128), 89.4 / 81.0 (256), 192 rows 57.3 / 63.7 (128), 384 rows 78.8 / 68.1 (192); K = 14 336 96 rows 185 / 206 (64), 214 / 225 (128), 292 / 272 (256);
+// N = 2816, K = 2048 384 rows 29.8 / 34.8 (66), 37.4 / 36.2 (132).  A wide tile of up to 64 rows runs half its loop: there the slim one is ahead only in launches of
+// few tiles of few steps in K (tiles times K up to kSlimWorkHalf): 33 rows, K = 1408 18.3 / 19.5 (8), 19.9 / 19.6 (32); K = 2048 24.7 / 25.6 (11), 25.2 / 26.1 (44), 30.3 / 29.6 (88);
+// K = 4096 44.0 / 45.4 (16), 51.4 / 48.4 (32), 54.1 / 52.2 (64); K = 14 336 181 / 171 (16).  Few tiles of one length beside many of another: the longer ones start
+// first and end last, the shorter ones fill the end, so that what counts is again the time of one (wide everywhere -> counted apart, N = 2048: 60 problems of 130 rows, K = 1408, and
+// one of 2000, K = 5632 228 -> 146; 30 of 200 rows, K = 2048, and 8 of K = 4096 158 -> 118; 30 of K = 4096 and 8 of K = 2048 166 -> 148).
+constexpr int kSlimTiles = 128, kSlimWorkHalf = 48 * 2048;
 // The choice of tile shapes for an M x N problem, as far as it does not depend on the rest of the launch.
 struct PlanPick {
   int branch = -1, bm = 0, tiles = 0, bm_log2 = 0, bn_log2 = 0;
@@ -545,10 +555,12 @@ struct PlanChoice {
   PlanPick unit, whole;  // cheapest per row of the problem; cheapest for all of it (cost of a block run with one shape = row tiles * column tiles * tile_cost)
   int full = 0;          // rows that fill whole tiles of `unit`
   double full_cost = 0;
-  // Tiles in the largest shape, what a problem of long K adds to its launch's `long_tiles` (up to kLongTiles: more makes no difference), or 0
+  // Tiles in the largest shape, what a problem adds to its launch's large tiles and one of long K to its `long_tiles` (clamped where more makes no difference), or 0
   // when it takes a shorter shape anyway or there is no other.
   int large_tiles = 0;
 };
+
+constexpr int kLargeTilesTop = (kSlimTiles > kLongTiles ? kSlimTiles : kLongTiles) + 1;
 
 // What a problem adds to its launch's `launch_tiles` (upper half) and `launch_cols` (lower half).  Clamped where more makes no difference: the sums over a wave's
 // problems stay within 16 bits each.
@@ -578,7 +590,7 @@ __host__ __device__ inline int plan_choose(const PlanInfo& k, int f, int M, int 
       c.full_cost = (double)(M >> b.bm_log2) * tn * b.cost;
     }
   }
-  if (hi - lo > 1 && (c.full > 0 || c.whole.branch == c.unit.branch)) c.large_tiles = c.whole.tiles < kLongTiles ? c.whole.tiles : kLongTiles;
+  if (hi - lo > 1 && (c.full > 0 || c.whole.branch == c.unit.branch)) c.large_tiles = c.whole.tiles < kLargeTilesTop ? c.whole.tiles : kLargeTilesTop;
   return 1;
 }
 
@@ -636,6 +648,16 @@ __host__ __device__ inline int plan_split(const PlanInfo& k, int f, int M, int N
   return 2;
 }
 
+// The segments of an M x N x K problem in a launch with `launch_tiles` large tiles for problems of its length: where those are few, wide ones become slim ones (kSlimTiles).
+__host__ __device__ inline void take_slim_tiles(const PlanInfo& k, int launch_tiles, int M, int N, int K, Segment sg[2], int ns) {
+  if (!k.has_slim || launch_tiles > kSlimTiles || (M <= 64 && (long)launch_tiles * K > kSlimWorkHalf)) return;
+  for (int j = 0; j < ns; ++j)
+    if (sg[j].branch == k.wide) {
+      sg[j].branch = k.slim;
+      sg[j].tiles = tiles_over(sg[j].rows, 7) * tiles_over(N, 7);
+    }
+}
+
 // Both steps for a problem by itself: the number of segments (0 for M == 0), or -1 when the kernel has no tile for `f`.
 inline int plan_segments(const PlanInfo& k, int f, int M, int N, Segment out[2]) {
   PlanChoice c;
@@ -655,16 +677,25 @@ inline PlanInfo make_plan_info(const std::vector<BranchInfo>& branches) {
     while ((1 << lg) < v) ++lg;
     return lg;
   };
+  for (int i = 0; i < k.nb; ++i)
+    for (int j = 0; j < k.nb; ++j)
+      if (branches[i].fmt == Fmt::W8A16 && branches[j].fmt == Fmt::W8A16 && branches[i].BM == 128 && branches[j].BM == 128 && branches[i].BN == 256 && branches[j].BN == 128) {
+        k.wide = i;
+        k.slim = j;
+        k.has_slim = 1;
+      }
   int at = 0;
+  auto add = [&](int i) {
+    const double cost = tile_cost(branches[i]);
+    k.b[at++] = PlanBranch{i, (int)branches[i].fmt, branches[i].BM, branches[i].BN, log2_of(branches[i].BM), log2_of(branches[i].BN), cost, cost / branches[i].BM};
+  };
   for (int f = 0; f < kNumFmts; ++f) {
     k.fmt_start[f] = (uint8_t)at;
     for (int i = 0; i < k.nb; ++i)
-      if ((int)branches[i].fmt == f) {
-        const double cost = tile_cost(branches[i]);
-        k.b[at++] = PlanBranch{i, f, branches[i].BM, branches[i].BN, log2_of(branches[i].BM), log2_of(branches[i].BN), cost, cost / branches[i].BM};
-      }
+      if ((int)branches[i].fmt == f && !(k.has_slim && i == k.slim)) add(i);
   }
   k.fmt_start[kNumFmts] = (uint8_t)at;
+  if (k.has_slim) add(k.slim);
   std::vector<int> order(k.nb);
   for (int i = 0; i < k.nb; ++i) order[i] = i;
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return branch_cost(branches[x]) > branch_cost(branches[y]); });
@@ -933,11 +964,12 @@ inline bool shape_ok(const BranchInfo& bi, const mxmoe_dim3& sz) {
   return sz.z != 0 && sz.z % bi.k_multiple == 0 && (int)sz.z >= bi.k_min && sz.y % 8 == 0 && !(wo && sz.y % 16 != 0);
 }
 
-// What the planning of one launch's problems has in common: its smallest K, its tiles (where it may have pairs), the large tiles of its long problems, whether it has
+// What the planning of one launch's problems has in common: its smallest K, its tiles (where it may have pairs), its large tiles and those of its long problems, whether it has
 // few blocks; and what was chosen for each problem on the way, so that the tables do not choose again.  Problems without rows
 // have no part in it: a list plans the same with and without them (the device planner sees every expert, the operators leave out empty ones).
 struct LaunchScope {
   int kmin = 0x7fffffff, long_tiles = 0, launch_tiles = 0, launch_cols = 0;
+  int tall_tiles[2] = {0, 0};  // of the problems of the smallest K, of the others
   bool few_blocks = false;
   int8_t have[kMaxProblems];          // plan_choose's answer for each problem (-1 too where its format is not supported)
   union {
@@ -946,7 +978,9 @@ struct LaunchScope {
   LaunchScope() {}  // (leaves the arrays alone)
   // A problem of `M` rows, N and K of `sz`, whose shapes are `c`: plan_split in this launch.
   int split(const PlanInfo& pi, int f, int M, const mxmoe_dim3& sz, const PlanChoice& c, Segment out[2]) const {
-    return plan_split(pi, f, M, (int)sz.y, c, runs_long((int)sz.z, kmin) ? long_tiles : few_blocks && integer_sums(f) ? c.large_tiles : 0, out);
+    const int ns = plan_split(pi, f, M, (int)sz.y, c, runs_long((int)sz.z, kmin) ? long_tiles : few_blocks && integer_sums(f) ? c.large_tiles : 0, out);
+    take_slim_tiles(pi, tall_tiles[(int)sz.z > kmin], M, (int)sz.y, (int)sz.z, out, ns);
+    return ns;
   }
   // The number of segments of problem i (0 without rows), or -1 when the kernel has no tile for it.
   int segments(const PlanInfo& pi, int i, const mxmoe_dim3& sz, int f, Segment out[2]) const {
@@ -955,7 +989,7 @@ struct LaunchScope {
 };
 inline void launch_scope(const PlanInfo& pi, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int n, LaunchScope& s) {
   s.kmin = 0x7fffffff;
-  s.long_tiles = s.launch_tiles = s.launch_cols = 0;
+  s.long_tiles = s.launch_tiles = s.launch_cols = s.tall_tiles[0] = s.tall_tiles[1] = 0;
   long blocks = 0;
   for (int i = 0; i < n; ++i)
     if (h_sizes[i].x != 0) {
@@ -974,6 +1008,7 @@ inline void launch_scope(const PlanInfo& pi, const mxmoe_dim3* h_sizes, const mx
       s.launch_tiles += (int)(load >> 16);
       s.launch_cols += (int)(load & 0xFFFF);
     }
+    s.tall_tiles[(int)h_sizes[i].z > s.kmin] += c.large_tiles;
     if (runs_long((int)h_sizes[i].z, s.kmin)) s.long_tiles = std::min(s.long_tiles + c.large_tiles, kLongTiles);
   }
 }

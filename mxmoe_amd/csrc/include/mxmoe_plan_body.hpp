@@ -60,8 +60,13 @@ struct PlanParams {
 inline PlanInfo plan_info_of_block(const FusedKernel& k, const mxmoe_block_desc* h_desc, int et) {
   PlanInfo info = plan_of(k);
   long blocks = 0;
-  for (int i = 0; i < et; ++i) blocks += (h_desc[i].N + 255) / 256;
+  bool w8a16 = false;
+  for (int i = 0; i < et; ++i) {
+    blocks += (h_desc[i].N + 255) / 256;
+    w8a16 = w8a16 || fmt_of(h_desc[i].q) == (int)Fmt::W8A16;
+  }
   info.few_blocks = info.narrow && blocks <= kPoleBlocks;
+  if (!w8a16) info.has_slim = 0;  // (nothing to look for)
   return info;
 }
 
@@ -93,6 +98,7 @@ struct PlanShared {
   int cnt_long[kMaxBranches][2], til_long[kMaxBranches][2];  // ... of which belong to long-K problems
   int kmin[2];
   unsigned load[2];                                  // launch_load_of, per wave
+  int tall_tiles[2], tall_tiles_kmin[2];             // large tiles of the wave's problems; of those with K = kmin
   int long_tiles[2], long_tiles_kmin[2];             // large tiles of the wave's problems with K >= kLongK; of those with K = kmin
   // the kernel's branch table, from the kernel arguments: the planning functions walk it entry by entry, and each step of such a
   // walk through the argument segment costs a trip to the scalar cache
@@ -198,6 +204,14 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
       const unsigned load = (unsigned)wave_last((int)wave_inclusive_scan(have > 0 ? launch_load_of(choice, (int)rows, N, K) : 0u));  // (unsigned: the upper half takes all 16 bits)
       if (lane == 0) sh.load[wave] = load;
     }
+    if (info.has_slim) {
+      const int tall = have > 0 ? choice.large_tiles : 0;
+      const int all = wave_last(wave_inclusive_scan(tall)), at_km = wave_last(wave_inclusive_scan(K == km ? tall : 0));
+      if (lane == 0) {
+        sh.tall_tiles[wave] = all;
+        sh.tall_tiles_kmin[wave] = at_km;
+      }
+    }
     const int large = have > 0 && K >= kLongK ? choice.large_tiles : 0;
     if (__ballot(large > 0) != 0) {
       const int all = wave_last(wave_inclusive_scan(large)), at_km = wave_last(wave_inclusive_scan(K == km ? large : 0));
@@ -215,6 +229,10 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
   const int long_tiles = sh.long_tiles[0] - (sh.kmin[0] == kmin ? sh.long_tiles_kmin[0] : 0) + sh.long_tiles[1] - (sh.kmin[1] == kmin ? sh.long_tiles_kmin[1] : 0);
   Segment sg[2];
   const int ns = have > 0 ? plan_split(info, fmt, (int)rows, N, choice, runs_long(K, kmin) ? min(long_tiles, kLongTiles) : info.few_blocks && integer_sums(fmt) ? choice.large_tiles : 0, sg) : 0;
+  if (info.has_slim) {
+    const int at_kmin = (sh.kmin[0] == kmin ? sh.tall_tiles_kmin[0] : 0) + (sh.kmin[1] == kmin ? sh.tall_tiles_kmin[1] : 0);
+    take_slim_tiles(info, long_k ? sh.tall_tiles[0] + sh.tall_tiles[1] - at_kmin : at_kmin, (int)rows, N, K, sg, ns);
+  }
   const PlanBranch& my_branch = info.b[info.order[min(lane, kMaxBranches - 1)]];  // lane r: the branch of rank r
   const int my_order = my_branch.index;
   unsigned pair = 0;  // the second segment goes beside the first: one item of two entries

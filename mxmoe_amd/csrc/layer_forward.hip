@@ -397,6 +397,7 @@ int mxmoe_layer_create(const mxmoe_layer_desc* d, void** handle) {
     for (const BranchInfo& b : registry()[kid].branches)
       if (!is_weight_only(b.fmt)) low = std::min(low, b.BM);
     if ((long)d->num_tokens * d->topk <= low) p.info.may_pair = 0;
+    if ((long)d->num_tokens * d->topk <= 32) p.info.has_slim = 0;  // (nor for 128-row tiles)
     return kid;
   };
   f->d.kernel_gate_up = fill(f->pair.p[0], d->kernel_gate_up, d->d_gate_up, d->h_gate_up, d->act, d->plan_gate_up);

@@ -273,6 +273,7 @@ int mxmoe_plan_grid_bound(int kernel_id, const mxmoe_block_desc* h_desc, int num
   for (int i = 0; i < nonempty; ++i) by_first += firsts[i];
   const long by_rows = extras + (long)(per_row * routed_rows_max) + 1;
   long bound = shared_tiles + std::min(by_first, by_rows);
+  if (pi.has_slim) bound += 2 * kSlimTiles;  // slim tiles: twice as many as the wide ones, which are at most that many then, of either length
   bound += (long)kNumXcd * (kMaxPhases + 1);  // every phase is padded to a multiple of the XCD count
   bound = (bound + kNumXcd - 1) / kNumXcd * kNumXcd;
   if (bound > (1l << 30)) {

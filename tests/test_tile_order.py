@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-W4, W8, FP, WO = (4, 4, -1, True), (8, 8, -1, True), (16, 16, -1, True), (16, 4, 128, False)
+W4, W8, FP, WO, WO8 = (4, 4, -1, True), (8, 8, -1, True), (16, 16, -1, True), (16, 4, 128, False), (16, 8, 128, False)
 
 
 def _launch(lib, probs, kid=-1):
@@ -36,6 +36,7 @@ def _pairs(tab):
     (W4, 300, 28672, 4096), (W8, 1060, 28672, 4096),                  # activations of several groups of row tiles: the second segment goes with the last
     (W8, 160, 2824, 2048),                                            # the last column tile is 8 wide
     (WO, 140, 2816, 2048), (W4, 144, 2816, 2048),                     # two segments, no pairs
+    (WO8, 140, 272, 2048), (WO8, 300, 16, 1408), (WO8, 140, 2816, 2048),  # slim tiles, wide tiles
 ])
 def test_every_output_is_computed_once(lib, q, rows, n, k):
     """Every element of every output in exactly one workgroup's tile, for problems of two row segments next to empty and small ones."""
@@ -43,7 +44,7 @@ def test_every_output_is_computed_once(lib, q, rows, n, k):
     tab, area = _launch(lib, probs)
     assert bool(_pairs(tab)) == (q is W8 or q is FP or n == 28672)
     area = area[area[:, 0] >= 0]
-    for p, (m, *_rest) in enumerate(probs[:6]):
+    for p, (m, *_rest) in enumerate(probs):
         cover = np.zeros((m, n), np.int8)
         for _, r0, r1, c0, c1 in area[area[:, 0] == p]:
             cover[r0:r1, c0:c1] += 1
@@ -93,6 +94,38 @@ def _device_plan_is_the_hosts(lib, q, counts, n, k):
     assert np.array_equal(hdr[4:5 + nph], tab[4:5 + nph]) and np.array_equal(hdr[13:14 + nph], tab[13:14 + nph])
     assert np.array_equal(hdr[23:23 + 4 * ne], tab[22:22 + 4 * ne].astype(np.int32))
     return tab
+
+
+# 8-bit weights, 128 rows: the 128 x 128 tile where a launch's 128 x 256 ones are up to 128, for up to 64 rows where they times K are up to 48 * 2048
+@pytest.mark.parametrize("count,rows,n,k,bn", [
+    (8, 96, 4096, 14336, 128), (8, 128, 4096, 4096, 128), (4, 192, 4096, 4096, 128), (2, 65, 4096, 4096, 128),          # 128 wide tiles and fewer
+    (1, 128, 28672, 4096, 128), (1, 129, 28672, 4096, 256), (9, 96, 4096, 14336, 256), (1, 1100, 4096, 4096, 256),       # 112, 224, 144, 144
+    (4, 64, 2816, 2048, 128), (5, 64, 2816, 2048, 256), (1, 33, 4096, 4096, 128), (2, 64, 4096, 4096, 256), (2, 65, 4096, 4096, 128), (1, 64, 4096, 14336, 256),
+])
+@pytest.mark.parametrize("kernel", ["groupgemm_hz_fused_wo8", "groupgemm_hz_fused_all"])
+def test_width_of_the_8_bit_weight_only_tile(lib, kernel, count, rows, n, k, bn):
+    kid = lib.mxmoe_find_kernel(kernel.encode())
+
+    def shapes(probs):
+        tab, _ = _launch(lib, probs, kid)
+        info, seen = (C.c_int32 * 8)(), {}
+        for first, row0, m, pb in tab[22:22 + 4 * tab[0]].reshape(-1, 4):
+            assert lib.mxmoe_kernel_branch(kid, int(pb) >> 16 & 31, info) == 0
+            seen.setdefault(int(pb) & 0xFFFF, []).append((int(m), info[1], info[2]))
+        return seen
+
+    for tiles in shapes([(rows, n, k, WO8)] * count + [(0, n, k, WO8), (7, 256, k, WO8)]).values():
+        assert all(t[1:] == (128, bn) if t[0] > 32 else t[1:] != (128, 384 - bn) for t in tiles), tiles
+    # other formats' large tiles count too, those of problems of another K do not
+    if kernel.endswith("all") and rows <= 128:
+        assert shapes([(rows, n, k, WO8), (128, 33024, k, WO)])[0] == [(rows, 128, 256)]
+        assert shapes([(rows, n, k, WO8)] * count + [(7, 256, k, WO8), (128, 33024, 2 * k, WO)])[0] == [(rows, 128, bn)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count,rows,n,k", [(8, 192, 2048, 1408), (16, 192, 2048, 1408), (17, 192, 2048, 1408), (60, 150, 2048, 1408), (4, 64, 2816, 2048), (5, 64, 2816, 2048), (1, 2000, 2048, 1408)])
+def test_device_planner_takes_the_same_width(lib, count, rows, n, k):
+    _device_plan_is_the_hosts(lib, WO8, [(rows, 0, 5)[i % 3] for i in range(count * 3)][:119], n, k)
 
 
 @pytest.mark.gpu
