@@ -698,7 +698,7 @@ __global__ void __launch_bounds__(256) row_quant_wave_kernel(const RowArgs a) {
         gmax.add(h[i]);
         float scale = round_h(row16_max_abs(gmax.get()) / 7.0f);
         if (scale == 0.0f) scale = 1.0f;
-          if ((c & 15) == 0) sout[c >> 4] = (_Float16)scale;
+        if ((c & 15) == 0) sout[c >> 4] = (_Float16)scale;
         *reinterpret_cast<unsigned*>(out + c * 4) = HalfDiv(scale).int4(h[i]);
       }
       continue;
@@ -1103,7 +1103,7 @@ __device__ __forceinline__ void row_quant_dense_body(const RowArgs& a, const int
         gmax.add(h[i]);
         float scale = round_h(row16_max_abs(gmax.get()) / 7.0f);
         if (scale == 0.0f) scale = 1.0f;
-          if (live) {
+        if (live) {
           if ((c & 15) == 0) sout[c >> 4] = (_Float16)scale;
           *reinterpret_cast<unsigned*>(out + c * 4) = HalfDiv(scale).int4(h[i]);
         }
@@ -1616,7 +1616,7 @@ __global__ void __launch_bounds__(512, 6) row_quant_wide_kernel(const RowArgs a)
         gmax.add(h[i]);
         float scale = round_h(row16_max_abs(gmax.get()) / 7.0f);
         if (scale == 0.0f) scale = 1.0f;
-          if ((c & 15) == 0) sout[c >> 4] = (_Float16)scale;
+        if ((c & 15) == 0) sout[c >> 4] = (_Float16)scale;
         *reinterpret_cast<unsigned*>(out + c * 4) = HalfDiv(scale).int4(h[i]);
       }
       continue;
@@ -1666,9 +1666,11 @@ __global__ void __launch_bounds__(512, 6) row_quant_wide_kernel(const RowArgs a)
 }
 
 constexpr int kSplitSharedRows = 512;
-// Shared rows up to which row_quant_pair_kernel takes them (us, 2304 in it / 2305 in launches after one another, six routed rows of 1408 values each: 2 x 1408 65.5 / 65.3,
-// 4 x 1408 71.0 / 80.2; side by side beyond it has been timed with older shared-row code only).
-constexpr int kPairSharedRows = 2304;
+// Shared rows up to which row_quant_pair_kernel takes them, of finished rows and with the SiLU.  Routed rows of 1408 values, 2, 4, 6, 8 a token; launches after one another /
+// side by side, us: shared rows of 2816 values, 3000 of them 36.3 / 32.7, 42.9 / 41.2, 49.8 / 48.2, 56.4 / 55.6, 4096 44.0 / 41.5, 52.3 / 51.1, 61.8 / 60.2, 71.1 / 72.1, 8192
+// 73.3 / 77.0, 94.9 / 101, 111 / 117, 134 / 139; of 5632 values, 4096 57.7 / 56.7, 67.2 / 59.5, 76.4 / 72.1, 85.4 / 84.8, 8192 102 / 107, 121 / 113, 147 / 142, 163 / 163.  With the SiLU: 2816 values, 2049
+// 38.1 / 36.8, 45.7 / 42.1, 51.2 / 51.4, 59.7 / 61.1, 4096 56.2 / 58.7, 72.2 / 73.4, 87.2 / 93.7, 106 / 114; 5632 values, 4096 78.9 / 69.5, 94.9 / 89.9, 112 / 103, 133 / 124.
+constexpr int kPairSharedRows = 4096, kPairSharedRowsSilu = 2304;
 
 static int make_plan(int n, int had_k, int had_f, bool rotate, RotPlan* p) {
   p->n = n;
@@ -1725,15 +1727,24 @@ static int launch_pair(const RowArgs& routed, const RowArgs& shared, bool dense,
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   // (dense_rows and block_rows: at most 64 KiB of LDS)
-  // (workgroups per CU: 2049 shared rows of 2816 values and 12 294 routed ones of 1408, us, shared + routed per CU, of which four are resident: 1 + 2 44.2, 1 + 3 46.0,
-  // 2 + 2 42.6, 1.5 + 2.5 40.8, 2 + 3 43.7, 1 + 4 43.8.  With the SiLU three are: 1 + 2.)
+  // Workgroups per CU, shared + routed, of which four are resident, with the SiLU three.  By the shared rows' work (rows times values) over the routed rows', us:
+  // 2049 shared rows, one length    1 + 2    1 + 3    1.5 + 2    1.5 + 2.5    2 + 2    2 + 3    2.5 + 1.5    with the SiLU:  1 + 2    1.5 + 2.5    2 + 2    2 + 3
+  //   2   (5632, 2 x 1408)           50.2     51.0     38.7       38.5         32.0     31.6     30.9                          56.0     45.5         41.6     39.1
+  //   1   (2816, 2 x 1408)           38.7     39.1     30.3       30.2         25.4     25.4     25.4                          44.1     36.5         36.8     34.6
+  //   1   (5632, 4 x 1408)           50.2     50.8     39.1       39.1         35.1     34.8     36.3                          56.0     53.1         51.0     48.4
+  //   2/3 (5632, 6 x 1408)           50.1     50.5     45.0       41.3         41.1     42.8     43.7                          56.8     62.0         60.8     61.4
+  //   1/2 (2816, 4 x 1408)           37.1     37.6     31.8       28.8         29.3     30.2     30.2                          42.1     45.1         44.8     43.2
+  //   1/3 (2816, 6 x 1408)           36.7     40.1     38.4       35.3         35.4     39.0     40.1                          51.4     57.9         54.7     52.4
+  //   1/4 (2816, 8 x 1408)           41.3     38.8     44.7       39.2         42.5     44.0     48.3                          61.1     61.2         64.4     58.7
+  // (600 and 1200 shared rows alike: at a ratio of one 15.6 and 23.1 with 1 + 2, 11.9 and 20.1 with 1.5 + 2.5, 12.1 and 16.1 with 2 + 2.)
   const int lds = std::max(BlockRows(shared.plan).lds(), dense ? dense_lds(routed.plan.kb) : BlockRows(routed.plan).lds());
-  const int shared_wgs = std::min(shared.rows, SILU ? cus : cus * 3 / 2) + 63 & ~63;
+  const bool even = (long)shared.rows * shared.plan.n >= (long)routed.rows * routed.plan.n;
+  const int shared_wgs = std::min(shared.rows, even ? cus * 2 : SILU ? cus : cus * 3 / 2) + 63 & ~63;
   if (!dense) {
     hipLaunchKernelGGL((row_quant_few_kernel<kFewThreads, 2, SILU, EXT>), dim3(shared.rows + routed.rows), dim3(kFewThreads), lds, s, routed, shared, shared.rows);
     return rows_launched();
   }
-  const int routed_wgs = std::min((routed.rows + 3) / 4, SILU ? cus * 2 : cus * 5 / 2) + 63 & ~63;
+  const int routed_wgs = std::min((routed.rows + 3) / 4, even || SILU ? cus * 2 : cus * 5 / 2) + 63 & ~63;
   const dim3 grid(shared_wgs + routed_wgs);
   switch ((routed.plan.n / 8 + 63) / 64) {
     case 1: hipLaunchKernelGGL((row_quant_pair_kernel<1, SILU, EXT>), grid, dim3(256), lds, s, routed, shared, shared_wgs); break;
@@ -1755,12 +1766,12 @@ static int launch_rows_as(const RowArgs& a, int lds_bytes, hipStream_t s) {
     shared.R = 0;
     shared.rows = a.rows - a.R;
     shared.plan = a.plan_shared;
-    // Shared rows beside routed ones: up to 512, or 2304 of those that row_quant_block_kernel is fastest for in any number (us, one after the other -> side by
+    // Shared rows beside routed ones: up to 512, or kPairSharedRows of those that row_quant_block_kernel is fastest for in any number (us, one after the other -> side by
     // side: 2 x 480 values 512 tokens top-6 19.1 -> 13.0, 1024 24.0 -> 21.7; 2 x 224, 512 13.3 -> 10.9, 1024 16.8 -> 18.4).  One row of either kind per workgroup up
     // to 512 rows in all, 256 with the SiLU (routed rows one per wave -> per workgroup: finished rows inside a planned forward, 4 x 1408 values beside, 280 rows 10.9 -> 10.0,
     // 500 11.3 -> 10.1, 600 11.3 -> 11.7; 2 x 1408, 448 9.7 -> 9.2, 560 9.9 -> 11.3; with the SiLU, launches back to back, 4 x 1408 252 9.7 -> 8.9, 280 9.7 -> 9.8; 2 x 1408
     // 280 8.2 -> 9.4, 511 8.4 -> 9.6).  Short routed rows are below kSplitSharedRows best off in the general kernel (2 x 224, 32 tokens 6.1, side by side 6.8).
-    if (a.R > 0 && dense_rows(routed) && block_rows(shared) && shared.rows <= std::min(std::max(block_row_limit(shared.plan), 512), kPairSharedRows)) {
+    if (a.R > 0 && dense_rows(routed) && block_rows(shared) && shared.rows <= std::min(std::max(block_row_limit(shared.plan), 512), SILU ? kPairSharedRowsSilu : kPairSharedRows)) {
       const int limit = block_row_limit(routed.plan);  // (dense_rows: block_rows as well)
       const bool few = a.R <= limit && a.rows <= (SILU ? 256 : 512);
       if (few || limit > 0 || a.R >= kSplitSharedRows) return launch_pair<SILU, EXT>(routed, shared, !few, s);

@@ -119,6 +119,15 @@ def test_routed_and_shared_rows_of_two_lengths_in_one_launch(monkeypatch, inter,
     _check(cfg, layer)
 
 
+@pytest.mark.parametrize("tokens,topk,num_shared", [(300, 2, 2), (300, 3, 2), (300, 2, 4), (2305, 1, 2), (4096, 2, 2), (4096, 3, 2), (4097, 2, 2)])
+def test_short_forward_of_many_shared_rows_beside_routed_ones(tokens, topk, num_shared):
+    """Work of the shared rows below, at and above the routed rows', which decides how the launch is shared out; the last number of shared rows in one launch with routed ones."""
+    from mxmoe_amd import synth as S
+
+    cfg, layer = _layer(tokens, topk, [(S.W4A4, S.W8A8), (S.W8A8, S.W4A4), (S.W4A4, S.W4A4), (S.W8A8, S.W4A4), (S.W4A4, S.W8A8)], num_shared=num_shared)
+    _check(cfg, layer)
+
+
 @pytest.mark.parametrize("tokens", [50, 1100])
 def test_short_forward_of_the_most_experts_it_takes(tokens):
     """512 experts, the most LDS the head asks for, in workgroups of 256 and of 512 threads; five launches per block to plan."""
