@@ -651,8 +651,9 @@ __host__ __device__ inline int plan_split(const PlanInfo& k, int f, int M, int N
 // The segments of an M x N x K problem in a launch with `launch_tiles` large tiles for problems of its length: where those are few, wide ones become slim ones (kSlimTiles).
 __host__ __device__ inline void take_slim_tiles(const PlanInfo& k, int launch_tiles, int M, int N, int K, Segment sg[2], int ns) {
   if (!k.has_slim || launch_tiles > kSlimTiles || (M <= 64 && (long)launch_tiles * K > kSlimWorkHalf)) return;
-  for (int j = 0; j < ns; ++j)
-    if (sg[j].branch == k.wide) {
+#pragma unroll
+  for (int j = 0; j < 2; ++j)  // (unrolled: indexed by a loop, the segments would not stay in the planner's registers)
+    if (j < ns && sg[j].branch == k.wide) {
       sg[j].branch = k.slim;
       sg[j].tiles = tiles_over(sg[j].rows, 7) * tiles_over(N, 7);
     }
