@@ -78,6 +78,8 @@ static_assert(kMaxBranches <= 64, "one lane per branch");
 struct PlanPair {
   PlanParams p[2];
   int chunks;  // launches per block
+  // Whether either block's tile shapes hang on its launch's totals (plan_block_body's TOTALS).
+  bool totals() const { return p[0].info.may_pair || p[0].info.has_slim || p[1].info.may_pair || p[1].info.has_slim; }
 };
 
 // One workgroup of two waves per launch, thread e = expert e0 + e of the launch's chunk of experts [e0, e0 + kMaxProblems) (the shared
@@ -98,7 +100,7 @@ struct PlanShared {
   int cnt_long[kMaxBranches][2], til_long[kMaxBranches][2];  // ... of which belong to long-K problems
   int kmin[2];
   unsigned load[2];                                  // launch_load_of, per wave
-  int tall_tiles[2], tall_tiles_kmin[2];             // large tiles of the wave's problems; of those with K = kmin
+  unsigned tall[2];                                  // large tiles of the wave's problems with K = kmin (lower half), of the others (upper half)
   int long_tiles[2], long_tiles_kmin[2];             // large tiles of the wave's problems with K >= kLongK; of those with K = kmin
   // the kernel's branch table, from the kernel arguments: the planning functions walk it entry by entry, and each step of such a
   // walk through the argument segment costs a trip to the scalar cache
@@ -123,7 +125,10 @@ __device__ __forceinline__ mxmoe_block_desc plan_block_prepare(const PlanParams&
 // `recv`: the tokens-per-expert counts (device memory, or LDS when the planning workgroup counted them itself); `d`: what
 // plan_block_prepare returned.  Every thread of the workgroup must call this (it holds workgroup barriers); threads with `active` false
 // (those past kPlanThreads of a wider workgroup) only pass the barriers.
-template <class Count>
+// TOTALS: with what a launch's totals decide, pairs of row segments and slim tiles.  In a body of its own, since a launch of few rows, which has neither, waits for the
+// fetching of that code even where a test skips it: layer_head_kernel, us, skipped by a test / without it: 1 token of 64 experts 7.9 / 7.2, 32 tokens 7.8 / 7.5, 8 tokens of 60
+// experts 8.9 / 8.4, 64 with a shared expert 9.7 / 8.7.
+template <bool TOTALS, class Count>
 __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int chunk, const int chunks, const Count* recv, const mxmoe_block_desc& d, PlanShared& sh,
                                                 const bool active) {
   const int e0 = chunk * kMaxProblems;                       // first expert of this launch
@@ -200,17 +205,14 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
     // what this problem's tile shapes are, as far as the rest of the launch has no say in it, and the large tiles of the long problems
     // (launch_scope): whether one of K >= kLongK is above the launch's smallest is known behind the barrier
     have = mine ? plan_choose(info, fmt, (int)rows, N, choice) : 0;
-    if (info.may_pair) {
+    if (TOTALS && info.may_pair) {
       const unsigned load = (unsigned)wave_last((int)wave_inclusive_scan(have > 0 ? launch_load_of(choice, (int)rows, N, K) : 0u));  // (unsigned: the upper half takes all 16 bits)
       if (lane == 0) sh.load[wave] = load;
     }
-    if (info.has_slim) {
-      const int tall = have > 0 ? choice.large_tiles : 0;
-      const int all = wave_last(wave_inclusive_scan(tall)), at_km = wave_last(wave_inclusive_scan(K == km ? tall : 0));
-      if (lane == 0) {
-        sh.tall_tiles[wave] = all;
-        sh.tall_tiles_kmin[wave] = at_km;
-      }
+    if (TOTALS && info.has_slim) {
+      const unsigned tall = have > 0 ? (unsigned)choice.large_tiles : 0u;
+      const unsigned all = (unsigned)wave_last((int)wave_inclusive_scan(K == km ? tall : tall << 16));
+      if (lane == 0) sh.tall[wave] = all;
     }
     const int large = have > 0 && K >= kLongK ? choice.large_tiles : 0;
     if (__ballot(large > 0) != 0) {
@@ -229,14 +231,16 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
   const int long_tiles = sh.long_tiles[0] - (sh.kmin[0] == kmin ? sh.long_tiles_kmin[0] : 0) + sh.long_tiles[1] - (sh.kmin[1] == kmin ? sh.long_tiles_kmin[1] : 0);
   Segment sg[2];
   const int ns = have > 0 ? plan_split(info, fmt, (int)rows, N, choice, runs_long(K, kmin) ? min(long_tiles, kLongTiles) : info.few_blocks && integer_sums(fmt) ? choice.large_tiles : 0, sg) : 0;
-  if (info.has_slim) {
-    const int at_kmin = (sh.kmin[0] == kmin ? sh.tall_tiles_kmin[0] : 0) + (sh.kmin[1] == kmin ? sh.tall_tiles_kmin[1] : 0);
-    take_slim_tiles(info, long_k ? sh.tall_tiles[0] + sh.tall_tiles[1] - at_kmin : at_kmin, (int)rows, N, K, sg, ns);
+  if (TOTALS && info.has_slim) {
+    const unsigned t0 = sh.tall[0], t1 = sh.tall[1];
+    const int at_kmin = (int)((sh.kmin[0] == kmin ? t0 & 0xFFFF : 0) + (sh.kmin[1] == kmin ? t1 & 0xFFFF : 0));
+    const int all = (int)((t0 & 0xFFFF) + (t0 >> 16) + (t1 & 0xFFFF) + (t1 >> 16));
+    take_slim_tiles(info, long_k ? all - at_kmin : at_kmin, (int)rows, N, K, sg, ns);
   }
   const PlanBranch& my_branch = info.b[info.order[min(lane, kMaxBranches - 1)]];  // lane r: the branch of rank r
   const int my_order = my_branch.index;
   unsigned pair = 0;  // the second segment goes beside the first: one item of two entries
-  if (info.may_pair && ns == 2 && pairs_pay(fmt, (int)((sh.load[0] >> 16) + (sh.load[1] >> 16)), (int)((sh.load[0] & 0xFFFF) + (sh.load[1] & 0xFFFF)))) pair = pair_word(sg);
+  if (TOTALS && info.may_pair && ns == 2 && pairs_pay(fmt, (int)((sh.load[0] >> 16) + (sh.load[1] >> 16)), (int)((sh.load[0] & 0xFFFF) + (sh.load[1] & 0xFFFF)))) pair = pair_word(sg);
   int seg_rank[2] = {-1, -1}, seg_pos[2] = {0, 0}, seg_first[2] = {0, 0};
   // per branch in run order, this wave's entries and tiles
   for (int r = 0; active && r < info.nb; ++r) {

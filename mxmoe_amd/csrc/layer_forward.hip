@@ -236,9 +236,8 @@ __device__ __forceinline__ void head_token(const HeadArgs& a, int t, int lane) {
   }
 }
 
-// Workgroups: planning first (the longest chain of dependent steps), then the permutation's entries, then tokens, one per wave.  (Four waves per SIMD: left to
-// itself the compiler takes 178 registers for tokens of 4096 values, and 8192 of them 54 us instead of 48.)
-template <int NI, int TH>
+// Workgroups: planning first (the longest chain of dependent steps), then the permutation's entries, then tokens, one per wave.
+template <int NI, int TH, bool TOTALS>
 __global__ void __launch_bounds__(TH) layer_head_kernel(const HeadArgs a, const PlanPair pair) {
   extern __shared__ __align__(16) int32_t head_lds[];
   const int plan_wgs = 2 * pair.chunks;
@@ -261,7 +260,7 @@ __global__ void __launch_bounds__(TH) layer_head_kernel(const HeadArgs a, const 
     } else {
       count_ids<TH>(a.ids, a.total, a.E, 0, nullptr, head_lds, head_lds + a.E);
     }
-    plan_block_body(p, chunk, pair.chunks, head_lds, d, sh, plans);
+    plan_block_body<TOTALS>(p, chunk, pair.chunks, head_lds, d, sh, plans);
     return;
   }
   wg -= plan_wgs;
@@ -462,10 +461,11 @@ int mxmoe_layer_run(const void* handle, const void* hidden, const int32_t* topk_
   if (h.hist) launch_perm_hist(topk_ids, h.total, h.E, const_cast<int32_t*>(h.hist), true, s);
   const dim3 grid(2 * pair.chunks + h.perm_wgs + f.token_wgs), block(f.threads);
   const size_t lds = (size_t)(2 + f.threads / 64 + 2 * kCountCopies) * h.E * sizeof(int32_t);
+  const bool totals = pair.totals();
   auto head = [&](auto ni) {
     constexpr int NI = decltype(ni)::value;
-    if (f.threads == kHeadSmall) hipLaunchKernelGGL((layer_head_kernel<NI, kHeadSmall>), grid, block, lds, s, h, pair);
-    else hipLaunchKernelGGL((layer_head_kernel<NI, kHeadLarge>), grid, block, lds, s, h, pair);
+    if (f.threads == kHeadSmall) hipLaunchKernelGGL((totals ? layer_head_kernel<NI, kHeadSmall, true> : layer_head_kernel<NI, kHeadSmall, false>), grid, block, lds, s, h, pair);
+    else hipLaunchKernelGGL((totals ? layer_head_kernel<NI, kHeadLarge, true> : layer_head_kernel<NI, kHeadLarge, false>), grid, block, lds, s, h, pair);
   };
   switch (d.hidden / 512) {
     case 1: head(std::integral_constant<int, 1>{}); break;
