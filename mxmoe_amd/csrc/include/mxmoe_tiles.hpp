@@ -604,7 +604,8 @@ struct WxAxTile {
   }
   // fp8 (e4m3): the fragment pairs of both k-steps of a block in one instruction over the 64 k of the slice (unit scales), at twice the rate of the 16-deep
   // one.  (Half w4a4, half fp8, 60 experts of N = 2816, K = 2048 and N = 2048, K = 1408, 8192 tokens: both launches 350 -> 321 us; a Mixtral layer of 2000 tokens 837 ->
-  // 751.  The sums are as far from the float64 ones as they were: 1.2e-5 .. 5.1e-5 of their 2-norm.)  Which k a byte stands for is the same on both sides, and the sum runs over all of them either way (w8a8_g-1_sym_E4M3 of the reference: MMA_E4M3_K32,
+  // 751.  The sums are as far from the float64 ones as they were, of their 2-norm: 1.2e-5 .. 5.1e-5 with normal operands, up to 7.1e-5 with outliers, 2.5e-6 .. 3.3e-6 with one sign.)
+  // Which k a byte stands for is the same on both sides, and the sum runs over all of them either way (w8a8_g-1_sym_E4M3 of the reference: MMA_E4M3_K32,
   // mxmoe/kernels/src/include/mm_tile.cuh:696-697).
   __device__ static __forceinline__ void mma_slice(Acc& c, const v4i& w0, const v4i& w1, const v4i& a0, const v4i& a1) {
     typedef int v8i __attribute__((ext_vector_type(8)));
