@@ -513,17 +513,27 @@ __host__ __device__ inline unsigned pair_word(const Segment (&s)[2]) {
   return width <= 255 ? width << 21 : 0;
 }
 // Whether the two row segments of a problem are dealt out as a pair.  What a pair saves is the second trip of its weights from memory;
-// what it costs is that cheap tiles no longer come last, where they fill the end of the launch, so a launch has to have many tiles for it: `launch_tiles`
-// counts them in the shapes that are cheapest per row (launch_tiles_of).  At most 512 run at a time, together with those they share weights with; and there
-// large tiles that come first get a CU each.  Weights from memory, us, phases / pairs: 64 problems of N = 2816, K = 2048: w8a8 144 rows 146 / 102, 192 rows
-// 155 / 114, 546 rows 297 / 247 (N = 2048, K = 1408: 74 / 61, 78 / 68, 160 / 145), fp16 301 / 219, 310 / 232, 583 / 510; fp8 267 rows 210 / 190.  8 problems of
-// N = 28 672, K = 4096: w8a8 160 rows 363 / 247, 575 rows 678 / 580; of N = 4096, K = 14 336: 575 rows (640 tiles) 347 / 319, but 300 rows (384 tiles) 184 / 247.
-// int4 operands take half the time to fetch and as long to multiply: 144 rows 79 / 86, 192 rows 87 / 90, 546 rows 201 / 200, but with
-// N = 28 672, K = 4096 160 rows 205 / 194, 300 rows 294 / 260, 575 rows 472 / 438.  Weight-only tiles are bound by their arithmetic: 135 rows 134 / 149, 267 rows 209 / 273.
-// (launch_cols: the launch's blocks of 256 channels, each counted K / 4096 times: how much there is to fetch.)
-constexpr int kPairTiles = 512, kPairColsInt4 = 768;
+// what it costs is that cheap tiles no longer come last, where they fill the end of the launch.  `launch_tiles` counts the launch's tiles in the shapes that are cheapest
+// per row, `launch_cols` what there is to fetch: blocks of 256 channels, each K / 4096 times (a megabyte with 8 bits).  512 tiles run at a time.  With
+// fewer, large ones that come first get a CU each; around that number the second trip is worth it only of weights that the 256 MB last-level cache does not keep beside
+// the rest; with many, always.  From 2219 lists (N = 2048 .. 28 672, K = 1408 .. 14 336, 1 .. 64 problems, even and uneven rows), time of pairs over that of phases, 8-bit and 16-bit
+// operands, by tiles and weights:
+//                    under 60 MB    60 .. 130    130 .. 250    250 .. 500    500 .. 1000    more    at worst
+//   150 .. 300       1.01           1.02         1.03          1.02          1.01           0.99    1.42
+//   301 .. 448       1.00           1.00         0.98          0.99          0.92           0.88    1.36
+//   449 .. 512       0.99           1.01         0.96          0.91          0.88           0.88    1.11
+//   513 .. 700       1.01           1.04         0.98          0.93          0.89           0.99    1.19
+//   701 .. 1100      1.00           0.98         0.92          0.84          0.86           0.89    1.12
+//   beyond           -              0.97         0.94          0.87          0.82           0.84    1.13
+// us, phases / pairs: 16 problems of 180 rows, N = 4096, K = 14 336 (512 tiles) w8a8 311 / 253, fp16 721 / 544, fp8 309 / 230; one of 546 rows, N = 28 672, K = 4096 (560 tiles,
+// 117 MB) w8a8 74 / 89; 64 of 192 rows, N = 2816, K = 2048 w8a8 155 / 114, fp16 310 / 232; 8 of 300 rows, N = 4096, K = 14 336 (384 tiles) w8a8 184 / 247.
+// int4 operands take half the time to fetch and as long to multiply: 1.06 .. 1.14 up to 700 tiles and 250 MB, 1.01 .. 1.06 up to 1100, beyond that 0.98 from 250 MB on, 1.02 .. 1.05 below.
+// Weight-only tiles are bound by their arithmetic: 135 rows 134 / 149, 267 rows 209 / 273.
+constexpr int kPairTiles = 448, kPairTilesMany = 700, kPairTilesInt4 = 1000, kPairCols = 192, kPairColsInt4 = 768;
 __host__ __device__ inline bool pairs_pay(int f, int launch_tiles, int launch_cols) {
-  return launch_tiles > kPairTiles && (f == (int)Fmt::W8A8 || f == (int)Fmt::FP16 || (f == (int)Fmt::W4A4 && launch_cols > kPairColsInt4));
+  if (f == (int)Fmt::W4A4) return launch_tiles > kPairTilesInt4 && launch_cols > kPairColsInt4;
+  if (f != (int)Fmt::W8A8 && f != (int)Fmt::FP16) return false;
+  return launch_tiles > kPairTilesMany || (launch_tiles > kPairTiles && launch_cols > (f == (int)Fmt::FP16 ? kPairCols / 2 : kPairCols));
 }
 
 // Large tiles of a launch's problems of one length (the smallest K; any longer one) up to which the 128 x 128 tile of 8-bit weights runs in the place of the 128 x 256
@@ -564,9 +574,10 @@ constexpr int kLargeTilesTop = (kSlimTiles > kLongTiles ? kSlimTiles : kLongTile
 
 // What a problem adds to its launch's `launch_tiles` (upper half) and `launch_cols` (lower half).  Clamped where more makes no difference: the sums over a wave's
 // problems stay within 16 bits each.
+static_assert(64 * (kPairTilesInt4 + 1) < 1 << 16 && 64 * (kPairColsInt4 + 1) < 1 << 16, "two sums in a word");
 __host__ __device__ inline unsigned launch_load_of(const PlanChoice& c, int M, int N, int K) {
   const unsigned tm = tiles_over(M, c.unit.bm_log2), tn = tiles_over(N, c.unit.bn_log2), blocks = tiles_over(N, 8);
-  const unsigned tiles = tm > kPairTiles || tn > kPairTiles || tm * tn > kPairTiles ? kPairTiles + 1 : tm * tn;
+  const unsigned tiles = tm > kPairTilesInt4 || tn > kPairTilesInt4 || tm * tn > kPairTilesInt4 ? kPairTilesInt4 + 1 : tm * tn;
   const unsigned cols = blocks > kPairColsInt4 || K > (kPairColsInt4 << 12) || blocks * (unsigned)K > (kPairColsInt4 << 12) ? kPairColsInt4 + 1 : blocks * (unsigned)K >> 12;
   return tiles << 16 | cols;
 }

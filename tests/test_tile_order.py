@@ -63,7 +63,11 @@ def test_tiles_of_a_pair_that_share_weights_are_neighbours(lib):
 
 @pytest.mark.parametrize("q,count,rows,n,k,pairs", [
     (W8, 64, 192, 2048, 1408, True), (W8, 8, 300, 4096, 14336, False),     # 1024 and 384 tiles: past and within what runs at a time
+    (W8, 16, 144, 4096, 14336, True), (W8, 12, 144, 4096, 14336, False), (FP, 7, 180, 4096, 14336, False), (FP, 8, 256 + 10, 4096, 4096, False),  # 512 and 384, 224, 384
+    (W8, 1, 546, 28672, 4096, False), (FP, 1, 546, 28672, 4096, True), (W8, 2, 290, 28672, 4096, True), (W8, 24, 290, 2048, 1408, False),  # 112, 224, 224, 48 columns
+    (W8, 16, 420, 2816, 2048, True), (FP, 32, 144, 2048, 1408, False),     # 704 tiles; 512 of little weight
     (W4, 64, 192, 2816, 2048, False), (W4, 8, 300, 28672, 4096, True),     # int4: by what there is to fetch
+    (W4, 24, 144, 4096, 14336, False), (W4, 32, 160, 4096, 14336, True),   # 768 and 1024 tiles
     (WO, 64, 140, 28672, 4096, False), ((4, 4, 128, True), 64, 90, 28672, 4096, False),
 ])
 def test_when_segments_are_paired(lib, q, count, rows, n, k, pairs):
