@@ -83,7 +83,8 @@ def _device_plan_is_the_hosts(lib, q, counts, n, k):
     from mxmoe_amd import _lib
 
     e = len(counts)
-    desc = (_lib.BlockDesc * e)(*[_lib.BlockDesc(q[0], q[1], q[2], int(q[3]), (C.c_uint8 * 3)(), n, k, 0, 0)] * e)
+    qs, ks = (q if isinstance(q, list) else [q] * e), (k if isinstance(k, list) else [k] * e)
+    desc = (_lib.BlockDesc * e)(*[_lib.BlockDesc(a, w, g, int(sym), (C.c_uint8 * 3)(), n, kk, 0, 0) for (a, w, g, sym), kk in zip(qs, ks)])
     kid = lib.mxmoe_plan_select_kernel(-1, desc, e)
     d_desc = torch.frombuffer(bytearray(bytes(desc)), dtype=torch.uint8).cuda()
     recv = torch.tensor(counts, dtype=torch.int64, device="cuda")
@@ -91,7 +92,7 @@ def _device_plan_is_the_hosts(lib, q, counts, n, k):
     some = torch.zeros(16, dtype=torch.uint8, device="cuda")
     _lib.check(lib, lib.mxmoe_plan_block(kid, recv.data_ptr(), e, 0, d_desc.data_ptr(), desc, some.data_ptr(), some.data_ptr(), some.data_ptr(), plan.data_ptr(),
                                          torch.cuda.current_stream().cuda_stream))
-    tab, _ = _launch(lib, [(m, n, k, q) for m in counts], kid)
+    tab, _ = _launch(lib, [(m, n, kk, qq) for m, kk, qq in zip(counts, ks, qs)], kid)
     ne, tiles, nph, grid = tab[:4]
     hdr = plan.cpu().numpy()[:4096].view(np.int32)[14:]
     assert list(hdr[:4]) == [0, ne, tiles, nph] and grid <= lib.mxmoe_plan_grid_bound(kid, desc, e, sum(counts), 0)
@@ -130,6 +131,18 @@ def test_width_of_the_8_bit_weight_only_tile(lib, kernel, count, rows, n, k, bn)
 @pytest.mark.parametrize("count,rows,n,k", [(8, 192, 2048, 1408), (16, 192, 2048, 1408), (17, 192, 2048, 1408), (60, 150, 2048, 1408), (4, 64, 2816, 2048), (5, 64, 2816, 2048), (1, 2000, 2048, 1408)])
 def test_device_planner_takes_the_same_width(lib, count, rows, n, k):
     _device_plan_is_the_hosts(lib, WO8, [(rows, 0, 5)[i % 3] for i in range(count * 3)][:119], n, k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("other", [[WO8], [WO8, WO, W8, FP]])
+@pytest.mark.parametrize("many,few", [(130, 1000), (20, 200), (300, 100), (130, 1100)])
+def test_device_planner_takes_the_same_width_beside_problems_of_another_length(lib, other, many, few):
+    """Few problems of K = 5632, and of K = 256, beside many of K = 1408: both waves of the planner hold some of each."""
+    e = 90
+    ks = [5632 if i % 29 == 7 else 1408 for i in range(e)]
+    counts = [few if k > 1408 else (many, 0, many + 3, 40)[i % 4] for i, k in enumerate(ks)]
+    _device_plan_is_the_hosts(lib, [other[i % len(other)] for i in range(e)], counts, 2048, ks)
+    _device_plan_is_the_hosts(lib, [other[i % len(other)] for i in range(e)], counts, 2048, [256 if k > 1408 else k for k in ks])
 
 
 @pytest.mark.gpu
