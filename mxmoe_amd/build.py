@@ -32,13 +32,19 @@ def check_no_spills(remarks: str) -> None:
 
     Those tiles load weight fragments with loads the compiler does not track (the waits are placed by hand): a fragment register
     that the compiler spills or re-uses while its load is in flight is overwritten when the load lands, and when that register
-    holds an address the next access faults.  `remarks` is hipcc's -Rpass-analysis=kernel-resource-usage output."""
+    holds an address the next access faults.  `remarks` is hipcc's -Rpass-analysis=kernel-resource-usage output.
+
+    Nor may a planning kernel (its name holds `PlanPair`, its argument) use scratch memory: that is a local array indexed by a loop the compiler
+    did not unroll, and every launch of the layer's first kernel is a microsecond longer for it, whether its workgroups plan or not."""
     name = None
     for line in remarks.splitlines():
         m = re.search(r"remark: Function Name: (\S+)", line)
         if m:
             name = m.group(1)
             continue
+        m = re.search(r"remark:\s+ScratchSize \[bytes/lane\]: (\d+)", line)
+        if m and name and "PlanPair" in name and int(m.group(1)) > 0:
+            raise RuntimeError(f"{name}: {m.group(1)} bytes of scratch memory per lane in a planning kernel; unroll the loop that indexes a local array")
         m = re.search(r"remark:\s+VGPRs Spill: (\d+)", line)
         if m and name and any(t in name for t in ("WxAxTile", "WxAxNarrowTile", "Bf6Tile")) and int(m.group(1)) > 0:
             raise RuntimeError(f"{name}: {m.group(1)} vector registers spilled in a kernel with hand-tracked loads; shrink the tile's "

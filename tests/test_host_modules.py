@@ -324,6 +324,17 @@ def test_build_refuses_spilling_kernels_of_every_tile_with_hand_tracked_loads(ti
         check_no_spills(fmt.format(tile, 1))
 
 
+def test_build_refuses_planning_kernels_with_scratch_memory():
+    from mxmoe_amd.build import check_no_spills
+
+    fmt = "t.hip:1:1: remark: Function Name: {} [-Rpass-analysis=kernel-resource-usage]\nt.hip:1:1: remark:     ScratchSize [bytes/lane]: {} [-Rpass-analysis=kernel-resource-usage]\n"
+    head = "_ZN5mxmoe17layer_head_kernelILi4ELi256ELb1EEEvNS_8HeadArgsENS_8PlanPairE"
+    check_no_spills(fmt.format(head, 0))
+    check_no_spills(fmt.format("_Z14combine_kernel11CombineArgs", 16))
+    with pytest.raises(RuntimeError, match="scratch"):
+        check_no_spills(fmt.format(head, 64))
+
+
 def test_build_refuses_moves_of_registers_with_loads_in_flight():
     """The build's ISA check: a register written by a hand-tracked (inline-assembly) load may not be moved before the wait that names it."""
     from mxmoe_amd.build import check_untracked_load_copies as chk
