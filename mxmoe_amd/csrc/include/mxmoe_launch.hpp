@@ -326,6 +326,7 @@ struct BranchInfo {
   // (w8a8_g-1_sym_E4M3, mxmoe/kernels/tile_config.py:45: QParams (8, 8, -1, sym) there as well).  A kernel with such a branch is
   // never chosen automatically: the caller names it, because only the caller knows what its operands hold.
   int variant = 0;
+  int n_multiple = 8;  // N must be a multiple of this
 };
 constexpr int kVariantBf6 = 1, kVariantFp8 = 2, kVariantBf16 = 3;
 
@@ -374,7 +375,7 @@ template <int WBITS, int BN, int MB, int WAVES>
 struct BranchOf<SkinnyWoTile<WBITS, BN, MB, WAVES>> {
   static BranchInfo get() {
     using T = SkinnyWoTile<WBITS, BN, MB, WAVES>;
-    return BranchInfo{WBITS == 8 ? Fmt::W8A16 : WBITS == 4 ? Fmt::W4A16 : WBITS == 3 ? Fmt::W3A16 : Fmt::W2A16, T::kABits, T::kWBits, T::BM, BN, 128, 1, 4, T::kLdsBytes, 128, 0};
+    return BranchInfo{WBITS == 16 ? Fmt::FP16 : WBITS == 8 ? Fmt::W8A16 : WBITS == 4 ? Fmt::W4A16 : WBITS == 3 ? Fmt::W3A16 : Fmt::W2A16, T::kABits, T::kWBits, T::BM, BN, 128, 1, 4, T::kLdsBytes, 128, 0, 0, 0, 16};
   }
 };
 
@@ -417,7 +418,7 @@ template <int WBITS, int BM, int BN>
 struct BranchOf<WoMfmaTile<WBITS, BM, BN>> {
   static BranchInfo get() {
     using T = WoMfmaTile<WBITS, BM, BN>;
-    return BranchInfo{WBITS == 8 ? Fmt::W8A16 : WBITS == 4 ? Fmt::W4A16 : WBITS == 3 ? Fmt::W3A16 : Fmt::W2A16, T::kABits, T::kWBits, BM, BN, 128, T::WM, 4 / T::WM, T::kLdsBytes, 128, 0};
+    return BranchInfo{WBITS == 8 ? Fmt::W8A16 : WBITS == 4 ? Fmt::W4A16 : WBITS == 3 ? Fmt::W3A16 : Fmt::W2A16, T::kABits, T::kWBits, BM, BN, 128, T::WM, 4 / T::WM, T::kLdsBytes, 128, 0, 0, 0, 16};
   }
 };
 
@@ -435,7 +436,7 @@ inline double tile_cost(const BranchInfo& b) {
       // advantage they show as single-tile kernels in the profile table)
       {Fmt::W4A4, 128, 256, 1.00}, {Fmt::W4A4, 64, 256, 0.58}, {Fmt::W4A4, 32, 256, 0.48}, {Fmt::W4A4, 32, 64, 0.13},
       {Fmt::W8A8, 128, 256, 1.00}, {Fmt::W8A8, 64, 256, 0.74}, {Fmt::W8A8, 32, 256, 0.56}, {Fmt::W8A8, 32, 64, 0.155},
-      {Fmt::FP16, 128, 256, 1.00}, {Fmt::FP16, 64, 256, 0.69}, {Fmt::FP16, 32, 256, 0.53}, {Fmt::FP16, 128, 128, 0.57}, {Fmt::FP16, 256, 128, 1.09},
+      {Fmt::FP16, 128, 256, 1.00}, {Fmt::FP16, 64, 256, 0.69}, {Fmt::FP16, 32, 256, 0.53}, {Fmt::FP16, 16, 64, 0.30}, {Fmt::FP16, 128, 128, 0.57}, {Fmt::FP16, 256, 128, 1.09},
       {Fmt::W4A16, 16, 128, 0.37}, {Fmt::W4A16, 16, 64, 0.20}, {Fmt::W4A16, 32, 128, 0.50}, {Fmt::W4A16, 128, 128, 1.00}, {Fmt::W4A16, 128, 256, 1.50},
       {Fmt::W3A16, 16, 128, 0.31}, {Fmt::W3A16, 16, 64, 0.20}, {Fmt::W3A16, 32, 128, 0.50}, {Fmt::W3A16, 128, 128, 1.00}, {Fmt::W3A16, 128, 256, 1.50},
       {Fmt::W2A16, 16, 128, 0.25}, {Fmt::W2A16, 16, 64, 0.20}, {Fmt::W2A16, 32, 128, 0.50}, {Fmt::W2A16, 128, 128, 1.00}, {Fmt::W2A16, 128, 256, 1.50},
@@ -871,7 +872,11 @@ struct RowSummary {
   long blocks = 0;                // of 256 channels
   uint32_t max_k = 0;
   bool w4a4 = false, w8a8 = false, other = false;  // formats among them
-  void add_format(Fmt f) { (f == Fmt::W4A4 ? w4a4 : f == Fmt::W8A8 ? w8a8 : other) = true; }
+  bool fp16 = true;                                // no other format than this one
+  void add_format(Fmt f) {
+    (f == Fmt::W4A4 ? w4a4 : f == Fmt::W8A8 ? w8a8 : other) = true;
+    fp16 = fp16 && f == Fmt::FP16;
+  }
   void add(Fmt f, long m, uint32_t N, uint32_t K) {
     if (m == 0) return;
     add_format(f);
@@ -928,10 +933,14 @@ inline bool few_rows(const RowSummary& s) {
 // a shared one, w4a16 / w3a16, 30.2 -> 28.2 (1 token), 42.7 -> 39.2 (4), 64 -> 61 (16), 75 -> 73 (64); 60 experts top-4 and a shared one 33.6 -> 29.0 (1),
 // 58 -> 51 (16); 8 experts of N = 28 672 / 4096 61.6 -> 52.1 (1), 144 -> 140 (16), but 144 -> 150 (32: 8 rows each).  (Launches of fewer than 8 blocks
 // would take 0.73 .. 0.81 of the time as well: 7 blocks of K = 2048, 1 row, 7.6 -> 5.9.)
-constexpr int kFewTokenRows = 6;
+// The same for lists with fp16 or 8-bit weight-only problems (a kernel of its own, 142 registers: three workgroups per CU), against the kernels of wider tiles, us a layer: 60 experts top-4
+// fp16 67 -> 35 (1 token), 86 -> 73 (4), 131 -> 108 (8), 166 -> 158 (16), 207 -> 196 (32), 216 -> 217 (64), with a shared expert 143 -> 68 (1), 208 -> 141 (16), 288 -> 232 (64); 8 experts of N = 28 672 /
+// 4096 fp16 327 -> 173 (1), 583 -> 447 (16), 622 -> 521 (32: 8 rows each), 639 -> 614 (48), 642 -> 705 (64): weights of 16 bits outweigh the activations for longer, up to 12 rows.  w8a16 / w2a16 half and
+// half, 64 experts top-6 and a shared one 37 -> 31 (1), 71 -> 65 (8), 103 -> 96 (32), 8 experts 100 -> 80 (1), 204 -> 200 (8), 213 -> 215 (32).
+constexpr int kFewTokenRows = 6, kFewTokenRowsFp16 = 12;
 inline bool only_narrow_few_token(const FusedKernel& k) {
   for (const BranchInfo& b : k.branches)
-    if (!is_weight_only(b.fmt) || b.BN != 64) return false;
+    if (b.a_bits != 16 || b.BN != 64) return false;
   return true;
 }
 
@@ -950,30 +959,34 @@ int few_row_kernel(const RowSummary& s, Covers&& covers) {
     if (kid >= 0) return kid;
   }
   if (4 * s.tall > s.live) return -1;
-  const int kid = first([&](const FusedKernel& k) { return k.max_rows_hint > 0 && s.max_rows <= k.max_rows_hint; });
-  if (kid >= 0 && s.rows <= kFewTokenRows * s.live && s.blocks >= kFewBlocksMin) {
-    const int narrow = first(only_narrow_few_token);
-    if (narrow >= 0) return narrow;
+  if (s.max_rows <= kFewRowsMax && s.rows <= (s.fp16 ? kFewTokenRowsFp16 : kFewTokenRows) * s.live && s.blocks >= kFewBlocksMin) {
+    const int kid = first(only_narrow_few_token);
+    if (kid >= 0) return kid;
   }
-  return kid;
+  return first([&](const FusedKernel& k) { return k.max_rows_hint > 0 && s.max_rows <= k.max_rows_hint; });
+}
+
+// K a multiple of the tile's K step, N a multiple of 8 (16 for the weight-only layouts and the few-token tiles)
+inline bool shape_ok(const BranchInfo& bi, const mxmoe_dim3& sz) {
+  return sz.z != 0 && sz.z % bi.k_multiple == 0 && (int)sz.z >= bi.k_min && sz.y % bi.n_multiple == 0;
 }
 
 // The kernel the launcher picks when the caller names none: one made for few rows, or the first fused kernel without operand variants that has a tile for every
 // format.
 inline int auto_kernel(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int count) {
   auto covers = [&](const FusedKernel& k) { return !kernel_has_variants(k) && kernel_covers(k, h_q, count); };
-  const int few = few_row_kernel(row_summary(h_sizes, h_q, count), covers);
+  auto fits = [&](const FusedKernel& k) {  // (an fp16 problem may have a shape that the few-token tiles do not take)
+    for (int i = 0; i < count; ++i)
+      for (const BranchInfo& b : k.branches)
+        if (h_sizes[i].x != 0 && b.fmt == classify(h_q[i]) && !shape_ok(b, h_sizes[i])) return false;
+    return true;
+  };
+  const int few = few_row_kernel(row_summary(h_sizes, h_q, count), [&](const FusedKernel& k) { return covers(k) && fits(k); });
   if (few >= 0) return few;
   auto& reg = registry();
   for (int i = 0; i < (int)reg.size(); ++i)
     if (reg[i].policy == Policy::Fused && reg[i].max_rows_hint == 0 && covers(reg[i])) return i;
   return -1;
-}
-
-// K a multiple of the tile's K step, N a multiple of 8 (16 for the weight-only layouts)
-inline bool shape_ok(const BranchInfo& bi, const mxmoe_dim3& sz) {
-  const bool wo = is_weight_only(bi.fmt);
-  return sz.z != 0 && sz.z % bi.k_multiple == 0 && (int)sz.z >= bi.k_min && sz.y % 8 == 0 && !(wo && sz.y % 16 != 0);
 }
 
 // What the planning of one launch's problems has in common: its smallest K, its tiles (where it may have pairs), its large tiles and those of its long problems, whether it has

@@ -1,4 +1,4 @@
-// Skinny weight-only tiles (w8a16 / w4a16 / w3a16 / w2a16, one (scale, zero) pair per channel and 128-wide K group) for experts that
+// Skinny weight-only tiles (w8a16 / w4a16 / w3a16 / w2a16, one (scale, zero) pair per channel and 128-wide K group; and fp16, plain_stream()) for experts that
 // receive a handful of tokens.  Per-channel formats (group size -1, the reference's cta_gemm_multistage_qb_v2 with GSIZE = -1,
 // mxmoe/kernels/src/include/cta_gemm.cuh:113-286) use the same tiles: their packer repeats the channel's pair for every group.
 //
@@ -37,7 +37,7 @@ namespace mxmoe {
 // tokens still streams its weights once (two 16-token tiles stream them twice, the second time out of L2 at best, and take nearly
 // twice as long).
 // 4, 3 and 2 bits: a wave walks its K range as one stream (stream()), with as many packed blocks in flight as the tile has channel blocks.
-// 8 bits, whose packed blocks take twice the registers: in passes (pass()) of KP k blocks (128 wide), whose activations live in registers, with
+// fp16: plain_stream().  8 bits, whose packed blocks take twice the registers, in tiles of 128 channels: in passes (pass()) of KP k blocks (128 wide), whose activations live in registers, with
 // kRing packed blocks in flight; the activations of a pass take MB times the registers, which is why both shrink as MB grows.
 // The stream replaced passes for every width but 8 (there it spills at 32 tokens and gains nothing at 16).  A pass starts with an empty ring and waits
 // out a memory latency, two or more times per tile.  64 problems of N = 2816, K = 2048, us, pass -> stream: 24 tokens w4 57 -> 45, w3 57 -> 44, w2
@@ -45,14 +45,15 @@ namespace mxmoe {
 template <int WBITS_, int BN_, int MB_ = 1, int WAVES_ = 2>
 struct SkinnyWoTile {
   static constexpr int WBITS = WBITS_, MB = MB_, BM = 16 * MB_, BN = BN_;
-  static_assert(WBITS == 8 || WBITS == 4 || WBITS == 3 || WBITS == 2, "w8 / w4 / w3 / w2");
+  static_assert(WBITS == 16 || WBITS == 8 || WBITS == 4 || WBITS == 3 || WBITS == 2, "fp16 / w8 / w4 / w3 / w2");
   static_assert(BN % 64 == 0, "the final reduction deals 16-channel blocks to 4 waves");
   static constexpr int NB = BN / 16;                 // 16-channel blocks per tile
   static constexpr int kRedBytes = kWaves * NB * MB * 64 * 16;  // per-wave partial sums for the final reduction
-  static constexpr bool kStream = WBITS != 8;                 // stream() instead of pass()
+  static constexpr bool kPlain = WBITS == 16;                 // fp16 weights: plain_stream()
+  static constexpr bool kStream = WBITS != 8 || (MB == 1 && BN == 64);  // stream() instead of pass()
   static constexpr int KP = MB == 1 ? 4 : 2, kRing = MB == 1 ? 6 : 4;  // of pass()
   static constexpr int kChunk = kStream ? 4 : KP;              // k blocks whose (scale, zero) pairs a wave holds at a time
-  static constexpr int kScaleBytes = NB * kChunk * 64;        // its patch for them
+  static constexpr int kScaleBytes = kPlain ? 0 : NB * kChunk * 64;  // its patch for them
   static constexpr int kLdsBytes = kRedBytes + kWaves * kScaleBytes;
   static constexpr int kAccRegs = NB * MB * 4;
   static constexpr int kWavesWanted = WAVES_;
@@ -354,6 +355,62 @@ struct SkinnyWoTile {
     }
   }
 
+  // fp16 weights, row-major [N][K]: the same walk without scales.  Bound by the weights' bytes, with few problems by how many workgroups there are to ask for them: four times as many
+  // as tiles of 256 channels (MfmaTile) make, each wave with 16 KB in flight and no barrier.  60 experts of N = 2816 / 2048, K = 2048 / 1408, top-4, us a layer: 1 token 67 -> 35, 8 tokens
+  // 131 -> 108; with a shared expert four times as wide, whose second block was one stream of K = 5632 in eight workgroups, 143 -> 68 and 182 -> 119; 8 experts of
+  // N = 28 672 / 4096 (6 experts hit by 4 tokens: 2.1 GB) 502 -> 367.  A lane holds weights k = 128 kb + 32 j + 8 lg + 0..7 of channel lm, j = 0..3 (16 rows x 64 bytes a
+  // load, four loads one after the other 256 bytes of each row), and its activations in the same order.
+  template <bool GU>
+  __device__ static __forceinline__ void plain_stream(const TileArgs& t, int kb_lo, int kb_hi, int n0, int nbv, int lane, const int (&src)[MB], v4f (&acc)[NB][MB]) {
+    if (kb_lo >= kb_hi) return;
+    const int K = t.K, lm = lane & 15, lg = lane >> 4;
+    const _Float16* wr[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      const int b = GU ? (nb % (NB / 2) < nbv ? nb % (NB / 2) : 0) : nb < nbv ? nb : 0;  // (blocks that do not exist re-read an existing one)
+      wr[nb] = reinterpret_cast<const _Float16*>(t.B) + (long)(n0 + b * 16 + lm + (GU && nb >= NB / 2 ? t.N / 2 : 0)) * K + lg * 8;
+    }
+    const _Float16* xr[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) xr[mb] = reinterpret_cast<const _Float16*>(t.A) + (long)src[mb] * K + lg * 8;
+    auto half8 = [&](const _Float16* p, int j, int kb) { return __builtin_bit_cast(v8h, gload<v4i>(p + kb * 128 + j * 32)); };
+    v8h w[NB][4], x[MB][4];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[mb][j] = half8(xr[mb], j, kb_lo);
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[nb][j] = half8(wr[nb], j, kb_lo);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+    for (int kb = kb_lo; kb < kb_hi; ++kb) {
+      const int next = min(kb + 1, kb_hi - 1);  // (the last refills read what is there already and are not used)
+      v8h xn[MB][4];
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) xn[mb][j] = half8(xr[mb], j, next);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[nb][j], x[mb][j], acc[nb][mb], 0, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[nb][j] = half8(wr[nb], j, next);
+        __builtin_amdgcn_sched_barrier(0);  // the refill is issued here
+      }
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[mb][j] = xn[mb][j];
+    }
+  }
+
   template <bool GU>
   __device__ static __forceinline__ void run(const TileArgs& t, uint8_t* __restrict__ smem) {
     const int tid = threadIdx.x;
@@ -382,7 +439,9 @@ struct SkinnyWoTile {
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = v4f{0.f, 0.f, 0.f, 0.f};
-    if constexpr (kStream) {
+    if constexpr (kPlain) {
+      plain_stream<GU>(t, kb_lo, kb_hi, n0, nbv, lane, src, acc);
+    } else if constexpr (kStream) {
       stream<GU>(t, kb_lo, kb_hi, n0, nbv, lane, src, spatch, acc);
     } else {
       for (int kb = kb_lo; kb < kb_hi; kb += KP) {

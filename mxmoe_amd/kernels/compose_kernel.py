@@ -26,7 +26,7 @@ from pathlib import Path
 
 from .. import build as _build
 from .kernel_sketch import ABI_TU, DEFAULT_ORDER_TEMPLATE, KERNEL_DECLARATION_TEMPLATE, KERNEL_DEFERRED_TEMPLATE, KERNEL_DEFINITION_TEMPLATE
-from .tile_config import QCFG_MAP, SUPPORTED_QCFG, TileConfig, get_gpu_info, get_info_from_qcfg_str, get_possible_tile_list, narrow_tile  # noqa: F401
+from .tile_config import QCFG_MAP, SUPPORTED_QCFG, TileConfig, few_token_tile, get_gpu_info, get_info_from_qcfg_str, get_possible_tile_list, narrow_tile  # noqa: F401
 
 
 class KernelType(str, enum.Enum):
@@ -211,6 +211,9 @@ def default_kernel_specs(arch: str = "gfx950"):
         ("groupgemm_hz_fused_wxax_few", KernelType.Fused, OrderedDict((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8))),
         ("groupgemm_hz_fused_all_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8)), *wo_all.items(),
                                                                        ("w8a16_g128_asym", _pick(arch, "w8a16_g128_asym", (16, 128), (32, 128), (128, 256), (128, 128)))])),
+        # the few-token tiles of 64 channels of every format with 16-bit activations: fp16 and 8-bit weights take 142 registers (three workgroups per CU) where the
+        # kernel without them has 125 (four)
+        ("groupgemm_hz_fused_a16_few", KernelType.Fused, OrderedDict((q, (few_token_tile(q),)) for q in (*(f"w{b}a16_g128_asym" for b in (4, 3, 2, 8)), "fp16"))),
     ]
 
 

@@ -204,6 +204,8 @@ class TileConfig:
 
     def smem_bytes_tile(self):
         """LDS bytes of the tile as compiled (csrc/include/mxmoe_tiles.hpp, mxmoe_wo_tiles.hpp)."""
+        if self.is_skinny() and self.QCFGB.QBITS == 16:
+            return 4 * (self.BN // 16) * 64 * 16  # (no scales)
         if self.is_skinny():  # per-wave partial sums of the final reduction + (scale, zero) patches of 4 k blocks (2 in the 32-token 8-bit tile's passes)
             kp = 2 if self.QCFGB.QBITS == 8 and self.BM == 32 else 4
             return 4 * (self.BN // 16) * (64 * 16 * (self.BM // 16) + kp * 64)
@@ -320,6 +322,12 @@ def get_possible_tile_list(arch: str, qcfg: str) -> list:
 def narrow_tile(qcfg: str) -> TileConfig:
     """The w4a4 / w8a8 tile for launches with few workgroups (not among the candidates of get_possible_tile_list: its kernels are chosen by launch)."""
     return _with_q(TileConfig(BM=32, BN=64, BK=128 if qcfg == "w4a4_g-1_sym" else 64, WM=1, WN=1, WK=4, STAGE=3, MMA=QCFG_TO_MMA[qcfg]), qcfg)
+
+
+def few_token_tile(qcfg: str) -> TileConfig:
+    """The 16 x 64 tile of the formats with 16-bit activations for a handful of rows, compiled for 3 waves per SIMD: for kernels made of such tiles alone (fp16 and w8a16: not
+    among the candidates of get_possible_tile_list either)."""
+    return _with_q(TileConfig(BM=16, BN=64, BK=128, WM=1, WN=4, WK=1, STAGE=4, MMA="MFMA_F32_16x16x32_F16"), qcfg)
 
 
 _FIELD = re.compile(r"(BM|BN|BK|WM|WN|WK|STAGE|SPLITK)=(-?\d+)")

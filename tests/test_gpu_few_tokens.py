@@ -1,0 +1,112 @@
+"""The few-token tiles of fp16 and of 8-bit weights (16 x 64, groupgemm_hz_fused_a16_few): where their ranges end, and what is sent to them."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import mxmoe_oracle as O
+
+FP16, W8A16 = (16, 16, -1, True), (16, 8, 128, False)
+
+
+def _problem(rng, m, n, k, q):
+    """Operands on the host and the product in float64 (8-bit weights: of the dequantised weights, not rounded)."""
+    from mxmoe_amd.weights import quantize_and_pack
+
+    x = rng.standard_normal((m, k)).astype(np.float16)
+    w = (rng.standard_normal((n, k)) * 0.02).astype(np.float16)
+    if q == FP16:
+        return x, torch.from_numpy(w), None, x.astype(np.float64) @ w.astype(np.float64).T
+    pw = quantize_and_pack(torch.from_numpy(w), q)
+    c, s, z = O.quant_minmax(w, 8, 128, False)
+    deq = c.reshape(n, k // 128, 128).astype(np.float64) * s.reshape(n, -1, 1).astype(np.float64) + z.reshape(n, -1, 1).astype(np.float64)
+    return x, pw.data, pw.scale, x.astype(np.float64) @ deq.reshape(n, k).T
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k", [128, 384, 512, 640, 2176])
+def test_few_token_tiles_of_16_and_8_bit_weights(k):
+    """K dealt to four waves: parts of no block, one, several, and unequal ones; 1 row, a whole row tile, one row more, several tiles; channels that end inside a tile's 64.
+    The output's rounding is at most 2^-11 of it; the fp32 sums add, for 8 bits, those of terms that still carry the codes' bias (as in
+    test_weight_only_streams_of_every_length): as much again."""
+    from mxmoe_amd import _lib
+    from mxmoe_amd.group_gemm import GroupGemmLaunch
+
+    rng = np.random.default_rng(k)
+    sizes = [(1, 64), (16, 144), (17, 16), (33, 80), (5, 256)]
+    probs = [(*_problem(rng, m, n, k, q), (m, n, k), q) for m, n in sizes for q in (FP16, W8A16)]
+    Cs = [torch.full(p[4][:2], float("nan"), dtype=torch.float16, device="cuda") for p in probs]
+    kid = _lib.load().mxmoe_find_kernel(b"groupgemm_hz_fused_a16_few")
+    GroupGemmLaunch([torch.from_numpy(p[0]).cuda() for p in probs], [p[1].cuda() for p in probs], [None] * len(probs), [None if p[2] is None else p[2].cuda() for p in probs], Cs,
+                    [p[4] for p in probs], [p[5] for p in probs], kernel_id=kid).run()
+    for p, c in zip(probs, Cs):
+        err = np.linalg.norm(c.cpu().numpy().astype(np.float64) - p[3]) / np.linalg.norm(p[3])
+        assert err <= (2.0 ** -11 if p[5] == FP16 else 2.0 ** -10), (p[4], p[5], err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [1, 5, 33])
+@pytest.mark.parametrize("q", [FP16, W8A16])
+def test_layer_on_the_few_token_tiles(tokens, q):
+    """Their gate_up form (rows gathered by token, several row tiles of one expert at 33 tokens, dropped ids) and the block behind it, against the layer in float64 on the same
+    weights: three roundings to fp16 (silu * up of rounded gate and up, down, combine), each at most 2^-11 of its result, add up to less than 2^-9 of the norm."""
+    from mxmoe_amd import _lib, synth
+    from mxmoe_amd.layer import MxMoELayer
+
+    cfg = synth.MoEConfig("t", "test", 6, 2, 512, 640, tokens, num_shared=1, rotate=0)
+    layer = MxMoELayer(cfg, formats=[(q, q)] * 7)
+    layer._planned_kernel = lambda *_: _lib.load().mxmoe_find_kernel(b"groupgemm_hz_fused_a16_few")
+    hidden = synth.make_hidden(cfg)
+    ids, w = synth.make_routing(cfg)
+    ids[:, 0] = 1
+    ids[-1, 1] = -1 if tokens > 1 else ids[-1, 1]
+    got = layer(hidden.cuda(), ids.cuda(), w.cuda()).cpu().numpy().astype(np.float64)
+
+    def dense(e):
+        out = []
+        for m in synth.expert_weights(cfg, e):
+            m = m.numpy()
+            if q == W8A16:
+                c, s, z = O.quant_minmax(m, 8, 128, False)
+                g = m.shape[1] // 128
+                m = c.reshape(m.shape[0], g, 128).astype(np.float64) * s.reshape(-1, g, 1).astype(np.float64) + z.reshape(-1, g, 1).astype(np.float64)
+            out.append(m.reshape(-1, m.shape[-1] if m.ndim == 2 else g * 128).astype(np.float64))
+        return out
+
+    def mlp(x, e):
+        w13, w2 = dense(e)
+        y = x @ w13.T
+        gate, up = y[..., :y.shape[-1] // 2], y[..., y.shape[-1] // 2:]
+        return (gate / (1 + np.exp(-gate)) * up) @ w2.T
+
+    x = hidden.numpy().astype(np.float64)
+    want = mlp(x, 6)
+    for t in range(tokens):
+        for k in range(2):
+            if 0 <= int(ids[t, k]) < 6:
+                want[t] += float(w[t, k]) * mlp(x[t], int(ids[t, k]))
+    assert np.linalg.norm(got - want) <= 2.0 ** -9 * np.linalg.norm(want)
+
+
+def test_lists_that_the_few_token_tiles_take():
+    """fp16 problems up to 12 rows on average, with 8-bit weights among them up to 6; a K or N that the tiles' blocks do not divide, more than 64 rows and few blocks of channels go where they went."""
+    from mxmoe_amd import _lib
+
+    lib = _lib.load()
+    fp, w8, w4 = FP16, W8A16, (16, 4, 128, False)
+
+    def picked(*probs):
+        sizes = (_lib.Dim3 * len(probs))(*[_lib.Dim3(*p[:3]) for p in probs])
+        qs = (_lib.QParams * len(probs))(*[_lib.QParams(p[3][0], p[3][1], p[3][2], int(p[3][3])) for p in probs])
+        rc = lib.mxmoe_group_gemm_plan(-1, sizes, qs, len(probs), None, None)
+        assert rc >= 1000, lib.mxmoe_last_error()
+        return lib.mxmoe_kernel_name(rc - 1000).decode().split("groupgemm_hz_fused_")[-1]
+
+    assert picked((12, 2816, 2048, fp)) == "a16_few" and picked((13, 2816, 2048, fp)) == "fp16"
+    assert picked((1, 2816, 2048, fp), (23, 2816, 2048, fp)) == "fp16"          # (more than a quarter of the problems exceed a row tile)
+    assert picked((6, 2816, 2048, fp), (6, 2816, 2048, w8)) == "a16_few" and picked((6, 2816, 2048, fp), (7, 2816, 2048, w8)) == "all"
+    assert picked((6, 2816, 2048, w8)) == "a16_few" and picked((7, 2816, 2048, w8)) == "all"
+    assert picked((6, 2816, 2048, w8), (6, 2816, 2048, w4)) == "a16_few" and picked((6, 2816, 2048, w4)) == "wo_few"
+    assert picked((4, 2816, 2080, fp)) == "fp16" and picked((4, 2824, 2048, fp)) == "fp16"
+    assert picked((4, 2816, 2080, fp), (4, 2816, 2048, w8)) == "all" and picked((0, 2816, 2080, fp), (4, 2816, 2048, fp)) == "a16_few"
+    assert picked((1, 1792, 2048, fp)) == "fp16" and picked((1, 2048, 2048, fp)) == "a16_few"
+    assert picked(*[(4, 2816, 2048, fp)] * 20, (65, 2816, 2048, fp)) == "fp16"
