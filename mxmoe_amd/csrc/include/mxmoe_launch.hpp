@@ -468,6 +468,12 @@ struct PlanBranch {
 // and share nothing but a few rows of activations with their neighbours.
 __host__ __device__ inline bool flat_phase(const PlanBranch& b) { return b.BM <= 16 || (is_weight_only((Fmt)b.fmt) && b.BM < 128); }
 // Tiles of size 2^lg that cover `x`.
+// Whether the tiles of a shape's problems above the launch's smallest K (a shared expert's second block, two or four times as long as the routed experts') are a phase of their own,
+// so that every XCD gets an eighth of them as well as of the others.  In one phase the XCDs get equal numbers of tiles, and the first of them all the long ones, which the launch then
+// waited for while half of the chip was idle (a second block of 64 experts and a shared one of twice their width, 2049 tokens: CUs busy 0.52 of the time, 173 us).  Layers, us, one phase / two: 64 experts
+// top-6 and a shared one, 2049 tokens, w4a16 385 / 332, w4a4 and w8a8 267 / 259; 60 experts top-4 and one four times as wide, w4a4 and w8a8 64 tokens 112 / 103, 2049 tokens 283 / 259, w4a16 / w3a16
+// 442 / 339, 8192 tokens 1375 / 1051; up to 2% either way between 128 and 512 tokens.
+__host__ __device__ inline bool long_phase(const PlanBranch& b, int long_tiles, int other_tiles) { return long_tiles > 0 && other_tiles > 0 && !flat_phase(b); }
 __host__ __device__ inline int tiles_over(int x, int lg) { return (x + (1 << lg) - 1) >> lg; }
 constexpr int kNumFmts = (int)Fmt::UNSUPPORTED;
 struct PlanInfo {
@@ -478,6 +484,7 @@ struct PlanInfo {
   // A 128 x 256 tile that has a 128 x 128 one for launches of few tiles (kSlimTiles): branches, and whether there is such a pair of shapes.  The slim one stands behind
   // the formats' branches in b: problems are planned without it.
   int wide, slim, has_slim;
+  int unequal_k;  // (the device planner's) the experts of the block differ in K
   uint8_t order[kMaxBranches];  // positions in b, most expensive tile first (branch_cost); ties keep the registration order
   uint8_t fmt_start[kNumFmts + 4];
   // by format, in registration order inside a format: those of format f are b[fmt_start[f]] .. b[fmt_start[f + 1] - 1], and the planners
@@ -1076,14 +1083,16 @@ inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, c
   }
   // Most expensive tile shape first.  Inside a shape, the problems whose K is above the launch's smallest K go first (their tiles
   // run longest: a shared expert with a wider intermediate, say; workgroups are dispatched in index order, and the longest
-  // jobs first is what keeps the tail of the launch short), then the others; problems keep their order otherwise (neighbouring tiles
+  // jobs first is what keeps the tail of the launch short), then the others, as a phase of their own (long_phase); problems keep their order otherwise (neighbouring tiles
   // share operands).
   int total = 0, ne = 0, wg = 0, np = 0;
   for (int oi = 0; oi < pi.nb; ++oi) {
     const PlanBranch& pb = pi.b[pi.order[oi]];
     const int b = pb.index;
     const int tile0 = total;
-    for (int pass = 0; pass < 2; ++pass)
+    int rest0 = total;  // first tile of the problems of the smallest K
+    for (int pass = 0; pass < 2; ++pass) {
+      if (pass == 1) rest0 = total;
       for (int ei = 0; ei < nent; ++ei) {
         const Entry& en = entries[ei];
         if (en.phase_branch != b || en.tiles == 0 || ((int)h_sizes[base + en.problem].z > scope.kmin) != (pass == 0)) continue;
@@ -1091,16 +1100,21 @@ inline int build_fused_tables(const FusedKernel& k, const mxmoe_dim3* h_sizes, c
         total += en.tiles;
         ++ne;
       }
-    if (total == tile0) continue;
-    // shapes beyond the phase table share the last phase (their relative order is kept)
-    if (np < kMaxPhases) {
-      a.phase_tile0[np] = tile0;
-      a.phase_wg0[np] = wg;
-      if (flat_phase(pb)) a.phase_flat |= 1 << np;
-      ++np;
     }
-    const int p0 = a.phase_tile0[np - 1];
-    wg = a.phase_wg0[np - 1] + (total - p0 + kNumXcd - 1) / kNumXcd * kNumXcd;
+    if (total == tile0) continue;
+    const bool split = long_phase(pb, rest0 - tile0, total - rest0);
+    for (int part = 0; part < (split ? 2 : 1); ++part) {
+      const int first = part ? rest0 : tile0, last = split && part == 0 ? rest0 : total;
+      // phases beyond the table share its last one (their relative order is kept)
+      if (np < kMaxPhases) {
+        a.phase_tile0[np] = first;
+        a.phase_wg0[np] = wg;
+        if (flat_phase(pb)) a.phase_flat |= 1 << np;
+        ++np;
+      }
+      const int p0 = a.phase_tile0[np - 1];
+      wg = a.phase_wg0[np - 1] + (last - p0 + kNumXcd - 1) / kNumXcd * kNumXcd;
+    }
   }
   a.num_entries = ne;
   a.total_tiles = total;

@@ -2,6 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "../../../include/mxmoe_amd.h"
 #include "mxmoe_launch.hpp"
 #include "mxmoe_perm.hpp"
@@ -67,6 +69,7 @@ inline PlanInfo plan_info_of_block(const FusedKernel& k, const mxmoe_block_desc*
   }
   info.few_blocks = info.narrow && blocks <= kPoleBlocks;
   if (!w8a16) info.has_slim = 0;  // (nothing to look for)
+  for (int i = 1; i < et; ++i) info.unequal_k |= h_desc[i].K != h_desc[0].K;
   return info;
 }
 
@@ -80,6 +83,14 @@ struct PlanPair {
   int chunks;  // launches per block
   // Whether either block's tile shapes hang on its launch's totals (plan_block_body's TOTALS).
   bool totals() const { return p[0].info.may_pair || p[0].info.has_slim || p[1].info.may_pair || p[1].info.has_slim; }
+  // Whether either block's experts differ in K (its LONG).
+  bool longs() const { return p[0].info.unequal_k || p[1].info.unequal_k; }
+  // f(TOTALS, LONG) with both as types.
+  template <class F>
+  void with_body(F&& f) const {
+    if (totals()) longs() ? f(std::true_type{}, std::true_type{}) : f(std::true_type{}, std::false_type{});
+    else longs() ? f(std::false_type{}, std::true_type{}) : f(std::false_type{}, std::false_type{});
+  }
 };
 
 // One workgroup of two waves per launch, thread e = expert e0 + e of the launch's chunk of experts [e0, e0 + kMaxProblems) (the shared
@@ -117,7 +128,7 @@ __device__ __forceinline__ mxmoe_block_desc plan_block_prepare(const PlanParams&
   for (int i = e; i < (int)(sizeof(PlanInfo) / 4); i += kPlanThreads) reinterpret_cast<int*>(&sh.info)[i] = reinterpret_cast<const int*>(&p.info)[i];
   if (e < kMaxBranches) {
     sh.cnt[e][0] = sh.cnt[e][1] = sh.til[e][0] = sh.til[e][1] = 0;
-    sh.cnt_long[e][0] = sh.cnt_long[e][1] = sh.til_long[e][0] = sh.til_long[e][1] = 0;
+    sh.cnt_long[e][0] = sh.cnt_long[e][1] = sh.til_long[e][0] = sh.til_long[e][1] = 0;  // (LONG)
   }
   return d;
 }
@@ -128,7 +139,8 @@ __device__ __forceinline__ mxmoe_block_desc plan_block_prepare(const PlanParams&
 // TOTALS: with what a launch's totals decide, pairs of row segments and slim tiles.  In a body of its own, since a launch of few rows, which has neither, waits for the
 // fetching of that code even where a test skips it: layer_head_kernel, us, skipped by a test / without it: 1 token of 64 experts 7.9 / 7.2, 32 tokens 7.8 / 7.5, 8 tokens of 60
 // experts 8.9 / 8.4, 64 with a shared expert 9.7 / 8.7.
-template <bool TOTALS, class Count>
+// LONG: some experts' K differ (PlanInfo::unequal_k): without, no problem is long against the launch's others, and what looks for those is left out the same way.
+template <bool TOTALS, bool LONG, class Count>
 __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int chunk, const int chunks, const Count* recv, const mxmoe_block_desc& d, PlanShared& sh,
                                                 const bool active) {
   const int e0 = chunk * kMaxProblems;                       // first expert of this launch
@@ -200,8 +212,11 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
     }
     if (kind == LayerForm::kBehind) sum_before(4);
     // smallest K of the launch's problems with rows: those above it run first inside their branch (see build_fused_tables)
-    const int km = -wave_last(wave_inclusive_max(mine && rows > 0 ? -K : -0x7fffffff));
-    if (lane == 0) sh.kmin[wave] = km;
+    int km = K;
+    if constexpr (LONG) {
+      km = -wave_last(wave_inclusive_max(mine && rows > 0 ? -K : -0x7fffffff));
+      if (lane == 0) sh.kmin[wave] = km;
+    }
     // what this problem's tile shapes are, as far as the rest of the launch has no say in it, and the large tiles of the long problems
     // (launch_scope): whether one of K >= kLongK is above the launch's smallest is known behind the barrier
     have = mine ? plan_choose(info, fmt, (int)rows, N, choice) : 0;
@@ -214,26 +229,28 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
       const unsigned all = (unsigned)wave_last((int)wave_inclusive_scan(K == km ? tall : tall << 16));
       if (lane == 0) sh.tall[wave] = all;
     }
-    const int large = have > 0 && K >= kLongK ? choice.large_tiles : 0;
-    if (__ballot(large > 0) != 0) {
-      const int all = wave_last(wave_inclusive_scan(large)), at_km = wave_last(wave_inclusive_scan(K == km ? large : 0));
-      if (lane == 0) {
-        sh.long_tiles[wave] = all;
-        sh.long_tiles_kmin[wave] = at_km;
+    if constexpr (LONG) {
+      const int large = have > 0 && K >= kLongK ? choice.large_tiles : 0;
+      if (__ballot(large > 0) != 0) {
+        const int all = wave_last(wave_inclusive_scan(large)), at_km = wave_last(wave_inclusive_scan(K == km ? large : 0));
+        if (lane == 0) {
+          sh.long_tiles[wave] = all;
+          sh.long_tiles_kmin[wave] = at_km;
+        }
+      } else if (lane == 0) {
+        sh.long_tiles[wave] = sh.long_tiles_kmin[wave] = 0;
       }
-    } else if (lane == 0) {
-      sh.long_tiles[wave] = sh.long_tiles_kmin[wave] = 0;
     }
   }
   __syncthreads();
-  const int kmin = min(sh.kmin[0], sh.kmin[1]);
-  const bool long_k = mine && K > kmin;
-  const int long_tiles = sh.long_tiles[0] - (sh.kmin[0] == kmin ? sh.long_tiles_kmin[0] : 0) + sh.long_tiles[1] - (sh.kmin[1] == kmin ? sh.long_tiles_kmin[1] : 0);
+  const int kmin = LONG ? min(sh.kmin[0], sh.kmin[1]) : K;
+  const bool long_k = LONG && mine && K > kmin;
+  const int long_tiles = !LONG ? 0 : sh.long_tiles[0] - (sh.kmin[0] == kmin ? sh.long_tiles_kmin[0] : 0) + sh.long_tiles[1] - (sh.kmin[1] == kmin ? sh.long_tiles_kmin[1] : 0);
   Segment sg[2];
   const int ns = have > 0 ? plan_split(info, fmt, (int)rows, N, choice, runs_long(K, kmin) ? min(long_tiles, kLongTiles) : info.few_blocks && integer_sums(fmt) ? choice.large_tiles : 0, sg) : 0;
   if (TOTALS && info.has_slim) {
     const unsigned t0 = sh.tall[0], t1 = sh.tall[1];
-    const int at_kmin = (int)((sh.kmin[0] == kmin ? t0 & 0xFFFF : 0) + (sh.kmin[1] == kmin ? t1 & 0xFFFF : 0));
+    const int at_kmin = (int)((!LONG || sh.kmin[0] == kmin ? t0 & 0xFFFF : 0) + (!LONG || sh.kmin[1] == kmin ? t1 & 0xFFFF : 0));
     const int all = (int)((t0 & 0xFFFF) + (t0 >> 16) + (t1 & 0xFFFF) + (t1 >> 16));
     take_slim_tiles(info, long_k ? all - at_kmin : at_kmin, (int)rows, N, K, sg, ns);
   }
@@ -255,9 +272,9 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
     // entries of this branch in this wave, long-K problems first: position = matching lanes that run earlier, first tile = their tiles
     const uint64_t has = __ballot(which >= 0);
     if (has == 0) continue;  // (most branches of a kernel are not used by a given launch: their counters stay zero)
-    const uint64_t has_long = __ballot(which >= 0 && long_k), two = __ballot(which >= 0 && pair);
-    const int inc_long = wave_inclusive_scan(long_k ? mine_tiles : 0), inc_rest = wave_inclusive_scan(long_k ? 0 : mine_tiles);
-    const int tt_long = wave_last(inc_long), tt = tt_long + wave_last(inc_rest);
+    const uint64_t has_long = LONG ? __ballot(which >= 0 && long_k) : 0, two = __ballot(which >= 0 && pair);
+    const int inc_long = LONG ? wave_inclusive_scan(long_k ? mine_tiles : 0) : 0, inc_rest = wave_inclusive_scan(long_k ? 0 : mine_tiles);
+    const int tt_long = LONG ? wave_last(inc_long) : 0, tt = tt_long + wave_last(inc_rest);
     const uint64_t before = (1ull << lane) - 1;
 #pragma unroll
     for (int j = 0; j < 2; ++j)
@@ -271,8 +288,10 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
     if (lane == 0) {
       sh.cnt[r][wave] = __popcll(has) + __popcll(two);
       sh.til[r][wave] = tt;
-      sh.cnt_long[r][wave] = __popcll(has_long) + __popcll(has_long & two);
-      sh.til_long[r][wave] = tt_long;
+      if (LONG) {
+        sh.cnt_long[r][wave] = __popcll(has_long) + __popcll(has_long & two);
+        sh.til_long[r][wave] = tt_long;
+      }
     }
   }
   if (pair) {
@@ -311,6 +330,7 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
   }
   // Branches in run order, one per lane (both waves hold the same): entries and tiles before each.
   const int b_til = lane < info.nb ? sh.til[lane][0] + sh.til[lane][1] : 0, b_cnt = lane < info.nb ? sh.cnt[lane][0] + sh.cnt[lane][1] : 0;
+  const int t_long = LONG && lane < info.nb ? sh.til_long[lane][0] + sh.til_long[lane][1] : 0;
   const int til_inc = wave_inclusive_scan(b_til), cnt_inc = wave_inclusive_scan(b_cnt);
   const int total = wave_last(til_inc), ne = wave_last(cnt_inc);
   const int tile0 = til_inc - b_til, ent0 = cnt_inc - b_cnt;
@@ -326,32 +346,48 @@ __device__ __forceinline__ void plan_block_body(const PlanParams& p, const int c
           first += sh.til_long[r][0];
         }
       } else {
-        pos += sh.cnt_long[r][0] + sh.cnt_long[r][1];
-        first += sh.til_long[r][0] + sh.til_long[r][1];
+        if (LONG) {
+          pos += sh.cnt_long[r][0] + sh.cnt_long[r][1];
+          first += sh.til_long[r][0] + sh.til_long[r][1];
+        }
         if (wave == 1) {
-          pos += sh.cnt[r][0] - sh.cnt_long[r][0];
-          first += sh.til[r][0] - sh.til_long[r][0];
+          pos += sh.cnt[r][0] - (LONG ? sh.cnt_long[r][0] : 0);
+          first += sh.til[r][0] - (LONG ? sh.til_long[r][0] : 0);
         }
       }
       fa->entry[pos] = FusedArgs::Entry{first, sg[j].row0, sg[j].rows, (int)((unsigned)(e | (sg[j].branch << 16)) | pair | (pair && j ? kPairSecond : 0u))};  // problem index relative to the launch's first
     }
   }
   if (wave == 0) {
-    // Phases: every branch with tiles is one, in run order; shapes beyond the phase table share the last phase.
-    const uint64_t live = __ballot(b_til > 0);
-    const int ord = __popcll(live & ((1ull << lane) - 1)), np = min(__popcll(live), kMaxPhases);
-    const bool starts = b_til > 0 && ord < kMaxPhases;
-    // workgroups of the phases that are one branch (all that may have a successor)
-    const int padded = b_til > 0 && ord < kMaxPhases - 1 ? (b_til + kNumXcd - 1) / kNumXcd * kNumXcd : 0;
-    const int wg0 = wave_inclusive_scan(padded) - padded;
-    const int flat = wave_last(wave_inclusive_scan(starts && flat_phase(my_branch) ? 1 << ord : 0));
-    if (starts) {
-      fa->phase_tile0[ord] = tile0;
-      fa->phase_wg0[ord] = wg0;
-      if (ord == np - 1) {  // the last phase: up to the last tile
-        fa->phase_tile0[np] = total;
-        fa->phase_wg0[np] = wg0 + (total - tile0 + kNumXcd - 1) / kNumXcd * kNumXcd;
+    // Phases: every branch with tiles is one, or two (long_phase), in run order; those beyond the phase table share the last phase.
+    const bool split = LONG && long_phase(my_branch, t_long, b_til - t_long);
+    const uint64_t live = __ballot(b_til > 0), twice = LONG ? __ballot(split) : 0, lower = (1ull << lane) - 1;
+    int ord = __popcll(live & lower), np = __popcll(live);
+    int head_tiles = b_til, padded1 = 0;  // tiles of a branch's first phase; workgroups of its second
+    if (LONG && twice) {                  // (a branch around code that most launches would fetch for nothing)
+      ord += __popcll(twice & lower);
+      np += __popcll(twice);
+      if (split) {
+        head_tiles = t_long;
+        padded1 = ord + 1 < kMaxPhases - 1 ? (b_til - t_long + kNumXcd - 1) / kNumXcd * kNumXcd : 0;
       }
+    }
+    np = min(np, kMaxPhases);
+    // workgroups of the phases that have a successor in the table
+    const int padded0 = b_til > 0 && ord < kMaxPhases - 1 ? (head_tiles + kNumXcd - 1) / kNumXcd * kNumXcd : 0;
+    const int wg0 = wave_inclusive_scan(padded0 + padded1) - padded0 - padded1;
+    const int flat = wave_last(wave_inclusive_scan(b_til > 0 && ord < kMaxPhases && flat_phase(my_branch) ? 1 << ord : 0));
+    auto begin = [&](int o, int first, int wg) {
+      fa->phase_tile0[o] = first;
+      fa->phase_wg0[o] = wg;
+      if (o == np - 1) {  // the last phase: up to the last tile
+        fa->phase_tile0[np] = total;
+        fa->phase_wg0[np] = wg + (total - first + kNumXcd - 1) / kNumXcd * kNumXcd;
+      }
+    };
+    if (b_til > 0 && ord < kMaxPhases) begin(ord, tile0, wg0);
+    if (LONG && twice) {
+      if (split && ord + 1 < kMaxPhases) begin(ord + 1, tile0 + t_long, wg0 + padded0);
     }
     if (lane == 0) {
       // rows routed: those of every launch without the shared expert's; the last launch knows them all

@@ -237,7 +237,7 @@ __device__ __forceinline__ void head_token(const HeadArgs& a, int t, int lane) {
 }
 
 // Workgroups: planning first (the longest chain of dependent steps), then the permutation's entries, then tokens, one per wave.
-template <int NI, int TH, bool TOTALS>
+template <int NI, int TH, bool TOTALS, bool LONG>
 __global__ void __launch_bounds__(TH) layer_head_kernel(const HeadArgs a, const PlanPair pair) {
   extern __shared__ __align__(16) int32_t head_lds[];
   const int plan_wgs = 2 * pair.chunks;
@@ -260,7 +260,7 @@ __global__ void __launch_bounds__(TH) layer_head_kernel(const HeadArgs a, const 
     } else {
       count_ids<TH>(a.ids, a.total, a.E, 0, nullptr, head_lds, head_lds + a.E);
     }
-    plan_block_body<TOTALS>(p, chunk, pair.chunks, head_lds, d, sh, plans);
+    plan_block_body<TOTALS, LONG>(p, chunk, pair.chunks, head_lds, d, sh, plans);
     return;
   }
   wg -= plan_wgs;
@@ -461,11 +461,13 @@ int mxmoe_layer_run(const void* handle, const void* hidden, const int32_t* topk_
   if (h.hist) launch_perm_hist(topk_ids, h.total, h.E, const_cast<int32_t*>(h.hist), true, s);
   const dim3 grid(2 * pair.chunks + h.perm_wgs + f.token_wgs), block(f.threads);
   const size_t lds = (size_t)(2 + f.threads / 64 + 2 * kCountCopies) * h.E * sizeof(int32_t);
-  const bool totals = pair.totals();
   auto head = [&](auto ni) {
     constexpr int NI = decltype(ni)::value;
-    if (f.threads == kHeadSmall) hipLaunchKernelGGL((totals ? layer_head_kernel<NI, kHeadSmall, true> : layer_head_kernel<NI, kHeadSmall, false>), grid, block, lds, s, h, pair);
-    else hipLaunchKernelGGL((totals ? layer_head_kernel<NI, kHeadLarge, true> : layer_head_kernel<NI, kHeadLarge, false>), grid, block, lds, s, h, pair);
+    pair.with_body([&](auto totals, auto longs) {
+      constexpr bool kTotals = decltype(totals)::value, kLong = decltype(longs)::value;
+      if (f.threads == kHeadSmall) hipLaunchKernelGGL((layer_head_kernel<NI, kHeadSmall, kTotals, kLong>), grid, block, lds, s, h, pair);
+      else hipLaunchKernelGGL((layer_head_kernel<NI, kHeadLarge, kTotals, kLong>), grid, block, lds, s, h, pair);
+    });
   };
   switch (d.hidden / 512) {
     case 1: head(std::integral_constant<int, 1>{}); break;

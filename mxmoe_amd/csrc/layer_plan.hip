@@ -16,14 +16,14 @@
 
 namespace mxmoe {
 
-template <bool TOTALS>
+template <bool TOTALS, bool LONG>
 __global__ void __launch_bounds__(kPlanThreads) plan_block_kernel(const PlanPair pair) {
   // one workgroup per launch of each block of the layer (gate_up, down): all only read the counts
   __shared__ PlanShared sh;
   const PlanParams& p = pair.p[blockIdx.x / pair.chunks];
   const mxmoe_block_desc d = plan_block_prepare(p, blockIdx.x % pair.chunks, sh);
   __syncthreads();
-  plan_block_body<TOTALS>(p, blockIdx.x % pair.chunks, pair.chunks, pair.p[0].recv, d, sh, true);
+  plan_block_body<TOTALS, LONG>(p, blockIdx.x % pair.chunks, pair.chunks, pair.p[0].recv, d, sh, true);
 }
 
 // Permutation and planning of a decode-sized batch (at most kPermChunk (token, slot) entries) in ONE launch: workgroup 0 builds the
@@ -38,7 +38,7 @@ struct PermSmallArgs {
   int64_t* slot;
   int32_t* row_of_slot;
 };
-template <bool TOTALS>
+template <bool TOTALS, bool LONG>
 __global__ void __launch_bounds__(kPlanThreads) perm_plan_small_kernel(const PermSmallArgs a, const PlanPair pair) {
   extern __shared__ __align__(8) uint8_t pp_lds[];  // E int32 counters (workgroup 0) or E int64 counts (planning workgroups)
   if (blockIdx.x == 0) {
@@ -57,7 +57,7 @@ __global__ void __launch_bounds__(kPlanThreads) perm_plan_small_kernel(const Per
     if (e >= 0 && e < a.E) atomicAdd(&cnt[e], 1ull);
   }
   __syncthreads();
-  plan_block_body<TOTALS>(pair.p[b / pair.chunks], chunk, pair.chunks, counts, d, sh, true);
+  plan_block_body<TOTALS, LONG>(pair.p[b / pair.chunks], chunk, pair.chunks, counts, d, sh, true);
 }
 
 // The same for larger batches, after perm_hist_kernel has counted the experts per chunk of kPermChunk entries: the first `blocks`
@@ -74,7 +74,7 @@ struct PermScatterArgs {
   int64_t* slot;
   int32_t* row_of_slot;
 };
-template <bool TOTALS>
+template <bool TOTALS, bool LONG>
 __global__ void __launch_bounds__(kPlanThreads) perm_scatter_plan_kernel(const PermScatterArgs a, const PlanPair pair) {
   extern __shared__ __align__(8) uint8_t pp_lds[];  // E int32 ranks (scatter workgroups) or E int64 counts (planning workgroups)
   if ((int)blockIdx.x < a.blocks) {
@@ -92,7 +92,7 @@ __global__ void __launch_bounds__(kPlanThreads) perm_scatter_plan_kernel(const P
     counts[e] = v;
   }
   __syncthreads();
-  plan_block_body<TOTALS>(pair.p[b / pair.chunks], chunk, pair.chunks, counts, d, sh, true);
+  plan_block_body<TOTALS, LONG>(pair.p[b / pair.chunks], chunk, pair.chunks, counts, d, sh, true);
 }
 
 // Whether a kernel has a tile for the format and operand layout of every block.
@@ -311,7 +311,7 @@ static int fill_plan_params(PlanParams& p, int kernel_id, const int64_t* d_recv,
 
 static int launch_plan(PlanPair& pair, int blocks, void* stream) {
   pair.chunks = PlanLayout(pair.p[0].Et).chunks;
-  hipLaunchKernelGGL((pair.totals() ? plan_block_kernel<true> : plan_block_kernel<false>), dim3(blocks * pair.chunks), dim3(kPlanThreads), 0, (hipStream_t)stream, pair);
+  pair.with_body([&](auto totals, auto longs) { hipLaunchKernelGGL((plan_block_kernel<decltype(totals)::value, decltype(longs)::value>), dim3(blocks * pair.chunks), dim3(kPlanThreads), 0, (hipStream_t)stream, pair); });
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     last_error() = std::string("kernel launch failed: ") + hipGetErrorString(e);
@@ -374,7 +374,7 @@ int mxmoe_permute_plan_layer(const int32_t* topk_ids, int num_tokens, int topk, 
   a.perm = perm_indices;
   a.slot = src_slot;
   a.row_of_slot = row_of_slot;
-  hipLaunchKernelGGL((pair.totals() ? perm_plan_small_kernel<true> : perm_plan_small_kernel<false>), dim3(1 + 2 * pair.chunks), dim3(kPlanThreads), (size_t)num_experts * 8, (hipStream_t)stream, a, pair);
+  pair.with_body([&](auto totals, auto longs) { hipLaunchKernelGGL((perm_plan_small_kernel<decltype(totals)::value, decltype(longs)::value>), dim3(1 + 2 * pair.chunks), dim3(kPlanThreads), (size_t)num_experts * 8, (hipStream_t)stream, a, pair); });
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     last_error() = std::string("kernel launch failed: ") + hipGetErrorString(e);
@@ -426,7 +426,7 @@ int mxmoe_permute_plan_layer_ws(const int32_t* topk_ids, int num_tokens, int top
   a.slot = src_slot;
   a.row_of_slot = row_of_slot;
   launch_perm_hist(topk_ids, a.total, num_experts, reinterpret_cast<int32_t*>(workspace), true, (hipStream_t)stream);
-  hipLaunchKernelGGL((pair.totals() ? perm_scatter_plan_kernel<true> : perm_scatter_plan_kernel<false>), dim3(a.blocks + 2 * pair.chunks), dim3(kPlanThreads), (size_t)num_experts * 8, (hipStream_t)stream, a, pair);
+  pair.with_body([&](auto totals, auto longs) { hipLaunchKernelGGL((perm_scatter_plan_kernel<decltype(totals)::value, decltype(longs)::value>), dim3(a.blocks + 2 * pair.chunks), dim3(kPlanThreads), (size_t)num_experts * 8, (hipStream_t)stream, a, pair); });
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     last_error() = std::string("kernel launch failed: ") + hipGetErrorString(e);

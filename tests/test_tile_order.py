@@ -174,3 +174,29 @@ def test_kernels_for_few_rows_make_no_pairs(lib, kernel, q):
     """More rows than such a kernel is chosen for: its two shapes one after the other."""
     tab, _ = _launch(lib, [(96, 28672, 4096, q)] * 12, lib.mxmoe_find_kernel(kernel.encode()))
     assert tab[2] == 2 and not _pairs(tab)
+
+
+@pytest.mark.parametrize("q,rows,shared,k", [(W8, 546, 8192, 5632), (WO, 192, 2049, 2816), (FP, 120, 1788, 5632), (W4, 4, 64, 5632)])
+def test_tiles_of_a_long_problem_are_spread_over_the_xcds(lib, q, rows, shared, k):
+    """A problem of two and four times the others' K: every XCD (workgroup w runs on XCD w mod 8) gets an eighth of its tiles of every shape, give or take one, and they run before the
+    others of their shape; every tile is run once."""
+    probs = [(rows, 2048, 1408, q)] * 60 + [(shared, 2048, k, q)]
+    tab, area = _launch(lib, probs)
+    long_of = [area[x::8] for x in range(8)]
+    for shape in {(r1 - r0, c1 - c0) for p, r0, r1, c0, c1 in area if p == 60}:
+        counts = [sum(1 for p, r0, r1, c0, c1 in a if p == 60 and (r1 - r0, c1 - c0) == shape) for a in long_of]
+        assert max(counts) - min(counts) <= -(-sum(counts) // 8), (shape, counts)
+        assert sum(counts) < 16 or min(counts) > 0, (shape, counts)
+    live = area[area[:, 0] >= 0]
+    for p, (m, n, *_r) in enumerate(probs):
+        assert (live[live[:, 0] == p][:, [2, 4]] - live[live[:, 0] == p][:, [1, 3]]).prod(axis=1).sum() == m * n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmts", [[W8], [WO, W4], [W4, W8, FP, WO, WO8, (4, 4, 128, True), (16, 3, 128, False), (16, 2, 128, False)]])
+@pytest.mark.parametrize("long_k", [2816, 256])
+def test_device_planner_makes_the_same_phases(lib, fmts, long_k):
+    """Problems of two lengths in one, two and eight formats: more phases than the table holds, most of the problems long or a few of them."""
+    e = 96
+    counts = [(150, 0, 40, 7, 300)[i % 5] for i in range(e)]
+    _device_plan_is_the_hosts(lib, [fmts[i % len(fmts)] for i in range(e)], counts, 2048, [long_k if i % 9 == 4 else 1408 for i in range(e)])
