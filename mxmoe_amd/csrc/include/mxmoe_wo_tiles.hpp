@@ -413,6 +413,14 @@ struct SkinnyWoTile {
 
   template <bool GU>
   __device__ static __forceinline__ void run(const TileArgs& t, uint8_t* __restrict__ smem) {
+    run_rows<GU>(t, smem, [&](int m) {
+      if constexpr (GU) return gload<int>(t.rows + m);
+      else return m;
+    });
+  }
+  // `row_of(m)`: the row of A behind row m of the problem.
+  template <bool GU, class RowOf>
+  __device__ static __forceinline__ void run_rows(const TileArgs& t, uint8_t* __restrict__ smem, RowOf&& row_of) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -424,11 +432,7 @@ struct SkinnyWoTile {
     const int nbv = min(NBO, (N - n0) / 16);  // output channel blocks of this tile that exist
     int src[MB];
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      const int m = min(m0 + mb * 16 + lm, M - 1);
-      if constexpr (GU) src[mb] = gload<int>(t.rows + m);
-      else src[mb] = m;
-    }
+    for (int mb = 0; mb < MB; ++mb) src[mb] = row_of(min(m0 + mb * 16 + lm, M - 1));
 
     // the K range is dealt to the 4 waves in contiguous quarters; each wave sums its quarter for every channel of the tile
     const int KW = (KB + kWaves - 1) / kWaves;

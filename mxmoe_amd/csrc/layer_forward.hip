@@ -1,4 +1,4 @@
-// The planned layer forward in its short form: four or five launches from (hidden, expert ids, weights) to the layer's output.
+// The planned layer forward in its short form: three to five launches from (hidden, expert ids, weights) to the layer's output.
 //
 //   head      permutation by expert, the tables of both GroupGEMMs, and every token quantised once per activation format: three
 //             jobs that need nothing of each other, in one launch;
@@ -6,6 +6,8 @@
 //   rows      rotation + quantisation of those rows for the second block (left out when every second block reads fp16 rows);
 //   down      the fused GroupGEMM of the second block;
 //   combine   un-permute, top-k weighted sum, shared expert.
+//
+// A few tokens of a layer whose first blocks take them as they are (16-bit activations) need no head: layer_first_kernel.
 //
 // Against the form that writes an activation row per destination (top-k of them per token, after the permutation is known) and stores
 // gate and up: the head is one launch instead of two or three in sequence, activations take 1 / top-k of the space, and 8 bytes per
@@ -236,6 +238,27 @@ __device__ __forceinline__ void head_token(const HeadArgs& a, int t, int lane) {
   }
 }
 
+// The tables of launch `wg` of both blocks' launches, from the ids (or from counts per chunk of them).
+template <int TH, bool TOTALS, bool LONG>
+__device__ __forceinline__ void head_plan(const HeadArgs& a, const PlanPair& pair, int wg, PlanShared& sh, int32_t* lds) {
+  const PlanParams& p = pair.p[wg / pair.chunks];
+  const int chunk = wg % pair.chunks;
+  mxmoe_block_desc d{};
+  const bool plans = __builtin_amdgcn_readfirstlane(threadIdx.x) < kPlanThreads;
+  if (plans) d = plan_block_prepare(p, chunk, sh);
+  if (a.hist) {
+    for (int e = threadIdx.x; e < a.E; e += TH) {
+      int v, before;
+      perm_hist_row_sums(a.hist + (long)e * perm_hist_stride(a.chunks), a.chunks, 0, &v, &before);
+      lds[e] = v;
+    }
+    __syncthreads();
+  } else {
+    count_ids<TH>(a.ids, a.total, a.E, 0, nullptr, lds, lds + a.E);
+  }
+  plan_block_body<TOTALS, LONG>(p, chunk, pair.chunks, lds, d, sh, plans);
+}
+
 // Workgroups: planning first (the longest chain of dependent steps), then the permutation's entries, then tokens, one per wave.
 template <int NI, int TH, bool TOTALS, bool LONG>
 __global__ void __launch_bounds__(TH) layer_head_kernel(const HeadArgs a, const PlanPair pair) {
@@ -245,22 +268,7 @@ __global__ void __launch_bounds__(TH) layer_head_kernel(const HeadArgs a, const 
   if (wg < plan_wgs) {
     __builtin_amdgcn_s_setprio(3);  // one chain of dependent steps against the token waves' full issue slots on the same SIMDs
     __shared__ PlanShared sh;
-    const PlanParams& p = pair.p[wg / pair.chunks];
-    const int chunk = wg % pair.chunks;
-    mxmoe_block_desc d{};
-    const bool plans = __builtin_amdgcn_readfirstlane(threadIdx.x) < kPlanThreads;
-    if (plans) d = plan_block_prepare(p, chunk, sh);
-    if (a.hist) {
-      for (int e = threadIdx.x; e < a.E; e += TH) {
-        int v, before;
-        perm_hist_row_sums(a.hist + (long)e * perm_hist_stride(a.chunks), a.chunks, 0, &v, &before);
-        head_lds[e] = v;
-      }
-      __syncthreads();
-    } else {
-      count_ids<TH>(a.ids, a.total, a.E, 0, nullptr, head_lds, head_lds + a.E);
-    }
-    plan_block_body<TOTALS, LONG>(p, chunk, pair.chunks, head_lds, d, sh, plans);
+    head_plan<TH, TOTALS, LONG>(a, pair, wg, sh, head_lds);
     return;
   }
   wg -= plan_wgs;
@@ -276,6 +284,133 @@ __global__ void __launch_bounds__(TH) layer_head_kernel(const HeadArgs a, const 
   for (int t = wg * (TH / 64) + wave; t < a.T; t += token_wgs * (TH / 64)) head_token<NI>(a, t, lane);
 }
 
+// Few tokens, first blocks of 16-bit activations: there is nothing to quantise in front of gate_up, and a workgroup finds its problem from the ids itself, so that the launch waits for no
+// head.  The permutation and the tables of both blocks, which the launches behind need, are made beside it by the first workgroups.  Grid: (column tiles of a routed expert) x (1 for those,
+// shared_slots rows of the shared expert's tiles, one row per expert that may have tokens).  A workgroup counts the ids in LDS, takes the slot-th expert with rows, lists its
+// rows, and runs their 16-row tiles one after the other (with 256 ids an expert of more than 16 rows is rare but under a skewed routing, and its weights come from L2 then).
+// What a launch of few tokens consists of is latency: a layer's, with the head in front -> without, us: 64 experts top-6 and a shared one, w4a16 / w3a16, 29 -> 22 (1 token), 54 -> 46 (8),
+// 77 -> 71 (32), w8a16 / w2a16 31 -> 23 (1), 65 -> 54 (8), 96 -> 85 (32); 60 experts top-4, w4a16 24 -> 18 (1), 55 -> 49 (16), 72 -> 68 (64), skewed 68 -> 64 (64), fp16 35 -> 27 (1),
+// 108 -> 99 (8), 217 -> 212 (64); 8 experts of N = 28 672 / 4096, w4a16 64 -> 58 (1), 134 -> 126 (16).  One id per thread: up to 256 of them, and no more tokens than the kernels for few rows take.
+constexpr int kDirectTokens = 64, kDirectEntries = kHeadSmall;
+struct DirectArgs {
+  const mxmoe_block_desc* desc;
+  const uint8_t* hidden;
+  _Float16* act;
+  int hidden_size, inter, inter_shared;
+  int cols, shared_rows, shared_slots;  // column tiles of a routed expert; rows of the grid that hold a row tile's column tiles of the shared expert, and all of its row tiles'
+  unsigned topk_inverse;  // ceil(2^16 / top-k): (i * topk_inverse) >> 16 = i / top-k for i < kDirectEntries and top-k <= 64
+  int tile_lds;           // bytes of LDS that the tiles use
+};
+constexpr size_t direct_lds(int E) { return (size_t)kDirectEntries * 4 + kWaves * kDirectEntries + (size_t)E * 4; }
+
+template <bool LONG, class... Tiles>
+__global__ void __launch_bounds__(kThreads, kWavesPerSimd<Tiles...>) layer_first_kernel(const HeadArgs a, const PlanPair pair, const DirectArgs x) {
+  static_assert(kThreads == kHeadSmall && ((Tiles::MB == 1 && Tiles::BN == 64) && ...), "one id per thread; 16 rows, 32 outputs a tile");
+  extern __shared__ __align__(16) uint8_t first_lds[];
+  const int col0 = blockIdx.x, E = a.E;
+  int slot = (int)blockIdx.y - 1;
+  if (slot < 0) {
+    if (col0 < 2 * pair.chunks) {
+      __builtin_amdgcn_s_setprio(3);
+      constexpr size_t kPlanBytes = (sizeof(PlanShared) + 15) & ~(size_t)15;
+      head_plan<kHeadSmall, false, LONG>(a, pair, col0, *reinterpret_cast<PlanShared*>(first_lds), reinterpret_cast<int32_t*>(first_lds + kPlanBytes));
+    } else if (col0 == 2 * pair.chunks) {
+      __builtin_amdgcn_s_setprio(2);
+      head_scatter<kHeadSmall>(a, 0, reinterpret_cast<int32_t*>(first_lds));
+    }
+    return;
+  }
+  const bool shared = slot < x.shared_slots;
+  int col = col0, shared_m0 = 0;
+  if (shared) {
+    int row = slot;
+    for (; row >= x.shared_rows; row -= x.shared_rows) shared_m0 += 16;
+    col += row * x.cols;
+  }
+  if (col0 >= x.cols || col * 32 >= (shared ? x.inter_shared : x.inter)) return;
+  slot -= x.shared_slots;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int32_t* const all_ids = reinterpret_cast<int32_t*>(first_lds + x.tile_lds);
+  uint8_t* const rows = reinterpret_cast<uint8_t*>(all_ids + kDirectEntries) + wave * kDirectEntries;  // this wave's copy of the problem's entries
+  int32_t* const count = all_ids + kDirectEntries + kWaves * kDirectEntries / 4;
+  const int id = (int)threadIdx.x < a.total ? gload<int>(a.ids + threadIdx.x) : -1;
+  for (int i = threadIdx.x; i < E; i += kThreads) count[i] = 0;
+  __syncthreads();
+  all_ids[threadIdx.x] = id;
+  if (id >= 0 && id < E) atomicAdd(count + id, 1);
+  __syncthreads();
+  int e = shared ? E : -1, before = 0;  // the problem's expert; rows of the experts before it
+  for (int x0 = 0; x0 < E; x0 += 64) {
+    const int c = x0 + lane < E ? count[x0 + lane] : 0;
+    const uint64_t hit = __ballot(c > 0);
+    const int hits = __popcll(hit);
+    uint64_t take = ~0ull;  // experts of these 64 in front of the problem's
+    if (!shared && slot < hits) {
+      const uint64_t it = __ballot(c > 0 && __popcll(hit & ((1ull << lane) - 1)) == slot);
+      e = x0 + __builtin_ctzll(it);
+      take = it - 1;
+    }
+    before += wave_last(wave_inclusive_scan((take >> lane & 1) ? c : 0));
+    if (!shared && e >= 0) break;
+    slot -= hits;
+  }
+  if (e < 0) return;  // (every wave of the workgroup has come to the same)
+  int M = 0;
+  if (shared) {
+    M = min(a.T, shared_m0 + 16);
+  } else {
+    for (int i0 = 0; i0 < a.total; i0 += 64) {
+      const bool mine = all_ids[i0 + lane] == e;
+      const uint64_t which = __ballot(mine);
+      if (mine) rows[M + __popcll(which & ((1ull << lane) - 1))] = (uint8_t)(i0 + lane);
+      M += __popcll(which);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  TileArgs t;
+  const mxmoe_block_desc* d = x.desc + e;
+  t.A = x.hidden;
+  t.B = reinterpret_cast<const uint8_t*>(cload(&d->B));
+  t.sa = nullptr;
+  t.sb = reinterpret_cast<const _Float16*>(cload(&d->scale_b));
+  t.C = x.act + (long)before * x.inter;
+  t.acc_dump = nullptr;
+  t.M = M;
+  t.N = 2 * (shared ? x.inter_shared : x.inter);
+  t.K = x.hidden_size;
+  t.row0 = 0;
+  t.tile_n = col;
+  t.rows = nullptr;
+  const int bits = cload(&d->q.w_bits);
+  auto token_of = [&](int m) { return shared ? m : (int)(rows[m] * x.topk_inverse >> 16); };
+  auto run = [&](auto type) {
+    using T = typename decltype(type)::type;
+    if (bits != T::WBITS) return;
+#pragma unroll 1
+    for (int m0 = shared_m0; m0 < M; m0 += T::BM) {
+      if (m0 > shared_m0) __syncthreads();  // the reduction behind the previous tile has been read
+      t.tile_m = m0 / T::BM;
+      T::template run_rows<true>(t, first_lds, token_of);
+    }
+  };
+  (run(TileType<Tiles>{}), ...);
+}
+
+// The same for the registered kernel of the layer's first block: those made of 16 x 64 tiles alone have one (the tile lists of groupgemm_hz_fused_wo_few and _a16_few).
+using LaunchFirstFn = void (*)(const HeadArgs&, const PlanPair&, const DirectArgs&, dim3, size_t, hipStream_t);
+template <class... Tiles>
+void launch_first(const HeadArgs& a, const PlanPair& pair, const DirectArgs& x, dim3 grid, size_t lds, hipStream_t s) {
+  if (pair.longs()) hipLaunchKernelGGL((layer_first_kernel<true, Tiles...>), grid, dim3(kThreads), lds, s, a, pair, x);
+  else hipLaunchKernelGGL((layer_first_kernel<false, Tiles...>), grid, dim3(kThreads), lds, s, a, pair, x);
+}
+static LaunchFirstFn first_launch_of(const FusedKernel& k) {
+  if (!only_narrow_few_token(k)) return nullptr;
+  for (const BranchInfo& b : k.branches)
+    if (b.fmt == Fmt::W8A16 || b.fmt == Fmt::FP16)
+      return &launch_first<SkinnyWoTile<4, 64, 1, 3>, SkinnyWoTile<3, 64, 1, 3>, SkinnyWoTile<2, 64, 1, 3>, SkinnyWoTile<8, 64, 1, 3>, SkinnyWoTile<16, 64, 1, 3>>;
+  return &launch_first<SkinnyWoTile<4, 64, 1, 3>, SkinnyWoTile<3, 64, 1, 3>, SkinnyWoTile<2, 64, 1, 3>>;
+}
+
 // What a layer keeps for one (tokens, top-k): its description and both launches' planning parameters.
 struct LayerForward {
   mxmoe_layer_desc d;
@@ -285,6 +420,10 @@ struct LayerForward {
   bool fp16_first;   // a first block reads the tokens as they are (its tiles load them straight into LDS)
   bool rows_step;    // a second block takes quantised (or rotated) rows
   RowsBehind rows;
+  LaunchFirstFn first;  // gate_up without a head in front of it, or null
+  DirectArgs direct;
+  dim3 first_grid;
+  size_t first_lds;
 };
 
 static int check_launch() {
@@ -416,6 +555,30 @@ int mxmoe_layer_create(const mxmoe_layer_desc* d, void** handle) {
   pd.form.kind = d->rotate == 2 ? LayerForm::kPlain : LayerForm::kBehind;
   pd.form.act = reinterpret_cast<const uint8_t*>(d->act);
 
+  // few tokens: no head (nothing is quantised in front of gate_up, its tables need no totals, and its workgroups fit the counters beside the tiles)
+  const FusedKernel& kg = registry()[f->d.kernel_gate_up];
+  bool plain = f->fp16_first && tags == 0 && !f->pair.totals() && h.T <= kDirectTokens && h.total <= kDirectEntries && d->topk <= 64;
+  for (int i = 0; i < et; ++i) {
+    const int n = i < d->num_experts ? d->inter : d->inter_shared;
+    plain = plain && (int)d->h_gate_up[i].N == 2 * n && (int)d->h_gate_up[i].K == d->hidden && n % 32 == 0;
+  }
+  f->first = plain ? first_launch_of(kg) : nullptr;
+  DirectArgs& x = f->direct;
+  x = DirectArgs{};
+  x.desc = d->d_gate_up;
+  x.act = reinterpret_cast<_Float16*>(d->act);
+  x.hidden_size = d->hidden;
+  x.inter = d->inter;
+  x.inter_shared = d->has_shared ? d->inter_shared : 0;
+  x.cols = d->inter / 32;
+  x.shared_rows = (x.inter_shared / 32 + x.cols - 1) / x.cols;
+  x.shared_slots = x.shared_rows * ((h.T + 15) / 16);
+  x.topk_inverse = (65536 + d->topk - 1) / d->topk;
+  x.tile_lds = kg.lds_bytes;
+  f->first_grid = dim3(std::max(x.cols, 2 * f->pair.chunks + 1), 1 + x.shared_slots + std::min(h.total, h.E));
+  f->first_lds = std::max(kg.lds_bytes + direct_lds(h.E), sizeof(PlanShared) + 16 + (size_t)(2 + kHeadSmall / 64 + 2 * kCountCopies) * h.E * sizeof(int32_t));
+  if (f->first_lds > 32 * 1024) f->first = nullptr;  // (counters of many experts would take the room of a workgroup)
+
   RowsBehind& r = f->rows;
   r = RowsBehind{};
   r.rows = d->act;
@@ -458,24 +621,7 @@ int mxmoe_layer_run(const void* handle, const void* hidden, const int32_t* topk_
   h.ids = topk_ids;
   h.hidden = reinterpret_cast<const _Float16*>(hidden);
   if (f.fp16_first) pair.p[0].form.store[0] = reinterpret_cast<const uint8_t*>(hidden);
-  if (h.hist) launch_perm_hist(topk_ids, h.total, h.E, const_cast<int32_t*>(h.hist), true, s);
-  const dim3 grid(2 * pair.chunks + h.perm_wgs + f.token_wgs), block(f.threads);
-  const size_t lds = (size_t)(2 + f.threads / 64 + 2 * kCountCopies) * h.E * sizeof(int32_t);
-  auto head = [&](auto ni) {
-    constexpr int NI = decltype(ni)::value;
-    pair.with_body([&](auto totals, auto longs) {
-      constexpr bool kTotals = decltype(totals)::value, kLong = decltype(longs)::value;
-      if (f.threads == kHeadSmall) hipLaunchKernelGGL((layer_head_kernel<NI, kHeadSmall, kTotals, kLong>), grid, block, lds, s, h, pair);
-      else hipLaunchKernelGGL((layer_head_kernel<NI, kHeadLarge, kTotals, kLong>), grid, block, lds, s, h, pair);
-    });
-  };
-  switch (d.hidden / 512) {
-    case 1: head(std::integral_constant<int, 1>{}); break;
-    case 2: head(std::integral_constant<int, 2>{}); break;
-    case 4: head(std::integral_constant<int, 4>{}); break;
-    default: head(std::integral_constant<int, 8>{}); break;
-  }
-  if (const int rc = check_launch()) return rc;
+  const FusedKernel &kg = registry()[d.kernel_gate_up], &kd = registry()[d.kernel_down];
   auto gemm = [&](LaunchPlannedFn fn, const FusedKernel& k, const void* plan, int launch_grid) {
     for (int c = 0; c < pair.chunks; ++c) {
       const hipError_t e = fn(reinterpret_cast<const FusedArgs*>(reinterpret_cast<const uint8_t*>(plan) + c * kFusedArgsStride), launch_grid, k.lds_bytes, s);
@@ -486,8 +632,32 @@ int mxmoe_layer_run(const void* handle, const void* hidden, const int32_t* topk_
     }
     return 0;
   };
-  const FusedKernel &kg = registry()[d.kernel_gate_up], &kd = registry()[d.kernel_down];
-  if (const int rc = gemm(kg.launch_gate_up, kg, d.plan_gate_up, d.grid_gate_up)) return rc;
+  if (f.first) {
+    DirectArgs x = f.direct;
+    x.hidden = reinterpret_cast<const uint8_t*>(hidden);
+    f.first(h, pair, x, f.first_grid, f.first_lds, s);
+    if (const int rc = check_launch()) return rc;
+  } else {
+    if (h.hist) launch_perm_hist(topk_ids, h.total, h.E, const_cast<int32_t*>(h.hist), true, s);
+    const dim3 grid(2 * pair.chunks + h.perm_wgs + f.token_wgs), block(f.threads);
+    const size_t lds = (size_t)(2 + f.threads / 64 + 2 * kCountCopies) * h.E * sizeof(int32_t);
+    auto head = [&](auto ni) {
+      constexpr int NI = decltype(ni)::value;
+      pair.with_body([&](auto totals, auto longs) {
+        constexpr bool kTotals = decltype(totals)::value, kLong = decltype(longs)::value;
+        if (f.threads == kHeadSmall) hipLaunchKernelGGL((layer_head_kernel<NI, kHeadSmall, kTotals, kLong>), grid, block, lds, s, h, pair);
+        else hipLaunchKernelGGL((layer_head_kernel<NI, kHeadLarge, kTotals, kLong>), grid, block, lds, s, h, pair);
+      });
+    };
+    switch (d.hidden / 512) {
+      case 1: head(std::integral_constant<int, 1>{}); break;
+      case 2: head(std::integral_constant<int, 2>{}); break;
+      case 4: head(std::integral_constant<int, 4>{}); break;
+      default: head(std::integral_constant<int, 8>{}); break;
+    }
+    if (const int rc = check_launch()) return rc;
+    if (const int rc = gemm(kg.launch_gate_up, kg, d.plan_gate_up, d.grid_gate_up)) return rc;
+  }
   if (f.rows_step)
     if (const int rc = quant_rows_behind(f.rows, s)) return rc;
   if (const int rc = gemm(kd.launch_planned, kd, d.plan_down, d.grid_down)) return rc;

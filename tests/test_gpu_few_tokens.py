@@ -110,3 +110,45 @@ def test_lists_that_the_few_token_tiles_take():
     assert picked((4, 2816, 2080, fp), (4, 2816, 2048, w8)) == "all" and picked((0, 2816, 2080, fp), (4, 2816, 2048, fp)) == "a16_few"
     assert picked((1, 1792, 2048, fp)) == "fp16" and picked((1, 2048, 2048, fp)) == "a16_few"
     assert picked(*[(4, 2816, 2048, fp)] * 20, (65, 2816, 2048, fp)) == "fp16"
+
+
+# tokens, top-k, experts, inter, shared experts, formats: one token; a partial row tile; 256 entries, the most; more experts than a wave has lanes and than one launch's tables hold;
+# two and four row tiles of the shared expert and of one expert; shared columns that end inside the grid's rows; quantised and rotated second blocks
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,topk,experts,inter,num_shared,mix", [
+    (1, 1, 8, 1408, 0, "fp16"), (1, 6, 64, 1408, 2, "wo"), (17, 3, 70, 96, 3, "fp16"), (33, 6, 130, 160, 1, "all"), (64, 4, 60, 256, 4, "wo"), (64, 4, 60, 352, 0, "all"),
+    (32, 8, 24, 1408, 1, "behind"), (5, 2, 66, 640, 2, "behind"), (16, 16, 8, 512, 1, "fp16"),
+])
+def test_first_launch_without_a_head(tokens, topk, experts, inter, num_shared, mix):
+    """gate_up that finds its problems from the ids, against the form with tables from launches in front on the same kernels: identical outputs.  Ids out of range,
+    one expert with most of the tokens, an expert twice in a token's list; a second call on other ids (nothing of the first is left); a misaligned view of the tokens."""
+    from mxmoe_amd import _lib, synth as S
+    from mxmoe_amd.layer import MxMoELayer
+
+    if inter % 128 and mix != "fp16":  # (their second block's K is in groups of 128)
+        mix = "first"
+    fm = {"fp16": [(FP16, FP16)], "wo": [(S.W4A16, S.W3A16), (S.W3A16, S.W2A16), (S.W2A16, S.W4A16)], "all": [(W8A16, FP16), (S.W4A16, W8A16), (FP16, S.W2A16)],
+          "first": [(W8A16, FP16), (S.W4A16, FP16), (S.W2A16, FP16)], "behind": [(S.W4A16, S.W4A4), (S.W3A16, S.W8A8), (S.W4A16, S.W4A16)]}[mix]
+    n = experts + (num_shared > 0)
+    cfg = S.MoEConfig("t", "test", experts, topk, 512, inter, tokens, num_shared=num_shared, rotate=int(mix == "behind"))
+    layer = MxMoELayer(cfg, formats=[fm[i % len(fm)] for i in range(n)])
+    kid = _lib.load().mxmoe_find_kernel(b"groupgemm_hz_fused_wo_few" if mix in ("wo", "behind") else b"groupgemm_hz_fused_a16_few")
+    planned = layer._planned_kernel
+    layer._planned_kernel = lambda h, t, k: kid if int(h[0].N) == 2 * inter else planned(h, t, k)
+    gen = torch.Generator().manual_seed(tokens)
+    store = torch.randn(tokens * 512 + 8, generator=gen).half().cuda()
+    calls = []
+    for call in range(3):
+        ids = torch.stack([torch.randperm(experts, generator=gen)[torch.arange(topk) % experts] for _ in range(tokens)]).to(torch.int32)
+        if tokens > 1:
+            ids[:, 0] = call
+            ids[0, -1], ids[tokens // 2, 0] = -1, experts + 3
+            ids[-1, -1] = ids[-1, 0]
+        w = torch.rand(tokens, topk, generator=gen)
+        off = 1 if call == 2 else 0
+        calls.append((store[off:off + tokens * 512].view(tokens, 512), ids.cuda(), w.cuda()))
+    got = [layer(*c).clone() for c in calls]
+    assert layer._short[(tokens, topk)] is not None
+    layer._short[(tokens, topk)] = None                                  # the form with launches in front
+    for c, g in zip(calls, got):
+        assert torch.equal(layer(*c), g)
