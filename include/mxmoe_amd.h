@@ -103,6 +103,10 @@ int mxmoe_last_status(void);
  * Host-only; used by the scheduler tests and the kernel-profile table.  Returns 1000 + kernel id on success. */
 int mxmoe_group_gemm_plan(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int problem_count, int32_t* branch_out, int32_t* tiles_out);
 
+/* The kernel that a list is better off on when it has few rows, of those whose operands are laid out as kernel_id's (a kernel with operand variants is never chosen
+ * automatically: this is the automatic choice among its siblings); kernel_id where there is none, or where it is negative (the launcher's own choice looks for itself). */
+int mxmoe_few_row_kernel(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int problem_count);
+
 /* The tile tables themselves (host-only; what the generated launcher keeps in its prefix-sum array, kernel_sketch.py:89-104): out receives
  * {entries, tiles, phases, workgroups}, phase_tile0[9], phase_wg0[9], then per entry {first tile, first row, rows, problem | branch << 16 |
  * what a pair of entries carries (bits 21 .. 29: mxmoe_launch.hpp, pair_word)}.  At most 120 problems; used by the tests that compare the device-side planner with the host launcher. */

@@ -58,6 +58,7 @@ SIGNATURES = {
     "mxmoe_quant_act": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P]),
     "mxmoe_quant_act_tokens": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P]),
     "mxmoe_silu_mul_quant": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P]),
+    "mxmoe_few_row_kernel": (_I, [_I, C.POINTER(Dim3), C.POINTER(QParams), _I]),
     "mxmoe_group_gemm_plan": (_I, [_I, C.POINTER(Dim3), C.POINTER(QParams), _I, C.POINTER(C.c_int32), C.POINTER(C.c_int32)]),
     "mxmoe_kernel_func": (_P, [_I]),
     "mxmoe_get_kernel": (_P, [C.c_char_p]),
@@ -95,7 +96,7 @@ _cached = {}
 
 
 GEMM_ONLY = ("mxmoe_last_error", "mxmoe_num_kernels", "mxmoe_kernel_name", "mxmoe_find_kernel", "mxmoe_kernel_num_branches", "mxmoe_kernel_branch",
-             "mxmoe_group_gemm", "mxmoe_group_gemm_plan", "mxmoe_group_gemm_plan_tables", "mxmoe_group_gemm_plan_tile_map", "mxmoe_group_gemm_plan_tile_area", "mxmoe_kernel_func", "mxmoe_get_kernel", "mxmoe_kernel_policy", "mxmoe_set_stream", "mxmoe_get_stream",
+             "mxmoe_group_gemm", "mxmoe_few_row_kernel", "mxmoe_group_gemm_plan", "mxmoe_group_gemm_plan_tables", "mxmoe_group_gemm_plan_tile_map", "mxmoe_group_gemm_plan_tile_area", "mxmoe_kernel_func", "mxmoe_get_kernel", "mxmoe_kernel_policy", "mxmoe_set_stream", "mxmoe_get_stream",
              "mxmoe_last_status")
 
 # the reference's FuncType (registry.cuh:28-39): 15 arguments, no return value

@@ -114,6 +114,15 @@ int mxmoe_group_gemm_plan(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_
   return kernel_id + 1000;  // plan succeeded: 1000 + the kernel that would run
 }
 
+int mxmoe_few_row_kernel(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int problem_count) {
+  if (kernel_id < 0) return kernel_id;
+  if (kernel_id >= (int)registry().size() || problem_count < 0 || (problem_count > 0 && (!h_sizes || !h_q))) {
+    last_error() = "bad argument";
+    return -2;
+  }
+  return few_row_sibling(kernel_id, h_sizes, h_q, problem_count);
+}
+
 int mxmoe_group_gemm_plan_tables(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int problem_count, int32_t* out, int out_ints) {
   auto& reg = registry();
   if (problem_count <= 0 || problem_count > kMaxProblems || !h_sizes || !h_q || !out || kernel_id < 0 || kernel_id >= (int)reg.size()) {

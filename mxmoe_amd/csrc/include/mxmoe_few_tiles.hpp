@@ -18,7 +18,7 @@ namespace mxmoe {
 
 template <Op OP>
 struct WxAxNarrowTile {
-  static_assert(OP == Op::I4 || OP == Op::I8, "integer accumulators: their partial sums may be added in any order");
+  static_assert(OP == Op::I4 || OP == Op::I8 || OP == Op::F8, "integer sums, which may be added in any order, or fp8, whose partial sums are added in the waves' order");
   static constexpr int BM = 32, BN = 64, FN = 2;
   static constexpr int BK = kRowBytes * 8 / OpTraits<OP>::kBitsPerElem;
   static constexpr int kLdsBytes = kWaves * FN * 4 * 64 * 16;  // partial sums
@@ -120,10 +120,14 @@ struct WxAxNarrowTile {
             acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wl, xl, acc[j], 0, 0, 0);
             acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wh, xh, acc[j], 0, 0, 0);
           }
-        } else {
+        } else if constexpr (OP == Op::I8) {
 #pragma unroll
           for (int j = 0; j < FN; ++j) acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[d][j][s], x[d][s], acc[j], 0, 0, 0);
         }
+      }
+      if constexpr (OP == Op::F8) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) WxAxTile<OP, 32, 256>::mma_slice(acc[j], w[d][j][0], w[d][j][1], x[d][0], x[d][1]);
       }
       __builtin_amdgcn_sched_barrier(0);
     };
@@ -148,11 +152,13 @@ struct WxAxNarrowTile {
     for (int j = 0; j < FN; ++j) vm_wait_for<0>(sb_bits[j]);
 
     // the four waves' sums meet in LDS; wave q adds and stores channels 8 q + nq .. + 3 of every 32-channel block
-    v4i* red = reinterpret_cast<v4i*>(smem);
+    typedef decltype(acc[0][0] + acc[0][0]) Sum;
+    typedef Sum v4s __attribute__((ext_vector_type(4)));
+    v4s* red = reinterpret_cast<v4s*>(smem);
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) red[((wave * FN + j) * 4 + q) * 64 + lane] = v4i{acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]};
+      for (int q = 0; q < 4; ++q) red[((wave * FN + j) * 4 + q) * 64 + lane] = v4s{acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]};
     __syncthreads();
     const _Float16 sa_h = __builtin_bit_cast(_Float16, (unsigned short)sa_bits);
     const float s_a = (float)sa_h * (OP == Op::I4 ? 0.00390625f : 1.0f);  // (the int4 accumulator holds 256 * sum)
@@ -160,7 +166,7 @@ struct WxAxNarrowTile {
     const bool live = m0 + lrow < M;
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
-      v4i sum = red[(j * 4 + wave) * 64 + lane];
+      v4s sum = red[(j * 4 + wave) * 64 + lane];
 #pragma unroll
       for (int v = 1; v < kWaves; ++v) sum += red[((v * FN + j) * 4 + wave) * 64 + lane];
       const v4h s_b = __builtin_bit_cast(v4h, sb_bits[j]);
@@ -173,7 +179,8 @@ struct WxAxNarrowTile {
         const int n = n0 + j * 32 + wave * 8 + nq;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int a = sum[e];
+          const Sum v = sum[e];
+          const int a = __builtin_bit_cast(int, v);
           if (live && n < N) gstore<int>(t.acc_dump + (long)(m0 + lrow) * N + n + e, OP == Op::I4 ? a >> 8 : a);
         }
       }

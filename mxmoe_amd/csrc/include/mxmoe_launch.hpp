@@ -359,7 +359,7 @@ template <Op OP>
 struct BranchOf<WxAxNarrowTile<OP>> {
   static BranchInfo get() {
     using T = WxAxNarrowTile<OP>;
-    return BranchInfo{OP == Op::I4 ? Fmt::W4A4 : Fmt::W8A8, T::kABits, T::kWBits, T::BM, T::BN, T::BK, 1, 1, T::kLdsBytes, T::BK, 0};
+    return BranchInfo{OP == Op::I4 ? Fmt::W4A4 : Fmt::W8A8, T::kABits, T::kWBits, T::BM, T::BN, T::BK, 1, 1, T::kLdsBytes, T::BK, 0, 0, OP == Op::F8 ? kVariantFp8 : 0};
   }
 };
 template <int BM>
@@ -978,17 +978,30 @@ inline bool shape_ok(const BranchInfo& bi, const mxmoe_dim3& sz) {
   return sz.z != 0 && sz.z % bi.k_multiple == 0 && (int)sz.z >= bi.k_min && sz.y % bi.n_multiple == 0;
 }
 
+// Whether kernel k's tiles take the shapes of a list's problems (an fp16 problem may have one that the few-token tiles do not take).
+inline bool fits_shapes(const FusedKernel& k, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int count) {
+  for (int i = 0; i < count; ++i)
+    for (const BranchInfo& b : k.branches)
+      if (h_sizes[i].x != 0 && b.fmt == classify(h_q[i]) && !shape_ok(b, h_sizes[i])) return false;
+  return true;
+}
+
+// The kernel made for the few rows of a list whose operands are those of kernel `kernel_id` (its operand variants, which QParams do not name), or kernel_id.
+inline int few_row_sibling(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int count) {
+  const FusedKernel& own = registry()[kernel_id];
+  const int kid = few_row_kernel(row_summary(h_sizes, h_q, count), [&](const FusedKernel& k) {
+    for (int i = 0; i < count; ++i)
+      if (kernel_variant(k, classify(h_q[i])) != kernel_variant(own, classify(h_q[i]))) return false;
+    return kernel_covers(k, h_q, count) && fits_shapes(k, h_sizes, h_q, count);
+  });
+  return kid >= 0 ? kid : kernel_id;
+}
+
 // The kernel the launcher picks when the caller names none: one made for few rows, or the first fused kernel without operand variants that has a tile for every
 // format.
 inline int auto_kernel(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int count) {
   auto covers = [&](const FusedKernel& k) { return !kernel_has_variants(k) && kernel_covers(k, h_q, count); };
-  auto fits = [&](const FusedKernel& k) {  // (an fp16 problem may have a shape that the few-token tiles do not take)
-    for (int i = 0; i < count; ++i)
-      for (const BranchInfo& b : k.branches)
-        if (h_sizes[i].x != 0 && b.fmt == classify(h_q[i]) && !shape_ok(b, h_sizes[i])) return false;
-    return true;
-  };
-  const int few = few_row_kernel(row_summary(h_sizes, h_q, count), [&](const FusedKernel& k) { return covers(k) && fits(k); });
+  const int few = few_row_kernel(row_summary(h_sizes, h_q, count), [&](const FusedKernel& k) { return covers(k) && fits_shapes(k, h_sizes, h_q, count); });
   if (few >= 0) return few;
   auto& reg = registry();
   for (int i = 0; i < (int)reg.size(); ++i)

@@ -168,7 +168,7 @@ def _pick(arch: str, qcfg: str, *shapes, bf6: bool = False, few_registers: bool 
 
 def default_kernel_specs(arch: str = "gfx950"):
     """The kernels of libmxmoe_amd.so: (function name, kernel type, {qcfg: shape set}) in registry order."""
-    w4, w8 = "w4a4_g-1_sym", "w8a8_g-1_sym"
+    w4, w8, f8 = "w4a4_g-1_sym", "w8a8_g-1_sym", "w8a8_g-1_sym_E4M3"
     wo = OrderedDict((f"w{b}a16_g128_asym", _pick(arch, f"w{b}a16_g128_asym", (16, 128), (32, 128))) for b in (4, 3, 2))
     wo_big = OrderedDict((f"w{b}a16_g128_asym", _pick(arch, f"w{b}a16_g128_asym", (128, 256))) for b in (4, 3, 2))
     wo_all = OrderedDict((q, wo[q] + wo_big[q]) for q in wo)
@@ -211,6 +211,11 @@ def default_kernel_specs(arch: str = "gfx950"):
         ("groupgemm_hz_fused_wxax_few", KernelType.Fused, OrderedDict((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8))),
         ("groupgemm_hz_fused_all_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8)), *wo_all.items(),
                                                                        ("w8a16_g128_asym", _pick(arch, "w8a16_g128_asym", (16, 128), (32, 128), (128, 256), (128, 128)))])),
+        # the two kernels with narrow tiles for 8-bit operands in fp8
+        ("groupgemm_hz_fused_wxax_e4m3_few", KernelType.Fused, OrderedDict((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, f8))),
+        ("groupgemm_hz_fused_all_e4m3_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, f8)), *wo_all.items(),
+                                                                           ("w4a4_g128_sym", _pick(arch, "w4a4_g128_sym", (64, 256), (32, 256))),
+                                                                           ("w8a16_g128_asym", _pick(arch, "w8a16_g128_asym", (16, 128), (32, 128), (128, 256), (128, 128)))])),
         # the few-token tiles of 64 channels of every format with 16-bit activations: fp16 and 8-bit weights take 142 registers (three workgroups per CU) where the
         # kernel without them has 125 (four)
         ("groupgemm_hz_fused_a16_few", KernelType.Fused, OrderedDict((q, (few_token_tile(q),)) for q in (*(f"w{b}a16_g128_asym" for b in (4, 3, 2, 8)), "fp16"))),

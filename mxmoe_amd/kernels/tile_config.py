@@ -251,7 +251,7 @@ class TileConfig:
                 raise ValueError(f"{self!r}: bf6 tiles are BM x 256 x 64 with 1 x 4 waves and 4 stages, BM in 32 / 64 / 128")
             return
         k_elems = {"MFMA_F32_32x32x16_F16": 32, "MFMA_F32_32x32x16_BF16": 32, "MFMA_I32_32x32x32_I8": 64, "MFMA_I32_32x32x32_I8_FROM_I4": 128, "MFMA_F32_32x32x16_FP8": 64}[self.MMA]
-        if self.is_narrow() and self.MMA in ("MFMA_I32_32x32x32_I8", "MFMA_I32_32x32x32_I8_FROM_I4") and not self.is_group_wa():
+        if self.is_narrow() and self.MMA in ("MFMA_I32_32x32x32_I8", "MFMA_I32_32x32x32_I8_FROM_I4", "MFMA_F32_32x32x16_FP8") and not self.is_group_wa():
             if (self.BM, self.WM, self.WN, self.BK) != (32, 1, 1, k_elems):
                 raise ValueError(f"{self!r}: tiles whose waves share K are 32 x 64 x {k_elems}")
             return

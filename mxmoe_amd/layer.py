@@ -74,7 +74,7 @@ class MxMoELayer:
         i_sh = cfg.inter * max(cfg.num_shared, 1)
         acc1 = [torch.zeros(m.shape, dtype=torch.int32, device=self.device) for m in st["mid"]] if dump_acc else None
         st["gg1"] = ops.prepare_gg(st["inp"], [w.data for w in self.w13], st["sa"], [w.scale for w in self.w13], st["mid"], 2 * cfg.inter, cfg.hidden,
-                                   2 * i_sh, cfg.hidden, self.qp_gate_up, st["recv"], kernel_id=self.kid_gate_up, acc_dump=acc1)
+                                   2 * i_sh, cfg.hidden, self.qp_gate_up, st["recv"], kernel_id=self.kid_gate_up, acc_dump=acc1, few_rows=True)
         st["acc1"] = acc1
         st["dump_acc"] = dump_acc
         st["hidden"], st["topk_ids"] = hidden, topk_ids
@@ -92,7 +92,7 @@ class MxMoELayer:
         i_sh = cfg.inter * max(cfg.num_shared, 1)
         acc2 = [torch.zeros(o.shape, dtype=torch.int32, device=self.device) for o in st["out"]] if st["dump_acc"] else None
         st["gg2"] = ops.prepare_gg(st["inp2"], [w.data for w in self.w2], st["sa2"], [w.scale for w in self.w2], st["out"], cfg.hidden, cfg.inter,
-                                   cfg.hidden, i_sh, self.qp_down, st["recv"], kernel_id=self.kid_down, acc_dump=acc2)
+                                   cfg.hidden, i_sh, self.qp_down, st["recv"], kernel_id=self.kid_down, acc_dump=acc2, few_rows=True)
         st["acc2"] = acc2
 
     def down(self):
@@ -418,8 +418,9 @@ class MxMoELayer:
 
         def launch(ptr_off, sizes_off, h_sizes, h_q, kid):
             row = lambda i: base + ptr_off + i * count * 8  # noqa: E731
-            _lib.check(lib, lib.mxmoe_group_gemm(kid, row(0), row(1), row(2), row(3), row(4), row(4), None, None, None, None, base + sizes_off,
-                                                 h_sizes.ctypes.data_as(C.POINTER(_lib.Dim3)), None, h_q.ctypes.data_as(C.POINTER(_lib.QParams)), count, None, stream))
+            dims, qs = h_sizes.ctypes.data_as(C.POINTER(_lib.Dim3)), h_q.ctypes.data_as(C.POINTER(_lib.QParams))
+            _lib.check(lib, lib.mxmoe_group_gemm(lib.mxmoe_few_row_kernel(kid, dims, qs, count), row(0), row(1), row(2), row(3), row(4), row(4), None, None, None, None, base + sizes_off,
+                                                 dims, None, qs, count, None, stream))
 
         hk, hf, sg = signs(cfg.hidden, cfg.hidden)
         _lib.check(lib, lib.mxmoe_quant_act(hidden.data_ptr(), inp1.data_ptr(), sa1.data_ptr(), dst.data_ptr(), perm.data_ptr(), base + off[0],
