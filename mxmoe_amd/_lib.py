@@ -96,7 +96,7 @@ _cached = {}
 
 
 GEMM_ONLY = ("mxmoe_last_error", "mxmoe_num_kernels", "mxmoe_kernel_name", "mxmoe_find_kernel", "mxmoe_kernel_num_branches", "mxmoe_kernel_branch",
-             "mxmoe_group_gemm", "mxmoe_few_row_kernel", "mxmoe_group_gemm_plan", "mxmoe_group_gemm_plan_tables", "mxmoe_group_gemm_plan_tile_map", "mxmoe_group_gemm_plan_tile_area", "mxmoe_kernel_func", "mxmoe_get_kernel", "mxmoe_kernel_policy", "mxmoe_set_stream", "mxmoe_get_stream",
+             "mxmoe_group_gemm", "mxmoe_group_gemm_plan", "mxmoe_group_gemm_plan_tables", "mxmoe_group_gemm_plan_tile_map", "mxmoe_group_gemm_plan_tile_area", "mxmoe_kernel_func", "mxmoe_get_kernel", "mxmoe_kernel_policy", "mxmoe_set_stream", "mxmoe_get_stream",
              "mxmoe_last_status")
 
 # the reference's FuncType (registry.cuh:28-39): 15 arguments, no return value

@@ -1,9 +1,10 @@
-// WxAxNarrowTile: w4a4 / w8a8 tile for launches with fewer workgroups than the chip has room for (decode batches on a few experts).
+// WxAxNarrowTile: w4a4 / w8a8 (int8 or fp8) tile for launches with fewer workgroups than the chip has room for (decode batches on a few experts).
 //
 // 32 tokens x 64 channels per workgroup, K dealt to the four waves in contiguous quarters, against 32 x 256 with all of K per wave (WxAxTile): four times the
 // workgroups and a quarter of the steps in each, for problems whose weight stream is all there is.  The 128 workgroups that the wide tile makes of eight
 // experts of N = 4096, K = 14336 leave half of the CUs idle: w4a4 and w8a8 half and half 90 us whatever the number of tokens, 62 here (w8a8 alone 97 -> 82, w4a4
-// 56 -> 44); by blocks, rows and formats, and for whole layers: few_rows in mxmoe_launch.hpp.  The partial sums are integers: the same result in any order.
+// 56 -> 44); by blocks, rows and formats, and for whole layers: few_rows in mxmoe_launch.hpp.  The partial sums are integers: the same result in any order.  (fp8: fp32 sums, added in the waves' order;
+// their errors in the 2-norm, 1.2e-5 .. 1.5e-5, are those of the wide tile's single chain, to three digits.)
 //
 // A wave streams the fragments of its channels (64 bytes of K of 32 channels are 2 KB, WxAxTile's layout) and of all 32 token rows straight into registers, kAhead
 // K slices ahead, without LDS or barriers; every load is an untracked one (gload16_untracked) awaited with the exact number of younger loads.  Rows past M

@@ -235,4 +235,129 @@ struct WxAxGTile {
   }
 };
 
+// The same problems with few rows: 16 tokens x 64 channels per workgroup, the groups dealt to the four waves one by one.  A round is four groups: a wave's integer sums of
+// its group, times their scales, go to LDS, and behind the barrier wave q adds the four groups' products to its quarter of the outputs in group order, which is all that has to happen in
+// order: the same additions as above, bit for bit.  Operands and scales stream straight into registers, kAhead rounds ahead; rows past M re-read the last one.
+// Bound: the weights' bytes; with few problems the latency of a round, of which there are a quarter as many as groups, in four times the workgroups.  Layers of four formats, a third of the
+// problems in this one, on narrow tiles but for these / with these too, us: eight experts of N = 28 672 / 4096, K = 4096 / 14 336 193 / 88 (1 token), 283 / 222 (8); 60 experts top-4 and a shared
+// one 56 / 43, 81 / 75.
+struct WxAxGNarrowTile {
+  static constexpr int BM = 16, BN = 64, BK = 128, NB = BN / 16;
+  static constexpr int kRoundBytes = kWaves * NB * 64 * 16;
+  static constexpr int kLdsBytes = 2 * kRoundBytes;  // a round's products are read while the next one's are written
+  static constexpr int kAccRegs = NB * 4 + 4;
+  static constexpr int kWavesWanted = 2;
+  static constexpr int kABits = 4, kWBits = 4;
+  static constexpr int kAhead = 3;
+
+  template <bool GU>
+  __device__ static __forceinline__ void run(const TileArgs& t, uint8_t* __restrict__ smem) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lm = lane & 15, lg = lane >> 4;
+    const int M = t.M, N = GU ? t.N / 2 : t.N;  // N: output channels
+    const int G = t.K / 128, rounds = (G + kWaves - 1) / kWaves;
+    const int m0 = t.row0 + t.tile_m * BM, n0 = t.tile_n * (GU ? BN / 2 : BN);
+    int src = min(m0 + lm, M - 1);
+    if constexpr (GU) src = gload<int>(t.rows + src);
+    const uint8_t* const xp = t.A + (long)src * (t.K / 2) + lg * 16;
+    const _Float16* const sa = t.sa + (long)src * G;
+    // 16 channels of the tile: half of a 32-channel block of fragments, of which lane (lm, lg) takes the 16-byte piece lg of channel lm's 64 bytes of a slice
+    const int nblk = (N + 31) / 32;
+    const uint8_t* wp[NB];
+    int ch[NB];  // first of the four channels whose products this lane gets
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int blk = GU ? min(n0 / 32, nblk - 1) + b / 2 * nblk : min(n0 / 32 + b / 2, nblk - 1);
+      wp[b] = t.B + (long)blk * G * 2048 + (lg >> 1) * 1024 + ((lg & 1) * 32 + b % 2 * 16 + lm) * 16;
+      ch[b] = GU ? b / 2 * N + min(n0 + b % 2 * 16 + lg * 4, N - 4) : min(n0 + b * 16 + lg * 4, N - 4);
+    }
+    v4i w[kAhead][NB], x[kAhead];
+    v4h s_b[kAhead][NB];
+    _Float16 s_a[kAhead];
+    auto load = [&](auto dc, int round) {
+      constexpr int d = decltype(dc)::value;
+      const int g = min(round * kWaves + wave, G - 1);
+#pragma unroll
+      for (int b = 0; b < NB; ++b) w[d][b] = gload<v4i>(wp[b] + (long)g * 2048);
+      x[d] = gload<v4i>(xp + (long)g * kRowBytes);
+#pragma unroll
+      for (int b = 0; b < NB; ++b) s_b[d][b] = gload<v4h>(t.sb + (long)g * t.N + ch[b]);
+      s_a[d] = gload<_Float16>(sa + g);
+    };
+    static_for<kAhead>([&](auto dc) { load(dc, decltype(dc)::value); });
+    __builtin_amdgcn_sched_barrier(0);
+
+    v4f sum = {0.f, 0.f, 0.f, 0.f};  // 256 times this lane's outputs: channels 4 lg .. + 3 of 16-channel block `wave`, token lm
+    auto multiply = [&](auto dc, int round) {
+      constexpr int d = decltype(dc)::value;
+      v4f* const out = reinterpret_cast<v4f*>(smem + (round & 1) * kRoundBytes);
+      const v4i xl = (x[d] << 4) & (int)0xF0F0F0F0, xh = x[d] & (int)0xF0F0F0F0;  // int4 pairs widened to bytes holding 16 v
+      const float a = (float)s_a[d];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const v4i wl = (w[d][b] << 4) & (int)0xF0F0F0F0, wh = w[d][b] & (int)0xF0F0F0F0;
+        v4i c = __builtin_amdgcn_mfma_i32_16x16x64_i8(wl, xl, v4i{}, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_i32_16x16x64_i8(wh, xh, c, 0, 0, 0);
+        v4f p;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) p[e] = (float)c[e] * (a * (float)s_b[d][b][e]);
+        out[(wave * NB + b) * 64 + lane] = p;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto add = [&](int round) {
+      const v4f* const in = reinterpret_cast<const v4f*>(smem + (round & 1) * kRoundBytes);
+      v4f p[kWaves];
+#pragma unroll
+      for (int v = 0; v < kWaves; ++v) p[v] = in[(v * NB + wave) * 64 + lane];
+#pragma unroll
+      for (int v = 0; v < kWaves; ++v)
+        if (round * kWaves + v < G) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sum[e] = sum[e] + p[v][e];
+        }
+    };
+#pragma unroll 1
+    for (int r0 = 0; r0 < rounds; r0 += kAhead)
+      static_for<kAhead>([&](auto dc) {
+        const int round = r0 + decltype(dc)::value;
+        if (round >= rounds) return;  // (uniform)
+        multiply(dc, round);
+        load(dc, round + kAhead);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();  // (behind it nobody reads the products of the round before the last any more: the next round overwrites those)
+        add(round);
+      });
+    v4h o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (_Float16)(sum[e] * 0.00390625f);  // exact
+    const int m = m0 + lm;
+    if constexpr (GU) {  // waves 0 and 1 hold gate channels, 2 and 3 the up channels of the same outputs
+      v4h* const up = reinterpret_cast<v4h*>(smem);
+      __syncthreads();
+      if (wave >= 2) up[(wave - 2) * 64 + lane] = o;
+      __syncthreads();
+      if (wave < 2) {
+        const v4h u = up[wave * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = silu_mul_half(o[e], u[e]);
+        const int n = n0 + wave * 16 + lg * 4;
+        if (m < M && n < N) gstore<v4h>(t.C + (long)m * N + n, o);
+      }
+    } else {
+      const int n = n0 + wave * 16 + lg * 4;
+      if (m < M && n < N) {
+        gstore<v4h>(t.C + (long)m * N + n, o);
+        if (t.acc_dump) {  // parity tests only: the fp32 sums as bit patterns
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float f = sum[e] * 0.00390625f;
+            gstore<int>(t.acc_dump + (long)m * N + n + e, __float_as_int(f));
+          }
+        }
+      }
+    }
+  }
+};
+
 }  // namespace mxmoe

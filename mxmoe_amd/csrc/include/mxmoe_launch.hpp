@@ -130,6 +130,8 @@ template <class T>
 constexpr bool kPairs = T::kABits == T::kWBits;
 template <int BM>
 constexpr bool kPairs<WxAxGTile<BM>> = false;
+template <>
+inline constexpr bool kPairs<WxAxGNarrowTile> = false;
 template <class T>
 constexpr bool kNarrow = false;
 template <Op OP>
@@ -348,6 +350,13 @@ struct BranchOf<WxAxGTile<BM>> {
     return BranchInfo{Fmt::W4A4G128, T::kABits, T::kWBits, BM, T::BN, T::BK, 1, 4, T::kLdsBytes, T::BK, 0};
   }
 };
+template <>
+struct BranchOf<WxAxGNarrowTile> {
+  static BranchInfo get() {
+    using T = WxAxGNarrowTile;
+    return BranchInfo{Fmt::W4A4G128, T::kABits, T::kWBits, T::BM, T::BN, T::BK, 1, 1, T::kLdsBytes, T::BK, 0};
+  }
+};
 template <Op OP, int BM, int BN>
 struct BranchOf<WxAxTile<OP, BM, BN>> {
   static BranchInfo get() {
@@ -441,7 +450,7 @@ inline double tile_cost(const BranchInfo& b) {
       {Fmt::W3A16, 16, 128, 0.31}, {Fmt::W3A16, 16, 64, 0.20}, {Fmt::W3A16, 32, 128, 0.50}, {Fmt::W3A16, 128, 128, 1.00}, {Fmt::W3A16, 128, 256, 1.50},
       {Fmt::W2A16, 16, 128, 0.25}, {Fmt::W2A16, 16, 64, 0.20}, {Fmt::W2A16, 32, 128, 0.50}, {Fmt::W2A16, 128, 128, 1.00}, {Fmt::W2A16, 128, 256, 1.50},
       {Fmt::W8A16, 16, 128, 0.60}, {Fmt::W8A16, 16, 64, 0.35}, {Fmt::W8A16, 32, 128, 0.66}, {Fmt::W8A16, 128, 128, 1.00}, {Fmt::W8A16, 128, 256, 1.50},
-      {Fmt::W4A4G128, 64, 256, 1.00}, {Fmt::W4A4G128, 32, 256, 0.60},
+      {Fmt::W4A4G128, 64, 256, 1.00}, {Fmt::W4A4G128, 32, 256, 0.60}, {Fmt::W4A4G128, 16, 64, 0.16},
   };
   for (const Row& r : table)
     if (r.f == b.fmt && r.bm == b.BM && r.bn == b.BN) return r.c;
@@ -880,7 +889,9 @@ struct RowSummary {
   uint32_t max_k = 0;
   bool w4a4 = false, w8a8 = false, other = false;  // formats among them
   bool fp16 = true;                                // no other format than this one
+  bool grouped = false;                            // w4a4 with scales per 128 values among them
   void add_format(Fmt f) {
+    grouped = grouped || f == Fmt::W4A4G128;
     (f == Fmt::W4A4 ? w4a4 : f == Fmt::W8A8 ? w8a8 : other) = true;
     fp16 = fp16 && f == Fmt::FP16;
   }
@@ -919,11 +930,17 @@ inline RowSummary row_summary(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_
 // A 128-row tile beside them would take the third workgroup of a CU (244 registers, 161 without): 60 experts 77 -> 83 (32).
 // (Launches of fewer than 8 blocks would run at 0.35 .. 0.6 of the wide kernel's time as well; the planning rules for long problems are stated, and tested, on lists of two or three
 // small problems in the wide shapes.)
+// The kernels for fp8 beside w4a4 (groupgemm_hz_fused_wxax_e4m3_few) by the same rules, us a layer: 60 experts top-4 40 -> 30 (1 token), 64 -> 55 (8), 94 -> 84 (32), 100 -> 92 (64); with a
+// shared expert, skewed, 53 -> 38 (1), 79 -> 67 (16), 105 -> 97 (64); 8 experts 103 -> 67 (1), 216 -> 184 (8), 232 -> 200 (64).  That with group-scaled w4a4 and weight-only problems
+// (groupgemm_hz_fused_all_e4m3_few: tiles of 64 channels alone, 155 registers; with the many-token tiles beside them, 255 registers, 8 experts, 64 tokens, took 343 us, not 265), four formats: 60 experts
+// 54 -> 32 (1), 78 -> 62 (8), 100 -> 101 (32); with a shared expert 75 -> 42 (1), 110 -> 92 (16), 140 -> 124 (64); 8 experts 228 -> 84 (1), 307 -> 213 (8), 326 -> 265 (64).
+// With group-scaled problems and more than 512 blocks, only up to 2 rows: a launch of 660 to 704 blocks 47.0 -> 47.7 (2 rows), 51.9 -> 53.5 (4), 59.4 -> 65.6 (5), one of 488 49.8 -> 34.8.
 constexpr int kFewRowsMax = 64, kFewBlocks = 768, kFewBlocksMin = 8;
 inline bool holds_narrow(const FusedKernel& k) { return plan_of(k).narrow; }
 // Rows per problem, on average, up to which those kernels are chosen.
 inline int few_rows_limit(const RowSummary& s) {
   if (s.blocks <= kPoleBlocks) return 24;
+  if (s.grouped && s.blocks > 512) return 2;
   if (s.max_k < 2048 && s.blocks > 384) return s.other ? 2 : 5;
   if (s.other || (s.w4a4 && s.w8a8 && s.max_k >= 2048)) return 16;
   return s.max_k < 2048 ? 8 : 12;

@@ -213,9 +213,8 @@ def default_kernel_specs(arch: str = "gfx950"):
                                                                        ("w8a16_g128_asym", _pick(arch, "w8a16_g128_asym", (16, 128), (32, 128), (128, 256), (128, 128)))])),
         # the two kernels with narrow tiles for 8-bit operands in fp8
         ("groupgemm_hz_fused_wxax_e4m3_few", KernelType.Fused, OrderedDict((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, f8))),
-        ("groupgemm_hz_fused_all_e4m3_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, f8)), *wo_all.items(),
-                                                                           ("w4a4_g128_sym", _pick(arch, "w4a4_g128_sym", (64, 256), (32, 256))),
-                                                                           ("w8a16_g128_asym", _pick(arch, "w8a16_g128_asym", (16, 128), (32, 128), (128, 256), (128, 128)))])),
+        ("groupgemm_hz_fused_all_e4m3_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q),)) for q in (w4, f8, "w4a4_g128_sym")),
+                                                                           *((f"w{b}a16_g128_asym", (few_token_tile(f"w{b}a16_g128_asym"),)) for b in (4, 3, 2, 8))])),
         # the few-token tiles of 64 channels of every format with 16-bit activations: fp16 and 8-bit weights take 142 registers (three workgroups per CU) where the
         # kernel without them has 125 (four)
         ("groupgemm_hz_fused_a16_few", KernelType.Fused, OrderedDict((q, (few_token_tile(q),)) for q in (*(f"w{b}a16_g128_asym" for b in (4, 3, 2, 8)), "fp16"))),

@@ -232,7 +232,7 @@ class TileConfig:
             return f"Bf6Tile<{self.BM}>"
         op = {"MFMA_F32_32x32x16_F16": "Op::F16", "MFMA_F32_32x32x16_BF16": "Op::BF16", "MFMA_I32_32x32x32_I8": "Op::I8", "MFMA_I32_32x32x32_I8_FROM_I4": "Op::I4", "MFMA_F32_32x32x16_FP8": "Op::F8"}[self.MMA]
         if self.is_narrow():
-            return f"WxAxNarrowTile<{op}>"
+            return "WxAxGNarrowTile" if self.is_group_wa() else f"WxAxNarrowTile<{op}>"
         if self.is_group_wa():
             return f"WxAxGTile<{self.BM}>"
         if op not in ("Op::F16", "Op::BF16"):
@@ -254,6 +254,8 @@ class TileConfig:
         if self.is_narrow() and self.MMA in ("MFMA_I32_32x32x32_I8", "MFMA_I32_32x32x32_I8_FROM_I4", "MFMA_F32_32x32x16_FP8") and not self.is_group_wa():
             if (self.BM, self.WM, self.WN, self.BK) != (32, 1, 1, k_elems):
                 raise ValueError(f"{self!r}: tiles whose waves share K are 32 x 64 x {k_elems}")
+            return
+        if self.is_narrow() and self.is_group_wa() and (self.BM, self.WM, self.WN, self.BK) == (16, 1, 1, k_elems):
             return
         if self.BK != k_elems or self.STAGE != 3 or self.WK != 1 or (self.BM // self.WM) % 32 or (self.BN // self.WN) % 32:
             raise ValueError(f"{self!r}: unsupported shape for {self.MMA} (BK must be {k_elems}, STAGE 3, wave tile a multiple of 32x32)")
@@ -321,7 +323,7 @@ def get_possible_tile_list(arch: str, qcfg: str) -> list:
 
 def narrow_tile(qcfg: str) -> TileConfig:
     """The w4a4 / w8a8 tile for launches with few workgroups (not among the candidates of get_possible_tile_list: its kernels are chosen by launch)."""
-    return _with_q(TileConfig(BM=32, BN=64, BK=128 if qcfg == "w4a4_g-1_sym" else 64, WM=1, WN=1, WK=4, STAGE=3, MMA=QCFG_TO_MMA[qcfg]), qcfg)
+    return _with_q(TileConfig(BM=16 if qcfg == "w4a4_g128_sym" else 32, BN=64, BK=128 if qcfg.startswith("w4a4") else 64, WM=1, WN=1, WK=4, STAGE=3, MMA=QCFG_TO_MMA[qcfg]), qcfg)
 
 
 def few_token_tile(qcfg: str) -> TileConfig:
