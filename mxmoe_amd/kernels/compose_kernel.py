@@ -209,8 +209,8 @@ def default_kernel_specs(arch: str = "gfx950"):
         ("groupgemm_hz_fused_wo_few", KernelType.Fused,
          OrderedDict((f"w{b}a16_g128_asym", _pick(arch, f"w{b}a16_g128_asym", (16, 64), few_registers=True)) for b in (4, 3, 2))),
         ("groupgemm_hz_fused_wxax_few", KernelType.Fused, OrderedDict((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8))),
-        ("groupgemm_hz_fused_all_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8)), *wo_all.items(),
-                                                                       ("w8a16_g128_asym", _pick(arch, "w8a16_g128_asym", (16, 128), (32, 128), (128, 256), (128, 128)))])),
+        ("groupgemm_hz_fused_all_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q),)) for q in (w4, w8, "w4a4_g128_sym")),
+                                                                      *((f"w{b}a16_g128_asym", (few_token_tile(f"w{b}a16_g128_asym"),)) for b in (4, 3, 2, 8))])),
         # the two kernels with narrow tiles for 8-bit operands in fp8
         ("groupgemm_hz_fused_wxax_e4m3_few", KernelType.Fused, OrderedDict((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, f8))),
         ("groupgemm_hz_fused_all_e4m3_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q),)) for q in (w4, f8, "w4a4_g128_sym")),
