@@ -40,6 +40,14 @@ struct WxAxNarrowTile {
 
   template <bool GU>
   __device__ static __forceinline__ void run(const TileArgs& t, uint8_t* __restrict__ smem) {
+    run_rows<GU, GU>(t, smem, [&](int m) {
+      if constexpr (GU) return gload4_untracked(t.rows + m);
+      else return m;
+    });
+  }
+  // `row_of(m)`: the row of A (and of sa) behind row m of the problem; IN_FLIGHT: it comes from an untracked load.
+  template <bool GU, bool IN_FLIGHT, class RowOf>
+  __device__ static __forceinline__ void run_rows(const TileArgs& t, uint8_t* __restrict__ smem, RowOf&& row_of) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int M = t.M, N = GU ? t.N / 2 : t.N;  // N: output channels
@@ -53,8 +61,7 @@ struct WxAxNarrowTile {
 
     // what the epilogue needs of this wave's outputs: rows q = wave of every four-channel run (see below)
     const int m = min(m0 + lrow, M - 1);
-    int src = m;
-    if constexpr (GU) src = gload4_untracked(t.rows + m);
+    int src = row_of(m);
     const _Float16* sb_ptr[FN];
     typedef int v2i __attribute__((ext_vector_type(2)));
     v2i sb_bits[FN];
@@ -88,7 +95,7 @@ struct WxAxNarrowTile {
       constexpr int d = decltype(dc)::value;
       load_w(dc, min(k0 + d, klast));
       if constexpr (d == 0) {
-        if constexpr (GU) vm_wait_for<FN + 2 * FN>(src);  // (younger: the channel scales and the fragments above)
+        if constexpr (IN_FLIGHT) vm_wait_for<FN + 2 * FN>(src);  // (younger: the channel scales and the fragments above)
         xoff = (unsigned)(GU ? src : src - m0) * row_bytes + (lane >> 5) * 16;  // (a gate_up form's store is below 2 GiB)
         sa_bits = gload2_untracked(t.sa + src);
       }

@@ -252,13 +252,20 @@ struct WxAxGNarrowTile {
 
   template <bool GU>
   __device__ static __forceinline__ void run(const TileArgs& t, uint8_t* __restrict__ smem) {
+    run_rows<GU>(t, smem, [&](int m) {
+      if constexpr (GU) return gload<int>(t.rows + m);
+      else return m;
+    });
+  }
+  // `row_of(m)`: the row of A (and of sa) behind row m of the problem.
+  template <bool GU, class RowOf>
+  __device__ static __forceinline__ void run_rows(const TileArgs& t, uint8_t* __restrict__ smem, RowOf&& row_of) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lm = lane & 15, lg = lane >> 4;
     const int M = t.M, N = GU ? t.N / 2 : t.N;  // N: output channels
     const int G = t.K / 128, rounds = (G + kWaves - 1) / kWaves;
     const int m0 = t.row0 + t.tile_m * BM, n0 = t.tile_n * (GU ? BN / 2 : BN);
-    int src = min(m0 + lm, M - 1);
-    if constexpr (GU) src = gload<int>(t.rows + src);
+    const int src = row_of(min(m0 + lm, M - 1));
     const uint8_t* const xp = t.A + (long)src * (t.K / 2) + lg * 16;
     const _Float16* const sa = t.sa + (long)src * G;
     // 16 channels of the tile: half of a 32-channel block of fragments, of which lane (lm, lg) takes the 16-byte piece lg of channel lm's 64 bytes of a slice

@@ -889,9 +889,7 @@ struct RowSummary {
   uint32_t max_k = 0;
   bool w4a4 = false, w8a8 = false, other = false;  // formats among them
   bool fp16 = true;                                // no other format than this one
-  bool grouped = false;                            // w4a4 with scales per 128 values among them
   void add_format(Fmt f) {
-    grouped = grouped || f == Fmt::W4A4G128;
     (f == Fmt::W4A4 ? w4a4 : f == Fmt::W8A8 ? w8a8 : other) = true;
     fp16 = fp16 && f == Fmt::FP16;
   }
@@ -934,13 +932,11 @@ inline RowSummary row_summary(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_
 // shared expert, skewed, 53 -> 38 (1), 79 -> 67 (16), 105 -> 97 (64); 8 experts 103 -> 67 (1), 216 -> 184 (8), 232 -> 200 (64).  That with group-scaled w4a4 and weight-only problems
 // (groupgemm_hz_fused_all_e4m3_few: tiles of 64 channels alone, 155 registers; with the many-token tiles beside them, 255 registers, 8 experts, 64 tokens, took 343 us, not 265), four formats: 60 experts
 // 54 -> 32 (1), 78 -> 62 (8), 100 -> 101 (32); with a shared expert 75 -> 42 (1), 110 -> 92 (16), 140 -> 124 (64); 8 experts 228 -> 84 (1), 307 -> 213 (8), 326 -> 265 (64).
-// With group-scaled problems and more than 512 blocks, only up to 2 rows: a launch of 660 to 704 blocks 47.0 -> 47.7 (2 rows), 51.9 -> 53.5 (4), 59.4 -> 65.6 (5), one of 488 49.8 -> 34.8.
 constexpr int kFewRowsMax = 64, kFewBlocks = 768, kFewBlocksMin = 8;
 inline bool holds_narrow(const FusedKernel& k) { return plan_of(k).narrow; }
 // Rows per problem, on average, up to which those kernels are chosen.
 inline int few_rows_limit(const RowSummary& s) {
   if (s.blocks <= kPoleBlocks) return 24;
-  if (s.grouped && s.blocks > 512) return 2;
   if (s.max_k < 2048 && s.blocks > 384) return s.other ? 2 : 5;
   if (s.other || (s.w4a4 && s.w8a8 && s.max_k >= 2048)) return 16;
   return s.max_k < 2048 ? 8 : 12;

@@ -14,6 +14,7 @@
 // intermediate value are neither written nor read.  The same kernels' arithmetic, bit for bit.  Measured, that form -> this one, us a
 // pass: DeepSeek-V2-Lite w4a16 / w3a16 47.7 -> 35.2 (1 token), 98.7 -> 84.9 (32), 163 -> 139 (201); Qwen1.5-MoE w4a4 456 -> 402 (8192,
 // of which the head 47 -> 24, the activation step 107 -> 72); Mixtral w4a4 / w8a8 / w4a16 3368 -> 3249 (8192).
+#include <algorithm>
 #include <climits>
 #include <hip/hip_runtime.h>
 
@@ -284,10 +285,11 @@ __global__ void __launch_bounds__(TH) layer_head_kernel(const HeadArgs a, const 
   for (int t = wg * (TH / 64) + wave; t < a.T; t += token_wgs * (TH / 64)) head_token<NI>(a, t, lane);
 }
 
-// Few tokens, first blocks of 16-bit activations: there is nothing to quantise in front of gate_up, and a workgroup finds its problem from the ids itself, so that the launch waits for no
-// head.  The permutation and the tables of both blocks, which the launches behind need, are made beside it by the first workgroups.  Grid: (column tiles of a routed expert) x (1 for those,
-// shared_slots rows of the shared expert's tiles, one row per expert that may have tokens).  A workgroup counts the ids in LDS, takes the slot-th expert with rows, lists its
-// rows, and runs their 16-row tiles one after the other (with 256 ids an expert of more than 16 rows is rare but under a skewed routing, and its weights come from L2 then).
+// Few tokens: a workgroup of gate_up finds its problem from the ids itself, so that the launch waits for no head.  The permutation and the tables of both blocks, which the launches behind
+// need, are made beside it by the first workgroups.  What is left in front is the quantisation of the tokens (layer_tokens_kernel), where first blocks take quantised ones.
+// Grid: (column tiles of a routed expert) x (1 for those, shared_slots rows of the shared expert's tiles, one row per expert that may have tokens).  A workgroup counts the ids in LDS, takes
+// the slot-th expert with rows, lists its rows, and runs their row tiles one after the other (with 256 ids an expert of more than one is rare but under a skewed routing, and its
+// weights come from L2 then).
 // What a launch of few tokens consists of is latency: a layer's, with the head in front -> without, us: 64 experts top-6 and a shared one, w4a16 / w3a16, 29 -> 22 (1 token), 54 -> 46 (8),
 // 77 -> 71 (32), w8a16 / w2a16 31 -> 23 (1), 65 -> 54 (8), 96 -> 85 (32); 60 experts top-4, w4a16 24 -> 18 (1), 55 -> 49 (16), 72 -> 68 (64), skewed 68 -> 64 (64), fp16 35 -> 27 (1),
 // 108 -> 99 (8), 217 -> 212 (64); 8 experts of N = 28 672 / 4096, w4a16 64 -> 58 (1), 134 -> 126 (16).  One id per thread: up to 256 of them, and no more tokens than the kernels for few rows take.
@@ -298,14 +300,46 @@ struct DirectArgs {
   _Float16* act;
   int hidden_size, inter, inter_shared;
   int cols, shared_rows, shared_slots;  // column tiles of a routed expert; rows of the grid that hold a row tile's column tiles of the shared expert, and all of its row tiles'
+  int shared_step;                      // rows of such a tile
   unsigned topk_inverse;  // ceil(2^16 / top-k): (i * topk_inverse) >> 16 = i / top-k for i < kDirectEntries and top-k <= 64
   int tile_lds;           // bytes of LDS that the tiles use
 };
 constexpr size_t direct_lds(int E) { return (size_t)kDirectEntries * 4 + kWaves * kDirectEntries + (size_t)E * 4; }
 
-template <bool LONG, class... Tiles>
-__global__ void __launch_bounds__(kThreads, kWavesPerSimd<Tiles...>) layer_first_kernel(const HeadArgs a, const PlanPair pair, const DirectArgs x) {
-  static_assert(kThreads == kHeadSmall && ((Tiles::MB == 1 && Tiles::BN == 64) && ...), "one id per thread; 16 rows, 32 outputs a tile");
+// A tile type of the launch: whether it is that of a format, and the tag of its activations.  (fp8 or int8 codes: a kernel holds the tile of one of them.)
+template <class T>
+struct DirectTile;
+template <int WBITS, int WAVES>
+struct DirectTile<SkinnyWoTile<WBITS, 64, 1, WAVES>> {
+  static constexpr int kTag = 0;
+  __device__ static bool takes(int a_bits, int w_bits, int) { return a_bits >= 16 && w_bits == WBITS; }
+  template <class RowOf>
+  __device__ static __forceinline__ void run(const TileArgs& t, uint8_t* smem, RowOf&& row_of) {
+    SkinnyWoTile<WBITS, 64, 1, WAVES>::template run_rows<true>(t, smem, row_of);
+  }
+};
+template <Op OP>
+struct DirectTile<WxAxNarrowTile<OP>> {
+  static constexpr int kTag = OP == Op::I4 ? 2 : OP == Op::I8 ? 1 : 5;
+  __device__ static bool takes(int a_bits, int, int gsize) { return a_bits == (OP == Op::I4 ? 4 : 8) && gsize == -1; }
+  template <class RowOf>
+  __device__ static __forceinline__ void run(const TileArgs& t, uint8_t* smem, RowOf&& row_of) {
+    WxAxNarrowTile<OP>::template run_rows<true, false>(t, smem, row_of);
+  }
+};
+template <>
+struct DirectTile<WxAxGNarrowTile> {
+  static constexpr int kTag = 3;
+  __device__ static bool takes(int a_bits, int, int gsize) { return a_bits == 4 && gsize == 128; }
+  template <class RowOf>
+  __device__ static __forceinline__ void run(const TileArgs& t, uint8_t* smem, RowOf&& row_of) {
+    WxAxGNarrowTile::run_rows<true>(t, smem, row_of);
+  }
+};
+
+template <class... Tiles>
+__global__ void __launch_bounds__(kThreads, 3) layer_first_kernel(const HeadArgs a, const PlanPair pair, const DirectArgs x) {
+  static_assert(kThreads == kHeadSmall && ((Tiles::BN == 64) && ...), "one id per thread; 32 outputs a tile");
   extern __shared__ __align__(16) uint8_t first_lds[];
   const int col0 = blockIdx.x, E = a.E;
   int slot = (int)blockIdx.y - 1;
@@ -313,7 +347,8 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd<Tiles...>) layer_first
     if (col0 < 2 * pair.chunks) {
       __builtin_amdgcn_s_setprio(3);
       constexpr size_t kPlanBytes = (sizeof(PlanShared) + 15) & ~(size_t)15;
-      head_plan<kHeadSmall, false, LONG>(a, pair, col0, *reinterpret_cast<PlanShared*>(first_lds), reinterpret_cast<int32_t*>(first_lds + kPlanBytes));
+      // (one planner body for every layer: nothing waits for it as long as gate_up runs)
+      head_plan<kHeadSmall, true, true>(a, pair, col0, *reinterpret_cast<PlanShared*>(first_lds), reinterpret_cast<int32_t*>(first_lds + kPlanBytes));
     } else if (col0 == 2 * pair.chunks) {
       __builtin_amdgcn_s_setprio(2);
       head_scatter<kHeadSmall>(a, 0, reinterpret_cast<int32_t*>(first_lds));
@@ -324,7 +359,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd<Tiles...>) layer_first
   int col = col0, shared_m0 = 0;
   if (shared) {
     int row = slot;
-    for (; row >= x.shared_rows; row -= x.shared_rows) shared_m0 += 16;
+    for (; row >= x.shared_rows; row -= x.shared_rows) shared_m0 += x.shared_step;
     col += row * x.cols;
   }
   if (col0 >= x.cols || col * 32 >= (shared ? x.inter_shared : x.inter)) return;
@@ -357,7 +392,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd<Tiles...>) layer_first
   if (e < 0) return;  // (every wave of the workgroup has come to the same)
   int M = 0;
   if (shared) {
-    M = min(a.T, shared_m0 + 16);
+    M = min(a.T, shared_m0 + x.shared_step);
   } else {
     for (int i0 = 0; i0 < a.total; i0 += 64) {
       const bool mine = all_ids[i0 + lane] == e;
@@ -369,46 +404,61 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd<Tiles...>) layer_first
   }
   TileArgs t;
   const mxmoe_block_desc* d = x.desc + e;
-  t.A = x.hidden;
   t.B = reinterpret_cast<const uint8_t*>(cload(&d->B));
-  t.sa = nullptr;
   t.sb = reinterpret_cast<const _Float16*>(cload(&d->scale_b));
   t.C = x.act + (long)before * x.inter;
   t.acc_dump = nullptr;
   t.M = M;
   t.N = 2 * (shared ? x.inter_shared : x.inter);
   t.K = x.hidden_size;
-  t.row0 = 0;
+  t.tile_m = 0;
   t.tile_n = col;
   t.rows = nullptr;
-  const int bits = cload(&d->q.w_bits);
+  const int a_bits = cload(&d->q.a_bits), w_bits = cload(&d->q.w_bits), gsize = cload(&d->q.gsize);
   auto token_of = [&](int m) { return shared ? m : (int)(rows[m] * x.topk_inverse >> 16); };
   auto run = [&](auto type) {
     using T = typename decltype(type)::type;
-    if (bits != T::WBITS) return;
+    using D = DirectTile<T>;
+    if (!D::takes(a_bits, w_bits, gsize)) return;
+    t.A = D::kTag == 0 ? x.hidden : a.store[D::kTag];
+    t.sa = D::kTag == 0 ? nullptr : a.scales[D::kTag];
 #pragma unroll 1
     for (int m0 = shared_m0; m0 < M; m0 += T::BM) {
       if (m0 > shared_m0) __syncthreads();  // the reduction behind the previous tile has been read
-      t.tile_m = m0 / T::BM;
-      T::template run_rows<true>(t, first_lds, token_of);
+      t.row0 = m0;
+      D::run(t, first_lds, token_of);
     }
   };
   (run(TileType<Tiles>{}), ...);
 }
 
-// The same for the registered kernel of the layer's first block: those made of 16 x 64 tiles alone have one (the tile lists of groupgemm_hz_fused_wo_few and _a16_few).
+// The tokens of the launch behind it, one per wave (the token part of layer_head_kernel).
+template <int NI>
+__global__ void __launch_bounds__(kHeadSmall) layer_tokens_kernel(const HeadArgs a) {
+  const int t = blockIdx.x * (kHeadSmall / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (t < a.T) head_token<NI>(a, t, threadIdx.x & 63);
+}
+
+// The launch for the registered kernel of a layer's first block: the kernels for few rows have one, of their 64-channel tiles.
 using LaunchFirstFn = void (*)(const HeadArgs&, const PlanPair&, const DirectArgs&, dim3, size_t, hipStream_t);
 template <class... Tiles>
 void launch_first(const HeadArgs& a, const PlanPair& pair, const DirectArgs& x, dim3 grid, size_t lds, hipStream_t s) {
-  if (pair.longs()) hipLaunchKernelGGL((layer_first_kernel<true, Tiles...>), grid, dim3(kThreads), lds, s, a, pair, x);
-  else hipLaunchKernelGGL((layer_first_kernel<false, Tiles...>), grid, dim3(kThreads), lds, s, a, pair, x);
+  hipLaunchKernelGGL((layer_first_kernel<Tiles...>), grid, dim3(kThreads), lds, s, a, pair, x);
 }
+template <int WBITS>
+using FewTokenTile = SkinnyWoTile<WBITS, 64, 1, 3>;
 static LaunchFirstFn first_launch_of(const FusedKernel& k) {
-  if (!only_narrow_few_token(k)) return nullptr;
-  for (const BranchInfo& b : k.branches)
-    if (b.fmt == Fmt::W8A16 || b.fmt == Fmt::FP16)
-      return &launch_first<SkinnyWoTile<4, 64, 1, 3>, SkinnyWoTile<3, 64, 1, 3>, SkinnyWoTile<2, 64, 1, 3>, SkinnyWoTile<8, 64, 1, 3>, SkinnyWoTile<16, 64, 1, 3>>;
-  return &launch_first<SkinnyWoTile<4, 64, 1, 3>, SkinnyWoTile<3, 64, 1, 3>, SkinnyWoTile<2, 64, 1, 3>>;
+  auto holds = [&](Fmt f) { return std::any_of(k.branches.begin(), k.branches.end(), [&](const BranchInfo& b) { return b.fmt == f; }); };
+  if (only_narrow_few_token(k)) {
+    if (holds(Fmt::W8A16) || holds(Fmt::FP16)) return &launch_first<FewTokenTile<4>, FewTokenTile<3>, FewTokenTile<2>, FewTokenTile<8>, FewTokenTile<16>>;
+    return &launch_first<FewTokenTile<4>, FewTokenTile<3>, FewTokenTile<2>>;
+  }
+  if (!holds_narrow(k)) return nullptr;
+  const bool others = holds(Fmt::W4A16), fp8 = kernel_variant(k, Fmt::W8A8) == kVariantFp8;
+  if (fp8 && others) return &launch_first<WxAxNarrowTile<Op::I4>, WxAxNarrowTile<Op::F8>, WxAxGNarrowTile, FewTokenTile<4>, FewTokenTile<3>, FewTokenTile<2>, FewTokenTile<8>>;
+  if (fp8) return &launch_first<WxAxNarrowTile<Op::I4>, WxAxNarrowTile<Op::F8>>;
+  if (others) return &launch_first<WxAxNarrowTile<Op::I4>, WxAxNarrowTile<Op::I8>, WxAxGNarrowTile, FewTokenTile<4>, FewTokenTile<3>, FewTokenTile<2>, FewTokenTile<8>>;
+  return &launch_first<WxAxNarrowTile<Op::I4>, WxAxNarrowTile<Op::I8>>;
 }
 
 // What a layer keeps for one (tokens, top-k): its description and both launches' planning parameters.
@@ -555,9 +605,9 @@ int mxmoe_layer_create(const mxmoe_layer_desc* d, void** handle) {
   pd.form.kind = d->rotate == 2 ? LayerForm::kPlain : LayerForm::kBehind;
   pd.form.act = reinterpret_cast<const uint8_t*>(d->act);
 
-  // few tokens: no head (nothing is quantised in front of gate_up, its tables need no totals, and its workgroups fit the counters beside the tiles)
+  // few tokens: no head
   const FusedKernel& kg = registry()[f->d.kernel_gate_up];
-  bool plain = f->fp16_first && tags == 0 && !f->pair.totals() && h.T <= kDirectTokens && h.total <= kDirectEntries && d->topk <= 64;
+  bool plain = (f->fp16_first || tags) && !(tags & 1u) && h.T <= kDirectTokens && h.total <= kDirectEntries && d->topk <= 64;
   for (int i = 0; i < et; ++i) {
     const int n = i < d->num_experts ? d->inter : d->inter_shared;
     plain = plain && (int)d->h_gate_up[i].N == 2 * n && (int)d->h_gate_up[i].K == d->hidden && n % 32 == 0;
@@ -572,12 +622,13 @@ int mxmoe_layer_create(const mxmoe_layer_desc* d, void** handle) {
   x.inter_shared = d->has_shared ? d->inter_shared : 0;
   x.cols = d->inter / 32;
   x.shared_rows = (x.inter_shared / 32 + x.cols - 1) / x.cols;
-  x.shared_slots = x.shared_rows * ((h.T + 15) / 16);
+  x.shared_step = d->has_shared && d->h_gate_up[d->num_experts].q.a_bits < 16 && d->h_gate_up[d->num_experts].q.gsize != 128 ? 32 : 16;  // (BM of the format's tile)
+  x.shared_slots = x.shared_rows * ((h.T + x.shared_step - 1) / x.shared_step);
   x.topk_inverse = (65536 + d->topk - 1) / d->topk;
   x.tile_lds = kg.lds_bytes;
   f->first_grid = dim3(std::max(x.cols, 2 * f->pair.chunks + 1), 1 + x.shared_slots + std::min(h.total, h.E));
   f->first_lds = std::max(kg.lds_bytes + direct_lds(h.E), sizeof(PlanShared) + 16 + (size_t)(2 + kHeadSmall / 64 + 2 * kCountCopies) * h.E * sizeof(int32_t));
-  if (f->first_lds > 32 * 1024) f->first = nullptr;  // (counters of many experts would take the room of a workgroup)
+  if (f->first_lds > 40 * 1024) f->first = nullptr;  // (counters of many experts would take the room of a workgroup)
 
   RowsBehind& r = f->rows;
   r = RowsBehind{};
@@ -632,29 +683,34 @@ int mxmoe_layer_run(const void* handle, const void* hidden, const int32_t* topk_
     }
     return 0;
   };
+  // by the row length: f(number of 512-value pieces)
+  auto by_length = [&](auto&& f) {
+    switch (d.hidden / 512) {
+      case 1: f(std::integral_constant<int, 1>{}); break;
+      case 2: f(std::integral_constant<int, 2>{}); break;
+      case 4: f(std::integral_constant<int, 4>{}); break;
+      default: f(std::integral_constant<int, 8>{}); break;
+    }
+  };
   if (f.first) {
     DirectArgs x = f.direct;
     x.hidden = reinterpret_cast<const uint8_t*>(hidden);
+    if (h.tags) by_length([&](auto ni) { hipLaunchKernelGGL((layer_tokens_kernel<decltype(ni)::value>), dim3((h.T + 3) / 4), dim3(kHeadSmall), 0, s, h); });
+    if (const int rc = check_launch()) return rc;
     f.first(h, pair, x, f.first_grid, f.first_lds, s);
     if (const int rc = check_launch()) return rc;
   } else {
     if (h.hist) launch_perm_hist(topk_ids, h.total, h.E, const_cast<int32_t*>(h.hist), true, s);
     const dim3 grid(2 * pair.chunks + h.perm_wgs + f.token_wgs), block(f.threads);
     const size_t lds = (size_t)(2 + f.threads / 64 + 2 * kCountCopies) * h.E * sizeof(int32_t);
-    auto head = [&](auto ni) {
+    by_length([&](auto ni) {
       constexpr int NI = decltype(ni)::value;
       pair.with_body([&](auto totals, auto longs) {
         constexpr bool kTotals = decltype(totals)::value, kLong = decltype(longs)::value;
         if (f.threads == kHeadSmall) hipLaunchKernelGGL((layer_head_kernel<NI, kHeadSmall, kTotals, kLong>), grid, block, lds, s, h, pair);
         else hipLaunchKernelGGL((layer_head_kernel<NI, kHeadLarge, kTotals, kLong>), grid, block, lds, s, h, pair);
       });
-    };
-    switch (d.hidden / 512) {
-      case 1: head(std::integral_constant<int, 1>{}); break;
-      case 2: head(std::integral_constant<int, 2>{}); break;
-      case 4: head(std::integral_constant<int, 4>{}); break;
-      default: head(std::integral_constant<int, 8>{}); break;
-    }
+    });
     if (const int rc = check_launch()) return rc;
     if (const int rc = gemm(kg.launch_gate_up, kg, d.plan_gate_up, d.grid_gate_up)) return rc;
   }

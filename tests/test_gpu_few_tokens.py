@@ -118,6 +118,8 @@ def test_lists_that_the_few_token_tiles_take():
 @pytest.mark.parametrize("tokens,topk,experts,inter,num_shared,mix", [
     (1, 1, 8, 1408, 0, "fp16"), (1, 6, 64, 1408, 2, "wo"), (17, 3, 70, 96, 3, "fp16"), (33, 6, 130, 160, 1, "all"), (64, 4, 60, 256, 4, "wo"), (64, 4, 60, 352, 0, "all"),
     (32, 8, 24, 1408, 1, "behind"), (5, 2, 66, 640, 2, "behind"), (16, 16, 8, 512, 1, "fp16"),
+    (1, 4, 60, 1408, 4, "int"), (64, 4, 60, 1408, 1, "int"), (33, 2, 9, 640, 2, "many"), (64, 4, 130, 1408, 1, "many"), (1, 1, 10, 512, 0, "many"),
+    (40, 6, 64, 1408, 1, "fp8"), (64, 2, 12, 512, 0, "many fp8"), (17, 6, 64, 1408, 2, "many fp8"),
 ])
 def test_first_launch_without_a_head(tokens, topk, experts, inter, num_shared, mix):
     """gate_up that finds its problems from the ids, against the form with tables from launches in front on the same kernels: identical outputs.  Ids out of range,
@@ -128,11 +130,15 @@ def test_first_launch_without_a_head(tokens, topk, experts, inter, num_shared, m
     if inter % 128 and mix != "fp16":  # (their second block's K is in groups of 128)
         mix = "first"
     fm = {"fp16": [(FP16, FP16)], "wo": [(S.W4A16, S.W3A16), (S.W3A16, S.W2A16), (S.W2A16, S.W4A16)], "all": [(W8A16, FP16), (S.W4A16, W8A16), (FP16, S.W2A16)],
-          "first": [(W8A16, FP16), (S.W4A16, FP16), (S.W2A16, FP16)], "behind": [(S.W4A16, S.W4A4), (S.W3A16, S.W8A8), (S.W4A16, S.W4A16)]}[mix]
+          "first": [(W8A16, FP16), (S.W4A16, FP16), (S.W2A16, FP16)], "behind": [(S.W4A16, S.W4A4), (S.W3A16, S.W8A8), (S.W4A16, S.W4A16)],
+          "int": [(S.W4A4, S.W8A8), (S.W8A8, S.W4A4), (S.W4A4, S.W4A4)], "many": [(S.W4A4, S.W8A8), (S.W4A4G128, S.W4A4), (W8A16, S.W4A4G128), (S.W8A8, S.W3A16), (S.W3A16, S.W4A4)]}
+    fm["fp8"], fm["many fp8"] = fm["int"], fm["many"]
+    fm = fm[mix]
     n = experts + (num_shared > 0)
-    cfg = S.MoEConfig("t", "test", experts, topk, 512, inter, tokens, num_shared=num_shared, rotate=int(mix == "behind"))
-    layer = MxMoELayer(cfg, formats=[fm[i % len(fm)] for i in range(n)])
-    kid = _lib.load().mxmoe_find_kernel(b"groupgemm_hz_fused_wo_few" if mix in ("wo", "behind") else b"groupgemm_hz_fused_a16_few")
+    cfg = S.MoEConfig("t", "test", experts, topk, 512, inter, tokens, num_shared=num_shared, rotate=int(mix not in ("fp16", "wo", "all", "first")))
+    layer = MxMoELayer(cfg, formats=[fm[i % len(fm)] for i in range(n)], fp8="fp8" in mix)
+    kid = _lib.load().mxmoe_find_kernel(b"groupgemm_hz_fused_" + {"wo": b"wo_few", "behind": b"wo_few", "int": b"wxax_few", "many": b"all_few", "fp8": b"wxax_e4m3_few",
+                                                                  "many fp8": b"all_e4m3_few"}.get(mix, b"a16_few"))
     planned = layer._planned_kernel
     layer._planned_kernel = lambda h, t, k: kid if int(h[0].N) == 2 * inter else planned(h, t, k)
     gen = torch.Generator().manual_seed(tokens)
