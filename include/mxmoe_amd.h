@@ -103,8 +103,8 @@ int mxmoe_last_status(void);
  * Host-only; used by the scheduler tests and the kernel-profile table.  Returns 1000 + kernel id on success. */
 int mxmoe_group_gemm_plan(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int problem_count, int32_t* branch_out, int32_t* tiles_out);
 
-/* The kernel that a list is better off on when it has few rows, of those whose operands are laid out as kernel_id's (a kernel with operand variants is never chosen
- * automatically: this is the automatic choice among its siblings); kernel_id where there is none, or where it is negative (the launcher's own choice looks for itself). */
+/* The kernel that a layer's list is better off on when it has few rows, of those whose operands are laid out as kernel_id's (-1: without operand variants); kernel_id
+ * where there is none.  -2: bad argument. */
 int mxmoe_few_row_kernel(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int problem_count);
 
 /* The tile tables themselves (host-only; what the generated launcher keeps in its prefix-sum array, kernel_sketch.py:89-104): out receives
@@ -254,6 +254,9 @@ size_t mxmoe_plan_bytes(int num_problems);
 size_t mxmoe_plan_offset(int which, int num_problems);
 int mxmoe_plan_select_kernel(int kernel_id, const mxmoe_block_desc* h_desc, int num_problems);
 int mxmoe_plan_select_kernel_rows(const mxmoe_block_desc* h_desc, int num_experts, int num_tokens, int topk, int shared_rows);
+/* The same for a block of a layer's forward (as mxmoe_few_row_kernel for a list).  first: the first block of one that mxmoe_layer_run runs: few tokens have no launch in
+ * front of it on the kernels for few rows, which then pay up to more experts. */
+int mxmoe_layer_kernel(const mxmoe_block_desc* h_desc, int num_experts, int num_tokens, int topk, int shared_rows, int first);
 int mxmoe_plan_grid_bound(int kernel_id, const mxmoe_block_desc* h_desc, int num_experts, int routed_rows_max, int shared_rows);
 int mxmoe_plan_block(int kernel_id, const int64_t* d_recv_tokens_per_exp, int num_experts, int shared_rows, const mxmoe_block_desc* d_desc,
                      const mxmoe_block_desc* h_desc, const void* inp_store, const void* scale_store, void* out_store, void* d_plan, void* stream);

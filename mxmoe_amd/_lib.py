@@ -70,6 +70,7 @@ SIGNATURES = {
     "mxmoe_plan_offset": (C.c_size_t, [_I, _I]),
     "mxmoe_plan_select_kernel": (_I, [_I, _P, _I]),
     "mxmoe_plan_select_kernel_rows": (_I, [_P, _I, _I, _I, _I]),
+    "mxmoe_layer_kernel": (_I, [_P, _I, _I, _I, _I, _I]),
     "mxmoe_plan_grid_bound": (_I, [_I, _P, _I, _I, _I]),
     "mxmoe_plan_block": (_I, [_I, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P]),
     "mxmoe_plan_layer": (_I, [_P, _P, _P, _I, _I, _P]),

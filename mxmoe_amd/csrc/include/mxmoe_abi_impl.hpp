@@ -115,12 +115,11 @@ int mxmoe_group_gemm_plan(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_
 }
 
 int mxmoe_few_row_kernel(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int problem_count) {
-  if (kernel_id < 0) return kernel_id;
-  if (kernel_id >= (int)registry().size() || problem_count < 0 || (problem_count > 0 && (!h_sizes || !h_q))) {
+  if (kernel_id < -1 || kernel_id >= (int)registry().size() || problem_count < 0 || (problem_count > 0 && (!h_sizes || !h_q))) {
     last_error() = "bad argument";
     return -2;
   }
-  return few_row_sibling(kernel_id, h_sizes, h_q, problem_count);
+  return problem_count > 0 ? few_row_sibling(kernel_id, h_sizes, h_q, problem_count) : kernel_id;
 }
 
 int mxmoe_group_gemm_plan_tables(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int problem_count, int32_t* out, int out_ints) {

@@ -887,6 +887,7 @@ struct RowSummary {
   long rows = 0, max_rows = 0;
   long blocks = 0;                // of 256 channels
   uint32_t max_k = 0;
+  bool headless = false;          // a planned layer of few tokens: no head in front of gate_up on these kernels (layer_first_kernel)
   bool w4a4 = false, w8a8 = false, other = false;  // formats among them
   bool fp16 = true;                                // no other format than this one
   void add_format(Fmt f) {
@@ -932,17 +933,20 @@ inline RowSummary row_summary(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_
 // shared expert, skewed, 53 -> 38 (1), 79 -> 67 (16), 105 -> 97 (64); 8 experts 103 -> 67 (1), 216 -> 184 (8), 232 -> 200 (64).  That with group-scaled w4a4 and weight-only problems
 // (groupgemm_hz_fused_all_e4m3_few: tiles of 64 channels alone, 155 registers; with the many-token tiles beside them, 255 registers, 8 experts, 64 tokens, took 343 us, not 265), four formats: 60 experts
 // 54 -> 32 (1), 78 -> 62 (8), 100 -> 101 (32); with a shared expert 75 -> 42 (1), 110 -> 92 (16), 140 -> 124 (64); 8 experts 228 -> 84 (1), 307 -> 213 (8), 326 -> 265 (64).
-constexpr int kFewRowsMax = 64, kFewBlocks = 768, kFewBlocksMin = 8;
+// Where such a layer starts with gate_up on these kernels (layer_first_kernel, 4 us less in front of it), up to 1024 blocks and 12 rows: 8 experts, first block of 896 blocks, us a layer, w4a4 119 -> 115 (4
+// tokens), 148 -> 144 (32), w4a4 / w8a8 skewed 146 -> 137 (4), 173 -> 167 (16), 201 -> 199 (48), 211 -> 219 (64), with w4a16 208 -> 202 (16), 212 -> 210 (48), 216 -> 222 (64).
+constexpr int kFewRowsMax = 64, kFewBlocks = 768, kFewBlocksHeadless = 1024, kFewBlocksMin = 8;
 inline bool holds_narrow(const FusedKernel& k) { return plan_of(k).narrow; }
 // Rows per problem, on average, up to which those kernels are chosen.
 inline int few_rows_limit(const RowSummary& s) {
   if (s.blocks <= kPoleBlocks) return 24;
+  if (s.blocks > kFewBlocks) return 12;
   if (s.max_k < 2048 && s.blocks > 384) return s.other ? 2 : 5;
   if (s.other || (s.w4a4 && s.w8a8 && s.max_k >= 2048)) return 16;
   return s.max_k < 2048 ? 8 : 12;
 }
 inline bool few_rows(const RowSummary& s) {
-  if (!(s.w4a4 || s.w8a8) || s.max_rows > kFewRowsMax || s.blocks < kFewBlocksMin || s.blocks > kFewBlocks) return false;
+  if (!(s.w4a4 || s.w8a8) || s.max_rows > kFewRowsMax || s.blocks < kFewBlocksMin || s.blocks > (s.headless ? kFewBlocksHeadless : kFewBlocks)) return false;
   if (s.blocks > kPoleBlocks && s.blocks <= 256 && s.max_rows > 32) return false;
   return s.rows <= few_rows_limit(s) * s.live;
 }
@@ -958,6 +962,8 @@ inline bool few_rows(const RowSummary& s) {
 // 4096 fp16 327 -> 173 (1), 583 -> 447 (16), 622 -> 521 (32: 8 rows each), 639 -> 614 (48), 642 -> 705 (64): weights of 16 bits outweigh the activations for longer, up to 12 rows.  w8a16 / w2a16 half and
 // half, 64 experts top-6 and a shared one 37 -> 31 (1), 71 -> 65 (8), 103 -> 96 (32), 8 experts 100 -> 80 (1), 204 -> 200 (8), 213 -> 215 (32).
 constexpr int kFewTokenRows = 6, kFewTokenRowsFp16 = 12;
+// Tokens and (token, slot) pairs up to which a planned layer has no head in front of gate_up on the kernels for few rows (layer_first_kernel: one pair per thread of a workgroup).
+constexpr int kDirectTokens = 64, kDirectEntries = 256;
 inline bool only_narrow_few_token(const FusedKernel& k) {
   for (const BranchInfo& b : k.branches)
     if (b.a_bits != 16 || b.BN != 64) return false;
@@ -999,14 +1005,33 @@ inline bool fits_shapes(const FusedKernel& k, const mxmoe_dim3* h_sizes, const m
   return true;
 }
 
-// The kernel made for the few rows of a list whose operands are those of kernel `kernel_id` (its operand variants, which QParams do not name), or kernel_id.
+// Of the kernels with narrow tiles, the one for a layer: without many-token tiles where there is one.  A launch of more formats than w4a4 and w8a8 by itself is chosen with them (lists of up to 64 rows
+// a problem); in a layer of few tokens a problem of more than a row tile is rare, and they cost every tile of the launch its third workgroup per CU.  w4a4 / w8a8 / w4a16, us a layer, with /
+// without them: 64 experts top-6 and a shared one 38.7 / 37.8 (1 token), 93 / 90 (16), 108 / 106 (32); 60 experts top-4 and a shared one 89 / 83 (16), 109 / 102 (32), 121 / 113 (64).
+template <class Covers>
+int without_many_token_tiles(int kid, Covers&& covers) {
+  auto many = [](const FusedKernel& k) {
+    for (const BranchInfo& b : k.branches)
+      if (b.BM == 128) return true;
+    return false;
+  };
+  auto& reg = registry();
+  if (kid < 0 || !holds_narrow(reg[kid]) || !many(reg[kid])) return kid;
+  for (int i = 0; i < (int)reg.size(); ++i)
+    if (reg[i].policy == Policy::Fused && holds_narrow(reg[i]) && !many(reg[i]) && covers(reg[i])) return i;
+  return kid;
+}
+
+// The kernel for a layer's list of few rows whose operands are those of kernel `kernel_id` (its operand variants, which QParams do not name; plain ones where it is negative), or kernel_id.
 inline int few_row_sibling(int kernel_id, const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_q, int count) {
-  const FusedKernel& own = registry()[kernel_id];
-  const int kid = few_row_kernel(row_summary(h_sizes, h_q, count), [&](const FusedKernel& k) {
-    for (int i = 0; i < count; ++i)
-      if (kernel_variant(k, classify(h_q[i])) != kernel_variant(own, classify(h_q[i]))) return false;
-    return kernel_covers(k, h_q, count) && fits_shapes(k, h_sizes, h_q, count);
-  });
+  auto covers = [&](const FusedKernel& k) {
+    for (int i = 0; i < count; ++i) {
+      const Fmt f = classify(h_q[i]);
+      if (kernel_variant(k, f) != (kernel_id < 0 ? 0 : kernel_variant(registry()[kernel_id], f))) return false;
+    }
+    return (kernel_id >= 0 || !kernel_has_variants(k)) && kernel_covers(k, h_q, count) && fits_shapes(k, h_sizes, h_q, count);
+  };
+  const int kid = without_many_token_tiles(few_row_kernel(row_summary(h_sizes, h_q, count), covers), covers);
   return kid >= 0 ? kid : kernel_id;
 }
 

@@ -293,7 +293,7 @@ __global__ void __launch_bounds__(TH) layer_head_kernel(const HeadArgs a, const 
 // What a launch of few tokens consists of is latency: a layer's, with the head in front -> without, us: 64 experts top-6 and a shared one, w4a16 / w3a16, 29 -> 22 (1 token), 54 -> 46 (8),
 // 77 -> 71 (32), w8a16 / w2a16 31 -> 23 (1), 65 -> 54 (8), 96 -> 85 (32); 60 experts top-4, w4a16 24 -> 18 (1), 55 -> 49 (16), 72 -> 68 (64), skewed 68 -> 64 (64), fp16 35 -> 27 (1),
 // 108 -> 99 (8), 217 -> 212 (64); 8 experts of N = 28 672 / 4096, w4a16 64 -> 58 (1), 134 -> 126 (16).  One id per thread: up to 256 of them, and no more tokens than the kernels for few rows take.
-constexpr int kDirectTokens = 64, kDirectEntries = kHeadSmall;
+static_assert(kDirectEntries == kHeadSmall, "one id per thread");
 struct DirectArgs {
   const mxmoe_block_desc* desc;
   const uint8_t* hidden;

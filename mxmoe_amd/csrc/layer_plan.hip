@@ -177,7 +177,7 @@ int mxmoe_plan_select_kernel(int kernel_id, const mxmoe_block_desc* h_desc, int 
   return resolve_kernel(kernel_id, h_desc, num_problems);
 }
 
-int mxmoe_plan_select_kernel_rows(const mxmoe_block_desc* h_desc, int num_experts, int num_tokens, int topk, int shared_rows) {
+static int select_kernel_rows(const mxmoe_block_desc* h_desc, int num_experts, int num_tokens, int topk, int shared_rows, bool headless) {
   const int et = num_experts + (shared_rows > 0 ? 1 : 0);
   const int plain = mxmoe_plan_select_kernel(-1, h_desc, et);
   if (plain < 0) return plain;
@@ -201,8 +201,23 @@ int mxmoe_plan_select_kernel_rows(const mxmoe_block_desc* h_desc, int num_expert
   s.max_rows = std::max<long>(s.max_rows, num_tokens);  // one expert may get them all
   // an uneven routing has problems of several 16-row tiles well before the average reaches 16
   if (routed > 12l * num_experts) s.tall = s.live;
+  s.headless = headless && num_tokens <= kDirectTokens && routed <= kDirectEntries;
   const int few = few_row_kernel(s, [&](const FusedKernel& k) { return covers_blocks(k, h_desc, et); });
   return few >= 0 && resolve_kernel(few, h_desc, et) == few ? few : plain;
+}
+
+int mxmoe_plan_select_kernel_rows(const mxmoe_block_desc* h_desc, int num_experts, int num_tokens, int topk, int shared_rows) {
+  return select_kernel_rows(h_desc, num_experts, num_tokens, topk, shared_rows, false);
+}
+
+int mxmoe_layer_kernel(const mxmoe_block_desc* h_desc, int num_experts, int num_tokens, int topk, int shared_rows, int first) {
+  // (the kernels' integer and fp16 sums are the same whichever runs; fp8 ones are not to the last bit, and stay where a list of the same rows would run)
+  const int et = num_experts + (shared_rows > 0 ? 1 : 0);
+  bool fp8 = false;
+  for (int i = 0; h_desc && i < et; ++i) fp8 = fp8 || wants_fp8(h_desc[i].q);
+  const int kid = select_kernel_rows(h_desc, num_experts, num_tokens, topk, shared_rows, first && !fp8);
+  const int lean = without_many_token_tiles(kid, [&](const FusedKernel& k) { return covers_blocks(k, h_desc, et); });
+  return lean == kid || resolve_kernel(lean, h_desc, et) == lean ? lean : kid;
 }
 
 int mxmoe_plan_grid_bound(int kernel_id, const mxmoe_block_desc* h_desc, int num_experts, int routed_rows_max, int shared_rows) {

@@ -42,7 +42,7 @@ class GroupGemmLaunch:
     """A prepared problem list: `run()` is a single allocation-free, sync-free kernel launch."""
 
     def __init__(self, As, Bs, scale_a, scale_b, Cs, sizes, qparams, kernel_id: int = -1, acc=None, lib=None, few_rows: bool = False):
-        """`few_rows`: kernel_id names how the operands are laid out; a list of few rows may run on the kernel made for it that takes the same."""
+        """`few_rows`: kernel_id names how the operands are laid out (-1: plainly); a list of few rows may run on the kernel made for a layer's that takes the same."""
         self.lib = lib or _lib.load()
         p = len(As)
         assert len(Bs) == len(Cs) == len(sizes) == len(qparams) == p

@@ -209,12 +209,16 @@ def default_kernel_specs(arch: str = "gfx950"):
         ("groupgemm_hz_fused_wo_few", KernelType.Fused,
          OrderedDict((f"w{b}a16_g128_asym", _pick(arch, f"w{b}a16_g128_asym", (16, 64), few_registers=True)) for b in (4, 3, 2))),
         ("groupgemm_hz_fused_wxax_few", KernelType.Fused, OrderedDict((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8))),
-        ("groupgemm_hz_fused_all_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q),)) for q in (w4, w8, "w4a4_g128_sym")),
-                                                                      *((f"w{b}a16_g128_asym", (few_token_tile(f"w{b}a16_g128_asym"),)) for b in (4, 3, 2, 8))])),
+        ("groupgemm_hz_fused_all_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8)), *wo_all.items(),
+                                                                       ("w8a16_g128_asym", _pick(arch, "w8a16_g128_asym", (16, 128), (32, 128), (128, 256), (128, 128)))])),
         # the two kernels with narrow tiles for 8-bit operands in fp8
         ("groupgemm_hz_fused_wxax_e4m3_few", KernelType.Fused, OrderedDict((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, f8))),
         ("groupgemm_hz_fused_all_e4m3_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q),)) for q in (w4, f8, "w4a4_g128_sym")),
                                                                            *((f"w{b}a16_g128_asym", (few_token_tile(f"w{b}a16_g128_asym"),)) for b in (4, 3, 2, 8))])),
+        # the same without many-token tiles (161 registers, three workgroups per CU, where those take 255), and with group-scaled w4a4: for layers of few tokens
+        ("groupgemm_hz_fused_mixed_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8)),
+                                                                        *((q, (narrow_tile(q) if q == "w4a4_g128_sym" else few_token_tile(q),))
+                                                                          for q in ("w4a4_g128_sym", *(f"w{b}a16_g128_asym" for b in (4, 3, 2, 8))))])),
         # the few-token tiles of 64 channels of every format with 16-bit activations: fp16 and 8-bit weights take 142 registers (three workgroups per CU) where the
         # kernel without them has 125 (four)
         ("groupgemm_hz_fused_a16_few", KernelType.Fused, OrderedDict((q, (few_token_tile(q),)) for q in (*(f"w{b}a16_g128_asym" for b in (4, 3, 2, 8)), "fp16"))),

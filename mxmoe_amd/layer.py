@@ -141,10 +141,10 @@ class MxMoELayer:
             h[e] = _lib.BlockDesc(int(a), int(wb), int(g), 1 if sym else 0, layout, int(ns[e]), int(ks[e]), w.data.data_ptr(), 0 if w.scale is None else w.scale.data_ptr())
         return h
 
-    def _planned_kernel(self, h, t: int, topk: int) -> int:
-        """The kernel that a block's planned launch runs on for t tokens."""
+    def _planned_kernel(self, h, t: int, topk: int, first: bool = False) -> int:
+        """The kernel that a block's planned launch runs on for t tokens (`first`: the first block of the short form)."""
         lib = _lib.load()
-        kid = lib.mxmoe_plan_select_kernel_rows(h, self.cfg.num_experts, t, topk, t if self.cfg.num_shared else 0)
+        kid = lib.mxmoe_layer_kernel(h, self.cfg.num_experts, t, topk, t if self.cfg.num_shared else 0, int(first))
         if kid < 0:
             raise RuntimeError(lib.mxmoe_last_error().decode())
         return kid
@@ -235,7 +235,7 @@ class MxMoELayer:
         down = self._block_descs(self.qp_down, [cfg.hidden] * et, [cfg.inter] * e_cnt + sh, self.w2, False)
         d = _lib.LayerDesc(num_tokens=t, topk=topk, num_experts=e_cnt, has_shared=int(has_shared), hidden=cfg.hidden, inter=cfg.inter, inter_shared=i_sh, rotate=cfg.rotate,
                            had_k=1, had_f=1, h_gate_up=C.cast(gate_up, C.c_void_p), h_down=C.cast(down, C.c_void_p))
-        d.kernel_gate_up, d.kernel_down = self._planned_kernel(gate_up, t, topk), self._planned_kernel(down, t, topk)
+        d.kernel_gate_up, d.kernel_down = self._planned_kernel(gate_up, t, topk, first=True), self._planned_kernel(down, t, topk)
         if not lib.mxmoe_layer_supported(C.byref(d)):
             cache[key] = None
             return None

@@ -54,7 +54,7 @@ def test_layer_on_the_few_token_tiles(tokens, q):
 
     cfg = synth.MoEConfig("t", "test", 6, 2, 512, 640, tokens, num_shared=1, rotate=0)
     layer = MxMoELayer(cfg, formats=[(q, q)] * 7)
-    layer._planned_kernel = lambda *_: _lib.load().mxmoe_find_kernel(b"groupgemm_hz_fused_a16_few")
+    layer._planned_kernel = lambda *_, **__: _lib.load().mxmoe_find_kernel(b"groupgemm_hz_fused_a16_few")
     hidden = synth.make_hidden(cfg)
     ids, w = synth.make_routing(cfg)
     ids[:, 0] = 1
@@ -137,10 +137,10 @@ def test_first_launch_without_a_head(tokens, topk, experts, inter, num_shared, m
     n = experts + (num_shared > 0)
     cfg = S.MoEConfig("t", "test", experts, topk, 512, inter, tokens, num_shared=num_shared, rotate=int(mix not in ("fp16", "wo", "all", "first")))
     layer = MxMoELayer(cfg, formats=[fm[i % len(fm)] for i in range(n)], fp8="fp8" in mix)
-    kid = _lib.load().mxmoe_find_kernel(b"groupgemm_hz_fused_" + {"wo": b"wo_few", "behind": b"wo_few", "int": b"wxax_few", "many": b"all_few", "fp8": b"wxax_e4m3_few",
+    kid = _lib.load().mxmoe_find_kernel(b"groupgemm_hz_fused_" + {"wo": b"wo_few", "behind": b"wo_few", "int": b"wxax_few", "many": b"mixed_few", "fp8": b"wxax_e4m3_few",
                                                                   "many fp8": b"all_e4m3_few"}.get(mix, b"a16_few"))
     planned = layer._planned_kernel
-    layer._planned_kernel = lambda h, t, k: kid if int(h[0].N) == 2 * inter else planned(h, t, k)
+    layer._planned_kernel = lambda h, t, k, **_: kid if int(h[0].N) == 2 * inter else planned(h, t, k)
     gen = torch.Generator().manual_seed(tokens)
     store = torch.randn(tokens * 512 + 8, generator=gen).half().cuda()
     calls = []
@@ -158,3 +158,21 @@ def test_first_launch_without_a_head(tokens, topk, experts, inter, num_shared, m
     layer._short[(tokens, topk)] = None                                  # the form with launches in front
     for c, g in zip(calls, got):
         assert torch.equal(layer(*c), g)
+
+
+def test_first_block_of_a_layer_takes_the_narrow_tiles_up_to_more_experts():
+    """896 blocks of 256 channels: up to 64 tokens, 256 pairs and 12 rows a problem where gate_up starts the layer, not at all elsewhere or in fp8; up to 768 blocks the same choice."""
+    import ctypes as C
+
+    from mxmoe_amd import _lib
+
+    lib = _lib.load()
+
+    def picked(tokens, n, variant=0, first=True, w=4):
+        desc = (_lib.BlockDesc * 8)(*[_lib.BlockDesc(w, w, -1, 1, (C.c_uint8 * 3)(variant, 0, 0), n, 4096, 0, 0) for _ in range(8)])
+        kid = lib.mxmoe_layer_kernel(desc, 8, tokens, 2, 0, int(first))
+        return lib.mxmoe_kernel_name(kid).decode().split("groupgemm_hz_fused_")[-1]
+
+    assert [picked(t, 28672) for t in (4, 48, 49, 64)] == ["wxax_few", "wxax_few", "wxax", "wxax"]
+    assert picked(4, 28672, first=False) == "wxax" and picked(4, 32768 + 256) == "wxax" and picked(4, 28672, 2, w=8) == "wxax_e4m3"
+    assert all(picked(t, 24576) == picked(t, 24576, first=False) for t in (1, 16, 64, 65))

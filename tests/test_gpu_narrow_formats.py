@@ -81,7 +81,7 @@ def test_layer_of_four_formats_on_the_narrow_tiles(tokens):
     cfg = S.MoEConfig("t", "test", 14, 2, 512, 1408, tokens, num_shared=1, rotate=1)
     layer = MxMoELayer(cfg, formats=[fm[i % 5] for i in range(15)], fp8=True)
     kid = _lib.load().mxmoe_find_kernel(b"groupgemm_hz_fused_all_e4m3_few")
-    layer._planned_kernel = lambda *_: kid
+    layer._planned_kernel = lambda *_, **__: kid
     layer.kid_gate_up = layer.kid_down = kid
     hidden = S.make_hidden(cfg).cuda()
     ids, w = S.make_routing(cfg)
@@ -96,7 +96,7 @@ def test_layer_of_four_formats_on_the_narrow_tiles(tokens):
 
 
 def test_lists_with_fp8_take_the_kernels_with_narrow_tiles():
-    """mxmoe_few_row_kernel: the sibling with the same operand variants for few rows, the kernel itself for many, for shapes and formats that no sibling takes, and negative ids as they are."""
+    """mxmoe_few_row_kernel: the sibling with the same operand variants for few rows, without many-token tiles; the kernel itself for many, for shapes and formats that no sibling takes."""
     from mxmoe_amd import _lib
 
     lib = _lib.load()
@@ -106,10 +106,14 @@ def test_lists_with_fp8_take_the_kernels_with_narrow_tiles():
     def picked(kernel, *probs):
         sizes = (_lib.Dim3 * len(probs))(*[_lib.Dim3(m, n, 2048) for m, n, _ in probs])
         qs = (_lib.QParams * len(probs))(*[_lib.QParams(q[0], q[1], q[2], int(q[3])) for *_, q in probs])
-        return name(lib.mxmoe_few_row_kernel(lib.mxmoe_find_kernel(kernel), sizes, qs, len(probs)))
+        kid = lib.mxmoe_few_row_kernel(-1 if kernel is None else lib.mxmoe_find_kernel(kernel), sizes, qs, len(probs))
+        return None if kid < 0 else name(kid)
 
     e4m3, whole = b"groupgemm_hz_fused_wxax_e4m3", b"groupgemm_hz_fused_all_e4m3"
     assert picked(e4m3, (4, 2816, f8), (3, 2816, w4)) == "wxax_e4m3_few" and picked(e4m3, (65, 2816, f8)) == "wxax_e4m3"
     assert picked(b"groupgemm_hz_fused_wxax", (4, 2816, f8)) == "wxax_few"                  # int8 codes: not the fp8 kernels
     assert picked(whole, (4, 2816, f8), (3, 2816, g128)) == "all_e4m3_few" and picked(whole, (4, 2816, f8), (3, 2816, fp)) == "all_e4m3"
-    assert lib.mxmoe_few_row_kernel(-1, None, None, 0) == -1 and lib.mxmoe_few_row_kernel(10 ** 6, None, None, 0) == -2
+    wo = (16, 4, 128, False)
+    assert picked(None, (4, 2816, (8, 8, -1, True)), (3, 2816, wo)) == "mixed_few" and picked(None, (4, 2816, w4), (3, 2816, g128)) == "mixed_few"
+    assert picked(None, (4, 2816, w4)) == "wxax_few" and picked(None, (4, 2816, wo)) == "wo_few" and picked(None, (65, 2816, w4)) is None
+    assert lib.mxmoe_few_row_kernel(-1, None, None, 0) == -1 and lib.mxmoe_few_row_kernel(-3, None, None, 0) == -2 and lib.mxmoe_few_row_kernel(10 ** 6, None, None, 0) == -2
