@@ -962,8 +962,9 @@ inline bool few_rows(const RowSummary& s) {
 // 4096 fp16 327 -> 173 (1), 583 -> 447 (16), 622 -> 521 (32: 8 rows each), 639 -> 614 (48), 642 -> 705 (64): weights of 16 bits outweigh the activations for longer, up to 12 rows.  w8a16 / w2a16 half and
 // half, 64 experts top-6 and a shared one 37 -> 31 (1), 71 -> 65 (8), 103 -> 96 (32), 8 experts 100 -> 80 (1), 204 -> 200 (8), 213 -> 215 (32).
 constexpr int kFewTokenRows = 6, kFewTokenRowsFp16 = 12;
-// Tokens and (token, slot) pairs up to which a planned layer has no head in front of gate_up on the kernels for few rows (layer_first_kernel: one pair per thread of a workgroup).
-constexpr int kDirectTokens = 64, kDirectEntries = 256;
+// Tokens and (token, slot) pairs up to which a planned layer has no head in front of gate_up on the kernels for few rows (layer_first_kernel: one or two pairs per thread of a
+// workgroup).  What that changes in the choice of a kernel (kFewBlocksHeadless) was measured, and holds, up to half as many pairs.
+constexpr int kDirectTokens = 64, kDirectEntries = 512;
 inline bool only_narrow_few_token(const FusedKernel& k) {
   for (const BranchInfo& b : k.branches)
     if (b.a_bits != 16 || b.BN != 64) return false;

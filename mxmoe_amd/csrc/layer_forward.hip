@@ -288,12 +288,14 @@ __global__ void __launch_bounds__(TH) layer_head_kernel(const HeadArgs a, const 
 // Few tokens: a workgroup of gate_up finds its problem from the ids itself, so that the launch waits for no head.  The permutation and the tables of both blocks, which the launches behind
 // need, are made beside it by the first workgroups.  What is left in front is the quantisation of the tokens (layer_tokens_kernel), where first blocks take quantised ones.
 // Grid: (column tiles of a routed expert) x (1 for those, shared_slots rows of the shared expert's tiles, one row per expert that may have tokens).  A workgroup counts the ids in LDS, takes
-// the slot-th expert with rows, lists its rows, and runs their row tiles one after the other (with 256 ids an expert of more than one is rare but under a skewed routing, and its
+// the slot-th expert with rows, lists its rows, and runs their row tiles one after the other (an expert of more than one is rare but under a skewed routing, and its
 // weights come from L2 then).
 // What a launch of few tokens consists of is latency: a layer's, with the head in front -> without, us: 64 experts top-6 and a shared one, w4a16 / w3a16, 29 -> 22 (1 token), 54 -> 46 (8),
 // 77 -> 71 (32), w8a16 / w2a16 31 -> 23 (1), 65 -> 54 (8), 96 -> 85 (32); 60 experts top-4, w4a16 24 -> 18 (1), 55 -> 49 (16), 72 -> 68 (64), skewed 68 -> 64 (64), fp16 35 -> 27 (1),
-// 108 -> 99 (8), 217 -> 212 (64); 8 experts of N = 28 672 / 4096, w4a16 64 -> 58 (1), 134 -> 126 (16).  One id per thread: up to 256 of them, and no more tokens than the kernels for few rows take.
-static_assert(kDirectEntries == kHeadSmall, "one id per thread");
+// 108 -> 99 (8), 217 -> 212 (64); 8 experts of N = 28 672 / 4096, w4a16 64 -> 58 (1), 134 -> 126 (16).  One or two ids per thread: up to 512 of them, and no more tokens than the kernels for few rows take.
+// 257 .. 512 of them, 64 experts top-6 and a shared one, us a layer, head -> none: w4a16 / w3a16 79 -> 74 (44 tokens), 77 -> 70 (52, skewed), w8a16 / w2a16 101 -> 87, 96 -> 84, fp16 249 -> 243 (44), 262 -> 252 (64),
+// skewed 258 -> 249, w4a4 82 -> 78, 83 -> 80, 82 -> 76, w4a4 / w8a8 104 -> 98, 107 -> 101, 104 -> 97, beside fp8 106 -> 99, 108 -> 102, 104 -> 98, four formats 120 -> 112, 124 -> 117, 122 -> 113.
+static_assert(kDirectEntries == 2 * kHeadSmall, "one or two ids per thread");
 struct DirectArgs {
   const mxmoe_block_desc* desc;
   const uint8_t* hidden;
@@ -302,9 +304,10 @@ struct DirectArgs {
   int cols, shared_rows, shared_slots;  // column tiles of a routed expert; rows of the grid that hold a row tile's column tiles of the shared expert, and all of its row tiles'
   int shared_step;                      // rows of such a tile
   unsigned topk_inverse;  // ceil(2^16 / top-k): (i * topk_inverse) >> 16 = i / top-k for i < kDirectEntries and top-k <= 64
+  int entries;            // ids in LDS: one or two per thread
   int tile_lds;           // bytes of LDS that the tiles use
 };
-constexpr size_t direct_lds(int E) { return (size_t)kDirectEntries * 4 + kWaves * kDirectEntries + (size_t)E * 4; }
+constexpr size_t direct_lds(int entries, int E) { return (size_t)entries * 4 + (size_t)kWaves * entries + (size_t)E * 4; }
 
 // A tile type of the launch: whether it is that of a format, and the tag of its activations.  (fp8 or int8 codes: a kernel holds the tile of one of them.)
 template <class T>
@@ -339,7 +342,7 @@ struct DirectTile<WxAxGNarrowTile> {
 
 template <class... Tiles>
 __global__ void __launch_bounds__(kThreads, 3) layer_first_kernel(const HeadArgs a, const PlanPair pair, const DirectArgs x) {
-  static_assert(kThreads == kHeadSmall && ((Tiles::BN == 64) && ...), "one id per thread; 32 outputs a tile");
+  static_assert(kThreads == kHeadSmall && ((Tiles::BN == 64) && ...), "one or two ids per thread; 32 outputs a tile");
   extern __shared__ __align__(16) uint8_t first_lds[];
   const int col0 = blockIdx.x, E = a.E;
   int slot = (int)blockIdx.y - 1;
@@ -349,9 +352,9 @@ __global__ void __launch_bounds__(kThreads, 3) layer_first_kernel(const HeadArgs
       constexpr size_t kPlanBytes = (sizeof(PlanShared) + 15) & ~(size_t)15;
       // (one planner body for every layer: nothing waits for it as long as gate_up runs)
       head_plan<kHeadSmall, true, true>(a, pair, col0, *reinterpret_cast<PlanShared*>(first_lds), reinterpret_cast<int32_t*>(first_lds + kPlanBytes));
-    } else if (col0 == 2 * pair.chunks) {
+    } else if (col0 < 2 * pair.chunks + a.perm_wgs) {
       __builtin_amdgcn_s_setprio(2);
-      head_scatter<kHeadSmall>(a, 0, reinterpret_cast<int32_t*>(first_lds));
+      head_scatter<kHeadSmall>(a, col0 - 2 * pair.chunks, reinterpret_cast<int32_t*>(first_lds));
     }
     return;
   }
@@ -366,13 +369,19 @@ __global__ void __launch_bounds__(kThreads, 3) layer_first_kernel(const HeadArgs
   slot -= x.shared_slots;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int32_t* const all_ids = reinterpret_cast<int32_t*>(first_lds + x.tile_lds);
-  uint8_t* const rows = reinterpret_cast<uint8_t*>(all_ids + kDirectEntries) + wave * kDirectEntries;  // this wave's copy of the problem's entries
-  int32_t* const count = all_ids + kDirectEntries + kWaves * kDirectEntries / 4;
+  uint8_t* const rows = reinterpret_cast<uint8_t*>(all_ids + x.entries) + wave * x.entries;  // this wave's copy of the problem's tokens
+  int32_t* const count = all_ids + x.entries + kWaves * x.entries / 4;
+  const bool two = x.entries > kThreads;
   const int id = (int)threadIdx.x < a.total ? gload<int>(a.ids + threadIdx.x) : -1;
+  const int id2 = two && (int)threadIdx.x + kThreads < a.total ? gload<int>(a.ids + threadIdx.x + kThreads) : -1;
   for (int i = threadIdx.x; i < E; i += kThreads) count[i] = 0;
   __syncthreads();
   all_ids[threadIdx.x] = id;
   if (id >= 0 && id < E) atomicAdd(count + id, 1);
+  if (two) {
+    all_ids[threadIdx.x + kThreads] = id2;
+    if (id2 >= 0 && id2 < E) atomicAdd(count + id2, 1);
+  }
   __syncthreads();
   int e = shared ? E : -1, before = 0;  // the problem's expert; rows of the experts before it
   for (int x0 = 0; x0 < E; x0 += 64) {
@@ -397,7 +406,7 @@ __global__ void __launch_bounds__(kThreads, 3) layer_first_kernel(const HeadArgs
     for (int i0 = 0; i0 < a.total; i0 += 64) {
       const bool mine = all_ids[i0 + lane] == e;
       const uint64_t which = __ballot(mine);
-      if (mine) rows[M + __popcll(which & ((1ull << lane) - 1))] = (uint8_t)(i0 + lane);
+      if (mine) rows[M + __popcll(which & ((1ull << lane) - 1))] = (uint8_t)((i0 + lane) * x.topk_inverse >> 16);
       M += __popcll(which);
     }
     __builtin_amdgcn_wave_barrier();
@@ -415,7 +424,7 @@ __global__ void __launch_bounds__(kThreads, 3) layer_first_kernel(const HeadArgs
   t.tile_n = col;
   t.rows = nullptr;
   const int a_bits = cload(&d->q.a_bits), w_bits = cload(&d->q.w_bits), gsize = cload(&d->q.gsize);
-  auto token_of = [&](int m) { return shared ? m : (int)(rows[m] * x.topk_inverse >> 16); };
+  auto token_of = [&](int m) { return shared ? m : (int)rows[m]; };
   auto run = [&](auto type) {
     using T = typename decltype(type)::type;
     using D = DirectTile<T>;
@@ -625,9 +634,10 @@ int mxmoe_layer_create(const mxmoe_layer_desc* d, void** handle) {
   x.shared_step = d->has_shared && d->h_gate_up[d->num_experts].q.a_bits < 16 && d->h_gate_up[d->num_experts].q.gsize != 128 ? 32 : 16;  // (BM of the format's tile)
   x.shared_slots = x.shared_rows * ((h.T + x.shared_step - 1) / x.shared_step);
   x.topk_inverse = (65536 + d->topk - 1) / d->topk;
+  x.entries = h.total <= kThreads ? kThreads : kDirectEntries;
   x.tile_lds = kg.lds_bytes;
-  f->first_grid = dim3(std::max(x.cols, 2 * f->pair.chunks + 1), 1 + x.shared_slots + std::min(h.total, h.E));
-  f->first_lds = std::max(kg.lds_bytes + direct_lds(h.E), sizeof(PlanShared) + 16 + (size_t)(2 + kHeadSmall / 64 + 2 * kCountCopies) * h.E * sizeof(int32_t));
+  f->first_grid = dim3(std::max(x.cols, 2 * f->pair.chunks + h.perm_wgs), 1 + x.shared_slots + std::min(h.total, h.E));
+  f->first_lds = std::max(kg.lds_bytes + direct_lds(x.entries, h.E), sizeof(PlanShared) + 16 + (size_t)(2 + kHeadSmall / 64 + 2 * kCountCopies) * h.E * sizeof(int32_t));
   if (f->first_lds > 40 * 1024) f->first = nullptr;  // (counters of many experts would take the room of a workgroup)
 
   RowsBehind& r = f->rows;

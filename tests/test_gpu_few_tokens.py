@@ -112,13 +112,14 @@ def test_lists_that_the_few_token_tiles_take():
     assert picked(*[(4, 2816, 2048, fp)] * 20, (65, 2816, 2048, fp)) == "fp16"
 
 
-# tokens, top-k, experts, inter, shared experts, formats: one token; a partial row tile; 256 entries, the most; more experts than a wave has lanes and than one launch's tables hold;
+# tokens, top-k, experts, inter, shared experts, formats: one token; a partial row tile; 256 and 512 entries, the most of one and two a thread, and a few more than 256; more experts than a wave has lanes and than one launch's tables hold;
 # two and four row tiles of the shared expert and of one expert; shared columns that end inside the grid's rows; quantised and rotated second blocks
 @pytest.mark.gpu
 @pytest.mark.parametrize("tokens,topk,experts,inter,num_shared,mix", [
     (1, 1, 8, 1408, 0, "fp16"), (1, 6, 64, 1408, 2, "wo"), (17, 3, 70, 96, 3, "fp16"), (33, 6, 130, 160, 1, "all"), (64, 4, 60, 256, 4, "wo"), (64, 4, 60, 352, 0, "all"),
     (32, 8, 24, 1408, 1, "behind"), (5, 2, 66, 640, 2, "behind"), (16, 16, 8, 512, 1, "fp16"),
     (1, 4, 60, 1408, 4, "int"), (64, 4, 60, 1408, 1, "int"), (33, 2, 9, 640, 2, "many"), (64, 4, 130, 1408, 1, "many"), (1, 1, 10, 512, 0, "many"),
+    (43, 6, 70, 96, 3, "fp16"), (64, 8, 64, 1408, 2, "wo"), (64, 6, 24, 1408, 1, "int"), (57, 7, 130, 640, 1, "many"),
     (40, 6, 64, 1408, 1, "fp8"), (64, 2, 12, 512, 0, "many fp8"), (17, 6, 64, 1408, 2, "many fp8"),
 ])
 def test_first_launch_without_a_head(tokens, topk, experts, inter, num_shared, mix):
