@@ -934,7 +934,8 @@ inline RowSummary row_summary(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_
 // (groupgemm_hz_fused_all_e4m3_few: tiles of 64 channels alone, 155 registers; with the many-token tiles beside them, 255 registers, 8 experts, 64 tokens, took 343 us, not 265), four formats: 60 experts
 // 54 -> 32 (1), 78 -> 62 (8), 100 -> 101 (32); with a shared expert 75 -> 42 (1), 110 -> 92 (16), 140 -> 124 (64); 8 experts 228 -> 84 (1), 307 -> 213 (8), 326 -> 265 (64).
 // Where such a layer starts with gate_up on these kernels (layer_first_kernel, 4 us less in front of it), up to 1024 blocks and 12 rows: 8 experts, first block of 896 blocks, us a layer, w4a4 119 -> 115 (4
-// tokens), 148 -> 144 (32), w4a4 / w8a8 skewed 146 -> 137 (4), 173 -> 167 (16), 201 -> 199 (48), 211 -> 219 (64), with w4a16 208 -> 202 (16), 212 -> 210 (48), 216 -> 222 (64).
+// tokens), 148 -> 144 (32), w4a4 / w8a8 skewed 146 -> 137 (4), 173 -> 167 (16), 201 -> 199 (48), 211 -> 219 (64), with w4a16 208 -> 202 (16), 212 -> 210 (48), 216 -> 222 (64);
+// 90 experts of N = 2816 top-6 (990 blocks) w4a4 96 -> 91 (44), 98 -> 95 (64), skewed 85 -> 76, 90 -> 83, w4a4 / w8a8 125 -> 117, 126 -> 119, skewed 105 -> 94, 114 -> 107.
 constexpr int kFewRowsMax = 64, kFewBlocks = 768, kFewBlocksHeadless = 1024, kFewBlocksMin = 8;
 inline bool holds_narrow(const FusedKernel& k) { return plan_of(k).narrow; }
 // Rows per problem, on average, up to which those kernels are chosen.
@@ -961,10 +962,13 @@ inline bool few_rows(const RowSummary& s) {
 // fp16 67 -> 35 (1 token), 86 -> 73 (4), 131 -> 108 (8), 166 -> 158 (16), 207 -> 196 (32), 216 -> 217 (64), with a shared expert 143 -> 68 (1), 208 -> 141 (16), 288 -> 232 (64); 8 experts of N = 28 672 /
 // 4096 fp16 327 -> 173 (1), 583 -> 447 (16), 622 -> 521 (32: 8 rows each), 639 -> 614 (48), 642 -> 705 (64): weights of 16 bits outweigh the activations for longer, up to 12 rows.  w8a16 / w2a16 half and
 // half, 64 experts top-6 and a shared one 37 -> 31 (1), 71 -> 65 (8), 103 -> 96 (32), 8 experts 100 -> 80 (1), 204 -> 200 (8), 213 -> 215 (32).
-constexpr int kFewTokenRows = 6, kFewTokenRowsFp16 = 12;
+// Where a layer starts with gate_up on these kernels (no head in front of it), up to 8 rows, us a layer: 64 experts top-6 and a shared one, 58 tokens w4a16 / w3a16 80 -> 74, skewed 80 -> 71, w8a16 / w2a16
+// 108 -> 92, 106 -> 89, 64 tokens 81 -> 75, 108 -> 93; 60 experts top-8, 64 tokens 76 -> 70, 100 -> 88; 8 experts of N = 28 672 / 4096 w4a16 161 -> 154 (28), 172 -> 166 (32), 175 -> 172 (40), 180 -> 180 (48),
+// w8a16 / w2a16 219 -> 210 (28), 222 -> 219 (32), 226 -> 230 (40), 234 -> 243 (48).
+constexpr int kFewTokenRows = 6, kFewTokenRowsHeadless = 8, kFewTokenRowsFp16 = 12;
 // Tokens and (token, slot) pairs up to which a planned layer has no head in front of gate_up on the kernels for few rows (layer_first_kernel: one or two pairs per thread of a
-// workgroup).  What that changes in the choice of a kernel (kFewBlocksHeadless) was measured, and holds, up to half as many pairs.
-constexpr int kDirectTokens = 64, kDirectEntries = 512;
+// workgroup).
+constexpr int kDirectTokens = 128, kDirectEntries = 512;
 inline bool only_narrow_few_token(const FusedKernel& k) {
   for (const BranchInfo& b : k.branches)
     if (b.a_bits != 16 || b.BN != 64) return false;
@@ -986,7 +990,7 @@ int few_row_kernel(const RowSummary& s, Covers&& covers) {
     if (kid >= 0) return kid;
   }
   if (4 * s.tall > s.live) return -1;
-  if (s.max_rows <= kFewRowsMax && s.rows <= (s.fp16 ? kFewTokenRowsFp16 : kFewTokenRows) * s.live && s.blocks >= kFewBlocksMin) {
+  if (s.max_rows <= kFewRowsMax && s.rows <= (s.fp16 ? kFewTokenRowsFp16 : s.headless ? kFewTokenRowsHeadless : kFewTokenRows) * s.live && s.blocks >= kFewBlocksMin) {
     const int kid = first(only_narrow_few_token);
     if (kid >= 0) return kid;
   }

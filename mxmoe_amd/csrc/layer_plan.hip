@@ -201,7 +201,7 @@ static int select_kernel_rows(const mxmoe_block_desc* h_desc, int num_experts, i
   s.max_rows = std::max<long>(s.max_rows, num_tokens);  // one expert may get them all
   // an uneven routing has problems of several 16-row tiles well before the average reaches 16
   if (routed > 12l * num_experts) s.tall = s.live;
-  s.headless = headless && num_tokens <= kDirectTokens && 2 * routed <= kDirectEntries;
+  s.headless = headless && num_tokens <= kFewRowsMax && routed <= kDirectEntries;
   const int few = few_row_kernel(s, [&](const FusedKernel& k) { return covers_blocks(k, h_desc, et); });
   return few >= 0 && resolve_kernel(few, h_desc, et) == few ? few : plain;
 }

@@ -119,7 +119,7 @@ def test_lists_that_the_few_token_tiles_take():
     (1, 1, 8, 1408, 0, "fp16"), (1, 6, 64, 1408, 2, "wo"), (17, 3, 70, 96, 3, "fp16"), (33, 6, 130, 160, 1, "all"), (64, 4, 60, 256, 4, "wo"), (64, 4, 60, 352, 0, "all"),
     (32, 8, 24, 1408, 1, "behind"), (5, 2, 66, 640, 2, "behind"), (16, 16, 8, 512, 1, "fp16"),
     (1, 4, 60, 1408, 4, "int"), (64, 4, 60, 1408, 1, "int"), (33, 2, 9, 640, 2, "many"), (64, 4, 130, 1408, 1, "many"), (1, 1, 10, 512, 0, "many"),
-    (43, 6, 70, 96, 3, "fp16"), (64, 8, 64, 1408, 2, "wo"), (64, 6, 24, 1408, 1, "int"), (57, 7, 130, 640, 1, "many"),
+    (43, 6, 70, 96, 3, "fp16"), (64, 8, 64, 1408, 2, "wo"), (64, 6, 24, 1408, 1, "int"), (57, 7, 130, 640, 1, "many"), (128, 4, 60, 512, 1, "all"), (128, 4, 12, 1408, 1, "int"),
     (40, 6, 64, 1408, 1, "fp8"), (64, 2, 12, 512, 0, "many fp8"), (17, 6, 64, 1408, 2, "many fp8"),
 ])
 def test_first_launch_without_a_head(tokens, topk, experts, inter, num_shared, mix):
@@ -162,7 +162,7 @@ def test_first_launch_without_a_head(tokens, topk, experts, inter, num_shared, m
 
 
 def test_first_block_of_a_layer_takes_the_narrow_tiles_up_to_more_experts():
-    """896 blocks of 256 channels: up to 64 tokens, 256 pairs and 12 rows a problem where gate_up starts the layer, not at all elsewhere or in fp8; up to 768 blocks the same choice."""
+    """896 blocks of 256 channels: up to 64 tokens, 512 pairs and 12 rows a problem where gate_up starts the layer, not at all elsewhere or in fp8; up to 768 blocks the same choice."""
     import ctypes as C
 
     from mxmoe_amd import _lib
