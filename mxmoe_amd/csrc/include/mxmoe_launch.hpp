@@ -888,11 +888,12 @@ struct RowSummary {
   long blocks = 0;                // of 256 channels
   uint32_t max_k = 0;
   bool headless = false;          // a planned layer of few tokens: no head in front of gate_up on these kernels (layer_first_kernel)
-  bool w4a4 = false, w8a8 = false, other = false;  // formats among them
+  bool w4a4 = false, w8a8 = false, other = false, any_fp16 = false;  // formats among them
   bool fp16 = true;                                // no other format than this one
   void add_format(Fmt f) {
     (f == Fmt::W4A4 ? w4a4 : f == Fmt::W8A8 ? w8a8 : other) = true;
     fp16 = fp16 && f == Fmt::FP16;
+    any_fp16 = any_fp16 || f == Fmt::FP16;
   }
   void add(Fmt f, long m, uint32_t N, uint32_t K) {
     if (m == 0) return;
@@ -936,7 +937,17 @@ inline RowSummary row_summary(const mxmoe_dim3* h_sizes, const mxmoe_qparams* h_
 // Where such a layer starts with gate_up on these kernels (layer_first_kernel, 4 us less in front of it), up to 1024 blocks and 12 rows: 8 experts, first block of 896 blocks, us a layer, w4a4 119 -> 115 (4
 // tokens), 148 -> 144 (32), w4a4 / w8a8 skewed 146 -> 137 (4), 173 -> 167 (16), 201 -> 199 (48), 211 -> 219 (64), with w4a16 208 -> 202 (16), 212 -> 210 (48), 216 -> 222 (64);
 // 90 experts of N = 2816 top-6 (990 blocks) w4a4 96 -> 91 (44), 98 -> 95 (64), skewed 85 -> 76, 90 -> 83, w4a4 / w8a8 125 -> 117, 126 -> 119, skewed 105 -> 94, 114 -> 107.
+// Where a layer starts with gate_up, up to 128 tokens: kDirectTokens.
 constexpr int kFewRowsMax = 64, kFewBlocks = 768, kFewBlocksHeadless = 1024, kFewBlocksMin = 8;
+// Tokens and (token, slot) pairs up to which a planned layer has no head in front of gate_up on the kernels for few rows (layer_first_kernel: one or two pairs per thread of a
+// workgroup).  Above 64 tokens, us a layer, wide kernels behind a head -> without, evenly routed / skewed: 60 experts top-4 w4a4 80 -> 73 / 72 -> 64 (66 tokens), 80 -> 75 / 82 -> 73 (128), w4a4 / w8a8
+// 99 -> 88 / 89 -> 79, 102 -> 93 / 101 -> 91, w4a4 / w8a8 / w4a16 102 -> 90 / 92 -> 81, 105 -> 95 / 103 -> 95, w4a16 / w3a16 75 -> 65 / 84 -> 65, 78 -> 70 / 97 -> 81, w8a16 / w2a16 96 -> 82 / 98 -> 79, 99 -> 88 /
+// 105 -> 97, with a shared expert 97 -> 89, 114 -> 107, 129 -> 121, 95 -> 78, 112 -> 97 (66); 64 experts top-6 and a shared one 93 -> 88, 117 -> 111, 122 -> 115, 96 -> 81, 114 -> 98 (84); 32 experts top-4 w4a4 57 -> 52 / 66 -> 57 (96), w4a4 / w8a8 69 -> 65 / 76 -> 67 (127),
+// w4a16 / w3a16 52 -> 45 / 80 -> 58 (72); 24 experts top-2, K = 4096, w4a4 74 -> 65 / 68 -> 64 (100).  fp16 (weights read
+// once per 16 rows from L2 outweigh the head) 223 -> 210 / 186 -> 189 (66), 223 -> 214 / 224 -> 231 (128), with a shared expert 278 -> 298: up to 64.
+constexpr int kDirectTokens = 128, kDirectEntries = 512;
+// The largest problem that those kernels take in a launch.
+inline long few_rows_max(const RowSummary& s) { return s.headless && !s.any_fp16 ? kDirectTokens : kFewRowsMax; }
 inline bool holds_narrow(const FusedKernel& k) { return plan_of(k).narrow; }
 // Rows per problem, on average, up to which those kernels are chosen.
 inline int few_rows_limit(const RowSummary& s) {
@@ -947,7 +958,7 @@ inline int few_rows_limit(const RowSummary& s) {
   return s.max_k < 2048 ? 8 : 12;
 }
 inline bool few_rows(const RowSummary& s) {
-  if (!(s.w4a4 || s.w8a8) || s.max_rows > kFewRowsMax || s.blocks < kFewBlocksMin || s.blocks > (s.headless ? kFewBlocksHeadless : kFewBlocks)) return false;
+  if (!(s.w4a4 || s.w8a8) || s.max_rows > few_rows_max(s) || s.blocks < kFewBlocksMin || s.blocks > (s.headless ? kFewBlocksHeadless : kFewBlocks)) return false;
   if (s.blocks > kPoleBlocks && s.blocks <= 256 && s.max_rows > 32) return false;
   return s.rows <= few_rows_limit(s) * s.live;
 }
@@ -962,13 +973,15 @@ inline bool few_rows(const RowSummary& s) {
 // fp16 67 -> 35 (1 token), 86 -> 73 (4), 131 -> 108 (8), 166 -> 158 (16), 207 -> 196 (32), 216 -> 217 (64), with a shared expert 143 -> 68 (1), 208 -> 141 (16), 288 -> 232 (64); 8 experts of N = 28 672 /
 // 4096 fp16 327 -> 173 (1), 583 -> 447 (16), 622 -> 521 (32: 8 rows each), 639 -> 614 (48), 642 -> 705 (64): weights of 16 bits outweigh the activations for longer, up to 12 rows.  w8a16 / w2a16 half and
 // half, 64 experts top-6 and a shared one 37 -> 31 (1), 71 -> 65 (8), 103 -> 96 (32), 8 experts 100 -> 80 (1), 204 -> 200 (8), 213 -> 215 (32).
-// Where a layer starts with gate_up on these kernels (no head in front of it), up to 8 rows, us a layer: 64 experts top-6 and a shared one, 58 tokens w4a16 / w3a16 80 -> 74, skewed 80 -> 71, w8a16 / w2a16
+// Where a layer starts with gate_up on these kernels (no head in front of it), up to 10 rows, or 8 where K is above 2048 and the head less of the layer's time, us a layer: 64 experts top-6 and a shared one, 58 tokens w4a16 / w3a16 80 -> 74, skewed 80 -> 71, w8a16 / w2a16
 // 108 -> 92, 106 -> 89, 64 tokens 81 -> 75, 108 -> 93; 60 experts top-8, 64 tokens 76 -> 70, 100 -> 88; 8 experts of N = 28 672 / 4096 w4a16 161 -> 154 (28), 172 -> 166 (32), 175 -> 172 (40), 180 -> 180 (48),
 // w8a16 / w2a16 219 -> 210 (28), 222 -> 219 (32), 226 -> 230 (40), 234 -> 243 (48).
-constexpr int kFewTokenRows = 6, kFewTokenRowsHeadless = 8, kFewTokenRowsFp16 = 12;
-// Tokens and (token, slot) pairs up to which a planned layer has no head in front of gate_up on the kernels for few rows (layer_first_kernel: one or two pairs per thread of a
-// workgroup).
-constexpr int kDirectTokens = 128, kDirectEntries = 512;
+constexpr int kFewTokenRows = 6, kFewTokenRowsHeadless = 10, kFewTokenRowsHeadlessLong = 8, kFewTokenRowsFp16 = 12;
+inline int few_token_rows(const RowSummary& s) {
+  if (s.fp16) return kFewTokenRowsFp16;
+  if (!s.headless) return kFewTokenRows;
+  return s.max_k > 2048 ? kFewTokenRowsHeadlessLong : kFewTokenRowsHeadless;
+}
 inline bool only_narrow_few_token(const FusedKernel& k) {
   for (const BranchInfo& b : k.branches)
     if (b.a_bits != 16 || b.BN != 64) return false;
@@ -990,7 +1003,7 @@ int few_row_kernel(const RowSummary& s, Covers&& covers) {
     if (kid >= 0) return kid;
   }
   if (4 * s.tall > s.live) return -1;
-  if (s.max_rows <= kFewRowsMax && s.rows <= (s.fp16 ? kFewTokenRowsFp16 : s.headless ? kFewTokenRowsHeadless : kFewTokenRows) * s.live && s.blocks >= kFewBlocksMin) {
+  if (s.max_rows <= few_rows_max(s) && s.rows <= few_token_rows(s) * s.live && s.blocks >= kFewBlocksMin) {
     const int kid = first(only_narrow_few_token);
     if (kid >= 0) return kid;
   }

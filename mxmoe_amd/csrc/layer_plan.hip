@@ -201,7 +201,7 @@ static int select_kernel_rows(const mxmoe_block_desc* h_desc, int num_experts, i
   s.max_rows = std::max<long>(s.max_rows, num_tokens);  // one expert may get them all
   // an uneven routing has problems of several 16-row tiles well before the average reaches 16
   if (routed > 12l * num_experts) s.tall = s.live;
-  s.headless = headless && num_tokens <= kFewRowsMax && routed <= kDirectEntries;
+  s.headless = headless && num_tokens <= kDirectTokens && routed <= kDirectEntries;
   const int few = few_row_kernel(s, [&](const FusedKernel& k) { return covers_blocks(k, h_desc, et); });
   return few >= 0 && resolve_kernel(few, h_desc, et) == few ? few : plain;
 }
@@ -211,7 +211,7 @@ int mxmoe_plan_select_kernel_rows(const mxmoe_block_desc* h_desc, int num_expert
 }
 
 int mxmoe_layer_kernel(const mxmoe_block_desc* h_desc, int num_experts, int num_tokens, int topk, int shared_rows, int first) {
-  // (the kernels' integer and fp16 sums are the same whichever runs; fp8 ones are not to the last bit, and stay where a list of the same rows would run)
+  // (integer sums are the same whichever kernel runs; fp8 ones are not to the last bit, and stay where a list of the same rows would run, nor are those of 16-bit activations in tiles of many tokens)
   const int et = num_experts + (shared_rows > 0 ? 1 : 0);
   bool fp8 = false;
   for (int i = 0; h_desc && i < et; ++i) fp8 = fp8 || wants_fp8(h_desc[i].q);

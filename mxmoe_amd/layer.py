@@ -235,7 +235,8 @@ class MxMoELayer:
         down = self._block_descs(self.qp_down, [cfg.hidden] * et, [cfg.inter] * e_cnt + sh, self.w2, False)
         d = _lib.LayerDesc(num_tokens=t, topk=topk, num_experts=e_cnt, has_shared=int(has_shared), hidden=cfg.hidden, inter=cfg.inter, inter_shared=i_sh, rotate=cfg.rotate,
                            had_k=1, had_f=1, h_gate_up=C.cast(gate_up, C.c_void_p), h_down=C.cast(down, C.c_void_p))
-        first = cfg.rotate != 2 or all(int(q[0]) < 16 for q in self.qp_gate_up)  # (rotated fp16 tokens are made by a head in front of gate_up)
+        # (what a first block needs to start the layer: rotated fp16 tokens are made by a head in front of it)
+        first = (cfg.rotate != 2 or all(int(q[0]) < 16 for q in self.qp_gate_up)) and cfg.inter % 32 == 0 and topk <= 64
         d.kernel_gate_up, d.kernel_down = self._planned_kernel(gate_up, t, topk, first=first), self._planned_kernel(down, t, topk)
         if not lib.mxmoe_layer_supported(C.byref(d)):
             cache[key] = None

@@ -177,3 +177,28 @@ def test_first_block_of_a_layer_takes_the_narrow_tiles_up_to_more_experts():
     assert [picked(t, 28672) for t in (4, 48, 49, 64)] == ["wxax_few", "wxax_few", "wxax", "wxax"]
     assert picked(4, 28672, first=False) == "wxax" and picked(4, 32768 + 256) == "wxax" and picked(4, 28672, 2, w=8) == "wxax_e4m3"
     assert all(picked(t, 24576) == picked(t, 24576, first=False) for t in (1, 16, 64, 65))
+
+
+def test_first_block_of_a_layer_takes_the_few_row_kernels_up_to_128_tokens():
+    """Where gate_up starts the layer: 128 tokens, 512 pairs, 10 weight-only rows an expert (8 of a K above 2048), 64 tokens with fp16 weights among them; elsewhere 64 tokens and 6 rows."""
+    import ctypes as C
+
+    from mxmoe_amd import _lib
+
+    lib = _lib.load()
+
+    def picked(tokens, topk, formats, experts=60, shared=0, k=2048, first=True):
+        n = experts + (shared > 0)
+        desc = (_lib.BlockDesc * n)(*[_lib.BlockDesc(*formats[i % len(formats)], (C.c_uint8 * 3)(0, 0, 0), 2816, k, 0, 0) for i in range(n)])
+        kid = lib.mxmoe_layer_kernel(desc, experts, tokens, topk, shared, int(first))
+        assert kid >= 0, lib.mxmoe_last_error()
+        return lib.mxmoe_kernel_name(kid).decode().split("groupgemm_hz_fused_")[-1]
+
+    w4a4, w8a8, w4, w8, fp = (4, 4, -1, 1), (8, 8, -1, 1), (16, 4, 128, 0), (16, 8, 128, 0), (16, 16, -1, 1)
+    assert [picked(t, 4, [w4a4]) for t in (64, 65, 128, 129)] == ["wxax_few", "wxax_few", "wxax_few", "wxax"]
+    assert picked(85, 6, [w4a4]) == "wxax_few" and picked(86, 6, [w4a4]) == "wxax" and picked(65, 4, [w4a4], first=False) == "wxax"
+    assert picked(128, 4, [w4a4, w8a8, w4]) == "mixed_few" and picked(64, 8, [w4]) == "wo_few" and picked(128, 4, [w8, w4]) == "a16_few"
+    assert picked(80, 6, [w4], shared=80) == "wo_few" and picked(85, 6, [w4], experts=50) == "wo"
+    assert picked(48, 4, [w4], experts=24, k=4096) == "wo_few" and picked(49, 4, [w4], experts=24, k=4096) != "wo_few"
+    assert picked(64, 4, [fp]) == "a16_few" and picked(65, 4, [fp]) == "fp16" and picked(65, 4, [w4, fp]) != "a16_few"
+    assert picked(65, 4, [w4], first=False) == "wo"
