@@ -448,26 +448,57 @@ __global__ void __launch_bounds__(kHeadSmall) layer_tokens_kernel(const HeadArgs
   if (t < a.T) head_token<NI>(a, t, threadIdx.x & 63);
 }
 
-// The launch for the registered kernel of a layer's first block: the kernels for few rows have one, of their 64-channel tiles.
+// A launch for first blocks of few tokens, and its tiles.
 using LaunchFirstFn = void (*)(const HeadArgs&, const PlanPair&, const DirectArgs&, dim3, size_t, hipStream_t);
+struct FirstLaunch {
+  LaunchFirstFn fn;
+  std::vector<BranchInfo> tiles;
+};
 template <class... Tiles>
 void launch_first(const HeadArgs& a, const PlanPair& pair, const DirectArgs& x, dim3 grid, size_t lds, hipStream_t s) {
   hipLaunchKernelGGL((layer_first_kernel<Tiles...>), grid, dim3(kThreads), lds, s, a, pair, x);
 }
+template <class... Tiles>
+FirstLaunch first_of() {
+  return {&launch_first<Tiles...>, {BranchOf<Tiles>::get()...}};
+}
 template <int WBITS>
 using FewTokenTile = SkinnyWoTile<WBITS, 64, 1, 3>;
-static LaunchFirstFn first_launch_of(const FusedKernel& k) {
-  auto holds = [&](Fmt f) { return std::any_of(k.branches.begin(), k.branches.end(), [&](const BranchInfo& b) { return b.fmt == f; }); };
-  if (only_narrow_few_token(k)) {
-    if (holds(Fmt::W8A16) || holds(Fmt::FP16)) return &launch_first<FewTokenTile<4>, FewTokenTile<3>, FewTokenTile<2>, FewTokenTile<8>, FewTokenTile<16>>;
-    return &launch_first<FewTokenTile<4>, FewTokenTile<3>, FewTokenTile<2>>;
+
+// Whether a launch's tile computes what kernel k does for a block of format f, to the bit, whatever its rows: k has that tile, and where its tables could name another one of the format, the sums are the
+// same in any (integers; group-scaled w4a4, whose additions are in the order of the groups).
+static bool same_sums(const FusedKernel& k, Fmt f, const BranchInfo& tile) {
+  bool has = false;
+  for (const BranchInfo& b : k.branches) {
+    if (b.fmt != f) continue;
+    const bool same = b.BM == tile.BM && b.BN == tile.BN && b.variant == tile.variant;
+    if (!same && (b.variant || tile.variant || !(integer_sums((int)f) || f == Fmt::W4A4G128))) return false;
+    has = has || same;
   }
-  if (!holds_narrow(k)) return nullptr;
-  const bool others = holds(Fmt::W4A16), fp8 = kernel_variant(k, Fmt::W8A8) == kVariantFp8;
-  if (fp8 && others) return &launch_first<WxAxNarrowTile<Op::I4>, WxAxNarrowTile<Op::F8>, WxAxGNarrowTile, FewTokenTile<4>, FewTokenTile<3>, FewTokenTile<2>, FewTokenTile<8>>;
-  if (fp8) return &launch_first<WxAxNarrowTile<Op::I4>, WxAxNarrowTile<Op::F8>>;
-  if (others) return &launch_first<WxAxNarrowTile<Op::I4>, WxAxNarrowTile<Op::I8>, WxAxGNarrowTile, FewTokenTile<4>, FewTokenTile<3>, FewTokenTile<2>, FewTokenTile<8>>;
-  return &launch_first<WxAxNarrowTile<Op::I4>, WxAxNarrowTile<Op::I8>>;
+  return has;
+}
+
+// The launch for a layer whose first block runs on kernel k: the one of fewest formats that takes each block as k would, or null (a kernel for many rows; one whose tables may take a larger tile with other
+// sums than the 64-channel one's).
+static LaunchFirstFn first_launch_of(const FusedKernel& k, const mxmoe_block_desc* h_desc, int et) {
+  using I4 = WxAxNarrowTile<Op::I4>;
+  using I8 = WxAxNarrowTile<Op::I8>;
+  using F8 = WxAxNarrowTile<Op::F8>;
+  static const FirstLaunch launches[] = {
+      first_of<FewTokenTile<4>, FewTokenTile<3>, FewTokenTile<2>>(),
+      first_of<I4, I8>(),
+      first_of<I4, F8>(),
+      first_of<FewTokenTile<4>, FewTokenTile<3>, FewTokenTile<2>, FewTokenTile<8>, FewTokenTile<16>>(),
+      first_of<I4, I8, WxAxGNarrowTile, FewTokenTile<4>, FewTokenTile<3>, FewTokenTile<2>, FewTokenTile<8>>(),
+      first_of<I4, F8, WxAxGNarrowTile, FewTokenTile<4>, FewTokenTile<3>, FewTokenTile<2>, FewTokenTile<8>>(),
+  };
+  auto takes = [&](const FirstLaunch& l, Fmt f) { return std::any_of(l.tiles.begin(), l.tiles.end(), [&](const BranchInfo& t) { return t.fmt == f && same_sums(k, f, t); }); };
+  for (const FirstLaunch& l : launches) {
+    bool all = true;
+    for (int i = 0; i < et && all; ++i) all = takes(l, (Fmt)fmt_of(h_desc[i].q));
+    if (all) return l.fn;
+  }
+  return nullptr;
 }
 
 // What a layer keeps for one (tokens, top-k): its description and both launches' planning parameters.
@@ -621,7 +652,7 @@ int mxmoe_layer_create(const mxmoe_layer_desc* d, void** handle) {
     const int n = i < d->num_experts ? d->inter : d->inter_shared;
     plain = plain && (int)d->h_gate_up[i].N == 2 * n && (int)d->h_gate_up[i].K == d->hidden && n % 32 == 0;
   }
-  f->first = plain ? first_launch_of(kg) : nullptr;
+  f->first = plain ? first_launch_of(kg, d->h_gate_up, et) : nullptr;
   DirectArgs& x = f->direct;
   x = DirectArgs{};
   x.desc = d->d_gate_up;

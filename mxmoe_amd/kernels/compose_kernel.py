@@ -211,8 +211,8 @@ def default_kernel_specs(arch: str = "gfx950"):
         ("groupgemm_hz_fused_wxax_few", KernelType.Fused, OrderedDict((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8))),
         ("groupgemm_hz_fused_all_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, w8)), *wo_all.items(),
                                                                        ("w8a16_g128_asym", _pick(arch, "w8a16_g128_asym", (16, 128), (32, 128), (128, 256), (128, 128)))])),
-        # the two kernels with narrow tiles for 8-bit operands in fp8
-        ("groupgemm_hz_fused_wxax_e4m3_few", KernelType.Fused, OrderedDict((q, (narrow_tile(q), *_pick(arch, q, (64, 256)))) for q in (w4, f8))),
+        # the two kernels with narrow tiles for 8-bit operands in fp8: for these the narrow tile alone, so that a problem's sums do not hang on its rows, nor on which form of a layer runs it
+        ("groupgemm_hz_fused_wxax_e4m3_few", KernelType.Fused, OrderedDict([(w4, (narrow_tile(w4), *_pick(arch, w4, (64, 256)))), (f8, (narrow_tile(f8),))])),
         ("groupgemm_hz_fused_all_e4m3_few", KernelType.Fused, OrderedDict([*((q, (narrow_tile(q),)) for q in (w4, f8, "w4a4_g128_sym")),
                                                                            *((f"w{b}a16_g128_asym", (few_token_tile(f"w{b}a16_g128_asym"),)) for b in (4, 3, 2, 8))])),
         # the same without many-token tiles (161 registers, three workgroups per CU, where those take 255), and with group-scaled w4a4: for layers of few tokens

@@ -202,3 +202,48 @@ def test_first_block_of_a_layer_takes_the_few_row_kernels_up_to_128_tokens():
     assert picked(48, 4, [w4], experts=24, k=4096) == "wo_few" and picked(49, 4, [w4], experts=24, k=4096) != "wo_few"
     assert picked(64, 4, [fp]) == "a16_few" and picked(65, 4, [fp]) == "fp16" and picked(65, 4, [w4, fp]) != "a16_few"
     assert picked(65, 4, [w4], first=False) == "wo"
+
+
+@pytest.mark.parametrize("kernel", ["groupgemm_hz_fused_wxax_e4m3_few", "groupgemm_hz_fused_all_e4m3_few"])
+def test_fp8_problems_of_few_rows_have_one_tile(kernel):
+    """Whatever the rows and the number of problems: the launch that starts a layer has that tile alone, and sums in another one are not the same to the bit."""
+    import ctypes as C
+
+    from mxmoe_amd import _lib
+
+    lib = _lib.load()
+    kid = lib.mxmoe_find_kernel(kernel.encode())
+    for count, n, k in ((1, 4096, 14336), (8, 2816, 2048), (60, 2816, 2048), (60, 2048, 1408)):
+        for m in (1, 31, 32, 33, 40, 64, 65, 128, 200):
+            sizes = (_lib.Dim3 * count)(*[_lib.Dim3(m if i == 0 else 3, n, k) for i in range(count)])
+            qs = (_lib.QParams * count)(*[_lib.QParams(8, 8, -1, 1)] * count)
+            branch, tiles = (C.c_int32 * count)(), C.c_int32(0)
+            assert lib.mxmoe_group_gemm_plan(kid, sizes, qs, count, branch, C.byref(tiles)) == 1000 + kid
+            assert len(set(branch)) == 1, (count, m, list(branch)[:2])
+            assert tiles.value == -(-n // 64) * (count - 1 + -(-m // 32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [33, 40, 64])
+@pytest.mark.parametrize("mix", ["fp8", "w4a4 and fp8"])
+def test_fp8_layer_with_and_without_a_head(tokens, mix):
+    """More than 32 rows of one expert and of the shared one, K = 2048, more than 256 blocks of channels, second blocks in fp16 (nothing is requantised behind the sums), tokens of values
+    of many sizes (the sums of normal ones hardly ever hang on their order): identical outputs of the layer that starts with gate_up and of the one with launches in front, on the kernel that the layer takes by itself."""
+    from mxmoe_amd import _lib, synth as S
+    from mxmoe_amd.layer import MxMoELayer
+
+    fm = [(S.W8A8, S.FP16)] if mix == "fp8" else [(S.W8A8, S.FP16), (S.W4A4, S.FP16)]
+    cfg = S.MoEConfig("t", "test", 30, 2, 2048, 1408, tokens, num_shared=1, rotate=0)
+    layer = MxMoELayer(cfg, formats=[fm[i % len(fm)] for i in range(31)], fp8=True)
+    gen = torch.Generator().manual_seed(tokens)
+    hidden = (torch.randn(tokens, 2048, generator=gen) * torch.exp(2 * torch.randn(tokens, 2048, generator=gen)) / 64).half().cuda()
+    ids, w = S.make_routing(cfg)
+    ids[:, 0] = 2
+    ids, w = ids.cuda(), w.cuda()
+    got = layer(hidden, ids, w).clone()
+    assert torch.isfinite(got).all()
+    kid = layer._planned_kernel(layer._block_descs(layer.qp_gate_up, [2816] * 31, [2048] * 31, layer.w13, False), tokens, 2, first=True)
+    assert _lib.load().mxmoe_kernel_name(kid).endswith(b"groupgemm_hz_fused_wxax_e4m3_few")
+    assert layer._short[(tokens, 2)] is not None
+    layer._short[(tokens, 2)] = None
+    assert torch.equal(layer(hidden, ids, w), got)
