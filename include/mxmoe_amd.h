@@ -254,8 +254,8 @@ size_t mxmoe_plan_bytes(int num_problems);
 size_t mxmoe_plan_offset(int which, int num_problems);
 int mxmoe_plan_select_kernel(int kernel_id, const mxmoe_block_desc* h_desc, int num_problems);
 int mxmoe_plan_select_kernel_rows(const mxmoe_block_desc* h_desc, int num_experts, int num_tokens, int topk, int shared_rows);
-/* The same for a block of a layer's forward (as mxmoe_few_row_kernel for a list).  first: the first block of one that mxmoe_layer_run runs: few tokens have no launch in
- * front of it on the kernels for few rows, which then pay up to more experts. */
+/* The same for a block of a layer's forward (as mxmoe_few_row_kernel for a list).  first: the first block of a layer that starts with it on that kernel
+ * (mxmoe_layer_starts_with_gate_up, to be asked with the kernel this names): the kernels for few rows then pay up to more tokens and experts. */
 int mxmoe_layer_kernel(const mxmoe_block_desc* h_desc, int num_experts, int num_tokens, int topk, int shared_rows, int first);
 int mxmoe_plan_grid_bound(int kernel_id, const mxmoe_block_desc* h_desc, int num_experts, int routed_rows_max, int shared_rows);
 int mxmoe_plan_block(int kernel_id, const int64_t* d_recv_tokens_per_exp, int num_experts, int shared_rows, const mxmoe_block_desc* d_desc,
@@ -317,17 +317,22 @@ int mxmoe_upload(void* dst, const void* host_src, size_t bytes, void* stream);
  *   plan_*         mxmoe_plan_bytes() each;
  *   dst_exp, token_of_row, row_of_slot   int32 [R]; iota   int32 [num_tokens] = 0, 1, 2, ...; recv   int64 [num_experts];
  *   workspace      mxmoe_permute_workspace_bytes(R, num_experts), 16-byte aligned.
- * kernel_*: from mxmoe_plan_select_kernel_rows (or -1: as mxmoe_plan_select_kernel).  grid_*: mxmoe_plan_grid_bound of each block with that kernel.  rotate, had_*: of the intermediate rows, as for mxmoe_silu_mul_quant (bits 0 - 1 only).
+ * kernel_*: from mxmoe_layer_kernel (or mxmoe_plan_select_kernel_rows, or -1: as mxmoe_plan_select_kernel); that of the first block with first = 1 only where
+ * mxmoe_layer_starts_with_gate_up then says 1 for the description, else with first = 0.  grid_*: mxmoe_plan_grid_bound of each block with that kernel.  rotate, had_*: of the intermediate rows, as for mxmoe_silu_mul_quant (bits 0 - 1 only).
  *
  * mxmoe_layer_supported   1 when the short form takes the layer: hidden 512, 1024, 2048 or 4096; at most 512 experts; inter a
  *                         multiple of 32; no bf6 operands; token stores and fp16 weights below 2 GiB; and R <= 65536, or
  *                         ceil(R / 256) * num_experts <= 16384.  Else 0: use the separate entry points.
+ * mxmoe_layer_starts_with_gate_up   1 when the short form takes the layer and has no launch for the permutation and the planning in front of gate_up (few tokens, a kernel for few rows:
+ *                         at most 128 tokens and 512 pairs; with kernel_gate_up, h_* and the sizes filled in, no buffers needed).  mxmoe_layer_has_head: the same of a handle (1: there is one).
  * mxmoe_layer_create      checks the description and copies it; the handle is read only afterwards (mxmoe_layer_run may be called from several
  *                         threads as far as the buffers it names allow) and is given back with mxmoe_layer_destroy.
  * mxmoe_layer_run         enqueues on `stream`; hidden fp16 [num_tokens][hidden], topk_ids int32 [num_tokens][topk] (ids out of range are
  *                         dropped), topk_weights fp32, out fp16 [num_tokens][hidden].  Neither allocates nor synchronises.  hidden is
  *                         16-byte aligned where a first block takes 16-bit activations and rotate is not 2 (error 3 otherwise). */
 int mxmoe_layer_supported(const mxmoe_layer_desc* desc);
+int mxmoe_layer_starts_with_gate_up(const mxmoe_layer_desc* desc);
+int mxmoe_layer_has_head(const void* handle);
 int mxmoe_layer_create(const mxmoe_layer_desc* desc, void** handle);
 void mxmoe_layer_destroy(void* handle);
 int mxmoe_layer_run(const void* handle, const void* hidden, const int32_t* topk_ids, const float* topk_weights, void* out, void* stream);

@@ -86,6 +86,8 @@ SIGNATURES = {
     "mxmoe_upload": (_I, [_P, _P, C.c_size_t, _P]),
     "mxmoe_combine_sorted": (_I, [_P, _P, _I, _I, _P, _P, _I, _I, _I, _P, _P]),
     "mxmoe_layer_supported": (_I, [_P]),
+    "mxmoe_layer_starts_with_gate_up": (_I, [_P]),
+    "mxmoe_layer_has_head": (_I, [_P]),
     "mxmoe_layer_create": (_I, [_P, C.POINTER(_P)]),
     "mxmoe_layer_destroy": (None, [_P]),
     "mxmoe_layer_run": (_I, [_P, _P, _P, _P, _P, _P]),

@@ -501,6 +501,45 @@ static LaunchFirstFn first_launch_of(const FusedKernel& k, const mxmoe_block_des
   return nullptr;
 }
 
+// gate_up without a head in front of it, as far as it follows from the layer, the batch and kernel `kg` of the first block: its launch, or null where the layer has a head.  The one place of this
+// rule: the choice of the kernel asks for it (mxmoe_layer_starts_with_gate_up) and so does the handle.
+struct FirstForm {
+  LaunchFirstFn fn;
+  DirectArgs x;
+  dim3 grid;
+  size_t lds;
+};
+constexpr size_t kFirstLdsMax = 40 * 1024;  // (counters of many experts would take the room of a workgroup)
+static FirstForm first_form(const mxmoe_layer_desc* d, const FusedKernel& kg) {
+  const int et = d->num_experts + (d->has_shared ? 1 : 0), total = d->num_tokens * d->topk;
+  FirstForm f{};
+  if (d->num_tokens > kDirectTokens || total > kDirectEntries || d->topk > 64) return f;
+  for (int i = 0; i < et; ++i) {
+    const mxmoe_block_desc& b = d->h_gate_up[i];
+    const int n = i < d->num_experts ? d->inter : d->inter_shared;
+    if ((int)b.N != 2 * n || (int)b.K != d->hidden || n % 32) return f;
+    if (d->rotate == 2 && act_tag_of(b.q) == 0) return f;  // (rotated fp16 tokens are made by a head)
+  }
+  DirectArgs& x = f.x;
+  x.desc = d->d_gate_up;
+  x.act = reinterpret_cast<_Float16*>(d->act);
+  x.hidden_size = d->hidden;
+  x.inter = d->inter;
+  x.inter_shared = d->has_shared ? d->inter_shared : 0;
+  x.cols = d->inter / 32;
+  x.shared_rows = (x.inter_shared / 32 + x.cols - 1) / x.cols;
+  x.shared_step = d->has_shared && d->h_gate_up[d->num_experts].q.a_bits < 16 && d->h_gate_up[d->num_experts].q.gsize != 128 ? 32 : 16;  // (BM of the format's tile)
+  x.shared_slots = x.shared_rows * ((d->num_tokens + x.shared_step - 1) / x.shared_step);
+  x.topk_inverse = (65536 + d->topk - 1) / d->topk;
+  x.entries = total <= kThreads ? kThreads : kDirectEntries;
+  x.tile_lds = kg.lds_bytes;
+  const int front = 2 * PlanLayout(et).chunks + (total + kHeadSmall - 1) / kHeadSmall;  // workgroups that plan, and that write the permutation
+  f.grid = dim3(std::max(x.cols, front), 1 + x.shared_slots + std::min(total, d->num_experts));
+  f.lds = std::max(kg.lds_bytes + direct_lds(x.entries, d->num_experts), sizeof(PlanShared) + 16 + (size_t)(2 + kHeadSmall / 64 + 2 * kCountCopies) * d->num_experts * sizeof(int32_t));
+  if (f.lds <= kFirstLdsMax) f.fn = first_launch_of(kg, d->h_gate_up, et);
+  return f;
+}
+
 // What a layer keeps for one (tokens, top-k): its description and both launches' planning parameters.
 struct LayerForward {
   mxmoe_layer_desc d;
@@ -510,10 +549,7 @@ struct LayerForward {
   bool fp16_first;   // a first block reads the tokens as they are (its tiles load them straight into LDS)
   bool rows_step;    // a second block takes quantised (or rotated) rows
   RowsBehind rows;
-  LaunchFirstFn first;  // gate_up without a head in front of it, or null
-  DirectArgs direct;
-  dim3 first_grid;
-  size_t first_lds;
+  FirstForm first;
 };
 
 static int check_launch() {
@@ -645,31 +681,7 @@ int mxmoe_layer_create(const mxmoe_layer_desc* d, void** handle) {
   pd.form.kind = d->rotate == 2 ? LayerForm::kPlain : LayerForm::kBehind;
   pd.form.act = reinterpret_cast<const uint8_t*>(d->act);
 
-  // few tokens: no head
-  const FusedKernel& kg = registry()[f->d.kernel_gate_up];
-  bool plain = (f->fp16_first || tags) && !(tags & 1u) && h.T <= kDirectTokens && h.total <= kDirectEntries && d->topk <= 64;
-  for (int i = 0; i < et; ++i) {
-    const int n = i < d->num_experts ? d->inter : d->inter_shared;
-    plain = plain && (int)d->h_gate_up[i].N == 2 * n && (int)d->h_gate_up[i].K == d->hidden && n % 32 == 0;
-  }
-  f->first = plain ? first_launch_of(kg, d->h_gate_up, et) : nullptr;
-  DirectArgs& x = f->direct;
-  x = DirectArgs{};
-  x.desc = d->d_gate_up;
-  x.act = reinterpret_cast<_Float16*>(d->act);
-  x.hidden_size = d->hidden;
-  x.inter = d->inter;
-  x.inter_shared = d->has_shared ? d->inter_shared : 0;
-  x.cols = d->inter / 32;
-  x.shared_rows = (x.inter_shared / 32 + x.cols - 1) / x.cols;
-  x.shared_step = d->has_shared && d->h_gate_up[d->num_experts].q.a_bits < 16 && d->h_gate_up[d->num_experts].q.gsize != 128 ? 32 : 16;  // (BM of the format's tile)
-  x.shared_slots = x.shared_rows * ((h.T + x.shared_step - 1) / x.shared_step);
-  x.topk_inverse = (65536 + d->topk - 1) / d->topk;
-  x.entries = h.total <= kThreads ? kThreads : kDirectEntries;
-  x.tile_lds = kg.lds_bytes;
-  f->first_grid = dim3(std::max(x.cols, 2 * f->pair.chunks + h.perm_wgs), 1 + x.shared_slots + std::min(h.total, h.E));
-  f->first_lds = std::max(kg.lds_bytes + direct_lds(x.entries, h.E), sizeof(PlanShared) + 16 + (size_t)(2 + kHeadSmall / 64 + 2 * kCountCopies) * h.E * sizeof(int32_t));
-  if (f->first_lds > 40 * 1024) f->first = nullptr;  // (counters of many experts would take the room of a workgroup)
+  f->first = first_form(d, registry()[f->d.kernel_gate_up]);
 
   RowsBehind& r = f->rows;
   r = RowsBehind{};
@@ -693,6 +705,13 @@ int mxmoe_layer_create(const mxmoe_layer_desc* d, void** handle) {
   *handle = f.release();
   return 0;
 }
+
+int mxmoe_layer_starts_with_gate_up(const mxmoe_layer_desc* d) {
+  if (!mxmoe_layer_supported(d)) return 0;
+  return first_form(d, registry()[resolve_kernel(d->kernel_gate_up, d->h_gate_up, d->num_experts + (d->has_shared ? 1 : 0))]).fn != nullptr;
+}
+
+int mxmoe_layer_has_head(const void* handle) { return handle && !reinterpret_cast<const LayerForward*>(handle)->first.fn; }
 
 void mxmoe_layer_destroy(void* handle) { delete reinterpret_cast<LayerForward*>(handle); }
 
@@ -733,12 +752,12 @@ int mxmoe_layer_run(const void* handle, const void* hidden, const int32_t* topk_
       default: f(std::integral_constant<int, 8>{}); break;
     }
   };
-  if (f.first) {
-    DirectArgs x = f.direct;
+  if (f.first.fn) {
+    DirectArgs x = f.first.x;
     x.hidden = reinterpret_cast<const uint8_t*>(hidden);
     if (h.tags) by_length([&](auto ni) { hipLaunchKernelGGL((layer_tokens_kernel<decltype(ni)::value>), dim3((h.T + 3) / 4), dim3(kHeadSmall), 0, s, h); });
     if (const int rc = check_launch()) return rc;
-    f.first(h, pair, x, f.first_grid, f.first_lds, s);
+    f.first.fn(h, pair, x, f.first.grid, f.first.lds, s);
     if (const int rc = check_launch()) return rc;
   } else {
     if (h.hist) launch_perm_hist(topk_ids, h.total, h.E, const_cast<int32_t*>(h.hist), true, s);

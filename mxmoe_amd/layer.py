@@ -142,7 +142,7 @@ class MxMoELayer:
         return h
 
     def _planned_kernel(self, h, t: int, topk: int, first: bool = False) -> int:
-        """The kernel that a block's planned launch runs on for t tokens (`first`: the first block of the short form)."""
+        """The kernel that a block's planned launch runs on for t tokens (`first`: the first block of a layer that starts with it)."""
         lib = _lib.load()
         kid = lib.mxmoe_layer_kernel(h, self.cfg.num_experts, t, topk, t if self.cfg.num_shared else 0, int(first))
         if kid < 0:
@@ -217,6 +217,22 @@ class MxMoELayer:
         cache[key] = ps
         return ps
 
+    def _layer_desc(self, t: int, topk: int):
+        """The layer's description for (tokens, top-k) with its sizes and both blocks' kernels, and the host's block descriptors that it points to.  The first block's kernel is chosen as that of a layer
+        which starts with gate_up where it then does (mxmoe_layer_starts_with_gate_up)."""
+        cfg, lib = self.cfg, _lib.load()
+        e_cnt, has_shared, et = cfg.num_experts, cfg.num_shared > 0, self.n_exp_total
+        i_sh = cfg.inter * max(cfg.num_shared, 1)
+        sh = [i_sh] if has_shared else []
+        gate_up = self._block_descs(self.qp_gate_up, [2 * cfg.inter] * e_cnt + [2 * n for n in sh], [cfg.hidden] * et, self.w13, self.bf6_gate_up)
+        down = self._block_descs(self.qp_down, [cfg.hidden] * et, [cfg.inter] * e_cnt + sh, self.w2, self.bf6_down)
+        d = _lib.LayerDesc(num_tokens=t, topk=topk, num_experts=e_cnt, has_shared=int(has_shared), hidden=cfg.hidden, inter=cfg.inter, inter_shared=i_sh, rotate=cfg.rotate,
+                           had_k=1, had_f=1, h_gate_up=C.cast(gate_up, C.c_void_p), h_down=C.cast(down, C.c_void_p))
+        d.kernel_gate_up, d.kernel_down = self._planned_kernel(gate_up, t, topk, first=True), self._planned_kernel(down, t, topk)
+        if not lib.mxmoe_layer_starts_with_gate_up(C.byref(d)):
+            d.kernel_gate_up = self._planned_kernel(gate_up, t, topk)
+        return d, gate_up, down
+
     def _short_setup(self, t: int, topk: int):
         """The short form of the planned forward for (tokens, top-k): a handle of `mxmoe_layer_create` with the buffers it names, or None
         when the library does not take the layer or the batch in that form (mxmoe_layer_supported).  Built once and reused."""
@@ -231,13 +247,7 @@ class MxMoELayer:
             return None
         r_cap, shared_rows, i_sh = t * topk, t if has_shared else 0, cfg.inter * max(cfg.num_shared, 1)
         sh = [i_sh] if has_shared else []
-        gate_up = self._block_descs(self.qp_gate_up, [2 * cfg.inter] * e_cnt + [2 * n for n in sh], [cfg.hidden] * et, self.w13, False)
-        down = self._block_descs(self.qp_down, [cfg.hidden] * et, [cfg.inter] * e_cnt + sh, self.w2, False)
-        d = _lib.LayerDesc(num_tokens=t, topk=topk, num_experts=e_cnt, has_shared=int(has_shared), hidden=cfg.hidden, inter=cfg.inter, inter_shared=i_sh, rotate=cfg.rotate,
-                           had_k=1, had_f=1, h_gate_up=C.cast(gate_up, C.c_void_p), h_down=C.cast(down, C.c_void_p))
-        # (what a first block needs to start the layer: rotated fp16 tokens are made by a head in front of it)
-        first = (cfg.rotate != 2 or all(int(q[0]) < 16 for q in self.qp_gate_up)) and cfg.inter % 32 == 0 and topk <= 64
-        d.kernel_gate_up, d.kernel_down = self._planned_kernel(gate_up, t, topk, first=first), self._planned_kernel(down, t, topk)
+        d, gate_up, down = self._layer_desc(t, topk)
         if not lib.mxmoe_layer_supported(C.byref(d)):
             cache[key] = None
             return None
