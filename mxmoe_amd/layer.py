@@ -51,6 +51,7 @@ class MxMoELayer:
         self.qp_down = [f[1] for f in self.formats]
         self.kid_gate_up = ops.select_kernel(self.qp_gate_up, self.bf6_gate_up, self.fp8)
         self.kid_down = ops.select_kernel(self.qp_down, self.bf6_down, self.fp8)
+        self._kids = (self.kid_gate_up, self.kid_down)
         self.state = None
         self._static = None
 
@@ -73,8 +74,9 @@ class MxMoELayer:
             hidden, topk_ids, cfg.num_experts, cfg.inter, cfg.num_shared, self.qp_gate_up, rotate=cfg.rotate, bf6=self.bf6_gate_up, fp8=self.fp8)
         i_sh = cfg.inter * max(cfg.num_shared, 1)
         acc1 = [torch.zeros(m.shape, dtype=torch.int32, device=self.device) for m in st["mid"]] if dump_acc else None
+        st["kernels"] = self._kernels(hidden.shape[0], topk_ids.shape[1], host=True)
         st["gg1"] = ops.prepare_gg(st["inp"], [w.data for w in self.w13], st["sa"], [w.scale for w in self.w13], st["mid"], 2 * cfg.inter, cfg.hidden,
-                                   2 * i_sh, cfg.hidden, self.qp_gate_up, st["recv"], kernel_id=self.kid_gate_up, acc_dump=acc1, few_rows=True)
+                                   2 * i_sh, cfg.hidden, self.qp_gate_up, st["recv"], kernel_id=st["kernels"][0], acc_dump=acc1)
         st["acc1"] = acc1
         st["dump_acc"] = dump_acc
         st["hidden"], st["topk_ids"] = hidden, topk_ids
@@ -92,7 +94,7 @@ class MxMoELayer:
         i_sh = cfg.inter * max(cfg.num_shared, 1)
         acc2 = [torch.zeros(o.shape, dtype=torch.int32, device=self.device) for o in st["out"]] if st["dump_acc"] else None
         st["gg2"] = ops.prepare_gg(st["inp2"], [w.data for w in self.w2], st["sa2"], [w.scale for w in self.w2], st["out"], cfg.hidden, cfg.inter,
-                                   cfg.hidden, i_sh, self.qp_down, st["recv"], kernel_id=self.kid_down, acc_dump=acc2, few_rows=True)
+                                   cfg.hidden, i_sh, self.qp_down, st["recv"], kernel_id=st["kernels"][1], acc_dump=acc2)
         st["acc2"] = acc2
 
     def down(self):
@@ -167,10 +169,11 @@ class MxMoELayer:
         def u8(n):
             return torch.empty(max(int(n), 16), dtype=torch.uint8, device=dev)
 
-        def block(qps, ns, ks, ws, bf6):
+        kernels = self._kernels(t, topk)
+
+        def block(qps, ns, ks, ws, bf6, kid):
             h = self._block_descs(qps, ns, ks, ws, bf6)
             d = torch.frombuffer(bytearray(bytes(h)), dtype=torch.uint8).to(dev)
-            kid = self._planned_kernel(h, t, topk)
             grid = lib.mxmoe_plan_grid_bound(kid, h, e_cnt, r_cap, shared_rows)
             if grid < 0:
                 raise RuntimeError(lib.mxmoe_last_error().decode())
@@ -187,8 +190,8 @@ class MxMoELayer:
             return {"h": h, "d": d, "kid": kid, "grid": grid, "plan": u8(lib.mxmoe_plan_bytes(et)), "inp": u8(inp), "scale": u8(sc), "out_bytes": out}
 
         sh = [1] if has_shared else []
-        b1 = block(self.qp_gate_up, [2 * cfg.inter] * e_cnt + [2 * i_sh for _ in sh], [cfg.hidden] * et, self.w13, self.bf6_gate_up)
-        b2 = block(self.qp_down, [cfg.hidden] * et, [cfg.inter] * e_cnt + [i_sh for _ in sh], self.w2, self.bf6_down)
+        b1 = block(self.qp_gate_up, [2 * cfg.inter] * e_cnt + [2 * i_sh for _ in sh], [cfg.hidden] * et, self.w13, self.bf6_gate_up, kernels[0])
+        b2 = block(self.qp_down, [cfg.hidden] * et, [cfg.inter] * e_cnt + [i_sh for _ in sh], self.w2, self.bf6_down, kernels[1])
         ps["b1"], ps["b2"] = b1, b2
         ps["mid"], ps["out"] = u8(b1["out_bytes"]), u8(b2["out_bytes"])
         call = lambda b, out_store: _lib.PlanCall(b["kid"], b["d"].data_ptr(), C.cast(b["h"], C.c_void_p), b["inp"].data_ptr(), b["scale"].data_ptr(),  # noqa: E731
@@ -232,6 +235,23 @@ class MxMoELayer:
         if not lib.mxmoe_layer_starts_with_gate_up(C.byref(d)):
             d.kernel_gate_up = self._planned_kernel(gate_up, t, topk)
         return d, gate_up, down
+
+    def _kernels(self, t: int, topk: int, host: bool = False):
+        """(gate_up, down): the kernels of the layer for (tokens, top-k), one choice for all of its forms: the sums of fp16, weight-only and fp8 blocks are the same to the bit on one kernel only, and which
+        one a list would take by its real row counts changes with the routing.  `host`: of a form with host tables, whose kernels a caller may have set (`kid_gate_up`, `kid_down`), and
+        which takes what no planned launch does (no tokens; a shape that a kernel refuses, of an expert without rows)."""
+        cache = self.__dict__.setdefault("_kernels_of", {})
+        if (t, topk) not in cache:
+            try:
+                d = self._layer_desc(t, topk)[0]
+                cache[t, topk] = (d.kernel_gate_up, d.kernel_down)
+            except RuntimeError:
+                if not host:
+                    raise
+                return self.kid_gate_up, self.kid_down
+        if not host:
+            return cache[t, topk]
+        return tuple(set_ if set_ != own else kid for set_, own, kid in zip((self.kid_gate_up, self.kid_down), self._kids, cache[t, topk]))
 
     def _short_setup(self, t: int, topk: int):
         """The short form of the planned forward for (tokens, top-k): a handle of `mxmoe_layer_create` with the buffers it names, or None
@@ -431,18 +451,18 @@ class MxMoELayer:
         def launch(ptr_off, sizes_off, h_sizes, h_q, kid):
             row = lambda i: base + ptr_off + i * count * 8  # noqa: E731
             dims, qs = h_sizes.ctypes.data_as(C.POINTER(_lib.Dim3)), h_q.ctypes.data_as(C.POINTER(_lib.QParams))
-            _lib.check(lib, lib.mxmoe_group_gemm(lib.mxmoe_few_row_kernel(kid, dims, qs, count), row(0), row(1), row(2), row(3), row(4), row(4), None, None, None, None, base + sizes_off,
-                                                 dims, None, qs, count, None, stream))
+            _lib.check(lib, lib.mxmoe_group_gemm(kid, row(0), row(1), row(2), row(3), row(4), row(4), None, None, None, None, base + sizes_off, dims, None, qs, count, None, stream))
 
         hk, hf, sg = signs(cfg.hidden, cfg.hidden)
         _lib.check(lib, lib.mxmoe_quant_act(hidden.data_ptr(), inp1.data_ptr(), sa1.data_ptr(), dst.data_ptr(), perm.data_ptr(), base + off[0],
                                             cfg.hidden, routed, t, e_cnt, int(has_shared), cfg.rotate | self._variants(self.bf6_gate_up), hk, hf, sg, stream))
-        launch(off[2], off[4], s1, q1, self.kid_gate_up)
+        kid_gate_up, kid_down = self._kernels(t, topk, host=True)
+        launch(off[2], off[4], s1, q1, kid_gate_up)
         i_sh = cfg.inter * max(cfg.num_shared, 1)
         hk, hf, sg = signs(cfg.inter, i_sh)
         _lib.check(lib, lib.mxmoe_silu_mul_quant(mid.data_ptr(), mid.data_ptr() + routed * 2 * cfg.inter * 2, inp2.data_ptr(), sa2.data_ptr(), dst.data_ptr(), base + off[1],
                                                  cfg.inter, i_sh, routed, t, e_cnt, int(has_shared), cfg.rotate | self._variants(self.bf6_down), hk, hf, sg, stream))
-        launch(off[3], off[5], s2, q2, self.kid_down)
+        launch(off[3], off[5], s2, q2, kid_down)
         ws = torch.empty(lib.mxmoe_combine_workspace_bytes(t, topk), dtype=torch.uint8, device=dev)
         shared_ptr = out.data_ptr() + routed * cfg.hidden * 2 if has_shared else None
         _lib.check(lib, lib.mxmoe_unpermute_combine(out.data_ptr(), shared_ptr, w.data_ptr(), slot.data_ptr(), routed, t, topk, cfg.hidden, final.data_ptr(), ws.data_ptr(), stream))
