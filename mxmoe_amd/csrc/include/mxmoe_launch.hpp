@@ -946,7 +946,7 @@ constexpr int kFewRowsMax = 64, kFewBlocks = 768, kFewBlocksHeadless = 1024, kFe
 // w4a16 / w3a16 52 -> 45 / 80 -> 58 (72); 24 experts top-2, K = 4096, w4a4 74 -> 65 / 68 -> 64 (100).  fp16 (weights read
 // once per 16 rows from L2 outweigh the head) 223 -> 210 / 186 -> 189 (66), 223 -> 214 / 224 -> 231 (128), with a shared expert 278 -> 298: up to 64.
 // Errors of weight-only problems against float64 in the 2-norm, many-token tiles (whose weights are rounded to fp16) / 64-channel tiles, K = 2048: w8 2.88e-4 / 2.06e-4, w4 2.89e-4 / 2.06e-4, w3 2.82e-4 /
-// 2.13e-4, w2 2.23e-4 / 2.29e-4 (the output's own rounding is 2.0e-4 of each).
+// 2.13e-4, w2 2.22e-4 / 2.09e-4 (the output's own rounding is 2.0e-4 of each).
 constexpr int kDirectTokens = 128, kDirectEntries = 512;
 // The largest problem that those kernels take in a launch.
 inline long few_rows_max(const RowSummary& s) { return s.headless && !s.any_fp16 ? kDirectTokens : kFewRowsMax; }

@@ -142,6 +142,35 @@ struct SkinnyWoTile {
     }
   }
 
+  // The operands of stream() and the bias that their values carry: of 2-bit codes a small one.  A sum of x * (q + bias) is rounded (on the matrix pipe: cut off) at the size of its biased terms: with
+  // 1024 beside codes of 0 .. 3 that is all there is to the error, and where the tokens have a mean it is of one sign.  Errors of such sums against float64 in the 2-norm, K = 1408 .. 14 336, biases of
+  // unpack() -> these, beside the many-token tile's, whose weights are rounded to fp16: normal tokens 9.3e-5 -> 3.7e-6 (7.6e-5), tokens of mean 0.7 and deviation 0.5 6.6e-4 .. 1.5e-3 ->
+  // 4.6e-5 .. 1.3e-4 (1.8e-4).  (Wider codes are closer than that tile's with unpack()'s: 3 bits 4.4e-5 and 1.9e-4, 4 bits 2.1e-5 and 2.0e-4, 8 bits 1.8e-6 and 2.0e-4; smaller biases there take a shift more per operand,
+  // 1% of a layer of 400 tokens.)  A code at bit P of a half is 2^(10-P) + q; two shifted copies of a dword bring its sixteen codes to bits 4, 6 and 8, one shift fewer than unpack() takes.
+  template <int P>
+  __device__ static __forceinline__ int place2(int d) {
+    int mask = (3 << P) * 0x00010001, magic = ((25 - P) << 10) * 0x00010001;
+    asm("" : "+s"(mask), "+v"(magic));  // (see cvt8)
+    return (d & mask) | magic;
+  }
+  __device__ static __forceinline__ void operands(const WReg& w, v8h out[4]) {
+    if constexpr (WBITS == 2) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int d = w.d[h], up = d << 4, down = (int)((unsigned)d >> 6);
+        out[2 * h] = __builtin_bit_cast(v8h, v4i{place2<4>(up), place2<4>(d), place2<8>(d), place2<6>(down)});
+        out[2 * h + 1] = __builtin_bit_cast(v8h, v4i{place2<6>(up), place2<6>(d), place2<4>(down), place2<8>(down)});
+      }
+    } else {
+      unpack(w, out);
+    }
+  }
+  __device__ static __forceinline__ v8h bias_of(int j) {  // (of operand j)
+    auto pairs = [](float a, float b, float c, float d) { return v8h{(_Float16)a, (_Float16)a, (_Float16)b, (_Float16)b, (_Float16)c, (_Float16)c, (_Float16)d, (_Float16)d}; };
+    if constexpr (WBITS == 2) return j % 2 ? pairs(16.f, 16.f, 64.f, 4.f) : pairs(64.f, 64.f, 4.f, 16.f);
+    else return bias8();
+  }
+
   // One pass of a wave: NKB (<= KP) consecutive k blocks starting at kb0, against all NB channel blocks of the tile.
   // The wave's activations of these k blocks are loaded once into registers and its (scale, zero) pairs into a private LDS
   // patch; the packed weight blocks then stream through a ring of kRing register buffers with no barrier in the loop, so
@@ -246,7 +275,7 @@ struct SkinnyWoTile {
     const int K = t.K, KB = K / 128;
     const int lg = lane >> 4;
     const v8h ones = {(_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f};
-    const v8h bias = bias8();
+    const v8h bias[2] = {bias_of(0), bias_of(1)};  // (of even and odd operands)
     auto block_of = [&](int nb) {
       if constexpr (GU) return (nb % (NB / 2) < nbv ? nb % (NB / 2) : 0) + (nb >= NB / 2 ? t.N / 32 : 0);
       else return nb < nbv ? nb : 0;
@@ -297,14 +326,14 @@ struct SkinnyWoTile {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           sx[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, xf[mb][j], sx[mb], 0, 0, 0);
-          sxb[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bias, xf[mb][j], sxb[mb], 0, 0, 0);
+          sxb[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bias[j % 2], xf[mb][j], sxb[mb], 0, 0, 0);
         }
       }
       // pipelined by channel block: between the matrix instructions of block nb, the sums of block nb - 1 are scaled and block nb + 1 is unpacked, operand
       // by operand into the registers that block nb has just used
       v8h wf[4], s8[2];
       v4f part[2][MB];
-      unpack(wr[0], wf);
+      operands(wr[0], wf);
       static_for<NB>([&](auto nbc) {
         constexpr int nb = decltype(nbc)::value, cur = nb & 1, prev = cur ^ 1;
         s8[cur] = __builtin_bit_cast(v8h, *reinterpret_cast<const v4i*>(sp + nb * (kChunk * 64)));  // (scale, zero) of channels 4*lg .. 4*lg+3
@@ -318,7 +347,7 @@ struct SkinnyWoTile {
           for (int mb = 0; mb < MB; ++mb) part[cur][mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[j], xf[mb][j], part[cur][mb], 0, 0, 0);
           if constexpr (nb + 1 < NB) {
             v8h w[4];
-            unpack(wr[nb + 1], w);
+            operands(wr[nb + 1], w);
             wf[j] = w[j];
           }
           if constexpr (nb > 0) {
