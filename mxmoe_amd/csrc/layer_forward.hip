@@ -289,7 +289,9 @@ __global__ void __launch_bounds__(TH) layer_head_kernel(const HeadArgs a, const 
 // need, are made beside it by the first workgroups.  What is left in front is the quantisation of the tokens (layer_tokens_kernel), where first blocks take quantised ones.
 // Grid: (column tiles of a routed expert) x (1 for those, shared_slots rows of the shared expert's tiles, one row per expert that may have tokens).  A workgroup counts the ids in LDS, takes
 // the slot-th expert with rows, lists its rows, and runs their row tiles one after the other (an expert of more than one is rare but under a skewed routing, and its
-// weights come from L2 then).
+// weights come from L2 then).  DEAL (fp16 weights and more than 32 tokens): where at most half of the grid's rows have an expert, since most tokens take the same ones as the padding of a captured batch does, the others
+// come to the experts in turn and take row tiles of those of more than two.  64 tokens on the same four of 60 fp16 experts, us a layer: one tile after the other 71.6, dealt 62.8 (behind a head, on the tiles of 64 rows, 62.1).
+// Elsewhere one after the other is the better of both or what was gained does not pay the look (0.4 us of a layer): weight-only 32 tokens 28.3 / 28.7, 128 tokens 64.4 / 53.6 (79.3 behind a head), integer tiles of 32 rows 36.8 / 37.3.
 // What a launch of few tokens consists of is latency: a layer's, with the head in front -> without, us: 64 experts top-6 and a shared one, w4a16 / w3a16, 29 -> 22 (1 token), 54 -> 46 (8),
 // 77 -> 71 (32), w8a16 / w2a16 31 -> 23 (1), 65 -> 54 (8), 96 -> 85 (32); 60 experts top-4, w4a16 24 -> 18 (1), 55 -> 49 (16), 72 -> 68 (64), skewed 68 -> 64 (64), fp16 35 -> 27 (1),
 // 108 -> 99 (8), 217 -> 212 (64); 8 experts of N = 28 672 / 4096, w4a16 64 -> 58 (1), 134 -> 126 (16).  One or two ids per thread: up to 512 of them, and no more tokens than the kernels for few rows take.
@@ -340,9 +342,10 @@ struct DirectTile<WxAxGNarrowTile> {
   }
 };
 
-template <class... Tiles>
+template <bool DEAL, class... Tiles>
 __global__ void __launch_bounds__(kThreads, 3) layer_first_kernel(const HeadArgs a, const PlanPair pair, const DirectArgs x) {
   static_assert(kThreads == kHeadSmall && ((Tiles::BN == 64) && ...), "one or two ids per thread; 32 outputs a tile");
+  static_assert(!DEAL || ((Tiles::BM == 16) && ...), "row tiles of one height are dealt out");
   extern __shared__ __align__(16) uint8_t first_lds[];
   const int col0 = blockIdx.x, E = a.E;
   int slot = (int)blockIdx.y - 1;
@@ -384,21 +387,35 @@ __global__ void __launch_bounds__(kThreads, 3) layer_first_kernel(const HeadArgs
   }
   __syncthreads();
   int e = shared ? E : -1, before = 0;  // the problem's expert; rows of the experts before it
-  for (int x0 = 0; x0 < E; x0 += 64) {
-    const int c = x0 + lane < E ? count[x0 + lane] : 0;
-    const uint64_t hit = __ballot(c > 0);
-    const int hits = __popcll(hit);
-    uint64_t take = ~0ull;  // experts of these 64 in front of the problem's
-    if (!shared && slot < hits) {
-      const uint64_t it = __ballot(c > 0 && __popcll(hit & ((1ull << lane) - 1)) == slot);
-      e = x0 + __builtin_ctzll(it);
-      take = it - 1;
+  auto find = [&](int k) {              // the k-th expert with rows; returns k less those with rows where there are no more than k
+    for (int x0 = 0; x0 < E; x0 += 64) {
+      const int c = x0 + lane < E ? count[x0 + lane] : 0;
+      const uint64_t hit = __ballot(c > 0);
+      const int hits = __popcll(hit);
+      uint64_t take = ~0ull;  // experts of these 64 in front of the problem's
+      if (!shared && k < hits) {
+        const uint64_t it = __ballot(c > 0 && __popcll(hit & ((1ull << lane) - 1)) == k);
+        e = x0 + __builtin_ctzll(it);
+        take = it - 1;
+      }
+      before += wave_last(wave_inclusive_scan((take >> lane & 1) ? c : 0));
+      if (!shared && e >= 0) break;
+      k -= hits;
     }
-    before += wave_last(wave_inclusive_scan((take >> lane & 1) ? c : 0));
-    if (!shared && e >= 0) break;
-    slot -= hits;
+    return k;
+  };
+  const int past = find(slot);
+  const int slots = (int)gridDim.y - 1 - x.shared_slots;
+  int tile0 = 0;
+  if (e < 0) {  // (every wave of the workgroup has come to the same)
+    if constexpr (!DEAL) return;
+    const int live = slot - past;
+    if (live == 0 || 2 * live > slots) return;
+    tile0 = slot / live;
+    slot -= tile0 * live;
+    before = 0;
+    find(slot);
   }
-  if (e < 0) return;  // (every wave of the workgroup has come to the same)
   int M = 0;
   if (shared) {
     M = min(a.T, shared_m0 + x.shared_step);
@@ -410,6 +427,7 @@ __global__ void __launch_bounds__(kThreads, 3) layer_first_kernel(const HeadArgs
       M += __popcll(which);
     }
     __builtin_amdgcn_wave_barrier();
+    if (DEAL && tile0 > 0 && (M <= 32 || tile0 * 16 >= M)) return;
   }
   TileArgs t;
   const mxmoe_block_desc* d = x.desc + e;
@@ -431,9 +449,16 @@ __global__ void __launch_bounds__(kThreads, 3) layer_first_kernel(const HeadArgs
     if (!D::takes(a_bits, w_bits, gsize)) return;
     t.A = D::kTag == 0 ? x.hidden : a.store[D::kTag];
     t.sa = D::kTag == 0 ? nullptr : a.scales[D::kTag];
+    const int m_first = shared_m0 + tile0 * T::BM;
+    int m_step = T::BM;
+    if (DEAL && !shared && M > 32) {
+      int live = 0;
+      for (int x0 = 0; x0 < E; x0 += 64) live += __popcll(__ballot(x0 + lane < E && count[x0 + lane] > 0));
+      if (2 * live <= slots) m_step *= (slots - slot + live - 1) / live;  // (as many rows of the grid come to this expert)
+    }
 #pragma unroll 1
-    for (int m0 = shared_m0; m0 < M; m0 += T::BM) {
-      if (m0 > shared_m0) __syncthreads();  // the reduction behind the previous tile has been read
+    for (int m0 = m_first; m0 < M; m0 += m_step) {
+      if (m0 > m_first) __syncthreads();  // the reduction behind the previous tile has been read
       t.row0 = m0;
       D::run(t, first_lds, token_of);
     }
@@ -451,16 +476,18 @@ __global__ void __launch_bounds__(kHeadSmall) layer_tokens_kernel(const HeadArgs
 // A launch for first blocks of few tokens, and its tiles.
 using LaunchFirstFn = void (*)(const HeadArgs&, const PlanPair&, const DirectArgs&, dim3, size_t, hipStream_t);
 struct FirstLaunch {
-  LaunchFirstFn fn;
+  LaunchFirstFn fn, deals;  // deals: with row tiles dealt to spare rows of the grid, or null
   std::vector<BranchInfo> tiles;
 };
-template <class... Tiles>
+template <bool DEAL, class... Tiles>
 void launch_first(const HeadArgs& a, const PlanPair& pair, const DirectArgs& x, dim3 grid, size_t lds, hipStream_t s) {
-  hipLaunchKernelGGL((layer_first_kernel<Tiles...>), grid, dim3(kThreads), lds, s, a, pair, x);
+  hipLaunchKernelGGL((layer_first_kernel<DEAL, Tiles...>), grid, dim3(kThreads), lds, s, a, pair, x);
 }
 template <class... Tiles>
 FirstLaunch first_of() {
-  return {&launch_first<Tiles...>, {BranchOf<Tiles>::get()...}};
+  LaunchFirstFn deals = nullptr;
+  if constexpr (((Tiles::kABits == 16) && ...) && ((Tiles::kWBits == 16) || ...)) deals = &launch_first<true, Tiles...>;
+  return {&launch_first<false, Tiles...>, deals, {BranchOf<Tiles>::get()...}};
 }
 template <int WBITS>
 using FewTokenTile = SkinnyWoTile<WBITS, 64, 1, 3>;
@@ -479,8 +506,8 @@ static bool same_sums(const FusedKernel& k, Fmt f, const BranchInfo& tile) {
 }
 
 // The launch for a layer whose first block runs on kernel k: the one of fewest formats that takes each block as k would, or null (a kernel for many rows; one whose tables may take a larger tile with other
-// sums than the 64-channel one's).
-static LaunchFirstFn first_launch_of(const FusedKernel& k, const mxmoe_block_desc* h_desc, int et) {
+// sums than the 64-channel one's).  With fp16 weights and more tokens than two row tiles hold, the one that deals row tiles out.
+static LaunchFirstFn first_launch_of(const FusedKernel& k, const mxmoe_block_desc* h_desc, int et, int num_tokens) {
   using I4 = WxAxNarrowTile<Op::I4>;
   using I8 = WxAxNarrowTile<Op::I8>;
   using F8 = WxAxNarrowTile<Op::F8>;
@@ -494,9 +521,13 @@ static LaunchFirstFn first_launch_of(const FusedKernel& k, const mxmoe_block_des
   };
   auto takes = [&](const FirstLaunch& l, Fmt f) { return std::any_of(l.tiles.begin(), l.tiles.end(), [&](const BranchInfo& t) { return t.fmt == f && same_sums(k, f, t); }); };
   for (const FirstLaunch& l : launches) {
-    bool all = true;
-    for (int i = 0; i < et && all; ++i) all = takes(l, (Fmt)fmt_of(h_desc[i].q));
-    if (all) return l.fn;
+    bool all = true, fp16 = false;
+    for (int i = 0; i < et && all; ++i) {
+      const Fmt f = (Fmt)fmt_of(h_desc[i].q);
+      all = takes(l, f);
+      fp16 = fp16 || f == Fmt::FP16;
+    }
+    if (all) return fp16 && l.deals && num_tokens > 32 ? l.deals : l.fn;
   }
   return nullptr;
 }
@@ -536,7 +567,7 @@ static FirstForm first_form(const mxmoe_layer_desc* d, const FusedKernel& kg) {
   const int front = 2 * PlanLayout(et).chunks + (total + kHeadSmall - 1) / kHeadSmall;  // workgroups that plan, and that write the permutation
   f.grid = dim3(std::max(x.cols, front), 1 + x.shared_slots + std::min(total, d->num_experts));
   f.lds = std::max(kg.lds_bytes + direct_lds(x.entries, d->num_experts), sizeof(PlanShared) + 16 + (size_t)(2 + kHeadSmall / 64 + 2 * kCountCopies) * d->num_experts * sizeof(int32_t));
-  if (f.lds <= kFirstLdsMax) f.fn = first_launch_of(kg, d->h_gate_up, et);
+  if (f.lds <= kFirstLdsMax) f.fn = first_launch_of(kg, d->h_gate_up, et, d->num_tokens);
   return f;
 }
 

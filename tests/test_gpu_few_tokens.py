@@ -275,3 +275,33 @@ def test_weight_only_sums_are_as_close_as_those_of_the_many_token_tiles(bits, k)
             err[kernel] = ((acc.view(torch.float32).double() - ref).norm() / ref.norm()).item()
         print(bits, k, mean, err)
         assert err["a16_few"] <= 1.1 * err["all"], (mean, err)
+
+
+# tokens, top-k, experts, first of the experts that most tokens take, tokens that take others: up to four (32 rows each) and eight (16) row tiles of an expert over rows of the grid that no expert needs, as many of them as
+# tiles, more, fewer and none; those experts behind the first 64; ids out of range
+@pytest.mark.gpu
+@pytest.mark.parametrize("mix", ["fp16", "wo", "int"])
+@pytest.mark.parametrize("tokens,topk,experts,first,others", [(64, 4, 60, 0, 0), (128, 4, 60, 7, 0), (128, 4, 130, 66, 0), (128, 4, 130, 126, 9), (128, 2, 5, 1, 0), (128, 3, 6, 2, 1), (65, 2, 2, 0, 0), (97, 1, 70, 69, 0),
+                                                              (128, 4, 60, 20, 64)])
+def test_row_tiles_of_an_expert_that_most_tokens_take(tokens, topk, experts, first, others, mix):
+    """Dealt to several workgroups where the grid has spare ones: identical outputs with the form that has launches in front."""
+    from mxmoe_amd import _lib, synth as S
+    from mxmoe_amd.layer import MxMoELayer
+
+    fm = {"fp16": [(FP16, FP16)], "wo": [(S.W4A16, S.W2A16), (S.W2A16, S.W4A16)], "int": [(S.W4A4, S.W8A8), (S.W8A8, S.W4A4)]}[mix]
+    cfg = S.MoEConfig("t", "test", experts, topk, 512, 256, tokens, num_shared=1, rotate=int(mix == "int"))
+    layer = MxMoELayer(cfg, formats=[fm[i % len(fm)] for i in range(experts + 1)])
+    lib = _lib.load()
+    kid = lib.mxmoe_find_kernel(b"groupgemm_hz_fused_" + {"fp16": b"a16_few", "wo": b"wo_few", "int": b"wxax_few"}[mix])
+    layer._planned_kernel = lambda *_, **__: kid
+    gen = torch.Generator().manual_seed(tokens + experts)
+    ids = (first + torch.arange(topk)).remainder(experts).repeat(tokens, 1).to(torch.int32)
+    for t in range(others):
+        ids[2 * t] = torch.randperm(experts, generator=gen)[:topk].to(torch.int32)
+    ids[-1, 0], ids[-2, -1] = -1, experts
+    ids, w = ids.cuda(), torch.rand(tokens, topk, generator=gen).cuda()
+    hidden = torch.randn(tokens, 512, generator=gen).half().cuda()
+    got = layer(hidden, ids, w).clone()
+    assert not lib.mxmoe_layer_has_head(layer._short[tokens, topk]._handle)
+    layer._short[tokens, topk] = None
+    assert torch.equal(layer(hidden, ids, w), got)
