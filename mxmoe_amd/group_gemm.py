@@ -41,8 +41,7 @@ def _upload(host: np.ndarray, device) -> torch.Tensor:
 class GroupGemmLaunch:
     """A prepared problem list: `run()` is a single allocation-free, sync-free kernel launch."""
 
-    def __init__(self, As, Bs, scale_a, scale_b, Cs, sizes, qparams, kernel_id: int = -1, acc=None, lib=None, few_rows: bool = False):
-        """`few_rows`: kernel_id names how the operands are laid out (-1: plainly); a list of few rows may run on the kernel made for a layer's that takes the same."""
+    def __init__(self, As, Bs, scale_a, scale_b, Cs, sizes, qparams, kernel_id: int = -1, acc=None, lib=None):
         self.lib = lib or _lib.load()
         p = len(As)
         assert len(Bs) == len(Cs) == len(sizes) == len(qparams) == p
@@ -70,8 +69,6 @@ class GroupGemmLaunch:
         sizes_t, qparams_t = _array_types(max(p, 1))
         self.h_sizes = sizes_t.from_buffer(block, 6 * p * 8)
         self.h_q = qparams_t.from_buffer_copy(b"".join([_qparams_bytes(q if type(q) is tuple else tuple(q)) for q in qparams]) or bytes(16))
-        if few_rows and p:
-            self.kernel_id = self.lib.mxmoe_few_row_kernel(kernel_id, self.h_sizes, self.h_q, p)
         self.d_block = _upload(block, dev)
         self._base = self.d_block.data_ptr()
         self.has_acc = acc is not None

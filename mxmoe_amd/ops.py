@@ -354,9 +354,8 @@ def gg_mxmoe_share_fused(inp, experts, scale_zp_a, scale_zp_b, output, N: int, K
     return output
 
 
-def prepare_gg(inp, experts, scale_zp_a, scale_zp_b, output, N, K, shared_N, shared_K, qparams_per_exp, recv_tokens_per_exp, kernel_id: int = -1, acc_dump=None,
-               few_rows: bool = False) -> GroupGemmLaunch:
-    """The pointer-table part of `gg_mxmoe_share_fused`, reusable across launches (CUDA-graph friendly).  `few_rows`: see GroupGemmLaunch."""
+def prepare_gg(inp, experts, scale_zp_a, scale_zp_b, output, N, K, shared_N, shared_K, qparams_per_exp, recv_tokens_per_exp, kernel_id: int = -1, acc_dump=None) -> GroupGemmLaunch:
+    """The pointer-table part of `gg_mxmoe_share_fused`, reusable across launches (CUDA-graph friendly)."""
     recv_cpu = recv_tokens_per_exp.cpu()
     e_cnt = recv_cpu.shape[0]
     num_tokens = output[-1].shape[0] if len(output) else 0             # rows of the last problem (the shared expert's, when there is one)
@@ -373,7 +372,7 @@ def prepare_gg(inp, experts, scale_zp_a, scale_zp_b, output, N, K, shared_N, sha
     qps = [qparams_per_exp[e] for e in idx]
     qps = qps if type(qps[0] if qps else ()) is tuple else [tuple(q) for q in qps]
     g = GroupGemmLaunch(inp, [experts[e] for e in idx], sa, None if scale_zp_b is None else [scale_zp_b[e] for e in idx], output[:len(idx)], sizes, qps,
-                        kernel_id=kernel_id, acc=acc_dump, few_rows=few_rows)
+                        kernel_id=kernel_id, acc=acc_dump)
     g.qparams = qps
     return g
 
