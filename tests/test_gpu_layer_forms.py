@@ -95,3 +95,29 @@ def test_layer_of_65_to_128_tokens_against_float64(mix, tokens):
         out = (gate / (1 + torch.exp(-gate)) * up) @ dense(weights[e][1], formats[e][1]).T.contiguous()
         want.index_add_(0, rows, out * (1.0 if slot is None else w[rows, slot].double()[:, None]))
     assert (got - want).norm() <= 1.5 * 2.0 ** -10 * want.norm()
+
+
+@pytest.mark.parametrize("tokens", [1, 24, 64])
+def test_layer_on_the_few_row_kernel_with_many_token_tiles(tokens):
+    """groupgemm_hz_fused_all_few, which lists of w4a4 / w8a8 beside weight-only problems take: a layer of such lists takes the kernel without tiles for many tokens; named for both blocks, with a head and by host tables,
+    identical outputs."""
+    from mxmoe_amd import _lib, synth as S
+    from mxmoe_amd.layer import MxMoELayer
+
+    lib = _lib.load()
+    name = lambda kid: lib.mxmoe_kernel_name(kid).decode().split("groupgemm_hz_fused_")[-1]  # noqa: E731
+    fm = [(S.W4A4, S.W8A8), (S.W8A8, S.W4A16), (S.W4A16, S.W4A4), (S.W3A16, S.W8A8), (W8A16, S.W2A16)]
+    cfg = S.MoEConfig("t", "test", 10, 2, 512, 512, tokens, num_shared=1, rotate=1)
+    layer = MxMoELayer(cfg, formats=[fm[i % 5] for i in range(11)])
+    assert "all_few" not in {name(k) for k in layer._kernels(tokens, 2)} and (tokens < 24 or name(layer._kernels(tokens, 2)[0]) == "mixed_few")
+    kid = lib.mxmoe_find_kernel(b"groupgemm_hz_fused_all_few")
+    layer = MxMoELayer(cfg, formats=layer.formats, packed=(layer.w13, layer.w2))
+    layer._planned_kernel = lambda *_, **__: kid
+    hidden, (ids, w) = S.make_hidden(cfg).cuda(), S.make_routing(cfg)
+    ids[:, 0] = 1
+    ids, w = ids.cuda(), w.cuda()
+    got = layer(hidden, ids, w).clone()
+    assert layer._kernels(tokens, 2) == (kid, kid) and lib.mxmoe_layer_has_head(layer._short[tokens, 2]._handle)
+    assert torch.equal(layer.call_with_host_tables(hidden, ids, w), got)
+    layer._short[tokens, 2] = None
+    assert torch.equal(layer(hidden, ids, w), got)

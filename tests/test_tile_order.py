@@ -200,3 +200,22 @@ def test_device_planner_makes_the_same_phases(lib, fmts, long_k):
     e = 96
     counts = [(150, 0, 40, 7, 300)[i % 5] for i in range(e)]
     _device_plan_is_the_hosts(lib, [fmts[i % len(fmts)] for i in range(e)], counts, 2048, [long_k if i % 9 == 4 else 1408 for i in range(e)])
+
+
+@pytest.mark.parametrize("q,rows,shared,k", [(W8, 546, 8192, 5632), (WO, 192, 2049, 2816), (FP, 120, 1788, 5632), (W4, 4, 64, 5632), (W8, 300, 1300, 2816), (W8, 100, 136, 2816)])
+def test_the_phase_of_a_long_problem_is_dealt_in_equal_runs(lib, q, rows, shared, k):
+    """All tiles of its phases together: every XCD the same number, but for the last ones, which get what is left."""
+    tab, area = _launch(lib, [(rows, 2048, 1408, q)] * 60 + [(shared, 2048, k, q)])
+    live = area[area[:, 0] >= 0]
+    bounds, seen = tab[13:14 + tab[2]], 0
+    for lo, hi in zip(bounds, bounds[1:]):
+        phase = area[lo:hi]
+        if not (phase[:, 0] == 60).any():
+            continue
+        per_xcd = [int((phase[x::8, 0] >= 0).sum()) for x in range(8)]
+        total = sum(per_xcd)
+        run = -(-total // 8)
+        if (phase[phase[:, 0] >= 0, 0] == 60).all():
+            assert per_xcd == [min(run, max(0, total - run * x)) for x in range(8)]
+            seen += total
+    assert seen >= 0.8 * (live[:, 0] == 60).sum()
