@@ -305,7 +305,7 @@ int mxmoe_upload(void* dst, const void* host_src, size_t bytes, void* stream);
  * One call enqueues the whole forward of one layer for one (tokens, top-k): permutation, planning and the quantisation of every
  * token once per activation format in one launch; the gate_up GroupGEMM with rows gathered by token and silu(gate) * up as its
  * output; quantisation of those rows (left out when every second block reads fp16); the down GroupGEMM; the combine.  Results are
- * bit for bit those of the separate entry points above.
+ * bit for bit those of the separate entry points above on the same kernels.
  *
  * mxmoe_layer_desc names everything that does not change from call to call; every buffer belongs to the caller, is device memory
  * (h_* excepted) and is sized for the worst routing (R = num_tokens * topk rows):

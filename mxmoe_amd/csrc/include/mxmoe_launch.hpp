@@ -476,13 +476,14 @@ struct PlanBranch {
 // A phase of such tiles keeps the plain workgroup order (no XCD remap): the few-token weight-only tiles stream their own weights
 // and share nothing but a few rows of activations with their neighbours.
 __host__ __device__ inline bool flat_phase(const PlanBranch& b) { return b.BM <= 16 || (is_weight_only((Fmt)b.fmt) && b.BM < 128); }
-// Tiles of size 2^lg that cover `x`.
 // Whether the tiles of a shape's problems above the launch's smallest K (a shared expert's second block, two or four times as long as the routed experts') are a phase of their own,
 // so that every XCD gets an eighth of them as well as of the others.  In one phase the XCDs get equal numbers of tiles, and the first of them all the long ones, which the launch then
 // waited for while half of the chip was idle (a second block of 64 experts and a shared one of twice their width, 2049 tokens: CUs busy 0.52 of the time, 173 us).  Layers, us, one phase / two: 64 experts
 // top-6 and a shared one, 2049 tokens, w4a16 385 / 332, w4a4 and w8a8 267 / 259; 60 experts top-4 and one four times as wide, w4a4 and w8a8 64 tokens 112 / 103, 2049 tokens 283 / 259, w4a16 / w3a16
-// 442 / 339, 8192 tokens 1375 / 1051; up to 2% either way between 128 and 512 tokens.
+// 442 / 339, 8192 tokens 1375 / 1051.  No lower limit: both layers in five mixes, even and skewed, 129 .. 400 tokens, two phases take 0.96 .. 1.01 of one's time (the planner with the code for it 0.2 to 0.5 us more, shared tiles of few rows
+// are mostly flat phases), 512 tokens 0.94 .. 1.02, 777 0.89 .. 1.01.
 __host__ __device__ inline bool long_phase(const PlanBranch& b, int long_tiles, int other_tiles) { return long_tiles > 0 && other_tiles > 0 && !flat_phase(b); }
+// Tiles of size 2^lg that cover `x`.
 __host__ __device__ inline int tiles_over(int x, int lg) { return (x + (1 << lg) - 1) >> lg; }
 constexpr int kNumFmts = (int)Fmt::UNSUPPORTED;
 struct PlanInfo {

@@ -7,7 +7,7 @@
 //   down      the fused GroupGEMM of the second block;
 //   combine   un-permute, top-k weighted sum, shared expert.
 //
-// A few tokens of a layer whose first blocks take them as they are (16-bit activations) need no head: layer_first_kernel.
+// Few tokens on the kernels for few rows need no head (layer_first_kernel); what is left of it in front of gate_up is the tokens' quantisation, where first blocks take quantised ones.
 //
 // Against the form that writes an activation row per destination (top-k of them per token, after the permutation is known) and stores
 // gate and up: the head is one launch instead of two or three in sequence, activations take 1 / top-k of the space, and 8 bytes per

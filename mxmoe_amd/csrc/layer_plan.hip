@@ -211,7 +211,7 @@ int mxmoe_plan_select_kernel_rows(const mxmoe_block_desc* h_desc, int num_expert
 }
 
 int mxmoe_layer_kernel(const mxmoe_block_desc* h_desc, int num_experts, int num_tokens, int topk, int shared_rows, int first) {
-  // (integer sums are the same whichever kernel runs; fp8 ones are not to the last bit, and stay where a list of the same rows would run, nor are those of 16-bit activations in tiles of many tokens)
+  // (fp8 blocks keep the limits of a layer with a head: 64 tokens, 768 blocks; beyond them both sides were not measured)
   const int et = num_experts + (shared_rows > 0 ? 1 : 0);
   bool fp8 = false;
   for (int i = 0; h_desc && i < et; ++i) fp8 = fp8 || wants_fp8(h_desc[i].q);

@@ -323,7 +323,7 @@ class MxMoELayer:
         Same kernels and results as `forward` + `combine`, but nothing here waits for the routing: the tables of both launches are
         derived from the tokens-per-expert counts by a planning kernel on the device (`mxmoe_plan_layer`: both blocks in one launch), the stores and plan
         buffers are allocated once per (tokens, top-k) for the worst case, and every launch argument is independent of the data.
-        The call only enqueues four or five kernels (`mxmoe_layer_run`; six to nine, in separate calls, for what that form does not take:
+        The call only enqueues three to six kernels (`mxmoe_layer_run`; six to nine, in separate calls, for what that form does not take:
         hidden sizes other than 512, 1024, 2048 and 4096, intermediate sizes that are no multiple of 32, more than 512 experts, bf6
         operands, and batches of more than 65536 (token, slot) pairs whose chunks of 256 times the experts exceed 16384, i.e. every
         larger batch from 64 experts on); no synchronisation, no allocation after the first call when `out` is given (but a copy of a
